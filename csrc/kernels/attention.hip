@@ -12,18 +12,18 @@
 // two 16-token S^T tiles whose token lists interleave in 4s
 // (tile a holds tokens 8*(row>>2) + 4a + (row&3)), so lane group h owns tokens
 // 8h..8h+7 of the group = exactly the k-slice its B fragment needs.
-// The contraction over D uses a k permutation (lane group h covers dims
-// 32h..32h+31 across the 4 MFMAs), making each lane's K and Q reads 64
-// contiguous bytes.  Softmax is online (running max / sum per query column),
+// MFMA i of the contraction over D takes dims 32 i + 8 h from lane group h: one
+// load instruction of the decode kernels reads 64 contiguous bytes of each of 16
+// K rows (a 64-byte run per lane, as the LDS-staged prompt kernel reads its tile,
+// touches twice the lines per instruction: 64 x 900 tokens 67 -> 63 us).  Softmax is online (running max / sum per query column),
 // in base 2 with the 1/sqrt(D)*log2(e) scale folded into one multiply.
 //
-// Decode (K5): grid (seq, kv_head, partition); 8 waves x 32 tokens = 256
-// tokens per partition (two workgroups resident per CU); the G = Hq/Hkv query heads of a kv head are the MFMA
-// columns (K/V are read once per kv head).  Multi-partition sequences write
-// fp32 partials that the last-arriving partition combines (split-KV,
-// flash-decoding, one launch).
-// The grid is sized for the max context so the launch is hipGraph-capturable;
-// partitions past a sequence's context exit at once.
+// Decode (K5): grid (seq, kv_head, partition), 8 waves, 256 tokens (32 per wave) a step; the
+// G = Hq/Hkv query heads of a kv head are the MFMA columns (K/V are read once per kv head).
+// Multi-partition sequences write fp32 partials that the last-arriving partition combines
+// (split-KV, flash-decoding, one launch).  The number of partitions comes from the number of
+// (sequence, kv head) units alone, so the launch is hipGraph-capturable; the kernel cuts every
+// context into that many equal parts, and workgroups past the last one exit at once.
 //
 // Prefill (K4): causal + varlen + chunked prefill (queries are the LAST qlen
 // positions of a context of length ctx), reading K/V from the paged cache.
@@ -47,304 +47,10 @@ template <int GMAX>
 __global__ __launch_bounds__(DWAVES * 64, 4) void attn_decode_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
     const int* __restrict__ block_tables, const int* __restrict__ ctx_lens, bf16* __restrict__ out,
-    float* __restrict__ tmp_o, float* __restrict__ tmp_ml, int* __restrict__ counters, int Hq, int Hkv, int BS,
-    int max_blocks, int max_parts, float scale_log2) {
-  attn_decode_unit<GMAX>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, Hq, Hkv, BS,
-                       max_blocks, max_parts, scale_log2, blockIdx.x, blockIdx.y, blockIdx.z);
-}
-
-// ---------------------------------------------------------------------------------------------
-// Decode, wide batches: one wave per (seq, kv head) walking its whole context
-// ---------------------------------------------------------------------------------------------
-// The grid kernel spends an 8-wave workgroup per (seq, kv head, 256-token partition): built for a few
-// sequences, where spreading one context over 8 waves shortens the step.  At wide decode batches (128-256
-// sequences of 0.5-4K tokens) the units outnumber the resident workgroups several times over and each
-// unit's latency chain (metadata, K/V, cross-wave LDS merge, split-KV publish) is paid per round: K/V
-// streams at 4.3-5.0 TB/s (grid / streaming kernels).  Here a unit is ONE wave that walks the 32-token
-// groups of its context with the next group's K/V loads in flight (two register sets), keeps the online
-// softmax in registers (compute_group, attn_decode.h) and writes its output rows itself: no LDS, no
-// barrier, no partials.  The 2048 units of a 256-sequence Llama-3-8B step are resident at once (two
-// waves per SIMD).  The block-table row (<= 64 entries) is read once, one entry per lane, and each
-// group's block number is a lane read (v_readlane) instead of a dependent load: no load in the loop
-// besides the K/V stream, so the compiler's counted waits keep the next group's loads in flight.
-constexpr int WAVE_UNITS = 4;  // units (waves) per workgroup
-
-__global__ __launch_bounds__(WAVE_UNITS * 64, 2) void attn_decode_wave_kernel(
-    const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
-    const int* __restrict__ block_tables, const int* __restrict__ ctx_lens, bf16* __restrict__ out, int num_units,
-    int Hq, int Hkv, int BS, int max_blocks, float scale_log2) {
-  const int lane = threadIdx.x & 63;
-  const int unit = blockIdx.x * WAVE_UNITS + (threadIdx.x >> 6);
-  if (unit >= num_units) return;  // uniform over the wave
-  const int seq = unit / Hkv, kvh = unit - seq * Hkv;
-  const int G = Hq / Hkv;
-  const int c = lane & 15, h = lane >> 4;
-  const int bsh = __builtin_ctz(BS);
-  const int* bt = block_tables + (long long)seq * max_blocks;
-  const int btv = bt[min(lane, max_blocks - 1)];  // max_blocks <= 64 (launcher)
-  bf16x8 qf[4];
-  load_q(q, seq, Hq, kvh, G, qf);
-  const int ctx = ctx_lens[seq];
-  const int ngroups = (ctx + 31) >> 5;
-
-  auto issue = [&](int g, KVFrag& f) {
-    const int tok0 = g << 5;
-    const int blk = __builtin_amdgcn_readlane(btv, tok0 >> bsh);
-    const int boff = tok0 & (BS - 1);
-    load_group(k_cache + (((long long)blk * Hkv + kvh) * BS + boff) * D,
-               v_cache + ((long long)blk * Hkv + kvh) * (long long)D * BS + boff, BS, f);
-    __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the compute (no load sinking)
-  };
-  f32x4 o[8];
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, lsum = 0.f;
-  auto compute = [&](const KVFrag& f, int g) {
-    const int tok0 = g << 5;
-    compute_group(f, qf, scale_log2, [&](int a, int r) { return tok0 + 8 * h + 4 * a + r < ctx; }, o, m, lsum);
-  };
-  // two register sets: group g computes while g + 1 loads.  The prefetch is unconditional (the last
-  // group is re-read past the end): a conditional one makes the compiler's wait before the compute drain
-  // the prefetched loads too (vmcnt(0) at the merge point), serialising the stream.
-  const int last = max(ngroups - 1, 0);
-  KVFrag f0, f1;
-  issue(0, f0);
-  for (int g = 0; g < ngroups; g += 2) {
-    issue(min(g + 1, last), f1);
-    compute(f0, g);
-    if (g + 1 >= ngroups) break;
-    issue(min(g + 2, last), f0);
-    compute(f1, g + 1);
-  }
-  lsum += __shfl_xor(lsum, 16, 64);
-  lsum += __shfl_xor(lsum, 32, 64);
-  if (c < G) {
-    // lane (c, h) holds dims 16 dt + 4 h .. + 3 of query column c
-    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-    bf16* op = out + ((long long)seq * Hq + kvh * G + c) * D + 4 * h;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      union {
-        uint2 u;
-        bf16 h[4];
-      } pk;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) pk.h[r] = (bf16)(o[dt][r] * inv);
-      *reinterpret_cast<uint2*>(op + 16 * dt) = pk.u;
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
-// Decode, long contexts: one wave per (seq, kv head, 384-token partition) streaming its K/V groups
-// through a private LDS ring by LDS-DMA
-// ---------------------------------------------------------------------------------------------
-// The grid kernel above gives every wave ONE 32-token group: at 2K+ contexts each unit is one load round
-// trip followed by a cross-wave merge and a split-KV publish, so HBM idles through the finish phases
-// (2.9 TB/s at 2K in a real decode step).  Here a single-wave workgroup walks SG groups of its partition
-// with up to 3 groups' K/V in flight by LDS-DMA (16 KB per group, a 64 KB ring, two workgroups per CU:
-// ~96 KB in flight per CU without spending registers), reuses the group math of attn_decode.h
-// (compute_group) on fragments read from the ring, and publishes one partial per 384 tokens into the same
-// split-KV combine.  LDS images are XOR-swizzled so every fragment read is bank-conflict free:
-//   K: 32 token rows x 256 B, 16-B chunk ^ ((t & 3) | ((t >> 4) & 1) << 3);
-//   V: 128 dim rows x 64 B (32 tokens), chunk ^ {0, 2, 3, 1}[(d >> 2) & 3].
-// SG: 32-token groups per streamed partition; SNS: ring slots (16 KB each: K 8 KB + V 8 KB)
-
-SYM_DEV int kswz(int t) { return (t & 3) | (((t >> 4) & 1) << 3); }
-SYM_DEV int vswz(int d) { return (0x1320 >> (4 * ((d >> 2) & 3))) & 3; }
-
-SYM_DEV unsigned sm_addr(const char* p) {
-  return (unsigned)(unsigned long long)(const __attribute__((address_space(3))) char*)p;
-}
-
-SYM_DEV void glds16(const bf16* src, char* lds) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                   (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
-}
-
-template <int N>
-SYM_DEV void wait_vm_groups() {  // all but the N youngest groups' 16 DMAs each
-  if constexpr (N == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  else if constexpr (N == 1) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-  else if constexpr (N == 2) asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
-  else asm volatile("s_waitcnt vmcnt(48)" ::: "memory");
-}
-
-template <int GMAX, int SG, int SNS>
-__global__ __launch_bounds__(64) void attn_decode_stream_kernel(
-    const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
-    const int* __restrict__ block_tables, const int* __restrict__ ctx_lens, bf16* __restrict__ out,
-    float* __restrict__ tmp_o, float* __restrict__ tmp_ml, int* __restrict__ counters, int Hq, int Hkv, int BS,
-    int max_blocks, int max_parts, float scale_log2) {
-  static_assert((SNS & (SNS - 1)) == 0 && SNS >= 2 && SNS <= 4 + 1, "ring slots");
-  constexpr int SPART = SG * 32;
-  __shared__ __attribute__((aligned(1024))) char smem[SNS * 16384];
-  const int seq = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
-  const int lane = threadIdx.x;
-  const int r16 = lane & 15, h = lane >> 4;
-  const int G = Hq / Hkv;
-  const int bsh = __builtin_ctz(BS);
-  const int* bt = block_tables + (long long)seq * max_blocks;
-  const int t0 = part * SPART;
-  // context, this lane's block-table entry (lane g: group g of the partition) and the query are
-  // independent loads: one round trip before the stream starts
-  const int myblk = bt[min((t0 + 32 * min(lane, SG - 1)) >> bsh, max_blocks - 1)];
-  bf16x8 qf[4];
-  load_q(q, seq, Hq, kvh, G, qf);
-  const int ctx = ctx_lens[seq];
-  if (t0 >= ctx) return;
-  const int ng = min(SG, (ctx - t0 + 31) >> 5);
-
-  // DMA of group g into ring slot so: K rows token-major (8 x 1 KB: 4 rows of 256 B each), V rows
-  // dim-major (8 x 1 KB: 16 dims x 64 B each); the swizzle permutes the SOURCE chunks, the LDS image
-  // is written lane-linear
-  const int kt = lane >> 4, kc = lane & 15;   // K: row within a 4-row piece, chunk
-  const int vd = lane >> 2, vc = lane & 3;    // V: dim within a 16-dim piece, chunk
-  auto issue = [&](int g, int so) {
-    const int blk = __shfl(myblk, g, 64);
-    const int boff = (t0 + 32 * g) & (BS - 1);
-    const bf16* kb = k_cache + (((long long)blk * Hkv + kvh) * BS + boff) * D;
-    const bf16* vb = v_cache + ((long long)blk * Hkv + kvh) * (long long)D * BS + boff;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int t = 4 * j + kt;
-      glds16(kb + t * D + 8 * (kc ^ kswz(t)), smem + so + j * 1024);
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int d = 16 * j + vd;
-      glds16(vb + (long long)d * BS + 8 * (vc ^ vswz(d)), smem + so + 8192 + j * 1024);
-    }
-  };
-
-  f32x4 o[8];
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, lsum = 0.f;
-
-  // fragment read offsets (load_group's layouts): K row trow(a), dims 32 h + 8 i = chunk 4 h + i;
-  // V row 16 dt + r16, chunk h
-  const unsigned base = sm_addr(smem);
-  int koff[2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a) {
-    const int trow = (r16 >> 2) * 8 + 4 * a + (r16 & 3);
-    koff[a] = trow * 256;
-  }
-#pragma unroll
-  for (int g = 0; g < SNS - 1; ++g)
-    if (g < ng) issue(g, g * 16384);
-  for (int g = 0; g < ng; ++g) {
-    // this group's 16 DMAs landed; the (up to SNS - 2) younger groups stay in flight
-    const int younger = min(ng - 1 - g, SNS - 2);
-    if (younger >= 3) wait_vm_groups<3>();
-    else if (younger == 2) wait_vm_groups<2>();
-    else if (younger == 1) wait_vm_groups<1>();
-    else wait_vm_groups<0>();
-    const int so = (g & (SNS - 1)) * 16384;
-    if (g + SNS - 1 < ng) issue(g + SNS - 1, ((g + SNS - 1) & (SNS - 1)) * 16384);  // slot of g - 1, read before
-    KVFrag f;
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const int trow = (r16 >> 2) * 8 + 4 * a + (r16 & 3);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        f.k[a][i] = *(const bf16x8*)(smem + so + koff[a] + 16 * ((4 * h + i) ^ kswz(trow)));
-    }
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      const int d = 16 * dt + r16;
-      f.v[dt] = *(const bf16x8*)(smem + so + 8192 + d * 64 + 16 * (h ^ vswz(d)));
-    }
-    const int tg = t0 + 32 * g;
-    compute_group(f, qf, scale_log2, [&](int a, int r) { return tg + 8 * h + 4 * a + r < ctx; }, o, m, lsum);
-  }
-  (void)base;
-
-  // ---- finish: one wave holds the whole partition state.  Lane (c = r16, h) owns query column c,
-  // dims 16 dt + 4 h + r.
-  lsum += __shfl_xor(lsum, 16, 64);
-  lsum += __shfl_xor(lsum, 32, 64);
-  const int nparts = (ctx + SPART - 1) / SPART;
-  const bool col = r16 < G;
-  const int head = kvh * G + r16;
-  if (nparts == 1) {
-    if (col) {
-      const float inv = 1.f / lsum;
-      bf16* op = out + ((long long)seq * Hq + head) * D + 4 * h;
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) {
-        bf16x4 v;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = (bf16)(o[dt][r] * inv);
-        *reinterpret_cast<bf16x4*>(op + 16 * dt) = v;
-      }
-    }
-    return;
-  }
-  // split-KV publish (write-through partials, drained, then the arrival counter; the last partition
-  // combines: the hand-off protocol of attn_finish in attn_decode.h)
-  if (col) {
-    const long long pb = (((long long)seq * Hq + head) * max_parts + part);
-    float* po = tmp_o + pb * D + 4 * h;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        __hip_atomic_store(po + 16 * dt + r, o[dt][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (h == 0) {
-      __hip_atomic_store(tmp_ml + pb * 2, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(tmp_ml + pb * 2 + 1, lsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  int* cnt = counters + (long long)seq * Hkv + kvh;
-  int old = 0;
-  if (lane == 0) old = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  old = __shfl(old, 0, 64);
-  if (old != nparts - 1) return;
-  // combine: lane (qq = lane >> 4 within a batch of 4 query columns, 8 dims d0 = (lane & 15) * 8)
-  const int d0 = (lane & 15) * 8;
-  for (int c0 = 0; c0 < G; c0 += 4) {
-    const int qq = c0 + (lane >> 4);
-    if (qq < G) {
-      const long long bb = ((long long)seq * Hq + kvh * G + qq) * max_parts;
-      float M = -INFINITY, L = 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      for (int p0 = 0; p0 < nparts; p0 += 4) {
-        float mp[4], lp[4], vp[4][8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int p = min(p0 + i, nparts - 1);
-          mp[i] = __hip_atomic_load(tmp_ml + (bb + p) * 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          lp[i] = __hip_atomic_load(tmp_ml + (bb + p) * 2 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          const float* po = tmp_o + (bb + p) * D + d0;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) vp[i][j] = __hip_atomic_load(po + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        float mb = M;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (p0 + i < nparts) mb = fmaxf(mb, mp[i]);
-        const float fo = __builtin_amdgcn_exp2f(M - mb);
-        L *= fo;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[j] *= fo;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float f = p0 + i < nparts ? __builtin_amdgcn_exp2f(mp[i] - mb) : 0.f;
-          L += lp[i] * f;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) acc[j] += vp[i][j] * f;
-        }
-        M = mb;
-      }
-      const float inv = 1.f / L;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) acc[j] *= inv;
-      store8(out + ((long long)seq * Hq + kvh * G + qq) * D + d0, acc);
-    }
-  }
-  if (lane == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    float* __restrict__ tmp_o, float* __restrict__ tmp_ml, int* __restrict__ counters, int Hq, int Hkv, int G, int BS,
+    int max_blocks, int max_parts, float scale_log2, unsigned inv_parts) {
+  attn_decode_unit<GMAX>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, Hq, Hkv, G, BS,
+                       max_blocks, max_parts, scale_log2, inv_parts, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -373,9 +79,9 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(
 
   bf16x8 qf[4];
   if (row_ok) {
-    const bf16* qp = q + ((long long)(qstart + myrow) * Hq + head) * D + 32 * h;
+    const bf16* qp = q + ((long long)(qstart + myrow) * Hq + head) * D + 8 * h;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) qf[i] = ld16(qp + 8 * i);
+    for (int i = 0; i < 4; ++i) qf[i] = ld16(qp + 32 * i);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) qf[i] = zero8();
@@ -839,37 +545,16 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_m32p_kernel(
 
 }  // namespace
 
-static int g_attn_stream_min = [] {
-  const char* knob = getenv("SYMMETRY_ATTN_STREAM_MIN");
-  return knob ? atoi(knob) : 1024;
-}();
-
-void set_attn_stream_min(int tokens) { g_attn_stream_min = tokens; }
-
-// wide batches: the one-wave-per-(seq, kv head) kernel from this many units (seqs x kv heads) for block
-// tables spanning at least this many tokens (and <= 64 blocks).  bench_attn_decode.py --wave 0 1
-// (profiles/attn_decode_wave_r2.jsonl): at >= 128 sequences x 700-3000 tokens it streams K/V at 5.1-5.9 TB/s
-// vs 4.3-5.0 for the grid / streaming kernels (-8..-20 %); at 64 sequences, or ~170-token contexts in the
-// 512-token bucket, those stay ahead.  SYMMETRY_ATTN_WAVE_UNITS (0: never) / SYMMETRY_ATTN_WAVE_SPAN.
-static int g_attn_wave_units = [] {
-  const char* knob = getenv("SYMMETRY_ATTN_WAVE_UNITS");
-  return knob ? atoi(knob) : 1024;
-}();
-static int g_attn_wave_span = [] {
-  const char* knob = getenv("SYMMETRY_ATTN_WAVE_SPAN");
-  return knob ? atoi(knob) : 513;
-}();
-
-void set_attn_wave(int min_units, int min_span) {
-  g_attn_wave_units = min_units;
-  g_attn_wave_span = min_span;
-}
-
-// A/B knob (partition length x ring depth of the streaming kernel): SYMMETRY_ATTN_STREAM_CFG
-static int g_attn_stream_cfg = [] {
-  const char* knob = getenv("SYMMETRY_ATTN_STREAM_CFG");
-  return knob ? atoi(knob) : 0;
-}();
+// Decode: a unit is a (sequence, kv head); contexts are cut so far that the workgroups just fill the chip, two 8-wave
+// workgroups on each of the 256 CUs (past it: 48 sequences x 8 kv heads, contexts around 250, one partition 20 us, two
+// 24).  The kernel replaced a one-wave-per-partition LDS-DMA streaming kernel and a one-wave-per-unit kernel; us for the
+// streaming / per-unit / this kernel, contexts spread by half around the mean and other weights read in between:
+//   1 sequence x 700 tokens, 8 kv heads   17.3 /  46 /  8.5      64 x 900      66 /  88 /  52  (236 MB: 4.6 TB/s)
+//   8 x 1100, 4 kv heads                  17.8 /  92 /  9.7      32 x 4000    148 /   - / 111
+//   5 x 5400, 4 kv heads                  28.7 /   - / 22.8      160 x 600    112 / 126 /  84
+//   48 x 60                                8.8 / 9.3 /  6.5      256 x 2000   428 / 370 / 335
+// Bound by the K/V stream from ~100 MB on, by four dependent round trips (context, K/V, publish, combine) below ~20 MB.
+constexpr int DECODE_UNITS = 512;
 
 void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache, const int* block_tables,
                         const int* ctx_lens, bf16* out, float* tmp_o, float* tmp_ml, int* counters, int num_seqs,
@@ -877,43 +562,17 @@ void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache,
   if (num_seqs == 0) return;
   const float scale_log2 = scale * 1.4426950408889634f;
   const int G = Hq / Hkv;
-  // block tables spanning >= g_attn_stream_min tokens (the graph's context bucket): the streaming
-  // one-wave kernel
-  const int span = max_blocks * BS;
-  if (g_attn_wave_units > 0 && num_seqs * Hkv >= g_attn_wave_units && span >= g_attn_wave_span && G <= 16 &&
-      max_blocks <= 64) {
-    const int units = num_seqs * Hkv;
-    attn_decode_wave_kernel<<<(units + WAVE_UNITS - 1) / WAVE_UNITS, WAVE_UNITS * 64, 0, s>>>(
-        q, k_cache, v_cache, block_tables, ctx_lens, out, units, Hq, Hkv, BS, max_blocks, scale_log2);
-    return;
-  }
-  if (g_attn_stream_min > 0 && span >= g_attn_stream_min && BS >= 32 && G <= 16) {
-    // partitions of SG 32-token groups (>= 256 tokens: sparts <= max_parts, sized for 256-token ones)
-    auto run = [&](auto kern, int sg) {
-      const dim3 g(num_seqs, Hkv, (span + 32 * sg - 1) / (32 * sg));
-      kern<<<g, 64, 0, s>>>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, Hq, Hkv, BS,
-                            max_blocks, max_parts, scale_log2);
-    };
-    switch (g_attn_stream_cfg) {
-      case 1: run(attn_decode_stream_kernel<16, 8, 4>, 8); break;
-      case 2: run(attn_decode_stream_kernel<16, 12, 2>, 12); break;
-      case 3: run(attn_decode_stream_kernel<16, 24, 4>, 24); break;
-      case 4: run(attn_decode_stream_kernel<16, 16, 4>, 16); break;
-      case 5: run(attn_decode_stream_kernel<16, 8, 2>, 8); break;
-      default: run(attn_decode_stream_kernel<16, 12, 4>, 12); break;
-    }
-    return;
-  }
-  dim3 grid(num_seqs, Hkv, max_parts);
-  if (G <= 4)
-    attn_decode_kernel<4><<<grid, DWAVES * 64, 0, s>>>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml,
-                                                       counters, Hq, Hkv, BS, max_blocks, max_parts, scale_log2);
-  else if (G <= 8)
-    attn_decode_kernel<8><<<grid, DWAVES * 64, 0, s>>>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml,
-                                                       counters, Hq, Hkv, BS, max_blocks, max_parts, scale_log2);
-  else
-    attn_decode_kernel<16><<<grid, DWAVES * 64, 0, s>>>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml,
-                                                        counters, Hq, Hkv, BS, max_blocks, max_parts, scale_log2);
+  const int units = num_seqs * Hkv;  // (parts <= 512: attn_decode_unit's exact division)
+  const int parts = min(max_parts, max(1, DECODE_UNITS / units));
+  const dim3 grid(num_seqs, Hkv, parts);
+  const unsigned inv = (unsigned)((1ull << 32) / parts) + 1;  // (not used for one partition)
+  auto run = [&](auto kern) {
+    kern<<<grid, DWAVES * 64, 0, s>>>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, Hq, Hkv,
+                                      G, BS, max_blocks, max_parts, scale_log2, inv);
+  };
+  if (G <= 4) run(attn_decode_kernel<4>);
+  else if (G <= 8) run(attn_decode_kernel<8>);
+  else run(attn_decode_kernel<16>);
 }
 
 void launch_attn_prefill(const bf16* q, const bf16* k_cache, const bf16* v_cache, const int* block_tables,

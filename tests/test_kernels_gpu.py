@@ -169,6 +169,31 @@ def test_attn_decode(gpu, attn_decode_kernel, Hq, Hkv, BS):
     assert torch.equal(out, out2)
 
 
+@pytest.mark.parametrize("S,Hq,Hkv", [(65, 32, 8), (40, 32, 8), (30, 32, 8), (7, 16, 16), (3, 64, 8), (1, 32, 4)])
+def test_attn_decode_equal_partitions(gpu, S, Hq, Hkv):
+    """Equal partitions of a context: one partition of several 256-token steps (512 / units < 2), two and
+    more, steps that do not divide by them, and block tables past the 128 preloaded entries.  Probabilities and outputs are
+    rounded to bf16 (2^-9 each) and the values are N(0, 1): 8 standard deviations of both roundings stay under 2e-2."""
+    g = torch.Generator(device=gpu).manual_seed(31 + S)
+    edges = [1, 256, 257, 512, 513, 767, 769, 1025, 2300, 4700]
+    ctx_lens = [edges[(3 * i + S) % len(edges)] for i in range(S)]
+    kc, vc, bt = _random_paged(gpu, ctx_lens, Hkv, 32, g)
+    q = torch.randn(S, Hq, 128, device=gpu, generator=g).bfloat16()
+    ctx = torch.tensor(ctx_lens, device=gpu, dtype=torch.int32)
+    max_parts = (bt.shape[1] * 32 + ops.ATTN_DECODE_PART - 1) // ops.ATTN_DECODE_PART
+    tmp_o = torch.empty(S, Hq, max_parts, 128, device=gpu)
+    tmp_ml = torch.empty(S, Hq, max_parts, 2, device=gpu)
+    out = torch.full((S, Hq, 128), float("nan"), device=gpu, dtype=torch.bfloat16)
+    cnt = torch.zeros(S * Hkv, device=gpu, dtype=torch.int32)
+    scale = 1 / math.sqrt(128)
+    for _ in range(2):  # (the second call finds the counters re-armed)
+        ops.attn_decode(q, kc, vc, bt, ctx, out, tmp_o, tmp_ml, cnt, scale)
+    assert int(cnt.abs().sum()) == 0
+    out_r = torch.empty(S, Hq, 128, dtype=torch.bfloat16)
+    ref.attn_decode(q.cpu(), kc.cpu(), vc.cpu(), bt.cpu(), ctx.cpu(), out_r, scale=scale)
+    _close(out, out_r, atol=2e-2, rtol=2e-2)
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(32, 8), (64, 8), (8, 1), (16, 16)])
 @pytest.mark.parametrize("BS", [32, 64])
 def test_attn_decode_wave(gpu, Hq, Hkv, BS):
