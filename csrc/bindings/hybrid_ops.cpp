@@ -402,6 +402,32 @@ void conv_state_update(const Tensor& xin, Tensor& state, const OptTensor& cu_q, 
   launch_conv_state_update(a, f32, cur_stream(xin));
 }
 
+// y = f(x) . W^T for 1 to 16 rows; x and out may be column ranges; relu2: squared ReLU of x first; glu: W's rows are
+// [gate | up] and out = silu(gate) * up
+void row_linear(const Tensor& x, const Tensor& w, Tensor& out, bool relu2, bool glu) {
+  gpu(x, "x", false);
+  gpu(out, "out", false);
+  dtype(w, at::kBFloat16, "w");
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "row_linear: x bf16, 2-d operands");
+  const int64_t M = x.size(0), K = x.size(1), N = out.size(1);
+  const bool f32 = out.scalar_type() == at::kFloat;
+  TORCH_CHECK(f32 || out.scalar_type() == at::kBFloat16, "row_linear: out bf16 or fp32");
+  TORCH_CHECK(!(f32 && (relu2 || glu)) && !(relu2 && glu), "row_linear: one of fp32 output, relu2, glu");
+  TORCH_CHECK(M >= 1 && M <= 16 && out.size(0) == M, "row_linear: 1 to 16 rows");
+  TORCH_CHECK(w.size(1) == K && w.size(0) == (glu ? 2 * N : N), "row_linear: w does not fit x and out");
+  TORCH_CHECK(K >= 8 && K % 8 == 0 && K <= (1 << 22) && N >= 4 && N % 4 == 0 && N <= (1 << 30), "row_linear: K in 8s, N in 4s");
+  TORCH_CHECK(x.stride(1) == 1 && out.stride(1) == 1, "row_linear: inner strides must be 1");
+  const int64_t ldx = M > 1 ? x.stride(0) : K, ldo = M > 1 ? out.stride(0) : N;
+  TORCH_CHECK(ldx >= 0 && ldx % 8 == 0 && ldx <= (1 << 24) && ldo >= N && ldo % 4 == 0, "row_linear: row strides");
+  TORCH_CHECK((uintptr_t)x.data_ptr() % 16 == 0 && (uintptr_t)w.data_ptr() % 16 == 0 &&
+                  (uintptr_t)out.data_ptr() % (f32 ? 16 : 8) == 0,
+              "row_linear: alignment");
+  const at::OptionalDeviceGuard g(x.device());
+  TORCH_CHECK(launch_row_linear(x.data_ptr(), ldx, w.data_ptr(), out.data_ptr(), ldo, (int)M, (int)N, (int)K, f32, relu2, glu,
+                                cur_stream(x)),
+              "row_linear: K = ", K, " is neither at most 256 nor a multiple of 256");
+}
+
 void relu_sq(const Tensor& a, Tensor& out) {
   const int f32 = act(out, "out");
   TORCH_CHECK(out.dim() == 2, "relu_sq: out [R, F]");
@@ -1124,6 +1150,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
       &causal_conv_silu);
   m.def("conv_state_update(Tensor xin, Tensor(a!) state, Tensor? cu_q, Tensor prev_row, Tensor save_slot, int runs) -> ()",
         &conv_state_update);
+  m.def("row_linear(Tensor x, Tensor w, Tensor(a!) out, bool relu2, bool glu) -> ()", &row_linear);
   m.def("relu_sq(Tensor a, Tensor(a!) out) -> ()", &relu_sq);
   m.def("silu_mul(Tensor gate, Tensor up, Tensor(a!) out) -> ()", &silu_mul);
   m.def(

@@ -246,8 +246,11 @@ class BeletarLM:
 
     def _ff(self, P: dict, h: torch.Tensor) -> torch.Tensor:
         F = P["mlp"].ff
-        gu = self._linear("ff.gu", h, P["w_gu"])
         act = self._buf("ff.act", (h.shape[0], F))
+        if self.dtype == torch.bfloat16 and ops.few_rows(h, P["w_gu"], act):  # gate, up and their product in one launch
+            ops.row_linear(h, P["w_gu"], act, glu=True)
+            return self._linear("ff.down", act, P["w_down"])
+        gu = self._linear("ff.gu", h, P["w_gu"])
         ops.silu_mul(gu[:, :F], gu[:, F:], act)
         return self._linear("ff.down", act, P["w_down"])
 

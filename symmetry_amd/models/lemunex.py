@@ -194,7 +194,7 @@ class LemunexLM:
         return self.ws.get(name, shape, dtype or self.dtype, self.device)
 
     def _linear(self, name: str, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-        """x [R, K] @ w[N, K]^T -> [R, N] in the activation dtype (library GEMM, fp32 accumulation)."""
+        """x [R, K] @ w[N, K]^T -> [R, N] in the activation dtype (fp32 accumulation)."""
         return ops.linear(x, w, out=self._buf(name, (x.shape[0], w.shape[0])))
 
     @staticmethod
@@ -251,8 +251,12 @@ class LemunexLM:
             return None
         if isinstance(mlp, RoutedSpec):
             return self._routed(P, h, z)
+        up, out = self._cols(z, P, "up"), self._buf("ff.down", (h.shape[0], P["down"].shape[0]))
+        if self.dtype == torch.bfloat16 and ops.few_rows(up, P["down"], out):  # the squared ReLU on the way in
+            ops.row_linear(up, P["down"], out, relu2=True)
+            return out
         act = self._buf("ff.act", (h.shape[0], mlp.ff))
-        ops.relu_sq(self._cols(z, P, "up"), act)
+        ops.relu_sq(up, act)
         return self._linear("ff.down", act, P["down"])
 
     def _pair(self, i: int, P: dict, b: ForwardBatch, cache: HybridCache, z: torch.Tensor, runs: int):

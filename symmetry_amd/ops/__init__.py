@@ -530,18 +530,58 @@ def logits_argmax(logits, temps, seeds, step, out_keys, out_ids, n_offset=0):
     return reference.logits_argmax(logits, temps, seeds, step, out_keys, out_ids, n_offset)
 
 
+FEW_ROWS = 16  # rows up to which a linear layer is a weight stream (csrc/kernels/row_linear.hip)
+
+
+def few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None) -> bool:
+    """Does x @ w.T into ``out`` (row_linear's layouts: glu takes w of twice out's columns) run on the few-row kernel?  bf16
+    x and w on the GPU, 1..16 rows, w contiguous, unit inner strides, 16-byte aligned rows of x and w, K at most 256 in
+    eights or a multiple of 256, outputs in fours; everything else, and anything autograd records, is the library's."""
+    if out is None or x.dim() != 2 or not 0 < x.shape[0] <= FEW_ROWS or w.dim() != 2 or out.dim() != 2:
+        return False
+    if not _gpu(x) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not w.is_contiguous():
+        return False
+    M, K = x.shape
+    if w.device != x.device or out.device != x.device or w.shape[1] != K or out.shape[0] != M:
+        return False
+    if not (K % 256 == 0 or (K < 256 and K % 8 == 0)) or K == 0 or out.shape[1] % 4 or not out.shape[1]:
+        return False
+    if x.stride(1) != 1 or out.stride(1) != 1 or (M > 1 and (x.stride(0) % 8 or not 0 < x.stride(0) <= 1 << 24)):
+        return False
+    if M > 1 and (out.stride(0) % 4 or out.stride(0) < out.shape[1]):
+        return False
+    if x.data_ptr() % 16 or w.data_ptr() % 16 or out.data_ptr() % (4 * out.element_size()):
+        return False
+    return not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or out.requires_grad))
+
+
+def row_linear(x, w, out, relu2: bool = False, glu: bool = False) -> None:
+    """out [M, N] (bf16, or fp32 = the unrounded accumulator) = x @ w.T for few_rows operands.  ``relu2``: relu(x)^2, rounded to
+    bf16, in place of x; ``glu``: w [2 N, K] holds [gate | up] rows and out = silu(gate) * up of the bf16 projections."""
+    if _gpu(x):
+        return _hyb().row_linear(x, w, out, bool(relu2), bool(glu))
+    return reference.row_linear(x, w, out, relu2, glu)
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-    """Plain library GEMM ``x @ w.T`` for prefill-sized M (hipBLASLt through torch, the library heuristic; a
+    """``x @ w.T``: the few-row kernel up to 16 rows (2048 x 2048 at 8 rows 4.8 us, the library 8.5; 17688 x 2048 21.9 / 49.6;
+    past 16 rows the library is ahead), else the library GEMM (hipBLASLt through torch, the library heuristic; a
     tuned-solution table measured neutral end to end and was removed: profiles/r4/blaslt_tuned_ab.jsonl)."""
+    if few_rows(x, w, out) and out.dtype == torch.bfloat16 and out.shape[1] == w.shape[0]:
+        row_linear(x, w, out)
+        return out
     return torch.matmul(x, w.t(), out=out)
 
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
-    """out (fp32) = x @ w.T with the library GEMM's fp32 accumulator left unrounded; x, w bf16 or fp32."""
+    """out (fp32) = x @ w.T with the GEMM's fp32 accumulator left unrounded; x, w bf16 or fp32."""
     if x.dtype == torch.float32:
         return torch.mm(x, w.t(), out=out)
     if x.device.type == "cpu":
         return out.copy_(x.float() @ w.float().t())
+    if few_rows(x, w, out) and out.dtype == torch.float32 and out.shape[1] == w.shape[0]:
+        row_linear(x, w, out)
+        return out
     return torch.mm(x, w.t(), out_dtype=torch.float32, out=out)
 
 

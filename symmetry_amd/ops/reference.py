@@ -941,6 +941,18 @@ def conv_state_update(xin, state, cu_q, prev_row, save_slot, runs) -> None:
         state[sv] = torch.cat([hist, xin[s0:s1].to(state.dtype)], 0)[-keep:] if keep else hist
 
 
+def row_linear(x, w, out, relu2=False, glu=False) -> None:
+    xf = x.float()
+    if relu2:
+        xf = (torch.relu(xf) ** 2).to(x.dtype).float()
+    y = xf @ w.float().t()
+    if glu:
+        n = out.shape[1]
+        y = y.to(x.dtype).float()
+        y = y[:, :n] * torch.sigmoid(y[:, :n]) * y[:, n:]
+    out.copy_(y.to(out.dtype))
+
+
 def relu_sq(a, out) -> None:
     out.copy_((torch.relu(a.float()) ** 2).to(out.dtype))
 

@@ -1,0 +1,86 @@
+"""The few-row linear kernel (csrc/kernels/row_linear.hip) against an fp64 product of the same bf16 operands, and the rule
+that sends a call to it.
+
+Bounds: fp32 accumulation of K terms errs by at most about sqrt(K) 2^-24 of the terms' norm, far below the rounding of a
+bf16 result, 2^-8 of itself.  A squared ReLU on the way in rounds every term by 2^-8 more: together 2^-7.  Of a gated pair
+gate, up and product are rounded, 2^-8 each; the gate's error reaches silu(y) times 1 + y (1 - sigmoid(y)), at most 1.28 for
+y > 0 (for y < 0 the value is below 0.28 of the pair's scale): 3.28 x 2^-8, under 2^-6.  All relative to the largest
+result.
+"""
+import pytest
+import torch
+
+from symmetry_amd import ops
+
+# (outputs, K): one and several 8- and 16-row tiles with remainders, one chunk, an odd and an even number of chunks, four waves
+SHAPES = [(4, 8), (1000, 16), (20, 200), (2052, 256), (2048, 2048), (68, 512), (3068, 8192), (3084, 1024), (4100, 1280),
+          (5000, 14336), (24580, 2048), (24588, 1536)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K", SHAPES)
+@pytest.mark.parametrize("M", [1, 3, 16])
+def test_row_linear(gpu, M, N, K):
+    g = torch.Generator(device=gpu).manual_seed(N + K + M)
+    wide = torch.randn(M, K + 24, device=gpu, generator=g).bfloat16()
+    x = wide[:, 8:8 + K]                                   # a column range of a wider matrix
+    w = (torch.randn(2 * N, K, device=gpu, generator=g) * K ** -0.5).bfloat16()
+    y = x.double() @ w[:N].double().t()
+    for dtype in (torch.bfloat16, torch.float32):
+        room = torch.full((M, N + 8), 7.0, device=gpu, dtype=dtype)
+        out = room[:, :N]
+        assert ops.few_rows(x, w[:N], out)
+        (ops.linear if dtype == torch.bfloat16 else ops.linear_f32)(x, w[:N], out)
+        assert float((out.double() - y).abs().max()) <= (2 ** -7 if dtype == torch.bfloat16 else 2 ** -14) * float(y.abs().max())
+        assert bool((room[:, N:] == 7).all())
+    out = torch.empty(M, N, device=gpu, dtype=torch.bfloat16)
+    r = torch.relu(x.double()) ** 2 @ w[:N].double().t()
+    ops.row_linear(x, w[:N], out, relu2=True)
+    assert float((out.double() - r).abs().max()) <= 2 ** -7 * float(r.abs().max())
+    u = x.double() @ w[N:].double().t()
+    ops.row_linear(x, w, out, glu=True)
+    p = y * torch.sigmoid(y) * u
+    assert float((out.double() - p).abs().max()) <= 2 ** -6 * max(float(p.abs().max()), 1.0)
+
+
+@pytest.mark.gpu
+def test_linear_accepts_every_form(gpu):
+    """Strides, types, sizes and alignments that the kernel does not take stay with the library and give the same product."""
+    g = torch.Generator(device=gpu).manual_seed(3)
+
+    def rnd(*shape):
+        return torch.randn(*shape, device=gpu, generator=g).bfloat16()
+
+    flat = rnd(40 * 300)
+    forms = [
+        (rnd(256, 8).t(), rnd(64, 256), None), (rnd(8, 256), rnd(256, 64).t(), None), (rnd(8, 512)[:, ::2], rnd(64, 256), None),
+        (rnd(8, 260)[:, :256], rnd(64, 256), None), (flat[1:1 + 8 * 256].view(8, 256), rnd(64, 256), None),
+        (rnd(8, 256), flat[1:1 + 40 * 256].view(40, 256), None), (rnd(8, 300), rnd(64, 300), None), (rnd(8, 256), rnd(63, 256), None),
+        (rnd(1, 256).expand(8, 256), rnd(64, 256), None), (rnd(17, 256), rnd(64, 256), None), (rnd(0, 256), rnd(64, 256), None),
+        (rnd(8, 256), rnd(64, 256), torch.empty(64, 8, device=gpu, dtype=torch.bfloat16).t()),
+    ]
+    for x, w, out in forms:
+        if out is None:
+            out = torch.empty(x.shape[0], w.shape[0], device=gpu, dtype=torch.bfloat16)
+        assert not ops.few_rows(x, w, out)
+        y = x.double() @ w.double().t()
+        ops.linear(x, w, out)
+        if y.numel():
+            assert float((out.double() - y).abs().max()) <= 2 ** -7 * float(y.abs().max())
+    x, w = rnd(8, 256), rnd(64, 256)
+    assert torch.equal(ops.linear(x, w), torch.matmul(x, w.t()))                 # no out: the library allocates it
+    w.requires_grad_(True)
+    assert not ops.few_rows(x, w, torch.empty(8, 64, device=gpu, dtype=torch.bfloat16))
+    ops.linear(x, w).float().sum().backward()
+    assert w.grad is not None
+
+
+def test_row_linear_reference_cpu():
+    x, w = torch.randn(3, 32).bfloat16(), torch.randn(16, 32).bfloat16()
+    out = torch.empty(3, 8, dtype=torch.bfloat16)
+    assert not ops.few_rows(x, w, out)                                            # CPU tensors: the plain product
+    ops.row_linear(x, w, out, glu=True)
+    y = (x.float() @ w.float().t()).bfloat16().float()
+    assert torch.equal(out, (y[:, :8] * torch.sigmoid(y[:, :8]) * y[:, 8:]).bfloat16())
+    ops.row_linear(x, w[:8], out, relu2=True)
+    assert torch.equal(out, ((torch.relu(x.float()) ** 2).bfloat16().float() @ w[:8].float().t()).bfloat16())
