@@ -262,7 +262,7 @@ int64_t window_attn(const Tensor& q, const Tensor& k_cache, const Tensor& v_cach
 void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dz, const Tensor& dbias,
                 const OptTensor& rate, double tau, const OptTensor& skip, double q_scale, int64_t H, int64_t N, int64_t P,
                 int64_t hpg, Tensor& state, const OptTensor& cu_q, const Tensor& prev_row, const Tensor& save_slot,
-                int64_t runs, Tensor& out, const OptTensor& mout) {
+                int64_t runs, Tensor& out, const OptTensor& mout, const OptTensor& tiles, const OptTensor& ws) {
   const int f32 = act(v, "v", false);
   dtype(out, at::kFloat, "out");
   dtype(dbias, at::kFloat, "dbias");
@@ -321,6 +321,14 @@ void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v,
   a.save_slot = ptr<int>(save_slot);
   a.runs = (int)runs, a.T = (int)T;
   a.out = ptr<float>(out);
+  if (tiles.has_value() && ws.has_value()) {
+    dtype(*tiles, at::kInt, "tiles");
+    dtype(*ws, at::kFloat, "ws");
+    TORCH_CHECK(tiles->dim() == 2 && tiles->size(1) == 2 && tiles->size(0) <= (1 << 30), "decay_scan: tiles [n, 2]");
+    TORCH_CHECK(ws->numel() >= T * H * (32 + N), "decay_scan: ws [T, H, 32 + N]");
+    a.tiles = ptr<int>(*tiles), a.ntiles = (int)tiles->size(0);
+    a.ws = ptr<float>(*ws);
+  }
   launch_decay_scan(a, f32, cur_stream(v));
 }
 
@@ -1139,7 +1147,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
   m.def(
       "decay_scan(int mode, Tensor q, Tensor k, Tensor v, Tensor dz, Tensor dbias, Tensor? rate, float tau, Tensor? skip, "
       "float q_scale, int H, int N, int P, int hpg, Tensor(a!) state, Tensor? cu_q, Tensor prev_row, Tensor save_slot, "
-      "int runs, Tensor(b!) out, Tensor(c!)? mout) -> ()",
+      "int runs, Tensor(b!) out, Tensor(c!)? mout, Tensor? tiles=None, Tensor(d!)? ws=None) -> ()",
       &decay_scan);
   m.def("gated_group_norm(Tensor y, Tensor gate, Tensor w, float eps, int group, bool gate_first, Tensor(a!) out, "
         "bool sigmoid=False) -> ()",

@@ -1,0 +1,481 @@
+// Chunked form of the decaying recurrences of decay_scan.hip for prompt steps in bf16:
+//
+//     S_t = diag(a_t) S_(t-1) + b_t k_t v_t^T,     o_t = q_scale S_t^T q_t (+ skip_h v_t)          S [N x P] fp32
+//
+// mode 0: a per key channel, b = 1 (gated linear attention); mode 1: a per head, b the step size (state-space layers).
+// Token by token a state costs 4 N P vector operations a token on the serial path (8100 tokens in 8 prompts: 1656 us at
+// 8 heads x 128 x 256, 1345 us at 64 x 128 x 64).  With chunks of C = 32 tokens, G_i the running sum of log2 a inside the
+// chunk and S_0 the state in front of it,
+//     o_i = (q_i 2^(G_i))^T S_0 + sum_{j <= i} A_ij v_j,     A_ij = b_j sum_n q_in k_jn 2^(G_in - G_jn)
+//     S_C = 2^(G_C) S_0 + sum_j (k_j 2^(G_C - G_j) b_j) v_j^T                 (every exponent <= 0: nothing overflows)
+// is matrix products; a run's chunks are walked in order.
+//
+// Precision: q, k and v are bf16, so they are exact operands of v_mfma_f32_16x16x32_bf16, which accumulates in fp32.  An
+// fp32 operand x (the state, a scaled vector, the scores) is used as the sum of three bf16 parts, hi = bf16(x), mid =
+// bf16(x - hi), lo = bf16(x - hi - mid), which hold all of its 24 bits; of a product of two such operands the six terms
+// down to 2^-16 of the largest are taken (what is left is 2^-24 of it, an fp32 rounding).  That is 3 / 8 or 3 / 16 of the
+// matrix cycles of v_mfma_f32_16x16x4_f32.
+//
+// Work split: grid (P / 64, heads, runs), 4 waves of 16 value columns and ALL of N: the state stays in accumulator registers
+// for the whole run.  An accumulator's rows are 4 (lane / 16) + r, a B operand's contraction index is 8 (lane / 16) + j; with
+// the contraction taken in the order j < 4: 4 g + j, else 16 + 4 g + j - 4, two accumulator tiles ARE a B operand, and the A
+// operand is read in the same order (two 8-byte LDS reads).  The same holds for the values and, computed transposed, for the
+// scores.  The next chunk's rows are loaded while the current one is multiplied (two LDS stages, one barrier a chunk).
+#include "common.h"
+#include "hybrid_launchers.h"
+
+namespace {
+
+constexpr int NT = 256;
+constexpr int C = 32;             // tokens per chunk
+constexpr int LT = C + 4;         // LDS pitch of a [.][C] matrix
+constexpr float LOG2E = 1.4426950408889634f;
+
+SYM_DEV float softplus_exact(float v) { return fmaxf(v, 0.f) + log1pf(expf(-fabsf(v))); }
+SYM_DEV float exp2_neg(float v) { return __builtin_amdgcn_exp2f(fminf(v, 0.f)); }
+SYM_DEV f32x4 mfma4(float x, float y, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); }
+SYM_DEV f32x4 lds4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+
+struct Parts {
+  bf16x8 h, m, l;
+};
+
+SYM_DEV Parts split(f32x4 a, f32x4 b) {
+  Parts s;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float x = i < 4 ? a[i & 3] : b[i & 3];
+    s.h[i] = (bf16)x;
+    const float r = x - (float)s.h[i];
+    s.m[i] = (bf16)r;
+    s.l[i] = (bf16)(r - (float)s.m[i]);
+  }
+  return s;
+}
+
+// an A operand in the accumulators' contraction order: 4 elements at p, 4 at p + 16
+SYM_DEV bf16x8 pair4(const bf16* p) {
+  union {
+    bf16x8 v;
+    uint2 u[2];
+  } r;
+  r.u[0] = *reinterpret_cast<const uint2*>(p);
+  r.u[1] = *reinterpret_cast<const uint2*>(p + 16);
+  return r.v;
+}
+
+SYM_DEV int ws_cols(int N) { return C + N; }   // mode 0's scratch per (row, head): row of A | G
+
+// ---- mode 0: running sums G and scores A of every chunk, grid (64-row tiles x 2 chunks, heads) --------------------------
+// Inside the two diagonal 16 x 16 tiles the exponents of differences are taken per (i, j, channel) on the vector unit; the
+// tile below them factors at the end of the first half, 2^(G_i - G_15) 2^(G_15 - G_j), both exponents <= 0, and is a matrix
+// product.
+template <int NN>
+__global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
+  constexpr int NP = 16 * NN, LD = NP + 4;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  float* kS = reinterpret_cast<float*>(smem);  // [C][LD]
+  float* qS = kS + C * LD;                     // [C][LD]
+  float* GS = qS + C * LD;                     // [C][LD]
+  float* XS = GS + C * LD;                     // [4][C][LT] partial scores
+  const int N = a.N, h = blockIdx.y, tile = blockIdx.x >> 1, sub = blockIdx.x & 1;
+  const int seq = a.tiles[2 * tile], off = a.tiles[2 * tile + 1];
+  const int q0 = a.cu_q[seq], qlen = a.cu_q[seq + 1] - q0;
+  if (off >= qlen) return;                     // padding tile
+  const int nt = min(C, qlen - off - C * sub);
+  if (nt <= 0) return;
+  const long long r0 = q0 + off + C * sub;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bf16* q = reinterpret_cast<const bf16*>(a.q) + r0 * a.ldq + (h / a.hpg) * N;
+  const bf16* k = reinterpret_cast<const bf16*>(a.k) + r0 * a.ldk + (h / a.hpg) * N;
+  const bf16* dz = reinterpret_cast<const bf16*>(a.dz) + r0 * a.ldd + (long long)h * N;
+  const float* db = a.dbias + (long long)h * N;
+  const float scale = -LOG2E / a.tau;
+#pragma unroll 4
+  for (int i = tid; i < C * NP; i += NT) {
+    const int tt = i / NP, n = i % NP;
+    const bool in = tt < nt && n < N;
+    kS[tt * LD + n] = in ? (float)k[tt * a.ldk + n] : 0.f;
+    qS[tt * LD + n] = in ? (float)q[tt * a.ldq + n] : 0.f;
+    GS[tt * LD + n] = in ? scale * softplus_exact(-((float)dz[tt * a.ldd + n] + db[n])) : 0.f;
+  }
+  __syncthreads();
+  const int wc = ws_cols(N);
+  float* ws = a.ws + (r0 * a.H + h) * wc;
+  const long long wrow = (long long)a.H * wc;
+  if (tid < NP) {
+    float g = 0.f;
+#pragma unroll 8
+    for (int tt = 0; tt < C; ++tt) {
+      g += GS[tt * LD + tid];
+      GS[tt * LD + tid] = g;
+      if (tt < nt && tid < N) ws[tt * wrow + C + tid] = g;
+    }
+  }
+  __syncthreads();
+  const int col = lane & 15, g = lane >> 4;
+  {  // rows 16 .., columns .. 15: the waves take the channel tiles in turn
+    f32x4 d = {0.f, 0.f, 0.f, 0.f};
+    for (int t = wave; t < NN; t += 4) {
+      const int c = 16 * t + 4 * g;
+      const f32x4 mid = lds4(GS + 15 * LD + c), gi = lds4(GS + (16 + col) * LD + c), gj = lds4(GS + col * LD + c);
+      const f32x4 qi = lds4(qS + (16 + col) * LD + c), kj = lds4(kS + col * LD + c);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d = mfma4(qi[r] * exp2_neg(gi[r] - mid[r]), kj[r] * exp2_neg(mid[r] - gj[r]), d);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) XS[(wave * C + 16 + 4 * g + r) * LT + col] = d[r];
+  }
+  {  // diagonal tiles: wave (channel half, tile), a 2 x 2 block of (i, j) per lane
+    constexpr int NH = NP / 2;
+    const int half = wave >> 1, dt = wave & 1, ib = lane >> 3, jb = lane & 7;
+    const int i0 = 16 * dt + 2 * ib, j0 = 16 * dt + 2 * jb;
+    float s[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+    if (jb <= ib) {
+#pragma unroll 2
+      for (int c = NH * half; c < NH * (half + 1); c += 4) {
+        f32x4 qi[2], gi[2], kj[2], gj[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          qi[e] = lds4(qS + (i0 + e) * LD + c);
+          gi[e] = lds4(GS + (i0 + e) * LD + c);
+          kj[e] = lds4(kS + (j0 + e) * LD + c);
+          gj[e] = lds4(GS + (j0 + e) * LD + c);
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[e][f] += qi[e][r] * (kj[f][r] * exp2_neg(gi[e][r] - gj[f][r]));
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int f = 0; f < 2; ++f) XS[(half * C + i0 + e) * LT + j0 + f] = s[e][f];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < C * C / NT; ++u) {
+    const int i = (tid + NT * u) / C, j = (tid + NT * u) % C;
+    const float* x = XS + i * LT + j;
+    float v = 0.f;
+    if (j <= i) {
+      v = x[0] + x[C * LT];
+      if (i >= 16 && j < 16) v += x[2 * C * LT] + x[3 * C * LT];
+    }
+    if (i < nt) ws[i * wrow + j] = v;
+  }
+}
+
+// ---- the walk ------------------------------------------------------------------------------------------------------------
+// NB: 32-channel blocks of the state (N <= 32 NB)
+template <int MODE, int NB>
+__global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a) {
+  constexpr int NP = 32 * NB, LQ = NP + 8;              // LQ: bf16 pitch of a [C][NP] matrix
+  constexpr int PL = MODE == 0 ? 3 : 1;                 // bf16 parts of the staged vectors
+  constexpr int oK = PL * C * LQ, oT = oK + (MODE == 1 ? C * LQ : 0), oF = oT + PL * NP * LT;   // in bf16: q | k (mode 1) | k^T
+  constexpr int FS = MODE == 0 ? C * LT + NP : 3 * C;   // floats: A | 2^(G_C), or G | its low part | b
+  constexpr int STAGE = oF * 2 + FS * 4;                // bytes
+  static_assert(STAGE % 16 == 0, "stages start at multiples of 16 bytes");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int N = a.N, P = a.P, h = blockIdx.y, run = blockIdx.z;
+  const int s0 = a.cu_q[run], s1 = a.cu_q[run + 1];
+  if (s1 <= s0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
+  const int p = blockIdx.x * 64 + wave * 16 + col;
+  const bool pin = p < P;
+  const int chunks = (s1 - s0 + C - 1) / C;
+  const int pr = a.prev_row[s0], sv = a.save_slot[s1 - 1];
+  const bf16* q = reinterpret_cast<const bf16*>(a.q) + s0 * a.ldq + (h / a.hpg) * N;
+  const bf16* k = reinterpret_cast<const bf16*>(a.k) + s0 * a.ldk + (h / a.hpg) * N;
+  const bf16* v = reinterpret_cast<const bf16*>(a.v) + s0 * a.ldv + (long long)h * P + p;
+  const bf16* dt = reinterpret_cast<const bf16*>(a.dz) + s0 * a.ldd + h;          // mode 1
+  const int wc = ws_cols(N);
+  const long long wrow = (long long)a.H * wc;
+  const float* ws = MODE == 0 ? a.ws + ((long long)s0 * a.H + h) * wc : nullptr;
+  float* out = a.out + ((long long)s0 * a.H + h) * P + p;
+  const long long orow = (long long)a.H * P;
+
+  // staging: thread (token tt, 8 channels from c8), PASS tokens apart
+  constexpr int GR = NP / 8, TSTEP = NT / GR, PASS = (C + TSTEP - 1) / TSTEP;
+  const int c8 = 8 * (tid % GR), tt0 = tid / GR;
+  const bool nin = c8 < N && tt0 < C;                   // (N is a multiple of 8)
+  Pack8 rq[PASS], rk[PASS];
+  f32x4 rg[MODE == 0 ? PASS : 1][2], gl[2], ra;
+  float rdt = 0.f;
+  bf16 vn[8];
+  auto fetch = [&](int c) {
+    const int t0 = c * C, nt = min(C, s1 - s0 - t0);
+#pragma unroll
+    for (int u = 0; u < PASS; ++u) {
+      const int tt = tt0 + TSTEP * u;
+      const bool in = nin && tt < nt;
+      rq[u].u = in ? *reinterpret_cast<const uint4*>(q + (t0 + tt) * a.ldq + c8) : make_uint4(0, 0, 0, 0);
+      rk[u].u = in ? *reinterpret_cast<const uint4*>(k + (t0 + tt) * a.ldk + c8) : make_uint4(0, 0, 0, 0);
+      if constexpr (MODE == 0) {
+        const float* G = ws + (t0 + tt) * wrow + C + c8;
+        rg[u][0] = in ? lds4(G) : f32x4{0.f, 0.f, 0.f, 0.f};
+        rg[u][1] = in ? lds4(G + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    if constexpr (MODE == 0) {
+      const float* G = ws + (t0 + nt - 1) * wrow + C + c8;
+      gl[0] = nin ? lds4(G) : f32x4{0.f, 0.f, 0.f, 0.f};
+      gl[1] = nin ? lds4(G + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+      ra = tid / 8 < nt ? lds4(ws + (t0 + tid / 8) * wrow + 4 * (tid % 8)) : f32x4{0.f, 0.f, 0.f, 0.f};
+    } else if (tid < C) {
+      rdt = tid < nt ? (float)dt[(long long)(t0 + tid) * a.ldd] + a.dbias[h] : 0.f;
+    }
+  };
+  auto fetch_v = [&](int c) {
+    const int nt = min(C, s1 - s0 - c * C);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int tt = 16 * (i >> 2) + 4 * g + (i & 3);
+      vn[i] = tt < nt && pin ? v[(c * C + tt) * a.ldv] : (bf16)0.f;
+    }
+  };
+  const float rate2 = MODE == 1 ? expf(a.rate[h]) * LOG2E : 0.f;
+  auto stash = [&](int c) {
+    bf16* st = reinterpret_cast<bf16*>(smem + (c & 1) * STAGE);
+    float* fs = reinterpret_cast<float*>(st + oF);
+    const int nt = min(C, s1 - s0 - c * C);
+#pragma unroll
+    for (int u = 0; u < PASS; ++u) {
+      const int tt = tt0 + TSTEP * u;
+      if (tt >= C) break;
+      if constexpr (MODE == 1) {
+        *reinterpret_cast<uint4*>(st + tt * LQ + c8) = rq[u].u;
+        *reinterpret_cast<uint4*>(st + oK + tt * LQ + c8) = rk[u].u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) st[oT + (c8 + i) * LT + tt] = rk[u].h[i];
+      } else {
+        f32x4 x[2], y[2];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float gi = rg[u][i >> 2][i & 3];
+          x[i >> 2][i & 3] = (float)rq[u].h[i] * __builtin_amdgcn_exp2f(gi);
+          y[i >> 2][i & 3] = (float)rk[u].h[i] * exp2_neg(gl[i >> 2][i & 3] - gi);   // (past the run's end: k = 0)
+        }
+        const Parts sx = split(x[0], x[1]), sy = split(y[0], y[1]);
+        *reinterpret_cast<bf16x8*>(st + tt * LQ + c8) = sx.h;
+        *reinterpret_cast<bf16x8*>(st + (C + tt) * LQ + c8) = sx.m;
+        *reinterpret_cast<bf16x8*>(st + (2 * C + tt) * LQ + c8) = sx.l;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          st[oT + (c8 + i) * LT + tt] = sy.h[i];
+          st[oT + (NP + c8 + i) * LT + tt] = sy.m[i];
+          st[oT + (2 * NP + c8 + i) * LT + tt] = sy.l[i];
+        }
+      }
+    }
+    if constexpr (MODE == 0) {
+      *reinterpret_cast<f32x4*>(fs + (tid / 8) * LT + 4 * (tid % 8)) = ra;
+      if (tt0 == 0) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) fs[C * LT + c8 + i] = __builtin_amdgcn_exp2f(gl[i >> 2][i & 3]);
+      }
+    } else if (wave == 0) {
+      // running sum over the chunk's tokens as a pair of floats: with step sizes that forget in a few tokens the sum grows
+      // to hundreds, and the differences of neighbours, which are what counts, would keep few of its digits
+      const float b = tid < nt ? softplus_exact(rdt) : 0.f;
+      double s = tid < nt ? -(double)rate2 * b : 0.0;
+#pragma unroll
+      for (int o = 1; o < C; o <<= 1) {
+        const double up = __shfl_up(s, o, 64);
+        if (tid >= o) s += up;
+      }
+      if (tid < C) {
+        fs[tid] = (float)s;
+        fs[C + tid] = (float)(s - (double)(float)s);
+        fs[2 * C + tid] = b;
+      }
+    }
+  };
+
+  f32x4 S[2 * NB];
+  const bool old = pr <= -2 && pin;
+  const float* st0 = a.state + (old ? (long long)(-(pr + 2)) * a.state_stride + (long long)h * N * P + p : 0);
+#pragma unroll
+  for (int t = 0; t < 2 * NB; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = 16 * t + 4 * g + r;
+      S[t][r] = old && n < N ? st0[(long long)n * P] : 0.f;
+    }
+  const float skip = a.skip ? a.skip[h] : 0.f;
+  fetch(0);
+  fetch_v(0);
+  stash(0);
+  __syncthreads();
+  for (int c = 0; c < chunks; ++c) {
+    const int nt = min(C, s1 - s0 - c * C);
+    Pack8 V;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) V.h[i] = vn[i];
+    const bool more = c + 1 < chunks;
+    if (more) {
+      fetch(c + 1);
+      fetch_v(c + 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);                  // the next chunk's loads in flight ahead of this one's products
+    const bf16* st = reinterpret_cast<const bf16*>(smem + (c & 1) * STAGE);
+    const float* fs = reinterpret_cast<const float*>(st + oF);
+    const bf16* Qr = st + col * LQ + 4 * g;
+    f32x4 O[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      const Parts s = split(S[2 * t], S[2 * t + 1]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const bf16x8 qh = pair4(Qr + 16 * i * LQ + 32 * t);
+        O[i] = mfma16(qh, s.l, O[i]);
+        if constexpr (MODE == 0) {
+          const bf16x8 qm = pair4(Qr + (C + 16 * i) * LQ + 32 * t), ql = pair4(Qr + (2 * C + 16 * i) * LQ + 32 * t);
+          O[i] = mfma16(ql, s.h, O[i]);
+          O[i] = mfma16(qm, s.m, O[i]);
+          O[i] = mfma16(qm, s.h, O[i]);
+        }
+        O[i] = mfma16(qh, s.m, O[i]);
+        O[i] = mfma16(qh, s.h, O[i]);
+      }
+    }
+    f32x4 A[2][2];                                      // scores of row tile i, columns 4 g + r and 16 + 4 g + r
+    f32x4 gj[2], lj[2], bj[2];
+    if constexpr (MODE == 0) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) A[i][j] = lds4(fs + (16 * i + col) * LT + 16 * j + 4 * g);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        gj[j] = lds4(fs + 16 * j + 4 * g);
+        lj[j] = lds4(fs + C + 16 * j + 4 * g);
+        bj[j] = lds4(fs + 2 * C + 16 * j + 4 * g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) O[j][r] *= __builtin_amdgcn_exp2f(gj[j][r]);      // (rows 4 g + r of O too)
+      }
+      const bf16* Kn = st + oK + col * LQ + 8 * g;
+      const bf16* Qn = st + col * LQ + 8 * g;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float gi = fs[16 * i + col], li = fs[C + 16 * i + col];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          f32x4 d = {0.f, 0.f, 0.f, 0.f};
+          if (j <= i) {
+#pragma unroll
+            for (int t = 0; t < NB; ++t)
+              d = mfma16(*reinterpret_cast<const bf16x8*>(Kn + 16 * j * LQ + 32 * t),
+                         *reinterpret_cast<const bf16x8*>(Qn + 16 * i * LQ + 32 * t), d);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float w = exp2_neg((gi - gj[j][r]) + (li - lj[j][r])) * bj[j][r];
+              d[r] = j < i || 4 * g + r <= col ? d[r] * w : 0.f;
+            }
+          }
+          A[i][j] = d;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const Parts s = split(A[i][0], A[i][1]);
+      O[i] = mfma16(s.l, V.v, O[i]);
+      O[i] = mfma16(s.m, V.v, O[i]);
+      O[i] = mfma16(s.h, V.v, O[i]);
+    }
+    if (pin) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int tt = 16 * i + 4 * g + r;
+          if (tt < nt) out[(c * C + tt) * orow] = a.q_scale * O[i][r] + skip * (float)V.h[4 * i + r];
+        }
+    }
+    const bf16* Kt = st + oT + col * LT + 4 * g;
+    if constexpr (MODE == 0) {
+#pragma unroll
+      for (int t = 0; t < 2 * NB; ++t) {
+        S[t] *= lds4(fs + C * LT + 16 * t + 4 * g);
+        S[t] = mfma16(pair4(Kt + (2 * NP + 16 * t) * LT), V.v, S[t]);
+        S[t] = mfma16(pair4(Kt + (NP + 16 * t) * LT), V.v, S[t]);
+        S[t] = mfma16(pair4(Kt + 16 * t * LT), V.v, S[t]);
+      }
+    } else {
+      const float gc = fs[C - 1], lc = fs[2 * C - 1], d = __builtin_amdgcn_exp2f(gc);     // (G stands still past the run's end)
+      f32x4 w[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) w[j][r] = exp2_neg((gc - gj[j][r]) + (lc - lj[j][r])) * bj[j][r] * (float)V.h[4 * j + r];
+      const Parts s = split(w[0], w[1]);
+#pragma unroll
+      for (int t = 0; t < 2 * NB; ++t) {
+        S[t] *= d;
+        const bf16x8 kt = pair4(Kt + 16 * t * LT);
+        S[t] = mfma16(kt, s.l, S[t]);
+        S[t] = mfma16(kt, s.m, S[t]);
+        S[t] = mfma16(kt, s.h, S[t]);
+      }
+    }
+    if (more) stash(c + 1);
+    __syncthreads();                                    // chunk c + 1 is staged, chunk c has been read
+  }
+  if (sv >= 0 && pin) {
+    float* so = a.state + (long long)sv * a.state_stride + (long long)h * N * P + p;
+#pragma unroll
+    for (int t = 0; t < 2 * NB; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n = 16 * t + 4 * g + r;
+        if (n < N) so[(long long)n * P] = S[t][r];
+      }
+  }
+}
+
+template <int MODE, int NB>
+void launch_chunks(const DecayScanArgs& a, hipStream_t s) {
+  constexpr int NP = 32 * NB, LQ = NP + 8, PL = MODE == 0 ? 3 : 1;
+  constexpr int elems = PL * C * LQ + (MODE == 1 ? C * LQ : 0) + PL * NP * LT;
+  constexpr int lds = 2 * (elems * 2 + (MODE == 0 ? C * LT + NP : 3 * C) * 4);
+  constexpr int prep = (3 * C * (NP + 4) + 4 * C * LT) * 4;
+  static const bool raised = [] {
+    const auto raise = [](const void* f, int bytes) {
+      if (bytes > 64 * 1024) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    };
+    raise(reinterpret_cast<const void*>(&decay_chunk_scan_kernel<MODE, NB>), lds);
+    if (MODE == 0) raise(reinterpret_cast<const void*>(&decay_chunk_prep_kernel<2 * NB>), prep);
+    return true;
+  }();
+  (void)raised;
+  if constexpr (MODE == 0) decay_chunk_prep_kernel<2 * NB><<<dim3(2 * a.ntiles, a.H), NT, prep, s>>>(a);
+  decay_chunk_scan_kernel<MODE, NB><<<dim3((a.P + 63) / 64, a.H, a.runs), NT, lds, s>>>(a);
+}
+
+template <int MODE>
+void launch_mode(const DecayScanArgs& a, hipStream_t s) {
+  if (a.N <= 32) launch_chunks<MODE, 1>(a, s);
+  else if (a.N <= 64) launch_chunks<MODE, 2>(a, s);
+  else launch_chunks<MODE, 4>(a, s);
+}
+
+}  // namespace
+
+// Is the call one the chunked form takes?  bf16 prompt steps of at least 8 tokens a run (below, a chunk's fixed cost is more
+// than the walk), up to 128 key channels, 16-byte aligned rows; mode 0 needs the 64-row tiles and the scratch.
+bool decay_chunk_takes(const DecayScanArgs& a) {
+  auto aligned = [](const void* p, long long ld) { return (uintptr_t)p % 16 == 0 && ld % 8 == 0; };
+  if (a.mode > 1 || !a.cu_q || a.T < 8LL * a.runs || a.N % 8 || a.N > 128) return false;
+  if (!aligned(a.q, a.ldq) || !aligned(a.k, a.ldk)) return false;
+  return a.mode == 1 || (a.tiles && a.ntiles > 0 && a.ws && (uintptr_t)a.ws % 16 == 0);
+}
+
+void launch_decay_chunks(const DecayScanArgs& a, hipStream_t s) {
+  if (a.mode == 0) launch_mode<0>(a, s);
+  else launch_mode<1>(a, s);
+}

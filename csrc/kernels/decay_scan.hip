@@ -12,8 +12,8 @@
 //                        that each column's owner reads and writes its own copy (no workgroup reads what another writes);
 //                        it is chained token by token by the first wave while a batch is staged.
 //
-// The state walks token by token in fp32, in the same order however a prompt is cut into steps, so a position's
-// output does not depend on the cut.  A run of rows (one sequence's tokens of this step) starts from its state slot
+// Prompt steps in bf16 take the chunked form (decay_chunk.hip) in modes 0 and 1.  Here the state walks token by token in
+// fp32, in the same order however a prompt is cut into steps, so a position's output does not depend on the cut.  A run of rows (one sequence's tokens of this step) starts from its state slot
 // (or zero at position 0) and ends in it.
 //
 // Work split: grid (P / 64 column tiles, heads, runs), 256 threads.  Wave w owns 16 value columns; inside a wave the
@@ -258,7 +258,8 @@ void launch_decay_scan(const DecayScanArgs& a, int f32, hipStream_t s) {
     else if (a.mode == 1) launch_mode<float, 1>(a, s);
     else launch_mode<float, 2>(a, s);
   } else {
-    if (a.mode == 0) launch_mode<bf16, 0>(a, s);
+    if (decay_chunk_takes(a)) launch_decay_chunks(a, s);
+    else if (a.mode == 0) launch_mode<bf16, 0>(a, s);
     else if (a.mode == 1) launch_mode<bf16, 1>(a, s);
     else launch_mode<bf16, 2>(a, s);
   }

@@ -260,7 +260,13 @@ struct DecayScanArgs {
   const int* save_slot;
   int runs, T;
   float* out;           // [T][H][P]
+  // chunked form (decay_chunk.hip), mode 0: 64-row tiles (run, first row), and fp32 scratch [T][H][32 + N]
+  const int* tiles;
+  int ntiles;
+  float* ws;
 };
+bool decay_chunk_takes(const DecayScanArgs& a);
+void launch_decay_chunks(const DecayScanArgs& a, hipStream_t s);
 void launch_decay_scan(const DecayScanArgs& a, int f32, hipStream_t s);
 
 // ---- delta_rule.hip ------------------------------------------------------------------------------------

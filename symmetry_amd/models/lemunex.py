@@ -277,9 +277,12 @@ class LemunexLM:
         # gated linear attention
         dz = self._linear("gla.dz", self._cols(z, P, "right.a1"), P["right.a2"])
         y = self._buf("rec.y", (T, g.heads * g.vdim), torch.float32)
+        tiles = ws = None
+        if prefill and self.dtype == torch.bfloat16 and self.device.type != "cpu":   # (the 32-bit model walks token by token)
+            tiles, ws = b.tiles, self._buf("gla.ws", (T, g.heads, ops.decay_ws_cols(g.dim)), torch.float32)
         ops.decay_scan(ops.DECAY_CHANNEL_GATE, self._cols(z, P, "right.q"), self._cols(z, P, "right.k"),
                        self._cols(z, P, "right.v"), dz, P["right.a2.b"], g.tau, None, g.dim ** -0.5, g.heads, g.dim,
-                       g.vdim, 1, cache.rec[i], b.cu_q if prefill else None, b.prev_row, b.save_slot, runs, y)
+                       g.vdim, 1, cache.rec[i], b.cu_q if prefill else None, b.prev_row, b.save_slot, runs, y, tiles=tiles, ws=ws)
         gy = self._buf("rec.gy", (T, g.heads * g.vdim))
         ops.gated_group_norm(y, self._cols(z, P, "right.g"), P["right.norm"], self.cfg.norm_eps, g.vdim, False, gy)
         right = self._linear("gla.out", gy, P["right.o"])

@@ -857,7 +857,7 @@ DECAY_CHANNEL_GATE, DECAY_STEP_SIZE, DECAY_LOG_GATES = 0, 1, 2
 
 
 def decay_scan(mode, q, k, v, dz, dbias, dparam, skip, q_scale, H, N, P, hpg, state, cu_q, prev_row, save_slot, runs,
-               out, mout=None):
+               out, mout=None, tiles=None, ws=None):
     """Linear recurrence with decaying state, per head h over every run of rows (cu_q[i] .. cu_q[i + 1]; cu_q None:
     every row its own run): S <- diag(a_t) S + b_t k_t v_t^T (S [N, P] fp32), out_t = S^T (q_scale q_t) (+ skip_h v_t).
     DECAY_CHANNEL_GATE: a = sigmoid(dz + dbias) ** (1 / dparam) per key channel (dz [T, H N], dparam a number), b = 1;
@@ -868,14 +868,21 @@ def decay_scan(mode, q, k, v, dz, dbias, dparam, skip, q_scale, H, N, P, hpg, st
     [T, H, P + 1] carry one more column, fed by v = 1 (the normaliser n_t and n_t . q_t), and the state one more row,
     which carries m (the same value in every column).
     q / k [T, (H / hpg) N]: head h reads group h // hpg.  A run starts from state[slot] if prev_row[first] <= -2
-    (slot = -(v + 2)), else from zero; it ends in state[save_slot[last]] (>= 0).  out fp32 [T, H, P]."""
+    (slot = -(v + 2)), else from zero; it ends in state[save_slot[last]] (>= 0).  out fp32 [T, H, P].
+    Prompt steps in bf16 walk their runs in chunks (csrc/kernels/decay_chunk.hip); the channel gate needs ``tiles`` (the
+    step's 64-row tiles) and ``ws`` (fp32, decay_ws_cols per row and head) for that, else it goes token by token."""
     if _gpu(out):
         dp = dparam if torch.is_tensor(dparam) else None
         return _hyb().decay_scan(int(mode), q, k, v, dz, dbias, dp, 0.0 if dp is not None else float(dparam), skip,
                                  float(q_scale), int(H), int(N), int(P), int(hpg), state, cu_q, prev_row, save_slot,
-                                 int(runs), out, mout)
+                                 int(runs), out, mout, tiles, ws)
     return reference.decay_scan(mode, q, k, v, dz, dbias, dparam, skip, q_scale, H, N, P, hpg, state, cu_q, prev_row,
                                 save_slot, runs, out, mout)
+
+
+def decay_ws_cols(N: int) -> int:
+    """Columns of decay_scan's chunk scratch per row and head: a score row and the channels' running decays."""
+    return 32 + N
 
 
 def memory_norm_gate(y, m, gate, w, eps, out):

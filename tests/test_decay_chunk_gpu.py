@@ -1,0 +1,106 @@
+"""The chunked recurrence (csrc/kernels/decay_chunk.hip) against the recurrence in 64 bits, and beside the token-by-token
+kernel (the same values as fp32 operands take that one).
+
+Bound: every term of an output passes a handful of fp32 roundings (2^-24 each) and at most a run's chunks of decays and sums,
+whose errors add up like a random walk: sqrt(200) 2^-24 = 8e-7 of the result's 2-norm at the longest run here; 2e-6 is asked
+for.  The largest single error is asked to stay under 4e-6 of the largest output."""
+import pytest
+import torch
+
+from symmetry_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _walk(q, k, v, a, b, S0, lens, skip):
+    o, ends, r = torch.zeros_like(v), [], 0
+    for i, n in enumerate(lens):
+        S = S0[i].clone()
+        for t in range(r, r + n):
+            S = a[t][:, :, None] * S + (b[t][:, None] * k[t])[:, :, None] * v[t][:, None, :]
+            o[t] = (S * q[t][:, :, None]).sum(1) + skip[:, None] * v[t]
+        ends.append(S)
+        r += n
+    return o, torch.stack(ends)
+
+
+@pytest.mark.parametrize("mode", [ops.DECAY_CHANNEL_GATE, ops.DECAY_STEP_SIZE])
+@pytest.mark.parametrize("shift", [0.0, -40.0, 15.0])       # decays of a few hundred tokens, of one, of none
+@pytest.mark.parametrize("H,N,P,G,lens", [
+    (3, 128, 80, 3, [33, 64, 5, 97, 1, 32]), (4, 64, 64, 2, [100, 31]), (2, 24, 16, 1, [40, 41]), (2, 8, 70, 2, [8]),
+    (2, 72, 70, 2, [200]), (2, 32, 130, 1, [63, 65])])
+def test_decay_chunks(gpu, mode, shift, H, N, P, G, lens):
+    g = torch.Generator(device=gpu).manual_seed(H * N + P)
+    T, R = sum(lens), len(lens)
+
+    def rnd(*s):
+        return torch.randn(*s, device=gpu, generator=g)
+
+    z = rnd(T, 2 * G * N + H * P).bfloat16()                  # q | k | v as column ranges of one projection
+    q, k, v = z[:, :G * N], z[:, G * N:2 * G * N], z[:, 2 * G * N:]
+    cols = H * N if mode == ops.DECAY_CHANNEL_GATE else H
+    dz, db = (rnd(T, cols) + shift).bfloat16(), rnd(cols) + (3.0 if mode == ops.DECAY_CHANNEL_GATE else -2.0)
+    par = 16.0 if mode == ops.DECAY_CHANNEL_GATE else torch.log(0.05 + 0.5 * torch.rand(H, device=gpu, generator=g))
+    skip, scale = rnd(H), 0.37
+    state = rnd(2 * R, H, N, P)
+    S0 = state[:R].double().clone()
+    prev, save = [], []
+    for i, n in enumerate(lens):                              # every third run is a sequence's first
+        prev += [-1 if i % 3 == 2 else -(i + 2)] + [0] * (n - 1)
+        save += [-1] * (n - 1) + [R + i]
+        if i % 3 == 2:
+            S0[i] = 0
+    i32 = dict(device=gpu, dtype=torch.int32)
+    prev, save = torch.tensor(prev, **i32), torch.tensor(save, **i32)
+    cu = torch.tensor([sum(lens[:i]) for i in range(R + 1)], **i32)
+    tiles = torch.tensor([(i, r) for i, n in enumerate(lens) for r in range(0, n, 64)] + [(0, 1 << 24)], **i32)
+    ws = torch.full((T, H, ops.decay_ws_cols(N)), float("nan"), device=gpu)
+    head = torch.arange(H, device=gpu) // (H // G)
+    y = dz.double().view(T, H, -1) + db.double().view(H, -1)
+    if mode == ops.DECAY_CHANNEL_GATE:
+        a, b = torch.exp(torch.nn.functional.logsigmoid(y) / par), torch.ones(T, H, device=gpu, dtype=torch.float64)
+    else:
+        b = torch.nn.functional.softplus(y[..., 0], threshold=1e9)
+        a = torch.exp(-torch.exp(par.double()) * b)[:, :, None].expand(T, H, N)
+    want, ends = _walk(q.double().view(T, G, N)[:, head] * scale, k.double().view(T, G, N)[:, head], v.double().reshape(T, H, P),
+                       a, b, S0, lens, skip.double())
+    out = torch.empty(T, H * P, device=gpu)
+    for chunked in (True, False):
+        x = [t if chunked else t.float() for t in (q, k, v, dz)]
+        ops.decay_scan(mode, *x, db, par, skip, scale, H, N, P, H // G, state, cu, prev, save, R, out, tiles=tiles, ws=ws)
+        d = out.double() - want.reshape(T, -1)
+        assert float(d.norm() / want.norm()) <= 2e-6, chunked
+        assert float(d.abs().max() / want.abs().max()) <= 4e-6, chunked
+        assert float((state[R:].double() - ends).norm() / ends.norm()) <= 2e-6, chunked
+
+
+@pytest.mark.parametrize("form", ["odd channels", "odd stride", "unaligned", "no scratch", "short runs", "wide"])
+def test_forms_that_walk_token_by_token(gpu, form):
+    """What the chunked form does not take gives the same recurrence (channel gate, one run from zero)."""
+    g = torch.Generator(device=gpu).manual_seed(11)
+    H, P, T = 2, 48, 40
+    N = {"odd channels": 12, "wide": 136}.get(form, 16)
+    lens = [4] * 10 if form == "short runs" else [T]
+
+    def rnd(*s):
+        return torch.randn(*s, device=gpu, generator=g)
+
+    pad = 1 if form in ("odd stride", "unaligned") else 0
+    z = rnd(T, 2 * H * N + (3 if form == "odd stride" else 8)).bfloat16()
+    q, k = z[:, pad:pad + H * N], z[:, pad + H * N:pad + 2 * H * N]
+    v, dz, db = rnd(T, H * P).bfloat16(), rnd(T, H * N).bfloat16(), rnd(H * N) + 2
+    state = torch.zeros(len(lens), H, N, P, device=gpu)
+    i32 = dict(device=gpu, dtype=torch.int32)
+    cu = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], **i32)
+    prev = torch.tensor([-1 if r in cu.tolist() else r - 1 for r in range(T)], **i32)
+    save = torch.full((T,), -1, **i32)
+    tiles = torch.tensor([(i, 0) for i in range(len(lens))], **i32)
+    ws = None if form == "no scratch" else torch.empty(T, H, ops.decay_ws_cols(N), device=gpu)
+    out = torch.empty(T, H * P, device=gpu)
+    ops.decay_scan(ops.DECAY_CHANNEL_GATE, q, k, v, dz, db, 16.0, None, 0.25, H, N, P, 1, state, cu, prev, save, len(lens), out,
+                   tiles=tiles, ws=ws)
+    a = torch.exp(torch.nn.functional.logsigmoid((dz.double() + db.double()).view(T, H, N)) / 16)
+    want, _ = _walk(q.double().reshape(T, H, N) * 0.25, k.double().reshape(T, H, N), v.double().view(T, H, P), a,
+                    torch.ones(T, H, device=gpu).double(), torch.zeros(len(lens), H, N, P, device=gpu).double(), lens,
+                    torch.zeros(H, device=gpu).double())
+    assert float((out.double() - want.reshape(T, -1)).norm() / want.norm()) <= 2e-6
