@@ -697,15 +697,18 @@ void route_topk(const Tensor& x, const Tensor& Wr, const OptTensor& bias, int64_
 }
 
 int64_t expert_linear(const Tensor& x, const OptTensor& src, const Tensor& W, const Tensor& offsets, Tensor& y, bool relu2,
-                      int64_t impl) {
+                      int64_t impl, bool glu) {
   const int f32 = act(x, "x");
   same_act(W, f32, "W");
-  same_act(y, f32, "y");
+  const int y32 = act(y, "y");
+  TORCH_CHECK(y32 || !f32, "y: activation dtypes differ");
+  TORCH_CHECK(!(relu2 && glu) && (y32 == f32 || !(relu2 || glu)), "expert_linear: one of relu2, glu, fp32 output");
   dtype(offsets, at::kInt, "offsets");
   TORCH_CHECK(x.dim() == 2 && W.dim() == 3 && y.dim() == 2, "expert_linear: x [T, K], W [E, N, K], y [R, N]");
   ExpertArgs a{};
   const int64_t R = y.size(0), E = W.size(0);
-  TORCH_CHECK(W.size(2) == x.size(1) && y.size(1) == W.size(1) && offsets.numel() >= E + 1 && (R + 63) / 64 + E <= 65535,
+  TORCH_CHECK(W.size(2) == x.size(1) && (glu ? 2 : 1) * y.size(1) == W.size(1) && offsets.numel() >= E + 1 &&
+                  (R + 63) / 64 + E <= 65535,
               "expert_linear: shapes");
   if (src.has_value()) {
     dtype(*src, at::kInt, "src");
@@ -715,7 +718,10 @@ int64_t expert_linear(const Tensor& x, const OptTensor& src, const Tensor& W, co
     TORCH_CHECK(x.size(0) >= R, "expert_linear: fewer rows of x than places");
   }
   a.x = x.data_ptr(), a.W = W.data_ptr(), a.offsets = ptr<int>(offsets), a.y = y.data_ptr();
-  a.R = (int)R, a.E = (int)E, a.N = (int)W.size(1), a.K = (int)W.size(2), a.relu2 = relu2;
+  a.R = (int)R, a.E = (int)E, a.N = (int)y.size(1), a.K = (int)W.size(2), a.relu2 = relu2;
+  a.glu = glu, a.f32_out = y32 && !f32;
+  TORCH_CHECK(!(a.glu || a.f32_out) || (expert_linear_mfma(a, f32) && E <= 65535 && (impl < 0 || (impl == 1) || (impl > 1 && a.K % 64 == 0))),
+              "expert_linear: glu and fp32 output take bf16 rows of a multiple of 32, 16-byte aligned");
   return launch_expert_linear(a, f32, (int)impl, cur_stream(x));
 }
 
@@ -1198,7 +1204,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
       "Tensor(e!) src) -> ()",
       &route_topk);
   m.def(
-      "expert_linear(Tensor x, Tensor? src, Tensor W, Tensor offsets, Tensor(a!) y, bool relu2, int impl=-1) -> int",
+      "expert_linear(Tensor x, Tensor? src, Tensor W, Tensor offsets, Tensor(a!) y, bool relu2, int impl=-1, bool glu=False) -> int",
       &expert_linear);
   m.def(
       "residual_routed_norm(Tensor(a!) x, Tensor? a, Tensor? y, Tensor? dst, Tensor? w, int k, Tensor? bias, Tensor? wn, "

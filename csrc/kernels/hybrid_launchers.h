@@ -189,7 +189,11 @@ struct ExpertArgs {
   const int* offsets;
   void* y;
   int R, E, N, K, relu2;
+  int glu;        // W [E][2 N][K] holds [gate | up] rows, y = silu(gate) * up
+  int f32_out;    // y fp32 (neither relu2 nor glu)
 };
+// the MFMA forms take it (the only ones with glu and f32_out)
+bool expert_linear_mfma(const ExpertArgs& a, int f32);
 // impl -1: by shape; 0 all shapes, 1 weight stream, 2 / 3 tiles.  Returns the form used.
 int launch_expert_linear(const ExpertArgs& a, int f32, int impl, hipStream_t s);
 

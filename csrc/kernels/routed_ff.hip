@@ -199,104 +199,160 @@ SYM_DEV float relu2f(float v) {
   return v * v;
 }
 
-// Few rows per expert: grid (ceil(N / 16), E), NW waves.  A workgroup owns 16 weight rows of one expert; its waves take the
-// width's 64-element steps in turn (weights streamed once, straight into registers), multiply them with up to 16 MT rows of
-// the segment per pass, and their sums meet in LDS.  K % 32 == 0.
-template <int MT, int NW>
+enum { EPI_BF16 = 0, EPI_RELU2 = 1, EPI_GLU = 2, EPI_F32 = 3 };   // EPI_GLU: W's rows are [gate | up], y = silu(gate) * up
+
+// Few rows per expert: grid (ceil(N / 16), E), NW waves.  A workgroup owns 16 outputs of one expert (EPI_GLU: their gate and up
+// rows, so the pair meets in LDS); its waves take the width's 64-element steps in turn (weights streamed once, straight into
+// registers), multiply them with up to 16 MT rows of the segment per pass, and their sums meet in LDS.  K % 32 == 0.
+template <int MT, int NW, int U, int EPI>
 __global__ __launch_bounds__(64 * NW) void expert_stream_kernel(ExpertArgs a) {
-  __shared__ float part[NW][MT * 256];
+  constexpr int G = EPI == EPI_GLU ? 2 : 1;       // weight rows of an output
+  __shared__ float part[NW][G * MT * 256];
   const int e = blockIdx.y, n0 = 16 * blockIdx.x;
   const int s0 = a.offsets[e], s1 = min(a.offsets[e + 1], a.R);
   if (s0 >= s1) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, hq = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, hq = lane >> 4;
   const int K = a.K, N = a.N;
-  const bf16* w = reinterpret_cast<const bf16*>(a.W) + ((long long)e * N + min(n0 + j, N - 1)) * K + 8 * hq;
+  const bf16* w[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+    w[g] = reinterpret_cast<const bf16*>(a.W) + ((long long)(G * e + g) * N + min(n0 + j, N - 1)) * K + 8 * hq;
   for (int r0 = s0; r0 < s1; r0 += 16 * MT) {
-    const bf16* x[MT];
-    f32x4 acc[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const int r = min(r0 + 16 * m + j, s1 - 1);
-      x[m] = reinterpret_cast<const bf16*>(a.x) + (long long)(a.src ? a.src[r] : r) * K + 8 * hq;
-      acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    // 64 elements of every weight row per step: whole 128-byte lines
-    constexpr int U = MT == 1 ? 4 : 2;
-    int c = 64 * wave;
-    for (; c + 64 * NW * (U - 1) + 64 <= K; c += 64 * NW * U) {
-      Pack8 wf[U][2];
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int v = 0; v < 2; ++v) wf[u][v].w = ld_nt16(w + c + 64 * NW * u + 32 * v);
+    // 64 elements of every weight row per step: whole 128-byte lines.  U steps are in flight, the first ones before the rows
+    // are looked up.
+    Pack8 wf[U][2][G];
+    auto load = [&](int c) {
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int v = 0; v < 2; ++v)
 #pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            Pack8 xf;
-            xf.u = *reinterpret_cast<const uint4*>(x[m] + c + 64 * NW * u + 32 * v);
-            acc[m] = mfma16(wf[u][v].v, xf.v, acc[m]);     // lane: row j, outputs n0 + 4 hq + 0..3
-          }
+          for (int g = 0; g < G; ++g) wf[u][v][g].w = ld_nt16(w[g] + c + 64 * NW * u + 32 * v);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    int c = 64 * wave;
+    bool more = c + 64 * NW * (U - 1) + 64 <= K;
+    if (more) load(c);
+    const bf16* x[MT];
+    f32x4 acc[G][MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const int r = min(r0 + 16 * m + j, s1 - 1);
+      x[m] = reinterpret_cast<const bf16*>(a.x) + (long long)(a.src ? a.src[r] : r) * K + 8 * hq;
+#pragma unroll
+      for (int g = 0; g < G; ++g) acc[g][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    while (more) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        Pack8 xf[U][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int v = 0; v < 2; ++v) xf[u][v].u = *reinterpret_cast<const uint4*>(x[m] + c + 64 * NW * u + 32 * v);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+              acc[g][m] = mfma16(wf[u][v][g].v, xf[u][v].v, acc[g][m]);     // lane: row j, outputs n0 + 4 hq + 0..3
+      }
+      c += 64 * NW * U;
+      more = c + 64 * NW * (U - 1) + 64 <= K;
+      if (more) load(c);
     }
     for (; c < K; c += 64 * NW)
 #pragma unroll
       for (int v = 0; v < 2; ++v) {
         if (c + 32 * v >= K) break;
-        Pack8 wf;
-        wf.w = ld_nt16(w + c + 32 * v);
+        Pack8 wt[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) wt[g].w = ld_nt16(w[g] + c + 32 * v);
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
           Pack8 xf;
           xf.u = *reinterpret_cast<const uint4*>(x[m] + c + 32 * v);
-          acc[m] = mfma16(wf.v, xf.v, acc[m]);
+#pragma unroll
+          for (int g = 0; g < G; ++g) acc[g][m] = mfma16(wt[g].v, xf.v, acc[g][m]);
         }
       }
 #pragma unroll
-    for (int m = 0; m < MT; ++m) *reinterpret_cast<f32x4*>(&part[wave][m * 256 + j * 16 + 4 * hq]) = acc[m];
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) *reinterpret_cast<f32x4*>(&part[wave][(g * MT + m) * 256 + j * 16 + 4 * hq]) = acc[g][m];
     __syncthreads();
     for (int i = threadIdx.x; i < MT * 256; i += 64 * NW) {
-      float s = part[0][i];
+      float s = part[0][i], t = G == 2 ? part[0][MT * 256 + i] : 0.f;
 #pragma unroll
-      for (int v = 1; v < NW; ++v) s += part[v][i];
+      for (int v = 1; v < NW; ++v) {
+        s += part[v][i];
+        if constexpr (G == 2) t += part[v][MT * 256 + i];
+      }
       const int r = r0 + (i >> 4), n = n0 + (i & 15);
-      if (r < s1 && n < N) reinterpret_cast<bf16*>(a.y)[(long long)r * N + n] = (bf16)(a.relu2 ? relu2f(s) : s);
+      if (r < s1 && n < N) {
+        const long long at = (long long)r * N + n;
+        if constexpr (EPI == EPI_F32) reinterpret_cast<float*>(a.y)[at] = s;
+        else reinterpret_cast<bf16*>(a.y)[at] = (bf16)(EPI == EPI_GLU ? silu(s) * t : EPI == EPI_RELU2 ? relu2f(s) : s);
+      }
     }
     __syncthreads();
   }
 }
 
-// Prompt steps: BM x BN output tiles, waves in WR rows x WC columns, K in steps of 64 through two LDS stages filled by direct
-// global -> LDS loads.  LDS rows are 128 B with the 16-byte chunk c stored at c ^ ((row >> 1) & 7) (swizzled on the load's
-// source), so fragment reads do not conflict.  The tile list is walked on the device: a slot past the last tile exits before
-// any barrier.  K % 64 == 0.
+template <int MT, int NW, int U>
+void launch_stream(const ExpertArgs& a, hipStream_t s) {
+  dim3 grid((a.N + 15) / 16, a.E);
+  if (a.glu) expert_stream_kernel<MT, NW, U, EPI_GLU><<<grid, 64 * NW, 0, s>>>(a);
+  else if (a.relu2) expert_stream_kernel<MT, NW, U, EPI_RELU2><<<grid, 64 * NW, 0, s>>>(a);
+  else if (a.f32_out) expert_stream_kernel<MT, NW, U, EPI_F32><<<grid, 64 * NW, 0, s>>>(a);
+  else expert_stream_kernel<MT, NW, U, EPI_BF16><<<grid, 64 * NW, 0, s>>>(a);
+}
+
+// Prompt steps: tiles of BM rows x BN weight rows, waves in WR rows x WC columns, K in steps of 64 through two LDS stages filled by
+// direct global -> LDS loads.  LDS rows are 128 B with the 16-byte chunk c stored at c ^ ((row >> 1) & 7) (swizzled on the
+// load's source), so fragment reads do not conflict.  K % 64 == 0.
+// EPI_GLU: half of a wave's weight rows are gate rows and half the same up
+// rows, so a pair meets in registers.
+// The tile list is counted on the device; a workgroup without a tile exits before any barrier.  Tiles are dealt to the 8 XCDs
+// in contiguous runs (workgroup i runs on XCD i % 8) and walk GN column tiles of every row tile of an expert before the next
+// GN, so an expert's weights and a tile row's activations are shared in one L2 (16384 rows, 8 experts of 2 x 14336 x 4096:
+// 0.78 -> 1.13 PFLOP/s).
+constexpr int GN = 8;
+
 SYM_DEV int chunk_swz(int row) { return (row >> 1) & 7; }
 
-template <int BM, int BN, int WR, int WC>
+template <int BM, int BN, int WR, int WC, int EPI>
 __global__ __launch_bounds__(64 * WR * WC) void expert_tile_kernel(ExpertArgs a) {
-  constexpr int NWV = WR * WC, MS = BM / WR / 16, NS = BN / WC / 16;   // 16-row subtiles of a wave
+  constexpr int NWV = WR * WC, WN = BN / WC, MS = BM / WR / 16, NS = WN / 16;   // 16-row subtiles of a wave
   constexpr int AB = BM * 128, BB = BN * 128, STAGE = AB + BB;         // bytes of a stage
   constexpr int AL = BM / 8 / NWV, BL = BN / 8 / NWV;                  // direct loads (8 rows each) per wave and stage
+  constexpr int OUT = EPI == EPI_GLU ? BN / 2 : BN, WO = OUT / WC, NO = WO / 16;   // outputs of a tile, of a wave; in 16s
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  int e = -1, r0 = 0, rows = 0;
+  const int K = a.K, N = a.N, nb = (N + OUT - 1) / OUT;
+  int e = -1, r0 = 0, rows = 0, bx = 0;
   {
-    int slot = blockIdx.y;
+    int total = 0;
+    for (int i = 0; i < a.E; ++i) total += (max(0, min(a.offsets[i + 1], a.R) - a.offsets[i]) + BM - 1) / BM;
+    total *= nb;
+    const int per = (total + 7) / 8, local = blockIdx.x >> 3;
+    int slot = (blockIdx.x & 7) * per + local;
+    if (local >= per || slot >= total) return;
     for (int i = 0; i < a.E; ++i) {
-      const int s0 = a.offsets[i], s1 = min(a.offsets[i + 1], a.R);
-      const int t = (max(0, s1 - s0) + BM - 1) / BM;
-      if (slot < t) {
+      const int s0 = a.offsets[i], s1 = min(a.offsets[i + 1], a.R), t = (max(0, s1 - s0) + BM - 1) / BM;
+      if (slot < t * nb) {
+        const int g = slot / (GN * t), in = slot - g * GN * t, w = min(GN, nb - GN * g), m = in / w;
         e = i;
-        r0 = s0 + slot * BM;
+        bx = GN * g + in - m * w;
+        r0 = s0 + m * BM;
         rows = min(BM, s1 - r0);
         break;
       }
-      slot -= t;
+      slot -= t * nb;
     }
   }
-  if (e < 0) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wr = wave / WC, wc = wave % WC;
-  const int n0 = BN * blockIdx.x, K = a.K, N = a.N;
+  const int n0 = OUT * bx;
   const bf16* asrc[AL];
   const bf16* bsrc[BL];
 #pragma unroll
@@ -308,7 +364,8 @@ __global__ __launch_bounds__(64 * WR * WC) void expert_tile_kernel(ExpertArgs a)
 #pragma unroll
   for (int i = 0; i < BL; ++i) {
     const int row = 8 * (NWV * i + wave) + (lane >> 3), ch = (lane & 7) ^ chunk_swz(row);
-    bsrc[i] = reinterpret_cast<const bf16*>(a.W) + ((long long)e * N + min(n0 + row, N - 1)) * K + 8 * ch;
+    const int n = EPI == EPI_GLU ? min(n0 + WO * (row / WN) + row % WO, N - 1) + (row % WN >= WO ? N : 0) : min(n0 + row, N - 1);
+    bsrc[i] = reinterpret_cast<const bf16*>(a.W) + ((long long)e * (EPI == EPI_GLU ? 2 : 1) * N + n) * K + 8 * ch;
   }
   const unsigned int lds0 = lds_address(smem) + __builtin_amdgcn_readfirstlane(wave) * 1024;
   auto stage = [&](int kt, int buf) {
@@ -338,7 +395,7 @@ __global__ __launch_bounds__(64 * WR * WC) void expert_tile_kernel(ExpertArgs a)
       Pack8 bf[NS], af[MS];
 #pragma unroll
       for (int i = 0; i < NS; ++i) {
-        const int row = (BN / WC) * wc + 16 * i + j;
+        const int row = WN * wc + 16 * i + j;
         bf[i].u = *reinterpret_cast<const uint4*>(B + row * 128 + 16 * (c ^ chunk_swz(row)));
       }
 #pragma unroll
@@ -353,41 +410,65 @@ __global__ __launch_bounds__(64 * WR * WC) void expert_tile_kernel(ExpertArgs a)
     }
   }
   // lane (j, hq): output row 16 q + j of the wave's rows, columns 16 i + 4 hq + 0..3 of its columns
-  bf16* y = reinterpret_cast<bf16*>(a.y);
   const bool vec = (N & 3) == 0;
 #pragma unroll
   for (int q = 0; q < MS; ++q) {
     const int m = (BM / WR) * wr + 16 * q + j;
     if (m >= rows) continue;
 #pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      const int n = n0 + (BN / WC) * wc + 16 * i + 4 * hq;
-      bf16* o = y + (long long)(r0 + m) * N + n;
-      bf16x4 v;
+    for (int i = 0; i < NO; ++i) {
+      const int n = n0 + WO * wc + 16 * i + 4 * hq;
+      const long long at = (long long)(r0 + m) * N + n;
+      f32x4 f = acc[i][q];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = (bf16)(a.relu2 ? relu2f(acc[i][q][u]) : acc[i][q][u]);
-      if (vec) {
-        if (n < N) *reinterpret_cast<bf16x4*>(o) = v;
+      for (int u = 0; u < 4; ++u) {
+        if constexpr (EPI == EPI_GLU) f[u] = silu(f[u]) * acc[i + NO][q][u];
+        if constexpr (EPI == EPI_RELU2) f[u] = relu2f(f[u]);
+      }
+      if constexpr (EPI == EPI_F32) {
+        float* o = reinterpret_cast<float*>(a.y) + at;
+        if (vec) {
+          if (n < N) *reinterpret_cast<f32x4*>(o) = f;
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (n + u < N) o[u] = f[u];
+        }
       } else {
+        bf16* o = reinterpret_cast<bf16*>(a.y) + at;
+        bf16x4 v;
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (n + u < N) o[u] = v[u];
+        for (int u = 0; u < 4; ++u) v[u] = (bf16)f[u];
+        if (vec) {
+          if (n < N) *reinterpret_cast<bf16x4*>(o) = v;
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (n + u < N) o[u] = v[u];
+        }
       }
     }
   }
 }
 
-template <int BM, int BN, int WR, int WC>
+template <int BM, int BN, int WR, int WC, int EPI>
 void launch_tile(const ExpertArgs& a, hipStream_t s) {
-  constexpr int lds = 2 * (BM + BN) * 128;
-  static bool once = false;
-  if (lds > 64 * 1024 && !once) {
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_tile_kernel<BM, BN, WR, WC>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    once = true;
+  constexpr int lds = 2 * (BM + BN) * 128, OUT = EPI == EPI_GLU ? BN / 2 : BN;
+  if (lds > 64 * 1024) {
+    static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_tile_kernel<BM, BN, WR, WC, EPI>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    (void)once;
   }
-  dim3 grid((a.N + BN - 1) / BN, (a.R + BM - 1) / BM + a.E);
-  expert_tile_kernel<BM, BN, WR, WC><<<grid, 64 * WR * WC, lds, s>>>(a);
+  const long long tiles = (long long)((a.N + OUT - 1) / OUT) * ((a.R + BM - 1) / BM + a.E);
+  expert_tile_kernel<BM, BN, WR, WC, EPI><<<(unsigned)((tiles + 7) / 8 * 8), 64 * WR * WC, lds, s>>>(a);
+}
+
+template <int BM, int BN, int WR, int WC>
+void launch_tiles(const ExpertArgs& a, hipStream_t s) {
+  if (a.glu) launch_tile<BM, BN, WR, WC, EPI_GLU>(a, s);
+  else if (a.relu2) launch_tile<BM, BN, WR, WC, EPI_RELU2>(a, s);
+  else if (a.f32_out) launch_tile<BM, BN, WR, WC, EPI_F32>(a, s);
+  else launch_tile<BM, BN, WR, WC, EPI_BF16>(a, s);
 }
 
 template <int NW, int NE>
@@ -426,28 +507,48 @@ void launch_route_topk(const RouteArgs& a, int f32, hipStream_t s) {
                                                                                                    a.offsets, a.dst, a.src);
 }
 
+bool expert_linear_mfma(const ExpertArgs& a, int f32) {
+  return !f32 && a.K % 32 == 0 && aligned16(a.x) && aligned16(a.W) && aligned16(a.y);
+}
+
 // Returns the form used: 0 all shapes, 1 weight stream, 2 / 3 tiles of 128 / 256
+// Stream or tile, measured at 16 experts, 4 rows each on average: [gate | up] of 1536 x 2048 46.0 us on both, 2048 x 1536 23.9
+// against 28.8; at 16 rows each 53 against 46.6 and 33 against 28.7.  Tiles of 256 have one workgroup on a CU, so a tile's
+// epilogue stands alone: they win where the width is long (16384 rows, 8 experts: 2 x 14336 x 4096 3401 us against 3742,
+// 4096 x 14336 1880 against 2156; 32400 rows, 16 experts: 2048 x 1536 274 against 281), not where a gated product over 2048
+// ends in its exponentials (480 against 454).
 int launch_expert_linear(const ExpertArgs& a, int f32, int impl, hipStream_t s) {
   if (a.R <= 0) return 0;
-  const bool mfma = !f32 && aligned16(a.x) && aligned16(a.W) && aligned16(a.y);
+  const bool mfma = expert_linear_mfma(a, f32);
   const int per = (a.R + a.E - 1) / a.E;      // rows per expert if they are spread evenly
-  const bool stream = mfma && a.K % 32 == 0 && a.E <= 65535, tile = mfma && a.K % 64 == 0;
-  if (impl < 0) impl = stream && (per <= 8 || !tile) ? 1 : (tile ? (per >= 512 && a.N >= 256 ? 3 : 2) : (stream ? 1 : 0));
+  const bool stream = mfma && a.E <= 65535, tile = mfma && a.K % 64 == 0;
+  const bool big = per >= 512 && a.N >= 256 && (!a.glu || a.K >= 4096);
+  if (impl < 0) impl = stream && (per <= 8 || !tile) ? 1 : (tile ? (big ? 3 : 2) : (stream ? 1 : 0));
   if (impl == 1 && stream) {
-    dim3 grid((a.N + 15) / 16, a.E);
-    if (per <= 8) expert_stream_kernel<1, 8><<<grid, 512, 0, s>>>(a);      // (8 waves: 31 us, 4 waves: 33 us at 16 x 2304 x 2048)
-    else if (per <= 24) expert_stream_kernel<2, 4><<<grid, 256, 0, s>>>(a);
-    else expert_stream_kernel<4, 4><<<grid, 256, 0, s>>>(a);
+    const int deep = a.K / 512;               // 64-element steps of each of 8 waves
+    if (per <= 8 && a.glu) {
+      // (both rows of a pair take twice the registers: 4 waves, 2 steps: 37.7 us, 8 waves: 38.5 with 2 steps and 43 with 4, at
+      // 32 rows, 16 x 2 x 1536 x 2048 with 14 experts chosen)
+      expert_stream_kernel<1, 4, 2, EPI_GLU><<<dim3((a.N + 15) / 16, a.E), 256, 0, s>>>(a);
+    } else if (per <= 8) {
+      if (deep == 3) launch_stream<1, 8, 3>(a, s);      // (no steps left over: 21.8 us, 25 with 4 at 2048 x 1536)
+      else launch_stream<1, 8, 4>(a, s);
+    } else if (per <= 24) {
+      launch_stream<2, 4, 2>(a, s);
+    } else {
+      launch_stream<4, 4, 2>(a, s);
+    }
     return 1;
   }
   if (impl == 2 && tile) {
-    launch_tile<128, 128, 2, 2>(a, s);
+    launch_tiles<128, 128, 2, 2>(a, s);
     return 2;
   }
   if (impl == 3 && tile) {
-    launch_tile<256, 256, 2, 4>(a, s);
+    launch_tiles<256, 256, 2, 4>(a, s);
     return 3;
   }
+  if (a.glu || a.f32_out) return -1;      // (the binding has refused it)
   launch_grouped_linear(a.x, a.W, a.offsets, a.E, a.R, a.N, a.K, a.y, f32, s, a.src, a.relu2);
   return 0;
 }

@@ -3,10 +3,11 @@
 Routing, permutation into expert segments, the per-expert GEMMs and the weighted combine run as HIP
 kernels (``csrc/kernels/moe.hip``) whose segment bounds live in device memory: no host sync anywhere in
 the block, so every step (decode and prefill, with or without expert parallelism) is hipGraph-capturable.
-Small routed batches (<= 64 rows: decode steps) use the grouped skinny MFMA GEMM or the weight-streaming kernel;
+Small routed batches (<= 64 rows: decode steps) use the grouped skinny MFMA GEMM or the weight-streaming kernels;
 prefill-sized ones the prefill GEMM kernel in grouped mode (``ops.pg_grouped``, csrc/kernels/pgemm.hip) or, below
-its row thresholds, the weight-streaming / 128 x 128 tile grouped GEMMs (``ops.grouped_gemm``), SwiGLU fused into
-the gate/up epilogue everywhere.
+its row thresholds, the weight-streaming grouped GEMM (``ops.grouped_gemm``) on the preshuffled copies, and the
+gathering tile products (``ops.expert_linear``, csrc/kernels/routed_ff.hip) on row-major experts; SwiGLU fused into
+the gate/up epilogue.
 
 Expert parallelism, ``ep_size = N`` ranks each owning ``E / N`` experts (attention is tensor-parallel, so
 every rank holds the same T tokens when the block starts):
@@ -242,15 +243,15 @@ class MoEBlock:
         counts = self._buf("counts", (E,), torch.int32)
         offsets = self._buf("offsets", (E + 1,), torch.int32)
         cursor = self._buf("cursor", (E,), torch.int32)
-        xs = self._buf("xs", (R, d), torch.bfloat16)
+        src = None
         if T <= ROUTE_FUSED_ROWS:
+            xs = self._buf("xs", (R, d), torch.bfloat16)
             ops.moe_decode_route(resid, lnw, eps, self.router[i][:E], k, ids, w, counts, offsets, cursor, xs, dst)
         else:  # the one-workgroup routing launch stops paying off past a few rows (bench_moe_decode.py)
             xn = self._buf("xn", (T, d), torch.bfloat16)
             ops.rms_norm(resid, lnw, eps, xn)
-            logits = self._router_logits(i, xn)
-            ops.moe_route_permute(logits, xn, k, E, ids, w, counts, offsets, cursor, xs, dst)
-        y2 = self._experts(i, xs, offsets, self.e_lo, self.E_local, out_f32=True)
+            ids, w, dst, offsets, xs, src = self._route(i, xn)
+        y2 = self._experts(i, xs, offsets, self.e_lo, self.E_local, out_f32=True, src=src)
         if self.ep > 1:
             out = self._buf("out", (T, d), torch.float32)
             ops.moe_combine(y2, dst, ids, self.e_lo, self.e_hi, w, k, out)
@@ -273,30 +274,44 @@ class MoEBlock:
             return logits
         return self.m._linear("router", x, self.router[i])
 
+    def _gathers(self, i, R: int, d: int) -> bool:
+        """The expert products read the tokens' rows through the source list (``ops.expert_linear``), so routing writes no
+        permuted copy: layers whose expert weights are row-major only.  Routed decode rows: widths up to 2048 (8 tokens, 16
+        experts of 1536: gate/up + SwiGLU 38.9 + 4.8 -> 37.7 us; 8 experts of 14336 x 4096: 270 + 4.6 -> 292, so wider ones
+        stay on the skinny GEMM)."""
+        return (self._grouped_ok(d) and not self.single_copy and (i, "w13") not in self.pre and (i, "w2") not in self.pre
+                and (R > SKINNY_ROWS or d <= 2048))
+
     def _route(self, i, x):
+        """-> (expert ids, weights, place of every choice, segment bounds, rows, source list): rows are x's own with the
+        token of every place in the source list where the products gather, else permuted into the places (and no list)."""
         T, d = x.shape
         k, E = self.k, self.E
         R = T * k
-        logits = self._router_logits(i, x)
         ids = self._buf("ids", (R,), torch.int32)
         w = self._buf("w", (R,), torch.float32)
         dst = self._buf("dst", (R,), torch.int32)
-        counts = self._buf("counts", (E,), torch.int32)
         offsets = self._buf("offsets", (E + 1,), torch.int32)
+        if self._gathers(i, R, d):
+            src = self._buf("src", (R,), torch.int32)
+            ops.route_topk(x, self.router[i][:E], None, k, ids, w, offsets, dst, src)
+            return ids, w, dst, offsets, x, src
+        logits = self._router_logits(i, x)
+        counts = self._buf("counts", (E,), torch.int32)
         cursor = self._buf("cursor", (E,), torch.int32)
         xs = self._buf("xs", (R, d), torch.bfloat16)
         ops.moe_route_permute(logits, x, k, E, ids, w, counts, offsets, cursor, xs, dst)
-        return ids, w, dst, offsets, xs
+        return ids, w, dst, offsets, xs, None
 
     def _grouped_ok(self, d: int) -> bool:
         return d % 128 == 0 and self.F % 64 == 0 and GROUPED
 
 
 
-    def _experts(self, i, xs, offsets, e_lo, n_local, out_f32: bool = False):
+    def _experts(self, i, xs, offsets, e_lo, n_local, out_f32: bool = False, src=None):
         """Apply experts [e_lo, e_lo + n_local) to their segments of xs (segment bounds: ``offsets``, device
-        memory, global expert numbering); returns a LinOut [.., R, d]."""
-        R, d = xs.shape
+        memory, global expert numbering; ``src``: place p's row is xs[src[p]]); returns a LinOut [.., R, d]."""
+        R, d = xs.shape[0] if src is None else src.shape[0], xs.shape[1]
         w13 = self.m.w.layer(i, "w13")
         w2 = self.m.w.layer(i, "w2")
         F = self.F
@@ -324,11 +339,15 @@ class MoEBlock:
             y2 = self._buf("y2", (s2, R, d), torch.float32)
             ops.grouped_skinny(act, w2, offsets, e_lo, y2)
             return y2
+        segments = offsets[e_lo : e_lo + n_local + 1]
         if R <= SKINNY_ROWS:  # (single copy: the skinny GEMM reads the preshuffled expert stacks)
-            s1 = ops.choose_splits(2 * F, d)
-            y1 = self._buf("y1", (s1, R, 2 * F), torch.float32)
-            ops.grouped_skinny(xs, w13, offsets, e_lo, y1, wshuf=self.single_copy)
-            ops.swiglu(y1, act)
+            if src is not None:
+                ops.expert_linear(xs, src, w13, segments, act, glu=True)
+            else:
+                s1 = ops.choose_splits(2 * F, d)
+                y1 = self._buf("y1", (s1, R, 2 * F), torch.float32)
+                ops.grouped_skinny(xs, w13, offsets, e_lo, y1, wshuf=self.single_copy)
+                ops.swiglu(y1, act)
             s2 = ops.choose_splits(d, F)
             y2 = self._buf("y2", (s2, R, d), torch.float32)
             ops.grouped_skinny(act, w2, offsets, e_lo, y2, wshuf=self.single_copy)
@@ -337,8 +356,9 @@ class MoEBlock:
             # prefill-sized.  From PG_ROWS_* mean routed rows per local expert: the prefill GEMM kernel in grouped mode
             # on the preshuffled copies (csrc/kernels/pgemm.hip: block -> (expert, m-tile) from the device offsets)
             # -- SwiGLU of the [gate; up] halves in the gate/up epilogue, w2 into fp32 k-split slabs the combine
-            # sums.  Below: the weight-streaming kernel on the preshuffled copies up to PRE_ROWS* rows, the 128 x 128
-            # tile kernel beyond
+            # sums.  Below: the weight-streaming kernel on the preshuffled copies up to PRE_ROWS* rows.  Row-major
+            # experts: expert_linear (32400 rows, 16 experts of 1536 x 2048, against grouped_gemm's 128 x 128 tiles:
+            # gate/up 645 -> 454 us, w2 357 -> 281; 4000 rows 81 -> 69 and 61 -> 46; 400 rows 39 -> 33 and 27 -> 21)
             rpe = R / max(1, n_local)
             pg13 = self.pre.get((i, "w13")) if PG_GROUPED and rpe >= PG_ROWS_W13 else None
             pg2 = self.pre.get((i, "w2")) if PG_GROUPED and rpe >= PG_ROWS_W2 else None
@@ -348,8 +368,10 @@ class MoEBlock:
                 ops.pg_grouped(xs, pg13, offsets, e_lo, act, ops.PG_EPI_SWIGLU_SPLIT, c13[0])
             else:
                 p13 = self.pre.get((i, "w13")) if self.single_copy or R <= PRE_ROWS_W13 * self.E else None
-                ops.grouped_gemm(xs, w13 if p13 is None else p13, offsets, e_lo, act,
-                                 ops.GROUPED_SWIGLU + (0 if p13 is None else ops.GROUPED_PRESHUFFLED))
+                if p13 is None:
+                    ops.expert_linear(xs, src, w13, segments, act, glu=True)
+                else:
+                    ops.grouped_gemm(xs, p13, offsets, e_lo, act, ops.GROUPED_SWIGLU + ops.GROUPED_PRESHUFFLED)
             if c2 is not None:
                 cfg2, s2 = c2
                 if out_f32:
@@ -361,9 +383,11 @@ class MoEBlock:
                 return y2
             p2 = self.pre.get((i, "w2")) if self.single_copy or R <= PRE_ROWS * self.E else None
             y2 = self._buf("y2f" if out_f32 else "y2b", (R, d), torch.float32 if out_f32 else torch.bfloat16)
-            ops.grouped_gemm(act, w2 if p2 is None else p2, offsets, e_lo, y2,
-                             (ops.GROUPED_F32 if out_f32 else ops.GROUPED_BF16)
-                             + (0 if p2 is None else ops.GROUPED_PRESHUFFLED))
+            if p2 is None:
+                ops.expert_linear(act, None, w2, segments, y2)
+            else:
+                ops.grouped_gemm(act, p2, offsets, e_lo, y2, (ops.GROUPED_F32 if out_f32 else ops.GROUPED_BF16)
+                                 + ops.GROUPED_PRESHUFFLED)
             return y2
         # shapes outside the grouped kernel's tiling (not the registered models): per-expert library GEMMs
         offs = offsets.tolist()
@@ -382,8 +406,8 @@ class MoEBlock:
 
     def _forward_local(self, i, x, reduce: bool) -> torch.Tensor:
         T, d = x.shape
-        ids, w, dst, offsets, xs = self._route(i, x)
-        y2 = self._experts(i, xs, offsets, self.e_lo, self.E_local, out_f32=True)
+        ids, w, dst, offsets, xs, src = self._route(i, x)
+        y2 = self._experts(i, xs, offsets, self.e_lo, self.E_local, out_f32=True, src=src)
         out = self._buf("out", (T, d), torch.float32)
         ops.moe_combine(y2, dst, ids, self.e_lo, self.e_hi, w, self.k, out)
         if reduce:
@@ -413,8 +437,8 @@ class MoEBlock:
         N, r, k = self.ep, self.ep_rank, self.k
         S = -(-T // N)
         lo, hi = min(T, r * S), min(T, (r + 1) * S)
-        ids, w, dst, offsets, xs = self._route(i, x)
-        y = self._experts(i, xs, offsets, self.e_lo, self.E_local, out_f32=True)
+        ids, w, dst, offsets, xs, src = self._route(i, x)
+        y = self._experts(i, xs, offsets, self.e_lo, self.E_local, out_f32=True, src=src)
         cap = S  # a token sends at most one (pre-combined) row to its owner
         send = self._buf("own.send", (N * cap, d), torch.float32)
         side = self._buf("own.side", (N * cap,), torch.int32)

@@ -1178,12 +1178,13 @@ def route_topk(x, Wr, bias, k, ids, w, offsets, dst, src):
     return reference.route_topk(x, Wr, bias, k, ids, w, offsets, dst, src)
 
 
-def expert_linear(x, src, W, offsets, y, relu2=False):
-    """y[i] = W[e] x[src[i]] (src None: x[i]) for the places i of expert e's segment, W [E, N, K]; ``relu2``: relu(.)^2.
+def expert_linear(x, src, W, offsets, y, relu2=False, glu=False):
+    """y[i] = W[e] x[src[i]] (src None: x[i]) for the places i of expert e's segment, W [E, N, K]; ``relu2``: relu(.)^2;
+    ``glu``: W [E, 2 N, K] holds [gate | up] rows, y = silu(gate) * up.  bf16 inputs may have an fp32 y (neither option).
     Segment bounds are read on the device (no host sync)."""
     if _gpu(x):
-        return _hyb().expert_linear(x, src, W, offsets, y, bool(relu2))
-    return reference.expert_linear(x, src, W, offsets, y, relu2)
+        return _hyb().expert_linear(x, src, W, offsets, y, bool(relu2), -1, bool(glu))
+    return reference.expert_linear(x, src, W, offsets, y, relu2, glu)
 
 
 def residual_routed_norm(x, a, y, dst, w, k, bias, wn=None, eps=0.0, out=None):

@@ -1204,7 +1204,7 @@ def route_topk(x, Wr, bias, k, ids, w, offsets, dst, src) -> None:
     src[: T * k].copy_((order // k).int())
 
 
-def expert_linear(x, src, W, offsets, y, relu2=False) -> None:
+def expert_linear(x, src, W, offsets, y, relu2=False, glu=False) -> None:
     for e in range(W.shape[0]):
         a, b = int(offsets[e]), int(offsets[e + 1])
         if b <= a:
@@ -1213,6 +1213,8 @@ def expert_linear(x, src, W, offsets, y, relu2=False) -> None:
         p = rows.float() @ W[e].float().t()
         if relu2:
             p = torch.relu(p) ** 2
+        if glu:
+            p = torch.nn.functional.silu(p[:, : y.shape[1]]) * p[:, y.shape[1] :]
         y[a:b] = p.to(y.dtype)
 
 

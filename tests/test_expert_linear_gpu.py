@@ -1,0 +1,67 @@
+"""Gated and fp32-output expert products (``ops.expert_linear``): every form at the edges of its tiles."""
+import pytest
+import torch
+
+from symmetry_amd import ops
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def segments(E: int, R: int) -> torch.Tensor:
+    """Uneven segments: an empty one, a single row, the rest at random cuts."""
+    cuts = sorted(torch.randint(min(1, R), R + 1, (E - 3,)).tolist())
+    return torch.tensor([0, 0, min(1, R)] + cuts + [R]).int()
+
+
+@pytest.mark.parametrize("shape", [(4, 128, 192), (7, 200, 64), (5, 262, 320), (4, 384, 1536), (16, 144, 2048)])
+@pytest.mark.parametrize("R", [1, 17, 64, 129, 700, 3000])
+def test_gated_and_fp32_products(R, shape):
+    """Against 64-bit products.  fp32: K products of bf16 values summed in fp32, |error| <= K 2^-24 sum |x w| and in practice
+    its root (4 sqrt(K) 2^-24 |x| |w| here); gated: the same error of both rows through silu(g) u (|silu'| <= 1.1, the
+    exponential to 2^-20), and the rounding to bf16 (2^-8)."""
+    E, N, K = shape
+    print("expert_linear", R, shape, flush=True)
+    torch.manual_seed(R + N)
+    off = segments(E, R)
+    x, W = torch.randn(R // 2 + 1, K).to(BF16), (torch.randn(E, 2 * N, K) * K ** -0.5).to(BF16)
+    src = torch.randint(0, x.shape[0], (R,)).int()
+    g, u = torch.zeros(R, N, dtype=torch.float64), torch.zeros(R, N, dtype=torch.float64)
+    for e in range(E):
+        a, b = int(off[e]), int(off[e + 1])
+        p = x[src[a:b].long()].double() @ W[e].double().t()
+        g[a:b], u[a:b] = p[:, :N], p[:, N:]
+    norm = x.double().norm(dim=1).max() * W.double().norm(dim=2).max()
+    eps = 4 * K ** 0.5 * 2.0 ** -24 * norm
+    H = ops._hyb()
+    xd, sd, Wd, od = x.cuda(), src.cuda(), W.cuda(), off.cuda()
+    gate = Wd[:, :N].contiguous()
+    want = g / (1 + torch.exp(-g)) * u
+    bound = 2.0 ** -8 * want.abs() + 1.1 * eps * (g.abs() + u.abs()) + 2.0 ** -20 * want.abs() + 1e-30
+    for impl in (1, 2, 3, -1):
+        y = torch.full((R, N), 7.0, device="cuda")
+        H.expert_linear(xd, sd, gate, od, y, False, impl)
+        assert ((y.cpu().double() - g).abs() <= eps).all(), (impl, "fp32")
+        z = torch.full((R + 1, N), 7.0, dtype=BF16, device="cuda")
+        H.expert_linear(xd, sd, Wd, od, z[:R], False, impl, True)
+        assert ((z[:R].cpu().double() - want).abs() <= bound).all(), (impl, "gated")
+        assert (z[R] == 7.0).all()
+        H.expert_linear(xd[src.cuda().long()], None, Wd, od, y2 := torch.empty_like(z[:R]), False, impl, True)
+        assert torch.equal(y2, z[:R]), (impl, "gathered")
+
+
+def test_refusals():
+    """The gated and fp32-output products are bf16 MFMA forms; what they cannot take is an error before any launch."""
+    H, off = ops._hyb(), torch.tensor([0, 4], dtype=torch.int32, device="cuda")
+    x, W = torch.zeros(4, 40, dtype=BF16, device="cuda"), torch.zeros(1, 32, 40, dtype=BF16, device="cuda")
+    with pytest.raises(RuntimeError):      # K % 32
+        H.expert_linear(x, None, W, off, torch.zeros(4, 16, dtype=BF16, device="cuda"), False, -1, True)
+    with pytest.raises(RuntimeError):
+        H.expert_linear(x, None, W, off, torch.zeros(4, 32, device="cuda"), False)
+    x, W = x[:, :32].contiguous(), W[:, :, :32].contiguous()
+    with pytest.raises(RuntimeError):      # both epilogues
+        H.expert_linear(x, None, W, off, torch.zeros(4, 16, dtype=BF16, device="cuda"), True, -1, True)
+    with pytest.raises(RuntimeError):      # fp32 inputs have no gated form
+        H.expert_linear(x.float(), None, W.float(), off, torch.zeros(4, 16, device="cuda"), False, -1, True)
+    with pytest.raises(RuntimeError):      # no all-shapes form of it
+        H.expert_linear(x, None, W, off, torch.zeros(4, 16, dtype=BF16, device="cuda"), False, 0, True)
