@@ -28,12 +28,14 @@
 // Prefill (K4): causal + varlen + chunked prefill (queries are the LAST qlen
 // positions of a context of length ctx), reading K/V from the paged cache.
 // Default: attn_prefill_m32p_kernel (32x32x16 MFMA, GQA heads share K/V tiles,
-// see its comment); the 16x16 kernels remain for GQA groups of 1/2 heads.
+// see its comment) or, for steps of few query rows, attn_prefill_rows_kernel (one head,
+// keys shared out over the waves); the 16x16 kernels remain for GQA groups of 1/2 heads.
 #include <stdlib.h>
 #include <string.h>
 
 #include "attn_decode.h"
 #include "common.h"
+#include "direct_lds.h"
 #include "launchers.h"
 
 namespace {
@@ -543,6 +545,182 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_m32p_kernel(
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Prefill of few query rows: a workgroup is 32 query rows of ONE head, its 8 waves share out the keys and meet in LDS, so a
+// short prompt behind a long context fills the chip without a workspace (the kernel above has a workgroup per 64 rows and 4
+// heads).  Every wave streams its own 32-key subtiles through 16 KB of LDS by direct loads: K of the next subtile is in flight
+// during the softmax and P.V, its V during the S product (counted waits, no barrier), its block id one subtile before that.
+// A load instruction covers 4 K rows of 256 B or 16 V rows of 64 B (operands read straight from memory touch 32 lines an
+// instruction: 26 us for the case below); the 16-byte chunks of a row are stored permuted so that operand reads do not conflict.  K/V are read
+// once per head and 32 rows, from the L2 of the XCD that the kv head's workgroups share (grid x = kv head).
+// 137 rows behind 1063 cached tokens, 32 heads: 42 -> 13.6 us, of which ~5 the start (lengths, block ids, first K) and the
+// merge, the rest each CU's own pull of K/V (64 bytes a cycle).
+// ---------------------------------------------------------------------------------------------
+constexpr float kNoMax = -3.0e38f;   // running max before any visible key (finite: a wave may see only masked keys)
+constexpr int OST = D + 4;           // floats of a partial row in LDS
+
+__global__ __launch_bounds__(512, 2) void attn_prefill_rows_kernel(
+    const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
+    const int* __restrict__ block_tables, const int* __restrict__ ctx_lens, const int* __restrict__ cu_q,
+    const int* __restrict__ tiles, bf16* __restrict__ out, int Hq, int Hkv, int bs_shift, int max_blocks,
+    float scale_log2) {
+  const int BS = 1 << bs_shift, bs_mask = BS - 1;
+  __shared__ __attribute__((aligned(16))) char smem[8 * 32 * (OST + 2) * 4];   // >= 8 x 16 KB
+  float (*po)[32][OST] = reinterpret_cast<float (*)[32][OST]>(smem);
+  float (*pm)[32] = reinterpret_cast<float (*)[32]>(smem + 8 * 32 * OST * 4), (*pl)[32] = pm + 8;
+  const int kvh = blockIdx.x, tile = blockIdx.y >> 1;
+  const int head = kvh * (Hq / Hkv) + blockIdx.z;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 31, hh = lane >> 5;
+  const int seq = tiles[2 * tile], row0 = tiles[2 * tile + 1] + 32 * (blockIdx.y & 1);
+  const int qstart = cu_q[seq], qlen = cu_q[seq + 1] - qstart;
+  if (row0 >= qlen) return;  // workgroup-uniform, before any barrier
+  const int ctx = ctx_lens[seq], pos0 = ctx - qlen, last = ctx - 1;
+  const int* bt = block_tables + (long long)seq * max_blocks;
+  const int kend = min(ctx, pos0 + min(row0 + 32, qlen));     // keys [0, kend) visible to some row
+  const int minpos = pos0 + row0;
+  const int nsub = max(0, (kend + 31) >> 5);                  // 32-key subtiles, shared out in runs
+  const int j0 = nsub * wid >> 3, j1 = nsub * (wid + 1) >> 3;
+  const int myrow = row0 + c;
+  const bool row_ok = myrow < qlen;
+  const int mypos = row_ok ? pos0 + myrow : last;
+
+  f32x16 o[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) o[dt] = f32x16{};
+  float m = kNoMax, lsum = 0.f;
+  if (j0 < j1) {
+    const bf16* qp = q + ((long long)(qstart + min(myrow, qlen - 1)) * Hq + head) * D + 8 * hh;
+    bf16x8 qf[8];
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) qf[kk] = ld16(qp + 16 * kk);
+    const unsigned bstride = (unsigned)(Hkv * BS * D);         // elements of a block
+    const bf16* kb = k_cache + (long long)kvh * BS * D;
+    const bf16* vb = v_cache + (long long)kvh * BS * D;
+    const unsigned lds_k = lds_address(smem) + wid * 16384, lds_v = lds_k + 8192;
+    const char* sk = smem + wid * 16384;
+    const char* sv = sk + 8192;
+    // the block of a subtile (32 keys lie in one; past the context: the last key's)
+    auto id_of = [&](int j) {
+      return (unsigned)__builtin_amdgcn_readfirstlane(bt[min(32 * j, last) >> bs_shift]);
+    };
+    // K: instruction n, lane l: row 4 n + (l >> 4), 16-byte slot l & 15 = chunk ^ (row's lane in the S product & 15)
+    const int krow = lane >> 4, kslot = (lane & 15) ^ krow;
+    auto load_k = [&](int j, unsigned id) {
+      const bf16* p = kb + (size_t)id * bstride;
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        const int key = min(32 * j + 4 * n + krow, last), ch = kslot ^ ((n & 1) << 3 | (n & 2) << 1);
+        direct_load16(p + (((key & bs_mask) << 7) + 8 * ch), lds_k + 1024 * n);
+      }
+    };
+    // V: instruction n, lane l: dim 16 n + (l >> 2), slot l & 3 = key group ^ ((dim >> 1) & 3)
+    const int vg = (lane & 3) ^ ((lane >> 3) & 3), vrow = lane >> 2;
+    auto load_v = [&](int j, unsigned id) {
+      const int key = min(32 * j + 8 * vg, last & ~7);
+      const bf16* p = vb + (size_t)id * bstride + ((vrow << bs_shift) + (key & bs_mask));
+#pragma unroll
+      for (int n = 0; n < 8; ++n) direct_load16(p + (16 * n << bs_shift), lds_v + 1024 * n);
+    };
+    const unsigned first = id_of(j0);
+    unsigned id = id_of(min(j0 + 1, j1 - 1));
+    wait_direct_loads();                    // (q: its waits inside the loop would be waits for the loop's loads)
+    load_k(j0, first);
+    load_v(j0, first);
+    const int pr = (c & 3) | ((c & 4) << 1) | ((c & 8) >> 1) | (c & 16);  // bits 2 <-> 3
+    const int koff = pr * 256, ksw = c & 15, voff = c * 64, vsw = (c >> 1) & 3;
+    for (int j = j0; j < j1; ++j) {
+      const bool more = j + 1 < j1;         // (wave-uniform, as are the branches on it)
+      __builtin_amdgcn_s_waitcnt(0x0f78);   // vmcnt(8): K of j has arrived (V of j may be in flight)
+      asm volatile("" ::: "memory");
+      f32x16 sc = f32x16{};
+      {
+        Pack8 kf[8];
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) kf[kk].u = *reinterpret_cast<const uint4*>(sk + koff + 16 * ((2 * kk + hh) ^ ksw));
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) sc = mfma32(kf[kk].v, qf[kk], sc);
+      }
+      __builtin_amdgcn_sched_barrier(0);    // (the operands are in registers before their place is filled again)
+      const unsigned cur = id;
+      if (more) {
+        load_k(j + 1, cur);
+        id = id_of(min(j + 2, j1 - 1));
+      }
+      if (32 * j + 31 > minpos) mask_subtile(sc, 32 * j, mypos);
+      const float tmax = subtile_max(sc, scale_log2);
+      if (!__all(tmax <= m + kRescaleThr)) {
+        const float mn = fmaxf(m, tmax);
+        const float alpha = __builtin_amdgcn_exp2f(m - mn);
+        m = mn;
+        lsum *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
+      }
+      Pack8 pf[2];
+      float psum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float p = __builtin_amdgcn_exp2f(fmaf(sc[i], scale_log2, -m));
+        psum += p;
+        pf[i >> 3].h[i & 7] = (bf16)p;
+      }
+      lsum += psum;
+      if (more) __builtin_amdgcn_s_waitcnt(0x0f78);   // vmcnt(8): V of j has arrived (K of the next may be in flight)
+      else wait_direct_loads();
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+          Pack8 vf;
+          vf.u = *reinterpret_cast<const uint4*>(sv + 32 * dt * 64 + voff + 16 * ((2 * ks + hh) ^ vsw));
+          o[dt] = mfma32(vf.v, pf[ks].v, o[dt]);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) load_v(j + 1, cur);
+    }
+  }
+  __syncthreads();                          // (no load is in flight: the staging becomes the partials' place)
+  const float l = xhalf_sum(lsum);
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = o[dt][4 * g + e];
+      *reinterpret_cast<f32x4*>(&po[wid][c][32 * dt + 8 * g + 4 * hh]) = v;
+    }
+  if (hh == 0) {
+    pm[wid][c] = m;
+    pl[wid][c] = l;
+  }
+  __syncthreads();
+  const int r = threadIdx.x >> 4, d0 = 8 * (threadIdx.x & 15);
+  if (row0 + r >= qlen) return;
+  float mx = pm[0][r], sum = 0.f, acc[8] = {};
+#pragma unroll
+  for (int w = 1; w < 8; ++w) mx = fmaxf(mx, pm[w][r]);
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    const float f = __builtin_amdgcn_exp2f(pm[w][r] - mx);
+    sum = fmaf(pl[w][r], f, sum);
+    const f32x4 a = *reinterpret_cast<const f32x4*>(&po[w][r][d0]), b = *reinterpret_cast<const f32x4*>(&po[w][r][d0 + 4]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      acc[e] = fmaf(a[e], f, acc[e]);
+      acc[4 + e] = fmaf(b[e], f, acc[4 + e]);
+    }
+  }
+  const float inv = nsub > 0 ? 1.f / sum : 0.f;   // (every row sees its own key; no sum at all only from infinite scores)
+  Pack8 res;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) res.h[e] = (bf16)(acc[e] * inv);
+  *reinterpret_cast<uint4*>(out + ((long long)(qstart + row0 + r) * Hq + head) * D + d0) = res.u;
+}
+
 }  // namespace
 
 // Decode: a unit is a (sequence, kv head); contexts are cut so far that the workgroups just fill the chip, two 8-wave
@@ -575,6 +753,12 @@ void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache,
   else run(attn_decode_kernel<16>);
 }
 
+// Workgroups of the 64-row x 4-head kernel up to which the row kernel takes a prompt step: below, most CUs would idle; above,
+// K/V read once per head costs more than it fills.  us, 64-row kernel / row kernel (query rows behind a context, 32 heads):
+//   24: 137 of 1200   42 / 13.6       48: 384 of 2000  65 / 34      96: 768 of 4000   133 / 106     128: 1024 of 1024  38 / 39
+//   32: 256 of 8000  233 / 69         64: 512 of 512   23 / 16      96: 1500 of 1500   49 / 35      128: 16 x 60 of 600  30 / 45
+constexpr int ROWS_WGS = 96;
+
 void launch_attn_prefill(const bf16* q, const bf16* k_cache, const bf16* v_cache, const int* block_tables,
                          const int* ctx_lens, const int* cu_q, const int* tiles, int num_tiles, bf16* out, int Hq,
                          int Hkv, int BS, int max_blocks, float scale, hipStream_t s) {
@@ -585,6 +769,11 @@ void launch_attn_prefill(const bf16* q, const bf16* k_cache, const bf16* v_cache
   static const char* knob = getenv("SYMMETRY_ATTN_PREFILL");
   static const bool use_lds = knob && strstr(knob, "lds");
   if (!use_lds && BS >= 8 && (BS & (BS - 1)) == 0 && G % 4 == 0) {
+    if (BS >= 32 && Hkv * num_tiles * (G / 4) <= ROWS_WGS) {
+      attn_prefill_rows_kernel<<<dim3(Hkv, 2 * num_tiles, G), 512, 0, s>>>(
+          q, k_cache, v_cache, block_tables, ctx_lens, cu_q, tiles, out, Hq, Hkv, __builtin_ctz(BS), max_blocks, scale_log2);
+      return;
+    }
     attn_prefill_m32p_kernel<<<dim3(Hkv, num_tiles, G / 4), 512, 0, s>>>(
         q, k_cache, v_cache, block_tables, ctx_lens, cu_q, tiles, out, Hq, Hkv, __builtin_ctz(BS), max_blocks,
         scale_log2);
