@@ -77,80 +77,106 @@ __global__ __launch_bounds__(NT) void rope_cache_kernel(LinOut qkv, const int* _
   }
 }
 
-// Prefill form: grid (T / 8, 8).  Workgroup (g, y) rotates row 8 g + y (as above) and writes the V rows
-// of kv heads y, y + 8, ... for the 8 rows of group g.  The dim-major V write -- 2-byte stores at a
-// BS-element stride, one cache line touched per element, which made the plain kernel ~3x slower than its
-// bytes (16.5 us at 1280 tokens) -- becomes one 16-byte store of 8 consecutive tokens per (kv head, dim)
-// whenever the 8 rows fill 8 consecutive, 8-aligned slots of one block (a prefill chunk of one
-// sequence); other groups fall back to per-token stores.  The 8 V loads per thread stay coalesced
-// across the wave (consecutive dims of one row).
-constexpr int RG = 8;
+// Prefill form, two kinds of workgroups in one launch.
+// V (the first nv): 64 tokens x 64 columns through LDS, so that the dim-major cache is written as 16-byte runs of 8 slots, the
+// runs of a dim by neighbouring lanes (64 tokens of a block: whole 128-byte lines, by one XCD).  Runs are cut where the SLOTS
+// are multiples of 8, so a prompt behind a cached context of any length has them too; tokens outside such a run (ends,
+// sequence changes, padding) are written one by one.
+// Rotation: one item (8 dim pairs of a head) per thread over all rows.
+// Bound by the bytes at long prompts (8100 tokens of 32 + 2 x 8 heads: 60 -> 39 us, from a place that is no multiple of 8
+// 101 -> 43) and by one chain of dependent loads at short ones (137 tokens behind 1063, fp32 slabs: 14.9 -> 7.1 us).  Before, a
+// workgroup took a row's rotation and then its share of V, and runs only where a group of 8 rows began at a multiple of 8.
+constexpr int VT = 64, VC = 64, VST = VC + 2;
+typedef bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-__global__ __launch_bounds__(NT) void rope_cache_grouped_kernel(LinOut qkv, const int* __restrict__ positions,
-                                                                const int* __restrict__ slots,
-                                                                const float* __restrict__ cos_sin,
-                                                                bf16* __restrict__ q_out, bf16* __restrict__ k_cache,
-                                                                bf16* __restrict__ v_cache, int T, int Hq, int Hkv,
-                                                                int D, int BS, int perm) {
-  const int t0 = blockIdx.x * RG;
-  const int nt = min(RG, T - t0);
+__global__ __launch_bounds__(NT) void rope_cache_prompt_kernel(LinOut qkv, const int* __restrict__ positions,
+                                                               const int* __restrict__ slots,
+                                                               const float* __restrict__ cos_sin,
+                                                               bf16* __restrict__ q_out, bf16* __restrict__ k_cache,
+                                                               bf16* __restrict__ v_cache, int T, int Hq, int Hkv,
+                                                               int D, int BS, int perm, int nv) {
   const int N = (Hq + 2 * Hkv) * D;
-  const int half = D / 2;
-  const int gpr = half / 8;
-  const int t = t0 + blockIdx.y;
-  if (t < T) {  // rotation of one row (uniform over the workgroup)
-    const long long row = (long long)t * N;
-    const float* cs = cos_sin + (long long)positions[t] * D;
-    const int slot = slots ? slots[t] : -1;
-    for (int it = threadIdx.x; it < (Hq + Hkv) * gpr; it += NT) {
-      const int h = it / gpr;
-      const int i0 = (it % gpr) * 8;
-      float x1[8], x2[8], c[8], sn[8];
-      const int p1 = perm ? 2 * i0 : i0, p2 = perm ? 2 * i0 + 8 : half + i0;
-      linout_load8(qkv, row + (long long)h * D + p1, x1);
-      linout_load8(qkv, row + (long long)h * D + p2, x2);
-      load8f(cs + i0, c);
-      load8f(cs + half + i0, sn);
-      float o1[8], o2[8];
+  if ((int)blockIdx.x >= nv) {
+    const int half = D / 2, gpr = half / 8, items = (Hq + Hkv) * gpr;
+    const unsigned idx = (blockIdx.x - nv) * NT + threadIdx.x;
+    const int t = idx / (unsigned)items, it = idx - (unsigned)t * items;
+    if (t >= T) return;
+    const int h = it / gpr, i0 = (it - h * gpr) * 8;
+    const int pos = positions[t], slot = slots ? slots[t] : -1;
+    const long long row = (long long)t * N + (long long)h * D;
+    float x1[8], x2[8], c[8], sn[8];
+    linout_load8(qkv, row + (perm ? 2 * i0 : i0), x1);
+    linout_load8(qkv, row + (perm ? 2 * i0 + 8 : half + i0), x2);
+    const float* cs = cos_sin + (long long)pos * D + i0;
+    load8f(cs, c);
+    load8f(cs + half, sn);
+    float o1[8], o2[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        o1[j] = x1[j] * c[j] - x2[j] * sn[j];
-        o2[j] = x2[j] * c[j] + x1[j] * sn[j];
-      }
-      if (h < Hq) {
-        bf16* q = q_out + ((long long)t * Hq + h) * D;
-        store8(q + i0, o1);
-        store8(q + half + i0, o2);
-      } else if (slot >= 0) {
-        const int kh = h - Hq;
-        const long long blk = slot / BS, off = slot % BS;
-        bf16* k = k_cache + ((blk * Hkv + kh) * BS + off) * D;
-        store8(k + i0, o1);
-        store8(k + half + i0, o2);
+    for (int j = 0; j < 8; ++j) {
+      o1[j] = x1[j] * c[j] - x2[j] * sn[j];
+      o2[j] = x2[j] * c[j] + x1[j] * sn[j];
+    }
+    bf16* o = q_out + ((long long)t * Hq + h) * D;
+    if (h >= Hq) {
+      if (slot < 0) return;
+      const long long blk = slot / BS, off = slot % BS;
+      o = k_cache + ((blk * Hkv + h - Hq) * BS + off) * D;
+    }
+    store8(o + i0, o1);
+    store8(o + half + i0, o2);
+    return;
+  }
+  __shared__ bf16 tile[VT * VST];
+  __shared__ int sl[VT], run[VT / 8 + 1];
+  const int cols = Hkv * D, nc = (cols + VC - 1) / VC;
+  const int t0 = (blockIdx.x / nc) * VT, c0 = (blockIdx.x % nc) * VC, nt = min(VT, T - t0);
+  if (threadIdx.x < VT) sl[threadIdx.x] = (int)threadIdx.x < nt ? slots[t0 + threadIdx.x] : -1;
+  {
+    const int tok = threadIdx.x >> 2, cc = (threadIdx.x & 3) * 16;
+    if (tok < nt && c0 + cc < cols) {                      // (columns come in sixteens)
+      const long long at = (long long)(t0 + tok) * N + (long long)(Hq + Hkv) * D + c0 + cc;
+      float x[16];
+      linout_load8(qkv, at, x);
+      linout_load8(qkv, at + 8, x + 8);
+      bf16* d = tile + tok * VST + cc;
+#pragma unroll
+      for (int j = 0; j < 16; j += 2) {
+        bf16x2 v;
+        v[0] = (bf16)x[j], v[1] = (bf16)x[j + 1];
+        *reinterpret_cast<bf16x2*>(d + j) = v;
       }
     }
   }
-  if (!slots) return;
-  // V of kv heads y, y + 8, ...: can this group go out as 16-byte token runs?  (uniform)
-  const int s0 = slots[t0];
-  bool run = nt == RG && s0 >= 0 && s0 % RG == 0 && BS % RG == 0;
-  for (int j = 1; j < RG && run; ++j) run = slots[t0 + j] == s0 + j;
-  const long long vbase = (long long)(Hq + Hkv) * D;
-  for (int it = blockIdx.y * D + threadIdx.x; it < Hkv * D; it += RG * D) {
-    if (threadIdx.x >= D) break;  // D threads per kv head
-    const int kh = it / D, d = it % D;
-    float x[RG];
+  __syncthreads();
+  const int phase = max(sl[0], 0) & 7;                     // run j: tokens 8 j - phase .. + 7
+  if (threadIdx.x <= VT / 8) {
+    const int s = 8 * threadIdx.x - phase;
+    bool r = BS % 8 == 0 && s >= 0 && s + 8 <= nt;
+    if (r) {
+      const int first = sl[s];
+      r = first >= 0 && first % 8 == 0;
+      for (int j = 1; j < 8; ++j) r = r && sl[s + j] == first + j;
+    }
+    run[threadIdx.x] = r;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < (VT / 8 + 1) * VC; i += NT) {
+    const int j = i < VT / 8 * VC ? i % (VT / 8) : VT / 8, c = i < VT / 8 * VC ? i / (VT / 8) : i - VT / 8 * VC;
+    if (c0 + c >= cols) continue;
+    const int kh = (c0 + c) / D, d = (c0 + c) - kh * D, s = 8 * j - phase;
+    if (run[j]) {
+      const int first = sl[s];
+      const long long blk = first / BS, off = first % BS;
+      Pack8 v;
 #pragma unroll
-    for (int j = 0; j < RG; ++j) x[j] = j < nt ? linout_load1(qkv, (long long)(t0 + j) * N + vbase + it) : 0.f;
-    if (run) {
-      const long long blk = s0 / BS, off = s0 % BS;
-      store8(v_cache + ((blk * Hkv + kh) * D + d) * BS + off, x);
+      for (int e = 0; e < 8; ++e) v.h[e] = tile[(s + e) * VST + c];
+      *reinterpret_cast<uint4*>(v_cache + ((blk * Hkv + kh) * D + d) * BS + off) = v.u;
     } else {
-      for (int j = 0; j < nt; ++j) {
-        const int slot = slots[t0 + j];
+      for (int e = max(s, 0); e < min(s + 8, nt); ++e) {
+        const int slot = sl[e];
         if (slot < 0) continue;
         const long long blk = slot / BS, off = slot % BS;
-        v_cache[((blk * Hkv + kh) * D + d) * BS + off] = (bf16)x[j];
+        v_cache[((blk * Hkv + kh) * D + d) * BS + off] = tile[e * VST + c];
       }
     }
   }
@@ -164,9 +190,11 @@ void launch_rope_cache(LinOut qkv, const int* positions, const int* slots, const
   if (T == 0) return;
   // decode rows belong to different sequences (no V token runs to gain): the per-row kernel with enough
   // workgroups per row that every thread handles one 8-dim item
-  if (!decode && T >= 4 * RG && D <= NT) {  // prefill chunks: 8-row groups with 16-byte V token runs
-    rope_cache_grouped_kernel<<<dim3((T + RG - 1) / RG, RG), NT, 0, s>>>(qkv, positions, slots, cos_sin, q_out,
-                                                                          k_cache, v_cache, T, Hq, Hkv, D, BS, perm);
+  const long long rot = (long long)T * (Hq + Hkv) * (D / 16);
+  if (!decode && T >= 32 && rot < (1ll << 31)) {
+    const int nv = slots ? (T + VT - 1) / VT * ((Hkv * D + VC - 1) / VC) : 0;
+    rope_cache_prompt_kernel<<<nv + (unsigned)((rot + NT - 1) / NT), NT, 0, s>>>(
+        qkv, positions, slots, cos_sin, q_out, k_cache, v_cache, T, Hq, Hkv, D, BS, perm, nv);
     return;
   }
   const int items = (Hq + Hkv) * (D / 16) + Hkv * (D / 8);
