@@ -675,7 +675,7 @@ void qk_row_norm_cache(const Tensor& z, const OptTensor& bias, int64_t H, int64_
 }
 
 void route_topk(const Tensor& x, const Tensor& Wr, const OptTensor& bias, int64_t k, Tensor& ids, Tensor& w, Tensor& offsets,
-                Tensor& dst, Tensor& src) {
+                Tensor& dst, Tensor& src, bool runs) {
   const int f32 = act(x, "x");
   same_act(Wr, f32, "Wr");
   dtype(w, at::kFloat, "w");
@@ -693,6 +693,8 @@ void route_topk(const Tensor& x, const Tensor& Wr, const OptTensor& bias, int64_
   a.x = x.data_ptr(), a.Wr = Wr.data_ptr();
   a.T = (int)T, a.d = (int)x.size(1), a.E = (int)E, a.k = (int)k;
   a.ids = ptr<int>(ids), a.w = ptr<float>(w), a.offsets = ptr<int>(offsets), a.dst = ptr<int>(dst), a.src = ptr<int>(src);
+  a.runs = runs;
+  TORCH_CHECK(!runs || (route_topk_runs(a, f32) && !a.bias), "route_topk: runs: bf16, at most 16 experts, d % 128 == 0, no bias");
   launch_route_topk(a, f32, cur_stream(x));
 }
 
@@ -1201,7 +1203,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
       &qk_row_norm_cache);
   m.def(
       "route_topk(Tensor x, Tensor Wr, Tensor? bias, int k, Tensor(a!) ids, Tensor(b!) w, Tensor(c!) offsets, Tensor(d!) dst, "
-      "Tensor(e!) src) -> ()",
+      "Tensor(e!) src, bool runs=False) -> ()",
       &route_topk);
   m.def(
       "expert_linear(Tensor x, Tensor? src, Tensor W, Tensor offsets, Tensor(a!) y, bool relu2, int impl=-1, bool glu=False) -> int",

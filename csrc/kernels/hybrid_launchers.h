@@ -179,7 +179,9 @@ struct RouteArgs {
   int* offsets;
   int* dst;
   int* src;
+  int runs;             // the sums and weights of moe_router + moe_route (where route_topk_runs)
 };
+bool route_topk_runs(const RouteArgs& a, int f32);
 void launch_route_topk(const RouteArgs& a, int f32, hipStream_t s);
 // y[i] = W[e] x[src ? src[i] : i] (relu2: relu(.)^2) for the places i of expert e's segment, W [E][N][K], y [R][N]
 struct ExpertArgs {

@@ -108,6 +108,8 @@ __global__ __launch_bounds__(PLAN_NT) void expert_layout_kernel(const int* __res
 
 // grid ceil(T / 16), NW waves; NE expert tiles of 16 (E <= 16 NE), d % 32 == 0.  Dynamic LDS: NW NE 256 floats (partial
 // logits) or, reused, 16 E floats + the layout's counters; PLAN: the single workgroup lays out the segments as well.
+// a.runs: every wave takes one run of the width (d % (32 NW) == 0), and the hardware exponential: the sums and weights of
+// moe_router_kernel and moe_route_kernel, to the bit.
 template <int NW, int NE, bool PLAN>
 __global__ __launch_bounds__(64 * NW) void route_mfma_kernel(RouteArgs a) {
   extern __shared__ float part[];
@@ -122,8 +124,9 @@ __global__ __launch_bounds__(64 * NW) void route_mfma_kernel(RouteArgs a) {
     w[n] = reinterpret_cast<const bf16*>(a.Wr) + (long long)min(16 * n + j, E - 1) * d + 8 * hq;
     acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  const int first = a.runs ? wave * (d / NW) : 32 * wave, last = a.runs ? first + d / NW : d, step = a.runs ? 32 : 32 * NW;
 #pragma unroll 4
-  for (int c = 32 * wave; c < d; c += 32 * NW) {
+  for (int c = first; c < last; c += step) {
     Pack8 xf;
     xf.u = *reinterpret_cast<const uint4*>(x + c);
 #pragma unroll
@@ -148,6 +151,7 @@ __global__ __launch_bounds__(64 * NW) void route_mfma_kernel(RouteArgs a) {
   for (int t = wave; t < 16; t += NW) {
     if (t0 + t >= a.T) break;
     float z = lane < 16 * NE ? part[((lane >> 4) * 16 + t) * 16 + (lane & 15)] : -INFINITY;   // (E <= 64: one per lane)
+    if (z != z) z = -INFINITY;      // a NaN logit never wins
     float zmax = 0.f, sum = 0.f, mine = 0.f;
     int my = 0;
     for (int q = 0; q < a.k; ++q) {
@@ -161,7 +165,7 @@ __global__ __launch_bounds__(64 * NW) void route_mfma_kernel(RouteArgs a) {
       }
       if (!(best > -INFINITY) || bi >= E) bi = q;   // only with non-finite logits: a valid segment index
       if (q == 0) zmax = best;
-      const float p = q == 0 ? 1.f : expf(best - zmax);
+      const float p = q == 0 || zmax == -INFINITY ? 1.f : a.runs ? __expf(best - zmax) : expf(best - zmax);
       sum += p;
       if (lane == q) my = bi, mine = p;
       if (lane == bi) z = -INFINITY;
@@ -487,13 +491,21 @@ void launch_route_ne(const RouteArgs& a, hipStream_t s) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+bool route_mfma(const RouteArgs& a, int f32) {
+  return !f32 && a.d % 32 == 0 && a.E <= 64 && a.k <= 64 && aligned16(a.x) && aligned16(a.Wr);
+}
+
 }  // namespace
+
+bool route_topk_runs(const RouteArgs& a, int f32) { return route_mfma(a, f32) && a.E <= 16 && a.d % 128 == 0; }
 
 void launch_route_topk(const RouteArgs& a, int f32, hipStream_t s) {
   if (a.T <= 0) return;
-  const bool mfma = !f32 && a.d % 32 == 0 && a.E <= 64 && a.k <= 64 && aligned16(a.x) && aligned16(a.Wr);
-  if (mfma) {
-    if (a.E <= 16) launch_route_ne<1>(a, s);
+  if (route_mfma(a, f32)) {
+    if (a.runs) {
+      if (a.d % 512 == 0) launch_route<16, 1>(a, s);
+      else launch_route<4, 1>(a, s);
+    } else if (a.E <= 16) launch_route_ne<1>(a, s);
     else if (a.E <= 32) launch_route_ne<2>(a, s);
     else launch_route_ne<4>(a, s);
     if (a.T <= 16) return;      // the single workgroup laid out the segments

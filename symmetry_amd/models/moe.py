@@ -294,7 +294,7 @@ class MoEBlock:
         offsets = self._buf("offsets", (E + 1,), torch.int32)
         if self._gathers(i, R, d):
             src = self._buf("src", (R,), torch.int32)
-            ops.route_topk(x, self.router[i][:E], None, k, ids, w, offsets, dst, src)
+            ops.route_topk(x, self.router[i][:E], None, k, ids, w, offsets, dst, src, runs=E <= 16)
             return ids, w, dst, offsets, x, src
         logits = self._router_logits(i, x)
         counts = self._buf("counts", (E,), torch.int32)

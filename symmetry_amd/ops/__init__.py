@@ -1169,12 +1169,13 @@ def qk_row_norm_cache(z, bias, H, G, dk, wq, wk, eps, temp_coef, temp_every, pos
                                        kv_cache, key_scale)
 
 
-def route_topk(x, Wr, bias, k, ids, w, offsets, dst, src):
+def route_topk(x, Wr, bias, k, ids, w, offsets, dst, src, runs=False):
     """Router: logits x @ Wr.T + bias (fp32; bias optional), the k largest (ties: the lowest index) -> ids [T k], w = softmax
     over the chosen logits; and the routed rows' places in expert order: offsets [E + 1] segment bounds, dst [T k] place of
-    every (token, choice), src [T k] token of every place."""
+    every (token, choice), src [T k] token of every place.  ``runs`` (bf16, at most 16 experts, d % 128 == 0, no bias): the
+    order of sums and the exponential of ``moe_router`` + ``moe_route``, so both choose and weigh alike to the bit."""
     if _gpu(x):
-        return _hyb().route_topk(x, Wr, bias, int(k), ids, w, offsets, dst, src)
+        return _hyb().route_topk(x, Wr, bias, int(k), ids, w, offsets, dst, src, bool(runs))
     return reference.route_topk(x, Wr, bias, k, ids, w, offsets, dst, src)
 
 

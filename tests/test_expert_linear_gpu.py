@@ -65,3 +65,28 @@ def test_refusals():
         H.expert_linear(x.float(), None, W.float(), off, torch.zeros(4, 16, device="cuda"), False, -1, True)
     with pytest.raises(RuntimeError):      # no all-shapes form of it
         H.expert_linear(x, None, W, off, torch.zeros(4, 16, dtype=BF16, device="cuda"), False, 0, True)
+
+
+@pytest.mark.parametrize("T", [1, 16, 17, 700])
+@pytest.mark.parametrize("E,k,d", [(16, 4, 2048), (8, 2, 384), (10, 3, 512), (2, 1, 128)])
+def test_router_in_runs(T, E, k, d):
+    """``runs`` chooses and weighs as moe_router + moe_route do, to the bit, also where a token's logits are not numbers, and
+    lays the segments out over them."""
+    print("route_topk runs", T, E, k, d, flush=True)
+    torch.manual_seed(T + E)
+    x, Wr = torch.randn(T, d).to(BF16).cuda(), torch.zeros(16, d, dtype=BF16)
+    Wr[:E] = torch.randn(E, d) * 2 * d ** -0.5
+    Wr[E // 2] = Wr[0]                         # a tie in every row
+    x[T // 2, 5] = float("nan")
+    Wr, R, i32 = Wr.cuda(), T * k, dict(dtype=torch.int32, device="cuda")
+    logits, ids0, w0 = torch.empty(T, 16, device="cuda"), torch.empty(R, **i32), torch.empty(R, device="cuda")
+    ops.moe_router(x, Wr, logits)
+    ops.moe_route(logits, T, k, E, ids0, w0)
+    ids, w, off = torch.empty(R, **i32), torch.empty(R, device="cuda"), torch.empty(E + 1, **i32)
+    dst, src = torch.empty(R, **i32), torch.empty(R, **i32)
+    ops.route_topk(x, Wr[:E], None, k, ids, w, off, dst, src, runs=True)
+    rows = torch.arange(T) != T // 2           # (a row without numbers: any valid experts, equal weights)
+    assert torch.equal(ids.view(T, k)[rows], ids0.view(T, k)[rows]) and torch.equal(w, w0)
+    assert int(ids.min()) >= 0 and int(ids.max()) < E
+    assert torch.equal(src[dst.long()].cpu(), (torch.arange(R) // k).int())
+    assert torch.equal(off.diff().cpu().long(), torch.bincount(ids.cpu().long(), minlength=E))
