@@ -87,12 +87,50 @@ SYM_DEV void dot_rows(const T* __restrict__ k, const float* __restrict__ qs, int
   }
 }
 
+// 64 keys' scores, a group of LPR lanes per key row (16 bytes a lane: dk = 8 LPR): lane i's own key (cache row `slot`) -> out.
+// Instruction n reads row n of every group, so a load touches whole rows; read lane by lane, 64 rows per instruction, a line
+// came from the L2 up to eight times (8 rows x 16 heads x 1024 keys of 128, 4 key heads: 23.3 -> 18.6 us per launch).
+template <int CTRL>
+SYM_DEV float dpp_add(float v) {
+  return v + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+template <int LPR, int REP>
+SYM_DEV void group_scores(const bf16* __restrict__ kc, int slot, int G, int g, const float* __restrict__ qs, float* out) {
+  constexpr int dk = 8 * LPR, B = REP == 1 ? LPR : 4;      // rows in flight per group
+  const int lane = threadIdx.x & 63, part = lane % LPR, first = lane - part;
+  float q[REP][8];
+#pragma unroll
+  for (int r = 0; r < REP; ++r)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[r][i] = qs[r * dk + 8 * part + i];
+  for (int n0 = 0; n0 < LPR; n0 += B) {
+    Pack8 f[B];
+#pragma unroll
+    for (int n = 0; n < B; ++n)
+      f[n].u = *reinterpret_cast<const uint4*>(kc + ((long long)__shfl(slot, first + n0 + n, 64) * G + g) * dk + 8 * part);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < B; ++n)
+#pragma unroll
+      for (int r = 0; r < REP; ++r) {
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s += (float)f[n].h[i] * q[r][i];
+        s = dpp_add<0xB1>(s);                              // lanes 1 apart
+        s = dpp_add<0x4E>(s);                              // 2
+        s = dpp_add<0x141>(s);                             // the other four of eight
+        if constexpr (LPR == 16) s = dpp_add<0x140>(s);    // the other eight of sixteen
+        if (part == n0 + n) out[r] = s;
+      }
+  }
+}
+
 // grid (H / REP, T), NW waves.  A workgroup serves REP query heads that share one key / value head (REP = H / G where
 // that is 1, 2, 4 or 8, else 1 with one workgroup per head): a key row is read once for the REP scores, a value row
 // once for the REP accumulators.  Wave w walks the key tiles w, w + NW, ... of the row's window with its own running
 // max / sum / accumulators; the waves' partial results meet in LDS at the end (rows of a decode step have few (row,
 // head) pairs and long windows: NW > 1 shortens each wave's walk).  Dynamic LDS: REP dk + NW REP (2 + 64 nvc) floats.
-template <typename T, int NW, int REP, bool PAIR>
+template <typename T, int NW, int REP, bool PAIR, int VC>
 __global__ __launch_bounds__(64 * NW) void window_attn_wave_kernel(WindowAttnArgs a) {
   extern __shared__ float lds[];
   float* qs = lds;                      // [REP][dk]
@@ -110,7 +148,8 @@ __global__ __launch_bounds__(64 * NW) void window_attn_wave_kernel(WindowAttnArg
   __syncthreads();
   const T* kc = reinterpret_cast<const T*>(a.k_cache);
   const T* vc = reinterpret_cast<const T*>(a.v_cache);
-  float acc[REP][MAX_VCOLS];
+  const bool grouped = (reinterpret_cast<uintptr_t>(kc) & 15) == 0;
+  float acc[REP][VC];
   float m[REP], l[REP], b1[REP], b2[REP];
 #pragma unroll
   for (int r = 0; r < REP; ++r) {
@@ -118,7 +157,7 @@ __global__ __launch_bounds__(64 * NW) void window_attn_wave_kernel(WindowAttnArg
     b2[r] = a.bias ? a.bias[a.H + h0 + r] : 0.f;
     m[r] = -INFINITY, l[r] = 0.f;
 #pragma unroll
-    for (int i = 0; i < MAX_VCOLS; ++i) acc[r][i] = 0.f;
+    for (int i = 0; i < VC; ++i) acc[r][i] = 0.f;
   }
   for (int t0 = 64 * wave; t0 < total; t0 += 64 * NW) {
     const int idx = t0 + lane;
@@ -126,9 +165,15 @@ __global__ __launch_bounds__(64 * NW) void window_attn_wave_kernel(WindowAttnArg
     const int j = idx < kf ? idx : j0 + idx - kf;
     float sc[REP], w[REP];
     long long slot = 0;                       // lanes past the row's last key: weight 0 on a finite row (slot 0)
+    if (on) slot = cache_row(bt, j, a.BS, a.bs_shift);
+    bool scored = false;
+    if constexpr (sizeof(T) == 2) {
+      // (wave-uniform; every lane takes part, those past the last key on row 0)
+      if (grouped && a.dk == 128) group_scores<16, REP>(reinterpret_cast<const bf16*>(kc), (int)slot, a.G, g, qs, sc), scored = true;
+      else if (grouped && a.dk == 64) group_scores<8, REP>(reinterpret_cast<const bf16*>(kc), (int)slot, a.G, g, qs, sc), scored = true;
+    }
     if (on) {
-      slot = cache_row(bt, j, a.BS, a.bs_shift);
-      dot_rows<T, REP>(kc + (slot * a.G + g) * a.dk, qs, a.dk, sc);
+      if (!scored) dot_rows<T, REP>(kc + (slot * a.G + g) * a.dk, qs, a.dk, sc);
       if (a.key_scale) {
         const float ks = a.key_scale[slot];
 #pragma unroll
@@ -155,7 +200,7 @@ __global__ __launch_bounds__(64 * NW) void window_attn_wave_kernel(WindowAttnArg
       l[r] = l[r] * corr + wave_sum(w[r]);
       m[r] = mt;
 #pragma unroll
-      for (int i = 0; i < MAX_VCOLS; ++i) acc[r][i] *= corr;
+      for (int i = 0; i < VC; ++i) acc[r][i] *= corr;
     }
     const int nt = min(64, total - t0);
     const int vslot = (int)slot;              // (cache rows fit 31 bits: checked by the op layer)
@@ -167,13 +212,13 @@ __global__ __launch_bounds__(64 * NW) void window_attn_wave_kernel(WindowAttnArg
       const T* vr[VB];
 #pragma unroll
       for (int u = 0; u < VB; ++u) {
-        vr[u] = vc + ((long long)__shfl(vslot, jj + u, 64) * a.G + g) * a.dv;
+        vr[u] = vc + ((long long)__builtin_amdgcn_readlane(vslot, jj + u) * a.G + g) * a.dv;
 #pragma unroll
-        for (int r = 0; r < REP; ++r) pw[r][u] = __shfl(w[r], jj + u, 64);
+        for (int r = 0; r < REP; ++r) pw[r][u] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w[r]), jj + u));
       }
       if constexpr (PAIR) {
 #pragma unroll
-        for (int i = 0; i < MAX_VCOLS; i += 2) {
+        for (int i = 0; i < VC; i += 2) {
           const int c = vcol<true>(lane, i);
           if (c < a.dv) {
             float v0[VB], v1[VB];
@@ -190,7 +235,7 @@ __global__ __launch_bounds__(64 * NW) void window_attn_wave_kernel(WindowAttnArg
         }
       } else {
 #pragma unroll
-        for (int i = 0; i < MAX_VCOLS; ++i) {
+        for (int i = 0; i < VC; ++i) {
           const int c = lane + 64 * i;
           if (c < a.dv) {
             float vv[VB];
@@ -211,7 +256,7 @@ __global__ __launch_bounds__(64 * NW) void window_attn_wave_kernel(WindowAttnArg
       float* mine = part + (wave * REP + r) * pstride;
       if (lane == 0) mine[0] = m[r], mine[1] = l[r];
 #pragma unroll
-      for (int i = 0; i < MAX_VCOLS; ++i)
+      for (int i = 0; i < VC; ++i)
         if (i < nvc) mine[2 + 64 * i + lane] = acc[r][i];
     }
     __syncthreads();
@@ -224,13 +269,13 @@ __global__ __launch_bounds__(64 * NW) void window_attn_wave_kernel(WindowAttnArg
       m[r] = M;
       l[r] *= f0;
 #pragma unroll
-      for (int i = 0; i < MAX_VCOLS; ++i) acc[r][i] *= f0;
+      for (int i = 0; i < VC; ++i) acc[r][i] *= f0;
       for (int w2 = 1; w2 < NW; ++w2) {
         const float* o = part + (w2 * REP + r) * pstride;
         const float f = expf(o[0] - M);       // a wave without tiles: exp(-inf) = 0
         l[r] += o[1] * f;
 #pragma unroll
-        for (int i = 0; i < MAX_VCOLS; ++i)
+        for (int i = 0; i < VC; ++i)
           if (i < nvc) acc[r][i] += o[2 + 64 * i + lane] * f;
       }
     }
@@ -250,7 +295,7 @@ __global__ __launch_bounds__(64 * NW) void window_attn_wave_kernel(WindowAttnArg
     const float inv = gate / l[r];
     T* o = reinterpret_cast<T*>(a.out) + ((long long)row * a.H + h) * a.dv;
 #pragma unroll
-    for (int i = 0; i < MAX_VCOLS; ++i) {
+    for (int i = 0; i < VC; ++i) {
       const int c = vcol<PAIR>(lane, i);
       if (i < nvc && c < a.dv) o[c] = (T)(acc[r][i] * inv * (a.gate_cols ? 1.f / (1.f + expf(-(float)gp[c])) : 1.f));
     }
@@ -262,7 +307,8 @@ void launch_wave_rep(const WindowAttnArgs& a, hipStream_t s) {
   dim3 grid(a.H / REP, a.T);
   const int nvc = PAIR ? 2 * ((a.dv + 127) / 128) : (a.dv + 63) / 64;
   const size_t lds = (size_t)(REP * a.dk + (NW > 1 ? NW * REP * (2 + 64 * nvc) : 0)) * sizeof(float);
-  window_attn_wave_kernel<T, NW, REP, PAIR><<<grid, 64 * NW, lds, s>>>(a);
+  if (nvc <= 2) window_attn_wave_kernel<T, NW, REP, PAIR, 2><<<grid, 64 * NW, lds, s>>>(a);
+  else window_attn_wave_kernel<T, NW, REP, PAIR, MAX_VCOLS><<<grid, 64 * NW, lds, s>>>(a);
 }
 
 template <typename T, int NW>
