@@ -466,11 +466,12 @@ void launch_mode(const DecayScanArgs& a, hipStream_t s) {
 
 }  // namespace
 
-// Is the call one the chunked form takes?  bf16 prompt steps of at least 8 tokens a run (below, a chunk's fixed cost is more
-// than the walk), up to 128 key channels, 16-byte aligned rows; mode 0 needs the 64-row tiles and the scratch.
+// Is the call one the chunked form takes?  bf16 prompt steps of at least 8 tokens a run, 48 in mode 0 with its second launch
+// (below, a chunk's fixed cost is more than the walk: 3 runs of 28 tokens, mode 0 35 us against 34, mode 1 15 against 28), up
+// to 128 key channels, 16-byte aligned rows; mode 0 needs the 64-row tiles and the scratch.
 bool decay_chunk_takes(const DecayScanArgs& a) {
   auto aligned = [](const void* p, long long ld) { return (uintptr_t)p % 16 == 0 && ld % 8 == 0; };
-  if (a.mode > 1 || !a.cu_q || a.T < 8LL * a.runs || a.N % 8 || a.N > 128) return false;
+  if (a.mode > 1 || !a.cu_q || a.T < (a.mode == 0 ? 48LL : 8LL) * a.runs || a.N % 8 || a.N > 128) return false;
   if (!aligned(a.q, a.ldq) || !aligned(a.k, a.ldk)) return false;
   return a.mode == 1 || (a.tiles && a.ntiles > 0 && a.ws && (uintptr_t)a.ws % 16 == 0);
 }
