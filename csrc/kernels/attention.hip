@@ -724,15 +724,17 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_rows_kernel(
 }  // namespace
 
 // Decode: a unit is a (sequence, kv head); contexts are cut so far that the workgroups just fill the chip, two 8-wave
-// workgroups on each of the 256 CUs (past it: 48 sequences x 8 kv heads, contexts around 250, one partition 20 us, two
-// 24).  The kernel replaced a one-wave-per-partition LDS-DMA streaming kernel and a one-wave-per-unit kernel; us for the
+// workgroups on each of the 256 CUs.  Between 256 and 384 units whole contexts would leave some CUs one workgroup and others
+// two: cut in three they run as two to three even rounds (304 units of 1514 tokens 64.8 -> 52.3 us, of 300 16.9 -> 14.5; 264
+// of 900 32.4 -> 31.6; 384 of 1000 49.8 -> 47.5, of 250 16.3 / 16.6); past that cutting costs more (480 of 600 34.4 -> 38.9).
+// The kernel replaced a one-wave-per-partition LDS-DMA streaming kernel and a one-wave-per-unit kernel; us for the
 // streaming / per-unit / this kernel, contexts spread by half around the mean and other weights read in between:
 //   1 sequence x 700 tokens, 8 kv heads   17.3 /  46 /  8.5      64 x 900      66 /  88 /  52  (236 MB: 4.6 TB/s)
 //   8 x 1100, 4 kv heads                  17.8 /  92 /  9.7      32 x 4000    148 /   - / 111
 //   5 x 5400, 4 kv heads                  28.7 /   - / 22.8      160 x 600    112 / 126 /  84
 //   48 x 60                                8.8 / 9.3 /  6.5      256 x 2000   428 / 370 / 335
 // Bound by the K/V stream from ~100 MB on, by four dependent round trips (context, K/V, publish, combine) below ~20 MB.
-constexpr int DECODE_UNITS = 512;
+constexpr int DECODE_UNITS = 512, DECODE_THIRDS = 384;
 
 void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache, const int* block_tables,
                         const int* ctx_lens, bf16* out, float* tmp_o, float* tmp_ml, int* counters, int num_seqs,
@@ -741,7 +743,8 @@ void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache,
   const float scale_log2 = scale * 1.4426950408889634f;
   const int G = Hq / Hkv;
   const int units = num_seqs * Hkv;  // (parts <= 512: attn_decode_unit's exact division)
-  const int parts = min(max_parts, max(1, DECODE_UNITS / units));
+  const int cut = units <= DECODE_UNITS / 2 ? DECODE_UNITS / units : units <= DECODE_THIRDS ? 3 : 1;
+  const int parts = min(max_parts, cut);
   const dim3 grid(num_seqs, Hkv, parts);
   const unsigned inv = (unsigned)((1ull << 32) / parts) + 1;  // (not used for one partition)
   auto run = [&](auto kern) {
