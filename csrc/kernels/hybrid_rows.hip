@@ -96,6 +96,57 @@ __global__ __launch_bounds__(BT) void residual_mix_norm_kernel(ResidualMixArgs a
   for (int c = threadIdx.x; c < d; c += BT) out[c] = (T)(xr[c] * r * (a.offset + a.w[c]));
 }
 
+// The same for widths of 8 to 8 NT in eights, bf16 out: a thread's eight columns stay in registers from the stream's load to the
+// norm's store (column by column, with the stream read back: 88 -> 44 us at 8100 x 2048, two bf16 summands).
+SYM_DEV void ld8f(const void* p, int f32, long long i, float* f) {
+  if (f32) load8f(reinterpret_cast<const float*>(p) + i, f);
+  else load8(reinterpret_cast<const bf16*>(p) + i, f);
+}
+__global__ __launch_bounds__(NT) void residual_mix_vec_kernel(ResidualMixArgs a) {
+  __shared__ float scratch[NT / 64];
+  const int c = 8 * threadIdx.x;
+  const long long o = (long long)blockIdx.x * a.d + c;
+  const bool on = c < a.d;
+  float x[8], sq = 0.f;
+  if (on) {
+    float s[8], t[8];
+    load8f(a.x + o, x);
+    ld8f(a.a, a.a_f32, o, s);
+    if (a.bias_a) {
+      load8f(a.bias_a + c, t);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[i] += t[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s[i] *= a.sa;
+    if (a.b) {
+      ld8f(a.b, a.b_f32, o, t);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[i] += a.sb * t[i];
+    }
+    if (a.c) {
+      ld8f(a.c, a.c_f32, o, t);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[i] += a.sc * t[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      x[i] += s[i];
+      sq += x[i] * x[i];
+    }
+    *reinterpret_cast<float4*>(a.x + o) = make_float4(x[0], x[1], x[2], x[3]);
+    *reinterpret_cast<float4*>(a.x + o + 4) = make_float4(x[4], x[5], x[6], x[7]);
+  }
+  if (!a.out) return;
+  const float r = 1.f / sqrtf(block_sum<NT>(sq, scratch) / (float)a.d + a.eps);
+  if (!on) return;
+  float w[8];
+  load8f(a.w + c, w);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i] = x[i] * r * (a.offset + w[i]);
+  store8(reinterpret_cast<bf16*>(a.out) + o, x);
+}
+
 template <typename T, int BT>
 __global__ __launch_bounds__(BT) void qkv_rope_cache_kernel(QkvRopeArgs a) {
   const int row = blockIdx.x;
@@ -178,6 +229,53 @@ __global__ __launch_bounds__(NT) void causal_conv_silu_kernel(ConvArgs a) {
   reinterpret_cast<T*>(a.out)[(long long)row * a.C + c] = (T)(acc * sigmoidf(acc));
 }
 
+// Prompt rows of four taps in bf16: grid (ceil(T / CR), ceil(C / 512)), a thread eight channels of CR rows, whose inputs stay
+// in registers for the four rows that take them (row by row and channel by channel every input was loaded four times in
+// 2-byte pieces: 230 -> 52 us at 8100 rows of 4352).  The branches at a run's first rows are uniform over the workgroup.
+constexpr int CR = 8;
+
+__global__ __launch_bounds__(64) void causal_conv_rows_kernel(ConvArgs a) {
+  const int r0 = blockIdx.x * CR, c = 8 * (blockIdx.y * 64 + threadIdx.x);
+  if (c >= a.C) return;
+  const bf16* x = reinterpret_cast<const bf16*>(a.xin) + c;
+  Pack8 xv[CR + 3], w[4];
+#pragma unroll
+  for (int i = 0; i < CR + 3; ++i)
+    xv[i].u = *reinterpret_cast<const uint4*>(x + (long long)min(max(r0 + i - 3, 0), a.T - 1) * a.ldx);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i].u = *reinterpret_cast<const uint4*>(reinterpret_cast<const bf16*>(a.w) + 4 * c + 8 * i);
+  float b[8];
+  load8f(a.b + c, b);
+#pragma unroll
+  for (int r = 0; r < CR; ++r) {
+    const int row = r0 + r;
+    if (row >= a.T) return;
+    const int s0 = a.cu_q[a.row_seq[row]], j = row - s0;
+    Pack8 v[4];                            // positions 0..3 back
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = xv[r + 3 - i];
+    if (j < 3) {
+      const int pr = a.prev_row[s0];
+      const bf16* st = pr <= -2 ? reinterpret_cast<const bf16*>(a.state) + (long long)(-(pr + 2)) * a.state_stride : nullptr;
+#pragma unroll
+      for (int i = 1; i < 4; ++i)
+        if (i > j) {
+          if (st) v[i].u = *reinterpret_cast<const uint4*>(st + (long long)(3 - (i - j)) * a.C + c);
+          else v[i].u = uint4{0, 0, 0, 0};
+        }
+    }
+    Pack8 o;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      float acc = b[k];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc += (float)w[k >> 1].h[4 * (k & 1) + 3 - i] * (float)v[i].h[k];
+      o.h[k] = (bf16)(acc * sigmoidf(acc));
+    }
+    *reinterpret_cast<uint4*>(reinterpret_cast<bf16*>(a.out) + (long long)row * a.C + c) = o.u;
+  }
+}
+
 constexpr int MAX_TAPS = 16;
 
 // grid (runs, ceil(C / NT)): one thread per (run, channel) owns that channel of the run's state slot
@@ -220,6 +318,22 @@ __global__ __launch_bounds__(NT) void relu_sq_kernel(const T* __restrict__ a, lo
     const float v = fmaxf((float)a[r * lda + c], 0.f);
     out[i] = (T)(v * v);
   }
+}
+
+// eight columns per thread (2-byte loads: 87 -> 40 us at 8100 x 8192)
+__global__ __launch_bounds__(NT) void relu_sq_vec_kernel(const bf16* __restrict__ a, long long lda, bf16* __restrict__ out, int R,
+                                                         int F) {
+  const unsigned per = F / 8;
+  const unsigned i = blockIdx.x * NT + threadIdx.x, r = i / per, c = 8 * (i - r * per);
+  if (r >= (unsigned)R) return;
+  Pack8 v;
+  v.u = *reinterpret_cast<const uint4*>(a + (long long)r * lda + c);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float f = fmaxf((float)v.h[k], 0.f);
+    v.h[k] = (bf16)(f * f);
+  }
+  *reinterpret_cast<uint4*>(out + (long long)r * F + c) = v.u;
 }
 
 template <typename T>
@@ -708,6 +822,12 @@ void launch_rms_norm_rows(const float* x, const long long* rows, const float* w,
 
 void launch_residual_mix_norm(const ResidualMixArgs& a, int f32, hipStream_t s) {
   if (a.T <= 0) return;
+  auto odd = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 != 0; };
+  if (!f32 && a.T > 512 && a.d % 8 == 0 && a.d <= 8 * NT && !odd(a.x) && !odd(a.a) && !odd(a.bias_a) && !odd(a.b) && !odd(a.c) &&
+      !odd(a.w) && !odd(a.out)) {
+    residual_mix_vec_kernel<<<a.T, NT, 0, s>>>(a);
+    return;
+  }
   if (wide_rows(a.T, a.d)) {
     DISPATCH_T(f32, (residual_mix_norm_kernel<T, 1024><<<a.T, 1024, 0, s>>>(a));)
   } else {
@@ -742,6 +862,13 @@ void launch_gated_group_norm(const float* y, const void* gate, long long ldg, co
 
 void launch_causal_conv_silu(const ConvArgs& a, int f32, hipStream_t s) {
   if (a.T <= 0) return;
+  auto rows16 = [](const void* p, long long ld) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 8 == 0; };
+  // (below 256 rows too few workgroups to gain: 84 rows 5 us either way)
+  if (!f32 && a.cu_q && a.taps == 4 && a.T >= 256 && a.C % 8 == 0 && rows16(a.xin, a.ldx) && rows16(a.state, a.state_stride) &&
+      rows16(a.w, 0) && rows16(a.out, 0) && rows16(a.b, 0)) {
+    causal_conv_rows_kernel<<<dim3((a.T + CR - 1) / CR, (a.C + 511) / 512), 64, 0, s>>>(a);
+    return;
+  }
   dim3 grid(a.T, (a.C + NT - 1) / NT);
   DISPATCH_T(f32, causal_conv_silu_kernel<T><<<grid, NT, 0, s>>>(a);)
 }
@@ -754,6 +881,12 @@ void launch_conv_state_update(const ConvArgs& a, int f32, hipStream_t s) {
 
 void launch_relu_sq(const void* a, long long lda, void* out, int R, int F, int f32, hipStream_t s) {
   if (R <= 0) return;
+  if (!f32 && F > 0 && F % 8 == 0 && lda % 8 == 0 && (reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(out)) % 16 == 0 &&
+      (long long)R * F < (1ll << 33)) {
+    const long long n = (long long)R * (F / 8);
+    relu_sq_vec_kernel<<<(unsigned)((n + NT - 1) / NT), NT, 0, s>>>((const bf16*)a, lda, (bf16*)out, R, F);
+    return;
+  }
   DISPATCH_T(f32, relu_sq_kernel<T><<<ew_grid((long long)R * F), NT, 0, s>>>((const T*)a, lda, (T*)out, R, F);)
 }
 

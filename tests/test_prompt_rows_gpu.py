@@ -1,0 +1,72 @@
+"""The prompt forms of the row kernels (short convolution, squared ReLU, residual + norm) against 64-bit rows, on both sides of
+the conditions that choose them."""
+import pytest
+import torch
+
+from symmetry_amd import ops
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+@pytest.mark.parametrize("C", [8, 24, 520, 1032, 13])
+@pytest.mark.parametrize("taps", [4, 3])
+@pytest.mark.parametrize("lens", [[300], [1, 2, 3, 4, 5, 250], [7, 130, 129], [255]])
+def test_causal_conv(C, taps, lens):
+    """Runs that begin anywhere in a group of 8 rows, with and without saved inputs; odd widths and other tap counts take the
+    general kernel.  Four products in fp32 and one rounding to bf16 (2^-8 relative with silu's slope <= 1.1)."""
+    print("causal_conv_silu", C, taps, lens, flush=True)
+    torch.manual_seed(C + len(lens))
+    T, S, i32 = sum(lens), len(lens), torch.int32
+    z = torch.randn(T, C + 8).to(BF16)
+    x, w, b = z[:, 8:], torch.randn(C, taps).to(BF16), torch.randn(C)
+    state = torch.randn(S + 1, taps - 1, C).to(BF16)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist())
+    prev = torch.full((T,), -1)
+    want = torch.zeros(T, C, dtype=torch.float64)
+    for s, n in enumerate(lens):
+        old = state[s].double() if s % 2 == 0 else torch.zeros(taps - 1, C, dtype=torch.float64)
+        prev[cu[s]] = -(s + 2) if s % 2 == 0 else -1
+        seq = torch.cat([old, x[cu[s]:cu[s + 1]].double()])
+        y = b.double() + sum(w[:, i].double() * seq[i:i + n] for i in range(taps))
+        want[cu[s]:cu[s + 1]] = y / (1 + torch.exp(-y))
+    zd = z.cuda()
+    out = torch.full((T, C), 7.0, dtype=BF16, device="cuda")
+    ops.causal_conv_silu(zd[:, 8:], w.cuda(), b.cuda(), state.cuda(), cu.to(i32).cuda(),
+                         torch.repeat_interleave(torch.arange(S), torch.tensor(lens)).to(i32).cuda(), prev.to(i32).cuda(), S, out)
+    err = (out.cpu().double() - want).abs()
+    assert (err <= 2.0 ** -8 * want.abs() + 2e-5).all(), float(err.max())
+
+
+@pytest.mark.parametrize("R,F,pad", [(1, 8, 0), (33, 264, 8), (257, 1032, 16), (40, 12, 0), (9, 64, 3)])
+def test_relu_sq(R, F, pad):
+    torch.manual_seed(F)
+    z = torch.randn(R, F + pad).to(BF16).cuda()
+    z[0, 0], z[R - 1, F - 1] = float("inf"), float("-inf")
+    out = torch.empty(R, F, dtype=BF16, device="cuda")
+    ops.relu_sq(z[:, :F], out)
+    assert torch.equal(out, (z[:, :F].float().clamp_min(0) ** 2).to(BF16))
+
+
+@pytest.mark.parametrize("T", [513, 512])
+@pytest.mark.parametrize("d", [8, 264, 2048, 2056, 100])
+@pytest.mark.parametrize("parts", ["a", "ab", "abc"])
+def test_residual_mix(T, d, parts):
+    """fp32 stream to 2^-22 of its summands; the norm's sum of d squares to 2^-20, its output rounded to bf16."""
+    print("residual_mix_norm", T, d, parts, flush=True)
+    torch.manual_seed(d)
+    x, w, bias = torch.randn(T, d).cuda(), torch.randn(d).cuda(), torch.randn(d).cuda()
+    a, b, c = torch.randn(T, d).to(BF16).cuda(), torch.randn(T, d).cuda(), torch.randn(T, d).to(BF16).cuda()
+    b_, c_ = (b if "b" in parts else None), (c if "c" in parts else None)
+    s = 0.5 * (a.double() + bias.double())
+    size = 0.5 * (a.double().abs() + bias.double().abs()) + x.double().abs()
+    if b_ is not None:
+        s, size = s + 0.25 * b.double(), size + 0.25 * b.double().abs()
+    if c_ is not None:
+        s, size = s - 2.0 * c.double(), size + 2.0 * c.double().abs()
+    want = x.double() + s
+    out = torch.full((T, d), 7.0, dtype=BF16, device="cuda")
+    ops.residual_mix_norm(x, a, 0.5, bias, b_, 0.25, c_, -2.0, w, 1e-5, 1.0, out)
+    assert ((x.double() - want).abs() <= 2.0 ** -22 * size).all()
+    n = want / (want.pow(2).mean(1, keepdim=True) + 1e-5).sqrt() * (1.0 + w.double())
+    assert ((out.double() - n).abs() <= 2.0 ** -8 * n.abs() + 2e-5).all()
