@@ -208,6 +208,35 @@ __global__ __launch_bounds__(BT) void gated_group_norm_kernel(const float* __res
   }
 }
 
+// The same for prompt rows in bf16, group <= 8 BT in eights: a thread's eight columns and their gates stay in registers (column
+// by column, the gate computed twice: 105 -> 47 us at 8100 rows of 4096).
+template <int BT>
+__global__ __launch_bounds__(BT) void gated_group_norm_vec_kernel(const float* __restrict__ y, const bf16* __restrict__ gate,
+                                                                  long long ldg, const float* __restrict__ w, int wlen,
+                                                                  float eps, int group, int gate_first, int sigmoid,
+                                                                  bf16* __restrict__ out, int C) {
+  __shared__ float scratch[BT / 64];
+  const int c = 8 * threadIdx.x, c0 = blockIdx.y * group + c;
+  const bool on = c < group;
+  float v[8], g[8], wv[8], sq = 0.f;
+  if (on) {
+    load8f(y + (long long)blockIdx.x * C + c0, v);
+    load8(gate + (long long)blockIdx.x * ldg + c0, g);
+    load8f(w + c0 % wlen, wv);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      g[i] = sigmoid ? sigmoidf(g[i]) : silu_exact(g[i]);
+      if (gate_first) v[i] *= g[i];
+      sq += v[i] * v[i];
+    }
+  }
+  const float r = 1.f / sqrtf(block_sum<BT>(sq, scratch) / (float)group + eps);
+  if (!on) return;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = gate_first ? v[i] * r * wv[i] : v[i] * r * wv[i] * g[i];
+  store8(out + (long long)blockIdx.x * C + c0, v);
+}
+
 // grid (T, ceil(C / NT)): one thread per (row, channel)
 template <typename T>
 __global__ __launch_bounds__(NT) void causal_conv_silu_kernel(ConvArgs a) {
@@ -848,6 +877,17 @@ void launch_gated_group_norm(const float* y, const void* gate, long long ldg, co
                              int group, int gate_first, int sigmoid, void* out, int T_, int C, int f32, hipStream_t s) {
   if (T_ <= 0) return;
   dim3 grid(T_, C / group);
+  const uintptr_t at = reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(w) |
+                       reinterpret_cast<uintptr_t>(out);
+  if (!f32 && T_ > 512 && group > 256 && group <= 4096 && group % 8 == 0 && wlen % 8 == 0 && ldg % 8 == 0 && at % 16 == 0) {
+    if (group <= 2048)
+      gated_group_norm_vec_kernel<256><<<grid, 256, 0, s>>>(y, (const bf16*)gate, ldg, w, wlen, eps, group, gate_first, sigmoid,
+                                                            (bf16*)out, C);
+    else
+      gated_group_norm_vec_kernel<512><<<grid, 512, 0, s>>>(y, (const bf16*)gate, ldg, w, wlen, eps, group, gate_first, sigmoid,
+                                                            (bf16*)out, C);
+    return;
+  }
   if (group <= 256) {
     DISPATCH_T(f32, (gated_group_norm_kernel<T, 64><<<grid, 64, 0, s>>>(y, (const T*)gate, ldg, w, wlen, eps, group,
                                                                           gate_first, sigmoid, (T*)out, C));)

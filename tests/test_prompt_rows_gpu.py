@@ -1,4 +1,5 @@
-"""The prompt forms of the row kernels (short convolution, squared ReLU, residual + norm) against 64-bit rows, on both sides of
+"""The prompt forms of the row kernels (short convolution, squared ReLU, residual + norm, gated
+group norm) against 64-bit rows, on both sides of
 the conditions that choose them."""
 import pytest
 import torch
@@ -69,4 +70,26 @@ def test_residual_mix(T, d, parts):
     ops.residual_mix_norm(x, a, 0.5, bias, b_, 0.25, c_, -2.0, w, 1e-5, 1.0, out)
     assert ((x.double() - want).abs() <= 2.0 ** -22 * size).all()
     n = want / (want.pow(2).mean(1, keepdim=True) + 1e-5).sqrt() * (1.0 + w.double())
+    assert ((out.double() - n).abs() <= 2.0 ** -8 * n.abs() + 2e-5).all()
+
+
+@pytest.mark.parametrize("T", [513, 512])
+@pytest.mark.parametrize("groups,group,wlen", [(2, 264, 528), (1, 2048, 2048), (3, 2056, 2056), (1, 4096, 4096), (2, 300, 12),
+                                               (1, 4104, 4104)])
+@pytest.mark.parametrize("gate_first,sigmoid", [(True, False), (False, True)])
+def test_gated_group_norm(T, groups, group, wlen, gate_first, sigmoid):
+    """The norm's sum of a group's squares to 2^-20, the gate to 2^-20, the output rounded to bf16."""
+    print("gated_group_norm", T, groups, group, gate_first, sigmoid, flush=True)
+    torch.manual_seed(group)
+    C = groups * group
+    z = torch.randn(T, C + 8).to(BF16).cuda()
+    y, w, gate = torch.randn(T, C).cuda(), torch.randn(wlen).cuda(), z[:, 8:]
+    out = torch.full((T, C), 7.0, dtype=BF16, device="cuda")
+    ops.gated_group_norm(y, gate, w, 1e-5, group, gate_first, out, sigmoid=sigmoid)
+    g = gate.double().sigmoid()
+    g = g if sigmoid else gate.double() * g
+    v = y.double() * g if gate_first else y.double()
+    n = v.view(T, groups, group)
+    n = (n / (n.pow(2).mean(2, keepdim=True) + 1e-5).sqrt()).view(T, C) * w.double().repeat(C // wlen)
+    n = n if gate_first else n * g
     assert ((out.double() - n).abs() <= 2.0 ** -8 * n.abs() + 2e-5).all()
