@@ -757,10 +757,12 @@ void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache,
 }
 
 // Workgroups of the 64-row x 4-head kernel up to which the row kernel takes a prompt step: below, most CUs would idle; above,
-// K/V read once per head costs more than it fills.  us, 64-row kernel / row kernel (query rows behind a context, 32 heads):
-//   24: 137 of 1200   42 / 13.6       48: 384 of 2000  65 / 34      96: 768 of 4000   133 / 106     128: 1024 of 1024  38 / 39
-//   32: 256 of 8000  233 / 69         64: 512 of 512   23 / 16      96: 1500 of 1500   49 / 35      128: 16 x 60 of 600  30 / 45
-constexpr int ROWS_WGS = 96;
+// K/V read once per head costs more than it fills, first for batches of short contexts.  us, 64-row kernel / row kernel (query
+// rows behind a context):
+//   24: 137 of 1200   42 / 13.6      48: 384 of 2000  65 / 34       64: 4 x 128 of 128  12.6 / 11.3    96: 768 of 4000   133 / 106
+//   32: 256 of 8000  233 / 69        48: 6 x 40 of 300  16.5 / 15.6   64: 8 x 60 of 600   27 / 21        96: 6 x 128 of 128  12.8 / 15.9
+//   48: 3 x 128 of 128  12.2 / 10.8  64: 512 of 512   23 / 16       64: 8 x 100, 4 kv heads  10.7 / 10.6   96: 12 x 60 of 600  29 / 31
+constexpr int ROWS_WGS = 64;
 
 void launch_attn_prefill(const bf16* q, const bf16* k_cache, const bf16* v_cache, const int* block_tables,
                          const int* ctx_lens, const int* cu_q, const int* tiles, int num_tiles, bf16* out, int Hq,

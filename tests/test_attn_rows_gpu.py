@@ -16,8 +16,8 @@ STEPS = [
     [(33, 33), (64, 700), (65, 300)],
     [(137, 1200)],
     [(3, 5000), (60, 60)],
-    [(64 * 12, 800)],           # 96 workgroups at 8 kv heads: the last of the row kernel
-    [(64 * 12 + 1, 800)],       # one tile more: the 64-row kernel
+    [(64 * 8, 800)],            # 64 workgroups at 8 kv heads: the last of the row kernel
+    [(64 * 8 + 1, 800)],        # one tile more: the 64-row kernel
 ]
 
 
