@@ -44,7 +44,7 @@ def main():
     ap.add_argument("--span", type=int, default=0, help="block-table width in tokens (the graph's context "
                     "bucket; 0: just the context)")
     ap.add_argument("--wave", type=int, nargs="+", default=[-1],
-                    help="attn_wave min-units settings to compare (-1: leave the default; 0: never; 1: always)")
+                    help="attn_wave settings to pass (one kernel takes every step: they change nothing)")
     ap.add_argument("--heads", type=int, nargs=2, default=[32, 8], metavar=("HQ", "HKV"),
                     help="query / kv heads (one TP rank's shard: 4 1 for Llama-3-8B at TP=8, 8 1 for 70B)")
     args = ap.parse_args()
