@@ -325,7 +325,7 @@ void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v,
     dtype(*tiles, at::kInt, "tiles");
     dtype(*ws, at::kFloat, "ws");
     TORCH_CHECK(tiles->dim() == 2 && tiles->size(1) == 2 && tiles->size(0) <= (1 << 30), "decay_scan: tiles [n, 2]");
-    TORCH_CHECK(ws->numel() >= T * H * (32 + N), "decay_scan: ws [T, H, 32 + N]");
+    TORCH_CHECK(ws->numel() >= T * H * (32 + 2 * N), "decay_scan: ws [T, H, 32 + 2 N]");
     a.tiles = ptr<int>(*tiles), a.ntiles = (int)tiles->size(0);
     a.ws = ptr<float>(*ws);
   }

@@ -64,10 +64,13 @@ SYM_DEV bf16x8 pair4(const bf16* p) {
   return r.v;
 }
 
-SYM_DEV int ws_cols(int N) { return C + N; }   // mode 0's scratch per (row, head): row of A | G
+// mode 0's scratch per (row, head): row of A | 2^(G_i) | k_i 2^(G_C - G_i)
+SYM_DEV int ws_cols(int N) { return C + 2 * N; }
 
-// ---- mode 0: running sums G and scores A of every chunk, grid (64-row tiles x 2 chunks, heads) --------------------------
-// Inside the two diagonal 16 x 16 tiles the exponents of differences are taken per (i, j, channel) on the vector unit; the
+// ---- mode 0: decays and scores A of every chunk, grid (64-row tiles x 2 chunks, heads) ----------------------------------
+// G is held as a pair of floats: what counts are its differences, and once a few tokens of a chunk forget hard, G is in the
+// hundreds and a float's differences of the tokens behind them keep few digits (a tenth of the tokens at -100 with tau 1: 9e-6
+// of the output's norm from G alone, the token walk 1e-7).  Inside the two diagonal 16 x 16 tiles the exponents of differences are taken per (i, j, channel) on the vector unit; the
 // tile below them factors at the end of the first half, 2^(G_i - G_15) 2^(G_15 - G_j), both exponents <= 0, and is a matrix
 // product.
 template <int NN>
@@ -76,8 +79,10 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* kS = reinterpret_cast<float*>(smem);  // [C][LD]
   float* qS = kS + C * LD;                     // [C][LD]
-  float* GS = qS + C * LD;                     // [C][LD]
-  float* XS = GS + C * LD;                     // [4][C][LT] partial scores
+  float* GS = qS + C * LD;                     // [C][LD] G: high part
+  float* LS = GS + C * LD;                     // [C][LD] low part
+  float* XS = kS;                              // [4][C][LT] partial scores, when the others have been read
+  static_assert(LT <= LD, "the partial scores fit");
   const int N = a.N, h = blockIdx.y, tile = blockIdx.x >> 1, sub = blockIdx.x & 1;
   const int seq = a.tiles[2 * tile], off = a.tiles[2 * tile + 1];
   const int q0 = a.cu_q[seq], qlen = a.cu_q[seq + 1] - q0;
@@ -104,57 +109,70 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
   float* ws = a.ws + (r0 * a.H + h) * wc;
   const long long wrow = (long long)a.H * wc;
   if (tid < NP) {
-    float g = 0.f;
+    double g = 0.;
 #pragma unroll 8
     for (int tt = 0; tt < C; ++tt) {
-      g += GS[tt * LD + tid];
-      GS[tt * LD + tid] = g;
-      if (tt < nt && tid < N) ws[tt * wrow + C + tid] = g;
+      g += (double)GS[tt * LD + tid];
+      const float hi = (float)g;
+      GS[tt * LD + tid] = hi;
+      LS[tt * LD + tid] = (float)(g - (double)hi);
     }
   }
   __syncthreads();
+#pragma unroll 4
+  for (int i = tid; i < C * NP; i += NT) {     // (G stands still past the run's end, so the last row's is G_C)
+    const int tt = i / NP, n = i % NP;
+    if (tt >= nt || n >= N) continue;
+    const float gi = GS[tt * LD + n], li = LS[tt * LD + n];
+    ws[tt * wrow + C + n] = __builtin_amdgcn_exp2f(gi);
+    ws[tt * wrow + C + N + n] = kS[tt * LD + n] * exp2_neg((GS[(C - 1) * LD + n] - gi) + (LS[(C - 1) * LD + n] - li));
+  }
   const int col = lane & 15, g = lane >> 4;
-  {  // rows 16 .., columns .. 15: the waves take the channel tiles in turn
-    f32x4 d = {0.f, 0.f, 0.f, 0.f};
-    for (int t = wave; t < NN; t += 4) {
-      const int c = 16 * t + 4 * g;
-      const f32x4 mid = lds4(GS + 15 * LD + c), gi = lds4(GS + (16 + col) * LD + c), gj = lds4(GS + col * LD + c);
-      const f32x4 qi = lds4(qS + (16 + col) * LD + c), kj = lds4(kS + col * LD + c);
+  // rows 16 .., columns .. 15: the waves take the channel tiles in turn
+  f32x4 d = {0.f, 0.f, 0.f, 0.f};
+  for (int t = wave; t < NN; t += 4) {
+    const int c = 16 * t + 4 * g;
+    const f32x4 mh = lds4(GS + 15 * LD + c), gi = lds4(GS + (16 + col) * LD + c), gj = lds4(GS + col * LD + c);
+    const f32x4 ml = lds4(LS + 15 * LD + c), li = lds4(LS + (16 + col) * LD + c), lj = lds4(LS + col * LD + c);
+    const f32x4 qi = lds4(qS + (16 + col) * LD + c), kj = lds4(kS + col * LD + c);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) d = mfma4(qi[r] * exp2_neg(gi[r] - mid[r]), kj[r] * exp2_neg(mid[r] - gj[r]), d);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) XS[(wave * C + 16 + 4 * g + r) * LT + col] = d[r];
+    for (int r = 0; r < 4; ++r)
+      d = mfma4(qi[r] * exp2_neg((gi[r] - mh[r]) + (li[r] - ml[r])), kj[r] * exp2_neg((mh[r] - gj[r]) + (ml[r] - lj[r])), d);
   }
-  {  // diagonal tiles: wave (channel half, tile), a 2 x 2 block of (i, j) per lane
-    constexpr int NH = NP / 2;
-    const int half = wave >> 1, dt = wave & 1, ib = lane >> 3, jb = lane & 7;
-    const int i0 = 16 * dt + 2 * ib, j0 = 16 * dt + 2 * jb;
-    float s[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-    if (jb <= ib) {
+  // diagonal tiles: wave (channel half, tile), a 2 x 2 block of (i, j) per lane
+  constexpr int NH = NP / 2;
+  const int half = wave >> 1, dt = wave & 1, ib = lane >> 3, jb = lane & 7;
+  const int i0 = 16 * dt + 2 * ib, j0 = 16 * dt + 2 * jb;
+  float s[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+  if (jb <= ib) {
 #pragma unroll 2
-      for (int c = NH * half; c < NH * (half + 1); c += 4) {
-        f32x4 qi[2], gi[2], kj[2], gj[2];
+    for (int c = NH * half; c < NH * (half + 1); c += 4) {
+      f32x4 qi[2], gi[2], li[2], kj[2], gj[2], lj[2];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          qi[e] = lds4(qS + (i0 + e) * LD + c);
-          gi[e] = lds4(GS + (i0 + e) * LD + c);
-          kj[e] = lds4(kS + (j0 + e) * LD + c);
-          gj[e] = lds4(GS + (j0 + e) * LD + c);
-        }
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-#pragma unroll
-          for (int f = 0; f < 2; ++f)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) s[e][f] += qi[e][r] * (kj[f][r] * exp2_neg(gi[e][r] - gj[f][r]));
+      for (int e = 0; e < 2; ++e) {
+        qi[e] = lds4(qS + (i0 + e) * LD + c);
+        gi[e] = lds4(GS + (i0 + e) * LD + c);
+        li[e] = lds4(LS + (i0 + e) * LD + c);
+        kj[e] = lds4(kS + (j0 + e) * LD + c);
+        gj[e] = lds4(GS + (j0 + e) * LD + c);
+        lj[e] = lds4(LS + (j0 + e) * LD + c);
       }
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            s[e][f] += qi[e][r] * (kj[f][r] * exp2_neg((gi[e][r] - gj[f][r]) + (li[e][r] - lj[f][r])));
     }
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-#pragma unroll
-      for (int f = 0; f < 2; ++f) XS[(half * C + i0 + e) * LT + j0 + f] = s[e][f];
   }
+  __syncthreads();                             // (the rows have been read: their place takes the partial scores)
+#pragma unroll
+  for (int r = 0; r < 4; ++r) XS[(wave * C + 16 + 4 * g + r) * LT + col] = d[r];
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+#pragma unroll
+    for (int f = 0; f < 2; ++f) XS[(half * C + i0 + e) * LT + j0 + f] = s[e][f];
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < C * C / NT; ++u) {
@@ -202,8 +220,8 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
   constexpr int GR = NP / 8, TSTEP = NT / GR, PASS = (C + TSTEP - 1) / TSTEP;
   const int c8 = 8 * (tid % GR), tt0 = tid / GR;
   const bool nin = c8 < N && tt0 < C;                   // (N is a multiple of 8)
-  Pack8 rq[PASS], rk[PASS];
-  f32x4 rg[MODE == 0 ? PASS : 1][2], gl[2], ra;
+  Pack8 rq[PASS], rk[MODE == 1 ? PASS : 1];
+  f32x4 rp[MODE == 0 ? PASS : 1][2], ry[MODE == 0 ? PASS : 1][2], pl, ra;   // mode 0: 2^(G_i), k_i 2^(G_C - G_i), 2^(G_C)
   float rdt = 0.f;
   bf16 vn[8];
   auto fetch = [&](int c) {
@@ -213,17 +231,19 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
       const int tt = tt0 + TSTEP * u;
       const bool in = nin && tt < nt;
       rq[u].u = in ? *reinterpret_cast<const uint4*>(q + (t0 + tt) * a.ldq + c8) : make_uint4(0, 0, 0, 0);
-      rk[u].u = in ? *reinterpret_cast<const uint4*>(k + (t0 + tt) * a.ldk + c8) : make_uint4(0, 0, 0, 0);
       if constexpr (MODE == 0) {
-        const float* G = ws + (t0 + tt) * wrow + C + c8;
-        rg[u][0] = in ? lds4(G) : f32x4{0.f, 0.f, 0.f, 0.f};
-        rg[u][1] = in ? lds4(G + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+        const float* x = ws + (t0 + tt) * wrow + C + c8;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          rp[u][i] = in ? lds4(x + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+          ry[u][i] = in ? lds4(x + N + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      } else {
+        rk[u].u = in ? *reinterpret_cast<const uint4*>(k + (t0 + tt) * a.ldk + c8) : make_uint4(0, 0, 0, 0);
       }
     }
     if constexpr (MODE == 0) {
-      const float* G = ws + (t0 + nt - 1) * wrow + C + c8;
-      gl[0] = nin ? lds4(G) : f32x4{0.f, 0.f, 0.f, 0.f};
-      gl[1] = nin ? lds4(G + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+      pl = 4 * tid < N ? lds4(ws + (t0 + nt - 1) * wrow + C + 4 * tid) : f32x4{0.f, 0.f, 0.f, 0.f};
       ra = tid / 8 < nt ? lds4(ws + (t0 + tid / 8) * wrow + 4 * (tid % 8)) : f32x4{0.f, 0.f, 0.f, 0.f};
     } else if (tid < C) {
       rdt = tid < nt ? (float)dt[(long long)(t0 + tid) * a.ldd] + a.dbias[h] : 0.f;
@@ -252,14 +272,10 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
 #pragma unroll
         for (int i = 0; i < 8; ++i) st[oT + (c8 + i) * LT + tt] = rk[u].h[i];
       } else {
-        f32x4 x[2], y[2];
+        f32x4 x[2];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float gi = rg[u][i >> 2][i & 3];
-          x[i >> 2][i & 3] = (float)rq[u].h[i] * __builtin_amdgcn_exp2f(gi);
-          y[i >> 2][i & 3] = (float)rk[u].h[i] * exp2_neg(gl[i >> 2][i & 3] - gi);   // (past the run's end: k = 0)
-        }
-        const Parts sx = split(x[0], x[1]), sy = split(y[0], y[1]);
+        for (int i = 0; i < 8; ++i) x[i >> 2][i & 3] = (float)rq[u].h[i] * rp[u][i >> 2][i & 3];
+        const Parts sx = split(x[0], x[1]), sy = split(ry[u][0], ry[u][1]);
         *reinterpret_cast<bf16x8*>(st + tt * LQ + c8) = sx.h;
         *reinterpret_cast<bf16x8*>(st + (C + tt) * LQ + c8) = sx.m;
         *reinterpret_cast<bf16x8*>(st + (2 * C + tt) * LQ + c8) = sx.l;
@@ -273,10 +289,7 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
     }
     if constexpr (MODE == 0) {
       *reinterpret_cast<f32x4*>(fs + (tid / 8) * LT + 4 * (tid % 8)) = ra;
-      if (tt0 == 0) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) fs[C * LT + c8 + i] = __builtin_amdgcn_exp2f(gl[i >> 2][i & 3]);
-      }
+      if (4 * tid < NP) *reinterpret_cast<f32x4*>(fs + C * LT + 4 * tid) = pl;
     } else if (wave == 0) {
       // running sum over the chunk's tokens as a pair of floats: with step sizes that forget in a few tokens the sum grows
       // to hundreds, and the differences of neighbours, which are what counts, would keep few of its digits
@@ -443,7 +456,7 @@ void launch_chunks(const DecayScanArgs& a, hipStream_t s) {
   constexpr int NP = 32 * NB, LQ = NP + 8, PL = MODE == 0 ? 3 : 1;
   constexpr int elems = PL * C * LQ + (MODE == 1 ? C * LQ : 0) + PL * NP * LT;
   constexpr int lds = 2 * (elems * 2 + (MODE == 0 ? C * LT + NP : 3 * C) * 4);
-  constexpr int prep = (3 * C * (NP + 4) + 4 * C * LT) * 4;
+  constexpr int prep = 4 * C * (NP + 4) * 4;
   static const bool raised = [] {
     const auto raise = [](const void* f, int bytes) {
       if (bytes > 64 * 1024) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);

@@ -266,7 +266,7 @@ struct DecayScanArgs {
   const int* save_slot;
   int runs, T;
   float* out;           // [T][H][P]
-  // chunked form (decay_chunk.hip), mode 0: 64-row tiles (run, first row), and fp32 scratch [T][H][32 + N]
+  // chunked form (decay_chunk.hip), mode 0: 64-row tiles (run, first row), and fp32 scratch [T][H][32 + 2 N]
   const int* tiles;
   int ntiles;
   float* ws;

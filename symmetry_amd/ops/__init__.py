@@ -881,8 +881,9 @@ def decay_scan(mode, q, k, v, dz, dbias, dparam, skip, q_scale, H, N, P, hpg, st
 
 
 def decay_ws_cols(N: int) -> int:
-    """Columns of decay_scan's chunk scratch per row and head: a score row and the channels' running decays."""
-    return 32 + N
+    """Columns of decay_scan's chunk scratch per row and head: a score row, the channels' decays since the chunk's start and the
+    keys decayed to its end."""
+    return 32 + 2 * N
 
 
 def memory_norm_gate(y, m, gate, w, eps, out):

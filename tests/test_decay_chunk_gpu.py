@@ -24,54 +24,92 @@ def _walk(q, k, v, a, b, S0, lens, skip):
     return o, torch.stack(ends)
 
 
+SHAPES = [(3, 128, 80, 3, [33, 64, 5, 97, 1, 32]), (4, 64, 64, 2, [100, 31]), (2, 24, 16, 1, [40, 41]), (2, 8, 70, 2, [8]),
+          (2, 72, 70, 2, [200]), (2, 32, 130, 1, [63, 65])]
+
+
+class _Case:
+    """Runs of the given lengths whose q, k and v are column ranges of one projection; every third run is a sequence's first."""
+
+    def __init__(self, gpu, mode, H, N, P, G, lens, tau=16.0):
+        g = torch.Generator(device=gpu).manual_seed(H * N + P)
+        T, R = sum(lens), len(lens)
+
+        def rnd(*s):
+            return torch.randn(*s, device=gpu, generator=g)
+
+        z = rnd(T, 2 * G * N + H * P).bfloat16()
+        self.q, self.k, self.v = z[:, :G * N], z[:, G * N:2 * G * N], z[:, 2 * G * N:]
+        cols = H * N if mode == ops.DECAY_CHANNEL_GATE else H
+        self.dz, self.db = rnd(T, cols).bfloat16(), rnd(cols) + (3.0 if mode == ops.DECAY_CHANNEL_GATE else -2.0)
+        self.par = tau if mode == ops.DECAY_CHANNEL_GATE else torch.log(0.05 + 0.5 * torch.rand(H, device=gpu, generator=g))
+        self.skip, self.scale = rnd(H), 0.37
+        self.state = rnd(2 * R, H, N, P)
+        self.fresh = [i for i in range(R) if i % 3 == 2]
+        prev, save = [], []
+        for i, n in enumerate(lens):
+            prev += [-1 if i in self.fresh else -(i + 2)] + [0] * (n - 1)
+            save += [-1] * (n - 1) + [R + i]
+        i32 = dict(device=gpu, dtype=torch.int32)
+        self.prev, self.save = torch.tensor(prev, **i32), torch.tensor(save, **i32)
+        self.cu = torch.tensor([sum(lens[:i]) for i in range(R + 1)], **i32)
+        self.tiles = torch.tensor([(i, r) for i, n in enumerate(lens) for r in range(0, n, 64)] + [(0, 1 << 24)], **i32)
+        self.ws = torch.full((T, H, ops.decay_ws_cols(N)), float("nan"), device=gpu)
+        self.mode, self.H, self.N, self.P, self.G, self.lens, self.T, self.R = mode, H, N, P, G, lens, T, R
+
+    def exact(self):
+        H, N, P, G, T = self.H, self.N, self.P, self.G, self.T
+        head = torch.arange(H, device=self.q.device) // (H // G)
+        y = self.dz.double().view(T, H, -1) + self.db.double().view(H, -1)
+        if self.mode == ops.DECAY_CHANNEL_GATE:
+            a, b = torch.exp(torch.nn.functional.logsigmoid(y) / self.par), torch.ones_like(y[..., 0])
+        else:
+            b = torch.nn.functional.softplus(y[..., 0], threshold=1e9)
+            a = torch.exp(-torch.exp(self.par.double()) * b)[:, :, None].expand(T, H, N)
+        S0 = self.state[:self.R].double().clone()
+        S0[self.fresh] = 0
+        return _walk(self.q.double().view(T, G, N)[:, head] * self.scale, self.k.double().view(T, G, N)[:, head],
+                     self.v.double().reshape(T, H, P), a, b, S0, self.lens, self.skip.double())
+
+    def run(self, chunked):
+        """-> (out [T, H, P], final states)"""
+        x = [t if chunked else t.float() for t in (self.q, self.k, self.v, self.dz)]
+        out = torch.empty(self.T, self.H * self.P, device=self.q.device)
+        ops.decay_scan(self.mode, *x, self.db, self.par, self.skip, self.scale, self.H, self.N, self.P, self.H // self.G, self.state,
+                       self.cu, self.prev, self.save, self.R, out, tiles=self.tiles, ws=self.ws)
+        return out.view(self.T, self.H, self.P), self.state[self.R:]
+
+    def check(self):
+        want, ends = self.exact()
+        for chunked in (True, False):
+            out, state = self.run(chunked)
+            d = out.double() - want
+            assert float(d.norm() / want.norm()) <= 2e-6, chunked
+            assert float(d.abs().max() / want.abs().max()) <= 4e-6, chunked
+            assert float((state.double() - ends).norm() / ends.norm()) <= 2e-6, chunked
+
+
 @pytest.mark.parametrize("mode", [ops.DECAY_CHANNEL_GATE, ops.DECAY_STEP_SIZE])
 @pytest.mark.parametrize("shift", [0.0, -40.0, 15.0])       # decays of a few hundred tokens, of one, of none
-@pytest.mark.parametrize("H,N,P,G,lens", [
-    (3, 128, 80, 3, [33, 64, 5, 97, 1, 32]), (4, 64, 64, 2, [100, 31]), (2, 24, 16, 1, [40, 41]), (2, 8, 70, 2, [8]),
-    (2, 72, 70, 2, [200]), (2, 32, 130, 1, [63, 65])])
+@pytest.mark.parametrize("H,N,P,G,lens", SHAPES)
 def test_decay_chunks(gpu, mode, shift, H, N, P, G, lens):
-    g = torch.Generator(device=gpu).manual_seed(H * N + P)
-    T, R = sum(lens), len(lens)
+    c = _Case(gpu, mode, H, N, P, G, lens)
+    c.dz = (c.dz.float() + shift).bfloat16()
+    c.check()
 
-    def rnd(*s):
-        return torch.randn(*s, device=gpu, generator=g)
 
-    z = rnd(T, 2 * G * N + H * P).bfloat16()                  # q | k | v as column ranges of one projection
-    q, k, v = z[:, :G * N], z[:, G * N:2 * G * N], z[:, 2 * G * N:]
-    cols = H * N if mode == ops.DECAY_CHANNEL_GATE else H
-    dz, db = (rnd(T, cols) + shift).bfloat16(), rnd(cols) + (3.0 if mode == ops.DECAY_CHANNEL_GATE else -2.0)
-    par = 16.0 if mode == ops.DECAY_CHANNEL_GATE else torch.log(0.05 + 0.5 * torch.rand(H, device=gpu, generator=g))
-    skip, scale = rnd(H), 0.37
-    state = rnd(2 * R, H, N, P)
-    S0 = state[:R].double().clone()
-    prev, save = [], []
-    for i, n in enumerate(lens):                              # every third run is a sequence's first
-        prev += [-1 if i % 3 == 2 else -(i + 2)] + [0] * (n - 1)
-        save += [-1] * (n - 1) + [R + i]
-        if i % 3 == 2:
-            S0[i] = 0
-    i32 = dict(device=gpu, dtype=torch.int32)
-    prev, save = torch.tensor(prev, **i32), torch.tensor(save, **i32)
-    cu = torch.tensor([sum(lens[:i]) for i in range(R + 1)], **i32)
-    tiles = torch.tensor([(i, r) for i, n in enumerate(lens) for r in range(0, n, 64)] + [(0, 1 << 24)], **i32)
-    ws = torch.full((T, H, ops.decay_ws_cols(N)), float("nan"), device=gpu)
-    head = torch.arange(H, device=gpu) // (H // G)
-    y = dz.double().view(T, H, -1) + db.double().view(H, -1)
-    if mode == ops.DECAY_CHANNEL_GATE:
-        a, b = torch.exp(torch.nn.functional.logsigmoid(y) / par), torch.ones(T, H, device=gpu, dtype=torch.float64)
-    else:
-        b = torch.nn.functional.softplus(y[..., 0], threshold=1e9)
-        a = torch.exp(-torch.exp(par.double()) * b)[:, :, None].expand(T, H, N)
-    want, ends = _walk(q.double().view(T, G, N)[:, head] * scale, k.double().view(T, G, N)[:, head], v.double().reshape(T, H, P),
-                       a, b, S0, lens, skip.double())
-    out = torch.empty(T, H * P, device=gpu)
-    for chunked in (True, False):
-        x = [t if chunked else t.float() for t in (q, k, v, dz)]
-        ops.decay_scan(mode, *x, db, par, skip, scale, H, N, P, H // G, state, cu, prev, save, R, out, tiles=tiles, ws=ws)
-        d = out.double() - want.reshape(T, -1)
-        assert float(d.norm() / want.norm()) <= 2e-6, chunked
-        assert float(d.abs().max() / want.abs().max()) <= 4e-6, chunked
-        assert float((state[R:].double() - ends).norm() / ends.norm()) <= 2e-6, chunked
+@pytest.mark.parametrize("mode,tau,share,hard", [
+    (ops.DECAY_CHANNEL_GATE, 16.0, 0.1, -40.0), (ops.DECAY_CHANNEL_GATE, 16.0, 0.25, -100.0),
+    (ops.DECAY_CHANNEL_GATE, 16.0, 0.1, -400.0), (ops.DECAY_CHANNEL_GATE, 1.0, 0.1, -40.0),
+    (ops.DECAY_CHANNEL_GATE, 1.0, 0.1, -100.0), (ops.DECAY_STEP_SIZE, 0.0, 0.1, 100.0)])
+@pytest.mark.parametrize("H,N,P,G,lens", SHAPES)
+def test_tokens_that_forget_hard_among_others(gpu, mode, tau, share, hard, H, N, P, G, lens):
+    """A few tokens of a chunk forget almost everything, so the chunk's running decay grows to hundreds, and the tokens behind
+    them remember: their mutual decays are small differences of large sums.  The same bounds."""
+    c = _Case(gpu, mode, H, N, P, G, lens, tau)
+    pick = torch.rand(c.dz.shape, device=gpu, generator=torch.Generator(device=gpu).manual_seed(7)) < share
+    c.dz = torch.where(pick, torch.full_like(c.dz, hard), c.dz)
+    c.check()
 
 
 @pytest.mark.parametrize("form", ["odd channels", "odd stride", "unaligned", "no scratch", "short runs", "wide"])
