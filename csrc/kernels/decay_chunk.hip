@@ -32,7 +32,12 @@ constexpr int LT = C + 4;         // LDS pitch of a [.][C] matrix
 constexpr float LOG2E = 1.4426950408889634f;
 
 SYM_DEV float softplus_exact(float v) { return fmaxf(v, 0.f) + log1pf(expf(-fabsf(v))); }
-SYM_DEV float exp2_neg(float v) { return __builtin_amdgcn_exp2f(fminf(v, 0.f)); }
+// A token's log2 decay, no lower than -256: 2^-256 is 0 in fp32 like everything below, and the chunk's sums stay finite where
+// a token forgets all (a pre-activation or bias of -inf, an infinite rate), so differences behind it are no inf - inf.  NaN
+// stays NaN.
+template <typename F>
+SYM_DEV F log_decay(F v) { return v < (F)-256 ? (F)-256 : v; }
+SYM_DEV float pow2(float v) { return __builtin_amdgcn_exp2f(v); }
 SYM_DEV f32x4 mfma4(float x, float y, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); }
 SYM_DEV f32x4 lds4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
@@ -102,7 +107,7 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
     const bool in = tt < nt && n < N;
     kS[tt * LD + n] = in ? (float)k[tt * a.ldk + n] : 0.f;
     qS[tt * LD + n] = in ? (float)q[tt * a.ldq + n] : 0.f;
-    GS[tt * LD + n] = in ? scale * softplus_exact(-((float)dz[tt * a.ldd + n] + db[n])) : 0.f;
+    GS[tt * LD + n] = in ? log_decay(scale * softplus_exact(-((float)dz[tt * a.ldd + n] + db[n]))) : 0.f;
   }
   __syncthreads();
   const int wc = ws_cols(N);
@@ -124,8 +129,8 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
     const int tt = i / NP, n = i % NP;
     if (tt >= nt || n >= N) continue;
     const float gi = GS[tt * LD + n], li = LS[tt * LD + n];
-    ws[tt * wrow + C + n] = __builtin_amdgcn_exp2f(gi);
-    ws[tt * wrow + C + N + n] = kS[tt * LD + n] * exp2_neg((GS[(C - 1) * LD + n] - gi) + (LS[(C - 1) * LD + n] - li));
+    ws[tt * wrow + C + n] = pow2(gi);
+    ws[tt * wrow + C + N + n] = kS[tt * LD + n] * pow2((GS[(C - 1) * LD + n] - gi) + (LS[(C - 1) * LD + n] - li));
   }
   const int col = lane & 15, g = lane >> 4;
   // rows 16 .., columns .. 15: the waves take the channel tiles in turn
@@ -137,7 +142,7 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
     const f32x4 qi = lds4(qS + (16 + col) * LD + c), kj = lds4(kS + col * LD + c);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      d = mfma4(qi[r] * exp2_neg((gi[r] - mh[r]) + (li[r] - ml[r])), kj[r] * exp2_neg((mh[r] - gj[r]) + (ml[r] - lj[r])), d);
+      d = mfma4(qi[r] * pow2((gi[r] - mh[r]) + (li[r] - ml[r])), kj[r] * pow2((mh[r] - gj[r]) + (ml[r] - lj[r])), d);
   }
   // diagonal tiles: wave (channel half, tile), a 2 x 2 block of (i, j) per lane
   constexpr int NH = NP / 2;
@@ -163,7 +168,7 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
         for (int f = 0; f < 2; ++f)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            s[e][f] += qi[e][r] * (kj[f][r] * exp2_neg((gi[e][r] - gj[f][r]) + (li[e][r] - lj[f][r])));
+            s[e][f] += qi[e][r] * (kj[f][r] * pow2((gi[e][r] - gj[f][r]) + (li[e][r] - lj[f][r])));
     }
   }
   __syncthreads();                             // (the rows have been read: their place takes the partial scores)
@@ -294,7 +299,7 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
       // running sum over the chunk's tokens as a pair of floats: with step sizes that forget in a few tokens the sum grows
       // to hundreds, and the differences of neighbours, which are what counts, would keep few of its digits
       const float b = tid < nt ? softplus_exact(rdt) : 0.f;
-      double s = tid < nt ? -(double)rate2 * b : 0.0;
+      double s = tid < nt ? log_decay(-(double)rate2 * b) : 0.0;
 #pragma unroll
       for (int o = 1; o < C; o <<= 1) {
         const double up = __shfl_up(s, o, 64);
@@ -369,7 +374,7 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
         lj[j] = lds4(fs + C + 16 * j + 4 * g);
         bj[j] = lds4(fs + 2 * C + 16 * j + 4 * g);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) O[j][r] *= __builtin_amdgcn_exp2f(gj[j][r]);      // (rows 4 g + r of O too)
+        for (int r = 0; r < 4; ++r) O[j][r] *= pow2(gj[j][r]);      // (rows 4 g + r of O too)
       }
       const bf16* Kn = st + oK + col * LQ + 8 * g;
       const bf16* Qn = st + col * LQ + 8 * g;
@@ -386,7 +391,7 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
                          *reinterpret_cast<const bf16x8*>(Qn + 16 * i * LQ + 32 * t), d);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              const float w = exp2_neg((gi - gj[j][r]) + (li - lj[j][r])) * bj[j][r];
+              const float w = pow2((gi - gj[j][r]) + (li - lj[j][r])) * bj[j][r];
               d[r] = j < i || 4 * g + r <= col ? d[r] * w : 0.f;
             }
           }
@@ -420,12 +425,12 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
         S[t] = mfma16(pair4(Kt + 16 * t * LT), V.v, S[t]);
       }
     } else {
-      const float gc = fs[C - 1], lc = fs[2 * C - 1], d = __builtin_amdgcn_exp2f(gc);     // (G stands still past the run's end)
+      const float gc = fs[C - 1], lc = fs[2 * C - 1], d = pow2(gc);     // (G stands still past the run's end)
       f32x4 w[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) w[j][r] = exp2_neg((gc - gj[j][r]) + (lc - lj[j][r])) * bj[j][r] * (float)V.h[4 * j + r];
+        for (int r = 0; r < 4; ++r) w[j][r] = pow2((gc - gj[j][r]) + (lc - lj[j][r])) * bj[j][r] * (float)V.h[4 * j + r];
       const Parts s = split(w[0], w[1]);
 #pragma unroll
       for (int t = 0; t < 2 * NB; ++t) {

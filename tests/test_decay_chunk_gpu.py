@@ -112,6 +112,20 @@ def test_tokens_that_forget_hard_among_others(gpu, mode, tau, share, hard, H, N,
     c.check()
 
 
+@pytest.mark.parametrize("mode", [ops.DECAY_CHANNEL_GATE, ops.DECAY_STEP_SIZE])
+@pytest.mark.parametrize("H,N,P,G,lens", SHAPES)
+def test_decays_of_exactly_zero(gpu, mode, H, N, P, G, lens):
+    """A gate of -inf, from the projection or as a channel's bias (or a head's infinite rate), forgets all there was: 0 x S + k v."""
+    c = _Case(gpu, mode, H, N, P, G, lens)
+    if mode == ops.DECAY_CHANNEL_GATE:
+        pick = torch.rand(c.dz.shape, device=gpu, generator=torch.Generator(device=gpu).manual_seed(9)) < 0.1
+        c.dz = torch.where(pick, torch.full_like(c.dz, -float("inf")), c.dz)
+        c.db[::5] = -float("inf")
+    else:
+        c.par[0] = 100.0
+    c.check()
+
+
 @pytest.mark.parametrize("form", ["odd channels", "odd stride", "unaligned", "no scratch", "short runs", "wide"])
 def test_forms_that_walk_token_by_token(gpu, form):
     """What the chunked form does not take gives the same recurrence (channel gate, one run from zero)."""
