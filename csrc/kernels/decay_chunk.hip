@@ -12,7 +12,7 @@
 //
 // Precision: q, k and v are bf16, so they are exact operands of v_mfma_f32_16x16x32_bf16, which accumulates in fp32.  An
 // fp32 operand x (the state, a scaled vector, the scores) is used as the sum of three bf16 parts, hi = bf16(x), mid =
-// bf16(x - hi), lo = bf16(x - hi - mid), which hold all of its 24 bits; of a product of two such operands the six terms
+// bf16(x - hi), lo = bf16(x - hi - mid), which hold all of its 24 bits (of an infinity the parts make NaN); of a product of two such operands the six terms
 // down to 2^-16 of the largest are taken (what is left is 2^-24 of it, an fp32 rounding).  That is 3 / 8 or 3 / 16 of the
 // matrix cycles of v_mfma_f32_16x16x4_f32.
 //
@@ -360,6 +360,22 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
         O[i] = mfma16(qh, s.h, O[i]);
       }
     }
+    // The product of scores and values runs over the scores' masked half as well, where 0 x inf would reach the rows in front
+    // of a value that is not finite: it is left out of the product, and its column is NaN from its token on.
+    Pack8 W = V;
+    int bad = C;
+    const uint4 e = V.u;
+    const auto ones = [](unsigned x) { return (x & 0x7f807f80u) + 0x00800080u; };     // bits 15, 31: an exponent of all ones
+    if (__any(((ones(e.x) | ones(e.y) | ones(e.z) | ones(e.w)) & 0x80008000u) != 0)) {
+#pragma unroll
+      for (int i = 7; i >= 0; --i)
+        if (!__builtin_isfinite((float)V.h[i])) {
+          W.h[i] = (bf16)0.f;
+          bad = 16 * (i >> 2) + 4 * g + (i & 3);
+        }
+      bad = min(bad, __shfl_xor(bad, 16, 64));
+      bad = min(bad, __shfl_xor(bad, 32, 64));
+    }
     f32x4 A[2][2];                                      // scores of row tile i, columns 4 g + r and 16 + 4 g + r
     f32x4 gj[2], lj[2], bj[2];
     if constexpr (MODE == 0) {
@@ -402,9 +418,16 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const Parts s = split(A[i][0], A[i][1]);
-      O[i] = mfma16(s.l, V.v, O[i]);
-      O[i] = mfma16(s.m, V.v, O[i]);
-      O[i] = mfma16(s.h, V.v, O[i]);
+      O[i] = mfma16(s.l, W.v, O[i]);
+      O[i] = mfma16(s.m, W.v, O[i]);
+      O[i] = mfma16(s.h, W.v, O[i]);
+    }
+    if (bad < C) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * i + 4 * g + r >= bad) O[i][r] = __builtin_nanf("");
     }
     if (pin) {
 #pragma unroll

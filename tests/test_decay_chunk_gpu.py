@@ -126,6 +126,25 @@ def test_decays_of_exactly_zero(gpu, mode, H, N, P, G, lens):
     c.check()
 
 
+@pytest.mark.parametrize("mode", [ops.DECAY_CHANNEL_GATE, ops.DECAY_STEP_SIZE])
+@pytest.mark.parametrize("what,value", [("v", float("inf")), ("v", float("nan")), ("k", -float("inf")), ("q", float("nan")),
+                                        ("q", float("inf")), ("dz", float("nan"))])
+@pytest.mark.parametrize("H,N,P,G,lens", [(3, 128, 80, 3, [33, 64, 5, 97, 1, 32]), (4, 64, 64, 2, [100, 31]), (2, 24, 16, 1, [40, 41])])
+def test_values_that_are_not_finite(gpu, mode, what, value, H, N, P, G, lens):
+    """They reach what the token-by-token kernel lets them reach, and nothing else: no earlier token, no other column."""
+    c = _Case(gpu, mode, H, N, P, G, lens)
+    clean, state = (t.clone() for t in c.run(True))
+    x = getattr(c, what).clone()
+    for r in (5, 21, 60):                                     # (a chunk's first tile, its second, another chunk)
+        x[r, (7 * r) % x.shape[1]] = value
+    setattr(c, what, x)
+    walk, walk_state = (t.clone() for t in c.run(False))
+    out, ends = c.run(True)
+    assert 0 < int((~walk.isfinite()).sum()) < walk.numel()
+    assert torch.equal(out.isfinite(), walk.isfinite()) and torch.equal(ends.isfinite(), walk_state.isfinite())
+    assert torch.equal(out[out.isfinite()], clean[out.isfinite()]) and torch.equal(ends[ends.isfinite()], state[ends.isfinite()])
+
+
 @pytest.mark.parametrize("form", ["odd channels", "odd stride", "unaligned", "no scratch", "short runs", "wide"])
 def test_forms_that_walk_token_by_token(gpu, form):
     """What the chunked form does not take gives the same recurrence (channel gate, one run from zero)."""
