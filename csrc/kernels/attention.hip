@@ -739,7 +739,7 @@ constexpr int DECODE_UNITS = 512, DECODE_THIRDS = 384;
 void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache, const int* block_tables,
                         const int* ctx_lens, bf16* out, float* tmp_o, float* tmp_ml, int* counters, int num_seqs,
                         int Hq, int Hkv, int BS, int max_blocks, int max_parts, float scale, hipStream_t s) {
-  if (num_seqs == 0) return;
+  if (num_seqs == 0 || max_blocks == 0) return;  // (an empty table: no context has a token)
   const float scale_log2 = scale * 1.4426950408889634f;
   const int G = Hq / Hkv;
   const int units = num_seqs * Hkv;  // (parts <= 512: attn_decode_unit's exact division)

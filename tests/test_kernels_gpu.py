@@ -194,6 +194,19 @@ def test_attn_decode_equal_partitions(gpu, S, Hq, Hkv):
     _close(out, out_r, atol=2e-2, rtol=2e-2)
 
 
+def test_attn_decode_empty_tables(gpu):
+    """Block tables without a column (and so scratch without a partition): nothing to read, nothing to write."""
+    S, Hq, Hkv = 3, 16, 4
+    kc, vc, bt = _random_paged(gpu, [0] * S, Hkv, 32, torch.Generator(device=gpu).manual_seed(1))
+    out = torch.full((S, Hq, 128), 7.0, device=gpu, dtype=torch.bfloat16)
+    i32 = dict(device=gpu, dtype=torch.int32)
+    for parts in (0, 1):
+        ops.attn_decode(torch.zeros_like(out), kc, vc, bt[:, :0].contiguous(), torch.zeros(S, **i32), out,
+                        torch.empty(S, Hq, parts, 128, device=gpu), torch.empty(S, Hq, parts, 2, device=gpu),
+                        torch.zeros(S * Hkv, **i32), 0.1)
+    assert bool((out == 7.0).all())
+
+
 @pytest.mark.parametrize("Hq,Hkv", [(32, 8), (64, 8), (8, 1), (16, 16)])
 @pytest.mark.parametrize("BS", [32, 64])
 def test_attn_decode_wave(gpu, Hq, Hkv, BS):
