@@ -21,9 +21,10 @@
 // Decode (K5): grid (seq, kv_head, partition), 8 waves, 256 tokens (32 per wave) a step; the
 // G = Hq/Hkv query heads of a kv head are the MFMA columns (K/V are read once per kv head).
 // Multi-partition sequences write fp32 partials that the last-arriving partition combines
-// (split-KV, flash-decoding, one launch).  The number of partitions comes from the number of
-// (sequence, kv head) units alone, so the launch is hipGraph-capturable; the kernel cuts every
-// context into that many equal parts, and workgroups past the last one exit at once.
+// (split-KV, flash-decoding, one launch).  The grid comes from the number of (sequence, kv head)
+// units and the tables' width alone, so the launch is hipGraph-capturable; the kernel cuts every
+// context into that many equal parts, one far above the others into more, and workgroups past the
+// last one exit at once.
 //
 // Prefill (K4): causal + varlen + chunked prefill (queries are the LAST qlen
 // positions of a context of length ctx), reading K/V from the paged cache.
@@ -45,14 +46,30 @@ namespace {
 // ---------------------------------------------------------------------------------------------
 // GMAX >= G query heads per kv head: the cross-wave merge stages GMAX columns in LDS (GMAX = 4 for
 // Llama-3 GQA: 17 KB instead of 68 KB, so LDS no longer caps the resident workgroups per CU)
-template <int GMAX>
+template <int GMAX, bool UNEVEN>
 __global__ __launch_bounds__(DWAVES * 64, 4) void attn_decode_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
     const int* __restrict__ block_tables, const int* __restrict__ ctx_lens, bf16* __restrict__ out,
-    float* __restrict__ tmp_o, float* __restrict__ tmp_ml, int* __restrict__ counters, int Hq, int Hkv, int G, int BS,
-    int max_blocks, int max_parts, float scale_log2, unsigned inv_parts) {
-  attn_decode_unit<GMAX>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, Hq, Hkv, G, BS,
-                       max_blocks, max_parts, scale_log2, inv_parts, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z);
+    float* __restrict__ tmp_o, float* __restrict__ tmp_ml, int* __restrict__ counters, int num_seqs, int Hq, int Hkv,
+    int G, int BS, int max_blocks, int max_parts, int parts, int slots_log2, int further, float scale_log2, unsigned inv,
+    unsigned inv_heads) {
+  // UNEVEN: grid y = part * Hkv + kvh, and past Hkv * parts the further partitions, `further` items for each head (items in
+  // the grid's last rows, so that they start behind the others: between them, a batch of like contexts that fills the chip
+  // found its workgroups spread unevenly over the CUs, 64 x 900 tokens 61 instead of 55 us).
+  int seq = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
+  if constexpr (UNEVEN) {
+    part = min((int)__umulhi(2 * blockIdx.y, inv_heads), parts);  // blockIdx.y / Hkv
+    kvh = blockIdx.y - part * Hkv;
+    if (part == parts) {
+      const int w = kvh * num_seqs + seq;
+      seq = (unsigned)w / (unsigned)Hkv;
+      kvh = w - seq * Hkv;
+      if (seq >= further) return;
+    }
+  }
+  attn_decode_unit<GMAX, UNEVEN>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, num_seqs,
+                                 Hq, Hkv, G, BS, max_blocks, max_parts, scale_log2, inv, seq, kvh, part, parts,
+                                 slots_log2);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -734,6 +751,13 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_rows_kernel(
 //   5 x 5400, 4 kv heads                  28.7 /   - / 22.8      160 x 600    112 / 126 /  84
 //   48 x 60                                8.8 / 9.3 /  6.5      256 x 2000   428 / 370 / 335
 // Bound by the K/V stream from ~100 MB on, by four dependent round trips (context, K/V, publish, combine) below ~20 MB.
+// A context far above the others' would leave its few workgroups walking alone, so where the block tables hold more than
+// LONG_STEPS steps a partition, contexts above 3 / 2 of their share of the batch are cut further (attn_decode_unit; us, the
+// streaming kernel / every context cut alike / now, 8 kv heads):
+//   60 x 300 + 1 x 8000     51 / 126 / 39      100 x 200 + 2 x 30000   148 /  472 /  80      56 x 1000 + 8 x 7000  201 / 216 / 107
+//   60 x 200 + 1 x 2000     33 /  38 / 24       60 x 200 + 1 x 120000  329 / 1816 / 112      100 x 100 .. 8000     194 / 258 / 172
+// A batch of like contexts pays for the rule: 64 x 900 54.9 -> 55.2, 32 x 4000 118 -> 119.5, 160 x 600 86.9 -> 87.8.  Shares of
+// half the size (twice the workgroups) were up to 15 % faster on uneven batches and lost as much on even ones (32 x 4000: 135).
 constexpr int DECODE_UNITS = 512, DECODE_THIRDS = 384;
 
 void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache, const int* block_tables,
@@ -745,15 +769,28 @@ void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache,
   const int units = num_seqs * Hkv;  // (parts <= 512: attn_decode_unit's exact division)
   const int cut = units <= DECODE_UNITS / 2 ? DECODE_UNITS / units : units <= DECODE_THIRDS ? 3 : 1;
   const int parts = min(max_parts, cut);
-  const dim3 grid(num_seqs, Hkv, parts);
+  // (max_parts is the steps of the longest context that the tables hold)
+  const bool uneven = num_seqs > 1 && max_parts > LONG_STEPS * parts;
+  // a context has no more further partitions than its steps / quota, the batch no more than 2^slots_log2 per kv head
+  const int slots_log2 = 31 - __builtin_clz(max(1, DECODE_UNITS / Hkv));
+  const int further = (int)min(1ll << slots_log2, (long long)num_seqs * (max_parts - parts));
+  const dim3 grid = uneven ? dim3(num_seqs, Hkv * parts + (further * Hkv + num_seqs - 1) / num_seqs)
+                           : dim3(num_seqs, Hkv, parts);
   const unsigned inv = (unsigned)((1ull << 32) / parts) + 1;  // (not used for one partition)
+  const unsigned inv_heads = (unsigned)((1ull << 31) / Hkv) + 1;
   auto run = [&](auto kern) {
-    kern<<<grid, DWAVES * 64, 0, s>>>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, Hq, Hkv,
-                                      G, BS, max_blocks, max_parts, scale_log2, inv);
+    kern<<<grid, DWAVES * 64, 0, s>>>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, num_seqs,
+                                      Hq, Hkv, G, BS, max_blocks, max_parts, parts, slots_log2, further, scale_log2, inv,
+                                      inv_heads);
   };
-  if (G <= 4) run(attn_decode_kernel<4>);
-  else if (G <= 8) run(attn_decode_kernel<8>);
-  else run(attn_decode_kernel<16>);
+  auto pick = [&](auto u) {
+    constexpr bool U = decltype(u)::value != 0;
+    if (G <= 4) run(attn_decode_kernel<4, U>);
+    else if (G <= 8) run(attn_decode_kernel<8, U>);
+    else run(attn_decode_kernel<16, U>);
+  };
+  if (uneven) pick(IntC<1>{});
+  else pick(IntC<0>{});
 }
 
 // Workgroups of the 64-row x 4-head kernel up to which the row kernel takes a prompt step: below, most CUs would idle; above,

@@ -258,20 +258,87 @@ SYM_DEV void load_q(const bf16* __restrict__ q, int seq, int Hq, int kvh, int G,
   }
 }
 
+SYM_DEV int steps_of(int ctx) { return (int)((unsigned)max(0, ctx + PART - 1) / PART); }
+
+// Sum over the wave, in a scalar register (DPP inside each row of 16 lanes, then the four rows).
+SYM_DEV int wave_total(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);   // lanes 1 apart
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);   // 2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);  // the other four of eight
+  v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);  // the other eight of sixteen
+  return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
+         __builtin_amdgcn_readlane(v, 48);
+}
+
+// Steps a partition of a long context has: the batch's steps shared out over 2^slots_log2 workgroups per kv head.  Every wave
+// that asks computes the same from the same lengths.
+SYM_DEV int batch_quota(const int* __restrict__ ctx_lens, int num_seqs, int slots_log2) {
+  int total = 0;
+#pragma unroll 4
+  for (int i = threadIdx.x & 63; i < num_seqs; i += 64) total += steps_of(ctx_lens[i]);
+  return max(1, (wave_total(total) + (1 << slots_log2) - 1) >> slots_log2);
+}
+
+// Partitions of a context: `parts` (none shorter than a step), or for one of more than 3 / 2 of its share of the batch as many
+// as make partitions of that share (half above the mean is left alone).  Contexts up to LONG_STEPS steps a partition are not asked about the batch: the sum over
+// the lengths is a round trip in front of their K/V (contexts of ~900 tokens, 64 of them: 0.6 us of 55 when all above four
+// steps asked).
+constexpr int LONG_STEPS = 6;
+
+SYM_DEV bool may_be_long(int steps, int parts) { return steps > LONG_STEPS * parts; }
+
+SYM_DEV int partitions_of(int steps, int parts, int quota, int max_parts) {
+  if (!may_be_long(steps, parts) || 2 * steps <= 3 * parts * quota) return min(steps, parts);
+  return min((int)((unsigned)(steps + quota - 1) / (unsigned)quota), max_parts);
+}
+
+// Item e of the further partitions (those past a context's first `parts`, in the order of the sequences) -> (seq, part);
+// false: there are fewer.
+SYM_DEV bool further_partition(const int* __restrict__ ctx_lens, int num_seqs, int parts, int quota, int max_parts, int e,
+                               int& seq, int& part) {
+  const int lane = threadIdx.x & 63;
+  for (int i0 = 0; i0 < num_seqs; i0 += 64) {
+    const int steps = i0 + lane < num_seqs ? steps_of(ctx_lens[i0 + lane]) : 0;
+    const int more = max(0, partitions_of(steps, parts, quota, max_parts) - parts);
+    int upto = more;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, 64);
+      if (lane >= o) upto += v;
+    }
+    const unsigned long long past = __ballot(upto > e);
+    if (past) {
+      const int l = __builtin_ctzll(past);
+      seq = i0 + l;
+      part = parts + e - __builtin_amdgcn_readlane(upto - more, l);
+      return true;
+    }
+    e -= __builtin_amdgcn_readlane(upto, 63);
+  }
+  return false;
+}
+
 // Split-KV decode attention unit (seq, kv head, partition) on an 8-wave workgroup; the G = Hq/Hkv query heads
 // of the kv head are the MFMA columns.  A context of n 256-token steps (8 waves x one 32-token group) is cut
 // into min(parts, n) partitions of whole steps, as equal as they allow: the launcher picks `parts` from the
-// number of units, the kernel the partition from the context, so that short and long contexts of one batch
-// give the chip about the same number of workgroups and a batch that fills it alone is not split at all.
-template <int GMAX>
+// number of units, the kernel the partition from the context, so that a batch of like contexts gives the chip
+// about the same number of workgroups and one that fills it alone is not split at all.
+// UNEVEN (block tables wide enough for contexts far above the others'): a context of more than 3 / 2 of its
+// share of the batch is cut into partitions of that share; part == parts then stands for the further partitions, and
+// seq is the item's number among them.
+template <int GMAX, bool UNEVEN>
 SYM_DEV void attn_decode_unit(const bf16* __restrict__ q, const bf16* __restrict__ k_cache,
                               const bf16* __restrict__ v_cache, const int* __restrict__ block_tables,
                               const int* __restrict__ ctx_lens, bf16* __restrict__ out, float* __restrict__ tmp_o,
-                              float* __restrict__ tmp_ml, int* __restrict__ counters, int Hq, int Hkv, int G, int BS,
-                              int max_blocks, int max_parts, float scale_log2, unsigned inv_parts, int seq, int kvh,
-                              int part, int parts) {
+                              float* __restrict__ tmp_ml, int* __restrict__ counters, int num_seqs, int Hq, int Hkv,
+                              int G, int BS, int max_blocks, int max_parts, float scale_log2, unsigned inv, int seq,
+                              int kvh, int part, int parts, int slots_log2) {
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = lane >> 4;
+  if (UNEVEN && __builtin_expect(part >= parts, 0)) {
+    const int quota = batch_quota(ctx_lens, num_seqs, slots_log2);
+    if (!further_partition(ctx_lens, num_seqs, parts, quota, max_parts, seq, seq, part)) return;
+  }
   const int* bt = block_tables + (long long)seq * max_blocks;
   const int bsh = __builtin_ctz(BS);  // block sizes are powers of two (launchers check)
   // The context length, the block of this wave's first group in a context of at most `parts` steps and the query are
@@ -281,16 +348,22 @@ SYM_DEV void attn_decode_unit(const bf16* __restrict__ q, const bf16* __restrict
   bf16x8 qf[4];
   load_q(q, seq, Hq, kvh, G, qf);
   const int ctx = ctx_lens[seq];
-  const int steps = (ctx + PART - 1) / PART;
-  const int nparts = min(parts, steps);
-  if (part >= nparts) return;  // (an empty context has no partition)
-  // first step of partition i: floor(i * steps / parts); inv_parts = floor(2^32 / parts) + 1 is exact for i * steps
+  const int steps = steps_of(ctx);
+  int nparts = min(parts, steps);
+  // first step of partition i: floor(i * steps / parts); `inv` = floor(2^32 / parts) + 1 is exact for i * steps
   // below 2^32 / parts (the launcher keeps parts <= 512).  Fewer steps than partitions: one step each.
-  auto first = [&](int i) {
-    return steps <= parts ? i : i == parts ? steps : (int)__umulhi((unsigned)(i * steps), inv_parts);
-  };
-  const int end = min(ctx, first(part + 1) * PART);
-  int tok0 = first(part) * PART + wid * 32;
+  auto first = [&](int i) { return steps <= parts ? i : i == parts ? steps : (int)__umulhi((unsigned)(i * steps), inv); };
+  int from = first(part), to = first(part + 1);
+  if (UNEVEN && __builtin_expect(may_be_long(steps, parts), 0)) {
+    nparts = partitions_of(steps, parts, batch_quota(ctx_lens, num_seqs, slots_log2), max_parts);
+    if (nparts > parts) {
+      from = (unsigned)(part * steps) / (unsigned)nparts;
+      to = (unsigned)(part * steps + steps) / (unsigned)nparts;
+    }
+  }
+  if (part >= nparts) return;  // (an empty context has no partition)
+  const int end = min(ctx, to * PART);
+  int tok0 = from * PART + wid * 32;
   if (steps > parts) blk = bt[min(tok0 >> bsh, max_blocks - 1)];
   f32x4 o[8];
 #pragma unroll
