@@ -695,6 +695,7 @@ void route_topk(const Tensor& x, const Tensor& Wr, const OptTensor& bias, int64_
   a.ids = ptr<int>(ids), a.w = ptr<float>(w), a.offsets = ptr<int>(offsets), a.dst = ptr<int>(dst), a.src = ptr<int>(src);
   a.runs = runs;
   TORCH_CHECK(!runs || (route_topk_runs(a, f32) && !a.bias), "route_topk: runs: bf16, at most 16 experts, d % 128 == 0, no bias");
+  const at::OptionalDeviceGuard g(x.device());
   launch_route_topk(a, f32, cur_stream(x));
 }
 
@@ -724,6 +725,7 @@ int64_t expert_linear(const Tensor& x, const OptTensor& src, const Tensor& W, co
   a.glu = glu, a.f32_out = y32 && !f32;
   TORCH_CHECK(!(a.glu || a.f32_out) || (expert_linear_mfma(a, f32) && E <= 65535 && (impl < 0 || (impl == 1) || (impl > 1 && a.K % 64 == 0))),
               "expert_linear: glu and fp32 output take bf16 rows of a multiple of 32, 16-byte aligned");
+  const at::OptionalDeviceGuard g(x.device());
   return launch_expert_linear(a, f32, (int)impl, cur_stream(x));
 }
 

@@ -90,3 +90,23 @@ def test_router_in_runs(T, E, k, d):
     assert int(ids.min()) >= 0 and int(ids.max()) < E
     assert torch.equal(src[dst.long()].cpu(), (torch.arange(R) // k).int())
     assert torch.equal(off.diff().cpu().long(), torch.bincount(ids.cpu().long(), minlength=E))
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs a second GPU")
+def test_a_device_that_is_not_the_current_one():
+    """Routing and expert products launch on their operands' device (an engine on "cuda:1" of a process whose current device is 0)."""
+    torch.manual_seed(3)
+    T, d, E, N, k = 40, 256, 8, 64, 2
+    x, Wr, W = torch.randn(T, d).to(BF16), torch.randn(E, d).to(BF16), (torch.randn(E, 2 * N, d) * d ** -0.5).to(BF16)
+    got = []
+    with torch.cuda.device(0):
+        for dev in ("cuda:0", "cuda:1"):
+            ids, off, dst, src = (torch.empty(n, dtype=torch.int32, device=dev) for n in (T * k, E + 1, T * k, T * k))
+            w, y = torch.empty(T * k, device=dev), torch.empty(T * k, N, dtype=BF16, device=dev)
+            xd = x.to(dev)
+            ops.route_topk(xd, Wr.to(dev), None, k, ids, w, off, dst, src, runs=True)
+            ops.expert_linear(xd, src, W.to(dev), off, y, glu=True)
+            torch.cuda.synchronize(dev)
+            got.append([t.cpu() for t in (ids, w, off, dst, src, y)])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
