@@ -530,21 +530,28 @@ def logits_argmax(logits, temps, seeds, step, out_keys, out_ids, n_offset=0):
     return reference.logits_argmax(logits, temps, seeds, step, out_keys, out_ids, n_offset)
 
 
+def _plain(*tensors: torch.Tensor) -> bool:
+    return all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors)
+
+
 FEW_ROWS = 16  # rows up to which a linear layer is a weight stream (csrc/kernels/row_linear.hip)
 
 
 def few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None) -> bool:
     """Does x @ w.T into ``out`` (row_linear's layouts: glu takes w of twice out's columns) run on the few-row kernel?  bf16
     x and w on the GPU, 1..16 rows, w contiguous, unit inner strides, 16-byte aligned rows of x and w, K at most 256 in
-    eights or a multiple of 256, outputs in fours; everything else, and anything autograd records, is the library's."""
-    if out is None or x.dim() != 2 or not 0 < x.shape[0] <= FEW_ROWS or w.dim() != 2 or out.dim() != 2:
+    eights or a multiple of 256, outputs in fours; everything else is the library's: tensors of other classes (fake ones of
+    a tracer, distributed ones), graphs that are being compiled, and whatever autograd records, backward or forward."""
+    if torch.compiler.is_compiling() or out is None or not _plain(x, w, out):
+        return False
+    if x.dim() != 2 or not 0 < x.shape[0] <= FEW_ROWS or w.dim() != 2 or out.dim() != 2:
         return False
     if not _gpu(x) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not w.is_contiguous():
         return False
     M, K = x.shape
     if w.device != x.device or out.device != x.device or w.shape[1] != K or out.shape[0] != M:
         return False
-    if not (K % 256 == 0 or (K < 256 and K % 8 == 0)) or K == 0 or out.shape[1] % 4 or not out.shape[1]:
+    if not (K % 256 == 0 or (K < 256 and K % 8 == 0)) or not 0 < K <= 1 << 22 or out.shape[1] % 4 or not 0 < out.shape[1] <= 1 << 30:
         return False
     if x.stride(1) != 1 or out.stride(1) != 1 or (M > 1 and (x.stride(0) % 8 or not 0 < x.stride(0) <= 1 << 24)):
         return False
@@ -552,7 +559,8 @@ def few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None) -> bool
         return False
     if x.data_ptr() % 16 or w.data_ptr() % 16 or out.data_ptr() % (4 * out.element_size()):
         return False
-    return not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or out.requires_grad))
+    return torch.autograd.forward_ad._current_level < 0 and not (
+        torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or out.requires_grad))
 
 
 def row_linear(x, w, out, relu2: bool = False, glu: bool = False) -> None:

@@ -75,6 +75,36 @@ def test_linear_accepts_every_form(gpu):
     assert w.grad is not None
 
 
+def test_linear_of_traced_tensors():
+    """A tracer's fake GPU tensors have no memory: they take the library's product (nothing is launched here)."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode():
+        x, w = torch.empty(8, 256, device="cuda", dtype=torch.bfloat16), torch.empty(64, 256, device="cuda", dtype=torch.bfloat16)
+        out, wide = torch.empty(8, 64, device="cuda", dtype=torch.bfloat16), torch.empty(8, 64, device="cuda")
+        assert not ops.few_rows(x, w, out)
+        assert ops.linear(x, w, out=out) is out
+        assert ops.linear_f32(x, w, out=wide) is wide
+
+
+def test_linear_while_compiling(monkeypatch):
+    monkeypatch.setattr(ops, "_gpu", lambda t: True)
+    x, w, out = torch.zeros(8, 256).bfloat16(), torch.zeros(64, 256).bfloat16(), torch.empty(8, 64).bfloat16()
+    assert ops.few_rows(x, w, out)
+    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
+    assert not ops.few_rows(x, w, out)
+
+
+def test_linear_of_dual_tensors(monkeypatch):
+    """A product into ``out`` has no forward derivative: refused by the library, not computed without it."""
+    monkeypatch.setattr(ops, "_gpu", lambda t: True)
+    x, w, out = torch.zeros(8, 256).bfloat16(), torch.zeros(64, 256).bfloat16(), torch.empty(8, 64).bfloat16()
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        with pytest.raises(RuntimeError, match="forward AD"):
+            ops.linear(dual, w, out=out)
+
+
 def test_row_linear_reference_cpu():
     x, w = torch.randn(3, 32).bfloat16(), torch.randn(16, 32).bfloat16()
     out = torch.empty(3, 8, dtype=torch.bfloat16)
