@@ -42,7 +42,7 @@ SYM_DEV void choose(float* z, int E, int k, int lane, int* ids, float* w) {
     }
     if (bi >= E) bi = j;       // only with non-finite logits: keep the id a valid segment index for the kernels downstream
     if (j == 0) zmax = best;
-    const float p = j == 0 ? 1.f : expf(best - zmax);
+    const float p = j == 0 || zmax == -INFINITY ? 1.f : expf(best - zmax);     // (no finite logit: equal weights)
     sum += p;
     if (lane == 0) {
       ids[j] = bi;

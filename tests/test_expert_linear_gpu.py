@@ -92,6 +92,33 @@ def test_router_in_runs(T, E, k, d):
     assert torch.equal(off.diff().cpu().long(), torch.bincount(ids.cpu().long(), minlength=E))
 
 
+@pytest.mark.parametrize("dtype,E,runs", [(BF16, 8, False), (BF16, 8, True), (BF16, 100, False), (torch.float32, 8, False)])
+@pytest.mark.parametrize("value", [-float("inf"), float("nan")])
+def test_rows_without_a_finite_logit(dtype, E, runs, value):
+    """Both routers give such a row its first k experts in equal parts, and the other rows what they had."""
+    T, d, k = 20, 128, 3
+    torch.manual_seed(E)
+    x, Wr = torch.rand(T, d).to(dtype).cuda(), torch.rand(E, d).to(dtype).cuda()
+    bad = [0, 7, 19]
+
+    def route(x):
+        ids, off, dst, src = (torch.full((n,), -1, dtype=torch.int32, device="cuda") for n in (T * k, E + 1, T * k, T * k))
+        w = torch.empty(T * k, device="cuda")
+        ops.route_topk(x, Wr, None, k, ids, w, off, dst, src, runs=runs)
+        assert sorted(dst.tolist()) == list(range(T * k)) and int(off[E]) == T * k
+        return ids.view(T, k).cpu(), w.view(T, k).cpu()
+
+    want, share = route(x)
+    x = x.clone()
+    x[bad] = value                                   # (positive router weights: every logit of the row is this value)
+    ids, w = route(x)
+    for t in range(T):
+        if t in bad:
+            assert ids[t].tolist() == list(range(k)) and torch.allclose(w[t], torch.full((k,), 1 / k))
+        else:
+            assert torch.equal(ids[t], want[t]) and torch.equal(w[t], share[t])
+
+
 @pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs a second GPU")
 def test_a_device_that_is_not_the_current_one():
     """Routing and expert products launch on their operands' device (an engine on "cuda:1" of a process whose current device is 0)."""
