@@ -6,8 +6,8 @@ the block, so every step (decode and prefill, with or without expert parallelism
 Small routed batches (<= 64 rows: decode steps) use the grouped skinny MFMA GEMM or the weight-streaming kernels;
 prefill-sized ones the prefill GEMM kernel in grouped mode (``ops.pg_grouped``, csrc/kernels/pgemm.hip) or, below
 its row thresholds, the weight-streaming grouped GEMM (``ops.grouped_gemm``) on the preshuffled copies, and the
-gathering tile products (``ops.expert_linear``, csrc/kernels/routed_ff.hip) on row-major experts; SwiGLU fused into
-the gate/up epilogue.
+gathering tile products (``ops.expert_linear``, csrc/kernels/routed_ff.hip) on row-major experts (the down products of
+many narrow ones: ``ops.grouped_gemm``); SwiGLU fused into the gate/up epilogue.
 
 Expert parallelism, ``ep_size = N`` ranks each owning ``E / N`` experts (attention is tensor-parallel, so
 every rank holds the same T tokens when the block starts):
@@ -276,11 +276,16 @@ class MoEBlock:
 
     def _gathers(self, i, R: int, d: int) -> bool:
         """The expert products read the tokens' rows through the source list (``ops.expert_linear``), so routing writes no
-        permuted copy: layers whose expert weights are row-major only.  Routed decode rows: widths up to 2048 (8 tokens, 16
-        experts of 1536: gate/up + SwiGLU 38.9 + 4.8 -> 37.7 us; 8 experts of 14336 x 4096: 270 + 4.6 -> 292, so wider ones
-        stay on the skinny GEMM)."""
-        return (self._grouped_ok(d) and not self.single_copy and (i, "w13") not in self.pre and (i, "w2") not in self.pre
-                and (R > SKINNY_ROWS or d <= 2048))
+        permuted copy: layers whose expert weights are row-major only.
+
+        Routed decode rows: widths up to 2048 and experts up to 4096, against the skinny GEMM and SwiGLU (us, routing
+        5 us less up to 16 experts and 0 to 4 more at 64): 16 experts of 1536 x 2048, 32 rows 45.9 -> 38.4, of 4096 115 -> 88,
+        of 8192 158 -> 165, of 14336 307 -> 334; 64 of 4096 247 -> 199, of 8192 358 -> 384; 1536 x 1024 19.8 -> 19.6;
+        14336 x 3072 411 -> 491.  Prompts: always (routing of 256 rows to 16 experts 15.5 -> 11.1 us, to 64 20.4 -> 25.2 with
+        fp32 logits in the place of the projection's bf16 ones)."""
+        if not self._grouped_ok(d) or self.single_copy or (i, "w13") in self.pre or (i, "w2") in self.pre:
+            return False
+        return R > SKINNY_ROWS or (d <= 2048 and (self.F <= 4096 or d % 256 != 0))      # (the skinny GEMM: widths in 256s)
 
     def _route(self, i, x):
         """-> (expert ids, weights, place of every choice, segment bounds, rows, source list): rows are x's own with the
@@ -358,7 +363,9 @@ class MoEBlock:
             # -- SwiGLU of the [gate; up] halves in the gate/up epilogue, w2 into fp32 k-split slabs the combine
             # sums.  Below: the weight-streaming kernel on the preshuffled copies up to PRE_ROWS* rows.  Row-major
             # experts: expert_linear (32400 rows, 16 experts of 1536 x 2048, against grouped_gemm's 128 x 128 tiles:
-            # gate/up 645 -> 454 us, w2 357 -> 281; 4000 rows 81 -> 69 and 61 -> 46; 400 rows 39 -> 33 and 27 -> 21)
+            # gate/up 645 -> 454 us, w2 357 -> 281; 4000 rows 81 -> 69 and 61 -> 46; 400 rows 39 -> 33 and 27 -> 21);
+            # w2 of many narrow experts stays on grouped_gemm (64 experts, 800 rows, us: 2048 x 512 33 against 44,
+            # 2048 x 768 45 / 52, 2048 x 1024 57 / 63, 2048 x 1536 84 / 87; 16 experts, 400 rows: 2048 x 768 16 / 13)
             rpe = R / max(1, n_local)
             pg13 = self.pre.get((i, "w13")) if PG_GROUPED and rpe >= PG_ROWS_W13 else None
             pg2 = self.pre.get((i, "w2")) if PG_GROUPED and rpe >= PG_ROWS_W2 else None
@@ -383,11 +390,12 @@ class MoEBlock:
                 return y2
             p2 = self.pre.get((i, "w2")) if self.single_copy or R <= PRE_ROWS * self.E else None
             y2 = self._buf("y2f" if out_f32 else "y2b", (R, d), torch.float32 if out_f32 else torch.bfloat16)
-            if p2 is None:
+            if p2 is None and not (n_local > 32 and F <= 1024):
                 ops.expert_linear(act, None, w2, segments, y2)
             else:
-                ops.grouped_gemm(act, p2, offsets, e_lo, y2, (ops.GROUPED_F32 if out_f32 else ops.GROUPED_BF16)
-                                 + ops.GROUPED_PRESHUFFLED)
+                ops.grouped_gemm(act, w2 if p2 is None else p2, offsets, e_lo, y2,
+                                 (ops.GROUPED_F32 if out_f32 else ops.GROUPED_BF16)
+                                 + (0 if p2 is None else ops.GROUPED_PRESHUFFLED))
             return y2
         # shapes outside the grouped kernel's tiling (not the registered models): per-expert library GEMMs
         offs = offsets.tolist()
