@@ -43,8 +43,6 @@ def main():
     ap.add_argument("--layers", type=int, default=32)
     ap.add_argument("--span", type=int, default=0, help="block-table width in tokens (the graph's context "
                     "bucket; 0: just the context)")
-    ap.add_argument("--wave", type=int, nargs="+", default=[-1],
-                    help="attn_wave settings to pass (one kernel takes every step: they change nothing)")
     ap.add_argument("--heads", type=int, nargs=2, default=[32, 8], metavar=("HQ", "HKV"),
                     help="query / kv heads (one TP rank's shard: 4 1 for Llama-3-8B at TP=8, 8 1 for 70B)")
     args = ap.parse_args()
@@ -71,15 +69,10 @@ def main():
         tmp_o = torch.empty(S, Hq, parts, D, device=dev)
         tmp_ml = torch.empty(S, Hq, parts, 2, device=dev)
         cnt = torch.zeros(S * Hkv, dtype=torch.int32, device=dev)
-        for wv in args.wave:
-            if wv >= 0:
-                torch.ops.symmetry_amd.attn_wave(wv, 0)
-            us = timed(lambda i: ops.attn_decode(q, kc[i % L], vc[i % L], bt, ctxs, out, tmp_o, tmp_ml, cnt,
-                                                 1 / math.sqrt(D)), L)
-            kv_bytes = 2 * S * ctx * Hkv * D * 2
-            print(json.dumps({"kernel": "attn_decode", "heads": [Hq, Hkv], "seqs": S, "ctx": ctx, "span": nb * BS, "wave": wv,
-                              "us": round(us, 2), "TBps": round(kv_bytes / us / 1e6, 3)}), flush=True)
-        torch.ops.symmetry_amd.attn_wave(1024, 513)
+        us = timed(lambda i: ops.attn_decode(q, kc[i % L], vc[i % L], bt, ctxs, out, tmp_o, tmp_ml, cnt, 1 / math.sqrt(D)), L)
+        kv_bytes = 2 * S * ctx * Hkv * D * 2
+        print(json.dumps({"kernel": "attn_decode", "heads": [Hq, Hkv], "seqs": S, "ctx": ctx, "span": nb * BS,
+                          "us": round(us, 2), "TBps": round(kv_bytes / us / 1e6, 3)}), flush=True)
         del kc, vc
 
 

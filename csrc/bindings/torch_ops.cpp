@@ -1214,9 +1214,6 @@ TORCH_LIBRARY(symmetry_amd, m) {
     return std::vector<int64_t>{bm, bn};
   });
   m.def("decode_halves(int on) -> ()", [](int64_t on) { set_decode_halves((int)on); });
-  // (decode attention is one kernel for every batch and context; the two settings that chose among several are accepted)
-  m.def("attn_stream_min(int tokens) -> ()", [](int64_t) {});
-  m.def("attn_wave(int min_units, int min_span) -> ()", [](int64_t, int64_t) {});
   m.def(
       "lm_head_sample(Tensor x, Tensor w, Tensor temps, Tensor seeds, Tensor step, Tensor(a!) tile_keys, "
       "Tensor(b!) out_keys, Tensor(c!) out_ids, int n_offset, Tensor(d!)? logits) -> ()",

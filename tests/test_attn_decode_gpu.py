@@ -1,4 +1,5 @@
-"""Decode attention: batches whose contexts differ widely, on both sides of the rules that cut them into partitions."""
+"""Decode attention within the rounding of every element: contexts around the edges of groups, steps and partitions, and batches
+whose contexts differ widely, on both sides of the rules that cut them into partitions."""
 import pytest
 import torch
 
@@ -61,8 +62,8 @@ class _Batch:
         ops.attn_decode(self.q, self.k, self.v, self.bt, self.ctx, self.out[:-1], self.tmp_o, self.tmp_ml, self.counters, D ** -0.5)
 
     def check(self):
-        """Against 64-bit attention.  P is rounded to bf16 (half a step of 2^-8 of every term), the result once more; the rest is
-        fp32 (scores of |q| |k| ~ 30 to 2^-20, the exponential to 2^-20): 2^-8 (sum p |v| + |o|) bounds it twice over."""
+        """Against 64-bit attention.  P is rounded to bf16 (2^-8 of a term at most, not all one way), the result once more; the rest is
+        fp32 (scores of |q| |k| ~ 30 to 2^-20, the exponential to 2^-20): 2^-8 (sum p |v| + |o|) bounds it."""
         assert not self.counters.any() and bool((self.out[-1] == 7.0).all())
         rep = self.H // self.G
         for s, c in enumerate(self.lens):
@@ -76,6 +77,30 @@ class _Batch:
             want, room = torch.einsum("grc,cgd->grd", p, v), torch.einsum("grc,cgd->grd", p, v.abs())
             err = (self.out[s].double().view(self.G, rep, D) - want).abs()
             assert bool((err <= 2.0 ** -8 * (room + want.abs())).all()), (s, c, float(err.max()))
+
+
+EDGES = [1, 17, 31, 32, 33, 64, 200, 255, 256, 257, 511, 512, 513, 700, 767, 769, 1000, 1025, 2049, 2300, 4100, 4700]
+
+
+def _edges(n):
+    return [EDGES[(5 * i + n) % len(EDGES)] for i in range(n)]
+
+
+@pytest.mark.parametrize("ctx,heads", [
+    (EDGES, (32, 8)), (EDGES, (64, 8)), (EDGES, (8, 1)), (EDGES, (16, 16)),
+    (_edges(65), (32, 8)),                                  # units past a third of the chip: one partition of several steps
+    (_edges(40), (32, 8)), (_edges(30), (32, 8)),           # two and three partitions, steps that do not divide by them
+    (_edges(7), (16, 16)), (_edges(3), (64, 8)),
+    ([4700], (32, 4)), ([4673], (32, 4)), ([33], (8, 2)),   # one sequence: a partition for every step
+])
+@pytest.mark.parametrize("BS", [32, 64])
+def test_contexts_around_the_edges(gpu, ctx, heads, BS):
+    b = _Batch(ctx, heads, BS)
+    b.run()
+    b.check()
+    first = b.out.clone()
+    b.run()                                                 # (finds the counters re-armed)
+    assert torch.equal(first, b.out)
 
 
 def _at(n, short, *longs):

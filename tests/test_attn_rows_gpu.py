@@ -25,8 +25,8 @@ STEPS = [
 @pytest.mark.parametrize("heads", [(8, 1), (32, 8), (16, 4)])
 @pytest.mark.parametrize("step", range(len(STEPS)))
 def test_prompt_rows(step, heads, BS):
-    """Against 64-bit attention.  P is rounded to bf16 (half a step of 2^-8 of every term), the result once more; the rest is
-    fp32 (scores of |q| |k| ~ 30 to 2^-20, the exponential to 2^-20): 2^-8 (sum p |v| + |o|) bounds it twice over.  Places past a
+    """Against 64-bit attention.  P is rounded to bf16 (2^-8 of a term at most, not all one way), the result once more; the rest is
+    fp32 (scores of |q| |k| ~ 30 to 2^-20, the exponential to 2^-20): 2^-8 (sum p |v| + |o|) bounds it.  Places past a
     context hold large values, which no row may see."""
     H, Hkv = heads
     runs = STEPS[step]
