@@ -8,9 +8,9 @@
 // head h / (H / G).  Key and value head sizes are independent (dk, dv).  Scores, softmax statistics, weights and the
 // weighted sum are fp32.
 //
-// window_attn_wave_kernel: one to eight waves per (row, head), every shape, bf16 or fp32.  The window is walked in
-// tiles of 64 keys: each lane scores one key (the query sits in LDS as fp32, the key row is read in 16-byte pieces
-// where the head size allows), the wave forms the tile's running max / sum, then the lanes switch to value columns
+// window_attn_wave_kernel: one to sixteen waves per (row, head), every shape, bf16 or fp32.  The window is walked in
+// tiles of 64 keys: each lane gets one key's score (the query sits in LDS as fp32; bf16 keys of 64 or 128 entries are read
+// row by row by groups of lanes, others lane by lane in 16-byte pieces where the head size allows), the wave forms the tile's running max / sum, then the lanes switch to value columns
 // and add the tile's weighted value rows (weights read lane by lane, value rows read coalesced).
 #include "common.h"
 #include "hybrid_launchers.h"
