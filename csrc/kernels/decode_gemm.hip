@@ -25,7 +25,6 @@
 // workgroups, so every epilogue sees final values), U 64-deep k blocks in flight per wave, partial
 // accumulators summed through LDS.  MFMA v_mfma_f32_16x16x32_bf16, natural k order (each load
 // instruction reads 16 rows x 64 contiguous bytes).
-#include "attn_decode.h"
 #include "common.h"
 #include "decode_epi.h"
 #include "launchers.h"

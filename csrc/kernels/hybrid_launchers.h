@@ -66,10 +66,10 @@ struct ConvArgs {
 };
 void launch_causal_conv_silu(const ConvArgs& a, int f32, hipStream_t s);
 void launch_conv_state_update(const ConvArgs& a, int f32, hipStream_t s);
-// out = relu(a)^2
-// false: this K has no kernel
+// out = x . W^T (relu2: of relu(x)^2; glu: silu(gate) * up of W's [gate | up] rows); false: this K has no kernel
 bool launch_row_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int f32_out,
                        int relu2, int glu, hipStream_t s);
+// out = relu(a)^2
 void launch_relu_sq(const void* a, long long lda, void* out, int R, int F, int f32, hipStream_t s);
 // out = silu(gate) * up
 void launch_silu_mul(const void* gate, long long ldg, const void* up, long long ldu, void* out, int R, int F, int f32,

@@ -316,8 +316,7 @@ void launch_stream(const ExpertArgs& a, hipStream_t s) {
 // Prompt steps: tiles of BM rows x BN weight rows, waves in WR rows x WC columns, K in steps of 64 through two LDS stages filled by
 // direct global -> LDS loads.  LDS rows are 128 B with the 16-byte chunk c stored at c ^ ((row >> 1) & 7) (swizzled on the
 // load's source), so fragment reads do not conflict.  K % 64 == 0.
-// EPI_GLU: half of a wave's weight rows are gate rows and half the same up
-// rows, so a pair meets in registers.
+// EPI_GLU: half of a wave's weight rows are gate rows and half the up rows of the same outputs, so a pair meets in registers.
 // The tile list is counted on the device; a workgroup without a tile exits before any barrier.  Tiles are dealt to the 8 XCDs
 // in contiguous runs (workgroup i runs on XCD i % 8) and walk GN column tiles of every row tile of an expert before the next
 // GN, so an expert's weights and a tile row's activations are shared in one L2 (16384 rows, 8 experts of 2 x 14336 x 4096:

@@ -186,7 +186,7 @@ def build_latent(verbose: bool = False, force: bool = False) -> str:
 
 
 def build_hybrid(verbose: bool = False, force: bool = False) -> str:
-    """csrc/kernels/{hybrid_rows,stream_rows,norm_rows,routed_ff,window_attention,prompt_attention,split_attention,decay_scan,decay_chunk,delta_rule,row_linear,expert_tiles,glu_moe}.hip + csrc/bindings/hybrid_ops.cpp ->
+    """csrc/kernels/{hybrid_rows,stream_rows,norm_rows,routed_ff,window_attention,prompt_attention,split_attention,decay_scan,decay_chunk,delta_rule,row_linear,glu_moe}.hip + csrc/bindings/hybrid_ops.cpp ->
     symmetry_amd/_C_hybrid.so (``torch.ops.symmetry_amd_hybrid``)."""
     os.makedirs(OBJ, exist_ok=True)
     kdir = os.path.join(CSRC, "kernels")
