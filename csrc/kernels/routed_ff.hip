@@ -542,7 +542,10 @@ int launch_expert_linear(const ExpertArgs& a, int f32, int impl, hipStream_t s) 
       // 32 rows, 16 x 2 x 1536 x 2048 with 14 experts chosen)
       expert_stream_kernel<1, 4, 2, EPI_GLU><<<dim3((a.N + 15) / 16, a.E), 256, 0, s>>>(a);
     } else if (per <= 8) {
-      if (deep == 3) launch_stream<1, 8, 3>(a, s);      // (no steps left over: 21.8 us, 25 with 4 at 2048 x 1536)
+      // widths of 1536 to 2016: every wave has 3 steps or 4, and with 4 in flight those of 3 would load them one by one (16
+      // experts, 32 rows, 2048 outputs, us, 4 -> 3 in flight: 1536 28.6 -> 23.6, 1568 29.5 -> 24.9, 1792 30.4 -> 28.2, 2016
+      // 35.8 -> 32.5)
+      if (deep == 3) launch_stream<1, 8, 3>(a, s);
       else launch_stream<1, 8, 4>(a, s);
     } else if (per <= 24) {
       launch_stream<2, 4, 2>(a, s);
