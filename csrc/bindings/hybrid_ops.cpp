@@ -722,7 +722,7 @@ int64_t expert_linear(const Tensor& x, const OptTensor& src, const Tensor& W, co
   }
   a.x = x.data_ptr(), a.W = W.data_ptr(), a.offsets = ptr<int>(offsets), a.y = y.data_ptr();
   a.R = (int)R, a.E = (int)E, a.N = (int)y.size(1), a.K = (int)W.size(2), a.relu2 = relu2;
-  a.glu = glu, a.f32_out = y32 && !f32;
+  a.xrows = (int)x.size(0), a.glu = glu, a.f32_out = y32 && !f32;
   TORCH_CHECK(!(a.glu || a.f32_out) || (expert_linear_mfma(a, f32) && E <= 65535 && (impl < 0 || (impl == 1) || (impl > 1 && a.K % 64 == 0))),
               "expert_linear: glu and fp32 output take bf16 rows of a multiple of 32, 16-byte aligned");
   const at::OptionalDeviceGuard g(x.device());

@@ -11,6 +11,11 @@ SYM_DEV unsigned int lds_address(const void* p) {
 SYM_DEV void direct_load16(const void* src, unsigned int lds) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }
+// the same through a buffer's four words: its base, + `off` bytes of the lane, + `soff` bytes
+SYM_DEV void direct_buffer_load16(u32x4 buf, int off, int soff, unsigned int lds) {
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(off), "s"(buf), "s"(soff)
+               : "memory", "m0");
+}
 SYM_DEV void direct_load4(const void* src, unsigned int lds) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }

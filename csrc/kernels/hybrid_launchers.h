@@ -191,6 +191,7 @@ struct ExpertArgs {
   const int* offsets;
   void* y;
   int R, E, N, K, relu2;
+  int xrows;      // rows of x
   int glu;        // W [E][2 N][K] holds [gate | up] rows, y = silu(gate) * up
   int f32_out;    // y fp32 (neither relu2 nor glu)
 };

@@ -9,13 +9,16 @@
 // bf16 values and their sums are exact to fp32 accumulation).  A step of at most 16 tokens is one workgroup, which then also
 // lays out the segments; larger steps take one more launch.
 // Expert products in bf16: a weight-streaming kernel for few rows per expert (a wave per 16 weight rows and width slice, the
-// rows of the segment as the other MFMA operand), and a 128 x 128 or 256 x 256 tile kernel staged through LDS by direct loads
-// for prompt steps.  Other shapes and fp32: the all-shapes segment product of glu_moe.hip.
+// rows of the segment as the other MFMA operand), and for prompt steps a 128 x 128 tile kernel and a persistent one of 256 x 256,
+// staged through LDS by direct loads.  Other shapes and fp32: the all-shapes segment product of glu_moe.hip.
 #include "common.h"
 #include "direct_lds.h"
 #include "hybrid_launchers.h"
 #include "latent_launchers.h"
 #include "wave_dot.h"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -323,6 +326,36 @@ void launch_stream(const ExpertArgs& a, hipStream_t s) {
 // 0.78 -> 1.13 PFLOP/s).
 constexpr int GN = 8;
 
+// outputs n .. n + 3 of a row (at: the first one's place); vec: N is a multiple of 4
+template <bool F32, bool NT = false>
+SYM_DEV void store_quad(void* y, long long at, f32x4 f, int n, int N, bool vec) {
+  if constexpr (F32) {
+    float* o = reinterpret_cast<float*>(y) + at;
+    if (vec) {
+      if (n < N) {
+        if constexpr (NT) __builtin_nontemporal_store(f, reinterpret_cast<f32x4*>(o));
+        else *reinterpret_cast<f32x4*>(o) = f;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (n + u < N) o[u] = f[u];
+    }
+  } else {
+    bf16* o = reinterpret_cast<bf16*>(y) + at;
+    bf16x4 v;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = (bf16)f[u];
+    if (vec) {
+      if (n < N) *reinterpret_cast<bf16x4*>(o) = v;
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (n + u < N) o[u] = v[u];
+    }
+  }
+}
+
 SYM_DEV int chunk_swz(int row) { return (row >> 1) & 7; }
 
 template <int BM, int BN, int WR, int WC, int EPI>
@@ -428,28 +461,7 @@ __global__ __launch_bounds__(64 * WR * WC) void expert_tile_kernel(ExpertArgs a)
         if constexpr (EPI == EPI_GLU) f[u] = silu(f[u]) * acc[i + NO][q][u];
         if constexpr (EPI == EPI_RELU2) f[u] = relu2f(f[u]);
       }
-      if constexpr (EPI == EPI_F32) {
-        float* o = reinterpret_cast<float*>(a.y) + at;
-        if (vec) {
-          if (n < N) *reinterpret_cast<f32x4*>(o) = f;
-        } else {
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (n + u < N) o[u] = f[u];
-        }
-      } else {
-        bf16* o = reinterpret_cast<bf16*>(a.y) + at;
-        bf16x4 v;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = (bf16)f[u];
-        if (vec) {
-          if (n < N) *reinterpret_cast<bf16x4*>(o) = v;
-        } else {
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (n + u < N) o[u] = v[u];
-        }
-      }
+      store_quad<EPI == EPI_F32>(a.y, at, f, n, N, vec);
     }
   }
 }
@@ -457,11 +469,6 @@ __global__ __launch_bounds__(64 * WR * WC) void expert_tile_kernel(ExpertArgs a)
 template <int BM, int BN, int WR, int WC, int EPI>
 void launch_tile(const ExpertArgs& a, hipStream_t s) {
   constexpr int lds = 2 * (BM + BN) * 128, OUT = EPI == EPI_GLU ? BN / 2 : BN;
-  if (lds > 64 * 1024) {
-    static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_tile_kernel<BM, BN, WR, WC, EPI>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    (void)once;
-  }
   const long long tiles = (long long)((a.N + OUT - 1) / OUT) * ((a.R + BM - 1) / BM + a.E);
   expert_tile_kernel<BM, BN, WR, WC, EPI><<<(unsigned)((tiles + 7) / 8 * 8), 64 * WR * WC, lds, s>>>(a);
 }
@@ -472,6 +479,250 @@ void launch_tiles(const ExpertArgs& a, hipStream_t s) {
   else if (a.relu2) launch_tile<BM, BN, WR, WC, EPI_RELU2>(a, s);
   else if (a.f32_out) launch_tile<BM, BN, WR, WC, EPI_F32>(a, s);
   else launch_tile<BM, BN, WR, WC, EPI_BF16>(a, s);
+}
+
+// Prompt steps with many rows an expert: one persistent workgroup a CU, 8 waves in 2 x 4, tiles of 256 rows x 256 weight rows (a
+// wave: 128 x 64) and of 128 x 256 for what a segment leaves over.  K in stages of 64.  A wave reads its fragments half a stage
+// ahead of their products, so a stage's LDS is free from its middle on, where its one barrier stands: the rows of the stage after
+// next (two buffers) load behind it, the weight rows of that stage (three buffers) in front of it, all between products.  The
+// stages run on over the tile boundaries: a tile's first two load while the last products and the epilogue of the one before run.
+// Every XCD walks its run of the tiles whole ones first; the whole ones that would be left for a last partial round are cut in two.
+// LDS rows as in expert_tile_kernel.  K % 64 == 0, K >= PERSIST_K, x and an expert's weights below 2 GiB.
+constexpr int PERSIST_K = 512, PERSIST_OP = 32 * 1024, PERSIST_LDS = 5 * PERSIST_OP;
+
+struct ExpertTile {
+  int e, r0, rows, n0, half;      // half: 128 rows at most
+};
+
+SYM_DEV u32x4 buffer_words(const void* base, long long bytes) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(base);
+  return u32x4{(unsigned int)p, (unsigned int)(p >> 32) & 0xffffu, (unsigned int)bytes, 0x00020000u};
+}
+
+SYM_DEV int lanes_upto(int v, int lane) {      // inclusive sum over the lanes
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int w = __shfl_up(v, o, 64);
+    if (lane >= o) v += w;
+  }
+  return v;
+}
+
+template <int EPI>
+__global__ __launch_bounds__(512, 1) void expert_persist_kernel(ExpertArgs a) {
+  constexpr int OUT = EPI == EPI_GLU ? 128 : 256, WO = OUT / 4, NO = WO / 16;      // outputs of a tile, of a wave; in 16s
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int K = a.K, N = a.N, nb = (N + OUT - 1) / OUT, nk = K / 64;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = wave >> 2, wc = wave & 3;
+
+  // ---- this workgroup's tiles.  Whole and half row tiles of an expert; lane l: those of all experts up to its share of them
+  auto segment = [&](int e, int& r0, int& r1, int& w, int& h) {
+    r0 = a.offsets[e], r1 = max(r0, min(a.offsets[e + 1], a.R));
+    const int left = (r1 - r0) & 255;
+    w = (r1 - r0) / 256 + (left > 128), h = left > 0 && left <= 128;
+  };
+  const int share = (a.E + 63) / 64;
+  int whole = 0, halves = 0;
+  for (int e = lane * share; e < min((lane + 1) * share, a.E); ++e) {
+    int r0, r1, w, h;
+    segment(e, r0, r1, w, h);
+    whole += w, halves += h;
+  }
+  whole = lanes_upto(whole, lane), halves = lanes_upto(halves, lane);
+  const int wgs = gridDim.x >> 3, xcd = blockIdx.x & 7;      // (the grid is a multiple of 8)
+  const int wtotal = __builtin_amdgcn_readlane(whole, 63) * nb, htotal = __builtin_amdgcn_readlane(halves, 63) * nb;
+  const int wper = (wtotal + 7) / 8, hper = (htotal + 7) / 8;
+  const int w0 = xcd * wper, wn = max(0, min(wper, wtotal - w0)), h0 = xcd * hper, hn = max(0, min(hper, htotal - h0));
+  const int over = wn % wgs;      // (a half tile takes 5 / 9 of a whole one's time)
+  const bool cut = over && 5 * ((2 * over + hn + wgs - 1) / wgs) < 9 + 5 * ((over + hn - 1) / wgs);
+  const int wkeep = cut ? wn - over : wn, wcut = cut ? 2 * over : 0, count = wkeep + wcut + hn;
+  auto find = [&](int s) {
+    ExpertTile r;
+    r.half = s >= wkeep;
+    const bool rest = s >= wkeep + wcut;
+    const int g = rest ? h0 + s - wkeep - wcut : w0 + (r.half ? wkeep + ((s - wkeep) >> 1) : s);
+    const int upto = rest ? halves : whole, l = __builtin_popcountll(__ballot(upto * nb <= g));      // (some lane's sum lies above)
+    int e = l * share, lo = l ? __builtin_amdgcn_readlane(upto, l - 1) : 0, s0, s1, w, h;
+    segment(e, s0, s1, w, h);
+    while ((lo + (rest ? h : w)) * nb <= g) {
+      lo += rest ? h : w;
+      segment(++e, s0, s1, w, h);
+    }
+    int m = w, n = g - lo * nb;
+    if (!rest) {
+      const int gr = n / (GN * w), in = n - gr * GN * w, cols = min(GN, nb - GN * gr);
+      m = in / cols;
+      n = GN * gr + in - m * cols;
+    }
+    r.e = e;
+    r.r0 = s0 + 256 * m + (!rest && r.half ? 128 * ((s - wkeep) & 1) : 0);
+    r.rows = min(r.half ? 128 : 256, s1 - r.r0);
+    r.n0 = OUT * n;
+    return r;
+  };
+  int slot = blockIdx.x >> 3;
+  if (slot >= count) return;
+
+  // ---- direct loads: instruction i of 4 covers rows 64 i + 8 wave + lane / 8 of an operand.  EPI_GLU: 32 gate rows and 32 up
+  // rows of the same outputs in every 64, so that a pair meets in a wave.
+  const int lrow = 8 * wave + (lane >> 3), lch = (lane & 7) ^ chunk_swz(lrow);
+  int aoff[4], boff = 0, blast = 0;      // (weight rows past the expert's last re-read it)
+  u32x4 xbuf = buffer_words(a.x, (long long)a.xrows * K * 2), wbuf;
+  int ahalf = 0, kx = 0;      // of the tile being loaded; bytes of a row behind the stage to load
+  auto bind = [&](const ExpertTile& t) {
+    ahalf = t.half;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int p = t.r0 + min(64 * i + lrow, t.rows - 1);          // rows past the segment re-read its last one (never stored)
+      aoff[i] = (a.src ? a.src[p] : p) * K * 2 + 16 * lch;
+    }
+    const int up = EPI == EPI_GLU ? (lrow >> 5) * N : 0;
+    boff = (t.n0 + (EPI == EPI_GLU ? lrow & 31 : lrow) + up) * K * 2 + 16 * lch;
+    blast = (N - 1 + up) * K * 2 + 16 * lch;
+    const long long wrows = (EPI == EPI_GLU ? 2LL : 1LL) * N;
+    wbuf = buffer_words(reinterpret_cast<const bf16*>(a.W) + t.e * wrows * K, wrows * K * 2);
+  };
+  const unsigned int lds0 = lds_address(smem) + wave * 1024;
+  const int wstep = OUT / 4 * K * 2;
+  unsigned int afill = 0, bfill = 0;      // the buffers to fill
+  auto load_a = [&](int i) {
+    if (i < 2 || !ahalf) direct_buffer_load16(xbuf, aoff[i], kx, lds0 + afill + 8192 * i);
+  };
+  auto load_b = [&](int i) {
+    direct_buffer_load16(wbuf, min(boff + i * wstep, blast), kx, lds0 + 2 * PERSIST_OP + bfill + 8192 * i);
+  };
+  ExpertTile cur = find(slot), next = cur;
+  bool more = slot + wgs < count;
+  if (more) next = find(slot + wgs);
+  auto turn_b = [&](unsigned int b) { return b == 2 * PERSIST_OP ? 0u : b + PERSIST_OP; };
+  auto loaded = [&]() {      // a stage's loads are out
+    afill ^= PERSIST_OP;
+    bfill = turn_b(bfill);
+    kx += 128;
+    if (kx == 2 * K) {
+      kx = 0;
+      if (more) bind(next);      // (behind the last tile: its own start again, into buffers that are not read any more)
+    }
+  };
+
+  f32x4 acc[4][8];
+  Pack8 f0[12], f1[12];      // the fragments of a stage's halves: 4 of weight rows, 8 of rows
+  const int j = lane & 15, hq = lane >> 4;
+  const int c0 = j * 128 + 16 * (hq ^ chunk_swz(j));      // of the first half; the second half's chunks are 64 bytes across
+  unsigned int ard = 0, brd = 0;      // the buffers of the stage at hand
+  auto fragment = [&](Pack8 (&f)[12], int c, unsigned int arow, int i) {
+    if (i < 4) f[i].u = *reinterpret_cast<const uint4*>(smem + 2 * PERSIST_OP + brd + 8192 * wc + c + 2048 * i);
+    else f[i].u = *reinterpret_cast<const uint4*>(smem + ard + arow + c + 2048 * (i - 4));
+  };
+  // one stage of a tile of 32 NQ rows; arow: where the wave's rows stand in a buffer, anext: in the next stage's
+  auto stage = [&](auto start, auto nq, unsigned int arow, unsigned int anext, bool stores) __attribute__((always_inline)) {
+    constexpr int NQ = decltype(nq)::value;
+    int c1 = c0;
+    asm volatile("v_xor_b32 %0, 64, %0" : "+v"(c1));      // (kept in a register it would cost another one's spill)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      load_b(i);
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        if (3 * i + u < 4 + NQ) fragment(f1, c1, arow, 3 * i + u);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) acc[i][q] = mfma16(f0[i].v, f0[4 + q].v, decltype(start)::value ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[i][q]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // every wave: the next stage has landed, this one's fragments are in registers
+    if (stores) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 + 8 * NO) : "memory");
+    else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    ard ^= PERSIST_OP;
+    brd = turn_b(brd);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      load_a(i);
+#pragma unroll
+      for (int u = 0; u < 3; ++u) fragment(f0, c0, anext, 3 * i + u);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) acc[i][q] = mfma16(f1[i].v, f1[4 + q].v, acc[i][q]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    loaded();
+  };
+  auto rows_at = [&](const ExpertTile& t) { return (unsigned int)(t.half ? 8192 : 16384) * wr; };
+  const bool vec = (N & 3) == 0;
+  bool stores = false;      // a whole tile's stores stand behind the loads that are waited for
+  auto tile = [&](auto nq) __attribute__((always_inline)) {
+    constexpr int NQ = decltype(nq)::value;
+    const unsigned int arow = rows_at(cur), anext = rows_at(next);
+    stage(std::true_type{}, nq, arow, arow, stores);
+    for (int k = 1; k < nk; ++k) stage(std::false_type{}, nq, arow, k + 1 < nk ? arow : anext, false);
+    // lane (j, hq): output row 16 q + j of the wave's rows, columns 16 i + 4 hq + 0..3 of its columns
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int m = 16 * NQ * wr + 16 * q + j;
+      if (m < cur.rows) {
+#pragma unroll
+        for (int i = 0; i < NO; ++i) {
+          const int n = cur.n0 + WO * wc + 16 * i + 4 * hq;
+          f32x4 v = acc[i][q];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if constexpr (EPI == EPI_GLU) v[u] = silu(v[u]) * acc[i + NO][q][u];
+            if constexpr (EPI == EPI_RELU2) v[u] = relu2f(v[u]);
+          }
+          // (fp32 rows go past the caches: a round of tiles writes twice what the L2 holds, and the operands stay there; 32400 rows,
+          // 16 experts of 2048 x 1536: 233 -> 212 us.  The 16-bit rows of a gated product are read next: 350 -> 369 that way)
+          store_quad<EPI == EPI_F32, EPI == EPI_F32>(a.y, (long long)(cur.r0 + m) * N + n, v, n, N, vec);
+        }
+      }
+    }
+    stores = NQ == 8 && vec && cur.rows == 256 && cur.n0 + OUT <= N;
+  };
+
+  bind(cur);
+  wait_direct_loads();
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load_b(i);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load_a(i);
+    loaded();
+  }
+  if (ahalf) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+  else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < 12; ++i) fragment(f0, c0, rows_at(cur), i);
+  while (true) {
+    if (cur.half) tile(std::integral_constant<int, 4>{});
+    else tile(std::integral_constant<int, 8>{});
+    if (!more) break;
+    cur = next;
+    slot += wgs;
+    more = slot + wgs < count;
+    if (more) next = find(slot + wgs);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // no load may land in LDS that is not this workgroup's any more
+}
+
+int cu_count() {
+  int dev = 0, cus = 256;
+  (void)hipGetDevice(&dev);
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  return cus;
+}
+
+template <int EPI>
+void launch_persist(const ExpertArgs& a, hipStream_t s) {
+  static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_persist_kernel<EPI>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, PERSIST_LDS);
+  (void)once;
+  constexpr int OUT = EPI == EPI_GLU ? 128 : 256;
+  const long long tiles = (long long)((a.N + OUT - 1) / OUT) * ((a.R + 127) / 128 + a.E);
+  const long long grid = std::min<long long>((tiles + 7) / 8 * 8, std::max(8, cu_count() / 8 * 8));
+  expert_persist_kernel<EPI><<<(unsigned)grid, 512, PERSIST_LDS, s>>>(a);
 }
 
 template <int NW, int NE>
@@ -524,17 +775,27 @@ bool expert_linear_mfma(const ExpertArgs& a, int f32) {
 
 // Returns the form used: 0 all shapes, 1 weight stream, 2 / 3 tiles of 128 / 256
 // Stream or tile, measured at 16 experts, 4 rows each on average: [gate | up] of 1536 x 2048 46.0 us on both, 2048 x 1536 23.9
-// against 28.8; at 16 rows each 53 against 46.6 and 33 against 28.7.  Tiles of 256 have one workgroup on a CU, so a tile's
-// epilogue stands alone: they win where the width is long (16384 rows, 8 experts: 2 x 14336 x 4096 3401 us against 3742,
-// 4096 x 14336 1880 against 2156; 32400 rows, 16 experts: 2048 x 1536 274 against 281), not where a gated product over 2048
-// ends in its exponentials (480 against 454).
+// against 28.8; at 16 rows each 53 against 46.6 and 33 against 28.7.
+// Persistent tiles against those of 128, us: 16 experts, gated 1536 x 2048 and 2048 x 1536, at 96 rows each 43.9 -> 46.0 and 29.0 ->
+// 30.5, 128 62.9 -> 52.2 and 35.2 -> 31.8, 512 124 -> 112 and 76 -> 77, 2025 446 -> 360 and 276 -> 212; 8 experts, gated 14336 x
+// 4096 and 4096 x 14336, at 64 rows 374 -> 420 and 244 -> 256, 128 511 -> 452 and 311 -> 270, 2048 3740 -> 3018 and 2160 -> 1650
+// (1.28 and 1.17 PFLOP/s); 64 experts, 2048 x 1024 at 128 rows 110 -> 83.  Widths below 1024 pay a tile's start and end over few
+// stages: 512, 16 experts, 2048 outputs, 512 rows 40.4 -> 47.7, 2025 rows 126.6 -> 122.4, gated 195.8 -> 175.7; 512 outputs of
+// 2025 rows 40.5 -> 48.3.  Where the gated tiles fill 0.7 to 1 round of the CUs, most of them get a second half tile: 16 experts
+// of 256 rows (0.75 rounds) 73 -> 80, of 224 65 -> 56, of 288 90 -> 88.
 int launch_expert_linear(const ExpertArgs& a, int f32, int impl, hipStream_t s) {
   if (a.R <= 0) return 0;
   const bool mfma = expert_linear_mfma(a, f32);
   const int per = (a.R + a.E - 1) / a.E;      // rows per expert if they are spread evenly
   const bool stream = mfma && a.E <= 65535, tile = mfma && a.K % 64 == 0;
-  const bool big = per >= 512 && a.N >= 256 && (!a.glu || a.K >= 4096);
-  if (impl < 0) impl = stream && (per <= 8 || !tile) ? 1 : (tile ? (big ? 3 : 2) : (stream ? 1 : 0));
+  const long long top = 0x7fffffffLL;      // (a buffer's range, and a lane's offset in it)
+  const bool fits = tile && a.K >= PERSIST_K && a.xrows * 2LL * a.K <= top && ((a.glu ? 2LL : 1LL) * a.N + 512) * 2 * a.K <= top;
+  if (impl < 0) {
+    const long long tiles = (long long)((a.N + 255) / 256) * (a.glu ? 2 : 1) * (a.R / 256), cus = cu_count();
+    const bool rounds = !a.glu || 10 * tiles <= 7 * cus || tiles >= cus;
+    const bool big = fits && a.N >= 256 && (a.K >= 1024 ? per >= 128 && rounds : per >= 1024 && a.N >= 1024);
+    impl = stream && (per <= 8 || !tile) ? 1 : (tile ? (big ? 3 : 2) : (stream ? 1 : 0));
+  }
   if (impl == 1 && stream) {
     const int deep = a.K / 512;               // 64-element steps of each of 8 waves
     if (per <= 8 && a.glu) {
@@ -554,12 +815,16 @@ int launch_expert_linear(const ExpertArgs& a, int f32, int impl, hipStream_t s) 
     }
     return 1;
   }
+  if (impl == 3 && !fits) impl = 2;
   if (impl == 2 && tile) {
     launch_tiles<128, 128, 2, 2>(a, s);
     return 2;
   }
   if (impl == 3 && tile) {
-    launch_tiles<256, 256, 2, 4>(a, s);
+    if (a.glu) launch_persist<EPI_GLU>(a, s);
+    else if (a.relu2) launch_persist<EPI_RELU2>(a, s);
+    else if (a.f32_out) launch_persist<EPI_F32>(a, s);
+    else launch_persist<EPI_BF16>(a, s);
     return 3;
   }
   if (a.glu || a.f32_out) return -1;      // (the binding has refused it)

@@ -137,3 +137,43 @@ def test_a_device_that_is_not_the_current_one():
             got.append([t.cpu() for t in (ids, w, off, dst, src, y)])
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("E,R,N,K", [(3, 700, 256, 512), (4, 1000, 300, 576), (5, 2600, 262, 1024), (2, 1, 512, 512),
+                                     (16, 9000, 2048, 512), (7, 5000, 1028, 1088), (70, 9100, 260, 512), (130, 3000, 512, 576)])
+def test_persistent_tiles(E, R, N, K):
+    """The persistent form where its tiles end: segments around 128 and 256 rows, several tiles a workgroup, whole ones cut for the
+    last round, more experts than lanes, odd stage counts, outputs that fill no tile.  Bounds as above; the squared ReLU of p
+    with error eps is off by 2 |p| eps + eps^2."""
+    print("persistent tiles", E, R, N, K, flush=True)
+    torch.manual_seed(R + K)
+    sizes = [0, 1, 127, 128, 129, 255, 256, 257, 384, 385][: E - 1]
+    while sum(sizes) > R:
+        sizes.pop()
+    sizes += [0] * (E - 1 - len(sizes))
+    rest = R - sum(sizes)
+    sizes = [s + rest // E for s in sizes]
+    off = torch.tensor([0] + sizes).cumsum(0).tolist() + [R]
+    x, W = torch.randn(R // 2 + 1, K).to(BF16).cuda(), (torch.randn(E, 2 * N, K) * K ** -0.5).to(BF16).cuda()
+    src = torch.randint(0, x.shape[0], (R,)).int().cuda()
+    p = torch.empty(R, 2 * N, dtype=torch.float64, device="cuda")
+    for e in range(E):
+        a, b = off[e], off[e + 1]
+        p[a:b] = x[src[a:b].long()].double() @ W[e].double().t()
+    g, u = p[:, :N], p[:, N:]
+    eps = 4 * K ** 0.5 * 2.0 ** -24 * x.double().norm(dim=1).max() * W.double().norm(dim=2).max()
+    H, od = ops._hyb(), torch.tensor(off, dtype=torch.int32, device="cuda")
+    half = W[:, :N].contiguous()
+    y = torch.full((R + 1, N), 7.0, device="cuda")
+    assert H.expert_linear(x, src, half, od, y[:R], False, 3) == 3
+    assert ((y[:R].double() - g).abs() <= eps).all() and (y[R] == 7.0).all()
+    z = torch.full((R + 1, N), 7.0, dtype=BF16, device="cuda")
+    assert H.expert_linear(x, src, W, od, z[:R], False, 3, True) == 3
+    want = g / (1 + torch.exp(-g)) * u
+    assert ((z[:R].double() - want).abs() <= (2.0 ** -8 + 2.0 ** -20) * want.abs() + 1.1 * eps * (g.abs() + u.abs()) + 1e-30).all()
+    assert (z[R] == 7.0).all()
+    assert H.expert_linear(x[src.long()], None, half, od, z[:R], True, 3) == 3
+    want = g.clamp(min=0) ** 2
+    assert ((z[:R].double() - want).abs() <= 2.0 ** -8 * want + 2 * g.abs() * eps + eps ** 2).all()
+    assert H.expert_linear(x, src, half, od, z[:R], False, 3) == 3
+    assert ((z[:R].double() - g).abs() <= 2.0 ** -8 * g.abs() + 2 * eps).all()
