@@ -69,9 +69,15 @@ SYM_DEV u32x4 half_swap(u32x4 keep, u32x4 from) {
 // lanes hold the block's first 32-deep step, lanes 8-15 its second.  Two such loads (rows 0-7, rows 8-15) become the two
 // steps' A operands by exchanging halves, 4 v_mov_dpp each.  With RH = 8 there is one load, and rows 8-15 of the product
 // are dropped.
-template <int RT, int RH, int NW, int U, int EPI, bool XF>
+//
+// M8: RH = 8 and at most 8 rows of x, which then are read like the weights.  One product of the two registers as they are
+// holds the first step's result in its upper left quarter and the second's in its lower right one (the others mix the steps
+// and are dropped): half the x traffic, which is twice the weights' otherwise, half the matrix products and no exchange.
+template <int RT, int RH, int NW, int U, int EPI, bool XF, bool M8 = false>
 __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
+  static_assert(!M8 || (RH == 8 && RT == 1 && EPI != EPI_GLU), "M8: one tile of 8 rows");
   constexpr int LD = RH / 8;  // loads of a block
+  constexpr int XL = M8 ? 1 : 2;
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, h = lane >> 4;
   const int n0 = blockIdx.x * (EPI == EPI_GLU ? RH : RH * RT);
@@ -89,14 +95,14 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
       wo[rt][l] = (unsigned)((min(first + 8 * l + (r16 & 7), a.N - 1) - base) * a.K + 4 * (r16 & 8) + 8 * h) * 2;
   }
   const char* xb = reinterpret_cast<const char*>(a.x);
-  const unsigned xo = (unsigned)(min(r16, a.M - 1) * a.ldx + 8 * h) * 2;
+  const unsigned xo = (unsigned)(min(M8 ? r16 & 7 : r16, a.M - 1) * a.ldx + (M8 ? 4 * (r16 & 8) : 0) + 8 * h) * 2;
 
   f32x4 acc[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) acc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   u32x4 w[2][U][RT][LD];
-  Pack8 xv[U][2];
+  Pack8 xv[U][XL];
   auto load_w = [&](int b, int blk) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -109,23 +115,28 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) xv[u][t].w = *reinterpret_cast<const u32x4*>(xb + 128 * (blk + u) + 64 * t + xo);
+      for (int t = 0; t < XL; ++t) xv[u][t].w = *reinterpret_cast<const u32x4*>(xb + 128 * (blk + u) + 64 * t + xo);
   };
   auto multiply = [&](int b) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if constexpr (XF) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t) relu_squared(xv[u][t]);
+        for (int t = 0; t < XL; ++t) relu_squared(xv[u][t]);
       }
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
         Pack8 f0, f1;
+        if constexpr (M8) {
+          f0.w = w[b][u][rt][0];
+          acc[rt] = mfma16(f0.v, xv[u][0].v, acc[rt]);
+          continue;
+        }
         const u32x4 lo = w[b][u][rt][0], hi = w[b][u][rt][LD - 1];
         f0.w = LD == 2 ? half_swap<0xc>(lo, hi) : lo;
         f1.w = half_swap<0x3>(hi, lo);
         acc[rt] = mfma16(f0.v, xv[u][0].v, acc[rt]);
-        acc[rt] = mfma16(f1.v, xv[u][1].v, acc[rt]);
+        acc[rt] = mfma16(f1.v, xv[u][XL - 1].v, acc[rt]);
       }
     }
   };
@@ -164,9 +175,98 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
     f32x4 v = red[0][rt][lane];
 #pragma unroll
     for (int i = 1; i < NW; ++i) v += red[i][rt][lane];
+    if constexpr (M8) {  // lane 40 on: the second step's part
+#pragma unroll
+      for (int i = 0; i < NW; ++i) v += red[i][rt][(lane + 40) & 63];
+    }
     return v;
   };
   store_rows<RH, EPI>(a, n0 + RH * wid, lane, sum(wid), EPI == EPI_GLU ? sum(RT - 1) : f32x4{});
+}
+
+// Many tiles: x stays in registers.  A workgroup's waves hold their shares of x (KB 64-deep blocks each, K = 64 NW KB) and walk
+// the 16-row tiles blockIdx.x, + gridDim.x, ..  Read per tile, x costs up to as much L2 traffic as the weights cost HBM.  The
+// next tile's weights are in flight while a tile is multiplied (two tiles ahead is slower, 8 rows of 8192 x 2048 gated 13.8 ->
+// 14.7 us: what the last tile reads for nothing grows); the waves sum a tile's parts in turn, and one barrier a tile (two
+// buffers) keeps them together.  EPI_GLU: 8 gate rows and the 8 up rows of the same outputs are one tile, so a pair meets
+// across the halves of the result.
+template <int NW, int KB, int EPI, bool XF>
+__global__ __launch_bounds__(NW * 64) void row_linear_walk_kernel(Args a) {
+  constexpr int OUT = EPI == EPI_GLU ? 8 : 16;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, h = lane >> 4;
+  const int tiles = (a.N + OUT - 1) / OUT, step = gridDim.x;
+  __shared__ f32x4 red[2][NW][64];
+
+  const char* xb = reinterpret_cast<const char*>(a.x) + 128 * KB * wid + (min(r16, a.M - 1) * a.ldx + 8 * h) * 2;
+  const char* Wb = reinterpret_cast<const char*>(a.W) + 128 * KB * wid;
+  const unsigned kin = (unsigned)(4 * (r16 & 8) + 8 * h) * 2;
+  u32x4 w[2][KB][2];
+  Pack8 xv[KB][2];
+  // (past the last tile: one line for all, so that a tile's wait never stands behind a branch)
+  auto load_w = [&](int b, int t) {
+    const bool in = t < tiles;
+    const int n0 = in ? t * OUT : 0;
+    const char* base = Wb + (long long)n0 * a.K * 2;
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+      const int row = min((EPI == EPI_GLU ? 0 : 8 * l) + (r16 & 7), a.N - 1 - n0);
+      const unsigned off = in ? (unsigned)(row * a.K) * 2 + kin : 0;
+      const char* src = base + (EPI == EPI_GLU && l ? (long long)a.N * a.K * 2 : 0);
+#pragma unroll
+      for (int u = 0; u < KB; ++u) w[b][u][l] = ld_nt16(reinterpret_cast<const bf16*>(src + 128 * u + off));
+    }
+  };
+  auto tile = [&](int b, int t, int turn) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < KB; ++u) {
+      Pack8 f0, f1;
+      f0.w = half_swap<0xc>(w[b][u][0], w[b][u][1]);
+      f1.w = half_swap<0x3>(w[b][u][1], w[b][u][0]);
+      acc = mfma16(f0.v, xv[u][0].v, acc);
+      acc = mfma16(f1.v, xv[u][1].v, acc);
+    }
+    red[b][wid][lane] = acc;
+    __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0): the next tile's loads stay in flight
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (wid != turn) return;
+    auto sum = [&](int from) {
+      f32x4 v = red[b][0][from];
+#pragma unroll
+      for (int i = 1; i < NW; ++i) v += red[b][i][from];
+      return v;
+    };
+    if constexpr (EPI == EPI_GLU) {
+      f32x4 v = sum(lane), up;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) up[r] = __shfl_down(v[r], 32, 64);
+      store_rows<8, EPI>(a, t * OUT, lane, v, up);
+    } else {
+      store_rows<16, EPI>(a, t * OUT, lane, sum(lane), f32x4{});
+    }
+  };
+  int t = blockIdx.x, turn = 0;
+  load_w(0, t);
+#pragma unroll
+  for (int u = 0; u < KB; ++u)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      xv[u][k].w = *reinterpret_cast<const u32x4*>(xb + 128 * u + 64 * k);
+      if constexpr (XF) relu_squared(xv[u][k]);
+    }
+  while (true) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      if (t >= tiles) return;
+      load_w(b ^ 1, t + step);
+      __builtin_amdgcn_sched_barrier(0);
+      tile(b, t, turn);
+      t += step;
+      turn = turn + 1 == NW ? 0 : turn + 1;
+    }
+  }
 }
 
 // Any K up to SMALL_K (low-rank factors): one wave per 16-row tile, 32 deep a step; lanes past K multiply zeros.
@@ -196,32 +296,53 @@ __global__ __launch_bounds__(64) void row_linear_small_kernel(Args a) {
   store_rows<16, EPI>(a, n0, lane, acc[0], acc[RT - 1]);
 }
 
-template <int RT, int RH, int NW, int U, int EPI, bool XF>
+template <int NW, int KB, int EPI, bool XF>
+bool walk(const Args& a, hipStream_t s) {
+  if (a.K != 64 * NW * KB) return false;
+  constexpr int OUT = EPI == EPI_GLU ? 8 : 16;
+  const int tiles = (a.N + OUT - 1) / OUT;
+  row_linear_walk_kernel<NW, KB, EPI, XF><<<tiles < 256 ? tiles : 256, NW * 64, 0, s>>>(a);
+  return true;
+}
+
+template <int RT, int RH, int NW, int U, int EPI, bool XF, bool M8 = false>
 bool run(const Args& a, hipStream_t s) {
   if (a.K % (64 * NW * U)) return false;
   constexpr int rows = EPI == EPI_GLU ? RH : RH * RT;
-  row_linear_kernel<RT, RH, NW, U, EPI, XF><<<(a.N + rows - 1) / rows, NW * 64, 0, s>>>(a);
+  row_linear_kernel<RT, RH, NW, U, EPI, XF, M8><<<(a.N + rows - 1) / rows, NW * 64, 0, s>>>(a);
   return true;
 }
 
 // Tile by the number of outputs (us at 8 rows, other weights read in between; the library and the launch it replaces in
 // brackets):
-//   up to 3071: 8-row tiles, so that 2048 outputs are 256 workgroups (2048 x 2048 4.8, 16-row tiles 5.5 [8.5]; 2048 x 4096
-//   7.3 / 9.0 [11.5]; 2048 x 8192 with the squared ReLU 11.9 / 15.2 [15.6])
-//   16-row tiles from there (17688 x 2048 21.9, 8-row tiles 23.9 [49.6]; 4096 x 14336 24.8 / 33 [27.2])
-//   two 16-row tiles that share x from 24576 (32768 x 2048 to fp32 32.1, one tile 35.4 [35.3])
-// Gated pairs are two tiles as well (8192 x 2048 17.2 [20.1], 14336 x 4096 49.2 [67.2]).  Four blocks a chunk where they
-// are all of a wave's share, else two (more bytes in flight cost waves); four waves where K does not divide by eight's.
+//   up to 3071: 8-row tiles, so that 2048 outputs are 256 workgroups (2048 x 2048 4.8, 16-row tiles 5.5 [8.5]).  M8, as one
+//   chunk where a wave's share is at most 8 blocks, else two blocks a chunk (x read twice / M8 at 1 and at 8 rows: 2048 x 4096
+//   6.5 / 5.6 and 7.8 / 6.8; 2048 x 8192 9.9 / 9.3 and 12.2 / 12.0, with the squared ReLU 11.5 / 10.6 and 12.8 / 12.3)
+//   the walk from 4097 on, where some workgroup has a second tile (8-row or 16-row tiles one by one / walk: 17440 x 2048 21.7 /
+//   16.5, 6144 x 2048 10.2 / 8.8, 32768 x 2048 to fp32 32.1 / 27.3, 28672 x 4096 50.7 / 38.6 = 6.1 TB/s; 4096 x 2048 7.8 / 7.6
+//   at 16 rows, 6.6 / 6.9 at 2), of the widths that are written out below; 1536 wide always (its other form has four waves of
+//   one block a chunk: 2048 outputs 5.5 / 4.6)
+//   16-row tiles between the two and for other widths (8-row tiles 3072 x 2048 at 16 rows 7.6, 6.6); two that share x from 24576
+// Gated pairs walk (8192 x 2048 18.1 / 13.9, 1024 x 2048 7.9 / 5.9, 14336 x 4096 50.6 / 39.4).  Four blocks a chunk where they are
+// all of a wave's share, else two (more bytes in flight cost waves); four waves where K does not divide by eight's.
 template <int EPI, bool XF>
 bool by_shape(const Args& a, hipStream_t s) {
   if (a.K <= SMALL_K) {
     row_linear_small_kernel<EPI, XF><<<(a.N + 15) / 16, 64, 0, s>>>(a);
     return true;
   }
+  const bool walks = EPI == EPI_GLU ? a.K >= 2048 : a.N > 4096 || a.K == 1536;
+  if (walks && (walk<8, 3, EPI, XF>(a, s) || walk<16, 2, EPI, XF>(a, s) || walk<8, 6, EPI, XF>(a, s) || walk<8, 8, EPI, XF>(a, s)))
+    return true;
   if constexpr (EPI == EPI_GLU) {
     return run<2, 16, 4, 4, EPI, XF>(a, s) || run<2, 16, 4, 1, EPI, XF>(a, s);
   } else {
-    const bool whole = a.K <= 64 * 8 * 4;
+    const int per = a.K / (64 * 8);  // blocks of each of eight waves
+    if (a.N < 3072 && a.M <= 8 &&
+        ((per <= 4 && run<1, 8, 8, 4, EPI, XF, true>(a, s)) || (per <= 8 && run<1, 8, 8, 8, EPI, XF, true>(a, s)) ||
+         run<1, 8, 8, 2, EPI, XF, true>(a, s)))
+      return true;
+    const bool whole = per <= 4;
     if (a.N < 3072 && ((whole && run<1, 8, 8, 4, EPI, XF>(a, s)) || run<1, 8, 8, 2, EPI, XF>(a, s))) return true;
     if (a.N >= 24576 && run<2, 16, 4, 4, EPI, XF>(a, s)) return true;
     return (whole && run<1, 16, 8, 4, EPI, XF>(a, s)) || run<1, 16, 8, 2, EPI, XF>(a, s) || run<1, 16, 4, 1, EPI, XF>(a, s);

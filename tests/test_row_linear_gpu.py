@@ -44,6 +44,15 @@ def test_row_linear(gpu, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,K", [(20, 1536), (4100, 1536), (4100, 2048), (12308, 2048), (4104, 3072), (4108, 4096), (20, 4096)])
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+def test_row_linear_tiles_in_turn(gpu, M, N, K):
+    """Workgroups that walk several tiles: every width they take, one tile, a second one of some, an odd number, a cut last one;
+    gated pairs of one tile; and up to 8 rows against up to 16 of the forms without a walk."""
+    test_row_linear(gpu, M, N, K)
+
+
+@pytest.mark.gpu
 def test_linear_accepts_every_form(gpu):
     """Strides, types, sizes and alignments that the kernel does not take stay with the library and give the same product."""
     g = torch.Generator(device=gpu).manual_seed(3)
