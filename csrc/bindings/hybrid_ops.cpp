@@ -231,7 +231,8 @@ int64_t window_attn(const Tensor& q, const Tensor& k_cache, const Tensor& v_cach
     dtype(*part_o, at::kFloat, "part_o");
     dtype(*part_ml, at::kFloat, "part_ml");
     dtype(*counters, at::kInt, "counters");
-    const int64_t span = (int64_t)a.max_blocks * a.BS, parts = (span + part_keys - 1) / part_keys;
+    // (a row's ranges start up to 31 keys in front of its window)
+    const int64_t span = std::min<int64_t>((int64_t)a.max_blocks * a.BS, window + 31), parts = (span + part_keys - 1) / part_keys;
     TORCH_CHECK(part_keys < (1LL << 30) && part_o->numel() >= (int64_t)a.T * a.H * parts * a.dv &&
                     part_ml->numel() >= (int64_t)a.T * a.H * parts * 2 && counters->numel() >= (int64_t)a.T * a.G,
                 "window_attn: part_o [T, H, parts, dv], part_ml [T, H, parts, 2], counters [T, G]");

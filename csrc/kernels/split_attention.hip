@@ -1,6 +1,10 @@
 // Causal softmax attention for single rows (decode steps, bf16): one workgroup per (row, key / value head, range of keys), the
-// query heads of the group together, so a cached row is read once.  Same arguments as window_attention.hip's kernels for a
-// window that never ends; optional sink, soft cap, per-key score factor and output gate (per head or per column).
+// query heads of the group together, so a cached row is read once.  Same arguments as window_attention.hip's kernels; optional
+// sink, soft cap, per-key score factor and output gate (per head or per column).
+//
+// WIN: a window that ends.  The ranges start at the 32-key step of the row's first key; keys in front of that key re-read its
+// row and weigh 0.  The weights enter the product as three bf16 parts, which hold all of an fp32 number, as the kernel with one
+// wave a head keeps them.  8 rows, 16 heads on 4 groups of 128, 1024 keys: 10.7 us, that kernel 19.0; 200 rows 87 (4.8 TB/s) / 156.
 //
 // Four waves, 32 keys per wave and step.  A step's key and value rows go to the wave's own LDS by direct loads (KEYV: the
 // values are the keys, one set of rows serves both products); the workgroups that share a CU cover each other's loads (a second
@@ -14,7 +18,7 @@
 
 namespace {
 
-constexpr int NW = 4, STEP = 32, MAX_REP = 16, MAX_PARTS = 64;
+constexpr int NW = 4, STEP = 32, MAX_REP = 16, MAX_PARTS = 64, NO_WINDOW = 1 << 30;
 
 SYM_DEV void wait_loads() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }   // rows landed, LDS reads done
 
@@ -28,16 +32,17 @@ SYM_DEV float2 collect(const float* p) {
   return make_float2(__uint_as_float((unsigned int)v), __uint_as_float((unsigned int)(v >> 32)));
 }
 
-template <int D, bool KEYV, bool ONE>
+template <int D, bool KEYV, bool ONE, bool WIN>
 __global__ __launch_bounds__(64 * NW) void split_attn_kernel(WindowAttnArgs a) {
   constexpr int CH = row_chunks(D), KD = (D + 31) / 32, VT = D / 16, ROWS = STEP * CH * 16;   // bytes of a step's rows
   constexpr int NL = STEP * CH / 64;                   // direct loads of a step's keys (and as many of its values)
   constexpr int STAGE = (KEYV ? 1 : 2) * ROWS + 256, LDO = D + 4;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int part = blockIdx.x, g = blockIdx.y, row = blockIdx.z;
-  const int ctx = a.positions[row] + 1, lo = part * a.part_keys;
+  const int ctx = a.positions[row] + 1, first = WIN ? max(0, ctx - a.window) : 0, base = first & ~(STEP - 1);
+  const int lo = base + part * a.part_keys;
   if (lo >= ctx) return;
-  const int hi_key = min(ctx, lo + a.part_keys), nparts = (ctx + a.part_keys - 1) / a.part_keys;
+  const int hi_key = min(ctx, lo + a.part_keys), nparts = (ctx - base + a.part_keys - 1) / a.part_keys;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int j = lane & 15, hq = lane >> 4, rep = a.H / a.G;
   const int* bt = a.block_tables + (long long)a.row_seq[row] * a.max_blocks;
@@ -50,7 +55,7 @@ __global__ __launch_bounds__(64 * NW) void split_attn_kernel(WindowAttnArgs a) {
   auto stage = [&](int k0) {
     const int blk = ONE ? bt[k0 >> a.bs_shift] : 0;
     auto row_of = [&](int kp) {
-      kp = min(kp, ctx - 1);
+      kp = min(WIN ? max(kp, first) : kp, ctx - 1);
       return ONE ? ((long long)blk << a.bs_shift) + (kp & (a.BS - 1)) : cache_row(bt, kp, a.BS, a.bs_shift);
     };
     if (scaled) direct_load4(a.key_scale + row_of(k0 + (lane & 31)), lds0 + STAGE - 256);
@@ -114,18 +119,19 @@ __global__ __launch_bounds__(64 * NW) void split_attn_kernel(WindowAttnArgs a) {
         float v = p[s][i];
         if (a.softcap > 0.f) v = cap2 - 2.f * cap2 * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(c1 * v));
         else v *= sl2;
-        p[s][i] = k0 + 16 * s + 4 * hq + i < hi_key ? v : -INFINITY;
+        const int key = k0 + 16 * s + 4 * hq + i;
+        p[s][i] = key < hi_key && (!WIN || key >= first) ? v : -INFINITY;
         mx = fmaxf(mx, p[s][i]);
       }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mt = fmaxf(m, mx);                     // (the step's first key is in range: finite)
+    const float mt = fmaxf(m, mx);                     // (a key of the step is in range: finite)
     const float corr = __builtin_amdgcn_exp2f(m - mt);
     l *= corr;
 #pragma unroll
     for (int t = 0; t < VT; ++t) o[t] *= corr;
     m = mt;
-    Pack8 pf;
+    Pack8 pf, pm, pl;
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -133,6 +139,11 @@ __global__ __launch_bounds__(64 * NW) void split_attn_kernel(WindowAttnArgs a) {
         const float w = __builtin_amdgcn_exp2f(p[s][i] - mt);
         l += w;
         pf.h[4 * s + i] = (bf16)w;
+        if constexpr (WIN) {
+          const float rest = w - (float)pf.h[4 * s + i];
+          pm.h[4 * s + i] = (bf16)rest;
+          pl.h[4 * s + i] = (bf16)(rest - (float)pm.h[4 * s + i]);
+        }
       }
 #pragma unroll
     for (int t = 0; t < VT; ++t) {
@@ -144,6 +155,10 @@ __global__ __launch_bounds__(64 * NW) void split_attn_kernel(WindowAttnArgs a) {
       }
       Pack8 vf;
       vf.u = make_uint4(x[0].x, x[0].y, x[1].x, x[1].y);
+      if constexpr (WIN) {
+        o[t] = mfma16(vf.v, pl.v, o[t]);
+        o[t] = mfma16(vf.v, pm.v, o[t]);
+      }
       o[t] = mfma16(vf.v, pf.v, o[t]);                 // head j, columns 16 t + 4 hq + 0..3
     }
     if (k0 + STEP * NW < hi_key) {
@@ -243,7 +258,7 @@ __global__ __launch_bounds__(64 * NW) void split_attn_kernel(WindowAttnArgs a) {
   if (threadIdx.x == 0) __hip_atomic_store(a.counters + group, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int D, bool KEYV, bool ONE>
+template <int D, bool KEYV, bool ONE, bool WIN>
 void launch(const WindowAttnArgs& a, hipStream_t s) {
   constexpr int stage = (KEYV ? 1 : 2) * STEP * row_chunks(D) * 16 + 256;
   const int rep = a.H / a.G;
@@ -252,17 +267,25 @@ void launch(const WindowAttnArgs& a, hipStream_t s) {
   lds = max(lds, (int)(a.max_parts * rep * 2 * sizeof(float)));
   static bool once = false;
   if (!once) {
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&split_attn_kernel<D, KEYV, ONE>),
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&split_attn_kernel<D, KEYV, ONE, WIN>),
                         hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
     once = true;
   }
-  split_attn_kernel<D, KEYV, ONE><<<dim3(a.max_parts, a.G, a.T), 64 * NW, lds, s>>>(a);
+  split_attn_kernel<D, KEYV, ONE, WIN><<<dim3(a.max_parts, a.G, a.T), 64 * NW, lds, s>>>(a);
 }
 
 template <int D, bool KEYV>
 void launch_kv(const WindowAttnArgs& a, hipStream_t s) {
-  if (a.bs_shift >= 5) launch<D, KEYV, true>(a, s);      // cache blocks of 32 tokens or a larger power of two
-  else launch<D, KEYV, false>(a, s);
+  const bool one = a.bs_shift >= 5;      // cache blocks of 32 tokens or a larger power of two
+  if constexpr (!KEYV) {
+    if (a.window < NO_WINDOW) {
+      if (one) launch<D, KEYV, true, true>(a, s);
+      else launch<D, KEYV, false, true>(a, s);
+      return;
+    }
+  }
+  if (one) launch<D, KEYV, true, false>(a, s);
+  else launch<D, KEYV, false, false>(a, s);
 }
 
 template <int D>
@@ -276,7 +299,7 @@ void launch_d(const WindowAttnArgs& a, hipStream_t s) {
 bool launch_split_attn(const WindowAttnArgs& a, hipStream_t s) {
   const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   if (!a.part_o || !a.part_ml || !a.counters || a.part_keys < STEP || a.part_keys % STEP || a.max_parts < 1 ||
-      a.max_parts > MAX_PARTS || a.dk != a.dv || a.bias || a.window < (1 << 30) || a.H / a.G > MAX_REP || a.T > 65535 ||
+      a.max_parts > MAX_PARTS || a.dk != a.dv || a.bias || (a.window < NO_WINDOW && (a.keep_first > 0 || a.k_cache == a.v_cache)) || a.H / a.G > MAX_REP || a.T > 65535 ||
       a.G > 65535 || !al(a.q) || !al(a.k_cache) || !al(a.v_cache) || !al(a.out) || !al(a.part_o))
     return false;
   switch (a.dk) {

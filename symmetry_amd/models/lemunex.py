@@ -271,8 +271,14 @@ class LemunexLM:
         ops.qkv_rope_cache(z[:, c0:c0 + n], P["left.b"], a.heads, a.kv_heads, a.dim, a.vdim, b.positions, b.slot_mapping,
                            P["rope"], q, cache.k[i], cache.v[i])
         att = self._buf("att.o", (T, a.heads, a.vdim))
+        split = None
+        if not prefill and self.device.type != "cpu" and self.dtype == torch.bfloat16 and ops.window_ranges(T, a.heads, a.kv_heads):
+            keys, parts = ops.window_attn_split(T, a.kv_heads, min(b.block_tables.shape[1] * cache.block_size, a.window + 31))
+            split = (self._buf("att.part_o", (T, a.heads, parts, a.vdim), torch.float32),
+                     self._buf("att.part_ml", (T, a.heads, parts, 2), torch.float32),
+                     self.ws.get("att.counters", (T * a.kv_heads,), torch.int32, self.device, zeros=True), keys)
         ops.window_attn(q, cache.k[i], cache.v[i], b.block_tables, b.row_seq, b.positions, a.window, a.scale,
-                        self._cols(z, P, "left.g"), att, b.tiles if prefill else None, b.cu_q if prefill else None)
+                        self._cols(z, P, "left.g"), att, b.tiles if prefill else None, b.cu_q if prefill else None, split=split)
         left = self._linear("att.out", att.view(T, a.heads * a.vdim), P["left.o"])
         # gated linear attention
         dz = self._linear("gla.dz", self._cols(z, P, "right.a1"), P["right.a2"])

@@ -861,6 +861,14 @@ def window_attn_split(rows: int, groups: int, span: int, target_wgs: int = 512, 
     return keys, -(-span // keys)
 
 
+def window_ranges(rows: int, heads: int, groups: int) -> bool:
+    """Do single rows behind a window that ends walk key ranges side by side rather than a wave or more a head?  Where a group of
+    heads reads its keys once, always (16 heads on 4 groups of 128, 1024 keys, us: 8 rows 19.0 -> 10.7, 64 rows 73 -> 38, 200 rows
+    156 -> 87; 8 heads on 4: 64 rows 49.8 -> 39.2); head for head only while the rows alone leave the chip idle (8 heads: 8 rows
+    17.0 -> 13.5, 16 rows 22.7 -> 22.6, 32 rows 30.3 -> 37.8)."""
+    return heads >= 2 * groups or rows * groups <= 64
+
+
 DECAY_CHANNEL_GATE, DECAY_STEP_SIZE, DECAY_LOG_GATES = 0, 1, 2
 
 

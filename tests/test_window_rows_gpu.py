@@ -39,7 +39,15 @@ def test_keys_off_16_bytes(gpu, H, G, D, T, window):
     _check(H, G, D, T, window, 0, 4)
 
 
-def _check(H, G, D, T, window, keep, off):
+@pytest.mark.parametrize("H,G,D,T,window", [(16, 4, 128, 23, 1024), (16, 4, 64, 40, 600), (16, 2, 32, 23, 1), (6, 2, 96, 23, 33),
+                                            (16, 1, 128, 30, 128), (5, 5, 112, 23, 97), (16, 4, 128, 300, 513)])
+def test_window_ranges(gpu, H, G, D, T, window):
+    """The key ranges of a window that ends, over every place of its first key in a step, and rows that end in their first range;
+    whatever a row may not see is not finite.  The weights' three parts hold their 24 bits: the bounds are the wave kernel's."""
+    _check(H, G, D, T, window, 0, 0, ranges=True)
+
+
+def _check(H, G, D, T, window, keep, off, ranges=False):
     """Scores, weights and sums are fp32.  A score of D products of |q k| scale ~ 7 in all is within D 2^-24 7 < 2^-14 of the
     exact one and so a weight, the exponential's own 2^-22 aside; numerator and denominator both have them: 2^-13 of the sum of
     p |v|, and the result is rounded to bf16, at most 2^-8 of it (seven fraction bits).  Rows that p may not see, and the cache's first row, hold large values."""
@@ -62,8 +70,8 @@ def _check(H, G, D, T, window, keep, off):
     bt = bt.cuda()
     shape = (at + 1, BS, G, D)
     k = torch.empty(math.prod(shape) + off, device="cuda", dtype=torch.bfloat16)[off:].view(shape)
-    k.fill_(60.0)
-    v = torch.full(shape, -900.0, device="cuda", dtype=torch.bfloat16)
+    k.fill_(math.nan if ranges else 60.0)
+    v = torch.full(shape, math.nan if ranges else -900.0, device="cuda", dtype=torch.bfloat16)
     rows = []
     for i, p in enumerate(pos):
         j0 = max(0, p - window + 1)
@@ -74,9 +82,15 @@ def _check(H, G, D, T, window, keep, off):
     q = rnd(T, H, D)
     out = torch.full((T + 1, H, D), 7.0, device="cuda", dtype=torch.bfloat16)
     i32 = dict(device="cuda", dtype=torch.int32)
-    used = ops.window_attn(q, k, v, bt, torch.arange(T, **i32), torch.tensor(pos, **i32), window, D ** -0.5, None, out[:-1], impl=0,
-                           keep_first=keep)
-    assert used == 0 and bool((out[-1] == 7.0).all())
+    split = None
+    if ranges:
+        keys, parts = ops.window_attn_split(T, G, min(window + 31, mb * BS))
+        split = (torch.empty(T, H, parts, D, device="cuda"), torch.empty(T, H, parts, 2, device="cuda"),
+                 torch.zeros(T * G, **i32), keys)
+    used = ops.window_attn(q, k, v, bt, torch.arange(T, **i32), torch.tensor(pos, **i32), window, D ** -0.5, None, out[:-1],
+                           impl=1 if ranges else 0, keep_first=keep, split=split)
+    assert used == (3 if ranges else 0) and bool((out[-1] == 7.0).all())
+    assert split is None or not bool(split[2].any())
     for i, (b, o) in enumerate(rows):
         ks, vs = k[b, o].double(), v[b, o].double()
         p = torch.einsum("grd,cgd->grc", q[i].double().view(G, H // G, D), ks).mul_(D ** -0.5).softmax(-1)
