@@ -282,6 +282,32 @@ def test_logits_argmax(gpu):
     assert int(((kk >> 32) - (keys_ref >> 32)).abs().max()) <= 4  # value bits: __logf vs torch.log ulps
 
 
+@pytest.mark.parametrize("V", [1, 3, 4, 129, 4092, 4096, 32764, 32768, 32770, 32772, 70004])
+@pytest.mark.parametrize("first", [0, 1])
+def test_logits_argmax_finds_the_first_largest(gpu, V, first):
+    """Greedy rows where a thread's share ends, 16 bytes a lane and entry by entry, against the keys' order over the bits: ties,
+    rows of one value, infinities, and a NaN of either sign (it orders by its bits).  Whole numbers: exact."""
+    g = torch.Generator(device=gpu).manual_seed(V)
+    flat = torch.randn(first + 9 * V, device=gpu, generator=g).mul_(4).round_()
+    x = flat[first:].view(9, V)
+    x[1] = -2.0
+    x[2, -1] = 99.0
+    x[3, V // 2:] = 98.0
+    x[4, V // 3] = float("nan")
+    x[5] = float("-inf")
+    x[6].view(torch.int32).fill_(-1)                       # the smallest key there is
+    x[7].view(torch.int32).fill_(-1)
+    x[7, V // 2] = float("-inf")
+    x[8, 0] = float("inf")
+    keys, ids = torch.empty(9, device=gpu, dtype=torch.int64), torch.empty(9, device=gpu, dtype=torch.int32)
+    ops.logits_argmax(x, torch.zeros(9, device=gpu), torch.zeros(9, device=gpu, dtype=torch.int64),
+                      torch.zeros(1, device=gpu, dtype=torch.int64), keys, ids, 7)
+    u = x.cpu().view(torch.int32).long() & 0xFFFFFFFF
+    k = torch.where(u >= 1 << 31, 0xFFFFFFFF - u, u + (1 << 31))
+    want = (k == k.max(1, keepdim=True).values).int().argmax(1) + 7
+    assert torch.equal(ids.cpu().long(), want) and torch.equal(keys.cpu() & 0xFFFFFFFF, 0xFFFFFFFF - want)
+
+
 def test_swiglu(gpu):
     T, F = 7, 14336
     g = torch.Generator(device=gpu).manual_seed(8)
