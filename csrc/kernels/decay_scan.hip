@@ -41,10 +41,9 @@ __global__ __launch_bounds__(NT) void decay_scan_kernel(DecayScanArgs a) {
   constexpr int NPAD = NPL * SLICES;
   constexpr int LROW = SLICES * (NPL + 4);                  // a token's LDS row: the four slices 16 bytes apart in bank
                                                             // space, so the lanes' four addresses of a read do not collide
-  constexpr int EPT = CH * NPAD / NT;                       // staged (token, channel) entries per thread
+  constexpr int EPT = (CH * NPAD + NT - 1) / NT;            // staged (token, channel) entries per thread
   constexpr int ASZ = MODE == 0 ? CH * LROW : (MODE == 1 ? 2 : 3) * CH;   // decays per channel, or (decay, step(, max)) per token
   constexpr int BUF = 2 * CH * LROW + ASZ;
-  static_assert(CH * NPAD % NT == 0, "staging split");
   const int N = a.N, P = a.P;
   const int h = blockIdx.y, run = blockIdx.z;
   const int s0 = a.cu_q ? a.cu_q[run] : run, s1 = a.cu_q ? a.cu_q[run + 1] : run + 1;
@@ -114,6 +113,7 @@ __global__ __launch_bounds__(NT) void decay_scan_kernel(DecayScanArgs a) {
     for (int u = 0; u < EPT; ++u) {
       const int i = threadIdx.x + NT * u;
       const int tt = i / NPAD, n = i - tt * NPAD;
+      if (tt >= CH) break;
       const int o = tt * LROW + (n / NPL) * (NPL + 4) + n % NPL;
       qS[o] = rq[u] * a.q_scale;
       kS[o] = rk[u];
@@ -232,6 +232,17 @@ void launch_one(const DecayScanArgs& a, hipStream_t s) {
 
 template <typename T, int MODE>
 void launch_mode(const DecayScanArgs& a, hipStream_t s) {
+  if (a.T == a.runs) {
+    // one token a run (decode steps): the state's traffic is the launch, and nothing is staged for tokens that are not there
+    // (8 runs, us: 8 heads x 128 x 256 with channel gates 10.3 -> 8.2, 64 x 128 x 64 11.2 -> 10.1)
+    const int need = (a.N + 3) / 4;
+    if (need <= 4) launch_one<T, MODE, 4, 1, 4>(a, s);
+    else if (need <= 8) launch_one<T, MODE, 8, 1, 4>(a, s);
+    else if (need <= 16) launch_one<T, MODE, 16, 1, 4>(a, s);
+    else if (need <= 32) launch_one<T, MODE, 32, 1, 4>(a, s);
+    else launch_one<T, MODE, 64, 1, 4>(a, s);
+    return;
+  }
   // waves with 16 columns each; under two per SIMD (1024 SIMDs) and enough key channels: 8 columns x 8 slices
   const long long waves16 = (long long)a.runs * a.H * ((a.P + 15) / 16);
   if (waves16 < 2048 && a.N >= 64 && a.T > a.runs) {
