@@ -395,9 +395,11 @@ ConvArgs conv_args(const Tensor& xin, const OptTensor& w, const OptTensor& b, Te
 }
 
 void causal_conv_silu(const Tensor& xin, const Tensor& w, const Tensor& b, Tensor& state, const OptTensor& cu_q,
-                      const OptTensor& row_seq, const Tensor& prev_row, int64_t runs, Tensor& out) {
+                      const OptTensor& row_seq, const Tensor& prev_row, int64_t runs, Tensor& out, const OptTensor& save_slot) {
   const int f32 = act(out, "out");
-  ConvArgs a = conv_args(xin, w, b, state, cu_q, row_seq, prev_row, std::nullopt, runs, f32);
+  ConvArgs a = conv_args(xin, w, b, state, cu_q, row_seq, prev_row, save_slot, runs, f32);
+  TORCH_CHECK(!(cu_q.has_value() && save_slot.has_value()) && (!save_slot.has_value() || runs == a.T),
+              "causal_conv_silu: the state moves on in this launch only where every row is a run of its own");
   TORCH_CHECK(!cu_q.has_value() || row_seq.has_value(), "causal_conv_silu: cu_q without row_seq");
   TORCH_CHECK(out.numel() == (int64_t)a.T * a.C, "causal_conv_silu: out shape");
   a.out = out.data_ptr();
@@ -1165,7 +1167,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
         &gated_group_norm);
   m.def(
       "causal_conv_silu(Tensor xin, Tensor w, Tensor b, Tensor(a!) state, Tensor? cu_q, Tensor? row_seq, Tensor prev_row, "
-      "int runs, Tensor(b!) out) -> ()",
+      "int runs, Tensor(b!) out, Tensor? save_slot=None) -> ()",
       &causal_conv_silu);
   m.def("conv_state_update(Tensor xin, Tensor(a!) state, Tensor? cu_q, Tensor prev_row, Tensor save_slot, int runs) -> ()",
         &conv_state_update);

@@ -64,6 +64,7 @@ struct ConvArgs {
   void* out;           // [T][C]
   int T, C, taps, runs;
 };
+// (save_slot: only with cu_q null; the state moves on in the same launch)
 void launch_causal_conv_silu(const ConvArgs& a, int f32, hipStream_t s);
 void launch_conv_state_update(const ConvArgs& a, int f32, hipStream_t s);
 // out = x . W^T (relu2: of relu(x)^2; glu: silu(gate) * up of W's [gate | up] rows); false: this K has no kernel

@@ -237,8 +237,11 @@ __global__ __launch_bounds__(BT) void gated_group_norm_vec_kernel(const float* _
   store8(out + (long long)blockIdx.x * C + c0, v);
 }
 
-// grid (T, ceil(C / NT)): one thread per (row, channel)
-template <typename T>
+constexpr int MAX_TAPS = 16;
+
+// grid (T, ceil(C / NT)): one thread per (row, channel).  SAVE: every row is a run of its own, whose newest inputs the same
+// thread moves on (one launch less of a decode step; each of the two takes 4.6 us at 8 rows of 4352)
+template <typename T, bool SAVE>
 __global__ __launch_bounds__(NT) void causal_conv_silu_kernel(ConvArgs a) {
   const int row = blockIdx.x, c = blockIdx.y * NT + threadIdx.x;
   if (c >= a.C) return;
@@ -249,6 +252,25 @@ __global__ __launch_bounds__(NT) void causal_conv_silu_kernel(ConvArgs a) {
   const T* x = reinterpret_cast<const T*>(a.xin);
   const T* w = reinterpret_cast<const T*>(a.w) + (long long)c * taps;
   float acc = a.b[c];
+  if constexpr (SAVE) {
+    const int sv = a.save_slot[row];
+    T old[MAX_TAPS];                     // old[m]: m + 1 positions back
+#pragma unroll
+    for (int m = 0; m < MAX_TAPS - 1; ++m)
+      if (m < taps - 1) old[m] = st ? st[(long long)(taps - 2 - m) * a.C + c] : (T)0.f;
+    const T now = x[(long long)row * a.ldx + c];
+    acc += (float)w[taps - 1] * (float)now;
+#pragma unroll
+    for (int m = 0; m < MAX_TAPS - 1; ++m)
+      if (m < taps - 1) acc += (float)w[taps - 2 - m] * (float)old[m];
+    reinterpret_cast<T*>(a.out)[(long long)row * a.C + c] = (T)(acc * sigmoidf(acc));
+    if (sv < 0) return;
+    T* dst = reinterpret_cast<T*>(a.state) + (long long)sv * a.state_stride + c;
+#pragma unroll
+    for (int m = 0; m < MAX_TAPS - 1; ++m)
+      if (m < taps - 1) dst[(long long)(taps - 2 - m) * a.C] = m == 0 ? now : old[m - 1];
+    return;
+  }
   for (int i = 0; i < taps; ++i) {       // i positions back
     float v = 0.f;
     if (i <= j) v = (float)x[(long long)(row - i) * a.ldx + c];
@@ -304,8 +326,6 @@ __global__ __launch_bounds__(64) void causal_conv_rows_kernel(ConvArgs a) {
     *reinterpret_cast<uint4*>(reinterpret_cast<bf16*>(a.out) + (long long)row * a.C + c) = o.u;
   }
 }
-
-constexpr int MAX_TAPS = 16;
 
 // grid (runs, ceil(C / NT)): one thread per (run, channel) owns that channel of the run's state slot
 template <typename T>
@@ -910,7 +930,11 @@ void launch_causal_conv_silu(const ConvArgs& a, int f32, hipStream_t s) {
     return;
   }
   dim3 grid(a.T, (a.C + NT - 1) / NT);
-  DISPATCH_T(f32, causal_conv_silu_kernel<T><<<grid, NT, 0, s>>>(a);)
+  if (a.save_slot) {
+    DISPATCH_T(f32, (causal_conv_silu_kernel<T, true><<<grid, NT, 0, s>>>(a));)
+  } else {
+    DISPATCH_T(f32, (causal_conv_silu_kernel<T, false><<<grid, NT, 0, s>>>(a));)
+  }
 }
 
 void launch_conv_state_update(const ConvArgs& a, int f32, hipStream_t s) {

@@ -23,7 +23,7 @@ v / sqrt(mean(v^2) + eps) * (1 + g))::
 Every projection that reads h is one row block of ONE fused weight per layer (a single library GEMM); the kernels take
 column ranges of its output as views.  Step launches per layer: GEMM (all of h's projections), then
 parallel: qkv_rope_cache, window_attn, GEMM W_o | GEMM W_a2, decay_scan, gated_group_norm, GEMM W_o
-mamba2:   causal_conv_silu, conv_state_update, decay_scan, gated_group_norm, GEMM W_o
+mamba2:   causal_conv_silu (+ conv_state_update in prompt steps), decay_scan, gated_group_norm, GEMM W_o
 ff:       relu_sq, GEMM down | softmax_topk, expert_offsets, scatter, grouped gate|up, silu_mul, grouped down,
           silu_mul + GEMM (shared), moe_mix
 and one residual_mix_norm that adds the scaled sublayer outputs to the stream and emits the next layer's h.
@@ -300,8 +300,10 @@ class LemunexLM:
         cu = b.cu_q if b.kind != "decode" else None
         xin = self._cols(z, P, "xbc")
         xc = self._buf("ssm.xc", (T, m.conv_channels))
-        ops.causal_conv_silu(xin, P["conv"], P["conv.b"], cache.conv[i], cu, b.row_seq, b.prev_row, runs, xc)
-        ops.conv_state_update(xin, cache.conv[i], cu, b.prev_row, b.save_slot, runs)
+        ops.causal_conv_silu(xin, P["conv"], P["conv.b"], cache.conv[i], cu, b.row_seq, b.prev_row, runs, xc,
+                             b.save_slot if cu is None else None)
+        if cu is not None:
+            ops.conv_state_update(xin, cache.conv[i], cu, b.prev_row, b.save_slot, runs)
         inner, gn = m.inner, m.groups * m.state
         y = self._buf("rec.y", (T, inner), torch.float32)
         ops.decay_scan(ops.DECAY_STEP_SIZE, xc[:, inner + gn:], xc[:, inner:inner + gn], xc[:, :inner],

@@ -919,13 +919,17 @@ def gated_group_norm(y, gate, w, eps, group, gate_first, out, sigmoid=False):
     return reference.gated_group_norm(y, gate, w, eps, group, gate_first, out, sigmoid)
 
 
-def causal_conv_silu(xin, w, b, state, cu_q, row_seq, prev_row, runs, out):
+def causal_conv_silu(xin, w, b, state, cu_q, row_seq, prev_row, runs, out, save_slot=None):
     """out_t = silu(b + sum_j w[:, taps - 1 - j] x_(t - j)) per channel over every run; inputs before the run come from
-    state[slot] [taps - 1, C] (prev_row[first] <= -2) or are zero.  xin [T, C] (view)."""
+    state[slot] [taps - 1, C] (prev_row[first] <= -2) or are zero.  xin [T, C] (view).  ``save_slot`` (every row a run of its
+    own, cu_q None): conv_state_update in the same launch."""
     if _gpu(out):
         return _hyb().causal_conv_silu(xin, w, b, state, cu_q, row_seq if cu_q is not None else None, prev_row, int(runs),
-                                       out)
-    return reference.causal_conv_silu(xin, w, b, state, cu_q, prev_row, runs, out)
+                                       out, save_slot)
+    reference.causal_conv_silu(xin, w, b, state, cu_q, prev_row, runs, out)
+    if save_slot is not None:
+        assert cu_q is None
+        reference.conv_state_update(xin, state, cu_q, prev_row, save_slot, runs)
 
 
 def conv_state_update(xin, state, cu_q, prev_row, save_slot, runs):

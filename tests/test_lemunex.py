@@ -456,6 +456,27 @@ def test_decay_scan_both_modes_and_cuts(device):
 
 
 @pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("taps", [1, 2, 4, 16])
+def test_conv_rows_move_their_state_on(device, dtype, taps):
+    """One launch for rows that are runs of their own against the two it stands for: the same results, in place and into another
+    slot, for a sequence's first row and for one that is not kept."""
+    say("op conv rows", device, dtype, taps)
+    torch.manual_seed(taps)
+    T, Cn = 5, 300
+    x, w = torch.randn(T, Cn + 4).to(dtype), torch.randn(Cn, taps).to(dtype)
+    state = torch.randn(8, taps - 1, Cn).to(dtype)
+    prev = torch.tensor([-2, -1, -5, -6, -7], dtype=torch.int32)       # slots 0, none, 3, 4, 5
+    save = torch.tensor([0, 1, 7, -1, 6], dtype=torch.int32)
+    a = _dev(device, x, w, torch.randn(Cn), state, prev, save, torch.empty(T, Cn, dtype=dtype), torch.empty(T, Cn, dtype=dtype))
+    one, two = a[3].clone(), a[3].clone()
+    ops.causal_conv_silu(a[0][:, 4:], a[1], a[2], one, None, None, a[4], T, a[6], a[5])
+    ops.causal_conv_silu(a[0][:, 4:], a[1], a[2], two, None, None, a[4], T, a[7])
+    ops.conv_state_update(a[0][:, 4:], two, None, a[4], a[5], T)
+    assert torch.equal(a[6], a[7]) and torch.equal(one, two)
+
+
+@pytest.mark.parametrize("device", DEVICES)
 def test_conv_norm_router_ops(device):
     """causal_conv_silu + conv_state_update over cut runs, gated_group_norm in both orders, softmax_topk with a
     correction that changes the choice but not the weights, moe_mix with identity experts."""
