@@ -21,6 +21,9 @@
 //     1 KB in fragment order, so its DMA and its ds_read_b128 are both lane-linear; the 16-B chunk index
 //     of each 128-B x row is XOR-swizzled with (row >> 1) & 7 on the DMA source and on the read, which
 //     makes the x fragment reads bank-conflict free;
+//   * a step's fragments are read from LDS while the step before is multiplied: with one wave a SIMD nothing else covers the
+//     reads (137 rows, us: 4096 x 14336 38.9 -> 30.6, 6144 x 4096 23.6 -> 18.5, 4096 x 4096 19.8 -> 14.4; a ring of its own for
+//     the weights, two chunks deeper, was slower).  x tiles come in steps of 32 rows (up to 64: 2 and 4; 96, 128, 160, 192, 256);
 //   * the 16x16 accumulator of (weight tile, token tile) holds 4 consecutive features of one token per
 //     lane: one float4 store per accumulator into the slab.
 #include "common.h"
@@ -58,7 +61,7 @@ struct MgCfg {
   static constexpr int NX = 16 * MT / 32;                    // x DMA instructions per wave per chunk (MT >= 2)
   static constexpr int NDMA = NX + 2 * RW;                   // DMA instructions per wave per chunk
   static constexpr int VM_KEEP = (D - 1) * NDMA;             // younger DMAs left in flight at the wait
-  static_assert(D >= 1 && VM_KEEP <= 63, "mgemm config");
+  static_assert(MT % 2 == 0 && D >= 1 && VM_KEEP <= 63, "mgemm config");
 };
 
 // MT: 16-token tiles (M <= 16 MT); RW: 16-row weight tiles per wave.  Weights MFMA-preshuffled
@@ -129,19 +132,28 @@ __global__ __launch_bounds__(MG_THR, 1) void mgemm_kernel(const bf16* __restrict
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  auto compute = [&](int slot) {
+  struct Frag {
+    bf16x8 w[RW], x[MT];
+  };
+  Frag f0, f1;      // a chunk's two 32-deep steps
+  // reads step s of a chunk's slot into `next`, between the products of `now`: with one wave a SIMD nothing else hides a read
+  auto step = [&](Frag& next, int slot, int s, const Frag& now, bool reads, bool multiplies) __attribute__((always_inline)) {
     const char* const sb = smem + slot * C::SLOT;
+    constexpr int READS = RW + MT, PER = (READS + MT - 1) / MT;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      bf16x8 wf[RW], xf[MT];
+    for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
-      for (int rt = 0; rt < RW; ++rt) wf[rt] = *(const bf16x8*)(sb + wo_l + (2 * rt + s) * 1024);
+      for (int u = 0; u < PER; ++u) {
+        const int i = PER * mt + u;
+        if (!reads || i >= READS) continue;
+        if (i < RW) next.w[i] = *(const bf16x8*)(sb + wo_l + (2 * i + s) * 1024);
+        else next.x[i - RW] = *(const bf16x8*)(sb + (s ? xo1 : xo0) + (i - RW) * 2048);
+      }
+      if (multiplies) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) xf[mt] = *(const bf16x8*)(sb + (s ? xo1 : xo0) + mt * 2048);
-#pragma unroll
-      for (int rt = 0; rt < RW; ++rt)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = mfma16(wf[rt], xf[mt], acc[rt][mt]);
+        for (int rt = 0; rt < RW; ++rt) acc[rt][mt] = mfma16(now.w[rt], now.x[mt], acc[rt][mt]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   };
 
@@ -175,9 +187,9 @@ __global__ __launch_bounds__(MG_THR, 1) void mgemm_kernel(const bf16* __restrict
     }
   }
 
-  // prologue: chunks 0 .. D-1 in flight
+  // prologue: every slot of the ring in flight
 #pragma unroll
-  for (int c = 0; c < C::D; ++c)
+  for (int c = 0; c < C::SLOTS; ++c)
     if (c < nch) issue(c, c);
 
   if constexpr (EPI >= 0) {
@@ -187,18 +199,32 @@ __global__ __launch_bounds__(MG_THR, 1) void mgemm_kernel(const bf16* __restrict
     }
   }
 
-  // chunk c lives in ring slot c % SLOTS.  Before computing it: wait until this wave's DMAs of chunk c
-  // have landed (the D - 1 younger chunks stay in flight), barrier (every wave's x rows of the chunk are
-  // visible), then refill the slot of chunk c - 1 (all its reads happened before this barrier) with c + D.
-  int slot = 0;
-  for (int c = 0; c < nch; ++c) {
+  // chunk c lives in ring slot c % SLOTS.  Its second step is read while the first is multiplied, then this wave waits until
+  // its DMAs of chunk c + 1 have landed (the younger ones stay in flight) and its reads of chunk c are in registers; behind the
+  // barrier every wave's x rows of chunk c + 1 are visible and slot c is free: it is refilled with c + SLOTS.
+  auto landed = [&](int c) {      // chunk c is; those up to c + D - 1 stay in flight
     if (c + C::D - 1 < nch) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::VM_KEEP) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+  if (C::SLOTS <= nch) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::VM_KEEP + C::NDMA < 63 ? C::VM_KEEP + C::NDMA : 63) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  step(f0, 0, 0, f1, true, false);
+  int slot = 0;
+  for (int c = 0; c + 1 < nch; ++c) {
+    const int after = slot == C::SLOTS - 1 ? 0 : slot + 1;
+    step(f1, slot, 1, f0, true, true);
+    landed(c + 1);
+    __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
-    if (c + C::D < nch) issue(c + C::D, slot == 0 ? C::SLOTS - 1 : slot - 1);
-    compute(slot);
-    slot = slot == C::SLOTS - 1 ? 0 : slot + 1;
+    asm volatile("" ::: "memory");
+    if (c + C::SLOTS < nch) issue(c + C::SLOTS, slot);
+    step(f0, after, 0, f1, true, true);
+    slot = after;
   }
+  step(f1, slot, 1, f0, true, true);
+  step(f0, slot, 0, f1, false, true);
 
   // ---- epilogue: lane holds features 16 t + 4 (lane >> 4) .. + 3 of token 16 mt + (lane & 15)
   const int S = gridDim.y;
@@ -298,28 +324,35 @@ void launch_mt_rw(const bf16* x, const bf16* W, float* y, int M, int N, int K, i
 template <int MT, int EPI>
 void launch_mt(const bf16* x, const bf16* W, float* y, int M, int N, int K, int S, int rw, const DecodeEpi& e,
                int* counters, hipStream_t s) {
-  if constexpr (MT > 8) {  // 256 rows: at most 2 weight tiles per wave (accumulators + LDS ring)
+  if constexpr (MT > 8) {  // 160 to 256 rows: at most 2 weight tiles per wave (accumulators + LDS ring)
     if (rw == 1) launch_mt_rw<MT, 1, EPI>(x, W, y, M, N, K, S, e, counters, s);
     else launch_mt_rw<MT, 2, EPI>(x, W, y, M, N, K, S, e, counters, s);
-    return;
-  }
-  switch (rw) {
-    case 1: launch_mt_rw<MT, 1, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
-    case 3: launch_mt_rw<MT, 3, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
-    case 4: launch_mt_rw<MT, 4, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
-    default: launch_mt_rw<MT, 2, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
+  } else {
+    switch (rw) {
+      case 1: launch_mt_rw<MT, 1, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
+      case 3: launch_mt_rw<MT, 3, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
+      case 4: launch_mt_rw<MT, 4, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
+      default: launch_mt_rw<MT, 2, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
+    }
   }
 }
 
 template <int EPI>
 void launch_epi_m(const bf16* x, const bf16* W, float* y, int M, int N, int K, int S, int rw, const DecodeEpi& e,
                   int* counters, hipStream_t s) {
+  constexpr bool fine = EPI < 0 || EPI == DECODE_EPI_SWIGLU;      // (the others are off by default)
   if (M <= 32)
     launch_mt<2, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
   else if (M <= 64)
     launch_mt<4, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
+  else if (fine && M <= 96)
+    launch_mt<fine ? 6 : 8, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
   else if (M <= 128)
     launch_mt<8, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
+  else if (fine && M <= 160)
+    launch_mt<fine ? 10 : 16, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
+  else if (fine && M <= 192)
+    launch_mt<fine ? 12 : 16, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
   else
     launch_mt<16, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
 }

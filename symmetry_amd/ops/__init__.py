@@ -132,16 +132,25 @@ def mgemm(x, w_shuf, y, rw: int):
 def choose_mgemm(M: int, N: int, K: int, cus: int = 256, fused: bool = False):
     """(rw, S) of mgemm for an [M, K] x [N, K]^T projection, or None where another kernel is the better
     choice.  Measured on MI355X (profiles/mgemm_r2.jsonl, mgemm_small_r2.jsonl; each arm followed by its
-    real consumer kernel): up to 64 rows mgemm beats both the split-K skinny GEMM and hipBLASLt on every
+    real consumer kernel, before the kernel read a step ahead): up to 64 rows mgemm beats both the split-K skinny GEMM and hipBLASLt on every
     Llama-3-8B projection; above 64 rows it wins for the narrow ones (N <= 8192: qkv / o / down) up to 192
     rows and for long-K or wider ones (down, qkv) up to 256, while the wide gate_up (N = 28672) stays on
     hipBLASLt.  A second wave of workgroups always lost, so only grids of 128..256 workgroups are
     considered, ranked by a linear model fitted to those sweeps: per-workgroup intake (64 rw weight rows +
     M activation rows over the k slice) at a per-CU rate that drops with the LDS ring depth (fewer slots
     at more rows), plus the S fp32 slabs written here and summed by the consumer, plus a fixed cost per
-    workgroup spread over the grid."""
+    workgroup spread over the grid.
+
+    ``fused`` (gate_up with its SwiGLU): wide projections past 64 rows as well, as one wave of whole columns, where those fill
+    three quarters of the CUs.  Against the library and the swiglu launch, us: 28672 x 4096 at 80 rows 49.6 / 62.3, 140 59.2 /
+    62.7, 192 66.1 / 68.9, 224 79.0 / 72.9; 16384 x 2048 at 80 rows 19.2 / 22.1, 140 23.3 / 30.0, 256 32.1 / 33.8; 57344 x 8192
+    at 96 rows 177 / 196; 22016 x 4096 (172 workgroups) at 128 rows 55.1 / 49.8."""
     if not _MGEMM_ON or M > MGEMM_MAX_M or K % 64:
         return None
+    if fused and M > 64 and N > 8192:
+        rw = next((r for r in (4, 3, 2, 1) if N % (64 * r) == 0 and (M <= 128 or r <= 2)
+                   and 3 * cus // 4 <= N // (64 * r) <= cus), None)
+        return None if rw is None or (M > 192 and K > 2048) else (rw, 1)
     if M > 64 and (N > 8192 or (M > 192 and K < 8192 and N < 6144)):
         return None
     mt = 2 if M <= 32 else 4 if M <= 64 else 8 if M <= 128 else 16

@@ -329,6 +329,25 @@ def _mg(gpu, M, N, K):
             rw), S
 
 
+@pytest.mark.parametrize("M", [65, 96, 97, 129, 160, 161, 192, 193, 256])
+def test_gate_up_of_one_wave(gpu, M):
+    """gate_up and its SwiGLU as whole columns in one launch, at the ends of the row tiles: no slab, the deferred norm's scale."""
+    from symmetry_amd.models.layout import preshuffle
+
+    N, K = 12288, 512
+    pick = ops.choose_mgemm(M, N, K, fused=True)
+    assert pick is not None and pick[1] == 1 and 192 <= N // (64 * pick[0]) <= 256
+    x, W, s = _inputs(gpu, M, N, K, seed=M)
+    W = W[gu_perm(N // 2).to(gpu)].contiguous()
+    out = torch.full((M + 1, N // 2), 7.0, device=gpu, dtype=torch.bfloat16)
+    ops.dg_swiglu(x, preshuffle(W), s, 1e-5, out[:M], wshuf=True,
+                  mg=(torch.empty(1, M, N, device=gpu), torch.zeros(N // 64, dtype=torch.int32, device=gpu), pick[0]))
+    want = torch.empty(M, N // 2, dtype=torch.bfloat16)
+    ref.dg_swiglu(x.cpu(), W.cpu(), s.cpu(), 1e-5, want)
+    _close(out[:M], want, atol=2e-2, rtol=2e-2)
+    assert bool((out[M] == 7.0).all())
+
+
 @pytest.mark.parametrize("M", [1, 20, 33, 64, 100])
 @pytest.mark.parametrize("kind", ["qkv", "resid", "swiglu"])
 def test_mgemm_fused_epilogues(gpu, M, kind):

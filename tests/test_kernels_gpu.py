@@ -282,6 +282,29 @@ def test_logits_argmax(gpu):
     assert int(((kk >> 32) - (keys_ref >> 32)).abs().max()) <= 4  # value bits: __logf vs torch.log ulps
 
 
+@pytest.mark.parametrize("M", [1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 256])
+@pytest.mark.parametrize("chunks", [1, 2, 3, 4, 5, 8, 9, 13])
+def test_mgemm_tiles_and_ring(gpu, M, chunks):
+    """Every tile of rows at its ends, over k slices of fewer chunks than the ring has slots, as many, and one to several more,
+    for each number of weight tiles a wave.  fp32 sums of K terms err by about sqrt(K) 2^-24 of the terms' norm."""
+    from symmetry_amd.models.layout import preshuffle
+
+    K = 2 * 64 * chunks
+    g = torch.Generator(device=gpu).manual_seed(M + chunks)
+    x = torch.randn(M, K, device=gpu, generator=g).bfloat16()
+    for rw in (1, 2, 3, 4):
+        if M > 128 and rw > 2:
+            continue
+        w = torch.randn(128 * rw, K, device=gpu, generator=g).bfloat16()
+        y = torch.full((2, M, 128 * rw), float("nan"), device=gpu)
+        ops.mgemm(x, preshuffle(w), y, rw)
+        half = K // 2
+        for s in range(2):
+            xs, wk = x[:, s * half:(s + 1) * half].double(), w[:, s * half:(s + 1) * half].double()
+            room = 8 * half ** 0.5 * 2.0 ** -24 * xs.norm(dim=1)[:, None] * wk.norm(dim=1)[None]
+            assert bool(((y[s].double() - xs @ wk.t()).abs() <= room).all()), (rw, s)
+
+
 @pytest.mark.parametrize("V", [1, 3, 4, 129, 4092, 4096, 32764, 32768, 32770, 32772, 70004])
 @pytest.mark.parametrize("first", [0, 1])
 def test_logits_argmax_finds_the_first_largest(gpu, V, first):

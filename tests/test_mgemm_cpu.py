@@ -22,6 +22,15 @@ def test_chooser_respects_kernel_contract(M, N, K):
     assert 128 <= N // (64 * rw) * S <= 256
 
 
+@pytest.mark.parametrize("M", [65, 128, 129, 192, 193, 256])
+@pytest.mark.parametrize("N,K", [(28672, 4096), (16384, 2048), (57344, 8192), (22016, 4096), (8256, 2048)])
+def test_wide_fused_columns_fill_one_wave(M, N, K):
+    pick = ops.choose_mgemm(M, N, K, fused=True)
+    if pick is not None:
+        assert pick[1] == 1 and N % (64 * pick[0]) == 0 and 192 <= N // (64 * pick[0]) <= 256 and (M <= 128 or pick[0] <= 2)
+    assert (pick is None) == (N == 22016 or N == 8256 or (M > 128 and N == 57344) or (M > 192 and K == 4096))
+
+
 def test_chooser_keeps_wide_and_long_prefills_on_the_library():
     assert ops.choose_mgemm(128, 28672, 4096) is None  # gate_up: hipBLASLt streams it at ~5.5 TB/s
     assert ops.choose_mgemm(300, 4096, 4096) is None   # beyond the medium range
