@@ -32,7 +32,6 @@
 
 namespace {
 
-constexpr int MG_THR = 256;
 constexpr int MG_LDS = 160 * 1024;
 
 typedef __attribute__((address_space(3))) void lds_t;
@@ -51,14 +50,15 @@ SYM_DEV void mg_dma_nt(__amdgpu_buffer_rsrc_t r, int voff, int soff, char* lds) 
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t*)lds, 16, voff, soff, 0, 2);
 }
 
-template <int MT, int RW>
+// WV waves, a multiple of 4 of them or not: a chunk's 2 MT x DMAs go round the waves, the last ones twice where they do not divide
+template <int MT, int RW, int WV>
 struct MgCfg {
   static constexpr int XB = 16 * MT * 128;                   // x bytes of one 64-deep chunk
-  static constexpr int WB = 4 * RW * 2 * 1024;               // weight bytes of one chunk (2 blocks per tile)
+  static constexpr int WB = WV * RW * 2 * 1024;               // weight bytes of one chunk (2 blocks per tile)
   static constexpr int SLOT = XB + WB;
   static constexpr int SLOTS = MG_LDS / SLOT > 8 ? 8 : MG_LDS / SLOT;
   static constexpr int D = SLOTS - 1;                        // chunks in flight ahead of the computed one
-  static constexpr int NX = 16 * MT / 32;                    // x DMA instructions per wave per chunk (MT >= 2)
+  static constexpr int NX = (2 * MT + WV - 1) / WV;          // x DMA instructions per wave per chunk
   static constexpr int NDMA = NX + 2 * RW;                   // DMA instructions per wave per chunk
   static constexpr int VM_KEEP = (D - 1) * NDMA;             // younger DMAs left in flight at the wait
   static_assert(MT % 2 == 0 && D >= 1 && VM_KEEP <= 63, "mgemm config");
@@ -73,11 +73,11 @@ struct MgCfg {
 // slabs of its columns in the accumulator layout, applies the deferred-RMSNorm row scale (e.ss_in) and runs
 // the epilogue -- the separate rope_cache / add+RMSNorm / SwiGLU launches of the slab path disappear.
 // `counters` [N / (64 RW)] start at zero and are re-armed by the last arriver (graph-replay safe).
-template <int MT, int RW, bool WNT, int EPI>
-__global__ __launch_bounds__(MG_THR, 1) void mgemm_kernel(const bf16* __restrict__ x, const bf16* __restrict__ W,
+template <int MT, int RW, bool WNT, int EPI, int WV>
+__global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restrict__ x, const bf16* __restrict__ W,
                                                            float* __restrict__ y, int M, int N, int K, int kslice,
                                                            DecodeEpi e, int* __restrict__ counters) {
-  using C = MgCfg<MT, RW>;
+  using C = MgCfg<MT, RW, WV>;
   __shared__ __attribute__((aligned(1024))) char smem[C::SLOTS * C::SLOT];
   asm volatile("" ::: "a0");  // accumulators may live in AGPRs
 
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(MG_THR, 1) void mgemm_kernel(const bf16* __restrict
   const int split = blockIdx.y;
   const int k0 = split * kslice;
   const int nch = kslice / 64;
-  const int tile0 = (blockIdx.x * 4 + wid) * RW;  // first 16-row weight tile of this wave
+  const int tile0 = (blockIdx.x * WV + wid) * RW;  // first 16-row weight tile of this wave
 
   // ---- x DMA: wave w fills rows (NX w + i) * 8 .. + 8 of each chunk; lane -> (row lane >> 3, 16-B chunk
   // lane & 7), source chunk swizzled by (row >> 1) & 7.  Rows >= M read as zeros (buffer range).
@@ -93,20 +93,19 @@ __global__ __launch_bounds__(MG_THR, 1) void mgemm_kernel(const bf16* __restrict
   int vx[C::NX];
 #pragma unroll
   for (int i = 0; i < C::NX; ++i) {
-    const int row = (C::NX * wid + i) * 8 + (lane >> 3);
+    const int row = min(C::NX * wid + i, 2 * MT - 1) * 8 + (lane >> 3);
     vx[i] = row * K * 2 + 16 * ((lane & 7) ^ ((row >> 1) & 7)) + k0 * 2;
   }
   // ---- weight DMA: the wave's own tiles, block (tile, 2c + s) -> its 1 KB LDS block, lane-linear
   const __amdgpu_buffer_rsrc_t rw = mg_rsrc(W, (long long)N * K * 2);
   const int vw = (tile0 * (K / 32) + k0 / 32) * 1024 + lane * 16;
   const int wstride = (K / 32) * 1024;  // bytes between consecutive weight tiles
-  char* const dx = smem + (C::NX * wid) * 1024;
   char* const dw = smem + C::XB + wid * RW * 2 * 1024;
 
   auto issue = [&](int c, int slot) {
     const int xo = c * 128, wo = c * 2048;
 #pragma unroll
-    for (int i = 0; i < C::NX; ++i) mg_dma(rx, vx[i], xo, dx + slot * C::SLOT + i * 1024);
+    for (int i = 0; i < C::NX; ++i) mg_dma(rx, vx[i], xo, smem + slot * C::SLOT + min(C::NX * wid + i, 2 * MT - 1) * 1024);
 #pragma unroll
     for (int rt = 0; rt < RW; ++rt) {
       if constexpr (WNT) {
@@ -167,7 +166,7 @@ __global__ __launch_bounds__(MG_THR, 1) void mgemm_kernel(const bf16* __restrict
   int tpr = 1;
   if constexpr (EPI >= 0) {
     if (e.ss_in) {
-      while (tpr < 64 && tpr * 2 * M <= MG_THR) tpr *= 2;
+      while (tpr < 64 && tpr * 2 * M <= 64 * WV) tpr *= 2;
       const int row = threadIdx.x / tpr, sub = threadIdx.x % tpr;
       if (row < M) {
         rn_row = row;
@@ -310,20 +309,32 @@ __global__ __launch_bounds__(MG_THR, 1) void mgemm_kernel(const bf16* __restrict
 
 int g_mgemm_nt = 0;
 
-template <int MT, int RW, int EPI>
+template <int MT, int RW, int EPI, int WV = 4>
 void launch_mt_rw(const bf16* x, const bf16* W, float* y, int M, int N, int K, int S, const DecodeEpi& e,
                   int* counters, hipStream_t s) {
+  const dim3 grid(N / (16 * WV * RW), S);
   if (g_mgemm_nt && EPI < 0)
-    mgemm_kernel<MT, RW, true, EPI><<<dim3(N / (64 * RW), S), dim3(MG_THR), 0, s>>>(x, W, y, M, N, K, K / S, e,
-                                                                                   counters);
+    mgemm_kernel<MT, RW, true, EPI, WV><<<grid, 64 * WV, 0, s>>>(x, W, y, M, N, K, K / S, e, counters);
   else
-    mgemm_kernel<MT, RW, false, EPI><<<dim3(N / (64 * RW), S), dim3(MG_THR), 0, s>>>(x, W, y, M, N, K, K / S, e,
-                                                                                    counters);
+    mgemm_kernel<MT, RW, false, EPI, WV><<<grid, 64 * WV, 0, s>>>(x, W, y, M, N, K, K / S, e, counters);
 }
 
 template <int MT, int EPI>
 void launch_mt(const bf16* x, const bf16* W, float* y, int M, int N, int K, int S, int rw, const DecodeEpi& e,
                int* counters, hipStream_t s) {
+  if constexpr (EPI == DECODE_EPI_SWIGLU && MT <= 12) {
+    // Seven waves where their columns fill the CUs better than four waves' do (widths of 7 x 2^n, as 2 x 14336): a CU's intake
+    // is what bounds the stream.  28672 x 4096, 224 workgroups -> 256,
+    // us: 64 rows 50.8 -> 44.5, 96 52.4 -> 46.9, 128 56.9 -> 51.4, 192 67.3 -> 64.3; 57344 x 8192 at 96 rows 177 -> 175
+    if (S == 1 && N % 112 == 0 && N / 112 <= 256 && N / 112 > N / (64 * rw)) {
+      launch_mt_rw<MT, 1, EPI, 7>(x, W, y, M, N, K, S, e, counters, s);
+      return;
+    }
+    if (S == 1 && N % 224 == 0 && N / 224 <= 256 && N / 224 > N / (64 * rw)) {
+      launch_mt_rw<MT, 2, EPI, 7>(x, W, y, M, N, K, S, e, counters, s);
+      return;
+    }
+  }
   if constexpr (MT > 8) {  // 160 to 256 rows: at most 2 weight tiles per wave (accumulators + LDS ring)
     if (rw == 1) launch_mt_rw<MT, 1, EPI>(x, W, y, M, N, K, S, e, counters, s);
     else launch_mt_rw<MT, 2, EPI>(x, W, y, M, N, K, S, e, counters, s);

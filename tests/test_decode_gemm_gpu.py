@@ -329,19 +329,22 @@ def _mg(gpu, M, N, K):
             rw), S
 
 
-@pytest.mark.parametrize("M", [65, 96, 97, 129, 160, 161, 192, 193, 256])
-def test_gate_up_of_one_wave(gpu, M):
-    """gate_up and its SwiGLU as whole columns in one launch, at the ends of the row tiles: no slab, the deferred norm's scale."""
+@pytest.mark.parametrize("N,K", [(12288, 512), (28672, 320), (57344, 128)])
+@pytest.mark.parametrize("M", [17, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 256])
+def test_gate_up_of_one_wave(gpu, M, N, K):
+    """gate_up and its SwiGLU as whole columns in one launch, at the ends of the row tiles, four waves and seven (one and two
+    weight tiles each): no slab, the deferred norm's scale."""
     from symmetry_amd.models.layout import preshuffle
 
-    N, K = 12288, 512
-    pick = ops.choose_mgemm(M, N, K, fused=True)
-    assert pick is not None and pick[1] == 1 and 192 <= N // (64 * pick[0]) <= 256
+    rw = {12288: 1, 28672: 2, 57344: 4}[N]
+    if M > 128 and rw > 2:
+        pytest.skip("rw <= 2 above 128 rows")
+    assert M <= 64 or M > 192 or ops.choose_mgemm(M, N, 4096, fused=True) == (rw, 1)
     x, W, s = _inputs(gpu, M, N, K, seed=M)
     W = W[gu_perm(N // 2).to(gpu)].contiguous()
     out = torch.full((M + 1, N // 2), 7.0, device=gpu, dtype=torch.bfloat16)
     ops.dg_swiglu(x, preshuffle(W), s, 1e-5, out[:M], wshuf=True,
-                  mg=(torch.empty(1, M, N, device=gpu), torch.zeros(N // 64, dtype=torch.int32, device=gpu), pick[0]))
+                  mg=(torch.empty(1, M, N, device=gpu), torch.zeros(N // 64, dtype=torch.int32, device=gpu), rw))
     want = torch.empty(M, N // 2, dtype=torch.bfloat16)
     ref.dg_swiglu(x.cpu(), W.cpu(), s.cpu(), 1e-5, want)
     _close(out[:M], want, atol=2e-2, rtol=2e-2)
