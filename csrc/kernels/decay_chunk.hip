@@ -21,8 +21,13 @@
 // the contraction taken in the order j < 4: 4 g + j, else 16 + 4 g + j - 4, two accumulator tiles ARE a B operand, and the A
 // operand is read in the same order (two 8-byte LDS reads).  The same holds for the values and, computed transposed, for the
 // scores.  The next chunk's rows are loaded while the current one is multiplied (two LDS stages, one barrier a chunk).
-#include "common.h"
+// One or two waves a SIMD: what a chunk costs is its vector instructions and every wait that nothing covers.  8100 tokens in 8
+// runs, us: 8 heads x 128 x 256 300 -> 228, 64 x 128 x 64 258 -> 200 with pairs rounded at once, rows through a buffer's range,
+// k turned by LDS transpose reads instead of 2-byte stores (a third of the time in bank conflicts) and reads a step ahead.
+#include "attn_tiles.h"
 #include "hybrid_launchers.h"
+
+#include <algorithm>
 
 namespace {
 
@@ -41,21 +46,32 @@ SYM_DEV float pow2(float v) { return __builtin_amdgcn_exp2f(v); }
 SYM_DEV f32x4 mfma4(float x, float y, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); }
 SYM_DEV f32x4 lds4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
 struct Parts {
   bf16x8 h, m, l;
 };
 
+// (two at a time: v_cvt_pk_bf16_f32 rounds a pair, and a bf16 is a float's upper half; 5.5 instructions a number, 9.7 one by one)
 SYM_DEV Parts split(f32x4 a, f32x4 b) {
-  Parts s;
+  union {
+    unsigned int u[4];
+    bf16x8 v;
+  } h, m, l;
+  auto round2 = [](float x, float y) {
+    const bf16x2 p = __builtin_convertvector((f32x2){x, y}, bf16x2);
+    return __builtin_bit_cast(unsigned int, p);
+  };
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float x = i < 4 ? a[i & 3] : b[i & 3];
-    s.h[i] = (bf16)x;
-    const float r = x - (float)s.h[i];
-    s.m[i] = (bf16)r;
-    s.l[i] = (bf16)(r - (float)s.m[i]);
+  for (int i = 0; i < 4; ++i) {
+    const float x = i < 2 ? a[2 * i] : b[2 * i - 4], y = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+    h.u[i] = round2(x, y);
+    const float rx = x - __uint_as_float(h.u[i] << 16), ry = y - __uint_as_float(h.u[i] & 0xffff0000u);
+    m.u[i] = round2(rx, ry);
+    l.u[i] = round2(rx - __uint_as_float(m.u[i] << 16), ry - __uint_as_float(m.u[i] & 0xffff0000u));
   }
-  return s;
+  return Parts{h.v, m.v, l.v};
 }
 
 // an A operand in the accumulators' contraction order: 4 elements at p, 4 at p + 16
@@ -69,8 +85,44 @@ SYM_DEV bf16x8 pair4(const bf16* p) {
   return r.v;
 }
 
+// Rows of a chunk through a buffer whose range ends with the chunk's last row: what lies behind it reads 0 and is not stored, and a
+// lane's places in a chunk are the same 32-bit offsets in every chunk (64-bit products per load and a check each were a third of
+// the walk's vector time).  row, width: bytes from row to row, of a row's part; off: OUT for a lane without a place.
+constexpr int OUT = 0x7fffffff;
+SYM_DEV __amdgpu_buffer_rsrc_t chunk_rows(const void* base, long long row, int nt, int width) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)((nt - 1) * row) + width, 0x00020000);
+}
+SYM_DEV uint4 row16(__amdgpu_buffer_rsrc_t r, int off) {
+  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+SYM_DEV f32x4 row16f(__amdgpu_buffer_rsrc_t r, int off) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+SYM_DEV bf16 row2(__amdgpu_buffer_rsrc_t r, int off) {
+  return __builtin_bit_cast(bf16, __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
+}
+
+// inclusive sums over lanes 0 .. 31, in the vector unit
+template <int CTRL>
+SYM_DEV double lanes_before(double v) {      // (lanes without one: 0)
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned int lo = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xf, 0xf, false);
+  const unsigned int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+SYM_DEV double prefix32(double v, int lane) {
+  v += lanes_before<0x111>(v);               // row_shr 1, 2, 4, 8
+  v += lanes_before<0x112>(v);
+  v += lanes_before<0x114>(v);
+  v += lanes_before<0x118>(v);
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned int lo = __builtin_amdgcn_readlane((int)u, 15), hi = __builtin_amdgcn_readlane((int)(u >> 32), 15);
+  return lane < 16 ? v : v + __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
 // mode 0's scratch per (row, head): row of A | 2^(G_i) | k_i 2^(G_C - G_i)
-SYM_DEV int ws_cols(int N) { return C + 2 * N; }
+__host__ __device__ inline int ws_cols(int N) { return C + 2 * N; }
 
 // ---- mode 0: decays and scores A of every chunk, grid (64-row tiles x 2 chunks, heads) ----------------------------------
 // G is held as a pair of floats: what counts are its differences, and once a few tokens of a chunk forget hard, G is in the
@@ -195,10 +247,10 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
 // ---- the walk ------------------------------------------------------------------------------------------------------------
 // NB: 32-channel blocks of the state (N <= 32 NB)
 template <int MODE, int NB>
-__global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a) {
+__global__ __launch_bounds__(NT, MODE == 0 ? 1 : 2) void decay_chunk_scan_kernel(DecayScanArgs a) {
   constexpr int NP = 32 * NB, LQ = NP + 8;              // LQ: bf16 pitch of a [C][NP] matrix
   constexpr int PL = MODE == 0 ? 3 : 1;                 // bf16 parts of the staged vectors
-  constexpr int oK = PL * C * LQ, oT = oK + (MODE == 1 ? C * LQ : 0), oF = oT + PL * NP * LT;   // in bf16: q | k (mode 1) | k^T
+  constexpr int oK = PL * C * LQ, oF = oK + PL * C * LQ;      // in bf16: q | k, a part behind the other
   constexpr int FS = MODE == 0 ? C * LT + NP : 3 * C;   // floats: A | 2^(G_C), or G | its low part | b
   constexpr int STAGE = oF * 2 + FS * 4;                // bytes
   static_assert(STAGE % 16 == 0, "stages start at multiples of 16 bytes");
@@ -213,13 +265,15 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
   const int pr = a.prev_row[s0], sv = a.save_slot[s1 - 1];
   const bf16* q = reinterpret_cast<const bf16*>(a.q) + s0 * a.ldq + (h / a.hpg) * N;
   const bf16* k = reinterpret_cast<const bf16*>(a.k) + s0 * a.ldk + (h / a.hpg) * N;
-  const bf16* v = reinterpret_cast<const bf16*>(a.v) + s0 * a.ldv + (long long)h * P + p;
+  const bf16* v = reinterpret_cast<const bf16*>(a.v) + s0 * a.ldv + (long long)h * P;
   const bf16* dt = reinterpret_cast<const bf16*>(a.dz) + s0 * a.ldd + h;          // mode 1
   const int wc = ws_cols(N);
   const long long wrow = (long long)a.H * wc;
   const float* ws = MODE == 0 ? a.ws + ((long long)s0 * a.H + h) * wc : nullptr;
-  float* out = a.out + ((long long)s0 * a.H + h) * P + p;
+  float* out = a.out + ((long long)s0 * a.H + h) * P;
   const long long orow = (long long)a.H * P;
+  const int ldv = (int)a.ldv * 2, ldo = (int)orow * 4;                            // (decay_chunk_takes bounds them)
+  const int vo = pin ? 4 * g * ldv + 2 * p : OUT, oo = pin ? 4 * g * ldo + 4 * p : OUT;
 
   // staging: thread (token tt, 8 channels from c8), PASS tokens apart
   constexpr int GR = NP / 8, TSTEP = NT / GR, PASS = (C + TSTEP - 1) / TSTEP;
@@ -229,38 +283,41 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
   f32x4 rp[MODE == 0 ? PASS : 1][2], ry[MODE == 0 ? PASS : 1][2], pl, ra;   // mode 0: 2^(G_i), k_i 2^(G_C - G_i), 2^(G_C)
   float rdt = 0.f;
   bf16 vn[8];
+  int qo[PASS], ko[PASS], wo[PASS];
+#pragma unroll
+  for (int u = 0; u < PASS; ++u) {
+    const int tt = tt0 + TSTEP * u;
+    qo[u] = nin ? tt * (int)a.ldq * 2 + 2 * c8 : OUT;
+    ko[u] = nin ? tt * (int)a.ldk * 2 + 2 * c8 : OUT;
+    wo[u] = nin ? tt * (int)wrow * 4 + 4 * (C + c8) : OUT;
+  }
   auto fetch = [&](int c) {
     const int t0 = c * C, nt = min(C, s1 - s0 - t0);
+    const __amdgpu_buffer_rsrc_t bq = chunk_rows(q + t0 * a.ldq, a.ldq * 2, nt, N * 2);
 #pragma unroll
-    for (int u = 0; u < PASS; ++u) {
-      const int tt = tt0 + TSTEP * u;
-      const bool in = nin && tt < nt;
-      rq[u].u = in ? *reinterpret_cast<const uint4*>(q + (t0 + tt) * a.ldq + c8) : make_uint4(0, 0, 0, 0);
-      if constexpr (MODE == 0) {
-        const float* x = ws + (t0 + tt) * wrow + C + c8;
+    for (int u = 0; u < PASS; ++u) rq[u].u = row16(bq, qo[u]);
+    if constexpr (MODE == 0) {
+      const __amdgpu_buffer_rsrc_t bw = chunk_rows(ws + t0 * wrow, wrow * 4, nt, wc * 4);
+#pragma unroll
+      for (int u = 0; u < PASS; ++u)
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          rp[u][i] = in ? lds4(x + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
-          ry[u][i] = in ? lds4(x + N + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+          rp[u][i] = row16f(bw, wo[u] + (nin ? 16 * i : 0));
+          ry[u][i] = row16f(bw, wo[u] + (nin ? 4 * N + 16 * i : 0));
         }
-      } else {
-        rk[u].u = in ? *reinterpret_cast<const uint4*>(k + (t0 + tt) * a.ldk + c8) : make_uint4(0, 0, 0, 0);
-      }
-    }
-    if constexpr (MODE == 0) {
       pl = 4 * tid < N ? lds4(ws + (t0 + nt - 1) * wrow + C + 4 * tid) : f32x4{0.f, 0.f, 0.f, 0.f};
-      ra = tid / 8 < nt ? lds4(ws + (t0 + tid / 8) * wrow + 4 * (tid % 8)) : f32x4{0.f, 0.f, 0.f, 0.f};
-    } else if (tid < C) {
-      rdt = tid < nt ? (float)dt[(long long)(t0 + tid) * a.ldd] + a.dbias[h] : 0.f;
+      ra = row16f(bw, (tid / 8) * (int)wrow * 4 + 16 * (tid % 8));
+    } else {
+      const __amdgpu_buffer_rsrc_t bk = chunk_rows(k + t0 * a.ldk, a.ldk * 2, nt, N * 2);
+#pragma unroll
+      for (int u = 0; u < PASS; ++u) rk[u].u = row16(bk, ko[u]);
+      if (tid < C) rdt = (float)row2(chunk_rows(dt + t0 * a.ldd, a.ldd * 2, nt, 2), tid * (int)a.ldd * 2) + a.dbias[h];
     }
   };
   auto fetch_v = [&](int c) {
-    const int nt = min(C, s1 - s0 - c * C);
+    const __amdgpu_buffer_rsrc_t bv = chunk_rows(v + (long long)c * C * a.ldv, a.ldv * 2, min(C, s1 - s0 - c * C), P * 2);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int tt = 16 * (i >> 2) + 4 * g + (i & 3);
-      vn[i] = tt < nt && pin ? v[(c * C + tt) * a.ldv] : (bf16)0.f;
-    }
+    for (int i = 0; i < 8; ++i) vn[i] = row2(bv, vo + (pin ? (16 * (i >> 2) + (i & 3)) * ldv : 0));
   };
   const float rate2 = MODE == 1 ? expf(a.rate[h]) * LOG2E : 0.f;
   auto stash = [&](int c) {
@@ -274,8 +331,6 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
       if constexpr (MODE == 1) {
         *reinterpret_cast<uint4*>(st + tt * LQ + c8) = rq[u].u;
         *reinterpret_cast<uint4*>(st + oK + tt * LQ + c8) = rk[u].u;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) st[oT + (c8 + i) * LT + tt] = rk[u].h[i];
       } else {
         f32x4 x[2];
 #pragma unroll
@@ -284,12 +339,9 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
         *reinterpret_cast<bf16x8*>(st + tt * LQ + c8) = sx.h;
         *reinterpret_cast<bf16x8*>(st + (C + tt) * LQ + c8) = sx.m;
         *reinterpret_cast<bf16x8*>(st + (2 * C + tt) * LQ + c8) = sx.l;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          st[oT + (c8 + i) * LT + tt] = sy.h[i];
-          st[oT + (NP + c8 + i) * LT + tt] = sy.m[i];
-          st[oT + (2 * NP + c8 + i) * LT + tt] = sy.l[i];
-        }
+        *reinterpret_cast<bf16x8*>(st + oK + tt * LQ + c8) = sy.h;
+        *reinterpret_cast<bf16x8*>(st + oK + (C + tt) * LQ + c8) = sy.m;
+        *reinterpret_cast<bf16x8*>(st + oK + (2 * C + tt) * LQ + c8) = sy.l;
       }
     }
     if constexpr (MODE == 0) {
@@ -300,11 +352,7 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
       // to hundreds, and the differences of neighbours, which are what counts, would keep few of its digits
       const float b = tid < nt ? softplus_exact(rdt) : 0.f;
       double s = tid < nt ? log_decay(-(double)rate2 * b) : 0.0;
-#pragma unroll
-      for (int o = 1; o < C; o <<= 1) {
-        const double up = __shfl_up(s, o, 64);
-        if (tid >= o) s += up;
-      }
+      s = prefix32(s, tid);
       if (tid < C) {
         fs[tid] = (float)s;
         fs[C + tid] = (float)(s - (double)(float)s);
@@ -343,22 +391,54 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
     const float* fs = reinterpret_cast<const float*>(st + oF);
     const bf16* Qr = st + col * LQ + 4 * g;
     f32x4 O[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    f32x4 A[2][2];                                      // scores of row tile i, columns 4 g + r and 16 + 4 g + r
+    f32x4 gj[2], lj[2], bj[2];
+    // A wave or two a SIMD: LDS reads stand a step ahead of the products that take them, and the parts of the next state tiles
+    // are formed between products (left to the compiler, every read was waited for: half of the walk).
+    bf16x8 qf[2][PL][2];
+    auto load_q = [&](int t) {
+#pragma unroll
+      for (int part = 0; part < PL; ++part)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) qf[t & 1][part][i] = pair4(Qr + (part * C + 16 * i) * LQ + 32 * t);
+    };
+    load_q(0);
+    if (NB > 1) load_q(1);
+    if constexpr (MODE == 0) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) A[i][j] = lds4(fs + (16 * i + col) * LT + 16 * j + 4 * g);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        gj[j] = lds4(fs + 16 * j + 4 * g);
+        lj[j] = lds4(fs + C + 16 * j + 4 * g);
+        bj[j] = lds4(fs + 2 * C + 16 * j + 4 * g);
+      }
+    }
+    Parts s = split(S[0], S[1]);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < NB; ++t) {
-      const Parts s = split(S[2 * t], S[2 * t + 1]);
+      Parts next = s;
+      if (t + 1 < NB) next = split(S[2 * t + 2], S[2 * t + 3]);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const bf16x8 qh = pair4(Qr + 16 * i * LQ + 32 * t);
-        O[i] = mfma16(qh, s.l, O[i]);
-        if constexpr (MODE == 0) {
-          const bf16x8 qm = pair4(Qr + (C + 16 * i) * LQ + 32 * t), ql = pair4(Qr + (2 * C + 16 * i) * LQ + 32 * t);
-          O[i] = mfma16(ql, s.h, O[i]);
-          O[i] = mfma16(qm, s.m, O[i]);
-          O[i] = mfma16(qm, s.h, O[i]);
+      for (int term = 0; term < (MODE == 0 ? 6 : 3); ++term)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {                   // the smallest terms first
+          const auto& f = qf[t & 1];
+          if constexpr (MODE == 0) {
+            constexpr int qp[6] = {0, 2, 1, 1, 0, 0};
+            const bf16x8 sp = term == 0 ? s.l : term == 2 || term == 4 ? s.m : s.h;
+            O[i] = mfma16(f[qp[term]][i], sp, O[i]);
+          } else {
+            O[i] = mfma16(f[0][i], term == 0 ? s.l : term == 1 ? s.m : s.h, O[i]);
+          }
         }
-        O[i] = mfma16(qh, s.m, O[i]);
-        O[i] = mfma16(qh, s.h, O[i]);
-      }
+      if (t + 2 < NB) load_q(t + 2);
+      s = next;
+      __builtin_amdgcn_sched_barrier(0);
     }
     // The product of scores and values runs over the scores' masked half as well, where 0 x inf would reach the rows in front
     // of a value that is not finite: it is left out of the product, and its column is NaN from its token on.
@@ -376,51 +456,68 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
       bad = min(bad, __shfl_xor(bad, 16, 64));
       bad = min(bad, __shfl_xor(bad, 32, 64));
     }
-    f32x4 A[2][2];                                      // scores of row tile i, columns 4 g + r and 16 + 4 g + r
-    f32x4 gj[2], lj[2], bj[2];
-    if constexpr (MODE == 0) {
+    if constexpr (MODE == 1) {
+      bf16x8 kf[2][NB], qn[2][NB];
+      float gi[2], li[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        gi[i] = fs[16 * i + col], li[i] = fs[C + 16 * i + col];
+#pragma unroll
+        for (int t = 0; t < NB; ++t) {
+          kf[i][t] = *reinterpret_cast<const bf16x8*>(st + oK + (16 * i + col) * LQ + 8 * g + 32 * t);
+          qn[i][t] = *reinterpret_cast<const bf16x8*>(st + (16 * i + col) * LQ + 8 * g + 32 * t);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) O[j][r] *= pow2(gj[j][r]);      // (rows 4 g + r of O too)
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) A[i][j] = lds4(fs + (16 * i + col) * LT + 16 * j + 4 * g);
-    } else {
+        for (int j = 0; j < 2; ++j) A[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        gj[j] = lds4(fs + 16 * j + 4 * g);
-        lj[j] = lds4(fs + C + 16 * j + 4 * g);
-        bj[j] = lds4(fs + 2 * C + 16 * j + 4 * g);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) O[j][r] *= pow2(gj[j][r]);      // (rows 4 g + r of O too)
+      for (int t = 0; t < NB; ++t) {
+        A[0][0] = mfma16(kf[0][t], qn[0][t], A[0][0]);
+        A[1][0] = mfma16(kf[0][t], qn[1][t], A[1][0]);
+        A[1][1] = mfma16(kf[1][t], qn[1][t], A[1][1]);
       }
-      const bf16* Kn = st + oK + col * LQ + 8 * g;
-      const bf16* Qn = st + col * LQ + 8 * g;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const float gi = fs[16 * i + col], li = fs[C + 16 * i + col];
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          f32x4 d = {0.f, 0.f, 0.f, 0.f};
-          if (j <= i) {
+        for (int j = 0; j <= i; ++j)
 #pragma unroll
-            for (int t = 0; t < NB; ++t)
-              d = mfma16(*reinterpret_cast<const bf16x8*>(Kn + 16 * j * LQ + 32 * t),
-                         *reinterpret_cast<const bf16x8*>(Qn + 16 * i * LQ + 32 * t), d);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const float w = pow2((gi - gj[j][r]) + (li - lj[j][r])) * bj[j][r];
-              d[r] = j < i || 4 * g + r <= col ? d[r] * w : 0.f;
-            }
+          for (int r = 0; r < 4; ++r) {
+            const float w = pow2((gi[i] - gj[j][r]) + (li[i] - lj[j][r])) * bj[j][r];
+            float y = A[i][j][r] * w;
+            asm volatile("" : "+v"(y));                 // (a select, no branch around the exponential)
+            A[i][j][r] = j < i || 4 * g + r <= col ? y : 0.f;
           }
-          A[i][j] = d;
-        }
-      }
     }
+    // k^T as an A operand in the accumulators' order: 16 channels of 4 tokens at 4 g, 4 at 16 + 4 g (LDS transpose reads)
+    const char* Kt = reinterpret_cast<const char*>(st + oK + (4 * g + (col >> 2)) * LQ) + 8 * (col & 3);
+    auto turned = [&](int part, int t) {
+      Pack8 f;
+      const uint2 x = read_tr(Kt + (part * C * LQ + 16 * t) * 2), y = read_tr(Kt + ((part * C + 16) * LQ + 16 * t) * 2);
+      f.u = make_uint4(x.x, x.y, y.x, y.y);
+      return f.v;
+    };
+    bf16x8 kt[2 * NB];                                  // of the part at hand
+#pragma unroll
+    for (int t = 0; t < 2 * NB; ++t) kt[t] = turned(PL - 1, t);
+    f32x4 dec[MODE == 0 ? 2 * NB : 1];
+    if constexpr (MODE == 0) {
+#pragma unroll
+      for (int t = 0; t < 2 * NB; ++t) dec[t] = lds4(fs + C * LT + 16 * t + 4 * g);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const Parts s = split(A[i][0], A[i][1]);
-      O[i] = mfma16(s.l, W.v, O[i]);
-      O[i] = mfma16(s.m, W.v, O[i]);
-      O[i] = mfma16(s.h, W.v, O[i]);
+      const Parts u = split(A[i][0], A[i][1]);
+      O[i] = mfma16(u.l, W.v, O[i]);
+      O[i] = mfma16(u.m, W.v, O[i]);
+      O[i] = mfma16(u.h, W.v, O[i]);
     }
     if (bad < C) {
 #pragma unroll
@@ -429,23 +526,31 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
         for (int r = 0; r < 4; ++r)
           if (16 * i + 4 * g + r >= bad) O[i][r] = __builtin_nanf("");
     }
-    if (pin) {
+    {
+      const __amdgpu_buffer_rsrc_t bo = chunk_rows(out + (long long)c * C * orow, orow * 4, nt, P * 4);
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int tt = 16 * i + 4 * g + r;
-          if (tt < nt) out[(c * C + tt) * orow] = a.q_scale * O[i][r] + skip * (float)V.h[4 * i + r];
+          const float y = a.q_scale * O[i][r] + skip * (float)V.h[4 * i + r];
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), bo, oo + (pin ? (16 * i + r) * ldo : 0), 0, 0);
         }
     }
-    const bf16* Kt = st + oT + col * LT + 4 * g;
     if constexpr (MODE == 0) {
 #pragma unroll
-      for (int t = 0; t < 2 * NB; ++t) {
-        S[t] *= lds4(fs + C * LT + 16 * t + 4 * g);
-        S[t] = mfma16(pair4(Kt + (2 * NP + 16 * t) * LT), V.v, S[t]);
-        S[t] = mfma16(pair4(Kt + (NP + 16 * t) * LT), V.v, S[t]);
-        S[t] = mfma16(pair4(Kt + 16 * t * LT), V.v, S[t]);
+      for (int t = 0; t < 2 * NB; ++t) S[t] *= dec[t];
+#pragma unroll
+      for (int part = 2; part >= 0; --part) {
+        bf16x8 nk[2 * NB];
+#pragma unroll
+        for (int t = 0; t < 2 * NB; ++t)
+          if (part) nk[t] = turned(part - 1, t);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < 2 * NB; ++t) S[t] = mfma16(kt[t], V.v, S[t]);
+#pragma unroll
+        for (int t = 0; t < 2 * NB; ++t)
+          if (part) kt[t] = nk[t];
       }
     } else {
       const float gc = fs[C - 1], lc = fs[2 * C - 1], d = pow2(gc);     // (G stands still past the run's end)
@@ -454,15 +559,13 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) w[j][r] = pow2((gc - gj[j][r]) + (lc - lj[j][r])) * bj[j][r] * (float)V.h[4 * j + r];
-      const Parts s = split(w[0], w[1]);
+      const Parts u = split(w[0], w[1]);
 #pragma unroll
-      for (int t = 0; t < 2 * NB; ++t) {
-        S[t] *= d;
-        const bf16x8 kt = pair4(Kt + 16 * t * LT);
-        S[t] = mfma16(kt, s.l, S[t]);
-        S[t] = mfma16(kt, s.m, S[t]);
-        S[t] = mfma16(kt, s.h, S[t]);
-      }
+      for (int t = 0; t < 2 * NB; ++t) S[t] = mfma16(kt[t], u.l, S[t] * d);
+#pragma unroll
+      for (int t = 0; t < 2 * NB; ++t) S[t] = mfma16(kt[t], u.m, S[t]);
+#pragma unroll
+      for (int t = 0; t < 2 * NB; ++t) S[t] = mfma16(kt[t], u.h, S[t]);
     }
     if (more) stash(c + 1);
     __syncthreads();                                    // chunk c + 1 is staged, chunk c has been read
@@ -482,7 +585,7 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
 template <int MODE, int NB>
 void launch_chunks(const DecayScanArgs& a, hipStream_t s) {
   constexpr int NP = 32 * NB, LQ = NP + 8, PL = MODE == 0 ? 3 : 1;
-  constexpr int elems = PL * C * LQ + (MODE == 1 ? C * LQ : 0) + PL * NP * LT;
+  constexpr int elems = 2 * PL * C * LQ;
   constexpr int lds = 2 * (elems * 2 + (MODE == 0 ? C * LT + NP : 3 * C) * 4);
   constexpr int prep = 4 * C * (NP + 4) * 4;
   static const bool raised = [] {
@@ -514,6 +617,8 @@ bool decay_chunk_takes(const DecayScanArgs& a) {
   auto aligned = [](const void* p, long long ld) { return (uintptr_t)p % 16 == 0 && ld % 8 == 0; };
   if (a.mode > 1 || !a.cu_q || a.T < (a.mode == 0 ? 48LL : 8LL) * a.runs || a.N % 8 || a.N > 128) return false;
   if (!aligned(a.q, a.ldq) || !aligned(a.k, a.ldk)) return false;
+  constexpr long long top = 1 << 24;      // (a chunk of 32 rows is addressed by 32-bit offsets)
+  if (std::max({a.ldq, a.ldk, a.ldv, a.ldd, (long long)a.H * a.P, (long long)a.H * ws_cols(a.N)}) > top) return false;
   return a.mode == 1 || (a.tiles && a.ntiles > 0 && a.ws && (uintptr_t)a.ws % 16 == 0);
 }
 
