@@ -207,6 +207,13 @@ SYM_DEV f32x4 exp2_neg(f32x4 v) {       // 2^v for exponents that are <= 0 where
   return r;
 }
 
+// rows of a chunk through a buffer whose range ends with the chunk's last row: what lies behind it reads 0 and is not stored.
+// row, width: bytes from row to row, of a row's part; OUT: the place of a lane without one
+constexpr int OUT = 0x7fffffff;
+SYM_DEV __amdgpu_buffer_rsrc_t chunk_rows(const void* base, long long row, int nt, int width) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)((nt - 1) * row) + width, 0x00020000);
+}
+
 // grid (64-row tiles x 2 chunks, heads); NN: 16-channel tiles (N <= 16 NN)
 template <bool CHANNEL, int NN>
 __global__ __launch_bounds__(NT) void delta_chunk_prep_kernel(DeltaRuleArgs a) {
@@ -408,11 +415,13 @@ __global__ __launch_bounds__(NT) void delta_chunk_prep_kernel(DeltaRuleArgs a) {
   }
 }
 
-// grid (P / 64, heads, runs), 512 threads: waves 0 .. 3 multiply (16 value columns each), waves 4 .. 7 stage.  NN: 16-row
-// tiles of the state (N <= 16 NN); NBUF: LDS stages (two where they fit)
-template <typename T, bool CHANNEL, int NN, int NBUF>
-__global__ __launch_bounds__(2 * NT) void delta_chunk_scan_kernel(DeltaRuleArgs a) {
+// grid (P / (16 MW), heads, runs): waves 0 .. MW - 1 multiply (16 value columns each), as many more stage.  NN: 16-row tiles of
+// the state (N <= 16 NN); NBUF: LDS stages (two where they fit).  With four and four a multiplying and a staging wave share a
+// SIMD, and their times all but add up (68 us alone and 42 alone, 95 together); two and two have a SIMD each.
+template <typename T, bool CHANNEL, int NN, int NBUF, int MW>
+__global__ __launch_bounds__(128 * MW) void delta_chunk_scan_kernel(DeltaRuleArgs a) {
   extern __shared__ float lds[];
+  constexpr int NT = 64 * MW;                  // staging threads
   constexpr int NP = 16 * NN;                  // padded key channels
   constexpr int LD = NP + 4;
   constexpr int TSTEP = NT / NP, EPT = C / TSTEP;      // a staging thread owns channel n of the tokens tt0, tt0 + TSTEP, ..
@@ -425,7 +434,7 @@ __global__ __launch_bounds__(2 * NT) void delta_chunk_scan_kernel(DeltaRuleArgs 
   const int chunks = (s1 - s0 + C - 1) / C;
   const int wc = ws_cols(CHANNEL, N);
   const long long wrow = (long long)a.H * wc;
-  if (wave >= 4) {
+  if (wave >= MW) {
     // ---- staging waves -----------------------------------------------------------------------------------------
     const int tid = threadIdx.x - NT, n = tid % NP, tt0 = tid / NP;
     const bool nin = n < N;
@@ -508,20 +517,22 @@ __global__ __launch_bounds__(2 * NT) void delta_chunk_scan_kernel(DeltaRuleArgs 
   }
   // ---- multiplying waves -----------------------------------------------------------------------------------------
   const int col = lane & 15, g = lane >> 4;
-  const int p = blockIdx.x * 64 + wave * 16 + col;
+  const int p = blockIdx.x * 16 * MW + wave * 16 + col;
   const bool pin = p < P;
   const int pr = a.prev_row[s0];
   const int sv = a.save_slot[s1 - 1];
   const long long hp = (long long)a.H * P;
-  const T* v = reinterpret_cast<const T*>(a.v) + (long long)s0 * hp + (long long)h * P + p;
-  float* out = a.out + (long long)s0 * hp + (long long)h * P + p;
+  const T* v = reinterpret_cast<const T*>(a.v) + (long long)s0 * hp + (long long)h * P;
+  float* out = a.out + (long long)s0 * hp + (long long)h * P;
+  const int vo = (int)sizeof(T) * (4 * g * (int)hp + p), oo = 4 * (4 * g * (int)hp + p);      // (launch_delta_rule bounds H P)
   float vn[8];
   auto fetch_v = [&](int c) {
-    const int nt = min(C, s1 - s0 - c * C);
+    const __amdgpu_buffer_rsrc_t bv = chunk_rows(v + (long long)c * C * hp, sizeof(T) * hp, min(C, s1 - s0 - c * C), (int)sizeof(T) * P);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int tt = 16 * (i >> 2) + 4 * g + (i & 3);
-      vn[i] = tt < nt && pin ? (float)v[(long long)(c * C + tt) * hp] : 0.f;
+      const int off = pin ? vo + (16 * (i >> 2) + (i & 3)) * (int)(sizeof(T) * hp) : OUT;
+      if constexpr (sizeof(T) == 2) vn[i] = (float)__builtin_bit_cast(bf16, __builtin_amdgcn_raw_buffer_load_b16(bv, off, 0, 0));
+      else vn[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(bv, off, 0, 0));
     }
   };
   f32x4 S[NN];
@@ -544,61 +555,72 @@ __global__ __launch_bounds__(2 * NT) void delta_chunk_scan_kernel(DeltaRuleArgs 
     const float* Tm = st + oT + col * LC + 4 * g;
     const float* Aq = st + oA + col * LC + 4 * g;
     const float* D = st + oD + 4 * g;
+    // One multiplying wave a SIMD: every LDS read stands a step ahead of the products that take it (left to the compiler each
+    // was waited for, more time than the products: 17 chunks of 8 heads x 128 x 256, 3 runs, 110 us; 88 this way).
+    f32x4 x[2][4];
+    auto load = [&](int t) {
+      x[t & 1][0] = lds4(Kt + 16 * t), x[t & 1][1] = lds4(Kt + 16 * LD + 16 * t);
+      x[t & 1][2] = lds4(Qt + 16 * t), x[t & 1][3] = lds4(Qt + 16 * LD + 16 * t);
+    };
+    load(0);
     const f32x4 V0 = {vn[0], vn[1], vn[2], vn[3]}, V1 = {vn[4], vn[5], vn[6], vn[7]};
     if (c + 1 < chunks) fetch_v(c + 1);
-    f32x4 K0 = {0.f, 0.f, 0.f, 0.f}, K1 = K0, O0 = K0, O1 = K0;
+    f32x4 K0 = {0.f, 0.f, 0.f, 0.f}, K1 = K0, O0 = K0, O1 = K0, m[6], d[2], kh[2][2];
 #pragma unroll
     for (int t = 0; t < NN; ++t) {
-      const f32x4 x0 = lds4(Kt + 16 * t), x1 = lds4(Kt + 16 * LD + 16 * t);
-      const f32x4 y0 = lds4(Qt + 16 * t), y1 = lds4(Qt + 16 * LD + 16 * t);
+      if (t + 1 < NN) {
+        load(t + 1);
+      } else {
+        m[0] = lds4(Tm), m[1] = lds4(Tm + 16 * LC), m[2] = lds4(Tm + 16 * LC + 16);
+        m[3] = lds4(Aq), m[4] = lds4(Aq + 16 * LC), m[5] = lds4(Aq + 16 * LC + 16);
+      }
+      d[t & 1] = lds4(D + 16 * t);
+      __builtin_amdgcn_sched_barrier(0);
+      const f32x4(&y)[4] = x[t & 1];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        K0 = mfma4(x0[r], S[t][r], K0);
-        K1 = mfma4(x1[r], S[t][r], K1);
-        O0 = mfma4(y0[r], S[t][r], O0);
-        O1 = mfma4(y1[r], S[t][r], O1);
+        K0 = mfma4(y[0][r], S[t][r], K0);
+        K1 = mfma4(y[1][r], S[t][r], K1);
+        O0 = mfma4(y[2][r], S[t][r], O0);
+        O1 = mfma4(y[3][r], S[t][r], O1);
       }
+      if (t) S[t - 1] *= d[(t - 1) & 1];       // (its products are out)
+      __builtin_amdgcn_sched_barrier(0);
     }
+    S[NN - 1] *= d[(NN - 1) & 1];
+    kh[0][0] = lds4(Kh), kh[0][1] = lds4(Kh + 16);
+    __builtin_amdgcn_sched_barrier(0);
     const f32x4 R0 = V0 - K0, R1 = V1 - K1;
     f32x4 U0 = {0.f, 0.f, 0.f, 0.f}, U1 = U0;
-    {
-      const f32x4 x00 = lds4(Tm), x10 = lds4(Tm + 16 * LC), x11 = lds4(Tm + 16 * LC + 16);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        U0 = mfma4(x00[r], R0[r], U0);
-        U1 = mfma4(x10[r], R0[r], U1);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) U1 = mfma4(x11[r], R1[r], U1);
-    }
-    {
-      const f32x4 x00 = lds4(Aq), x10 = lds4(Aq + 16 * LC), x11 = lds4(Aq + 16 * LC + 16);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        O0 = mfma4(x00[r], U0[r], O0);
-        O1 = mfma4(x10[r], U0[r], O1);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) O1 = mfma4(x11[r], U1[r], O1);
+    for (int r = 0; r < 4; ++r) {
+      U0 = mfma4(m[0][r], R0[r], U0);
+      U1 = mfma4(m[1][r], R0[r], U1);
     }
 #pragma unroll
-    for (int t = 0; t < NN; ++t) S[t] = S[t] * lds4(D + 16 * t);
+    for (int r = 0; r < 4; ++r) U1 = mfma4(m[2][r], R1[r], U1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      O0 = mfma4(m[3][r], U0[r], O0);
+      O1 = mfma4(m[4][r], U0[r], O1);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) O1 = mfma4(m[5][r], U1[r], O1);
 #pragma unroll
     for (int t = 0; t < NN; ++t) {
-      const f32x4 x0 = lds4(Kh + 16 * t * LC), x1 = lds4(Kh + 16 * t * LC + 16);
+      if (t + 1 < NN) kh[(t + 1) & 1][0] = lds4(Kh + 16 * (t + 1) * LC), kh[(t + 1) & 1][1] = lds4(Kh + 16 * (t + 1) * LC + 16);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) S[t] = mfma4(x0[r], U0[r], S[t]);
+      for (int r = 0; r < 4; ++r) S[t] = mfma4(kh[t & 1][0][r], U0[r], S[t]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) S[t] = mfma4(x1[r], U1[r], S[t]);
+      for (int r = 0; r < 4; ++r) S[t] = mfma4(kh[t & 1][1][r], U1[r], S[t]);
     }
-    if (pin) {
-      const int nt = min(C, s1 - s0 - c * C);
+    const int nt = min(C, s1 - s0 - c * C);
+    const __amdgpu_buffer_rsrc_t bo = chunk_rows(out + (long long)c * C * hp, 4 * hp, nt, 4 * P);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i0 = 4 * g + r, i1 = 16 + i0;
-        if (i0 < nt) out[(long long)(c * C + i0) * hp] = O0[r];
-        if (i1 < nt) out[(long long)(c * C + i1) * hp] = O1[r];
-      }
+    for (int r = 0; r < 4; ++r) {
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(O0[r]), bo, pin ? oo + r * 4 * (int)hp : OUT, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(O1[r]), bo, pin ? oo + (16 + r) * 4 * (int)hp : OUT, 0, 0);
     }
     if (NBUF == 1) __syncthreads();            // chunk c has been read
     __syncthreads();                           // chunk c + 1 is staged (two stages: and chunk c has been read)
@@ -646,21 +668,31 @@ void serial(const DeltaRuleArgs& a, hipStream_t s) {
   else launch_serial<T, CHANNEL, 32, 8, 8>(a, s);      // N <= 256 (checked by the op layer)
 }
 
-template <typename T, bool CHANNEL, int NN>
-void launch_chunks(const DeltaRuleArgs& a, hipStream_t s) {
+template <typename T, bool CHANNEL, int NN, int MW>
+void launch_scan(const DeltaRuleArgs& a, hipStream_t s) {
   constexpr int NP = 16 * NN, LD = NP + 4;
   constexpr int STAGE = 2 * C * LD + NP * LC + 2 * C * LC + NP;
   constexpr int NBUF = 2 * STAGE * (int)sizeof(float) <= 160 * 1024 ? 2 : 1;
+  static const bool raised = (raise_lds(reinterpret_cast<const void*>(&delta_chunk_scan_kernel<T, CHANNEL, NN, NBUF, MW>)), true);
+  (void)raised;
+  const dim3 grid((a.P + 16 * MW - 1) / (16 * MW), a.H, a.runs);
+  delta_chunk_scan_kernel<T, CHANNEL, NN, NBUF, MW><<<grid, 128 * MW, (size_t)NBUF * STAGE * sizeof(float), s>>>(a);
+}
+
+template <typename T, bool CHANNEL, int NN>
+void launch_chunks(const DeltaRuleArgs& a, hipStream_t s) {
+  constexpr int LD = 16 * NN + 4;
   const size_t prep = (size_t)((CHANNEL ? 3 : 2) * C * LD + 4 * C * LC + 2 * C) * sizeof(float);
-  const size_t scan = (size_t)NBUF * STAGE * sizeof(float);
-  static bool raised = false;
-  if (!raised) {
-    raise_lds(reinterpret_cast<const void*>(&delta_chunk_prep_kernel<CHANNEL, NN>));
-    raise_lds(reinterpret_cast<const void*>(&delta_chunk_scan_kernel<T, CHANNEL, NN, NBUF>));
-    raised = true;
-  }
+  static const bool raised = (raise_lds(reinterpret_cast<const void*>(&delta_chunk_prep_kernel<CHANNEL, NN>)), true);
+  (void)raised;
   delta_chunk_prep_kernel<CHANNEL, NN><<<dim3(2 * a.ntiles, a.H), NT, prep, s>>>(a);
-  delta_chunk_scan_kernel<T, CHANNEL, NN, NBUF><<<dim3((a.P + 63) / 64, a.H, a.runs), 2 * NT, scan, s>>>(a);
+  // 32 columns a workgroup while those are at most one a CU (256) and runs are long enough that the first chunk's staging, which
+  // half as many waves do, is not what counts; else 64 (8 heads x 128 x 256, us with 32 / with 64 columns: 3 runs of 512 tokens
+  // 76 / 88, 5 runs 146 / 87, one of 4000 498 / 639, 3 runs of 200 40.7 / 40.3, of 60 17.6 / 14.9)
+  if constexpr (NN <= 8) {
+    if ((long long)((a.P + 31) / 32) * a.H * a.runs <= 256 && a.T >= 8LL * C * a.runs) return launch_scan<T, CHANNEL, NN, 2>(a, s);
+  }
+  launch_scan<T, CHANNEL, NN, 4>(a, s);
 }
 
 template <typename T, bool CHANNEL>
@@ -677,7 +709,7 @@ void chunked(const DeltaRuleArgs& a, hipStream_t s) {
 
 int launch_delta_rule(const DeltaRuleArgs& a, int channel, int f32, int impl, hipStream_t s) {
   if (a.runs <= 0 || a.T <= 0) return 1;
-  const bool chunk = impl == 0 && a.tiles && a.ntiles > 0 && a.ws && a.cu_q;
+  const bool chunk = impl == 0 && a.tiles && a.ntiles > 0 && a.ws && a.cu_q && (long long)a.H * a.P <= 1 << 23;      // (32-bit places in a chunk)
   if (f32) {
     if (chunk) channel ? chunked<float, true>(a, s) : chunked<float, false>(a, s);
     else channel ? serial<float, true>(a, s) : serial<float, false>(a, s);

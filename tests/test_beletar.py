@@ -656,6 +656,40 @@ def test_delta_rule_handed_over_through_slots(device, impl, channel, shape):
     assert float(state[1].min()) == 1e4            # the unused slot was never written
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("shape", [(2, 1, 9, 33), (3, 3, 64, 70), (1, 1, 128, 16), (2, 2, 40, 32), (1, 1, 130, 40), (40, 40, 16, 128)])
+def test_delta_rule_long_runs(channel, shape):
+    """Runs of more than 256 rows, which walk 32 value columns a workgroup where those are at most one a CU (the last shape has
+    more, and key channels past 128 keep 64): columns that fill no workgroup, a last chunk of one row, a state carried in.
+    Rounding adds up with the root of the rows: 4e-6 at 117 of them (above) is 6.5e-6 here."""
+    H, G, N, P = shape
+    say("op delta_rule long", channel, shape)
+    na, nb = 300, 257
+    qa, ka, va, dza, dtb, A, bza, lga, _, _ = _delta_case(channel, H, G, N, P, na, 1)
+    qb, kb, vb, dzb, _, _, bzb, _, _, _ = _delta_case(channel, H, G, N, P, nb, 2)
+    lgb = -torch.exp(A.double())[None, :, None] * O.softplus((dzb + dtb).double().view(nb, H, -1)).expand(nb, H, N)
+    start = 0.1 * torch.randn(H, N, P)
+    want_a, Sa = O.delta_rule(qa.double(), ka.double(), va.double(), lga, torch.sigmoid(bza.double()))
+    want_b, Sb = O.delta_rule(qb.double(), kb.double(), vb.double(), lgb, torch.sigmoid(bzb.double()), start.double())
+    prev = torch.tensor([-1] + list(range(na - 1)) + [-3] + list(range(na, na + nb - 1)), dtype=torch.int32)      # (-3: slot 1)
+    save = torch.full((na + nb,), -1, dtype=torch.int32)
+    save[na - 1], save[-1] = 0, 2
+    tiles = torch.tensor([[0, r] for r in range(0, na, 64)] + [[1, r] for r in range(0, nb, 64)], dtype=torch.int32)
+    state = torch.full((3, H, N, P), 1e4)
+    state[1] = start
+    y = torch.full((na + nb, H, P), 1e4)
+    ws = torch.full((na + nb, H, ops.delta_ws_cols(channel, N)), float("nan"))
+    cat = [torch.cat([x, z]) for x, z in ((qa, qb), (ka, kb), (va, vb), (dza, dzb), (bza, bzb))]
+    q, k, v, dz, bz, y, ws, prev, save, cu, tiles, state, dtb, A = _dev(
+        "cuda", *cat, y, ws, prev, save, torch.tensor([0, na, na + nb], dtype=torch.int32), tiles, state, dtb, A)
+    assert ops.delta_rule(channel, q, k, v, dz, dtb, A, bz, state, cu, prev, save, 2, y, tiles, ws) == 0
+    assert float((y[:na].cpu().double() - want_a).abs().max()) < 6.5e-6
+    assert float((y[na:].cpu().double() - want_b).abs().max()) < 6.5e-6
+    assert float((state[0].cpu().double() - Sa).abs().max()) < 3.2e-5 and float((state[2].cpu().double() - Sb).abs().max()) < 3.2e-5
+    assert torch.equal(state[1].cpu(), start)
+
+
 @pytest.mark.parametrize("device,impl", FORMS)
 @pytest.mark.parametrize("channel", [False, True])
 def test_delta_rule_strong_decays_and_one_key_again(device, impl, channel):
