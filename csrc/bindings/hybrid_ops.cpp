@@ -439,6 +439,29 @@ void row_linear(const Tensor& x, const Tensor& w, Tensor& out, bool relu2, bool 
               "row_linear: K = ", K, " is neither at most 256 nor a multiple of 256");
 }
 
+// y = x . W^T of 17 to 256 rows in bf16; x and out may be column ranges; glu as above; false: the sizes have no kernel
+bool mid_linear(const Tensor& x, const Tensor& w, Tensor& out, bool glu, Tensor& slab, Tensor& counters) {
+  gpu(x, "x", false);
+  gpu(out, "out", false);
+  dtype(w, at::kBFloat16, "w");
+  dtype(slab, at::kFloat, "slab");
+  dtype(counters, at::kInt, "counters");
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16 && x.dim() == 2 && w.dim() == 2 && out.dim() == 2,
+              "mid_linear: bf16, 2-d operands");
+  const int64_t M = x.size(0), K = x.size(1), N = out.size(1);
+  TORCH_CHECK(M >= 1 && M <= 256 && out.size(0) == M && w.size(1) == K && w.size(0) == (glu ? 2 * N : N), "mid_linear: shapes");
+  TORCH_CHECK(K >= 64 && K % 64 == 0 && K <= (1 << 22) && N >= 4 && N % 4 == 0 && N <= (1 << 28), "mid_linear: K in 64s, N in 4s");
+  TORCH_CHECK(x.stride(1) == 1 && out.stride(1) == 1, "mid_linear: inner strides must be 1");
+  const int64_t ldx = M > 1 ? x.stride(0) : K, ldo = M > 1 ? out.stride(0) : N;
+  TORCH_CHECK(ldx >= K && ldx % 8 == 0 && ldx <= (1 << 24) && ldo >= N && ldo % 4 == 0 && ldo <= (1 << 28), "mid_linear: row strides");
+  TORCH_CHECK((uintptr_t)x.data_ptr() % 16 == 0 && (uintptr_t)w.data_ptr() % 16 == 0 && (uintptr_t)out.data_ptr() % 8 == 0 &&
+                  (uintptr_t)slab.data_ptr() % 16 == 0, "mid_linear: alignment");
+  TORCH_CHECK(slab.numel() >= MID_SLAB && counters.numel() >= 256, "mid_linear: workspace too small");
+  const at::OptionalDeviceGuard g(x.device());
+  return launch_mid_linear(x.data_ptr(), ldx, w.data_ptr(), out.data_ptr(), ldo, (int)M, (int)N, (int)K, glu, ptr<float>(slab),
+                           ptr<int>(counters), cur_stream(x));
+}
+
 void relu_sq(const Tensor& a, Tensor& out) {
   const int f32 = act(out, "out");
   TORCH_CHECK(out.dim() == 2, "relu_sq: out [R, F]");
@@ -1172,6 +1195,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
   m.def("conv_state_update(Tensor xin, Tensor(a!) state, Tensor? cu_q, Tensor prev_row, Tensor save_slot, int runs) -> ()",
         &conv_state_update);
   m.def("row_linear(Tensor x, Tensor w, Tensor(a!) out, bool relu2, bool glu) -> ()", &row_linear);
+  m.def("mid_linear(Tensor x, Tensor w, Tensor(a!) out, bool glu, Tensor(b!) slab, Tensor(c!) counters) -> bool", &mid_linear);
   m.def("relu_sq(Tensor a, Tensor(a!) out) -> ()", &relu_sq);
   m.def("silu_mul(Tensor gate, Tensor up, Tensor(a!) out) -> ()", &silu_mul);
   m.def(

@@ -67,6 +67,11 @@ struct ConvArgs {
 // (save_slot: only with cu_q null; the state moves on in the same launch)
 void launch_causal_conv_silu(const ConvArgs& a, int f32, hipStream_t s);
 void launch_conv_state_update(const ConvArgs& a, int f32, hipStream_t s);
+// out = x . W^T of 17 to 256 rows (glu: silu(gate) * up of W's [gate | up] rows); slab: MID_SLAB floats, counters: 256 zeros, left
+// zero; false: not one of its sizes
+constexpr long long MID_SLAB = 256LL * 128 * 256;
+bool launch_mid_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int glu, float* slab,
+                       int* counters, hipStream_t s);
 // out = x . W^T (relu2: of relu(x)^2; glu: silu(gate) * up of W's [gate | up] rows); false: this K has no kernel
 bool launch_row_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int f32_out,
                        int relu2, int glu, hipStream_t s);

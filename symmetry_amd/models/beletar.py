@@ -92,6 +92,8 @@ class BeletarLM:
         self.dtype = dtype
         self.tp_size, self.tp_rank = 1, 0
         self.ws = Workspace()
+        if self.device.type != "cpu" and dtype == torch.bfloat16:
+            ops.mid_workspace(self.ws, self.device)      # (before any graph is captured)
         self.last_ids = torch.zeros(MAX_STEP_SEQS, dtype=torch.int32, device=self.device)
         self.last_logits = None
         self.layer_outputs: list | None = None   # set to a list: every forward appends the stream after each layer run
@@ -175,7 +177,7 @@ class BeletarLM:
 
     def _linear(self, name: str, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """x [R, K] @ w[N, K]^T -> [R, N] in the activation dtype (library GEMM, fp32 accumulation)."""
-        return ops.linear(x, w, out=self._buf(name, (x.shape[0], w.shape[0])))
+        return ops.linear(x, w, self._buf(name, (x.shape[0], w.shape[0])), self.ws)
 
     def _linear_f32(self, name: str, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """x [R, K] @ w[N, K]^T -> fp32 [R, N] (the library GEMM's accumulator, unrounded)."""
@@ -247,8 +249,7 @@ class BeletarLM:
     def _ff(self, P: dict, h: torch.Tensor) -> torch.Tensor:
         F = P["mlp"].ff
         act = self._buf("ff.act", (h.shape[0], F))
-        if self.dtype == torch.bfloat16 and ops.few_rows(h, P["w_gu"], act):  # gate, up and their product in one launch
-            ops.row_linear(h, P["w_gu"], act, glu=True)
+        if self.dtype == torch.bfloat16 and ops.linear_glu(h, P["w_gu"], act, self.ws):  # gate, up and their product in one launch
             return self._linear("ff.down", act, P["w_down"])
         gu = self._linear("ff.gu", h, P["w_gu"])
         ops.silu_mul(gu[:, :F], gu[:, F:], act)

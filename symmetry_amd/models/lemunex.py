@@ -111,6 +111,8 @@ class LemunexLM:
         self.dtype = dtype
         self.tp_size, self.tp_rank = 1, 0
         self.ws = Workspace()
+        if self.device.type != "cpu" and dtype == torch.bfloat16:
+            ops.mid_workspace(self.ws, self.device)      # (before any graph is captured)
         self.last_ids = torch.zeros(MAX_STEP_SEQS, dtype=torch.int32, device=self.device)
         self.last_logits = None
         cfg = self.cfg
@@ -195,7 +197,7 @@ class LemunexLM:
 
     def _linear(self, name: str, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """x [R, K] @ w[N, K]^T -> [R, N] in the activation dtype (fp32 accumulation)."""
-        return ops.linear(x, w, out=self._buf(name, (x.shape[0], w.shape[0])))
+        return ops.linear(x, w, self._buf(name, (x.shape[0], w.shape[0])), self.ws)
 
     @staticmethod
     def _cols(z: torch.Tensor, P: dict, name: str) -> torch.Tensor:

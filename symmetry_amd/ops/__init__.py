@@ -551,16 +551,22 @@ def few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None) -> bool
     x and w on the GPU, 1..16 rows, w contiguous, unit inner strides, 16-byte aligned rows of x and w, K at most 256 in
     eights or a multiple of 256, outputs in fours; everything else is the library's: tensors of other classes (fake ones of
     a tracer, distributed ones), graphs that are being compiled, and whatever autograd records, backward or forward."""
-    if torch.compiler.is_compiling() or out is None or not _plain(x, w, out):
+    if out is None or x.dim() != 2 or not 0 < x.shape[0] <= FEW_ROWS:
         return False
-    if x.dim() != 2 or not 0 < x.shape[0] <= FEW_ROWS or w.dim() != 2 or out.dim() != 2:
+    K = x.shape[1]
+    return (K % 256 == 0 or (K < 256 and K % 8 == 0)) and 0 < K <= 1 << 22 and _own_linear(x, w, out)
+
+
+def _own_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+    """What the kernels of few and of medium rows ask of their operands beside the rows and K."""
+    if torch.compiler.is_compiling() or not _plain(x, w, out) or w.dim() != 2 or out.dim() != 2:
         return False
     if not _gpu(x) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not w.is_contiguous():
         return False
     M, K = x.shape
     if w.device != x.device or out.device != x.device or w.shape[1] != K or out.shape[0] != M:
         return False
-    if not (K % 256 == 0 or (K < 256 and K % 8 == 0)) or not 0 < K <= 1 << 22 or out.shape[1] % 4 or not 0 < out.shape[1] <= 1 << 30:
+    if out.shape[1] % 4 or not 0 < out.shape[1] <= 1 << 30:
         return False
     if x.stride(1) != 1 or out.stride(1) != 1 or (M > 1 and (x.stride(0) % 8 or not 0 < x.stride(0) <= 1 << 24)):
         return False
@@ -572,6 +578,59 @@ def few_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None) -> bool
         torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or out.requires_grad))
 
 
+MID_ROWS = 256  # rows up to which a linear layer may be the medium kernel's (csrc/kernels/mid_linear.hip)
+
+
+def mid_pays(M: int, N: int, K: int, glu: bool = False) -> bool:
+    """Is the medium-row kernel ahead of the library for N outputs (glu: pairs)?  Measured with other weights read in between, us,
+    library / kernel.  Wide outputs always: 17440 x 2048 at 32 rows 23.3 / 19.4, 64 26.0 / 24.4, 160 39.3 / 31.2, 256 44.4 / 40.3.
+    Long K while the parts of K's slices are few: 2048 x 8192 at 32 rows 16.7 / 12.3, 64 25.0 / 15.6, 96 22.0 / 20.0, 128 22.0 /
+    23.0; 4096 x 14336 at 128 rows 91.8 / 48.1, 224 62.2 / 66.8.  Others at the ends of the range: 6144 x 2048 at 32 rows 12.6 /
+    10.4, 64 13.5 / 14.2, 192 26.5 / 22.5; 2048 x 2048 at 32 rows 8.5 / 8.0, 48 8.6 / 9.7; 2048 x 4096 at 48 12.4 / 11.7.  Pairs
+    with the launch that multiplied them: 8192 x 2048 at 64 rows 23.5 / 22.5, 128 27.3 / 29.9, 192 41.0 / 35.3; 14336 x 4096 at
+    96 rows 58.5 / 56.6, 160 68.7 / 72.9."""
+    if K < 2048 or N < 2048:
+        return False
+    if glu:
+        return M <= 64 or (K <= 2048 and M > 128)
+    if N >= 16384:
+        return True
+    if K >= 8192:
+        return M <= 96 or (N >= 4096 and M <= 192)
+    return M <= 32 or (M <= 48 and (N >= 4096 or K >= 4096)) or (M > 160 and N >= 4096)
+
+
+def mid_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None, ws, glu: bool = False) -> bool:
+    """Does x @ w.T into ``out`` (glu: w of twice out's columns) run on the medium-row kernel?  17..256 rows in bf16 with a
+    workspace to split K in, K in 64s, where it pays; few_rows' conditions otherwise."""
+    if ws is None or out is None or x.dim() != 2 or not FEW_ROWS < x.shape[0] <= MID_ROWS or out.dim() != 2:
+        return False
+    M, K = x.shape
+    if not mid_pays(M, out.shape[1], K, glu) or K % 64 or K > 1 << 20 or out.dtype != torch.bfloat16 or 2 * w.numel() > 0x7FFFFFFF:
+        return False
+    return K <= x.stride(0) <= 1 << 20 and out.stride(0) <= 1 << 28 and _own_linear(x, w, out)
+
+
+def mid_linear(x, w, out, ws, glu: bool = False) -> bool:
+    """out [M, N] bf16 = x @ w.T for mid_rows operands (``glu`` as in row_linear); False where the kernel has no plan for the sizes."""
+    slab, counters = mid_workspace(ws, x.device)
+    return _hyb().mid_linear(x, w, out, bool(glu), slab, counters)
+
+
+def mid_workspace(ws, device):
+    """The medium-row kernel's parts and arrival counters (zero before and after every launch) in a model's workspace."""
+    return (ws.get("linear.slab", (256 * 128 * 256,), torch.float32, device),
+            ws.get("linear.counters", (256,), torch.int32, device, zeros=True))
+
+
+def linear_glu(x, w, out, ws) -> bool:
+    """out = silu(gate) * up with w's [gate | up] rows in one launch, where a kernel takes the operands."""
+    if few_rows(x, w, out):
+        row_linear(x, w, out, glu=True)
+        return True
+    return mid_rows(x, w, out, ws, True) and w.shape[0] == 2 * out.shape[1] and mid_linear(x, w, out, ws, True)
+
+
 def row_linear(x, w, out, relu2: bool = False, glu: bool = False) -> None:
     """out [M, N] (bf16, or fp32 = the unrounded accumulator) = x @ w.T for few_rows operands.  ``relu2``: relu(x)^2, rounded to
     bf16, in place of x; ``glu``: w [2 N, K] holds [gate | up] rows and out = silu(gate) * up of the bf16 projections."""
@@ -580,12 +639,14 @@ def row_linear(x, w, out, relu2: bool = False, glu: bool = False) -> None:
     return reference.row_linear(x, w, out, relu2, glu)
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-    """``x @ w.T``: the few-row kernel up to 16 rows (2048 x 2048 at 8 rows 4.8 us, the library 8.5; 17688 x 2048 21.9 / 49.6;
-    past 16 rows the library is ahead), else the library GEMM (hipBLASLt through torch, the library heuristic; a
+def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, ws=None) -> torch.Tensor:
+    """``x @ w.T``: the few-row kernel up to 16 rows (2048 x 2048 at 8 rows 4.8 us, the library 8.5; 17688 x 2048 21.9 / 49.6),
+    with a workspace ``ws`` (a model's: ``get(name, shape, dtype, device, zeros)``) the medium-row kernel up to 256, else the library GEMM (hipBLASLt through torch, the library heuristic; a
     tuned-solution table measured neutral end to end and was removed: profiles/r4/blaslt_tuned_ab.jsonl)."""
     if few_rows(x, w, out) and out.dtype == torch.bfloat16 and out.shape[1] == w.shape[0]:
         row_linear(x, w, out)
+        return out
+    if ws is not None and mid_rows(x, w, out, ws) and out.shape[1] == w.shape[0] and mid_linear(x, w, out, ws):
         return out
     return torch.matmul(x, w.t(), out=out)
 
