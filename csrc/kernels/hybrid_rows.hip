@@ -59,6 +59,32 @@ __global__ __launch_bounds__(BT) void embed_norm_kernel(const int* __restrict__ 
   for (int c = threadIdx.x; c < d; c += BT) x[(long long)row * d + c] = (float)t[c] * r * (offset + w[c]);
 }
 
+// The same for prompt rows in bf16, d <= 8 BT in eights: a row is read once, in 16-byte pieces (column by column and twice: 40 ->
+// 24 us at 8100 rows of 2048, whose traffic takes 20).
+template <int BT>
+__global__ __launch_bounds__(BT) void embed_norm_vec_kernel(const int* __restrict__ ids, const int* __restrict__ src,
+                                                            const int* __restrict__ prev, const bf16* __restrict__ table,
+                                                            const float* __restrict__ w, float eps, float offset,
+                                                            float* __restrict__ x, int d) {
+  __shared__ float scratch[BT / 64];
+  const int row = blockIdx.x, c = 8 * threadIdx.x;
+  const int sr = src ? src[row] : -1;
+  const long long tok = sr >= 0 ? prev[sr] : ids[row];
+  const bool on = c < d;
+  float v[8], wv[8], sq = 0.f;
+  if (on) {
+    load8(table + tok * d + c, v);
+    load8f(w + c, wv);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) sq += v[i] * v[i];
+  }
+  const float r = 1.f / sqrtf(block_sum<BT>(sq, scratch) / (float)d + eps);
+  if (!on) return;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = v[i] * r * (offset + wv[i]);
+  store8f(x + (long long)row * d + c, v);
+}
+
 template <typename T, int BT>
 __global__ __launch_bounds__(BT) void rms_norm_rows_kernel(const float* __restrict__ x, const long long* __restrict__ rows,
                                                            const float* __restrict__ w, float eps, float offset,
@@ -183,6 +209,42 @@ __global__ __launch_bounds__(BT) void qkv_rope_cache_kernel(QkvRopeArgs a) {
       vc[i] = (T)((float)z[nq + nk + i] + (a.bias ? a.bias[nq + nk + i] : 0.f));
 }
 
+// The same for prompt rows in bf16 whose pairs are neighbours: eight entries a thread, heads and rotary part in eights, so a piece is
+// of one head and rotates whole or not (entry by entry with a division each: 58 -> 24 us at 8100 rows of 16 + 4 + 4 heads of 128).
+constexpr int QT = 128;
+
+__global__ __launch_bounds__(QT) void qkv_rope_cache_vec_kernel(QkvRopeArgs a) {
+  const int row = blockIdx.x, nq = a.H * a.dk, nk = a.G * a.dk, nv = a.G * a.dv, rot = 2 * a.pairs;
+  const bf16* z = reinterpret_cast<const bf16*>(a.z) + (long long)row * a.ldz;
+  const float* cs = a.rope ? a.rope + (long long)a.positions[row] * rot : nullptr;   // [pairs][2]
+  const int slot = a.slots[row];
+  bf16* qo = reinterpret_cast<bf16*>(a.q_out) + (long long)row * nq;
+  bf16* kc = slot >= 0 ? reinterpret_cast<bf16*>(a.k_cache) + (long long)slot * nk : nullptr;
+  bf16* vc = slot >= 0 ? reinterpret_cast<bf16*>(a.v_cache) + (long long)slot * nv : nullptr;
+  const int all = slot >= 0 ? nq + nk + nv : nq;
+#pragma unroll 4
+  for (int i = 8 * threadIdx.x; i < all; i += 8 * QT) {
+    float v[8], b[8], t[8];
+    load8(z + i, v);
+    if (a.bias) {
+      load8f(a.bias + i, b);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] += b[u];
+    }
+    const int e = i < nq ? i % a.dk : (i - nq) % a.dk;
+    if (i < nq + nk && e < rot) {
+      load8f(cs + e, t);
+#pragma unroll
+      for (int u = 0; u < 8; u += 2) {
+        const float x = v[u], y = v[u + 1];
+        v[u] = x * t[u] - y * t[u + 1];
+        v[u + 1] = y * t[u] + x * t[u + 1];
+      }
+    }
+    store8(i < nq ? qo + i : i < nq + nk ? kc + i - nq : vc + i - nq - nk, v);
+  }
+}
+
 // grid (T, C / group); BT threads over the group's columns
 template <typename T, int BT>
 __global__ __launch_bounds__(BT) void gated_group_norm_kernel(const float* __restrict__ y, const T* __restrict__ gate,
@@ -235,6 +297,32 @@ __global__ __launch_bounds__(BT) void gated_group_norm_vec_kernel(const float* _
 #pragma unroll
   for (int i = 0; i < 8; ++i) v[i] = gate_first ? v[i] * r * wv[i] : v[i] * r * wv[i] * g[i];
   store8(out + (long long)blockIdx.x * C + c0, v);
+}
+
+// The same for groups of 8 to 256 columns that are powers of two: eight columns a thread, a group in neighbouring lanes of a wave, its
+// sum four or five lane exchanges (a workgroup of one wave a group, column by column: 51 -> 26 us at 8100 rows of 8 x 256).
+__global__ __launch_bounds__(NT) void gated_group_norm_lanes_kernel(const float* __restrict__ y, const bf16* __restrict__ gate,
+                                                                    long long ldg, const float* __restrict__ w, int wlen, float eps,
+                                                                    int group, int gate_first, int sigmoid,
+                                                                    bf16* __restrict__ out, int C) {
+  const int c = 8 * (blockIdx.y * NT + threadIdx.x);
+  if (c >= C) return;                                      // (whole groups of lanes)
+  const long long at = (long long)blockIdx.x * C + c;
+  float v[8], g[8], wv[8], sq = 0.f;
+  load8f(y + at, v);
+  load8(gate + (long long)blockIdx.x * ldg + c, g);
+  load8f(w + c % wlen, wv);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    g[i] = sigmoid ? sigmoidf(g[i]) : silu_exact(g[i]);
+    if (gate_first) v[i] *= g[i];
+    sq += v[i] * v[i];
+  }
+  for (int o = 1; o < group >> 3; o <<= 1) sq += __shfl_xor(sq, o, 64);
+  const float r = 1.f / sqrtf(sq / (float)group + eps);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = gate_first ? v[i] * r * wv[i] : v[i] * r * wv[i] * g[i];
+  store8(out + at, v);
 }
 
 constexpr int MAX_TAPS = 16;
@@ -852,6 +940,12 @@ static inline bool wide_rows(int rows, int width) { return rows <= 512 && width 
 void launch_embed_norm(const int* ids, const int* src, const int* prev, const void* table, const float* w, float eps,
                        float offset, float* x, int T_, int d, int f32, hipStream_t s) {
   if (T_ <= 0) return;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x);
+  if (!f32 && T_ > 512 && d % 8 == 0 && d <= 4096 && at % 16 == 0) {      // (fewer rows: the wider workgroups' latency counts)
+    if (d <= 2048) embed_norm_vec_kernel<256><<<T_, 256, 0, s>>>(ids, src, prev, (const bf16*)table, w, eps, offset, x, d);
+    else embed_norm_vec_kernel<512><<<T_, 512, 0, s>>>(ids, src, prev, (const bf16*)table, w, eps, offset, x, d);
+    return;
+  }
   if (wide_rows(T_, d)) {
     DISPATCH_T(f32, (embed_norm_kernel<T, 1024><<<T_, 1024, 0, s>>>(ids, src, prev, (const T*)table, w, eps, offset, x, d));)
   } else {
@@ -886,6 +980,12 @@ void launch_residual_mix_norm(const ResidualMixArgs& a, int f32, hipStream_t s) 
 
 void launch_qkv_rope_cache(const QkvRopeArgs& a, int T_, int f32, hipStream_t s) {
   if (T_ <= 0) return;
+  auto odd = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 != 0; };
+  if (!f32 && T_ > 512 && !a.half && a.dk % 8 == 0 && a.dv % 8 == 0 && (!a.rope || a.pairs % 4 == 0) && a.ldz % 8 == 0 && !odd(a.z) &&
+      !odd(a.bias) && !odd(a.rope) && !odd(a.q_out) && !odd(a.k_cache) && !odd(a.v_cache)) {
+    qkv_rope_cache_vec_kernel<<<T_, QT, 0, s>>>(a);
+    return;
+  }
   if (wide_rows(T_, a.H * a.dk)) {
     DISPATCH_T(f32, (qkv_rope_cache_kernel<T, 1024><<<T_, 1024, 0, s>>>(a));)
   } else {
@@ -906,6 +1006,11 @@ void launch_gated_group_norm(const float* y, const void* gate, long long ldg, co
     else
       gated_group_norm_vec_kernel<512><<<grid, 512, 0, s>>>(y, (const bf16*)gate, ldg, w, wlen, eps, group, gate_first, sigmoid,
                                                             (bf16*)out, C);
+    return;
+  }
+  if (!f32 && T_ > 512 && group >= 8 && group <= 256 && (group & (group - 1)) == 0 && wlen % 8 == 0 && ldg % 8 == 0 && at % 16 == 0) {
+    gated_group_norm_lanes_kernel<<<dim3(T_, (C + 8 * NT - 1) / (8 * NT)), NT, 0, s>>>(y, (const bf16*)gate, ldg, w, wlen, eps, group,
+                                                                                    gate_first, sigmoid, (bf16*)out, C);
     return;
   }
   if (group <= 256) {

@@ -93,3 +93,66 @@ def test_gated_group_norm(T, groups, group, wlen, gate_first, sigmoid):
     n = (n / (n.pow(2).mean(2, keepdim=True) + 1e-5).sqrt()).view(T, C) * w.double().repeat(C // wlen)
     n = n if gate_first else n * g
     assert ((out.double() - n).abs() <= 2.0 ** -8 * n.abs() + 2e-5).all()
+
+
+@pytest.mark.parametrize("T", [513, 512])
+@pytest.mark.parametrize("groups,group,wlen", [(8, 256, 256), (9, 256, 256), (5, 64, 320), (3, 8, 8), (40, 128, 128), (4, 96, 96)])
+@pytest.mark.parametrize("gate_first,sigmoid", [(True, False), (False, True)])
+def test_gated_group_norm_of_small_groups(T, groups, group, wlen, gate_first, sigmoid):
+    """Groups of neighbouring lanes, rows that end inside a workgroup, and a width that keeps the general kernel; bounds as above."""
+    test_gated_group_norm(T, groups, group, wlen, gate_first, sigmoid)
+
+
+@pytest.mark.parametrize("T", [513, 512])
+@pytest.mark.parametrize("d", [8, 264, 2048, 2056, 4096, 4104, 100])
+def test_embed_norm(T, d):
+    """A sum of d squares to 2^-20, the fp32 row to that as well; tokens from ids and from the step before."""
+    print("embed_norm", T, d, flush=True)
+    torch.manual_seed(d)
+    table, w = torch.randn(50, d).to(BF16).cuda(), torch.randn(d).cuda()
+    ids, prev = torch.randint(0, 50, (T,)).int().cuda(), torch.randint(0, 50, (9,)).int().cuda()
+    src = torch.full((T,), -1).int().cuda()
+    src[3], src[T - 1] = 5, 8
+    x = torch.full((T + 1, d), 7.0, device="cuda")
+    ops.embed_norm(ids, table, w, 1e-5, 1.0, x[:T], src, prev)
+    tok = torch.where(src >= 0, prev[src.clamp_min(0).long()], ids).long()
+    t = table[tok].double()
+    want = t / (t.pow(2).mean(1, keepdim=True) + 1e-5).sqrt() * (1.0 + w.double())
+    assert ((x[:T].double() - want).abs() <= 2.0 ** -19 * want.abs() + 1e-30).all() and (x[T] == 7.0).all()
+
+
+@pytest.mark.parametrize("T", [513, 512])
+@pytest.mark.parametrize("H,G,dk,dv,pairs,bias", [(16, 4, 128, 128, 32, True), (3, 1, 24, 40, 12, False), (2, 2, 8, 8, 0, True),
+                                                  (5, 5, 64, 16, 32, True), (4, 2, 20, 16, 4, True), (4, 2, 16, 16, 3, True)])
+def test_qkv_rope_cache(T, H, G, dk, dv, pairs, bias):
+    """Pieces of eight entries: a head rotated in part, whole or not at all, rows without a place in the cache, and sizes that keep the
+    general kernel.  Two products and a sum in fp32 of bf16 values, rounded to bf16."""
+    print("qkv_rope_cache", T, H, G, dk, dv, pairs, flush=True)
+    torch.manual_seed(T + dk)
+    n, BS, NB = (H + G) * dk + G * dv, 16, 40
+    z = torch.randn(T, n + 8).to(BF16).cuda()
+    b = torch.randn(n).cuda() if bias else None
+    pos = torch.randint(0, 200, (T,)).int().cuda()
+    slots = torch.randperm(NB * BS)[:T].int().cuda()
+    slots[2] = -1
+    rope = torch.randn(200, pairs, 2).cuda() if pairs else None
+    q = torch.full((T, H, dk), 7.0, dtype=BF16, device="cuda")
+    k, v = (torch.full((NB, BS, G, e), 7.0, dtype=BF16, device="cuda") for e in (dk, dv))
+    ops.qkv_rope_cache(z[:, 8:], b, H, G, dk, dv, pos, slots, rope, q, k, v)
+    y = z[:, 8:].double() + (b.double() if bias else 0.0)
+    qk, size = y[:, :(H + G) * dk].reshape(T, H + G, dk).clone(), y[:, :(H + G) * dk].reshape(T, H + G, dk).abs()
+    if pairs:
+        c, s = rope[pos.long()].double()[:, None, :, 0], rope[pos.long()].double()[:, None, :, 1]
+        x0, x1 = qk[..., 0:2 * pairs:2].clone(), qk[..., 1:2 * pairs:2].clone()
+        size = size.clone()
+        size[..., 0:2 * pairs:2] = (x0 * c).abs() + (x1 * s).abs()
+        size[..., 1:2 * pairs:2] = (x1 * c).abs() + (x0 * s).abs()
+        qk[..., 0:2 * pairs:2], qk[..., 1:2 * pairs:2] = x0 * c - x1 * s, x1 * c + x0 * s
+    kept = slots >= 0
+    at = slots[kept].long()
+    for got, want, room in ((q, qk[:, :H], size[:, :H]), (k.view(-1, G, dk)[at], qk[kept, H:], size[kept, H:]),
+                            (v.view(-1, G, dv)[at], y[kept, (H + G) * dk:].view(-1, G, dv), y[kept, (H + G) * dk:].view(-1, G, dv).abs())):
+        assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -21 * room).all()
+    rest = torch.ones(NB * BS, dtype=torch.bool, device="cuda")
+    rest[at] = False
+    assert (k.view(-1, G, dk)[rest] == 7.0).all() and (v.view(-1, G, dv)[rest] == 7.0).all()
