@@ -1,6 +1,9 @@
 // Causal softmax attention for prompt rows (bf16): one workgroup per (128 consecutive rows of a sequence's run, query head),
-// grouped key / value heads over the paged token-major cache.  Same arguments as window_attention.hip's kernels for a window
-// that never ends; optional sink, soft cap, per-key score factor and output gate (per head or per column).
+// grouped key / value heads over the paged token-major cache.  Same arguments as window_attention.hip's kernels; optional sink,
+// soft cap, per-key score factor and output gate (per head or per column).  WIN: a window that ends (no cap); the walk starts at
+// the tile of the first row's first key, rows in front of that key are not read.  16 heads on 4 groups of 128, window 1024, us against 64-row
+// tiles staged through registers: 8 runs of 1012 167 -> 58 (1.0 PFLOP/s), one of 200 17.7 -> 10.3, 137 rows behind 1200 64.8 -> 32.5;
+// window 100: 58.8 -> 36.7, 15.4 -> 10.6, 15.1 -> 11.1.
 //
 // Four waves of 32 rows each; keys walk in tiles of 64 up to the last row's own position.  A tile's rows go from the cache to
 // LDS by direct loads, one tile ahead of the products (two stages), in 16-byte chunks whose place within the row is XORed with
@@ -17,11 +20,11 @@
 namespace {
 
 constexpr float MAX_CAP = 60.f;      // e^60 times any number of keys and e^-60 are well inside fp32 and bf16
-constexpr int PW = 4, ROWS = 32 * PW;
+constexpr int PW = 4, ROWS = 32 * PW, NO_WINDOW = 1 << 30;
 
 SYM_DEV f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 
-template <int D, bool CAP, bool KEYV, bool ONE>
+template <int D, bool CAP, bool KEYV, bool ONE, bool WIN>
 __global__ __launch_bounds__(64 * PW, 2) void prompt_attn_kernel(WindowAttnArgs a) {
   constexpr int CH = row_chunks(D), KD = D / 16, VT = (D + 31) / 32, TILE = 64 * CH * 16;   // bytes of a staged tile
   constexpr int NL = CH / PW;                          // direct loads per wave and tile (64 / CH rows each)
@@ -38,6 +41,7 @@ __global__ __launch_bounds__(64 * PW, 2) void prompt_attn_kernel(WindowAttnArgs 
   const bool rv = 32 * wave + j < nrows;
   const int p_first = a.positions[first], p_last = p_first + nrows - 1;
   const int wq_lo = p_first + 32 * wave, wq_hi = wq_lo + 31, qp = wq_lo + j;
+  const int k_lo = WIN ? max(0, p_first - a.window + 1) : 0, kt0 = k_lo & ~63;
   const int* bt = a.block_tables + (long long)a.row_seq[first] * a.max_blocks;
   const bf16* kc = reinterpret_cast<const bf16*>(a.k_cache) + g * D;
   const bf16* vc = reinterpret_cast<const bf16*>(a.v_cache) + g * D;
@@ -59,7 +63,7 @@ __global__ __launch_bounds__(64 * PW, 2) void prompt_attn_kernel(WindowAttnArgs 
   const int uw = __builtin_amdgcn_readfirstlane(wave);
   int blk = 0;
   auto row_of = [&](int kp) {
-    kp = min(kp, p_last);
+    kp = min(WIN ? max(kp, k_lo) : kp, p_last);
     return ONE ? ((long long)blk << a.bs_shift) + (kp & (a.BS - 1)) : cache_row(bt, kp, a.BS, a.bs_shift);
   };
   auto stage = [&](int kt, int buf) {
@@ -100,11 +104,11 @@ __global__ __launch_bounds__(64 * PW, 2) void prompt_attn_kernel(WindowAttnArgs 
   const float c1 = CAP ? 2.f * sl2 / a.softcap : 0.f, c2 = CAP ? a.softcap * ATT_LOG2E : 0.f;
   const bool scaled = a.key_scale != nullptr;
 
-  if (ONE) blk = bt[0];
-  stage(0, 0);
-  if (ONE && 64 <= p_last) blk = bt[64 >> a.bs_shift];
+  if (ONE) blk = bt[kt0 >> a.bs_shift];
+  stage(kt0, 0);
+  if (ONE && kt0 + 64 <= p_last) blk = bt[(kt0 + 64) >> a.bs_shift];
   int buf = 0;
-  for (int kt = 0; kt <= p_last; kt += 64, buf ^= 1) {
+  for (int kt = kt0; kt <= p_last; kt += 64, buf ^= 1) {
     wait_direct_loads();
     __syncthreads();                                   // the tile has landed; every wave is done with the other stage
     if (kt + 64 <= p_last) {
@@ -112,6 +116,7 @@ __global__ __launch_bounds__(64 * PW, 2) void prompt_attn_kernel(WindowAttnArgs 
       if (ONE && kt + 128 <= p_last) blk = bt[(kt + 128) >> a.bs_shift];
     }
     if (kt > wq_hi || 32 * wave >= nrows) continue;    // (wave-uniform) nothing of this tile is visible here
+    if (WIN && kt + 63 <= wq_lo - a.window) continue;
     const char* S = smem + buf * STAGE;
     float p[2][16];
     {
@@ -144,7 +149,14 @@ __global__ __launch_bounds__(64 * PW, 2) void prompt_attn_kernel(WindowAttnArgs 
         }
     }
     const bool edge = kt + 63 > wq_lo;                 // (wave-uniform) some row does not see the whole tile
-    const int vis = qp - kt - 4 * hi;                  // key offsets <= vis are visible
+    const int vis = qp - kt - 4 * hi;                  // key offsets <= vis are visible, those > vis - window
+    if (WIN && kt <= wq_hi - a.window) {               // (wave-uniform) some row's window starts inside the tile or behind it
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (32 * b + 8 * (e / 4) + e % 4 <= vis - a.window) p[b][e] = -INFINITY;
+    }
     if constexpr (CAP) {
 #pragma unroll
       for (int b = 0; b < 2; ++b)
@@ -253,22 +265,23 @@ __global__ __launch_bounds__(64 * PW, 2) void prompt_attn_kernel(WindowAttnArgs 
     }
 }
 
-template <int D, bool CAP, bool KEYV, bool ONE>
+template <int D, bool CAP, bool KEYV, bool ONE, bool WIN = false>
 void launch(const WindowAttnArgs& a, hipStream_t s) {
   constexpr int lds = 2 * ((KEYV ? 1 : 2) * 64 * row_chunks(D) * 16 + 256);
   static bool once = false;
   if (lds > 64 * 1024 && !once) {
-    hipFuncSetAttribute(reinterpret_cast<const void*>(&prompt_attn_kernel<D, CAP, KEYV, ONE>),
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&prompt_attn_kernel<D, CAP, KEYV, ONE, WIN>),
                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     once = true;
   }
-  prompt_attn_kernel<D, CAP, KEYV, ONE><<<dim3(a.H, a.ntiles), 64 * PW, lds, s>>>(a);
+  prompt_attn_kernel<D, CAP, KEYV, ONE, WIN><<<dim3(a.H, a.ntiles), 64 * PW, lds, s>>>(a);
 }
 
 template <int D>
 void launch_d(const WindowAttnArgs& a, hipStream_t s) {
   const bool one = a.bs_shift >= 6;      // cache blocks of 64 tokens or a larger power of two
-  if (a.softcap > 0.f) one ? launch<D, true, false, true>(a, s) : launch<D, true, false, false>(a, s);
+  if (a.window < NO_WINDOW) one ? launch<D, false, false, true, true>(a, s) : launch<D, false, false, false, true>(a, s);
+  else if (a.softcap > 0.f) one ? launch<D, true, false, true>(a, s) : launch<D, true, false, false>(a, s);
   else if (a.k_cache == a.v_cache) one ? launch<D, false, true, true>(a, s) : launch<D, false, true, false>(a, s);
   else one ? launch<D, false, false, true>(a, s) : launch<D, false, false, false>(a, s);
 }
@@ -277,7 +290,8 @@ void launch_d(const WindowAttnArgs& a, hipStream_t s) {
 
 bool launch_prompt_attn(const WindowAttnArgs& a, hipStream_t s) {
   const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (!a.tiles || !a.cu_q || a.ntiles <= 0 || a.ntiles > 65535 || a.dk != a.dv || a.bias || a.window < (1 << 30) ||
+  if (!a.tiles || !a.cu_q || a.ntiles <= 0 || a.ntiles > 65535 || a.dk != a.dv || a.bias ||
+      (a.window < NO_WINDOW && (a.keep_first > 0 || a.softcap > 0.f || a.k_cache == a.v_cache)) ||
       !(a.scale > 0.f) || a.softcap > MAX_CAP || !al(a.q) || !al(a.k_cache) || !al(a.v_cache) || !al(a.out))
     return false;
   switch (a.dk) {

@@ -544,7 +544,7 @@ int launch_window_attn(const WindowAttnArgs& args, int f32, int impl, hipStream_
   for (int b = 0; b < 31; ++b)
     if (a.BS == 1 << b) a.bs_shift = b;
   if (impl >= 1 && impl != 3 && !f32) {
-    if (launch_prompt_attn(a, s)) return 2;
+    if (launch_prompt_attn(a, s)) return a.window < (1 << 30) ? 1 : 2;      // (1: tiles of a window, whichever kernel)
     if (!a.tiles && launch_split_attn(a, s)) return 3;
   }
   const bool plain = !a.gate_cols && !a.key_scale && a.softcap <= 0.f;   // (what the tiled kernel has no code for)

@@ -97,3 +97,54 @@ def _check(H, G, D, T, window, keep, off, ranges=False):
         want, room = torch.einsum("grc,cgd->grd", p, vs), torch.einsum("grc,cgd->grd", p, vs.abs())
         err = (out[i].double().view(G, H // G, D) - want).abs()
         assert bool((err <= 2.0 ** -13 * room + 2.0 ** -8 * (want.abs() + 2.0 ** -13 * room)).all()), (i, pos[i], float(err.max()))
+
+
+@pytest.mark.parametrize("H,G,D,block", [(4, 2, 128, 64), (3, 3, 64, 16), (4, 1, 32, 48), (2, 1, 80, 128)])
+@pytest.mark.parametrize("window", [1, 31, 64, 65, 129, 300])
+def test_window_prompts(gpu, H, G, D, block, window):
+    """Prompt runs behind a window that ends: runs that start and end anywhere in a tile of 64 keys and in one of 128 rows, with and
+    without cached rows, blocks that hold a tile and others.  Rows in front of a run's first window are not finite.  The weights are
+    rounded to bf16 for their product: 2^-8 of the sum of p |v|, their scores' 2^-13 beside it, and the result's own rounding."""
+    print("window prompts", H, G, D, block, window, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(D + window)
+    runs = [(0, 1), (0, 200), (37, 130), (64, 64), (300, 65), (511, 3), (190, 129)]         # (cached, new)
+    need = [-(-(c + n) // block) for c, n in runs]
+    order = torch.randperm(sum(need), generator=torch.Generator().manual_seed(D)).add_(1).tolist()
+    bt = torch.zeros(len(runs), max(need), dtype=torch.int32)
+    k = torch.full((sum(need) + 1, block, G, D), math.nan, device="cuda", dtype=torch.bfloat16)
+    v = torch.full_like(k, math.nan)
+    at, places = 0, []
+    for i, (c, n) in enumerate(runs):
+        bt[i, :need[i]] = torch.tensor(order[at:at + need[i]])
+        at += need[i]
+        j = torch.arange(max(0, c - window + 1), c + n)
+        b, o = bt[i][j // block].long().cuda(), (j % block).cuda()
+        k[b, o] = torch.randn(len(j), G, D, device="cuda", generator=g).bfloat16()
+        v[b, o] = torch.randn(len(j), G, D, device="cuda", generator=g).bfloat16()
+        places.append((j.cuda(), b, o))
+    T, i32 = sum(n for _, n in runs), dict(device="cuda", dtype=torch.int32)
+    q = torch.randn(T, H, D, device="cuda", generator=g).bfloat16()
+    gate = torch.randn(T, H, device="cuda", generator=g).bfloat16()
+    sink = torch.randn(H, device="cuda", generator=g)
+    out = torch.full((T + 1, H, D), 7.0, device="cuda", dtype=torch.bfloat16)
+    pos = torch.cat([torch.arange(c, c + n) for c, n in runs])
+    rs = torch.repeat_interleave(torch.arange(len(runs)), torch.tensor([n for _, n in runs]))
+    cu = [0]
+    for _, n in runs:
+        cu.append(cu[-1] + n)
+    tiles = [(i, r) for i, (_, n) in enumerate(runs) for r in range(0, n, 64)]
+    used = ops.window_attn(q, k, v, bt.cuda(), rs.to(**i32), pos.to(**i32), window, D ** -0.5, gate, out[:-1], torch.tensor(tiles, **i32),
+                           torch.tensor(cu, **i32), sink=sink)
+    assert used == 1 and bool((out[-1] == 7.0).all())
+    for i, (c, n) in enumerate(runs):
+        j, b, o = places[i]
+        p = torch.arange(c, c + n, device="cuda")[:, None]
+        hidden = (j[None] > p) | (j[None] <= p - window)
+        qs = q[cu[i]:cu[i + 1]].double().view(n, G, H // G, D)
+        s = torch.einsum("ngrd,cgd->ngrc", qs, k[b, o].double()).mul_(D ** -0.5).masked_fill_(hidden[:, None, None], -math.inf)
+        s = torch.cat([s, sink.double().view(1, G, H // G, 1).expand(n, -1, -1, 1)], -1).softmax(-1)[..., :-1]
+        f = gate[cu[i]:cu[i + 1]].double().sigmoid().view(n, G, H // G, 1)
+        want = torch.einsum("ngrc,cgd->ngrd", s, v[b, o].double()) * f
+        room = torch.einsum("ngrc,cgd->ngrd", s, v[b, o].double().abs()) * f
+        err = (out[cu[i]:cu[i + 1]].double().view(n, G, H // G, D) - want).abs()
+        assert bool((err <= (2.0 ** -8 + 2.0 ** -12) * room + 2.0 ** -8 * want.abs() + 1e-30).all()), (i, float(err.max()))
