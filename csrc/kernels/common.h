@@ -70,6 +70,15 @@ SYM_DEV void load8(const bf16* p, float* f) {
 // Non-temporal 16-byte load (streamed-once weights: MI355X_MICROARCH.md row nt-weights).
 SYM_DEV u32x4 ld_nt16(const bf16* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
 
+// A lane's registers from the lane 8 further in its row of 16, in the banks of MASK only (0x3: lanes 0-7, 0xc: 8-15).
+template <int MASK>
+SYM_DEV u32x4 half_swap(u32x4 keep, u32x4 from) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = __builtin_amdgcn_update_dpp(keep[i], from[i], 0x128 /* row_ror:8 */, 0xf, MASK, false);
+  return r;
+}
+
 SYM_DEV void store8(bf16* p, const float* f) {
   Pack8 pk;
 #pragma unroll

@@ -203,7 +203,7 @@ struct ExpertArgs {
 };
 // the MFMA forms take it (the only ones with glu and f32_out)
 bool expert_linear_mfma(const ExpertArgs& a, int f32);
-// impl -1: by shape; 0 all shapes, 1 weight stream, 2 / 3 tiles.  Returns the form used.
+// impl -1: by shape; 0 all shapes, 1 weight stream, 2 / 3 tiles, 4 weight walk.  Returns the form used.
 int launch_expert_linear(const ExpertArgs& a, int f32, int impl, hipStream_t s);
 
 // ---- window_attention.hip ------------------------------------------------------------------------------

@@ -8,8 +8,8 @@
 // Router in bf16: 16 tokens x 16 experts per MFMA, the waves of a workgroup split the width and meet in LDS (the products of
 // bf16 values and their sums are exact to fp32 accumulation).  A step of at most 16 tokens is one workgroup, which then also
 // lays out the segments; larger steps take one more launch.
-// Expert products in bf16: a weight-streaming kernel for few rows per expert (a wave per 16 weight rows and width slice, the
-// rows of the segment as the other MFMA operand), and for prompt steps a 128 x 128 tile kernel and a persistent one of 256 x 256,
+// Expert products in bf16: weight-streaming kernels for few rows per expert (a wave per 16 weight rows and width slice, the
+// rows of the segment as the other MFMA operand; persistent where there are many weights), and for prompt steps a 128 x 128 tile kernel and a persistent one of 256 x 256,
 // staged through LDS by direct loads.  Other shapes and fp32: the all-shapes segment product of glu_moe.hip.
 #include "common.h"
 #include "direct_lds.h"
@@ -352,6 +352,134 @@ SYM_DEV void store_quad(void* y, long long at, f32x4 f, int n, int N, bool vec) 
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         if (n + u < N) o[u] = v[u];
+    }
+  }
+}
+
+// Few rows per expert, many weights: a workgroup per CU walks units of OUT outputs (EPI_GLU: 8, their gate and up rows, else 16) of
+// up to 16 rows of one expert: unit t, t + gridDim.x, ..  A wave holds its share of a unit's weights and rows in registers (KB
+// steps of 64 elements, K = 64 NW KB); the next unit's are loaded while a unit is multiplied, so the weights stream without a
+// gap from one expert to the next.  The waves sum a unit's parts in turn, one barrier a unit (two buffers).  A lane knows the
+// segment of expert `lane` and the units up to its end; the rows' places are kept in LDS.  E <= 64, R <= WALK_ROWS.  Bound by HBM:
+// the weights of 15 of 16 experts, gated 2 x 1536 x 2048, 32 rows, 189 MB 38.7 -> 32.7 us (5.8 TB/s), 62 of 64 679 MB 123.8 ->
+// 104.6 (6.5 TB/s).
+constexpr int WALK_ROWS = 512;
+
+template <int NW, int KB, int EPI>
+__global__ __launch_bounds__(64 * NW) void expert_walk_kernel(ExpertArgs a) {
+  constexpr int OUT = EPI == EPI_GLU ? 8 : 16;
+  __shared__ f32x4 red[2][NW][64];
+  __shared__ int rows[WALK_ROWS];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 15, hq = lane >> 4;
+  const int K = 64 * NW * KB, N = a.N, tiles = (N + OUT - 1) / OUT, step = gridDim.x;
+  const int begin = lane < a.E ? a.offsets[lane] : 0;
+  const int count = lane < a.E ? max(0, min(a.offsets[lane + 1], a.R) - begin) : 0;
+  int place = 0;
+  if (threadIdx.x < a.R) place = a.src ? a.src[threadIdx.x] : threadIdx.x;
+  const int units = (count + 15) / 16 * tiles;
+  int end = units;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(end, o, 64);
+    if (lane >= o) end += v;
+  }
+  const int first = end - units, total = __builtin_amdgcn_readlane(end, 63);
+  if ((int)blockIdx.x >= total) return;
+
+  struct Unit {
+    int e, r0, r1, n0;
+    bool in;
+  };
+  // (past the last unit: one line for all lanes, so that a unit's wait never stands behind a branch)
+  auto unit = [&](int t) {
+    Unit u;
+    u.in = t < total;
+    if (!u.in) t = 0;
+    u.e = __popcll(__ballot(end <= t));
+    int rem = t - __builtin_amdgcn_readlane(first, u.e);
+    u.r0 = __builtin_amdgcn_readlane(begin, u.e);
+    u.r1 = u.r0 + __builtin_amdgcn_readlane(count, u.e);
+    while (rem >= tiles) {
+      rem -= tiles;
+      u.r0 += 16;
+    }
+    u.n0 = rem * OUT;
+    return u;
+  };
+  const unsigned kin = (unsigned)(4 * (j & 8) + 8 * hq) * 2;
+  const char* Wb = reinterpret_cast<const char*>(a.W) + 128 * KB * wave;
+  const char* xb = reinterpret_cast<const char*>(a.x) + 128 * KB * wave + 16 * hq;
+  u32x4 w[2][KB][2];
+  Pack8 xv[2][KB][2];
+  auto load_w = [&](int b, const Unit& t) {
+    const char* base = Wb + ((long long)t.e * (EPI == EPI_GLU ? 2 : 1) * N + t.n0) * K * 2;
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+      const int row = min((EPI == EPI_GLU ? 0 : 8 * l) + (j & 7), N - 1 - t.n0);
+      const unsigned off = t.in ? (unsigned)(row * K) * 2 + kin : 0;
+      const char* from = base + (EPI == EPI_GLU && l ? (long long)N * K * 2 : 0);
+#pragma unroll
+      for (int u = 0; u < KB; ++u) w[b][u][l] = ld_nt16(reinterpret_cast<const bf16*>(from + 128 * u + off));
+    }
+  };
+  auto load_x = [&](int b, const Unit& t) {
+    const char* from = xb + (long long)rows[min(t.r0 + j, t.r1 - 1)] * K * 2;
+#pragma unroll
+    for (int u = 0; u < KB; ++u)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) xv[b][u][k].w = *reinterpret_cast<const u32x4*>(from + 128 * u + 64 * k);
+  };
+  auto multiply = [&](int b, const Unit& t, int turn) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < KB; ++u) {
+      Pack8 f0, f1;
+      f0.w = half_swap<0xc>(w[b][u][0], w[b][u][1]);
+      f1.w = half_swap<0x3>(w[b][u][1], w[b][u][0]);
+      acc = mfma16(f0.v, xv[b][u][0].v, acc);
+      acc = mfma16(f1.v, xv[b][u][1].v, acc);      // lane: row j, outputs n0 + 4 hq + 0..3
+    }
+    red[b][wave][lane] = acc;
+    __builtin_amdgcn_s_waitcnt(0xc07f);      // lgkmcnt(0): the next unit's loads stay in flight
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (wave != turn) return;
+    f32x4 v = red[b][0][lane];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) v += red[b][i][lane];
+    if constexpr (EPI == EPI_GLU) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = silu(v[r]) * __shfl_down(v[r], 32, 64);
+      if (hq >= 2) return;
+    }
+    if constexpr (EPI == EPI_RELU2)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = relu2f(v[r]);
+    const int n = t.n0 + 4 * hq;
+    if (t.r0 + j < t.r1) store_quad<EPI == EPI_F32>(a.y, (long long)(t.r0 + j) * N + n, v, n, N, N % 4 == 0);
+  };
+
+  Unit cur = unit(blockIdx.x);
+  load_w(0, cur);
+  if (threadIdx.x < a.R) rows[threadIdx.x] = place;
+  for (int i = threadIdx.x + 64 * NW; i < a.R; i += 64 * NW) rows[i] = a.src ? a.src[i] : i;
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  load_x(0, cur);
+  int t = blockIdx.x, turn = 0;
+  while (true) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      if (!cur.in) return;
+      t += step;
+      const Unit next = unit(t);
+      load_w(b ^ 1, next);
+      load_x(b ^ 1, next);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(b, cur, turn);
+      cur = next;
+      turn = turn + 1 == NW ? 0 : turn + 1;
     }
   }
 }
@@ -769,11 +897,27 @@ void launch_route_topk(const RouteArgs& a, int f32, hipStream_t s) {
                                                                                                    a.offsets, a.dst, a.src);
 }
 
+template <int NW, int KB>
+bool launch_walk(const ExpertArgs& a, hipStream_t s) {
+  if (a.K != 64 * NW * KB) return false;
+  const int tiles = a.glu ? (a.N + 7) / 8 : (a.N + 15) / 16;
+  const long long most = (long long)tiles * std::min(a.R, a.E + a.R / 16);      // (units, at most)
+  // (two small workgroups share a CU: 2048 x 512 of 64 experts, 32 rows, 19.7 -> 11.5 us; at 1536 wide one of 12 waves, 17.8 us
+  // where one of 8 takes 18.3 and two 19.5)
+  const int grid = (int)std::min<long long>(most, (NW == 8 ? 2 : 1) * cu_count());
+  if (a.glu) expert_walk_kernel<NW, KB, EPI_GLU><<<grid, 64 * NW, 0, s>>>(a);
+  else if (a.relu2) expert_walk_kernel<NW, KB, EPI_RELU2><<<grid, 64 * NW, 0, s>>>(a);
+  else if (a.f32_out) expert_walk_kernel<NW, KB, EPI_F32><<<grid, 64 * NW, 0, s>>>(a);
+  else expert_walk_kernel<NW, KB, EPI_BF16><<<grid, 64 * NW, 0, s>>>(a);
+  return true;
+}
+
 bool expert_linear_mfma(const ExpertArgs& a, int f32) {
   return !f32 && a.K % 32 == 0 && aligned16(a.x) && aligned16(a.W) && aligned16(a.y);
 }
 
-// Returns the form used: 0 all shapes, 1 weight stream, 2 / 3 tiles of 128 / 256
+// Returns the form used: 0 all shapes, 1 weight stream, 2 / 3 tiles of 128 / 256, 4 the walk (widths 512, 1536, 2048, 3072; else
+// the weight stream)
 // Stream or tile, measured at 16 experts, 4 rows each on average: [gate | up] of 1536 x 2048 46.0 us on both, 2048 x 1536 23.9
 // against 28.8; at 16 rows each 53 against 46.6 and 33 against 28.7.
 // Persistent tiles against those of 128, us: 16 experts, gated 1536 x 2048 and 2048 x 1536, at 96 rows each 43.9 -> 46.0 and 29.0 ->
@@ -794,7 +938,19 @@ int launch_expert_linear(const ExpertArgs& a, int f32, int impl, hipStream_t s) 
     const long long tiles = (long long)((a.N + 255) / 256) * (a.glu ? 2 : 1) * (a.R / 256), cus = cu_count();
     const bool rounds = !a.glu || 10 * tiles <= 7 * cus || tiles >= cus;
     const bool big = fits && a.N >= 256 && (a.K >= 1024 ? per >= 128 && rounds : per >= 1024 && a.N >= 1024);
-    impl = stream && (per <= 8 || !tile) ? 1 : (tile ? (big ? 3 : 2) : (stream ? 1 : 0));
+    // The walk over many weights against a workgroup per 16 outputs, us: gated, 16 experts of 1536 x 2048, 4 / 16 / 32 / 128 rows 19.4 ->
+    // 12.5, 32.8 -> 26.1, 42.4 -> 39.3 (and 256 rows, where blocks of 16 read weights twice, 50.2 -> 62.9); 512 x 2048, 64 experts
+    // 32 rows 29.5 -> 24.7; 512 x 3072, 32 experts 38.3 -> 26.4; to fp32, 32 rows, 2048 x 1536 21.7 -> 17.7, 2048 x 2048 24.3 ->
+    // 20.2, 2048 x 512 of 64 experts 16.0 -> 11.5; few units do not fill it: 512 x 1536, 16 rows of 8 experts 5.0 -> 5.9, 1024 x
+    // 2048 11.7 -> 12.1, gated 1536 x 512 7.2 -> 8.0.
+    const bool walk = a.glu ? a.K >= 1536 : a.N >= 1536;
+    impl = stream && (per <= 8 || !tile) ? (per <= 8 && walk ? 4 : 1) : (tile ? (big ? 3 : 2) : (stream ? 1 : 0));
+  }
+  if (impl == 4) {
+    if (mfma && a.E <= 64 && a.R <= WALK_ROWS &&
+        (launch_walk<8, 1>(a, s) || launch_walk<12, 2>(a, s) || launch_walk<16, 2>(a, s) || launch_walk<16, 3>(a, s)))
+      return 4;
+    impl = 1;
   }
   if (impl == 1 && stream) {
     const int deep = a.K / 512;               // 64-element steps of each of 8 waves

@@ -53,15 +53,6 @@ SYM_DEV void store_rows(const Args& a, int n0, int lane, f32x4 v, f32x4 u) {
   }
 }
 
-// A lane's registers from the lane 8 further in its row of 16, in the banks of MASK only (0x3: lanes 0-7, 0xc: 8-15).
-template <int MASK>
-SYM_DEV u32x4 half_swap(u32x4 keep, u32x4 from) {
-  u32x4 r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) r[i] = __builtin_amdgcn_update_dpp(keep[i], from[i], 0x128 /* row_ror:8 */, 0xf, MASK, false);
-  return r;
-}
-
 // RT: weight tiles of a workgroup.  RH: weight rows of a tile, 16 or 8.  U: 64-deep k blocks of a chunk.  Every wave has
 // the same number of whole chunks.
 //

@@ -177,3 +177,47 @@ def test_persistent_tiles(E, R, N, K):
     assert ((z[:R].double() - want).abs() <= 2.0 ** -8 * want + 2 * g.abs() * eps + eps ** 2).all()
     assert H.expert_linear(x, src, half, od, z[:R], False, 3) == 3
     assert ((z[:R].double() - g).abs() <= 2.0 ** -8 * g.abs() + 2 * eps).all()
+
+
+@pytest.mark.parametrize("shape", [(1, 8, 512), (4, 132, 512), (7, 200, 1536), (5, 262, 2048), (64, 40, 2048), (16, 1536, 3072)])
+@pytest.mark.parametrize("R", [1, 16, 17, 64, 130, 512])
+def test_walk_over_the_experts(R, shape):
+    """The persistent form: empty experts, more than 16 rows of one, outputs that fill no unit, fewer units than workgroups and many
+    of each.  Bounds as above; the squared ReLU doubles the error times the value."""
+    E, N, K = shape
+    print("expert walk", R, shape, flush=True)
+    torch.manual_seed(R + N)
+    off = torch.tensor([0] + sorted(torch.randint(0, R + 1, (E - 1,)).tolist()) + [R]).int()
+    x, W = torch.randn(R // 2 + 1, K).to(BF16), (torch.randn(E, 2 * N, K) * K ** -0.5).to(BF16)
+    src = torch.randint(0, x.shape[0], (R,)).int()
+    p = torch.zeros(R, 2 * N, dtype=torch.float64)
+    for e in range(E):
+        a, b = int(off[e]), int(off[e + 1])
+        p[a:b] = x[src[a:b].long()].double() @ W[e].double().t()
+    g, u = p[:, :N], p[:, N:]
+    eps = 4 * K ** 0.5 * 2.0 ** -24 * x.double().norm(dim=1).max() * W.double().norm(dim=2).max()
+    H = ops._hyb()
+    xd, sd, Wd, od = x.cuda(), src.cuda(), W.cuda(), off.cuda()
+    gate = Wd[:, :N].contiguous()
+    y = torch.full((R + 1, N), 7.0, device="cuda")
+    assert H.expert_linear(xd, sd, gate, od, y[:R], False, 4) == 4
+    assert ((y[:R].cpu().double() - g).abs() <= eps).all() and (y[R] == 7.0).all()
+    z = torch.full((R + 1, N), 7.0, dtype=BF16, device="cuda")
+    assert H.expert_linear(xd, sd, Wd, od, z[:R], False, 4, True) == 4
+    want = g / (1 + torch.exp(-g)) * u
+    bound = 2.0 ** -8 * want.abs() + 1.1 * eps * (g.abs() + u.abs()) + 2.0 ** -20 * want.abs() + 1e-30
+    assert ((z[:R].cpu().double() - want).abs() <= bound).all() and (z[R] == 7.0).all()
+    assert H.expert_linear(xd[sd.long()], None, gate, od, z[:R], True, 4) == 4
+    want = g.clamp(min=0) ** 2
+    assert ((z[:R].cpu().double() - want).abs() <= 2.0 ** -8 * want + 2 * eps * g.abs() + eps ** 2).all() and (z[R] == 7.0).all()
+    H.expert_linear(xd[sd.long()], None, gate, od, z[:R], False, 4)
+    assert ((z[:R].cpu().double() - g).abs() <= 2.0 ** -8 * g.abs() + eps).all() and (z[R] == 7.0).all()
+
+
+@pytest.mark.parametrize("R,N,K,glu,form", [(32, 1536, 2048, True, 4), (32, 2048, 1536, False, 4), (512, 512, 1536, True, 4),
+                                            (32, 1024, 2048, False, 1), (32, 1536, 512, True, 1), (32, 1536, 1024, False, 1)])
+def test_who_walks(R, N, K, glu, form):
+    x, W = torch.randn(R, K).to(BF16).cuda(), torch.randn(64, N * (2 if glu else 1), K).to(BF16).cuda()
+    off = torch.arange(65).mul(R).div(64, rounding_mode="floor").int().cuda()
+    y = torch.empty(R, N, dtype=BF16, device="cuda")
+    assert ops._hyb().expert_linear(x, None, W, off, y, False, -1, glu) == form
