@@ -701,7 +701,7 @@ void qk_row_norm_cache(const Tensor& z, const OptTensor& bias, int64_t H, int64_
 }
 
 void route_topk(const Tensor& x, const Tensor& Wr, const OptTensor& bias, int64_t k, Tensor& ids, Tensor& w, Tensor& offsets,
-                Tensor& dst, Tensor& src, bool runs) {
+                Tensor& dst, Tensor& src, bool runs, const OptTensor& resid, const OptTensor& norm, double eps) {
   const int f32 = act(x, "x");
   same_act(Wr, f32, "Wr");
   dtype(w, at::kFloat, "w");
@@ -721,6 +721,14 @@ void route_topk(const Tensor& x, const Tensor& Wr, const OptTensor& bias, int64_
   a.ids = ptr<int>(ids), a.w = ptr<float>(w), a.offsets = ptr<int>(offsets), a.dst = ptr<int>(dst), a.src = ptr<int>(src);
   a.runs = runs;
   TORCH_CHECK(!runs || (route_topk_runs(a, f32) && !a.bias), "route_topk: runs: bf16, at most 16 experts, d % 128 == 0, no bias");
+  if (resid.has_value()) {
+    TORCH_CHECK(norm.has_value() && !f32, "route_topk: resid goes with norm and a bf16 x");
+    dtype(*resid, at::kFloat, "resid");
+    dtype(*norm, at::kBFloat16, "norm");
+    TORCH_CHECK(resid->sizes() == x.sizes() && norm->numel() == x.size(1), "route_topk: resid [T, d], norm [d]");
+    a.resid = ptr<float>(*resid), a.norm = norm->data_ptr(), a.eps = (float)eps;
+    TORCH_CHECK(route_norm_fits(a), "route_topk: resid: at most 16 rows and 64 experts, d % 512 == 0, d <= 2048, 16-byte addresses");
+  }
   const at::OptionalDeviceGuard g(x.device());
   launch_route_topk(a, f32, cur_stream(x));
 }
@@ -1231,8 +1239,8 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
       "Tensor positions, Tensor slots, Tensor(a!) q_out, Tensor(b!) kv_cache, Tensor(c!) key_scale) -> ()",
       &qk_row_norm_cache);
   m.def(
-      "route_topk(Tensor x, Tensor Wr, Tensor? bias, int k, Tensor(a!) ids, Tensor(b!) w, Tensor(c!) offsets, Tensor(d!) dst, "
-      "Tensor(e!) src, bool runs=False) -> ()",
+      "route_topk(Tensor(f!) x, Tensor Wr, Tensor? bias, int k, Tensor(a!) ids, Tensor(b!) w, Tensor(c!) offsets, Tensor(d!) dst, "
+      "Tensor(e!) src, bool runs=False, Tensor? resid=None, Tensor? norm=None, float eps=0.0) -> ()",
       &route_topk);
   m.def(
       "expert_linear(Tensor x, Tensor? src, Tensor W, Tensor offsets, Tensor(a!) y, bool relu2, int impl=-1, bool glu=False) -> int",

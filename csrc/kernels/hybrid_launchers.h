@@ -186,7 +186,11 @@ struct RouteArgs {
   int* dst;
   int* src;
   int runs;             // the sums and weights of moe_router + moe_route (where route_topk_runs)
+  const float* resid;   // [T][d] or null: x is written first, RMSNorm(resid) (where route_norm_fits)
+  const void* norm;     // [d] bf16
+  float eps;
 };
+bool route_norm_fits(const RouteArgs& a);
 bool route_topk_runs(const RouteArgs& a, int f32);
 void launch_route_topk(const RouteArgs& a, int f32, hipStream_t s);
 // y[i] = W[e] x[src ? src[i] : i] (relu2: relu(.)^2) for the places i of expert e's segment, W [E][N][K], y [R][N]

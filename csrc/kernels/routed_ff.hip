@@ -113,9 +113,13 @@ __global__ __launch_bounds__(PLAN_NT) void expert_layout_kernel(const int* __res
 // logits) or, reused, 16 E floats + the layout's counters; PLAN: the single workgroup lays out the segments as well.
 // a.runs: every wave takes one run of the width (d % (32 NW) == 0), and the hardware exponential: the sums and weights of
 // moe_router_kernel and moe_route_kernel, to the bit.
-template <int NW, int NE, bool PLAN>
+// NORM (PLAN; d % 512 == 0, d <= 2048): x = RMSNorm(resid) is made here, a wave a row, and written to x for the experts; it meets
+// the router in LDS, behind the partial logits (rows 16 B longer, so a fragment's 16 rows lie in different banks).
+// Latency is all of it: 8 rows of 2048, 16 experts 8.6 -> 6.8 us with the norm's launch.  A token's choices are counted places of
+// its logits: the k reductions over the wave that stood here were a chain of 12 lane exchanges each (4 of 16, alone 8.7 -> 6.5).
+template <int NW, int NE, bool PLAN, bool NORM = false>
 __global__ __launch_bounds__(64 * NW) void route_mfma_kernel(RouteArgs a) {
-  extern __shared__ float part[];
+  extern __shared__ __attribute__((aligned(16))) float part[];
   __shared__ int chosen[PLAN ? 1024 : 1];      // PLAN: the workgroup's choices (at most 16 tokens x 64)
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, hq = lane >> 4;
   const int t0 = 16 * blockIdx.x, d = a.d, E = a.E;
@@ -128,6 +132,56 @@ __global__ __launch_bounds__(64 * NW) void route_mfma_kernel(RouteArgs a) {
     acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const int first = a.runs ? wave * (d / NW) : 32 * wave, last = a.runs ? first + d / NW : d, step = a.runs ? 32 : 32 * NW;
+  constexpr int AHEAD = NORM && NW == 16 ? 4 : 0;      // (all of a wave's steps)
+  Pack8 ahead[NE][AHEAD + 1];
+  if constexpr (NORM) {
+    bf16* rows = reinterpret_cast<bf16*>(part + NW * NE * 256);
+    const int pitch = d + 8;
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+      for (int n = 0; n < NE; ++n)
+        ahead[n][i].u = *reinterpret_cast<const uint4*>(w[n] + min(first + i * step, last - 32));
+    for (int t = wave; t < a.T; t += NW) {
+      const float* from = a.resid + (long long)t * d + 8 * lane;
+      float v[4][8], ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (512 * i < d) load8f(from + 512 * i, v[i]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (512 * i < d)
+#pragma unroll
+          for (int u = 0; u < 8; ++u) ss += v[i][u] * v[i][u];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+      const float inv = rsqrtf(ss / (float)d + a.eps);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (512 * i < d) {
+          float g[8];
+          load8(reinterpret_cast<const bf16*>(a.norm) + 512 * i + 8 * lane, g);
+          Pack8 o;
+#pragma unroll
+          for (int u = 0; u < 8; ++u) o.v[u] = (bf16)(g[u] * (v[i][u] * inv));
+          *reinterpret_cast<uint4*>(rows + t * pitch + 512 * i + 8 * lane) = o.u;
+          *reinterpret_cast<uint4*>(const_cast<bf16*>(reinterpret_cast<const bf16*>(a.x)) + (long long)t * d + 512 * i + 8 * lane) = o.u;
+        }
+    }
+    __syncthreads();
+    x = rows + min(j, a.T - 1) * pitch + 8 * hq;
+  }
+  if constexpr (AHEAD > 0) {
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const int c = first + i * step;
+      if (c >= last) break;
+      Pack8 xf;
+      xf.u = *reinterpret_cast<const uint4*>(x + c);
+#pragma unroll
+      for (int n = 0; n < NE; ++n) acc[n] = mfma16(ahead[n][i].v, xf.v, acc[n]);
+    }
+  } else
 #pragma unroll 4
   for (int c = first; c < last; c += step) {
     Pack8 xf;
@@ -155,24 +209,21 @@ __global__ __launch_bounds__(64 * NW) void route_mfma_kernel(RouteArgs a) {
     if (t0 + t >= a.T) break;
     float z = lane < 16 * NE ? part[((lane >> 4) * 16 + t) * 16 + (lane & 15)] : -INFINITY;   // (E <= 64: one per lane)
     if (z != z) z = -INFINITY;      // a NaN logit never wins
-    float zmax = 0.f, sum = 0.f, mine = 0.f;
-    int my = 0;
-    for (int q = 0; q < a.k; ++q) {
-      float best = z;
-      int bi = lane;
+    // a logit's place: how many stand before it (larger, or equal and of a lower index)
+    int place = 0;
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const float ob = __shfl_xor(best, o, 64);
-        const int oi = __shfl_xor(bi, o, 64);
-        if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
-      }
-      if (!(best > -INFINITY) || bi >= E) bi = q;   // only with non-finite logits: a valid segment index
-      if (q == 0) zmax = best;
-      const float p = q == 0 || zmax == -INFINITY ? 1.f : a.runs ? __expf(best - zmax) : expf(best - zmax);
-      sum += p;
-      if (lane == q) my = bi, mine = p;
-      if (lane == bi) z = -INFINITY;
+    for (int e = 0; e < 16 * NE; ++e) {
+      const float v = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(z), e));
+      place += v > z || (v == z && e < lane);
     }
+    const int to = 4 * (lane < 16 * NE ? place : lane);
+    const float best = __uint_as_float(__builtin_amdgcn_ds_permute(to, __float_as_uint(z)));      // lane: the choice of this place
+    int my = __builtin_amdgcn_ds_permute(to, lane);
+    if (lane >= __popcll(__ballot(z > -INFINITY))) my = lane;   // only with non-finite logits: a valid segment index
+    const float zmax = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(best)));
+    const float mine = lane == 0 || zmax == -INFINITY ? 1.f : a.runs ? __expf(best - zmax) : expf(best - zmax);
+    float sum = 0.f;
+    for (int q = 0; q < a.k; ++q) sum += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), q));
     if (lane < a.k) {
       const long long o = (long long)(t0 + t) * a.k + lane;
       a.ids[o] = my;
@@ -857,6 +908,14 @@ template <int NW, int NE>
 void launch_route(const RouteArgs& a, hipStream_t s) {
   const int tiles = (a.T + 15) / 16;
   const size_t lds = (size_t)NW * NE * 256 * sizeof(float);
+  if (a.resid) {
+    const int room = (int)lds + 16 * (a.d + 8) * 2;      // (at most 32 + 64 KB)
+    static const hipError_t once = hipFuncSetAttribute(reinterpret_cast<const void*>(&route_mfma_kernel<NW, NE, true, true>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 98304 + 1024);
+    (void)once;
+    route_mfma_kernel<NW, NE, true, true><<<1, 64 * NW, room, s>>>(a);
+    return;
+  }
   if (tiles == 1) route_mfma_kernel<NW, NE, true><<<1, 64 * NW, lds, s>>>(a);
   else route_mfma_kernel<NW, NE, false><<<tiles, 64 * NW, lds, s>>>(a);
 }
@@ -874,6 +933,10 @@ bool route_mfma(const RouteArgs& a, int f32) {
 }
 
 }  // namespace
+
+bool route_norm_fits(const RouteArgs& a) {
+  return route_mfma(a, 0) && a.T <= 16 && a.d % 512 == 0 && a.d <= 2048 && aligned16(a.resid) && aligned16(a.norm);
+}
 
 bool route_topk_runs(const RouteArgs& a, int f32) { return route_mfma(a, f32) && a.E <= 16 && a.d % 128 == 0; }
 

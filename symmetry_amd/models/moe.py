@@ -65,7 +65,7 @@ A2A_STATS = os.environ.get("SYMMETRY_MOE_A2A_STATS", "0") == "1"
 # decode steps: routing in one launch and the combine fused with the residual prep (A/B: 0 = five routing launches
 # + combine + add_prep; profiles/r4/moe_decode_fused.jsonl)
 DECODE_FUSED = os.environ.get("SYMMETRY_MOE_DECODE_FUSED", "1") != "0"
-# rows up to which the routing runs as the one-workgroup launch: 8.8 vs 12.0 us at 1 row, 12.8 vs 14.0 at 4,
+# rows up to which the routing of layers that permute their rows runs as the one-workgroup launch: 8.8 vs 12.0 us at 1 row, 12.8 vs 14.0 at 4,
 # 17.8 vs 14.1 at 8 (profiles/r4/moe_decode_fused.jsonl)
 ROUTE_FUSED_ROWS = int(os.environ.get("SYMMETRY_MOE_ROUTE_FUSED_ROWS", "4"))
 
@@ -228,7 +228,8 @@ class MoEBlock:
 
     def forward_decode(self, i: int, resid, lnw, eps: float, w_next, xw, ss_1) -> torch.Tensor:
         """A decode step's MoE block straight off the fp32 residual stream: ONE routing launch (RMSNorm + router
-        + top-k + segments + permuted rows, ``ops.moe_decode_route``), the grouped expert GEMMs, and the weighted
+        + top-k + segments: ``ops.route_topk`` where the products gather, 8 rows of 2048 to 16 experts 6.8 us where the norm
+        apart takes 8.6; else with permuted rows, ``ops.moe_decode_route``, 22.6), the grouped expert GEMMs, and the weighted
         combine fused with the residual add + next-norm prep (``ops.moe_combine_prep``); under expert
         parallelism the combine stays separate (its partial sum is all-reduced first).  resid += MoE(RMSNorm(
         resid)); xw and the returned sum-of-squares partials ([T, P]; ``ss_1`` [T, 1] under EP): the next layer's
@@ -244,7 +245,11 @@ class MoEBlock:
         offsets = self._buf("offsets", (E + 1,), torch.int32)
         cursor = self._buf("cursor", (E,), torch.int32)
         src = None
-        if T <= ROUTE_FUSED_ROWS:
+        if self._gathers(i, R, d) and ops.route_norm_fits(T, d, E):
+            xs = self._buf("xn", (T, d), torch.bfloat16)
+            src = self._buf("src", (R,), torch.int32)
+            ops.route_topk(xs, self.router[i][:E], None, k, ids, w, offsets, dst, src, runs=E <= 16, resid=resid, norm=lnw, eps=eps)
+        elif T <= ROUTE_FUSED_ROWS:
             xs = self._buf("xs", (R, d), torch.bfloat16)
             ops.moe_decode_route(resid, lnw, eps, self.router[i][:E], k, ids, w, counts, offsets, cursor, xs, dst)
         else:  # the one-workgroup routing launch stops paying off past a few rows (bench_moe_decode.py)

@@ -1260,14 +1260,22 @@ def qk_row_norm_cache(z, bias, H, G, dk, wq, wk, eps, temp_coef, temp_every, pos
                                        kv_cache, key_scale)
 
 
-def route_topk(x, Wr, bias, k, ids, w, offsets, dst, src, runs=False):
+def route_topk(x, Wr, bias, k, ids, w, offsets, dst, src, runs=False, resid=None, norm=None, eps=0.0):
     """Router: logits x @ Wr.T + bias (fp32; bias optional), the k largest (ties: the lowest index) -> ids [T k], w = softmax
     over the chosen logits; and the routed rows' places in expert order: offsets [E + 1] segment bounds, dst [T k] place of
     every (token, choice), src [T k] token of every place.  ``runs`` (bf16, at most 16 experts, d % 128 == 0, no bias): the
-    order of sums and the exponential of ``moe_router`` + ``moe_route``, so both choose and weigh alike to the bit."""
+    order of sums and the exponential of ``moe_router`` + ``moe_route``, so both choose and weigh alike to the bit.  With
+    ``resid`` (fp32) and ``norm``, x (bf16, where ``route_norm_fits``) is written first: RMSNorm(resid)."""
     if _gpu(x):
-        return _hyb().route_topk(x, Wr, bias, int(k), ids, w, offsets, dst, src, bool(runs))
+        return _hyb().route_topk(x, Wr, bias, int(k), ids, w, offsets, dst, src, bool(runs), resid, norm, float(eps))
+    if resid is not None:
+        reference.rms_norm(resid, norm, eps, x)
     return reference.route_topk(x, Wr, bias, k, ids, w, offsets, dst, src)
+
+
+def route_norm_fits(rows: int, d: int, experts: int) -> bool:
+    """Shapes that ``route_topk`` normalises by itself: one workgroup's rows, which it keeps in LDS."""
+    return rows <= 16 and experts <= 64 and d % 512 == 0 and d <= 2048
 
 
 def expert_linear(x, src, W, offsets, y, relu2=False, glu=False):

@@ -221,3 +221,46 @@ def test_who_walks(R, N, K, glu, form):
     off = torch.arange(65).mul(R).div(64, rounding_mode="floor").int().cuda()
     y = torch.empty(R, N, dtype=BF16, device="cuda")
     assert ops._hyb().expert_linear(x, None, W, off, y, False, -1, glu) == form
+
+
+@pytest.mark.parametrize("T", [1, 7, 16])
+@pytest.mark.parametrize("E,k,d", [(16, 4, 2048), (8, 2, 512), (5, 5, 1536), (20, 3, 1024), (64, 8, 2048)])
+def test_router_of_the_residual(T, E, k, d):
+    """The norm inside the router: its rows are ops.rms_norm's but for sums in another order (fp32: a bf16 step, 2^-7 of a value, on
+    a few), and from those rows the choices, weights and segments are route_topk's own, to the bit."""
+    print("route_topk resid", T, E, k, d, flush=True)
+    torch.manual_seed(T + E)
+    resid, norm = torch.randn(T, d).cuda() * 3, torch.rand(d).to(BF16).cuda()
+    Wr, R, i32 = (torch.randn(E, d) * 2 * d ** -0.5).to(BF16).cuda(), T * k, dict(dtype=torch.int32, device="cuda")
+    xn, x = torch.empty(T, d, dtype=BF16, device="cuda"), torch.full((T + 1, d), 7.0, dtype=BF16, device="cuda")
+    ops.rms_norm(resid, norm, 1e-5, xn)
+    got, want = ([torch.empty(R, **i32), torch.empty(R, device="cuda")] + [torch.empty(n, **i32) for n in (E + 1, R, R)]
+                 for _ in range(2))
+    assert ops.route_norm_fits(T, d, E)
+    ops.route_topk(x[:T], Wr, None, k, *got, runs=E <= 16, resid=resid, norm=norm, eps=1e-5)
+    diff = (x[:T].float() - xn.float()).abs()
+    assert bool((diff <= 2.0 ** -7 * xn.float().abs()).all()) and int((diff > 0).sum()) <= T * d // 100 and bool((x[T] == 7).all())
+    ops.route_topk(x[:T], Wr, None, k, *want, runs=E <= 16)
+    for a, b in zip(got[:3], want[:3]):
+        assert torch.equal(a, b)
+    assert torch.equal(got[4][got[3].long()].cpu(), (torch.arange(R) // k).int())
+    with pytest.raises(RuntimeError):      # (17 rows are two workgroups' work)
+        big = torch.empty(17, d, dtype=BF16, device="cuda")
+        ops.route_topk(big, Wr, None, 1, *(torch.empty(99, dtype=t.dtype, device="cuda") for t in got), resid=big.float(), norm=norm, eps=1e-5)
+
+
+@pytest.mark.parametrize("R", [4, 60])
+def test_choices_among_infinite_logits(R):
+    """Infinite and missing logits keep their places: +inf first, ties to the lowest index, -inf and NaN never before a number."""
+    d, E, k = 512, 16, 4
+    bias = torch.zeros(E)
+    bias[3], bias[5], bias[9] = float("inf"), float("-inf"), float("nan")
+    x, Wr = torch.zeros(R, d, dtype=BF16).cuda(), torch.zeros(E, d, dtype=BF16).cuda()
+    ids, off, dst, src = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (R * k, E + 1, R * k, R * k))
+    ops.route_topk(x, Wr, bias.cuda(), k, ids, torch.empty(R * k, device="cuda"), off, dst, src)
+    assert ids.view(R, k).tolist() == [[3, 0, 1, 2]] * R
+    bias[:] = float("-inf")
+    bias[7] = 1.0
+    w = torch.empty(R * k, device="cuda")
+    ops.route_topk(x, Wr, bias.cuda(), k, ids, w, off, dst, src)
+    assert ids.view(R, k).tolist() == [[7, 1, 2, 3]] * R and w.view(R, k).tolist() == [[1.0, 0.0, 0.0, 0.0]] * R

@@ -54,3 +54,28 @@ def test_routed_experts(gpu, monkeypatch, E, k, d, F, T, gathers, grouped):
         gate, up = (x[t].double() @ w["layers.0.w13"][e].double().t()).split(F, 1)
         want.index_add_(0, t, p[t, j, None] * ((torch.nn.functional.silu(gate) * up) @ w["layers.0.w2"][e].double().t()))
     assert float((got - want).norm() / want.norm()) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("T", [1, 3, 8])
+def test_decode_off_the_residual(gpu, monkeypatch, T):
+    """A decode step's block (norm, routing, experts, residual, next norm's input) at one row and more, in one routing launch."""
+    monkeypatch.setenv("SYMMETRY_MOE_PRESHUFFLE", "0")
+    E, k, d, F = 16, 4, 1536, 1536
+    moe, w = _block(E, k, d, F)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    resid = torch.randn(T, d, device="cuda", generator=g)
+    norm, after = (torch.rand(d, device="cuda", generator=g).bfloat16() + 0.5 for _ in range(2))
+    x = (resid.double() * (resid.double().square().mean(-1, keepdim=True) + 1e-5).rsqrt() * norm.double())
+    p, pick = (x @ w["layers.0.router"].double().t()).topk(k, -1)
+    p = p.softmax(-1)
+    want = resid.double().clone()
+    for e in range(E):
+        t, j = (pick == e).nonzero(as_tuple=True)
+        gate, up = (x[t] @ w["layers.0.w13"][e].double().t()).split(F, 1)
+        want.index_add_(0, t, p[t, j, None] * ((torch.nn.functional.silu(gate) * up) @ w["layers.0.w2"][e].double().t()))
+    xw = torch.empty(T, d, device="cuda", dtype=torch.bfloat16)
+    start = resid.clone()
+    moe.forward_decode(0, resid, norm, 1e-5, after, xw, None)
+    # x and the gated rows rounded to bf16, and the routing weights' logits off x by its rounding: under 2^-7 of the block's part
+    assert float((resid.double() - want).norm() / (want - start.double()).norm()) <= 2.0 ** -7
+    assert float((xw.double() - resid.double() * after.double()).abs().max()) <= 2.0 ** -8 * float((resid.double() * after.double()).abs().max())
