@@ -69,6 +69,11 @@ DECODE_FUSED = os.environ.get("SYMMETRY_MOE_DECODE_FUSED", "1") != "0"
 # 17.8 vs 14.1 at 8 (profiles/r4/moe_decode_fused.jsonl)
 ROUTE_FUSED_ROWS = int(os.environ.get("SYMMETRY_MOE_ROUTE_FUSED_ROWS", "4"))
 
+# expert widths whose down products of few rows are ``expert_linear``'s walk, one fp32 result, and not the skinny GEMM's split
+# slabs, which the combine sums (2048 outputs, with the combine, us: 16 experts, 32 rows of 1536 24.1 -> 20.5, 4 rows 12.5 ->
+# 11.3; 64 experts, 64 rows of 2048 87 -> 62.6; 8 experts, 16 rows of 3072 27 -> 22.6; 512 wide is no split and as fast, 12.2 / 12.3)
+DOWN_WALKS = (1536, 2048, 3072)
+
 
 class MoEBlock:
     def __init__(self, model, ep_comm=None, mode: str | None = None):
@@ -358,6 +363,10 @@ class MoEBlock:
                 y1 = self._buf("y1", (s1, R, 2 * F), torch.float32)
                 ops.grouped_skinny(xs, w13, offsets, e_lo, y1, wshuf=self.single_copy)
                 ops.swiglu(y1, act)
+            if src is not None and d >= 1536 and F in DOWN_WALKS and n_local <= 64 and R <= 8 * n_local:
+                y2 = self._buf("y2f", (R, d), torch.float32)
+                ops.expert_linear(act, None, w2, segments, y2)
+                return y2
             s2 = ops.choose_splits(d, F)
             y2 = self._buf("y2", (s2, R, d), torch.float32)
             ops.grouped_skinny(act, w2, offsets, e_lo, y2, wshuf=self.single_copy)

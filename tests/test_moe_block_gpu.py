@@ -56,6 +56,27 @@ def test_routed_experts(gpu, monkeypatch, E, k, d, F, T, gathers, grouped):
     assert float((got - want).norm() / want.norm()) <= 2.0 ** -8
 
 
+@pytest.mark.parametrize("E,k,d,F,T,walks", [(16, 4, 1536, 1536, 8, True), (64, 4, 2048, 2048, 16, True), (9, 1, 1536, 3072, 64, True),
+                                             (16, 4, 1024, 1536, 8, False), (16, 4, 1536, 1024, 8, False)])
+def test_down_products_of_few_rows(gpu, monkeypatch, E, k, d, F, T, walks):
+    """One fp32 product by the walk against the skinny GEMM's slabs, bounds as above."""
+    monkeypatch.setenv("SYMMETRY_MOE_PRESHUFFLE", "0")
+    moe, w = _block(E, k, d, F)
+    calls, plain = [], ops.grouped_skinny
+    monkeypatch.setattr(ops, "grouped_skinny", lambda *a, **kw: calls.append(1) or plain(*a, **kw))
+    x = torch.randn(T, d, device="cuda", generator=torch.Generator(device="cuda").manual_seed(T)).bfloat16()
+    got = moe._forward_local(0, x, False).double()
+    assert calls == ([] if walks else [1])
+    p, pick = (x.double() @ w["layers.0.router"].double().t()).topk(k, -1)
+    p = p.softmax(-1)
+    want = torch.zeros(T, d, dtype=torch.float64, device="cuda")
+    for e in range(E):
+        t, j = (pick == e).nonzero(as_tuple=True)
+        gate, up = (x[t].double() @ w["layers.0.w13"][e].double().t()).split(F, 1)
+        want.index_add_(0, t, p[t, j, None] * ((torch.nn.functional.silu(gate) * up) @ w["layers.0.w2"][e].double().t()))
+    assert float((got - want).norm() / want.norm()) <= 2.0 ** -8
+
+
 @pytest.mark.parametrize("T", [1, 3, 8])
 def test_decode_off_the_residual(gpu, monkeypatch, T):
     """A decode step's block (norm, routing, experts, residual, next norm's input) at one row and more, in one routing launch."""
