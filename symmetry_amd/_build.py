@@ -105,7 +105,7 @@ HIP_FLAGS = [
     "-munsafe-fp-atomics",
     "-Wno-unused-result",
 ]
-# no packed-fp32 instruction selection (v_pk_*_f32): scalar fp32 code only
+# no packed-fp32 instruction selection (v_pk_*_f32), in any library: some of their forms have given wrong results now and then
 NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 
@@ -125,8 +125,7 @@ def build_kernels(verbose: bool = False, force: bool = False) -> str:
         obj = os.path.join(OBJ, os.path.basename(src) + ".o")
         objs.append(obj)
         if force or _newer(obj, [src] + headers):
-            cmd = [HIPCC, "-c", src, "-o", obj, "-I", kdir] + HIP_FLAGS
-            jobs.append(cmd)
+            jobs.append([HIPCC, "-c", src, "-o", obj, "-I", kdir] + HIP_FLAGS + NO_PACKED_FP32)
     for bsrc in sorted(b for b in glob.glob(os.path.join(CSRC, "bindings", "*.cpp"))
                        if os.path.basename(b) not in LATENT_BINDINGS + HYBRID_BINDINGS):
         bobj = os.path.join(OBJ, "bind_" + os.path.basename(bsrc) + ".o")
