@@ -10,8 +10,8 @@
 //   * orientation Y^T = W . x^T on v_mfma_f32_16x16x32_bf16: the weight tile is the A operand and comes
 //     from the MFMA-preshuffled weight copy (models/layout.py::preshuffle, the decode layout), so every
 //     weight DMA instruction reads 1 KB contiguous; x fragments are the B operand;
-//   * workgroup = 4 waves x RW 16-row weight tiles (64 RW output features) x all M tokens x one k slice;
-//     the k split S is chosen on the host so the grid fills the 256 CUs; partial sums go to fp32 slabs
+//   * workgroup = CT 16-row weight tiles (4 waves x RW of them, or 3, 6, 7 or 14 where those fill more CUs) x all M tokens x
+//     one k slice; the k split S is chosen on the host so the grid fills the 256 CUs; partial sums go to fp32 slabs
 //     that the consumer (rope_cache / add_rms_norm / swiglu, LinOut) sums in its prologue, as the skinny
 //     decode GEMM's do;
 //   * x AND the weight blocks stream through an LDS ring of 64-deep chunks by LDS-DMA (buffer loads: x
@@ -22,8 +22,13 @@
 //     of each 128-B x row is XOR-swizzled with (row >> 1) & 7 on the DMA source and on the read, which
 //     makes the x fragment reads bank-conflict free;
 //   * a step's fragments are read from LDS while the step before is multiplied: with one wave a SIMD nothing else covers the
-//     reads (137 rows, us: 4096 x 14336 38.9 -> 30.6, 6144 x 4096 23.6 -> 18.5, 4096 x 4096 19.8 -> 14.4; a ring of its own for
-//     the weights, two chunks deeper, was slower).  x tiles come in steps of 32 rows (up to 64: 2 and 4; 96, 128, 160, 192, 256);
+//     reads (a ring of its own for the weights, two chunks deeper, was slower, also with waves of its own that fill it);
+//   * what bounds it is the bytes in flight: 137 rows of 28672 x 4096 take 50 us with no product at all, and as many with them.
+//     So x tiles come in steps of 16 rows (a slot less of padding is a slot more of the ring), the chunk's DMAs are dealt to the
+//     waves one by one, and the weights are loaded past the caches (read once; x stays in the L2).  Against row tiles in steps of
+//     32 and cached weights, us: 28672 x 4096 at 20 rows 41.9 -> 38.7, 64 43.1 -> 40.5, 137 57.8 -> 50.9, 192 65.0 -> 62.9;
+//     4096 x 14336 at 64 24.3 -> 22.8, 137 31.6 -> 28.6, 240 46.1 -> 40.4; 4096 x 4096 at 137 14.5 -> 13.4.  A K range for every
+//     wave, x in registers, was slower (64 to 70 at 137 rows): its waves wait for the weights each by itself;
 //   * the 16x16 accumulator of (weight tile, token tile) holds 4 consecutive features of one token per
 //     lane: one float4 store per accumulator into the slab.
 #include "common.h"
@@ -45,26 +50,29 @@ SYM_DEV void mg_dma(__amdgpu_buffer_rsrc_t r, int voff, int soff, char* lds) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t*)lds, 16, voff, soff, 0, 0);
 }
 
-// non-temporal (aux = 2) LDS-DMA for the once-read weight stream (MI355X_MICROARCH.md row nt-weights)
+// non-temporal (aux = 2) LDS-DMA for the once-read weight stream
 SYM_DEV void mg_dma_nt(__amdgpu_buffer_rsrc_t r, int voff, int soff, char* lds) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t*)lds, 16, voff, soff, 0, 2);
 }
 
-// WV waves, a multiple of 4 of them or not: a chunk's 2 MT x DMAs go round the waves, the last ones twice where they do not divide
-template <int MT, int RW, int WV>
+// CT weight tiles, WV waves of RW of them (the last wave may have fewer).  A chunk's 2 MT x DMAs and 2 CT weight DMAs, 1 KB each, go
+// round the waves; where they do not divide, the last ones twice
+template <int MT, int CT, int WV>
 struct MgCfg {
+  static constexpr int RW = (CT + WV - 1) / WV;
   static constexpr int XB = 16 * MT * 128;                   // x bytes of one 64-deep chunk
-  static constexpr int WB = WV * RW * 2 * 1024;               // weight bytes of one chunk (2 blocks per tile)
+  static constexpr int WB = CT * 2 * 1024;                   // weight bytes of one chunk (2 blocks per tile)
   static constexpr int SLOT = XB + WB;
   static constexpr int SLOTS = MG_LDS / SLOT > 8 ? 8 : MG_LDS / SLOT;
   static constexpr int D = SLOTS - 1;                        // chunks in flight ahead of the computed one
-  static constexpr int NX = (2 * MT + WV - 1) / WV;          // x DMA instructions per wave per chunk
-  static constexpr int NDMA = NX + 2 * RW;                   // DMA instructions per wave per chunk
+  static constexpr int NX = (2 * MT + WV - 1) / WV;          // x, weight DMA instructions per wave per chunk
+  static constexpr int NB = (2 * CT + WV - 1) / WV;
+  static constexpr int NDMA = NX + NB;
   static constexpr int VM_KEEP = (D - 1) * NDMA;             // younger DMAs left in flight at the wait
-  static_assert(MT % 2 == 0 && D >= 1 && VM_KEEP <= 63, "mgemm config");
+  static_assert(D >= 1 && VM_KEEP <= 63, "mgemm config");
 };
 
-// MT: 16-token tiles (M <= 16 MT); RW: 16-row weight tiles per wave.  Weights MFMA-preshuffled
+// MT: 16-token tiles (M <= 16 MT); CT: 16-row weight tiles.  nt: the weights past the caches.  Weights MFMA-preshuffled
 // (models/layout.py::preshuffle): block (t, kb) = 16 rows x 32 k, 1 KB in fragment order.
 // EPI < 0: the k split's fp32 slab is the output (the consumer kernel sums the slabs).  EPI >= 0: a fused
 // consumer (decode_epi.h): with one split the accumulators go straight to epilogue<EPI>; with S splits every
@@ -72,20 +80,21 @@ struct MgCfg {
 // acquire around a per-group counter, cdna_hip_programming.md §5 "In-launch split-K reduction") sums the S
 // slabs of its columns in the accumulator layout, applies the deferred-RMSNorm row scale (e.ss_in) and runs
 // the epilogue -- the separate rope_cache / add+RMSNorm / SwiGLU launches of the slab path disappear.
-// `counters` [N / (64 RW)] start at zero and are re-armed by the last arriver (graph-replay safe).
-template <int MT, int RW, bool WNT, int EPI, int WV>
+// `counters` [N / (16 CT)] start at zero and are re-armed by the last arriver (graph-replay safe).
+template <int MT, int CT, int EPI, int WV>
 __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restrict__ x, const bf16* __restrict__ W,
                                                            float* __restrict__ y, int M, int N, int K, int kslice,
-                                                           DecodeEpi e, int* __restrict__ counters) {
-  using C = MgCfg<MT, RW, WV>;
+                                                           DecodeEpi e, int* __restrict__ counters, int nt) {
+  using C = MgCfg<MT, CT, WV>;
+  constexpr int RW = C::RW;
   __shared__ __attribute__((aligned(1024))) char smem[C::SLOTS * C::SLOT];
   asm volatile("" ::: "a0");  // accumulators may live in AGPRs
 
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int split = blockIdx.y;
   const int k0 = split * kslice;
   const int nch = kslice / 64;
-  const int tile0 = (blockIdx.x * WV + wid) * RW;  // first 16-row weight tile of this wave
+  const int tile0 = blockIdx.x * CT + wid * RW;  // first 16-row weight tile of this wave
 
   // ---- x DMA: wave w fills rows (NX w + i) * 8 .. + 8 of each chunk; lane -> (row lane >> 3, 16-B chunk
   // lane & 7), source chunk swizzled by (row >> 1) & 7.  Rows >= M read as zeros (buffer range).
@@ -96,25 +105,26 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
     const int row = min(C::NX * wid + i, 2 * MT - 1) * 8 + (lane >> 3);
     vx[i] = row * K * 2 + 16 * ((lane & 7) ^ ((row >> 1) & 7)) + k0 * 2;
   }
-  // ---- weight DMA: the wave's own tiles, block (tile, 2c + s) -> its 1 KB LDS block, lane-linear
+  // ---- weight DMA: block (tile, 2c + s) -> its 1 KB LDS block, lane-linear; wave w fills blocks NB w + i of the chunk's 2 CT
   const __amdgpu_buffer_rsrc_t rw = mg_rsrc(W, (long long)N * K * 2);
-  const int vw = (tile0 * (K / 32) + k0 / 32) * 1024 + lane * 16;
-  const int wstride = (K / 32) * 1024;  // bytes between consecutive weight tiles
-  char* const dw = smem + C::XB + wid * RW * 2 * 1024;
+  int vw[C::NB];
+#pragma unroll
+  for (int i = 0; i < C::NB; ++i) {
+    const int b = min(C::NB * wid + i, 2 * CT - 1);
+    vw[i] = ((blockIdx.x * CT + (b >> 1)) * (K / 32) + k0 / 32 + (b & 1)) * 1024 + lane * 16;
+  }
 
   auto issue = [&](int c, int slot) {
     const int xo = c * 128, wo = c * 2048;
 #pragma unroll
     for (int i = 0; i < C::NX; ++i) mg_dma(rx, vx[i], xo, smem + slot * C::SLOT + min(C::NX * wid + i, 2 * MT - 1) * 1024);
+    char* const dw = smem + slot * C::SLOT + C::XB;
+    if (nt) {
 #pragma unroll
-    for (int rt = 0; rt < RW; ++rt) {
-      if constexpr (WNT) {
-        mg_dma_nt(rw, vw + rt * wstride, wo, dw + slot * C::SLOT + (2 * rt) * 1024);
-        mg_dma_nt(rw, vw + rt * wstride, wo + 1024, dw + slot * C::SLOT + (2 * rt + 1) * 1024);
-      } else {
-        mg_dma(rw, vw + rt * wstride, wo, dw + slot * C::SLOT + (2 * rt) * 1024);
-        mg_dma(rw, vw + rt * wstride, wo + 1024, dw + slot * C::SLOT + (2 * rt + 1) * 1024);
-      }
+      for (int i = 0; i < C::NB; ++i) mg_dma_nt(rw, vw[i], wo, dw + min(C::NB * wid + i, 2 * CT - 1) * 1024);
+    } else {
+#pragma unroll
+      for (int i = 0; i < C::NB; ++i) mg_dma(rw, vw[i], wo, dw + min(C::NB * wid + i, 2 * CT - 1) * 1024);
     }
   };
 
@@ -123,7 +133,7 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
   const int fr = lane & 15;
   const int xo0 = fr * 128 + 16 * ((lane >> 4) ^ ((fr >> 1) & 7));
   const int xo1 = fr * 128 + 16 * ((4 + (lane >> 4)) ^ ((fr >> 1) & 7));
-  const int wo_l = C::XB + wid * RW * 2 * 1024 + lane * 16;
+  const int wo_l = C::XB + lane * 16;
 
   f32x4 acc[RW][MT];
 #pragma unroll
@@ -145,7 +155,7 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
       for (int u = 0; u < PER; ++u) {
         const int i = PER * mt + u;
         if (!reads || i >= READS) continue;
-        if (i < RW) next.w[i] = *(const bf16x8*)(sb + wo_l + (2 * i + s) * 1024);
+        if (i < RW) next.w[i] = *(const bf16x8*)(sb + wo_l + (2 * min(wid * RW + i, CT - 1) + s) * 1024);
         else next.x[i - RW] = *(const bf16x8*)(sb + (s ? xo1 : xo0) + (i - RW) * 2048);
       }
       if (multiplies) {
@@ -231,6 +241,7 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
   if (EPI < 0 || S > 1) {
 #pragma unroll
     for (int rt = 0; rt < RW; ++rt) {
+      if (CT % RW && wid * RW + rt >= CT) continue;
       const int n = 16 * (tile0 + rt) + 4 * (lane >> 4);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
@@ -276,6 +287,7 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
     }
 #pragma unroll
     for (int rt = 0; rt < RW; ++rt) {
+      if (CT % RW && wid * RW + rt >= CT) continue;
       const int n = 16 * (tile0 + rt) + 4 * (lane >> 4);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
@@ -307,16 +319,12 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
   }
 }
 
-int g_mgemm_nt = 0;
+int g_mgemm_nt = 1;
 
-template <int MT, int RW, int EPI, int WV = 4>
-void launch_mt_rw(const bf16* x, const bf16* W, float* y, int M, int N, int K, int S, const DecodeEpi& e,
-                  int* counters, hipStream_t s) {
-  const dim3 grid(N / (16 * WV * RW), S);
-  if (g_mgemm_nt && EPI < 0)
-    mgemm_kernel<MT, RW, true, EPI, WV><<<grid, 64 * WV, 0, s>>>(x, W, y, M, N, K, K / S, e, counters);
-  else
-    mgemm_kernel<MT, RW, false, EPI, WV><<<grid, 64 * WV, 0, s>>>(x, W, y, M, N, K, K / S, e, counters);
+template <int MT, int CT, int EPI, int WV = 4>
+void launch_ct(const bf16* x, const bf16* W, float* y, int M, int N, int K, int S, const DecodeEpi& e, int* counters,
+               hipStream_t s) {
+  mgemm_kernel<MT, CT, EPI, WV><<<dim3(N / (16 * CT), S), 64 * WV, 0, s>>>(x, W, y, M, N, K, K / S, e, counters, g_mgemm_nt);
 }
 
 template <int MT, int EPI>
@@ -324,48 +332,42 @@ void launch_mt(const bf16* x, const bf16* W, float* y, int M, int N, int K, int 
                int* counters, hipStream_t s) {
   if constexpr (EPI == DECODE_EPI_SWIGLU && MT <= 12) {
     // Seven waves where their columns fill the CUs better than four waves' do (widths of 7 x 2^n, as 2 x 14336): a CU's intake
-    // is what bounds the stream.  28672 x 4096, 224 workgroups -> 256,
-    // us: 64 rows 50.8 -> 44.5, 96 52.4 -> 46.9, 128 56.9 -> 51.4, 192 67.3 -> 64.3; 57344 x 8192 at 96 rows 177 -> 175
-    if (S == 1 && N % 112 == 0 && N / 112 <= 256 && N / 112 > N / (64 * rw)) {
-      launch_mt_rw<MT, 1, EPI, 7>(x, W, y, M, N, K, S, e, counters, s);
-      return;
-    }
-    if (S == 1 && N % 224 == 0 && N / 224 <= 256 && N / 224 > N / (64 * rw)) {
-      launch_mt_rw<MT, 2, EPI, 7>(x, W, y, M, N, K, S, e, counters, s);
-      return;
-    }
+    // is what bounds the stream.  28672 x 4096, 224 workgroups of four waves / 256 of seven, us: 20 rows 42.6 / 38.7, 64
+    // 41.3 / 40.5, 112 48.0 / 45.0, 137 53.0 / 50.9, 192 65.4 / 62.9; 57344 x 8192 at 96 rows 177 / 175
+    if (S == 1 && N % 112 == 0 && N / 112 <= 256 && N / 112 > N / (64 * rw)) return launch_ct<MT, 7, EPI, 7>(x, W, y, M, N, K, S, e, counters, s);
+    if (S == 1 && N % 224 == 0 && N / 224 <= 256 && N / 224 > N / (64 * rw)) return launch_ct<MT, 14, EPI, 7>(x, W, y, M, N, K, S, e, counters, s);
   }
-  if constexpr (MT > 8) {  // 160 to 256 rows: at most 2 weight tiles per wave (accumulators + LDS ring)
-    if (rw == 1) launch_mt_rw<MT, 1, EPI>(x, W, y, M, N, K, S, e, counters, s);
-    else launch_mt_rw<MT, 2, EPI>(x, W, y, M, N, K, S, e, counters, s);
-  } else {
-    switch (rw) {
-      case 1: launch_mt_rw<MT, 1, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
-      case 3: launch_mt_rw<MT, 3, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
-      case 4: launch_mt_rw<MT, 4, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
-      default: launch_mt_rw<MT, 2, EPI>(x, W, y, M, N, K, S, e, counters, s); break;
-    }
+  if constexpr (EPI < 0) {
+    // ... and three or six waves of a tile each for widths of 3 x 2^n, by the same rule (4 / 3 tiles, us: 6144 x 4096 at 40 rows
+    // 13.1 / 10.9, 64 13.9 / 12.5; 3072 x 2048 at 40 5.8 / 5.4, 240 11.5 / 10.9; 8 / 6 tiles: 6144 x 4096 at 100 rows 15.2 / 14.6,
+    // 137 17.7 / 16.2, 240 24.4 / 21.5)
+    if (rw == 1 && N % 48 == 0 && N / 48 * S <= 256) return launch_ct<MT, 3, EPI, 3>(x, W, y, M, N, K, S, e, counters, s);
+    if (rw == 2 && N % 96 == 0 && N / 96 * S <= 256) return launch_ct<MT, 6, EPI, 6>(x, W, y, M, N, K, S, e, counters, s);
   }
+  if constexpr (MT <= 8) {  // 144 to 256 rows: at most 2 weight tiles per wave (accumulators + LDS ring)
+    if (rw == 3) return launch_ct<MT, 12, EPI>(x, W, y, M, N, K, S, e, counters, s);
+    if (rw == 4) return launch_ct<MT, 16, EPI>(x, W, y, M, N, K, S, e, counters, s);
+  }
+  if (rw == 1) launch_ct<MT, 4, EPI>(x, W, y, M, N, K, S, e, counters, s);
+  else launch_ct<MT, 8, EPI>(x, W, y, M, N, K, S, e, counters, s);
 }
 
+// Row tiles by EPI: steps of 16 rows where the form is used by default (the others, coarser)
 template <int EPI>
 void launch_epi_m(const bf16* x, const bf16* W, float* y, int M, int N, int K, int S, int rw, const DecodeEpi& e,
                   int* counters, hipStream_t s) {
-  constexpr bool fine = EPI < 0 || EPI == DECODE_EPI_SWIGLU;      // (the others are off by default)
-  if (M <= 32)
-    launch_mt<2, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
-  else if (M <= 64)
-    launch_mt<4, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
-  else if (fine && M <= 96)
-    launch_mt<fine ? 6 : 8, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
-  else if (M <= 128)
-    launch_mt<8, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
-  else if (fine && M <= 160)
-    launch_mt<fine ? 10 : 16, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
-  else if (fine && M <= 192)
-    launch_mt<fine ? 12 : 16, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
-  else
-    launch_mt<16, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
+  const int tiles = (M + 15) / 16;
+#define MG_TILES(t) \
+  if (tiles <= t) return launch_mt<t, EPI>(x, W, y, M, N, K, S, rw, e, counters, s)
+  MG_TILES(2);
+  if constexpr (EPI < 0 || EPI == DECODE_EPI_SWIGLU) {
+    MG_TILES(3); MG_TILES(4); MG_TILES(5); MG_TILES(6); MG_TILES(7); MG_TILES(8); MG_TILES(9); MG_TILES(10); MG_TILES(11);
+    MG_TILES(12); MG_TILES(14);
+  } else {
+    MG_TILES(4); MG_TILES(8);
+  }
+#undef MG_TILES
+  launch_mt<16, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
 }
 
 }  // namespace

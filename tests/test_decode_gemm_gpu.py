@@ -330,7 +330,7 @@ def _mg(gpu, M, N, K):
 
 
 @pytest.mark.parametrize("N,K", [(12288, 512), (28672, 320), (57344, 128)])
-@pytest.mark.parametrize("M", [17, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 256])
+@pytest.mark.parametrize("M", [17, 33, 48, 64, 65, 80, 96, 97, 113, 128, 129, 144, 145, 160, 161, 192, 193, 224, 256])
 def test_gate_up_of_one_wave(gpu, M, N, K):
     """gate_up and its SwiGLU as whole columns in one launch, at the ends of the row tiles, four waves and seven (one and two
     weight tiles each): no slab, the deferred norm's scale."""

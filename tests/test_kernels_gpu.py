@@ -305,6 +305,28 @@ def test_mgemm_tiles_and_ring(gpu, M, chunks):
             assert bool(((y[s].double() - xs @ wk.t()).abs() <= room).all()), (rw, s)
 
 
+@pytest.mark.parametrize("M", [17, 48, 49, 80, 81, 112, 113, 128, 144, 145, 176, 177, 224, 225, 256])
+@pytest.mark.parametrize("rw,N", [(1, 192), (2, 384), (1, 128), (2, 256)])
+def test_mgemm_tile_columns(gpu, M, rw, N):
+    """Row tiles at the ends of their 16-row steps, with three, six, four and eight weight tiles a workgroup, over k slices of
+    1 and 11 chunks; the slabs' last rows are the last that are written.  fp32 sums of K terms err by about sqrt(K) 2^-24."""
+    from symmetry_amd.models.layout import preshuffle
+
+    g = torch.Generator(device=gpu).manual_seed(M + N)
+    for K in (128, 1408):
+        x = torch.randn(M, K, device=gpu, generator=g).bfloat16()
+        w = torch.randn(N, K, device=gpu, generator=g).bfloat16()
+        mem = torch.full((2 * M * N + N,), 7.0, device=gpu)
+        y = mem[:2 * M * N].view(2, M, N)
+        ops.mgemm(x, preshuffle(w), y, rw)
+        assert bool((mem[2 * M * N:] == 7.0).all())
+        half = K // 2
+        for s in range(2):
+            xs, wk = x[:, s * half:(s + 1) * half].double(), w[:, s * half:(s + 1) * half].double()
+            room = 8 * half ** 0.5 * 2.0 ** -24 * xs.norm(dim=1)[:, None] * wk.norm(dim=1)[None]
+            assert bool(((y[s].double() - xs @ wk.t()).abs() <= room).all()), (K, s)
+
+
 @pytest.mark.parametrize("V", [1, 3, 4, 129, 4092, 4096, 32764, 32768, 32770, 32772, 70004])
 @pytest.mark.parametrize("first", [0, 1])
 def test_logits_argmax_finds_the_first_largest(gpu, V, first):
