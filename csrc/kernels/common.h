@@ -79,6 +79,46 @@ SYM_DEV u32x4 half_swap(u32x4 keep, u32x4 from) {
   return r;
 }
 
+// Rows from memory to MFMA operands.  A lane holds a row's 8 values, neighbouring lanes different rows; but the load path takes
+// 64 bytes of one line from 4 neighbouring lanes at once, and lanes of different lines one by one: 1 KB loads whose neighbours
+// differ by a row move 37 bytes a ns into a CU (all 256 read from the L2), whose quads read 64 contiguous bytes 126.  So load i of
+// four takes rows 4 r + i, the quad q of lanes a row's bytes 64 q on, and quad_transpose turns 4 loads into 4 operands: lane 4 r + q
+// of 16 then holds row 4 r + q, operand i its chunk 4 h + i (h: the lane's 16).  The order of k is another than the lanes', the
+// same for both operands.
+// One step: a's odd (BIT 1; BIT 2: upper) lanes of every quad change places with b's even (lower) ones.
+template <int BIT>
+SYM_DEV void quad_exchange(u32x4& a, u32x4& b) {
+  constexpr unsigned long long keep = BIT == 1 ? 0x5555555555555555ull : 0x3333333333333333ull;
+  u32x4 n;
+// (s_nop: a VALU result is read by a DPP operand, or by an MFMA behind this, two states later)
+#define QUAD_EXCHANGE(perm)                                                                                \
+  asm("s_nop 1\n\t"                                                                                        \
+      "s_mov_b64 vcc, %12\n\t"                                                                             \
+      "v_cndmask_b32_dpp %0, %4, %8, vcc " perm " row_mask:0xf bank_mask:0xf\n\t"                          \
+      "v_cndmask_b32_dpp %1, %5, %9, vcc " perm " row_mask:0xf bank_mask:0xf\n\t"                          \
+      "v_cndmask_b32_dpp %2, %6, %10, vcc " perm " row_mask:0xf bank_mask:0xf\n\t"                         \
+      "v_cndmask_b32_dpp %3, %7, %11, vcc " perm " row_mask:0xf bank_mask:0xf\n\t"                         \
+      "s_mov_b64 vcc, %13\n\t"                                                                             \
+      "v_cndmask_b32_dpp %4, %8, %4, vcc " perm " row_mask:0xf bank_mask:0xf\n\t"                          \
+      "v_cndmask_b32_dpp %5, %9, %5, vcc " perm " row_mask:0xf bank_mask:0xf\n\t"                          \
+      "v_cndmask_b32_dpp %6, %10, %6, vcc " perm " row_mask:0xf bank_mask:0xf\n\t"                         \
+      "v_cndmask_b32_dpp %7, %11, %7, vcc " perm " row_mask:0xf bank_mask:0xf\n\t"                         \
+      "s_nop 1"                                                                                            \
+      : "=&v"(n[0]), "=&v"(n[1]), "=&v"(n[2]), "=&v"(n[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]) \
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "s"(keep), "s"(~keep)                                  \
+      : "vcc")
+  if constexpr (BIT == 1) QUAD_EXCHANGE("quad_perm:[1,0,3,2]");
+  else QUAD_EXCHANGE("quad_perm:[2,3,0,1]");
+#undef QUAD_EXCHANGE
+  a = n;
+}
+SYM_DEV void quad_transpose(u32x4& a, u32x4& b, u32x4& c, u32x4& d) {
+  quad_exchange<1>(a, b);
+  quad_exchange<1>(c, d);
+  quad_exchange<2>(a, c);
+  quad_exchange<2>(b, d);
+}
+
 // Rows of a chunk through a buffer whose range ends with the chunk's last row: what lies behind it reads 0 and is not stored, and a
 // lane's places in a chunk are the same 32-bit offsets in every chunk.  row, width: bytes from row to row, of a row's part;
 // NO_PLACE: the offset of a lane without one.

@@ -53,28 +53,31 @@ SYM_DEV void store_rows(const Args& a, int n0, int lane, f32x4 v, f32x4 u) {
   }
 }
 
-// RT: weight tiles of a workgroup.  RH: weight rows of a tile, 16 or 8.  U: 64-deep k blocks of a chunk.  Every wave has
-// the same number of whole chunks.
+// RT: weight tiles of a workgroup.  RH: weight rows of a tile, 16 or 8.  Every wave has the same number of whole blocks, UK deep
+// each: four load instructions a tile.
 //
-// One load instruction reads 128 contiguous bytes (a 64-deep k block) of each of 8 weight rows: lanes 0-7 of each row of 16
-// lanes hold the block's first 32-deep step, lanes 8-15 its second.  Two such loads (rows 0-7, rows 8-15) become the two
-// steps' A operands by exchanging halves, 4 v_mov_dpp each.  With RH = 8 there is one load, and rows 8-15 of the product
-// are dropped.
+// Four load instructions read a block: 256 contiguous bytes of 16 rows (RH 8: 512 of 8), and quad_transpose makes four operands of
+// them.  x is read the same way.  What bounds the launch is what a CU takes in, x among it (16 rows of 2048 x 8192: 256 KB of x
+// behind 128 KB of weights); while neighbouring lanes read different rows, that went at 37 bytes a ns.
+// With RH = 8, lanes 0-7 of 16 hold an operand's first 128 of k, lanes 8-15 its second, which a half_swap brings to the rows' own
+// lanes for the second product; rows 8-15 of the products are dropped.
 //
 // M8: RH = 8 and at most 8 rows of x, which then are read like the weights.  One product of the two registers as they are
-// holds the first step's result in its upper left quarter and the second's in its lower right one (the others mix the steps
+// holds the first half's result in its upper left quarter and the second's in its lower right one (the others mix the halves
 // and are dropped): half the x traffic, which is twice the weights' otherwise, half the matrix products and no exchange.
-template <int RT, int RH, int NW, int U, int EPI, bool XF, bool M8 = false>
+template <int RT, int RH, int NW, int EPI, bool XF, bool M8 = false>
 __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
   static_assert(!M8 || (RH == 8 && RT == 1 && EPI != EPI_GLU), "M8: one tile of 8 rows");
-  constexpr int LD = RH / 8;  // loads of a block
-  constexpr int XL = M8 ? 1 : 2;
+  constexpr int UK = RH == 16 ? 128 : 256;
+  constexpr int XL = RH == 16 || M8 ? 1 : 2;      // x: 128-deep (M8: 256-deep) parts of a block
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r16 = lane & 15, h = lane >> 4;
   const int n0 = blockIdx.x * (EPI == EPI_GLU ? RH : RH * RT);
+  // the lane's row among those of load 0 (load i: i rows on) and its bytes in a row of a block, of a tile of 16 and of 8 rows
+  const int row16 = lane & 12, row8 = lane & 4;
+  const unsigned in16 = 16 * ((lane & 3) + 4 * (lane >> 4)), in8 = in16 + 32 * (lane & 8);
 
   // rows past the end repeat the last one; their products are not stored
-  unsigned wo[RT][LD];
+  unsigned wo[RT][4], xo[4];
   const char* wb[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
@@ -82,75 +85,74 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
     const int base = min(first, a.N - 1);
     wb[rt] = reinterpret_cast<const char*>(a.W + (long long)(base + (EPI == EPI_GLU ? rt * a.N : 0)) * a.K);
 #pragma unroll
-    for (int l = 0; l < LD; ++l)
-      wo[rt][l] = (unsigned)((min(first + 8 * l + (r16 & 7), a.N - 1) - base) * a.K + 4 * (r16 & 8) + 8 * h) * 2;
+    for (int i = 0; i < 4; ++i)
+      wo[rt][i] = (unsigned)((min(first + (RH == 16 ? row16 : row8) + i, a.N - 1) - base) * a.K) * 2 + (RH == 16 ? in16 : in8);
   }
   const char* xb = reinterpret_cast<const char*>(a.x);
-  const unsigned xo = (unsigned)(min(M8 ? r16 & 7 : r16, a.M - 1) * a.ldx + (M8 ? 4 * (r16 & 8) : 0) + 8 * h) * 2;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) xo[i] = (unsigned)(min((M8 ? row8 : row16) + i, a.M - 1) * a.ldx) * 2 + (M8 ? in8 : in16);
 
   f32x4 acc[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) acc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  u32x4 w[2][U][RT][LD];
-  Pack8 xv[U][XL];
-  auto load_w = [&](int b, int blk) {
+  u32x4 w[2][RT][4], xv[2][XL][4];
+  // (x first: it comes from the L2, and is turned while the weights are on their way)
+  auto load = [&](int b, int blk) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int t = 0; t < XL; ++t)
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
+      for (int i = 0; i < 4; ++i) xv[b][t][i] = *reinterpret_cast<const u32x4*>(xb + 2 * UK * blk + 256 * t + xo[i]);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int l = 0; l < LD; ++l) w[b][u][rt][l] = ld_nt16(reinterpret_cast<const bf16*>(wb[rt] + 128 * (blk + u) + wo[rt][l]));
-  };
-  auto load_x = [&](int blk) {
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int t = 0; t < XL; ++t) xv[u][t].w = *reinterpret_cast<const u32x4*>(xb + 128 * (blk + u) + 64 * t + xo);
+      for (int i = 0; i < 4; ++i) w[b][rt][i] = ld_nt16(reinterpret_cast<const bf16*>(wb[rt] + 2 * UK * blk + wo[rt][i]));
   };
   auto multiply = [&](int b) {
+    Pack8 f[XL][4];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if constexpr (XF) {
+    for (int t = 0; t < XL; ++t) {
+      u32x4(&x)[4] = xv[b][t];
+      quad_transpose(x[0], x[1], x[2], x[3]);
 #pragma unroll
-        for (int t = 0; t < XL; ++t) relu_squared(xv[u][t]);
+      for (int i = 0; i < 4; ++i) {
+        f[t][i].w = x[i];
+        if constexpr (XF) relu_squared(f[t][i]);
       }
+    }
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        Pack8 f0, f1;
-        if constexpr (M8) {
-          f0.w = w[b][u][rt][0];
-          acc[rt] = mfma16(f0.v, xv[u][0].v, acc[rt]);
-          continue;
+    for (int rt = 0; rt < RT; ++rt) {
+      u32x4(&v)[4] = w[b][rt];
+      quad_transpose(v[0], v[1], v[2], v[3]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        Pack8 p;
+        p.w = v[i];
+        acc[rt] = mfma16(p.v, f[0][i].v, acc[rt]);
+        if constexpr (XL == 2) {
+          p.w = half_swap<0x3>(v[i], v[i]);
+          acc[rt] = mfma16(p.v, f[1][i].v, acc[rt]);
         }
-        const u32x4 lo = w[b][u][rt][0], hi = w[b][u][rt][LD - 1];
-        f0.w = LD == 2 ? half_swap<0xc>(lo, hi) : lo;
-        f1.w = half_swap<0x3>(hi, lo);
-        acc[rt] = mfma16(f0.v, xv[u][0].v, acc[rt]);
-        acc[rt] = mfma16(f1.v, xv[u][XL - 1].v, acc[rt]);
       }
     }
   };
-  // The loads of a chunk stand ahead of the products of the one before (the scheduler, left alone, moves them behind to
-  // save registers), and the last chunk's successor is itself, read again: behind a branch every wait would drain all
+  // The loads of a block stand ahead of the products of the one before (the scheduler, left alone, moves them behind to
+  // save registers), and the last block's successor is itself, read again: behind a branch every wait would drain all
   // loads.
-  const int per = (a.K >> 6) / NW, s0 = wid * per;
-  load_w(0, s0);
-  if (per <= U) {  // one chunk
-    load_x(s0);
-    __builtin_amdgcn_sched_barrier(0);
+  const int per = a.K / UK / NW, s0 = wid * per, last = s0 + per - 1;
+  load(0, s0);
+  __builtin_amdgcn_sched_barrier(0);
+  if (per == 1) {
     multiply(0);
   } else {
-    const int end = s0 + per, last = end - U;
-    for (int s = s0; s < end; s += 2 * U) {
-      load_x(s);
-      load_w(1, min(s + U, last));
+    for (int s = s0; s <= last; s += 2) {
+      load(1, min(s + 1, last));
       __builtin_amdgcn_sched_barrier(0);
       multiply(0);
-      if (s + U >= end) break;
+      if (s == last) break;
       __builtin_amdgcn_sched_barrier(0);
-      load_x(s + U);
-      load_w(0, min(s + 2 * U, last));
+      load(0, min(s + 2, last));
       __builtin_amdgcn_sched_barrier(0);
       multiply(1);
       __builtin_amdgcn_sched_barrier(0);
@@ -161,7 +163,6 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) red[wid][rt][lane] = acc[rt];
   __syncthreads();
-  if (wid >= (EPI == EPI_GLU ? 1 : RT)) return;
   auto sum = [&](int rt) {
     f32x4 v = red[0][rt][lane];
 #pragma unroll
@@ -172,7 +173,8 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
     }
     return v;
   };
-  store_rows<RH, EPI>(a, n0 + RH * wid, lane, sum(wid), EPI == EPI_GLU ? sum(RT - 1) : f32x4{});
+  for (int rt = wid; rt < (EPI == EPI_GLU ? 1 : RT); rt += NW)
+    store_rows<RH, EPI>(a, n0 + RH * rt, lane, sum(rt), EPI == EPI_GLU ? sum(RT - 1) : f32x4{});
 }
 
 // Many tiles: x stays in registers.  A workgroup's waves hold their shares of x (KB 64-deep blocks each, K = 64 NW KB) and walk
@@ -296,47 +298,86 @@ bool walk(const Args& a, hipStream_t s) {
   return true;
 }
 
-template <int RT, int RH, int NW, int U, int EPI, bool XF, bool M8 = false>
+template <int RT, int RH, int NW, int EPI, bool XF, bool M8>
 bool run(const Args& a, hipStream_t s) {
-  if (a.K % (64 * NW * U)) return false;
+  if (a.K % ((RH == 16 ? 128 : 256) * NW)) return false;
   constexpr int rows = EPI == EPI_GLU ? RH : RH * RT;
-  row_linear_kernel<RT, RH, NW, U, EPI, XF, M8><<<(a.N + rows - 1) / rows, NW * 64, 0, s>>>(a);
+  row_linear_kernel<RT, RH, NW, EPI, XF, M8><<<(a.N + rows - 1) / rows, NW * 64, 0, s>>>(a);
   return true;
 }
 
-// Tile by the number of outputs (us at 8 rows, other weights read in between; the library and the launch it replaces in
-// brackets):
-//   up to 3071: 8-row tiles, so that 2048 outputs are 256 workgroups (2048 x 2048 4.8, 16-row tiles 5.5 [8.5]).  M8, as one
-//   chunk where a wave's share is at most 8 blocks, else two blocks a chunk (x read twice / M8 at 1 and at 8 rows: 2048 x 4096
-//   6.5 / 5.6 and 7.8 / 6.8; 2048 x 8192 9.9 / 9.3 and 12.2 / 12.0, with the squared ReLU 11.5 / 10.6 and 12.8 / 12.3)
-//   the walk from 4097 on, where some workgroup has a second tile (8-row or 16-row tiles one by one / walk: 17440 x 2048 21.7 /
-//   16.5, 6144 x 2048 10.2 / 8.8, 32768 x 2048 to fp32 32.1 / 27.3, 28672 x 4096 50.7 / 38.6 = 6.1 TB/s; 4096 x 2048 7.8 / 7.6
-//   at 16 rows, 6.6 / 6.9 at 2), of the widths that are written out below; 1536 wide always (its other form has four waves of
-//   one block a chunk: 2048 outputs 5.5 / 4.6)
-//   16-row tiles between the two and for other widths (8-row tiles 3072 x 2048 at 16 rows 7.6, 6.6); two that share x from 24576
-// Gated pairs walk (8192 x 2048 18.1 / 13.9, 1024 x 2048 7.9 / 5.9, 14336 x 4096 50.6 / 39.4).  Four blocks a chunk where they are
-// all of a wave's share, else two (more bytes in flight cost waves); four waves where K does not divide by eight's.
+// With `waves` waves if these divide K's blocks, else with another number of them
+template <int RT, int RH, int EPI, bool XF, bool M8 = false>
+bool run_waves(const Args& a, int waves, hipStream_t s) {
+  switch (waves) {
+    case 8: if (run<RT, RH, 8, EPI, XF, M8>(a, s)) return true; break;
+    case 6: if (run<RT, RH, 6, EPI, XF, M8>(a, s)) return true; break;
+    case 2: if (run<RT, RH, 2, EPI, XF, M8>(a, s)) return true; break;
+    default: break;
+  }
+  if (run<RT, RH, 4, EPI, XF, M8>(a, s)) return true;
+  if constexpr (RH == 8)
+    if (run<RT, RH, 7, EPI, XF, M8>(a, s) || run<RT, RH, 6, EPI, XF, M8>(a, s) || run<RT, RH, 5, EPI, XF, M8>(a, s) ||
+        run<RT, RH, 3, EPI, XF, M8>(a, s))
+      return true;
+  return run<RT, RH, 2, EPI, XF, M8>(a, s);      // (RH 16: takes every K, an even number of blocks)
+}
+
+// Tile by the number of outputs (us; before / now: rows of neighbouring lanes / of lane quads, at 1, 8, 16 rows):
+//   up to 2048: 8-row tiles, so that 2048 outputs are 256 workgroups.  Up to 8 blocks of K a wave each, then four waves (2048 x
+//   2048 3.9, 4.5, 5.2 / 4.0, 4.2, 4.8; x 4096 5.5, 6.6, 8.4 / 5.4, 5.6, 7.2; x 14336 12.7, 15.7, 21.6 / 11.6, 12.4, 16.7); M8
+//   with eight where their shares would lie 4 KB apart (2048 x 8192, 8 rows: four 8.9, eight 8.8, before 10.3; x 16384 19.4,
+//   16.7, 18.1)
+//   from 2049 on 16-row tiles, RT of them sharing x: 1 or 2 while that is one round of the 256 CUs (2560 x 2048 4.9, 6.2, 7.7 /
+//   4.9, 5.0, 5.2 (8-row tiles 5.0, 5.2, 7.5); 4096 x 2048 6.4, 6.6, 7.5 / 5.2, 5.3, 5.6; 6144 x 2048 8.3, 8.5, 9.0 / 6.9, 6.9,
+//   7.1 (RT 1: 7.5, 7.7, 8.1); 8192 x 4096 13.7, 14.1, 15.5 / 13.3, 12.9, 12.7), then 2 or 3 by the rounds, whose cost is
+//   a tile's each and half a tile's for x (10240 x 2048 RT 2 / 3 10.8 / 9.3 [before 11.6]; 17440 16.0 / 14.7 [16.0]; 32768
+//   23.0 / 26 [27.1])
+//   one from 8192 deep on (8192 x 8192 23.8, 27.4, 33.0 / 23.4, 23.3, 25.6; RT 2 28.7, 29.1, 29.6)
+//   the walk where many tiles of few blocks, or of many, pass: 12288 x 1536 walk / tiles 8.5 / 8.8, 32768 x 1536 16.9 / 19.2 (8192 x
+//   1536 at 1, 16 rows 6.4, 7.5 / 6.9, 6.9), 28672 x 4096 37.9 / 40.2, against 16384 x 4096 23.6 / 22.6; 12288 x 3072 even
+// Waves of 16-row tiles: a block each up to 8 in one round (12288 x 1024, RT 3: eight 6.2, two 6.9); then four (two of RT 3), eight
+// from 8192 deep on (3000 x 8192 12.4 / 11.4).  Where more rounds cover a wait, one for 8 blocks, at least two (32768 x 2048 two /
+// four 23.0 / 23.7, 16384 x 4096 four / two 22.6 / 25; gated 8192 x 1024 two / eight 7.7 / 9.3), four for 4 blocks.
+// Gated pairs are two tiles of 16 outputs' (1024 x 1024 4.4, 4.8, 5.0 / 4.2, 4.3, 4.3; 8192 x 8192 56, 57, 59 / 45, 46, 47).  Of the
+// walk's widths they are where they come near whole rounds (8192 x 2048 12.7, 13.0, 13.6 / 12.6, 12.6, 12.8; 4096 x 4096 14.0 to
+// 15.9 / 12.2 to 12.5; but 4360 x 2048 9.9 / 10.7, 14336 x 4096 38.7 / 41.1), with few outputs for more than 8 rows (512 x 4096
+// at 1, 16 rows 8.6, 10.7 / 9.4, 9.5).
 template <int EPI, bool XF>
 bool by_shape(const Args& a, hipStream_t s) {
   if (a.K <= SMALL_K) {
     row_linear_small_kernel<EPI, XF><<<(a.N + 15) / 16, 64, 0, s>>>(a);
     return true;
   }
-  const bool walks = EPI == EPI_GLU ? a.K >= 2048 : a.N > 4096 || a.K == 1536;
-  if (walks && (walk<8, 3, EPI, XF>(a, s) || walk<16, 2, EPI, XF>(a, s) || walk<8, 6, EPI, XF>(a, s) || walk<8, 8, EPI, XF>(a, s)))
-    return true;
+  const int tiles = (a.N + 15) / 16, blocks = a.K / 128;
+  bool walks;
   if constexpr (EPI == EPI_GLU) {
-    return run<2, 16, 4, 4, EPI, XF>(a, s) || run<2, 16, 4, 1, EPI, XF>(a, s);
+    const bool near = (tiles > 128 && tiles <= 256) || (tiles >= 384 && tiles <= 512) || (tiles <= 128 && a.M > 8);
+    walks = a.K == 3072 || ((a.K == 2048 || a.K == 4096) && !near);
   } else {
-    const int per = a.K / (64 * 8);  // blocks of each of eight waves
-    if (a.N < 3072 && a.M <= 8 &&
-        ((per <= 4 && run<1, 8, 8, 4, EPI, XF, true>(a, s)) || (per <= 8 && run<1, 8, 8, 8, EPI, XF, true>(a, s)) ||
-         run<1, 8, 8, 2, EPI, XF, true>(a, s)))
-      return true;
-    const bool whole = per <= 4;
-    if (a.N < 3072 && ((whole && run<1, 8, 8, 4, EPI, XF>(a, s)) || run<1, 8, 8, 2, EPI, XF>(a, s))) return true;
-    if (a.N >= 24576 && run<2, 16, 4, 4, EPI, XF>(a, s)) return true;
-    return (whole && run<1, 16, 8, 4, EPI, XF>(a, s)) || run<1, 16, 8, 2, EPI, XF>(a, s) || run<1, 16, 4, 1, EPI, XF>(a, s);
+    walks = ((a.K == 1536 || a.K == 3072) && a.N > 8192) || (a.K == 1536 && a.N > 4096 && a.M <= 4) || (a.K == 4096 && a.N > 16384);
+  }
+  if (walks && (walk<8, 3, EPI, XF>(a, s) || walk<8, 6, EPI, XF>(a, s) || walk<8, 8, EPI, XF>(a, s))) return true;
+  auto waves = [&](int rt, int wgs) {
+    const bool one = wgs <= 256;
+    if (blocks <= (one ? 8 : 4)) return blocks;
+    if (blocks >= 64) return 8;
+    return one && rt < 3 ? 4 : blocks <= 20 ? 2 : 4;
+  };
+  if constexpr (EPI == EPI_GLU) {
+    if (walks && walk<16, 2, EPI, XF>(a, s)) return true;
+    return run_waves<2, 16, EPI, XF>(a, waves(2, tiles), s);
+  } else {
+    if (a.N <= 2048 && a.K % 256 == 0) {
+      const int deep = a.K / 256;
+      if (a.M <= 8 ? run_waves<1, 8, EPI, XF, true>(a, deep <= 8 ? deep : deep % 32 ? 4 : 8, s)
+                   : run_waves<1, 8, EPI, XF>(a, deep <= 8 ? deep : 4, s))
+        return true;
+    }
+    const int two = (tiles + 1) / 2, three = (tiles + 2) / 3;
+    if (tiles <= 256 || blocks >= 64) return run_waves<1, 16, EPI, XF>(a, waves(1, tiles), s);
+    if (two > 256 && 7 * ((three + 255) / 256) < 5 * ((two + 255) / 256)) return run_waves<3, 16, EPI, XF>(a, waves(3, three), s);
+    return run_waves<2, 16, EPI, XF>(a, waves(2, two), s);
   }
 }
 

@@ -53,6 +53,17 @@ def test_row_linear_tiles_in_turn(gpu, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,K", [(12, 512), (2044, 768), (2048, 1024), (60, 1280), (28, 1536), (36, 1792), (2048, 2816), (20, 8192),
+                                 (2052, 512), (4096, 768), (4092, 1280), (4100, 1024), (8192, 512), (8188, 2816), (8196, 768), (12292, 512),
+                                 (17444, 1280), (24572, 512), (2052, 8192)])
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+def test_row_linear_waves_and_tiles(gpu, M, N, K):
+    """Every number of waves, 8-row tiles up to 2048 outputs, then one, two and three 16-row tiles a workgroup, at the lines between
+    them with cut last tiles, one block of K a wave, an odd and an even number of them."""
+    test_row_linear(gpu, M, N, K)
+
+
+@pytest.mark.gpu
 def test_linear_accepts_every_form(gpu):
     """Strides, types, sizes and alignments that the kernel does not take stay with the library and give the same product."""
     g = torch.Generator(device=gpu).manual_seed(3)
