@@ -28,11 +28,13 @@
 //    G_j), both exponents <= 0, and is a matrix product again.
 //    delta_chunk_scan_kernel (grid (P / 64, heads, runs)) then walks a run's chunks with
 //        R = V - Kt S,   U = T R,   O = Qt S + Aqk U,   S <- D S + Kh^T U
-//    as fp32 matrix products (v_mfma_f32_16x16x4_f32).  A wave owns 16 value columns and ALL of N: its state stays in
+//    as fp32 matrix products (v_mfma_f32_16x16x4_f32; in bf16 parts up to 128 key channels of the bf16 model).  A wave owns 16 value columns and ALL of N: its state stays in
 //    accumulator registers for the whole run, and since an accumulator's rows are 4 (lane / 16) + r and a B operand's
 //    contraction index is lane / 16, register r of the state IS the B operand of a step that contracts over the rows
 //    4 g + r (the A operand is read in the same order: one 16-byte LDS read feeds four steps).  The same holds for R and U.
 //    Four waves multiply, four others stage the next chunk (loads, exponentials, LDS) on the same SIMDs meanwhile.
+#include "attn_tiles.h"
+#include "bf16_parts.h"
 #include "common.h"
 #include "hybrid_launchers.h"
 
@@ -630,6 +632,297 @@ __global__ __launch_bounds__(128 * MW) void delta_chunk_scan_kernel(DeltaRuleArg
   }
 }
 
+// The same walk on v_mfma_f32_16x16x32_bf16, for up to 128 key channels in the bf16 model: the fp32 products were what bound it (8 x
+// 128 x 256: 224 of 32 cycles a chunk and wave).  State, keys, queries and corrections go in as three bf16 parts, six terms a
+// product; T R and Aqk U, a tenth, stay fp32 products, their matrices straight from the scratch, a chunk ahead.
+// A B operand's contraction index is 8 (lane / 16) + j and an accumulator's rows 4 (lane / 16) + r: with the contraction in the
+// order j < 4: 4 g + j, else 16 + 4 g + j - 4, two accumulator tiles are a B operand.  Keys and queries lie in LDS in that order
+// along a row, so that an A operand is one 16-byte read; the last product takes the keys' tokens as its contraction, by LDS transpose reads.
+// One decay per head: rows and corrections are scaled behind the products (E = 2^(G_i), W = 2^(G_C - G_i)) and the keys serve both;
+// decays per channel: k 2^G, q 2^G and k 2^(G_C - G) are staged.  NB: 32-channel blocks (N <= 32 NB, N a multiple of 8).
+// What is left is the chain of a chunk, its products a third (4000 tokens in one run, us a chunk: 2.5; without the products of the
+// state 1.8, without staging 2.4).  256 registers a lane: with more allowed the compiler keeps a part in AGPRs (348 -> 396).
+// Prep and walk, fp32 products / parts, 8 x 128 x 256, us: one decay per head 3 runs of 510 91 / 62, 8 of 1000 222 / 161, one of
+// 4000 529 / 348, of 100 35 / 26; per channel 108 / 87, 290 / 217, 567 / 420, 45 / 38.  Error against 64 bits no larger (rms of the outputs
+// 2.2e-7 / 2.1e-7 at 510 rows, 3.8e-7 / 3.2e-7 with slow decays).
+template <bool CHANNEL, int NB, int MW>
+__global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(DeltaRuleArgs a) {
+  constexpr int ST = 64 * MW;                            // staging threads
+  constexpr int NP = 32 * NB, LQ = NP + 8;               // LQ: bf16 pitch of a [C][NP] matrix
+  constexpr int PART = C * LQ, oQ = 3 * PART, oH = CHANNEL ? 6 * PART : 0, MATS = CHANNEL ? 3 : 2;
+  constexpr int FS = CHANNEL ? NP : 2 * C + 4;           // floats: 2^(G_C) per channel, or E | W | 2^(G_C)
+  constexpr int STAGE = MATS * 3 * PART * 2 + FS * 4;    // bytes
+  static_assert(STAGE % 16 == 0 && 2 * STAGE <= 160 * 1024, "two stages");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int N = a.N, P = a.P;
+  const int h = blockIdx.y, run = blockIdx.z;
+  const int s0 = a.cu_q[run], s1 = a.cu_q[run + 1];
+  if (s1 <= s0) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int chunks = (s1 - s0 + C - 1) / C;
+  const int wc = ws_cols(CHANNEL, N);
+  const long long wrow = (long long)a.H * wc;
+  const float* ws = a.ws + (long long)s0 * wrow + (long long)h * wc;
+  if (wave >= MW) {
+    // ---- staging waves: thread (token tt0, 8 channels from c8), TSTEP tokens apart -----------------------------------
+    constexpr int GR = NP / 8, TSTEP = ST / GR, PASS = (C + TSTEP - 1) / TSTEP;
+    const int tid = threadIdx.x - ST, c8 = 8 * (tid % GR), tt0 = tid / GR;
+    const bool nin = c8 < N && tt0 < C;
+    const int gn = a.G * N;
+    const float* k = a.k + (long long)s0 * gn + (h / a.hpg) * N;
+    const float* q = a.q + (long long)s0 * gn + (h / a.hpg) * N;
+    const int at = 32 * (c8 / 32) + 8 * (c8 % 16 / 4) + 4 * (c8 % 32 / 16);      // the 4 from c8; the 4 behind them 8 on
+    int ko[PASS], go[PASS];
+#pragma unroll
+    for (int u = 0; u < PASS; ++u) {
+      const int tt = tt0 + TSTEP * u;
+      ko[u] = nin ? 4 * (tt * gn + c8) : NO_PLACE;
+      go[u] = nin ? 4 * (tt * (int)wrow + 2 * C + c8) : NO_PLACE;
+    }
+    f32x4 rk[PASS][2], rq[PASS][2], rg[CHANNEL ? PASS : 1][2], gl[2];
+    float g1 = 0.f, glast = 0.f;
+    auto fetch = [&](int c) {
+      const int t0 = c * C, nt = min(C, s1 - s0 - t0);
+      const __amdgpu_buffer_rsrc_t bk = chunk_rows(k + (long long)t0 * gn, 4LL * gn, nt, 4 * N);
+      const __amdgpu_buffer_rsrc_t bq = chunk_rows(q + (long long)t0 * gn, 4LL * gn, nt, 4 * N);
+      const __amdgpu_buffer_rsrc_t bg = chunk_rows(ws + t0 * wrow, 4 * wrow, nt, 4 * wc);
+#pragma unroll
+      for (int u = 0; u < PASS; ++u)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          rk[u][i] = row16f(bk, ko[u] + (nin ? 16 * i : 0));
+          rq[u][i] = row16f(bq, ko[u] + (nin ? 16 * i : 0));
+          if constexpr (CHANNEL) rg[u][i] = row16f(bg, go[u] + (nin ? 16 * i : 0));
+        }
+      const float* last = ws + (t0 + nt - 1) * wrow + 2 * C;
+      if constexpr (CHANNEL) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) gl[i] = nin ? lds4(last + c8 + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+      } else {
+        g1 = tid < C ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(bg, 4 * (tid * (int)wrow + 2 * C), 0, 0)) : 0.f;
+        glast = last[0];
+      }
+    };
+    auto put = [&](bf16* m, int tt, f32x4 lo, f32x4 hi) {
+      const Parts x = split(lo, hi);
+      auto half = [&](int part, bf16x8 v) {
+        Pack8 w;
+        w.v = v;
+        bf16* to = m + part * PART + tt * LQ + at;
+        *reinterpret_cast<uint2*>(to) = make_uint2(w.u.x, w.u.y);
+        *reinterpret_cast<uint2*>(to + 8) = make_uint2(w.u.z, w.u.w);
+      };
+      half(0, x.h), half(1, x.m), half(2, x.l);
+    };
+    auto stash = [&](int c) {
+      bf16* st = reinterpret_cast<bf16*>(smem + (c & 1) * STAGE);
+      float* fs = reinterpret_cast<float*>(st + MATS * 3 * PART);
+#pragma unroll
+      for (int u = 0; u < PASS; ++u) {
+        const int tt = tt0 + TSTEP * u;
+        if (tt >= C) break;
+        if constexpr (CHANNEL) {
+          f32x4 e[2], w[2];
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              e[i][r] = __builtin_amdgcn_exp2f(rg[u][i][r]);
+              w[i][r] = __builtin_amdgcn_exp2f(fminf(gl[i][r] - rg[u][i][r], 0.f));      // (rows past the run's end: k = 0)
+            }
+          put(st, tt, rk[u][0] * e[0], rk[u][1] * e[1]);
+          put(st + oQ, tt, rq[u][0] * e[0], rq[u][1] * e[1]);
+          put(st + oH, tt, rk[u][0] * w[0], rk[u][1] * w[1]);
+        } else {
+          put(st, tt, rk[u][0], rk[u][1]);
+          put(st + oQ, tt, rq[u][0], rq[u][1]);
+        }
+      }
+      if constexpr (CHANNEL) {
+        if (tt0 == 0)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) fs[c8 + 4 * i + r] = __builtin_amdgcn_exp2f(gl[i][r]);
+      } else if (tid < C) {
+        fs[tid] = __builtin_amdgcn_exp2f(g1);
+        fs[C + tid] = __builtin_amdgcn_exp2f(fminf(glast - g1, 0.f));
+        if (tid == 0) fs[2 * C] = __builtin_amdgcn_exp2f(glast);
+      }
+    };
+    fetch(0);
+    stash(0);
+    if (chunks > 1) fetch(1);
+    __syncthreads();                           // chunk 0 is staged
+    for (int c = 0; c < chunks; ++c) {
+      if (c + 1 < chunks) {
+        stash(c + 1);
+        if (c + 2 < chunks) fetch(c + 2);
+      }
+      __syncthreads();                         // chunk c + 1 is staged, chunk c has been read
+    }
+    return;
+  }
+  // ---- multiplying waves -----------------------------------------------------------------------------------------
+  const int col = lane & 15, g = lane >> 4;
+  const int p = blockIdx.x * 16 * MW + wave * 16 + col;
+  const bool pin = p < P;
+  const int pr = a.prev_row[s0];
+  const int sv = a.save_slot[s1 - 1];
+  const long long hp = (long long)a.H * P;
+  const bf16* v = reinterpret_cast<const bf16*>(a.v) + (long long)s0 * hp + (long long)h * P;
+  float* out = a.out + (long long)s0 * hp + (long long)h * P;
+  const int vo = 2 * (4 * g * (int)hp + p), oo = 4 * (4 * g * (int)hp + p);      // (launch_delta_rule bounds H P)
+  float vn[8];
+  auto fetch_v = [&](int c) {
+    const __amdgpu_buffer_rsrc_t bv = chunk_rows(v + (long long)c * C * hp, 2 * hp, min(C, s1 - s0 - c * C), 2 * P);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      vn[i] = (float)__builtin_bit_cast(bf16, __builtin_amdgcn_raw_buffer_load_b16(bv, pin ? vo + (16 * (i >> 2) + (i & 3)) * 2 * (int)hp : NO_PLACE, 0, 0));
+  };
+  // T and Aqk: rows col, 16 + col; a row's 4 from 4 g, 16 + 4 g (rows past the run's end and what lies above the diagonal: 0)
+  f32x4 m[6];
+  auto fetch_m = [&](int c) {
+    const __amdgpu_buffer_rsrc_t bm = chunk_rows(ws + (long long)c * C * wrow, 4 * wrow, min(C, s1 - s0 - c * C), 8 * C);
+    const int o = 4 * (col * (int)wrow + 4 * g), o16 = o + 64 * (int)wrow;
+    m[0] = row16f(bm, o), m[1] = row16f(bm, o16), m[2] = row16f(bm, o16 + 64);
+    m[3] = row16f(bm, o + 4 * C), m[4] = row16f(bm, o16 + 4 * C), m[5] = row16f(bm, o16 + 4 * C + 64);
+  };
+  f32x4 S[2 * NB];
+  const bool old = pr <= -2 && pin;
+  const float* st0 = a.state + (old ? (long long)(-(pr + 2)) * a.state_stride + (long long)h * N * P + p : 0);
+#pragma unroll
+  for (int t = 0; t < 2 * NB; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int n = 16 * t + 4 * g + r;
+      S[t][r] = old && n < N ? st0[(long long)n * P] : 0.f;
+    }
+  fetch_v(0);
+  fetch_m(0);
+  __syncthreads();                             // chunk 0 is staged
+  for (int c = 0; c < chunks; ++c) {
+    const bf16* st = reinterpret_cast<const bf16*>(smem + (c & 1) * STAGE);
+    const float* fs = reinterpret_cast<const float*>(st + MATS * 3 * PART);
+    const bf16* Kr = st + col * LQ + 8 * g;
+    // (one multiplying wave a SIMD: LDS reads stand a step ahead of the products that take them)
+    bf16x8 f[2][2][3][2];                      // of a block's turn: keys, queries; parts; row tiles
+    auto load = [&](int b) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int part = 0; part < 3; ++part)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            f[b & 1][x][part][i] = *reinterpret_cast<const bf16x8*>(Kr + x * oQ + part * PART + 16 * i * LQ + 32 * b);
+    };
+    load(0);
+    const f32x4 V0 = {vn[0], vn[1], vn[2], vn[3]}, V1 = {vn[4], vn[5], vn[6], vn[7]};
+    if (c + 1 < chunks) fetch_v(c + 1);
+    f32x4 e[2], w[2];                          // one decay per head: of the rows 4 g + r, 16 + 4 g + r
+    float dh = 1.f;
+    if constexpr (!CHANNEL) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) e[i] = lds4(fs + 16 * i + 4 * g), w[i] = lds4(fs + C + 16 * i + 4 * g);
+      dh = fs[2 * C];
+    }
+    f32x4 K[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, O[2] = {K[0], K[0]};
+    Parts s = split(S[0], S[1]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if (b + 1 < NB) load(b + 1);
+      f32x4 d[2];
+      if constexpr (CHANNEL) d[0] = lds4(fs + 32 * b + 4 * g), d[1] = lds4(fs + 32 * b + 16 + 4 * g);
+      Parts next = s;
+      if (b + 1 < NB) next = split(S[2 * b + 2], S[2 * b + 3]);
+#pragma unroll
+      for (int term = 0; term < 6; ++term) {   // the smallest terms first
+        constexpr int mine[6] = {0, 2, 1, 1, 0, 0};
+        const bf16x8 sp = term == 0 ? s.l : term == 2 || term == 4 ? s.m : s.h;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          K[i] = mfma16(f[b & 1][0][mine[term]][i], sp, K[i]);
+          O[i] = mfma16(f[b & 1][1][mine[term]][i], sp, O[i]);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if constexpr (CHANNEL) S[2 * b + i] *= d[i];
+        else S[2 * b + i] *= dh;
+      }
+      s = next;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // keys of the last product: 16 channels of the tokens 4 g .. + 3 and 16 + 4 g .. + 3
+    const char* Ht = reinterpret_cast<const char*>(st + oH + (4 * g + (col >> 2)) * LQ) + 16 * (col & 3);
+    bf16x8 kh[2][3];
+    auto load_h = [&](int t) {
+#pragma unroll
+      for (int part = 0; part < 3; ++part) {
+        const char* at = Ht + part * PART * 2 + 64 * (t >> 1) + 8 * (t & 1);
+        Pack8 x;
+        const uint2 lo = read_tr(at), hi = read_tr(at + 32 * LQ);
+        x.u = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        kh[t & 1][part] = x.v;
+      }
+    };
+    load_h(0);
+    if constexpr (!CHANNEL) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) K[i] *= e[i], O[i] *= e[i];
+    }
+    const f32x4 R0 = V0 - K[0], R1 = V1 - K[1];
+    f32x4 U0 = {0.f, 0.f, 0.f, 0.f}, U1 = U0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      U0 = mfma4(m[0][r], R0[r], U0);
+      U1 = mfma4(m[1][r], R0[r], U1);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) U1 = mfma4(m[2][r], R1[r], U1);
+    const Parts u = CHANNEL ? split(U0, U1) : split(U0 * w[0], U1 * w[1]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      O[0] = mfma4(m[3][r], U0[r], O[0]);
+      O[1] = mfma4(m[4][r], U0[r], O[1]);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) O[1] = mfma4(m[5][r], U1[r], O[1]);
+    if (c + 1 < chunks) fetch_m(c + 1);
+#pragma unroll
+    for (int t = 0; t < 2 * NB; ++t) {
+      if (t + 1 < 2 * NB) load_h(t + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      const bf16x8(&x)[3] = kh[t & 1];
+      S[t] = mfma16(x[0], u.l, S[t]);
+      S[t] = mfma16(x[2], u.h, S[t]);
+      S[t] = mfma16(x[1], u.m, S[t]);
+      S[t] = mfma16(x[1], u.h, S[t]);
+      S[t] = mfma16(x[0], u.m, S[t]);
+      S[t] = mfma16(x[0], u.h, S[t]);
+    }
+    const int nt = min(C, s1 - s0 - c * C);
+    const __amdgpu_buffer_rsrc_t bo = chunk_rows(out + (long long)c * C * hp, 4 * hp, nt, 4 * P);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(O[i][r]), bo, pin ? oo + (16 * i + r) * 4 * (int)hp : NO_PLACE, 0, 0);
+    __syncthreads();                           // chunk c + 1 is staged, chunk c has been read
+  }
+  if (sv >= 0 && pin) {
+    float* so = a.state + (long long)sv * a.state_stride + (long long)h * N * P + p;
+#pragma unroll
+    for (int t = 0; t < 2 * NB; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int n = 16 * t + 4 * g + r;
+        if (n < N) so[(long long)n * P] = S[t][r];
+      }
+  }
+}
+
 void raise_lds(const void* f) { hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); }
 
 template <typename T, bool CHANNEL, int NPL, int CH, int SLICES>
@@ -672,6 +965,14 @@ void launch_scan(const DeltaRuleArgs& a, hipStream_t s) {
   delta_chunk_scan_kernel<T, CHANNEL, NN, NBUF, MW><<<grid, 128 * MW, (size_t)NBUF * STAGE * sizeof(float), s>>>(a);
 }
 
+template <bool CHANNEL, int NB, int MW>
+void launch_parts(const DeltaRuleArgs& a, hipStream_t s) {
+  constexpr int lds = 2 * ((CHANNEL ? 9 : 6) * C * (32 * NB + 8) * 2 + (CHANNEL ? 32 * NB : 2 * C + 4) * 4);
+  static const bool raised = (raise_lds(reinterpret_cast<const void*>(&delta_chunk_parts_kernel<CHANNEL, NB, MW>)), true);
+  (void)raised;
+  delta_chunk_parts_kernel<CHANNEL, NB, MW><<<dim3((a.P + 16 * MW - 1) / (16 * MW), a.H, a.runs), 128 * MW, lds, s>>>(a);
+}
+
 template <typename T, bool CHANNEL, int NN>
 void launch_chunks(const DeltaRuleArgs& a, hipStream_t s) {
   constexpr int LD = 16 * NN + 4;
@@ -681,9 +982,17 @@ void launch_chunks(const DeltaRuleArgs& a, hipStream_t s) {
   delta_chunk_prep_kernel<CHANNEL, NN><<<dim3(2 * a.ntiles, a.H), NT, prep, s>>>(a);
   // 32 columns a workgroup while those are at most one a CU (256) and runs are long enough that the first chunk's staging, which
   // half as many waves do, is not what counts; else 64 (8 heads x 128 x 256, us with 32 / with 64 columns: 3 runs of 512 tokens
-  // 76 / 88, 5 runs 146 / 87, one of 4000 498 / 639, 3 runs of 200 40.7 / 40.3, of 60 17.6 / 14.9)
+  // 76 / 88, 5 runs 146 / 87, one of 4000 498 / 639, 3 runs of 200 40.7 / 40.3, of 60 17.6 / 14.9; in parts, prep included, 5 runs of
+  // 512 109 / 71, 8 of 20 25 / 20, 3 of 200 37.6 / 38.1)
+  const bool narrow = NN <= 8 && (long long)((a.P + 31) / 32) * a.H * a.runs <= 256 && a.T >= 8LL * C * a.runs;
+  if constexpr (sizeof(T) == 2 && NN <= 8) {
+    const auto a16 = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+    // (whole groups of 8 channels in 16-byte loads; a chunk's rows at 32-bit offsets)
+    if (a.N % 8 == 0 && a16(a.q) && a16(a.k) && a16(a.ws) && (long long)a.H * (2 * C + a.N) <= 1 << 22 && (long long)a.G * a.N <= 1 << 22)
+      return narrow ? launch_parts<CHANNEL, (NN + 1) / 2, 2>(a, s) : launch_parts<CHANNEL, (NN + 1) / 2, 4>(a, s);
+  }
   if constexpr (NN <= 8) {
-    if ((long long)((a.P + 31) / 32) * a.H * a.runs <= 256 && a.T >= 8LL * C * a.runs) return launch_scan<T, CHANNEL, NN, 2>(a, s);
+    if (narrow) return launch_scan<T, CHANNEL, NN, 2>(a, s);
   }
   launch_scan<T, CHANNEL, NN, 4>(a, s);
 }

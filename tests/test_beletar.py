@@ -690,6 +690,51 @@ def test_delta_rule_long_runs(channel, shape):
     assert torch.equal(state[1].cpu(), start)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("strong", [False, True])
+@pytest.mark.parametrize("rows", [(65, 31), (300, 257), (1, 32)])
+@pytest.mark.parametrize("shape", [(3, 3, 8, 16), (2, 1, 24, 40), (1, 1, 32, 70), (2, 1, 40, 16), (2, 2, 64, 80), (1, 1, 72, 33),
+                                   (2, 1, 104, 32), (1, 1, 128, 96), (1, 1, 12, 20), (1, 1, 136, 16)])
+def test_delta_rule_in_parts(channel, strong, rows, shape):
+    """The bf16 model's chunk walk (operands of three bf16 parts): every number of 32-channel blocks, cut ones, columns that fill no
+    wave, chunks of one row and cut ones, 32 and 64 columns a workgroup, a state carried in; key channels that it leaves to the
+    fp32 products.  Bounds as for those: rounding adds up with the root of the rows, 6.5e-6 at 300 of unit values.  Decays inside a
+    chunk are powers of differences of its running sum in fp32: where that sum reaches s, a weight errs by 2^-24 s at either
+    end of the difference, which strong decays (s of a few hundred) show."""
+    H, G, N, P = shape
+    na, nb = rows
+    if strong and nb < 64:
+        pytest.skip("the strong case places its tokens past row 40")
+    say("op delta_rule parts", channel, strong, rows, shape)
+    qa, ka, va, dza, dtb, A, bza, lga, _, _ = _delta_case(channel, H, G, N, P, na, 1, strong)
+    qb, kb, vb, dzb, _, _, bzb, _, _, _ = _delta_case(channel, H, G, N, P, nb, 2, strong)
+    va, vb = va.bfloat16(), vb.bfloat16()
+    lgb = -torch.exp(A.double())[None, :, None] * O.softplus((dzb + dtb).double().view(nb, H, -1)).expand(nb, H, N)
+    start = 0.1 * torch.randn(H, N, P)
+    want_a, Sa = O.delta_rule(qa.double(), ka.double(), va.double(), lga, torch.sigmoid(bza.double()))
+    want_b, Sb = O.delta_rule(qb.double(), kb.double(), vb.double(), lgb, torch.sigmoid(bzb.double()), start.double())
+    sums = max(float(x[i:i + 32].sum(0).abs().max()) for x in (lga, lgb) for i in range(0, x.shape[0], 32))
+    room = 2 * 2.0 ** -24 * sums
+    prev = torch.tensor([-1] + list(range(na - 1)) + [-3] + list(range(na, na + nb - 1)), dtype=torch.int32)      # (-3: slot 1)
+    save = torch.full((na + nb,), -1, dtype=torch.int32)
+    save[na - 1], save[-1] = 0, 2
+    tiles = torch.tensor([[0, r] for r in range(0, na, 64)] + [[1, r] for r in range(0, nb, 64)], dtype=torch.int32)
+    state = torch.full((3, H, N, P), 1e4)
+    state[1] = start
+    y = torch.full((na + nb + 1, H, P), 1e4)
+    ws = torch.full((na + nb, H, ops.delta_ws_cols(channel, N)), float("nan"))
+    cat = [torch.cat([x, z]) for x, z in ((qa, qb), (ka, kb), (va, vb), (dza, dzb), (bza, bzb))]
+    q, k, v, dz, bz, y, ws, prev, save, cu, tiles, state, dtb, A = _dev(
+        "cuda", *cat, y, ws, prev, save, torch.tensor([0, na, na + nb], dtype=torch.int32), tiles, state, dtb, A)
+    assert ops.delta_rule(channel, q, k, v, dz, dtb, A, bz, state, cu, prev, save, 2, y[:na + nb], tiles, ws) == 0
+    for got, want in ((y[:na], want_a), (y[na:na + nb], want_b)):
+        assert float((got.cpu().double() - want).abs().max()) < (6.5e-6 + room) * max(1.0, float(want.abs().max()))
+    for got, want in ((state[0], Sa), (state[2], Sb)):
+        assert float((got.cpu().double() - want).abs().max()) < (3.2e-5 + room) * max(1.0, float(want.abs().max()))
+    assert torch.equal(state[1].cpu(), start) and float(y[na + nb].min()) == 1e4
+
+
 @pytest.mark.parametrize("device,impl", FORMS)
 @pytest.mark.parametrize("channel", [False, True])
 def test_delta_rule_strong_decays_and_one_key_again(device, impl, channel):
