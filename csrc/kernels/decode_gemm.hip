@@ -872,10 +872,11 @@ void launch_decode_gemm(int epi, const bf16* x, const bf16* W, int M, int N, int
     case DECODE_EPI_QKV: launch_epi<DECODE_EPI_QKV>(x, W, M, N, K, e, s); break;
     case DECODE_EPI_RESID: launch_epi<DECODE_EPI_RESID>(x, W, M, N, K, e, s); break;
     case DECODE_EPI_SWIGLU: launch_epi<DECODE_EPI_SWIGLU>(x, W, M, N, K, e, s); break;
-    default: launch_epi<DECODE_EPI_ARGMAX>(x, W, M, N, K, e, s); break;
+    default:
+      if (g_variant >= 0 || !launch_mgemm_argmax(x, W, M, N, K, e, s)) launch_epi<DECODE_EPI_ARGMAX>(x, W, M, N, K, e, s);
+      break;
   }
 }
-
 
 bool launch_decode_gemm_xar(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEpi& e, hipStream_t s) {
   if (M < 1 || M > 64 || N % 16 || N / 16 >= XG_KEYS_WG) return false;

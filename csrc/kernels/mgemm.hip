@@ -105,13 +105,14 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
     const int row = min(C::NX * wid + i, 2 * MT - 1) * 8 + (lane >> 3);
     vx[i] = row * K * 2 + 16 * ((lane & 7) ^ ((row >> 1) & 7)) + k0 * 2;
   }
-  // ---- weight DMA: block (tile, 2c + s) -> its 1 KB LDS block, lane-linear; wave w fills blocks NB w + i of the chunk's 2 CT
-  const __amdgpu_buffer_rsrc_t rw = mg_rsrc(W, (long long)N * K * 2);
+  // ---- weight DMA: block (tile, 2c + s) -> its 1 KB LDS block, lane-linear; wave w fills blocks NB w + i of the chunk's 2 CT.
+  // Tiles past N (EPI_ARGMAX) read zeros (buffer range)
+  const __amdgpu_buffer_rsrc_t rw = mg_rsrc(W + (long long)blockIdx.x * CT * 16 * K, (long long)min(16 * CT, N - (int)blockIdx.x * CT * 16) * K * 2);
   int vw[C::NB];
 #pragma unroll
   for (int i = 0; i < C::NB; ++i) {
     const int b = min(C::NB * wid + i, 2 * CT - 1);
-    vw[i] = ((blockIdx.x * CT + (b >> 1)) * (K / 32) + k0 / 32 + (b & 1)) * 1024 + lane * 16;
+    vw[i] = ((b >> 1) * (K / 32) + k0 / 32 + (b & 1)) * 1024 + lane * 16;
   }
 
   auto issue = [&](int c, int slot) {
@@ -135,11 +136,17 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
   const int xo1 = fr * 128 + 16 * ((4 + (lane >> 4)) ^ ((fr >> 1) & 7));
   const int wo_l = C::XB + lane * 16;
 
-  f32x4 acc[RW][MT];
+  // EPI_ARGMAX sums all of K here, in parts of 256, of a short K 128: longer chains lose bits (K = 2048, 32768 outputs: one chain
+  // 1.9e-7 of the result off, parts of 512 1.3e-7, 256 1.0e-7)
+  constexpr bool PARTS = EPI == DECODE_EPI_ARGMAX;
+  f32x4 acc[RW][MT], total[PARTS ? RW : 1][PARTS ? MT : 1];
 #pragma unroll
   for (int rt = 0; rt < RW; ++rt)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int mt = 0; mt < MT; ++mt) {
+      acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (PARTS) total[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 
   struct Frag {
     bf16x8 w[RW], x[MT];
@@ -220,6 +227,7 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   step(f0, 0, 0, f1, true, false);
+  const int part = K < 2048 ? 1 : 3;
   int slot = 0;
   for (int c = 0; c + 1 < nch; ++c) {
     const int after = slot == C::SLOTS - 1 ? 0 : slot + 1;
@@ -230,6 +238,15 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
     asm volatile("" ::: "memory");
     if (c + C::SLOTS < nch) issue(c + C::SLOTS, slot);
     step(f0, after, 0, f1, true, true);
+    if (PARTS && (c & part) == part) {
+#pragma unroll
+      for (int rt = 0; rt < (PARTS ? RW : 0); ++rt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          total[rt][mt] += acc[rt][mt];
+          acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
     slot = after;
   }
   step(f1, slot, 1, f0, true, true);
@@ -288,12 +305,14 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
 #pragma unroll
     for (int rt = 0; rt < RW; ++rt) {
       if (CT % RW && wid * RW + rt >= CT) continue;
+      if (EPI == DECODE_EPI_ARGMAX && 16 * (tile0 + rt) >= N) continue;
       const int n = 16 * (tile0 + rt) + 4 * (lane >> 4);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         const int m = 16 * mt + (lane & 15);
         const bool mok = m < M;
         f32x4 v = acc[rt][mt];
+        if constexpr (PARTS) v += total[rt][mt];
         if (S > 1) {
           v = f32x4{0.f, 0.f, 0.f, 0.f};
           if (mok)
@@ -370,7 +389,34 @@ void launch_epi_m(const bf16* x, const bf16* W, float* y, int M, int N, int K, i
   launch_mt<16, EPI>(x, W, y, M, N, K, S, rw, e, counters, s);
 }
 
+template <int CT>
+void launch_argmax(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEpi& e, hipStream_t s) {
+  const int groups = (N + 16 * CT - 1) / (16 * CT);
+#define MG_ARGMAX(t) \
+  mgemm_kernel<t, CT, DECODE_EPI_ARGMAX, 4><<<groups, 256, 0, s>>>(x, W, nullptr, M, N, K, K, e, nullptr, g_mgemm_nt)
+  if (M <= 32) MG_ARGMAX(2);
+  else if (M <= 48) MG_ARGMAX(3);
+  else MG_ARGMAX(4);
+#undef MG_ARGMAX
+}
+
 }  // namespace
+
+// Many outputs of 17 to 64 rows (an lm_head) in whole columns, rounds of workgroups of 64 outputs, or of 128.  The decode GEMM reads
+// x once for 16 outputs: with its launch that reduces the keys, us, it on either layout's better one / 64 / 128 outputs: 32768 x
+// 2048 at 24 rows 34.3 / 31.7 / 36.0, 64 43.2 / 36.5 / 38.8; 32768 x 4096 at 17 57.8 / 55.3 / 56.2, 64 67.3 / 63.4 / 57.0; 32000 x
+// 8192 at 48 119 / 97 / 92; 128256 x 2048 at 64 150 / 123 / 126; 128256 x 4096 at 32 195 / 193 / 188, 64 233 / 235 / 203; 64000 x
+// 1024 at 17 34.1 / 35.6 / 36.0, 64 49 / 44 / 43.  So 128 past 32 rows of a long K, and where 64 make a second round of few (20480 x
+// 2048 at 24 rows 29.5 / 26.5 / 25.1, 24576 x 4096 at 48 54.5 / 50.4 / 42.1), but 64 in one round (16384 x 4096 at 64 51.1 / 34.1 /
+// 40.7).  Fewer outputs leave CUs idle (10240 x 8192 at 17 rows 51.4 / 33.8, but 8192 x 4096 20.5 / 23.1).
+bool launch_mgemm_argmax(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEpi& e, hipStream_t s) {
+  if (!e.wshuf || M <= 16 || M > 64 || K % 64 || K < 1024 || K > 1 << 20 || N % 16 || N < 10240) return false;
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W)) % 16) return false;
+  const int groups = (N + 63) / 64;
+  if (groups > 256 && (groups < 448 || (M > 32 && K > 2048))) launch_argmax<8>(x, W, M, N, K, e, s);
+  else launch_argmax<4>(x, W, M, N, K, e, s);
+  return true;
+}
 
 void set_mgemm_nt(int on) { g_mgemm_nt = on; }
 

@@ -286,10 +286,10 @@ class TransformerLM:
         return n
 
     def _lm_head(self, rows: int):
-        """(weight, wshuf) of the decode lm_head for a ``rows``-row sampling launch: the MFMA-preshuffled copy up
-        to 16 rows, the row-major stream's row-tile variants above (profiles/r3/lmhead_preshuffle_ab.jsonl: 1 row
-        189.5 -> 175.1 us, 6 rows 192.9 -> 168.8; 24 rows 222.6 vs 232.3, 32 rows 220 vs 228; 64 rows even)."""
-        return self._dgw(-1, "lm_head") if rows <= 16 else (self.w["lm_head"], False)
+        """(weight, wshuf) of the decode lm_head for a ``rows``-row sampling launch: the MFMA-preshuffled copy, if there is one (1
+        row of 128256 x 4096 189.5 -> 175.1 us, 24 rows 209 -> 188, 64 rows 233 -> 203; narrow models' row-tile variants of 17 rows
+        and more read the row-major weight: 32 rows of 50304 x 1024 33.0 / 33.2)."""
+        return self._dgw(-1, "lm_head") if rows <= 16 or self.cfg.hidden_size >= 1024 else (self.w["lm_head"], False)
 
     def _dgw(self, i: int, name: str):
         """(weight, wshuf) for decode GEMM `name` of layer i (i = -1: the lm_head)."""

@@ -145,6 +145,43 @@ def test_dg_argmax_preshuffled(gpu, M, N):
     assert torch.equal(outs[1][1].cpu().long(), outs[1][0].cpu().argmax(1))
 
 
+# workgroups of 64 outputs and of 128, the last with one 16-row tile; row tiles of 32, 48 and 64; K shorter than the ring and one
+# with a part of a part left over; with and without row scales; 17 rows at the fewest outputs that take the path, and just below
+@pytest.mark.parametrize("M,N,K,ss", [(17, 10240, 1024, True), (32, 10256, 1024, False), (33, 16400, 2304, True), (48, 16400, 2304, False),
+                                      (49, 16640, 2304, True), (64, 28688, 2304, False), (64, 28688, 1280, True), (31, 20496, 2048, True),
+                                      (64, 10224, 1024, True)])
+def test_dg_argmax_wide_batches(gpu, M, N, K, ss):
+    """17 to 64 rows on the preshuffled copy: logits within the row-major kernel's own distance of the product in 64 bits (K's parts of
+    256 are chains of 8 instructions in both or shorter; a twentieth for the order of the parts), the keys those of the logits, and
+    nothing written past the last output's."""
+    from symmetry_amd.models.layout import preshuffle
+
+    x, W, s = _inputs(gpu, M, N, K, seed=M + N)
+    s = s if ss else None
+    temps = torch.where(torch.arange(M, device=gpu) % 3 == 0, 0.0, 0.7).float()
+    seeds = torch.arange(M, device=gpu, dtype=torch.int64) * 77 + 5
+    step = torch.tensor([2], device=gpu, dtype=torch.int64)
+    exact = x.double() @ W.double().t()
+    if ss:
+        exact *= torch.rsqrt(s.double().sum(1, keepdim=True) / K + 1e-5)
+    off = []
+    for sh in (False, True):
+        tk = torch.full((M * (N // 16) + 64,), -7, device=gpu, dtype=torch.int64)
+        keys = torch.empty(M, device=gpu, dtype=torch.int64)
+        ids = torch.empty(M, device=gpu, dtype=torch.int32)
+        buf = torch.full((M * N + 4096,), 9.5, device=gpu)
+        logits = buf[:M * N].view(M, N)
+        ops.dg_argmax(x, preshuffle(W) if sh else W, s, 1e-5, temps, seeds, step, tk, keys, ids, 100, logits, wshuf=sh)
+        off.append(((logits.double() - exact).norm() / exact.norm()).item())
+        assert (tk[M * (N // 16):] == -7).all() and (buf[M * N:] == 9.5).all()
+        k_ref, i_ref = ref.sample_keys(logits.cpu(), temps.cpu(), seeds.cpu(), 2, 100)
+        assert torch.equal(ids.cpu().long(), i_ref)
+        greedy = temps.cpu() == 0
+        assert torch.equal(keys.cpu()[greedy], k_ref[greedy])
+    # (a row's scale is the rsqrt of a sum taken in another order: an ulp of it, 2^-23, shifts the whole row)
+    assert off[1] <= 1.05 * off[0] + (2.0 ** -23 if ss else 0.0), off
+
+
 @pytest.mark.parametrize("T,P", [(33, 4), (64, 4), (3, 2)])
 def test_add_prep_partial_sums_from_slabs(gpu, T, P):
     """add_prep over fp32 k-split slabs with P workgroups per row: ss holds P column-slice partials."""
