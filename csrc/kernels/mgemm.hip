@@ -27,7 +27,10 @@
 //     So x tiles come in steps of 16 rows (a slot less of padding is a slot more of the ring), the chunk's DMAs are dealt to the
 //     waves one by one, and the weights are loaded past the caches (read once; x stays in the L2).  Against row tiles in steps of
 //     32 and cached weights, us: 28672 x 4096 at 20 rows 41.9 -> 38.7, 64 43.1 -> 40.5, 137 57.8 -> 50.9, 192 65.0 -> 62.9;
-//     4096 x 14336 at 64 24.3 -> 22.8, 137 31.6 -> 28.6, 240 46.1 -> 40.4; 4096 x 4096 at 137 14.5 -> 13.4.  A K range for every
+//     4096 x 14336 at 64 24.3 -> 22.8, 137 31.6 -> 28.6, 240 46.1 -> 40.4; 4096 x 4096 at 137 14.5 -> 13.4.
+//     Workgroups start at different chunks (first_chunk), in step -> so, us: 28672 x 4096 at 24 rows 38.8 -> 37.9, 64 40.7 -> 39.7;
+//     16384 x 2048 at 24 14.7 -> 13.1, 137 21.6 -> 20.9; 4096 x 4096 at 24 10.1 -> 8.0, 64 10.8 -> 9.2; 2048 x 8192 at 24 8.9 -> 7.9;
+//     8192 x 8192 at 24 25.3 -> 21.9; 22016 x 4096 at 137 48.9 -> 47.5.  A K range for every
 //     wave, x in registers, was slower (64 to 70 at 137 rows): its waves wait for the weights each by itself;
 //   * the 16x16 accumulator of (weight tile, token tile) holds 4 consecutive features of one token per
 //     lane: one float4 store per accumulator into the slab.
@@ -115,7 +118,9 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
     vw[i] = ((b >> 1) * (K / 32) + k0 / 32 + (b & 1)) * 1024 + lane * 16;
   }
 
+  const int turn = first_chunk(blockIdx.x + gridDim.x * split, nch, (long long)M * K * 2);
   auto issue = [&](int c, int slot) {
+    c = c + turn < nch ? c + turn : c + turn - nch;
     const int xo = c * 128, wo = c * 2048;
 #pragma unroll
     for (int i = 0; i < C::NX; ++i) mg_dma(rx, vx[i], xo, smem + slot * C::SLOT + min(C::NX * wid + i, 2 * MT - 1) * 1024);
