@@ -7,7 +7,11 @@
 // fragments of a step are read while the step before is multiplied (one wave a SIMD: nothing else covers the reads), and the
 // barrier stands in a chunk's middle, behind which its slot is free.  K is split where whole columns would leave CUs idle; of
 // a column group's workgroups the last to arrive adds the others' parts, in their order, to the sum (nobody waits; the counter is
-// set back to zero).
+// set back to zero).  The last one's loads go out for eight parts at once: a round trip past the L2 is what they cost.
+//
+// The weights pass by the caches, which keep x, and workgroups start at different chunks (first_chunk).  With column groups of 32 and
+// 48 outputs beside 64 and 80 and row tiles of 48, us: 17440 x 2048 at 24 rows 17.5 -> 13.7, 64 19.2 -> 16.6; pairs of 8192 x 2048
+// at 24 16.3 -> 12.7, 64 18.7 -> 14.9; 2048 x 8192 at 40 13.3 -> 10.9; 8192 x 8192 at 24 34.7 -> 24.5; 2048 x 2048 at 40 9.4 -> 6.9.
 #include "common.h"
 #include "hybrid_launchers.h"
 
@@ -76,14 +80,19 @@ __global__ __launch_bounds__(64 * WV, 1) void mid_linear_kernel(Args a) {
   auto load = [](__amdgpu_buffer_rsrc_t r, int off, int soff, char* lds) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t*)lds, 16, off, soff, 0, 0);
   };
+  auto load_once = [](__amdgpu_buffer_rsrc_t r, int off, int soff, char* lds) {      // (past the caches, which keep x)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t*)lds, 16, off, soff, 0, 2);
+  };
+  const int turn = first_chunk(blockIdx.x + gridDim.x * split, nch, (long long)M * K * 2);
   auto issue = [&](int c, int slot) {
+    c = c + turn < nch ? c + turn : c + turn - nch;
     char* const s = smem + slot * C::SLOT;
 #pragma unroll
     for (int i = 0; i < C::NX; ++i) load(rx, vx[i], c * 128, s + min(C::NX * wid + i, 2 * MT - 1) * 1024);
 #pragma unroll
     for (int rt = 0; rt < RW; ++rt)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) load(rw, vw[rt][i], c * 128, s + C::XB + ((wid * RW + rt) * 2 + i) * 1024);
+      for (int i = 0; i < 2; ++i) load_once(rw, vw[rt][i], c * 128, s + C::XB + ((wid * RW + rt) * 2 + i) * 1024);
   };
 
   const int j = lane & 15, h = lane >> 4;
@@ -162,33 +171,29 @@ __global__ __launch_bounds__(64 * WV, 1) void mid_linear_kernel(Args a) {
     }
     __syncthreads();
     if (!*last) return;
-    constexpr int MB = RW * MT < 8 ? RW * MT : 8, SB = 4;
+    constexpr int MB = RW * MT < 8 ? RW * MT : 8, SB = MB <= 4 ? 8 : 4;
+    const __amdgpu_buffer_rsrc_t rp = rows_buffer(a.slab, 4LL * MID_SLAB);
+    const int from = (int)((blockIdx.x * S * WV + wid) * (RW * MT * 256) + lane * 4) * 4;
 #pragma unroll
     for (int t0 = 0; t0 < RW * MT; t0 += MB) {
 #pragma unroll
       for (int u = 0; u < MB; ++u)
         if (t0 + u < RW * MT) acc[(t0 + u) / MT][(t0 + u) % MT] = f32x4{0.f, 0.f, 0.f, 0.f};
       for (int s0 = 0; s0 < S; s0 += SB) {
-        unsigned long long v[SB][MB][2];
+        u32x4 v[SB][MB];
 #pragma unroll
         for (int e = 0; e < SB; ++e)
 #pragma unroll
-          for (int u = 0; u < MB; ++u) {
-            if (t0 + u >= RW * MT) continue;
-            const unsigned long long* p = reinterpret_cast<const unsigned long long*>(mine + min(s0 + e, S - 1) * PART + (t0 + u) * 256);
-            v[e][u][0] = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            v[e][u][1] = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
+          for (int u = 0; u < MB; ++u)
+            if (t0 + u < RW * MT)
+              v[e][u] = __builtin_amdgcn_raw_buffer_load_b128(rp, from, (int)(min(s0 + e, S - 1) * PART + (t0 + u) * 256) * 4, 17);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int e = 0; e < SB; ++e) {
           if (s0 + e >= S) break;
 #pragma unroll
           for (int u = 0; u < MB; ++u)
-            if (t0 + u < RW * MT)
-              acc[(t0 + u) / MT][(t0 + u) % MT] +=
-                  f32x4{__uint_as_float((unsigned)v[e][u][0]), __uint_as_float((unsigned)(v[e][u][0] >> 32)),
-                        __uint_as_float((unsigned)v[e][u][1]), __uint_as_float((unsigned)(v[e][u][1] >> 32))};
+            if (t0 + u < RW * MT) acc[(t0 + u) / MT][(t0 + u) % MT] += __builtin_bit_cast(f32x4, v[e][u]);
         }
       }
     }
@@ -222,6 +227,7 @@ void run(const Args& a, int S, hipStream_t s) {
 template <int WV, bool GLU>
 void run_rows(const Args& a, int S, hipStream_t s) {
   if (a.M <= 32) run<2, WV, GLU>(a, S, s);
+  else if (a.M <= 48) run<3, WV, GLU>(a, S, s);
   else if (a.M <= 64) run<4, WV, GLU>(a, S, s);
   else if (a.M <= 96) run<6, WV, GLU>(a, S, s);
   else if (a.M <= 128) run<8, WV, GLU>(a, S, s);
@@ -230,10 +236,13 @@ void run_rows(const Args& a, int S, hipStream_t s) {
   else run<16, WV, GLU>(a, S, s);
 }
 
-// A plan's time, us: a workgroup takes in its weight rows and x at about 36 KB / us, and the last arriver the other parts at 50.
-float plan_time(const Args& a, int cols, int rows, int S) {
+// A plan's time beside what all have, us: a workgroup takes in its weight rows at 31 KB / us, all together at 7.3 MB / us, x from its
+// L2 at 110 KB / us; to hand parts over costs 3.3, and 87 KB / us of the others' parts.  (Fitted to all plans of 1463 sizes, 17 to 250
+// rows, 2048 to 17440 outputs, K of 2048 to 14336; the plan that it picks takes 1.007 of the best one's time, at worst 1.15.)
+float plan_time(const Args& a, int groups, int rows, int S) {
   const int per = (a.K / 64 + S - 1) / S;
-  return per * 128e-3f * (rows + a.M) / 36.f + (S - 1) * 4e-3f * cols * a.M / 50.f;
+  const float weights = std::max(per * 128e-3f * rows / 31.f, 2e-3f * groups * rows * a.K / 7300.f);
+  return weights + per * 128e-3f * a.M / 110.f + (S > 1 ? 3.3f : 0.f) + (S - 1) * 4e-3f * rows * a.M / 87.f;
 }
 
 }  // namespace
@@ -247,18 +256,20 @@ bool launch_mid_linear(const void* x, long long ldx, const void* W, void* out, l
   const int rw = glu ? 2 : 1;
   int best = 0, splits = 1;
   float least = 1e30f;
-  for (int wv : {4, 5, 2}) {
-    if (glu ? wv == 5 : wv == 2) continue;
+  for (int wv : {4, 5, 3, 2}) {
+    if (glu && wv == 5) continue;
     const int groups = (N + 16 * wv - 1) / (16 * wv);
     for (int S = 1; S <= 16 && groups * S <= CUS && S <= K / 64; ++S) {
-      const float t = plan_time(a, 16 * wv * rw, 16 * wv * rw, S);
+      const float t = plan_time(a, groups, 16 * wv * rw, S);
       if (t < least) least = t, best = wv, splits = S;
     }
   }
   if (!best) return false;
   a.per = (K / 64 + splits - 1) / splits;
   splits = (K / 64 + a.per - 1) / a.per;
-  if (glu) best == 4 ? run_rows<4, true>(a, splits, s) : run_rows<2, true>(a, splits, s);
-  else best == 4 ? run_rows<4, false>(a, splits, s) : run_rows<5, false>(a, splits, s);
+  if (best == 2) glu ? run_rows<2, true>(a, splits, s) : run_rows<2, false>(a, splits, s);
+  else if (best == 3) glu ? run_rows<3, true>(a, splits, s) : run_rows<3, false>(a, splits, s);
+  else if (best == 4) glu ? run_rows<4, true>(a, splits, s) : run_rows<4, false>(a, splits, s);
+  else run_rows<5, false>(a, splits, s);
   return true;
 }

@@ -628,6 +628,34 @@ def mid_pays(M: int, N: int, K: int, glu: bool = False) -> bool:
     return not power and K <= ((9216 if M <= 32 else 1 << 20) if N <= 10240 else 4608)
 
 
+def mid_pays_wide(M: int, N: int, K: int, glu: bool = False) -> bool:
+    """... and where the kernel came ahead when its weights went past the caches, its workgroups started at spread places of K and its
+    column groups came in 32s and 48s too: 0.73 of the library's time on the sizes that mid_pays names (0.85 of its own before), 0.76
+    on these.  5763 measured sizes (17 to 256 rows, 1024 to 20480 outputs, K of 1536 to 14336), us, library / kernel.
+
+    Up to 64 rows nearly everywhere: 2048 x 2048 at 40 8.6 / 7.0, 1024 x 2048 at 32 8.5 / 6.2, 3664 x 2048 at 48 12.1 / 8.8, 14336 x
+    4096 at 64 27.0 / 24.4, but 2560 x 1536 at 64 7.9 / 8.4.  Past that short K over few outputs is the library's (2048 x 2048 at 100
+    8.6 / 9.3, 3072 x 1536 at 100 8.1 / 10.1), past 104 also outputs where its tiles come out even (8192 x 2560 at 144 18.6 / 20.6,
+    14336 x 3072 at 128 26.5 / 27.8, 17440 x 5120 at 128 49.0 / 52.9; 14336 x 5120 at 176 47.1 / 52.9); past 160 rows K is to be long
+    (4096 x 4096 at 176 22.6 / 18.0, 8192 x 3072 21.1 / 24.6), past 192 longer, but the library has no good tile for 209 to 256 rows
+    of 5120 to 10240 outputs (5120 x 5120 at 224 45.1 / 27.7).  Pairs are ahead nearly everywhere, a launch being saved (8192 x 3072 at
+    64 25.9 / 21.9, 5120 x 5120 at 160 48.0 / 36.5; not 2048 x 1536 at 200 13.9 / 17.6)."""
+    if K < 1536 or N < 1024:
+        return False
+    if glu:
+        return N <= 16384 and (M <= 64 or N >= 5120 or (M <= 192 and (N >= 3072 or (N >= 2048 and K >= 2048)))
+                               or (N >= 3072 and K >= 4096))
+    if M <= 64 or N > 20480:
+        return N <= 20480 and (M <= 48 or K >= 2048 or not 2304 < N < 3584)
+    if M <= 160:
+        even = K > 2304 and ((8192 <= N <= 10240 and 104 < M <= 144 and K <= 3072)
+                             or (12288 <= N and M > 112 and K <= 6144 and (N < 16384 or M <= 128)))
+        return (N >= 6144 or (N >= 3072 and K >= 2048) or (N >= 2048 and K >= 3072)) and not even
+    if M <= 192:
+        return (N >= 16384 and K <= 8192) if N >= 12288 else (K < 2048 and N >= 6144) or (K >= 4096 and N >= 3072) or (K >= 8192 and N >= 2048)
+    return (K < 2048 and N >= 8192) or (2048 <= N <= 10240 and (K >= 6144 or (M > 208 and N >= 5120 and K >= 2560)))
+
+
 def mid_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None, ws, glu: bool = False) -> bool:
     """Does x @ w.T into ``out`` (glu: w of twice out's columns) run on the medium-row kernel?  17..256 rows in bf16 with a
     workspace to split K in, K in 64s, where it pays; few_rows' conditions otherwise."""
@@ -638,7 +666,8 @@ def _mid(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu: bool = False)
     if x.dim() != 2 or not FEW_ROWS < x.shape[0] <= MID_ROWS or out.dim() != 2:
         return False
     M, K = x.shape
-    if not mid_pays(M, out.shape[1], K, glu) or K % 64 or K > 1 << 20 or out.dtype != torch.bfloat16 or 2 * w.numel() > 0x7FFFFFFF:
+    N = out.shape[1]
+    if not (mid_pays(M, N, K, glu) or mid_pays_wide(M, N, K, glu)) or K % 64 or K > 1 << 20 or out.dtype != torch.bfloat16 or 2 * w.numel() > 0x7FFFFFFF:
         return False
     return K <= x.stride(0) <= 1 << 20 and out.stride(0) <= 1 << 28 and _own_linear(x, w, out)
 

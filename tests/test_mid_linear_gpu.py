@@ -130,3 +130,35 @@ def test_the_rule_names_no_size_without_a_plan():
     for glu, most in ((False, 256 * 80), (True, 256 * 64)):
         assert any(ops.mid_pays(M, most, K, glu) for M in ROWS for K in (2048, 4096))
         assert not any(ops.mid_pays(M, most + 4, K, glu) for M in ROWS for K in (2048, 4096, 8192, 14336))
+
+
+# column groups of 2, 3, 4 and 5 tiles with one slice of K, few and up to 16, whole ones and a shorter last one; row tiles of 48; chunks
+# walked from a spread of places of K, from one for every XCD (256 rows of 8192: x is past an L2's share), from fewer chunks than XCDs
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,glu", [(48, 1284, 2112, False), (33, 2500, 2112, False), (100, 20, 4096, False), (48, 20, 8192, False),
+                                       (17, 8204, 64, False), (40, 3664, 2112, False), (256, 2500, 4096, False), (48, 6160, 4096, False),
+                                       (200, 3664, 8192, False), (256, 8204, 2112, False), (256, 2048, 8192, False),
+                                       (48, 2500, 2112, True), (33, 3664, 2112, True), (256, 2500, 8192, True), (40, 6160, 4096, True),
+                                       (48, 20, 8192, True), (17, 100, 4096, True)])
+def test_plans(gpu, M, N, K, glu):
+    g = torch.Generator(device=gpu).manual_seed(N + K + M)
+    ws = Workspace()
+    x = torch.randn(M, K, device=gpu, generator=g).bfloat16()
+    w = (torch.randn((1 + glu) * N, K, device=gpu, generator=g) * K ** -0.5).bfloat16()
+    want = x.double() @ w.double().t()
+    if glu:
+        want = want[:, :N] * torch.sigmoid(want[:, :N]) * want[:, N:]
+    room = torch.full((M + 1, N + 8), 7.0, device=gpu, dtype=torch.bfloat16)
+    out = room[:M, :N]
+    for _ in range(2):
+        assert ops.mid_linear(x, w, out, ws, glu=glu)
+        assert float((out.double() - want).abs().max()) <= (2 ** -6 if glu else 2 ** -7) * max(float(want.abs().max()), 1.0)
+    assert bool((room[:, N:] == 7).all()) and bool((room[M] == 7).all())
+    assert not bool(ops.mid_workspace(ws, x.device)[1].any())
+
+
+def test_the_wide_rule_names_no_size_without_a_plan():
+    for glu, most in ((False, 256 * 80), (True, 256 * 64)):
+        assert all(ops.mid_pays_wide(64, most, K, glu) for K in (1536, 4096, 8192))
+        assert not any(ops.mid_pays_wide(M, most + 4, K, glu) for M in ROWS for K in (1536, 2048, 4096, 8192, 14336))
+        assert not any(ops.mid_pays_wide(M, 1020, 4096, glu) or ops.mid_pays_wide(M, 4096, 1472, glu) for M in ROWS)
