@@ -44,6 +44,27 @@ namespace {
 // ---------------------------------------------------------------------------------------------
 // Decode (body: attn_decode.h)
 // ---------------------------------------------------------------------------------------------
+// Whole contexts on more units (sequence, kv head) than CUs: workgroup i gets the i-th longest, and those of the second round (of
+// two at most), from the last CU to the first, the rest, so that a CU's two share out evenly; of more rounds the short ones come
+// last.  All of a round is resident: what a CU has to read is what it takes (64 contexts of 450 .. 1350 tokens, 8 heads: in the
+// order of the batch 60.3 us, rows of it turned 59.4, so 56.1; the longest first 59.0; pairs on neighbouring CUs 61.3; 236 MB that are
+// read and not used 40.6).  A group's K loaded under the softmax before it took as long.
+constexpr int DECODE_CUS = 256;
+
+SYM_DEV void by_length(const int* __restrict__ ctx_lens, int num_seqs, int Hkv, int& seq, int& kvh) {
+  const int units = num_seqs * Hkv, id = kvh * num_seqs + seq, lane = threadIdx.x & 63;
+  const int k = id < DECODE_CUS || units > 2 * DECODE_CUS ? id : units - 1 - (id - DECODE_CUS);
+  const int mine = (unsigned)k / (unsigned)Hkv;
+  kvh = k - mine * Hkv;
+  const int len = lane < num_seqs ? ctx_lens[lane] : -1;
+  int rank = 0;
+  for (int j = 0; j < num_seqs; ++j) {
+    const int other = __builtin_amdgcn_readlane(len, j);
+    rank += other > len || (other == len && j < lane);
+  }
+  seq = __builtin_ctzll(__ballot(rank == mine));
+}
+
 // GMAX >= G query heads per kv head: the cross-wave merge stages GMAX columns in LDS (GMAX = 4 for
 // Llama-3 GQA: 17 KB instead of 68 KB, so LDS no longer caps the resident workgroups per CU)
 template <int GMAX, bool UNEVEN>
@@ -66,6 +87,15 @@ __global__ __launch_bounds__(DWAVES * 64, 4) void attn_decode_kernel(
       kvh = w - seq * Hkv;
       if (seq >= further) return;
     }
+  }
+  if (parts == 1 && part == 0 && num_seqs <= 64 && num_seqs * Hkv > DECODE_CUS) {
+    by_length(ctx_lens, num_seqs, Hkv, seq, kvh);
+  } else if (num_seqs >= 8 && 2 * num_seqs * Hkv > DECODE_CUS && part < parts) {
+    // Workgroups go round the eight XCDs, and on one round its CUs: of 8 n sequences an XCD would get every eighth with all its
+    // heads, and a CU two heads of one.  Each row of the grid starts a sequence further on (48 of 300 .. 900 tokens, 4 heads, in
+    // halves: 22.4 -> 20.2 us; 24 in fifths 13.4 / 13.4, fewer are left as they are).
+    seq += (blockIdx.y + gridDim.y * blockIdx.z) & 7;
+    if (seq >= num_seqs) seq -= num_seqs;
   }
   attn_decode_unit<GMAX, UNEVEN>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, num_seqs,
                                  Hq, Hkv, G, BS, max_blocks, max_parts, scale_log2, inv, seq, kvh, part, parts,

@@ -159,6 +159,33 @@ def test_attn_decode(gpu, Hq, Hkv, BS):
     assert torch.equal(out, out2)
 
 
+# more units than CUs (whole contexts, given out by length): two full rounds, a ragged second, more rounds, one head; a context far above
+# the others; past 64 sequences and below 256 units the batch's order, turned
+@pytest.mark.parametrize("S,Hq,Hkv,long", [(64, 32, 8, 0), (49, 32, 8, 0), (64, 32, 16, 0), (64, 32, 8, 3000), (65, 32, 8, 0), (48, 16, 4, 0),
+                                           (33, 32, 8, 1500), (63, 63, 63, 0)])
+def test_attn_decode_many_sequences(gpu, S, Hq, Hkv, long):
+    """Every (sequence, head) is somebody's: lengths with ties, the shortest and an empty context, whose rows stay as they are."""
+    g = torch.Generator(device=gpu).manual_seed(S + Hkv)
+    lens = [(37 * i * i + 11 * i) % 400 + 1 for i in range(S)]
+    lens[3] = lens[S - 1] = lens[7]
+    lens[5], lens[9] = 0, 1
+    if long:
+        lens[S // 2] = long
+    kc, vc, bt = _random_paged(gpu, lens, Hkv, 64, g)
+    q = torch.randn(S, Hq, 128, device=gpu, generator=g).bfloat16()
+    ctx = torch.tensor(lens, device=gpu, dtype=torch.int32)
+    max_parts = (bt.shape[1] * 64 + ops.ATTN_DECODE_PART - 1) // ops.ATTN_DECODE_PART
+    tmp_o, tmp_ml = torch.empty(S, Hq, max_parts, 128, device=gpu), torch.empty(S, Hq, max_parts, 2, device=gpu)
+    out = torch.full((S, Hq, 128), 7.0, device=gpu, dtype=torch.bfloat16)
+    cnt = torch.zeros(S * Hkv, device=gpu, dtype=torch.int32)
+    ops.attn_decode(q, kc, vc, bt, ctx, out, tmp_o, tmp_ml, cnt, 128 ** -0.5)
+    kept = [i for i in range(S) if lens[i]]
+    out_r = torch.empty(len(kept), Hq, 128, dtype=torch.bfloat16)
+    ref.attn_decode(q.cpu()[kept], kc.cpu(), vc.cpu(), bt.cpu()[kept], ctx.cpu()[kept], out_r, scale=128 ** -0.5)
+    _close(out[kept], out_r, atol=2e-2, rtol=2e-2)
+    assert bool((out[5] == 7.0).all()) and int(cnt.abs().sum()) == 0
+
+
 def test_attn_decode_empty_tables(gpu):
     """Block tables without a column (and so scratch without a partition): nothing to read, nothing to write."""
     S, Hq, Hkv = 3, 16, 4
