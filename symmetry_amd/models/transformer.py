@@ -153,9 +153,13 @@ class Workspace:
 
     buffers: dict = field(default_factory=dict)
     retired: list = field(default_factory=list)
+    views: dict = field(default_factory=dict)    # each buffer's last view: a step's layers ask for the same ones
 
     def get(self, name: str, shape, dtype, device, zeros: bool = False) -> torch.Tensor:
         """``zeros``: zero-fill on (re)allocation only -- for state the kernels keep re-armed themselves."""
+        last = self.views.get((name, dtype))
+        if last is not None and last.shape == shape:
+            return last
         numel = math.prod(shape)
         buf = self.buffers.get((name, dtype))
         if buf is None or buf.numel() < numel:
@@ -163,7 +167,8 @@ class Workspace:
                 self.retired.append(buf)
             buf = (torch.zeros if zeros else torch.empty)(numel, dtype=dtype, device=device)
             self.buffers[(name, dtype)] = buf
-        return buf[:numel].view(*shape)
+        view = self.views[(name, dtype)] = buf[:numel].view(*shape)
+        return view
 
     def nbytes(self) -> int:
         return sum(b.numel() * b.element_size() for b in list(self.buffers.values()) + self.retired)

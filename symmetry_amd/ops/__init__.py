@@ -62,7 +62,7 @@ def native_available() -> bool:
 
 
 def _gpu(t: torch.Tensor) -> bool:
-    return t.device.type != "cpu" and not _TORCH_MODE
+    return not t.is_cpu and not _TORCH_MODE
 
 
 def rms_norm(x, w, eps, out):

@@ -21,6 +21,8 @@ _error: str | None = None
 def load(build_if_missing: bool = False) -> bool:
     """Load ``_C.so`` once.  Returns True when the kernels are registered."""
     global _loaded, _error
+    if _loaded:      # (set once, when the kernels are registered: no lock on the way of every call)
+        return True
     with _lock:
         if _loaded:
             return True
@@ -64,6 +66,8 @@ def latent_ops():
     """``torch.ops.symmetry_amd_latent`` (loaded once; built first if the library is missing: three translation
     units, about half a minute).  Raises if it cannot be built or loaded: no eager fallback on the device."""
     global _latent_loaded
+    if _latent_loaded:
+        return torch.ops.symmetry_amd_latent
     with _lock:
         if not _latent_loaded:
             if not os.path.exists(_LATENT_LIB):
@@ -88,6 +92,8 @@ def hybrid_ops():
     """``torch.ops.symmetry_amd_hybrid`` (loaded once; built first if the library is missing: eleven translation units,
     about a minute).  Raises if it cannot be built or loaded: no eager fallback on the device."""
     global _hybrid_loaded
+    if _hybrid_loaded:
+        return torch.ops.symmetry_amd_hybrid
     with _lock:
         if not _hybrid_loaded:
             if not os.path.exists(_HYBRID_LIB):
