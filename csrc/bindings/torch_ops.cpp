@@ -694,6 +694,33 @@ void grouped_skinny(const Tensor& xs, const Tensor& W, const Tensor& offsets, in
                         (int)N, (int)K, (int)S, cur_stream(xs), wshuf);
 }
 
+// residual += moe_combine; out = rmsnorm(residual) * wn
+void moe_combine_norm(const Tensor& y, const Tensor& dst, const Tensor& ids, int64_t e_lo, int64_t e_hi, const Tensor& w, int64_t k,
+                      Tensor& residual, const Tensor& wn, double eps, Tensor& out) {
+  check_gpu(residual, "residual");
+  check_dtype(residual, at::kFloat, "residual");
+  check_gpu(out, "out");
+  check_dtype(out, at::kBFloat16, "out");
+  check_gpu(wn, "wn");
+  check_dtype(wn, at::kBFloat16, "wn");
+  check_gpu(dst, "dst");
+  check_dtype(dst, at::kInt, "dst");
+  check_gpu(ids, "ids");
+  check_dtype(ids, at::kInt, "ids");
+  check_gpu(w, "w");
+  check_dtype(w, at::kFloat, "w");
+  TORCH_CHECK(residual.dim() == 2 && k >= 1, "residual must be [T, d]");
+  const int64_t T = residual.size(0), d = residual.size(1);
+  const int64_t R = y.dim() == 3 ? y.size(1) : y.size(0);
+  TORCH_CHECK(d % 8 == 0 && d <= 16384, "moe_combine_norm: d must be a multiple of 8 and <= 16384");
+  TORCH_CHECK(wn.numel() == d && out.numel() == T * d, "moe_combine_norm: shape mismatch");
+  TORCH_CHECK(dst.numel() >= T * k && w.numel() >= T * k && ids.numel() >= T * k && T * k < (1LL << 31), "moe_combine_norm: dst/w too small");
+  if (T == 0) return;
+  const at::OptionalDeviceGuard g(residual.device());
+  launch_combine_rms_norm(linout(y, R, d, "y"), (int)R, ptr<int>(dst), ptr<int>(ids), (int)e_lo, (int)e_hi, ptr<float>(w), (int)k,
+                          ptr<float>(residual), ptr<bf16>(wn), ptr<bf16>(out), (int)T, (int)d, (float)eps, cur_stream(residual));
+}
+
 void moe_combine(const Tensor& y, const Tensor& dst, const Tensor& ids, int64_t e_lo, int64_t e_hi, const Tensor& w,
                  int64_t k, Tensor& out, bool accumulate) {
   check_gpu(out, "out");
@@ -1273,6 +1300,10 @@ TORCH_LIBRARY(symmetry_amd, m) {
         "Tensor(a!) cursor, Tensor(b!) send, Tensor(c!) side) -> ()", &moe_owner_pack);
   m.def("moe_owner_combine(Tensor recv, Tensor side, Tensor rcnt, int Tr, Tensor(a!) pos, Tensor(b!) out) -> ()",
         &moe_owner_combine);
+  m.def(
+      "moe_combine_norm(Tensor y, Tensor dst, Tensor ids, int e_lo, int e_hi, Tensor w, int k, Tensor(a!) residual, Tensor wn, "
+      "float eps, Tensor(b!) out) -> ()",
+      &moe_combine_norm);
   m.def(
       "moe_combine(Tensor y, Tensor dst, Tensor ids, int e_lo, int e_hi, Tensor w, int k, Tensor(a!) out, "
       "bool accumulate) -> ()",

@@ -152,6 +152,9 @@ void launch_pgemm_grouped(int epi, int cfg, const bf16* x, const bf16* Wshuf, in
 void launch_rms_norm(LinOut x, const bf16* w, bf16* out, int T, int d, float eps, hipStream_t s);
 void launch_add_rms_norm(LinOut delta, float* residual, const bf16* w, bf16* out, int T, int d, float eps,
                          hipStream_t s);
+// moe_combine and add_rms_norm in one launch
+void launch_combine_rms_norm(LinOut y, int R, const int* dst, const int* ids, int e_lo, int e_hi, const float* cw, int k, float* residual,
+                             const bf16* w, bf16* out, int T, int d, float eps, hipStream_t s);
 void launch_embed_rms_norm(const int* ids, const bf16* table, float* residual, const bf16* w, bf16* out, int T,
                            int d, float eps, hipStream_t s, const int* src = nullptr, const int* prev = nullptr);
 

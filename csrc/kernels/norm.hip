@@ -5,6 +5,9 @@
 //   mode 2 (embed_norm): residual = table[tok]; out = rmsnorm(residual) * w, tok = src[row] >= 0 ?
 //                        prev[src[row]] : ids[row] (src/prev optional: a pipelined decode row's token is the
 //                        previous step's on-device sample)
+//   mode 3 (combine):   mode 1 with delta = sum_j w[t][j] y[dst[t][j]], the routed experts' rows (moe_combine's sum, bit for bit).
+//                       One launch where the fp32 sum went through memory: 8100 rows of 2048, 4 experts each, us: 60 + 33 ->
+//                       75.8 (430 MB, 5.7 TB/s)
 //
 // The residual stream is kept in fp32 ([T][d]) for accuracy; activations fed
 // to the projections are bf16.  One 256-thread workgroup per row, 16 B per
@@ -19,13 +22,20 @@
 
 namespace {
 
+struct Combine {      // mode 3: R rows of y; token t's k places, experts (those of e_lo .. e_hi - 1 count) and weights
+  const int* dst;
+  const int* ids;
+  const float* w;
+  int R, e_lo, e_hi, k;
+};
+
 template <int NT, int MAXV, int MODE>
 __global__ __launch_bounds__(NT) void rms_norm_kernel(LinOut x, const int* __restrict__ ids,
                                                       const bf16* __restrict__ table,
                                                       float* __restrict__ residual,
                                                       const bf16* __restrict__ w,
                                                       bf16* __restrict__ out, int d, float eps,
-                                                      const int* __restrict__ src, const int* __restrict__ prev) {
+                                                      const int* __restrict__ src, const int* __restrict__ prev, Combine c) {
   __shared__ float scratch[NT / 64];
   const int row = blockIdx.x;
   const int nvec = d >> 3;
@@ -43,6 +53,22 @@ __global__ __launch_bounds__(NT) void rms_norm_kernel(LinOut x, const int* __res
         float r[8];
         load8f(residual + off, r);
         linout_load8(x, off, v[k]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[k][i] += r[i];
+        store8f(residual + off, v[k]);
+      } else if constexpr (MODE == 3) {
+        float r[8], y[8];
+        load8f(residual + off, r);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[k][i] = 0.f;
+        for (int j = 0; j < c.k; ++j) {
+          const int from = c.dst[row * c.k + j], ex = c.ids[row * c.k + j];
+          if (from < 0 || from >= c.R || ex < c.e_lo || ex >= c.e_hi) continue;
+          const float wj = c.w[row * c.k + j];
+          linout_load8(x, (long long)from * d + vi * 8, y);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v[k][i] += wj * y[i];
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[k][i] += r[i];
         store8f(residual + off, v[k]);
@@ -73,7 +99,7 @@ __global__ __launch_bounds__(NT) void rms_norm_kernel(LinOut x, const int* __res
 
 template <int MODE>
 void launch_mode(LinOut x, const int* ids, const bf16* table, float* residual, const bf16* w, bf16* out,
-                 int T, int d, float eps, hipStream_t s, const int* src = nullptr, const int* prev = nullptr) {
+                 int T, int d, float eps, hipStream_t s, const int* src = nullptr, const int* prev = nullptr, Combine c = {}) {
   constexpr int NT = 256;
   const int nvec = d / 8;
   dim3 grid(T);
@@ -84,13 +110,13 @@ void launch_mode(LinOut x, const int* ids, const bf16* table, float* residual, c
     return !(e && e[0] == '0');
   }();
   if (wide && nvec <= 512) {
-    rms_norm_kernel<512, 1, MODE><<<grid, 512, 0, s>>>(x, ids, table, residual, w, out, d, eps, src, prev);
+    rms_norm_kernel<512, 1, MODE><<<grid, 512, 0, s>>>(x, ids, table, residual, w, out, d, eps, src, prev, c);
   } else if (nvec <= NT * 2) {
-    rms_norm_kernel<NT, 2, MODE><<<grid, NT, 0, s>>>(x, ids, table, residual, w, out, d, eps, src, prev);
+    rms_norm_kernel<NT, 2, MODE><<<grid, NT, 0, s>>>(x, ids, table, residual, w, out, d, eps, src, prev, c);
   } else if (nvec <= NT * 4) {
-    rms_norm_kernel<NT, 4, MODE><<<grid, NT, 0, s>>>(x, ids, table, residual, w, out, d, eps, src, prev);
+    rms_norm_kernel<NT, 4, MODE><<<grid, NT, 0, s>>>(x, ids, table, residual, w, out, d, eps, src, prev, c);
   } else {
-    rms_norm_kernel<NT, 8, MODE><<<grid, NT, 0, s>>>(x, ids, table, residual, w, out, d, eps, src, prev);
+    rms_norm_kernel<NT, 8, MODE><<<grid, NT, 0, s>>>(x, ids, table, residual, w, out, d, eps, src, prev, c);
   }
 }
 
@@ -103,6 +129,11 @@ void launch_rms_norm(LinOut x, const bf16* w, bf16* out, int T, int d, float eps
 void launch_add_rms_norm(LinOut delta, float* residual, const bf16* w, bf16* out, int T, int d, float eps,
                          hipStream_t s) {
   launch_mode<1>(delta, nullptr, nullptr, residual, w, out, T, d, eps, s);
+}
+
+void launch_combine_rms_norm(LinOut y, int R, const int* dst, const int* ids, int e_lo, int e_hi, const float* cw, int k, float* residual,
+                             const bf16* w, bf16* out, int T, int d, float eps, hipStream_t s) {
+  launch_mode<3>(y, nullptr, nullptr, residual, w, out, T, d, eps, s, nullptr, nullptr, Combine{dst, ids, cw, R, e_lo, e_hi, k});
 }
 
 void launch_embed_rms_norm(const int* ids, const bf16* table, float* residual, const bf16* w, bf16* out, int T,

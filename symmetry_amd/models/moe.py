@@ -221,6 +221,17 @@ class MoEBlock:
         self.calls["allreduce"] += 1
         return self._forward_local(i, x, reduce=self.ep > 1)
 
+    def forward_norm(self, i: int, x: torch.Tensor, resid, w_next, eps: float, out) -> None:
+        """resid += MoE(x); out = rmsnorm(resid) * w_next (``out`` may be x).  Where this rank has all experts the combine, the
+        residual and the norm are one launch."""
+        T, d = x.shape
+        if self.ep > 1 or self.use_a2a(T):
+            return ops.add_rms_norm(self.forward(i, x), resid, w_next, eps, out)
+        self.calls["allreduce"] += 1
+        ids, w, dst, offsets, xs, src = self._route(i, x)
+        y2 = self._experts(i, xs, offsets, self.e_lo, self.E_local, out_f32=True, src=src)
+        ops.moe_combine_norm(y2, dst, ids, self.e_lo, self.e_hi, w, self.k, resid, w_next, eps, out)
+
     def decode_fused_ok(self, T: int, d: int) -> bool:
         """The one-launch routing (+ fused combine / residual prep) of a decode step applies."""
         return (DECODE_FUSED and T <= 8 and not self.use_a2a(T) and self.E <= 64 and self.k <= 8 and d % 8 == 0

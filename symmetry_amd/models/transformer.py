@@ -593,6 +593,7 @@ class TransformerLM:
             pick = ops.choose_pgemm(T, (self.hq + 2 * self.hkv) * self.D, d, align=128, force=True)
             pg_qkv = None if pick is None else pick[0]
         for i in range(cfg.num_layers):
+            nxt = w.layer(i + 1, "ln1") if i + 1 < cfg.num_layers else w["norm"]
             if pg_qkv is not None:
                 ops.pg_qkv(x, self.dgw[(i, "wqkv")], None, eps, b.positions, b.slot_mapping, self.cos_sin, q, kv.k[i],
                            kv.v[i], self.hq, self.hkv, pg_qkv)
@@ -612,7 +613,8 @@ class TransformerLM:
                 mlp = self._linear("down", act, self._row_major(i, "w_down"), reduce=True, wshuf=self._shuf(i, "w_down"))
             elif cfg.is_moe:
                 ops.add_rms_norm(o, resid, w.layer(i, "ln2"), eps, x)
-                mlp = self.moe.forward(i, x)
+                self.moe.forward_norm(i, x, resid, nxt, eps, x)
+                continue
             else:
                 ops.add_rms_norm(o, resid, w.layer(i, "ln2"), eps, x)
                 if pg_gu is not None:
@@ -626,7 +628,6 @@ class TransformerLM:
                     act = self._buf("act", (T, F), torch.bfloat16)
                     ops.swiglu(gu, act, interleaved=True)
                 mlp = self._linear("down", act, self._row_major(i, "w_down"), reduce=True, wshuf=self._shuf(i, "w_down"))
-            nxt = w.layer(i + 1, "ln1") if i + 1 < cfg.num_layers else w["norm"]
             ops.add_rms_norm(mlp, resid, nxt, eps, x)
         return self.sample(b, x)
 

@@ -41,6 +41,7 @@ __all__ = [
     "moe_route_permute",
     "grouped_skinny",
     "moe_combine",
+    "moe_combine_norm",
     "dg_f32",
     "dg_qkv",
     "dg_resid",
@@ -502,6 +503,15 @@ def moe_combine_prep(y, dst, ids, E, w, k, resid, w_next, xw, ss):
     if _gpu(resid):
         return _native.ops().moe_combine_prep(y, dst, ids, int(E), w, int(k), resid, w_next, xw, ss)
     return reference.moe_combine_prep(y, dst, ids, E, w, k, resid, w_next, xw, ss)
+
+
+def moe_combine_norm(y, dst, ids, e_lo, e_hi, w, k, residual, wn, eps, out):
+    """residual += moe_combine(...); out = rmsnorm(residual) * wn, in one launch."""
+    if _gpu(residual):
+        return _native.ops().moe_combine_norm(y, dst, ids, int(e_lo), int(e_hi), w, int(k), residual, wn, float(eps), out)
+    total = torch.empty_like(residual)
+    reference.moe_combine(y, dst, ids, e_lo, e_hi, w, k, total)
+    return reference.add_rms_norm(total, residual, wn, eps, out)
 
 
 def moe_combine(y, dst, ids, e_lo, e_hi, w, k, out, accumulate=False):

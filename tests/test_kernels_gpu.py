@@ -443,3 +443,30 @@ def test_moe_owner_pack_and_combine(gpu, N, T, E, k):
         got = out[: hi - lo].float().cpu()
         assert ((got - want).abs() <= 1e-5 + want.abs() * 2.0 ** -8).all(), float((got - want).abs().max())
         assert (out[hi - lo:] == 0).all()
+
+
+# a row in one register set and in several; one expert a token and eight; slabs, fp32 and bf16 rows
+@pytest.mark.parametrize("T,d,k,form", [(1, 8, 1, "f32"), (37, 2048, 4, "f32"), (300, 4096, 2, "slabs"), (5, 4104, 8, "bf16"),
+                                        (9, 16384, 3, "f32"), (64, 520, 2, "slabs")])
+def test_moe_combine_norm(gpu, T, d, k, form):
+    """The combine, the residual and the norm in one launch are the two launches' bits; places that are nobody's and other ranks' experts
+    count for nothing."""
+    g = torch.Generator(device=gpu).manual_seed(T + d)
+    R, E = T * k, 8
+    shape = (3, R, d) if form == "slabs" else (R, d)
+    y = torch.randn(*shape, device=gpu, generator=g)
+    y = y.bfloat16() if form == "bf16" else y
+    dst = torch.randperm(R, device=gpu, generator=g).int()
+    ids = torch.randint(0, E, (R,), device=gpu, generator=g, dtype=torch.int32)
+    w = torch.rand(R, device=gpu, generator=g)
+    if R > 4:
+        dst[2], dst[4] = -1, R
+    resid = torch.randn(T, d, device=gpu, generator=g)
+    wn = torch.randn(d, device=gpu, generator=g).bfloat16()
+    for e_lo, e_hi in ((0, E), (2, 5)):
+        total, r0, r1 = torch.empty_like(resid), resid.clone(), resid.clone()
+        o0, o1 = (torch.full((T + 1, d), 7.0, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+        ops.moe_combine(y, dst, ids, e_lo, e_hi, w, k, total)
+        ops.add_rms_norm(total, r0, wn, 1e-5, o0[:T])
+        ops.moe_combine_norm(y, dst, ids, e_lo, e_hi, w, k, r1, wn, 1e-5, o1[:T])
+        assert torch.equal(r0, r1) and torch.equal(o0, o1)
