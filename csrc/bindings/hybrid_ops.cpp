@@ -462,6 +462,25 @@ bool mid_linear(const Tensor& x, const Tensor& w, Tensor& out, bool glu, Tensor&
                            ptr<int>(counters), cur_stream(x));
 }
 
+// y (fp32) = x . W^T of 17 to 64 rows in bf16; false: the sizes have no kernel
+bool mid_linear_f32(const Tensor& x, const Tensor& w, Tensor& out) {
+  gpu(x, "x", false);
+  gpu(out, "out", false);
+  dtype(w, at::kBFloat16, "w");
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kFloat && x.dim() == 2 && w.dim() == 2 && out.dim() == 2,
+              "mid_linear_f32: bf16 operands, fp32 out, 2-d");
+  const int64_t M = x.size(0), K = x.size(1), N = out.size(1);
+  TORCH_CHECK(M >= 1 && M <= 64 && out.size(0) == M && w.size(1) == K && w.size(0) == N && w.is_contiguous(), "mid_linear_f32: shapes");
+  TORCH_CHECK(K >= 64 && K % 64 == 0 && K <= (1 << 22) && N >= 4 && N % 4 == 0 && N <= (1 << 28), "mid_linear_f32: K in 64s, N in 4s");
+  TORCH_CHECK(x.stride(1) == 1 && out.stride(1) == 1, "mid_linear_f32: inner strides must be 1");
+  const int64_t ldx = M > 1 ? x.stride(0) : K, ldo = M > 1 ? out.stride(0) : N;
+  TORCH_CHECK(ldx >= K && ldx % 8 == 0 && ldx <= (1 << 20) && ldo >= N && ldo % 4 == 0 && ldo <= (1 << 28), "mid_linear_f32: row strides");
+  TORCH_CHECK((uintptr_t)x.data_ptr() % 16 == 0 && (uintptr_t)w.data_ptr() % 16 == 0 && (uintptr_t)out.data_ptr() % 16 == 0,
+              "mid_linear_f32: alignment");
+  const at::OptionalDeviceGuard g(x.device());
+  return launch_mid_linear_f32(x.data_ptr(), ldx, w.data_ptr(), out.data_ptr<float>(), ldo, (int)M, (int)N, (int)K, cur_stream(x));
+}
+
 void relu_sq(const Tensor& a, Tensor& out) {
   const int f32 = act(out, "out");
   TORCH_CHECK(out.dim() == 2, "relu_sq: out [R, F]");
@@ -1229,6 +1248,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
   m.def("conv_state_update(Tensor xin, Tensor(a!) state, Tensor? cu_q, Tensor prev_row, Tensor save_slot, int runs) -> ()",
         &conv_state_update);
   m.def("row_linear(Tensor x, Tensor w, Tensor(a!) out, bool relu2, bool glu) -> ()", &row_linear);
+  m.def("mid_linear_f32(Tensor x, Tensor w, Tensor(a!) out) -> bool", &mid_linear_f32);
   m.def("mid_linear(Tensor x, Tensor w, Tensor(a!) out, bool glu, Tensor(b!) slab, Tensor(c!) counters) -> bool", &mid_linear);
   m.def("relu_sq(Tensor a, Tensor(a!) out) -> ()", &relu_sq);
   m.def("silu_mul(Tensor gate, Tensor up, Tensor(a!) out) -> ()", &silu_mul);

@@ -74,6 +74,7 @@ void launch_conv_state_update(const ConvArgs& a, int f32, hipStream_t s);
 constexpr long long MID_SLAB = 256LL * 128 * 256;
 bool launch_mid_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int glu, float* slab,
                        int* counters, hipStream_t s);
+bool launch_mid_linear_f32(const void* x, long long ldx, const void* W, float* out, long long ldo, int M, int N, int K, hipStream_t s);
 // out = x . W^T (relu2: of relu(x)^2; glu: silu(gate) * up of W's [gate | up] rows); false: this K has no kernel
 bool launch_row_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int f32_out,
                        int relu2, int glu, hipStream_t s);

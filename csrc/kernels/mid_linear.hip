@@ -50,7 +50,7 @@ struct Cfg {
   static_assert(SLOTS >= 3 && KEEP <= 63, "ring");
 };
 
-template <int MT, int WV, bool GLU>
+template <int MT, int WV, bool GLU, bool F32 = false>
 __global__ __launch_bounds__(64 * WV, 1) void mid_linear_kernel(Args a) {
   using C = Cfg<MT, WV, GLU>;
   constexpr int RW = C::RW;
@@ -97,11 +97,15 @@ __global__ __launch_bounds__(64 * WV, 1) void mid_linear_kernel(Args a) {
 
   const int j = lane & 15, h = lane >> 4;
   const int fo = j * 128 + 16 * (h ^ ((j >> 1) & 7));      // a fragment's piece of the first step; of the second: 64 bytes across
-  f32x4 acc[RW][MT];
+  // F32: the sums are the result, of all of K: in parts of 256, as long chains lose bits
+  f32x4 acc[RW][MT], total[F32 ? RW : 1][F32 ? MT : 1];
 #pragma unroll
   for (int rt = 0; rt < RW; ++rt)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int mt = 0; mt < MT; ++mt) {
+      acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (F32) total[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
   struct Frag {
     bf16x8 w[RW], x[MT];
   };
@@ -146,6 +150,15 @@ __global__ __launch_bounds__(64 * WV, 1) void mid_linear_kernel(Args a) {
     asm volatile("" ::: "memory");
     if (c + C::SLOTS < nch) issue(c + C::SLOTS, slot);
     step(f0, after, 0, f1, true, true);
+    if (F32 && c % 4 == 3) {
+#pragma unroll
+      for (int rt = 0; rt < (F32 ? RW : 0); ++rt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          total[rt][mt] += acc[rt][mt];
+          acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
     slot = after;
   }
   step(f1, slot, 1, f0, true, true);
@@ -205,6 +218,10 @@ __global__ __launch_bounds__(64 * WV, 1) void mid_linear_kernel(Args a) {
   for (int mt = 0; mt < MT; ++mt) {
     const int m = 16 * mt + j;
     if (m >= M) continue;
+    if constexpr (F32) {
+      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + (long long)m * a.ldo + n) = acc[0][mt] + total[0][mt];
+      continue;
+    }
     bf16x4 y;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -271,5 +288,18 @@ bool launch_mid_linear(const void* x, long long ldx, const void* W, void* out, l
   else if (best == 3) glu ? run_rows<3, true>(a, splits, s) : run_rows<3, false>(a, splits, s);
   else if (best == 4) glu ? run_rows<4, true>(a, splits, s) : run_rows<4, false>(a, splits, s);
   else run_rows<5, false>(a, splits, s);
+  return true;
+}
+
+// ... of 17 to 64 rows into fp32, over all of K, in rounds of workgroups of 64 outputs: an lm_head, 32768 x 2048 at 24 rows 26.8 us
+// (5 TB/s; the library 36.4), 65536 x 4096 at 32 94 (125)
+bool launch_mid_linear_f32(const void* x, long long ldx, const void* W, float* out, long long ldo, int M, int N, int K, hipStream_t s) {
+  const Args a{(const bf16*)x, (const bf16*)W, (bf16*)out, nullptr, nullptr, (int)ldx, (int)ldo, M, N, K, K / 64};
+  constexpr long long top = 0x7fffffffLL;
+  if (M < 1 || M > 64 || K % 64 || N % 4 || 64 * ldx * 2 + K * 2LL > top || 2LL * N * K > top) return false;
+  const int groups = (N + 63) / 64;
+  if (M <= 32) mid_linear_kernel<2, 4, false, true><<<groups, 256, 0, s>>>(a);
+  else if (M <= 48) mid_linear_kernel<3, 4, false, true><<<groups, 256, 0, s>>>(a);
+  else mid_linear_kernel<4, 4, false, true><<<groups, 256, 0, s>>>(a);
   return true;
 }

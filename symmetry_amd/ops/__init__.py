@@ -735,7 +735,31 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Ten
     if few_rows(x, w, out) and out.dtype == torch.float32 and out.shape[1] == w.shape[0]:
         row_linear(x, w, out)
         return out
+    if mid_f32(x, w, out) and _hyb().mid_linear_f32(x, w, out):
+        return out
     return torch.mm(x, w.t(), out_dtype=torch.float32, out=out)
+
+
+def mid_f32_pays(M: int, N: int, K: int) -> bool:
+    """Is the medium-row kernel the better choice for fp32 outputs (an lm_head)?  Where the weight's rows lie a power of two apart: the
+    library's workgroups ask the same few memory channels then.  us, library / kernel: 32768 x 2048 at 24 rows 36.4 / 26.8, 64
+    37.5 / 33.1; 32000 x 4096 at 17 58.5 / 44.8, 48 67.0 / 49.3; 65536 x 4096 at 32 125 / 94; 10240 x 8192 at 40 44.0 / 40.6, 64
+    44.2 / 48.4; 50304 x 4096 at 64 99 / 106; 128256 x 4096 at 48 220 / 211.  Else they are even or the library's: 32000 x 5120 at
+    32 62.8 / 61.7, 65536 x 2560 at 40 69.4 / 72.8, 50304 x 1536 at 17 33.8 / 35.4, and so are outputs that leave CUs idle, in a
+    round or the second (8192 x 4096 at 17 17.1 / 20.2; 20480 x 3072 at 17 29.2 / 30.1)."""
+    if not FEW_ROWS < M <= (64 if K <= 2048 else 48) or K < 1024 or K & (K - 1):
+        return False
+    return 10240 <= N <= 16384 or N > 28608
+
+
+def mid_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None) -> bool:
+    """Does x @ w.T into fp32 ``out`` run on the medium-row kernel?  few_rows' conditions but for the rows, where it pays."""
+    if _traced(x, w, out) or x.dim() != 2 or out.dim() != 2 or out.dtype != torch.float32:
+        return False
+    M, K = x.shape
+    if not mid_f32_pays(M, out.shape[1], K) or w.shape[0] != out.shape[1] or 2 * w.numel() > 0x7FFFFFFF:
+        return False
+    return K <= x.stride(0) <= 1 << 20 and out.stride(0) <= 1 << 28 and _own_linear(x, w, out)
 
 
 def lib_splits(M: int, N: int, K: int) -> int:

@@ -162,3 +162,44 @@ def test_the_wide_rule_names_no_size_without_a_plan():
         assert all(ops.mid_pays_wide(64, most, K, glu) for K in (1536, 4096, 8192))
         assert not any(ops.mid_pays_wide(M, most + 4, K, glu) for M in ROWS for K in (1536, 2048, 4096, 8192, 14336))
         assert not any(ops.mid_pays_wide(M, 1020, 4096, glu) or ops.mid_pays_wide(M, 4096, 1472, glu) for M in ROWS)
+
+
+# row tiles at their ends; a last workgroup of one output quad and one round more; K of two parts and of many; wider rows of x and out
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(17, 10240, 1024), (32, 10244, 2048), (33, 16384, 1024), (48, 28612, 2048), (49, 10240, 2048),
+                                   (64, 32772, 1024), (48, 10300, 4096)])
+def test_fp32_outputs(gpu, M, N, K):
+    """linear_f32's sums against 64-bit ones: a chain of 8 instructions a part of 256 and the parts' own chain, each of fp32 sums: the
+    error's norm stays under 2^-24 (sqrt(8) + sqrt(K / 256)) of the result's."""
+    g = torch.Generator(device=gpu).manual_seed(N + K + M)
+    x = torch.randn(M, K + 64, device=gpu, generator=g).bfloat16()[:, 32:32 + K]
+    w = (torch.randn(N, K, device=gpu, generator=g) * K ** -0.5).bfloat16()
+    room = torch.full((M + 1, N + 8), 7.0, device=gpu)
+    out = room[:M, :N]
+    assert ops.mid_f32(x, w, out)
+    ops.linear_f32(x, w, out)
+    want = x.double() @ w.double().t()
+    assert float((out.double() - want).norm() / want.norm()) <= 2 ** -24 * (8 ** 0.5 + (K / 256) ** 0.5)
+    assert bool((room[:, N:] == 7).all()) and bool((room[M] == 7).all())
+    with torch.enable_grad():
+        assert not ops.mid_f32(x, w.requires_grad_(True), out)
+
+
+@pytest.mark.gpu
+def test_fp32_outputs_that_stay_with_the_library(gpu):
+    g = torch.Generator(device=gpu).manual_seed(4)
+
+    def rnd(*shape):
+        return torch.randn(*shape, device=gpu, generator=g).bfloat16()
+
+    flat = rnd(10240 * 2048 + 8)
+    forms = [(rnd(65, 2048), rnd(10240, 2048)), (rnd(49, 4096), rnd(10240, 4096)), (rnd(17, 2304), rnd(10240, 2304)),
+             (rnd(17, 2048), rnd(20480, 2048)), (rnd(17, 2048), rnd(10236, 2048)), (rnd(17, 2048), rnd(10242, 2048)),
+             (rnd(17, 2048), flat[1:1 + 10240 * 2048].view(10240, 2048)), (rnd(2048, 17).t(), rnd(10240, 2048)),
+             (rnd(17, 2048), rnd(2048, 10240).t()), (rnd(1, 2048).expand(20, 2048), rnd(10240, 2048))]
+    for x, w in forms:
+        out = torch.empty(x.shape[0], w.shape[0], device=gpu)
+        assert not ops.mid_f32(x, w, out)
+        ops.linear_f32(x, w, out)
+        want = x.double() @ w.double().t()
+        assert float((out.double() - want).norm() / want.norm()) <= 2 ** -24 * x.shape[1] ** 0.5
