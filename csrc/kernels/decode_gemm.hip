@@ -486,7 +486,9 @@ SYM_DEV void xres_body(const bf16* __restrict__ x, const bf16* __restrict__ W, i
 #pragma unroll
       for (int w = 1; w < NW; ++w) {
         v += red[buf][w][lane];
-        if ((w & 3) == 3) asm volatile("" : "+v"(v)::"memory");  // <= 4 partials in registers at a time
+        // partials in registers at a time: as many as the 128 of a lane of sixteen waves have room for beside the weights (four at a
+        // time were four LDS latencies at the end of every tile: a step of 17 such launches 418.0 -> 416.1 us, 2048 wide 265.6 -> 263.3)
+        if ((w & (U > 2 ? 7 : 15)) == (U > 2 ? 7 : 15)) asm volatile("" : "+v"(v)::"memory");
       }
       if (i < nf) {
         finish(v, unit_tile(i));
