@@ -510,7 +510,7 @@ def moe_combine_norm(y, dst, ids, e_lo, e_hi, w, k, residual, wn, eps, out):
     if _gpu(residual):
         return _native.ops().moe_combine_norm(y, dst, ids, int(e_lo), int(e_hi), w, int(k), residual, wn, float(eps), out)
     total = torch.empty_like(residual)
-    reference.moe_combine(y, dst, ids, e_lo, e_hi, w, k, total)
+    reference.moe_combine(y, dst, ids, e_lo, e_hi, w, k, total, False)
     return reference.add_rms_norm(total, residual, wn, eps, out)
 
 

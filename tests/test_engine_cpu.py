@@ -563,6 +563,43 @@ def test_single_copy_moe_experts_match_oracle(monkeypatch):
     assert {"pg_grouped", "grouped_skinny"} <= names, calls
 
 
+@pytest.mark.parametrize("form", ["f32", "slabs", "bf16"])
+def test_moe_combine_norm_is_combine_residual_and_norm(form):
+    """The plain form of the one launch: the bits of moe_combine, then add_rms_norm; a place that is nobody's and other ranks'
+    experts count for nothing."""
+    from symmetry_amd import ops
+
+    g = torch.Generator().manual_seed(3)
+    T, d, k, E = 7, 24, 2, 4
+    y = torch.randn(*((3, T * k, d) if form == "slabs" else (T * k, d)), generator=g)
+    y = y.bfloat16() if form == "bf16" else y
+    dst = torch.randperm(T * k, generator=g).int()
+    dst[2] = -1
+    ids, w = torch.randint(0, E, (T * k,), generator=g, dtype=torch.int32), torch.rand(T * k, generator=g)
+    resid, wn = torch.randn(T, d, generator=g), torch.randn(d, generator=g).bfloat16()
+    for e_lo, e_hi in ((0, E), (1, 3)):
+        total, r0, r1 = torch.empty_like(resid), resid.clone(), resid.clone()
+        o0, o1 = (torch.empty(T, d, dtype=torch.bfloat16) for _ in range(2))
+        ops.moe_combine(y, dst, ids, e_lo, e_hi, w, k, total)
+        ops.add_rms_norm(total, r0, wn, 1e-5, o0)
+        ops.moe_combine_norm(y, dst, ids, e_lo, e_hi, w, k, r1, wn, 1e-5, o1)
+        assert torch.equal(r0, r1) and torch.equal(o0, o1)
+
+
+def test_long_prompts_of_routed_experts_match_the_oracle():
+    """A prompt past the fused rows takes the general path's MoE layers: tokens come out, and they are the oracle's."""
+    from symmetry_amd.models import reference_model as rm
+
+    eng = LLMEngine(EngineConfig(model="tiny-mixtral", device="cpu", max_num_seqs=2, max_model_len=512, num_kv_blocks=64,
+                                 block_size=16, use_graphs=False, seed=0))
+    w = eng.weights.to("cpu")
+    prompt = [3 + (11 * i) % 500 for i in range(300)]
+    out = eng.generate(prompt, SamplingParams(max_tokens=4, temperature=0.0))
+    assert len(out) == 4
+    r = rm.check_tokens(rm.forward_logits(w, prompt + out[:-1]), len(prompt), out, tol=0.05)
+    assert r["mismatches"] == 0, r
+
+
 @pytest.mark.parametrize("local,devices,share", [(None, 8, 1), ("2", 1, 2), ("4", 1, 4), ("8", 8, 1), ("4", 2, 2)])
 def test_kv_auto_blocks_split_a_shared_gpu(monkeypatch, local, devices, share):
     """Ranks that share one GPU (the one-GPU TP / EP rehearsal) read the same free HBM at about the same time: each
