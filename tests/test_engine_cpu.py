@@ -531,6 +531,7 @@ def test_single_copy_preshuffled_weights_match_oracle():
     for n in (20, 300):
         prompt = [3 + (11 * i) % 30000 for i in range(n)]
         out = eng.generate(prompt, SamplingParams(max_tokens=4, temperature=0.0))
+        assert len(out) == 4, n                              # (a step that fails leaves none: nothing to mismatch)
         r = rm.check_tokens(rm.forward_logits(w, prompt + out[:-1]), len(prompt), out, tol=0.05)
         assert r["mismatches"] == 0, (n, r)
 
@@ -557,6 +558,7 @@ def test_single_copy_moe_experts_match_oracle(monkeypatch):
     for n in (20, 300):
         prompt = [3 + (11 * i) % 500 for i in range(n)]
         out = eng.generate(prompt, SamplingParams(max_tokens=4, temperature=0.0))
+        assert len(out) == 4, n                              # (a step that fails leaves none: nothing to mismatch)
         r = rm.check_tokens(rm.forward_logits(w, prompt + out[:-1]), len(prompt), out, tol=0.05)
         assert r["mismatches"] == 0, (n, r)
     names = {c[0] for c in calls}
