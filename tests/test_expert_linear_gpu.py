@@ -139,6 +139,26 @@ def test_a_device_that_is_not_the_current_one():
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("N,K", [(300, 2048), (2048, 1536)])
+def test_rows_of_tiles_sum_alike(N, K, glu):
+    """A row's bits do not depend on the tile that it lies in, nor on how many rows its expert and the others have."""
+    torch.manual_seed(N)
+    rows, W = torch.randn(30, K).to(BF16).cuda(), (torch.randn(4, N * (2 if glu else 1), K) * K ** -0.5).to(BF16).cuda()
+    H, seen = ops._hyb(), []
+    for counts in ((30, 30, 30, 30), (0, 300, 30, 270), (700, 60, 330, 30), (129, 2580, 30, 30)):
+        src = torch.cat([torch.arange(n) for n in counts]).remainder(30).int().cuda()
+        off = torch.tensor((0,) + counts).cumsum(0).int().cuda()
+        y = torch.empty(sum(counts), N, dtype=BF16 if glu else torch.float32, device="cuda")
+        assert H.expert_linear(rows, src, W, off, y, False, 2, glu) == 2
+        for e in range(4):
+            part = y[int(off[e]):int(off[e + 1])]
+            seen.append((e, part[:30]))
+            assert torch.equal(part[30:], part[:-30])
+    for e, part in seen:
+        assert len(part) == 0 or torch.equal(part, seen[e][1])
+
+
 @pytest.mark.parametrize("E,R,N,K", [(3, 700, 256, 512), (4, 1000, 300, 576), (5, 2600, 262, 1024), (2, 1, 512, 512),
                                      (16, 9000, 2048, 512), (7, 5000, 1028, 1088), (70, 9100, 260, 512), (130, 3000, 512, 576)])
 def test_persistent_tiles(E, R, N, K):
