@@ -12,6 +12,8 @@
 #include "common.h"
 #include "hybrid_launchers.h"
 
+#include <type_traits>
+
 namespace {
 
 enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_GLU = 2 };
@@ -62,6 +64,9 @@ SYM_DEV void store_rows(const Args& a, int n0, int lane, f32x4 v, f32x4 u) {
 // With RH = 8, lanes 0-7 of 16 hold an operand's first 128 of k, lanes 8-15 its second, which a half_swap brings to the rows' own
 // lanes for the second product; rows 8-15 of the products are dropped.
 //
+// EPI_F32 sums each 128 of k apart (32768 x 2048, two waves of 1024: off by 1.9e-7 of the result in one chain, 8.7e-8 so, 8192 x 2048 1.3e-7
+// and 8.3e-8, 2048 x 14336 at 16 rows 3.7e-7 and 1.2e-7; in the same time).
+//
 // M8: RH = 8 and at most 8 rows of x, which then are read like the weights.  One product of the two registers as they are
 // holds the first half's result in its upper left quarter and the second's in its lower right one (the others mix the halves
 // and are dropped): half the x traffic, which is twice the weights' otherwise, half the matrix products and no exchange.
@@ -109,7 +114,9 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) w[b][rt][i] = ld_nt16(reinterpret_cast<const bf16*>(wb[rt] + 2 * UK * blk + wo[rt][i]));
   };
-  auto multiply = [&](int b) {
+  // parts (EPI_F32, whose sums are the result): each block's sum apart
+  auto multiply = [&](int b, auto parts) {
+    constexpr bool PARTS = decltype(parts)::value;
     Pack8 f[XL][4];
 #pragma unroll
     for (int t = 0; t < XL; ++t) {
@@ -125,16 +132,20 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
     for (int rt = 0; rt < RT; ++rt) {
       u32x4(&v)[4] = w[b][rt];
       quad_transpose(v[0], v[1], v[2], v[3]);
+      f32x4 sum = PARTS ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[rt], half = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         Pack8 p;
         p.w = v[i];
-        acc[rt] = mfma16(p.v, f[0][i].v, acc[rt]);
+        sum = mfma16(p.v, f[0][i].v, sum);
         if constexpr (XL == 2) {
           p.w = half_swap<0x3>(v[i], v[i]);
-          acc[rt] = mfma16(p.v, f[1][i].v, acc[rt]);
+          f32x4& to = EPI == EPI_F32 ? half : sum;
+          to = mfma16(p.v, f[1][i].v, to);
         }
       }
+      if constexpr (XL == 2 && EPI == EPI_F32) sum += half;
+      acc[rt] = PARTS ? acc[rt] + sum : sum;
     }
   };
   // The loads of a block stand ahead of the products of the one before (the scheduler, left alone, moves them behind to
@@ -143,18 +154,19 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
   const int per = a.K / UK / NW, s0 = wid * per, last = s0 + per - 1;
   load(0, s0);
   __builtin_amdgcn_sched_barrier(0);
+  constexpr std::integral_constant<bool, EPI == EPI_F32> parts;
   if (per == 1) {
-    multiply(0);
+    multiply(0, std::false_type());
   } else {
     for (int s = s0; s <= last; s += 2) {
       load(1, min(s + 1, last));
       __builtin_amdgcn_sched_barrier(0);
-      multiply(0);
+      multiply(0, parts);
       if (s == last) break;
       __builtin_amdgcn_sched_barrier(0);
       load(0, min(s + 2, last));
       __builtin_amdgcn_sched_barrier(0);
-      multiply(1);
+      multiply(1, parts);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -164,12 +176,12 @@ __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
   for (int rt = 0; rt < RT; ++rt) red[wid][rt][lane] = acc[rt];
   __syncthreads();
   auto sum = [&](int rt) {
-    f32x4 v = red[0][rt][lane];
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 1; i < NW; ++i) v += red[i][rt][lane];
-    if constexpr (M8) {  // lane 40 on: the second step's part
-#pragma unroll
-      for (int i = 0; i < NW; ++i) v += red[i][rt][(lane + 40) & 63];
+    for (int i = 0; i < NW; ++i) {
+      f32x4 part = red[i][rt][lane];
+      if constexpr (M8) part += red[i][rt][(lane + 40) & 63];      // lane 40 on: the second half's
+      v = i ? v + part : part;
     }
     return v;
   };

@@ -64,6 +64,23 @@ def test_row_linear_waves_and_tiles(gpu, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,K", [(32768, 2048), (8192, 2048), (12292, 1024), (6148, 4096), (20484, 2560), (3000, 8192), (64, 4096), (2048, 14336)])
+@pytest.mark.parametrize("M", [1, 8, 16])
+def test_row_linear_fp32_sums(gpu, M, N, K):
+    """fp32 results are sums of parts.  An fp32 rounding errs by 0.4 x 2^-24 of the value (uniform in an ulp, values spread over a
+    binade) and the value of a chain of n grows as sqrt(j / n): 0.4 x 2^-24 sqrt(n / 2) of its end.  A matrix instruction
+    rounds once for each 8 products: 16 times in a block of 128 (outputs up to 2048: 32 in one of 256), then once a block.  A fifth
+    for what this model leaves out."""
+    g = torch.Generator(device=gpu).manual_seed(N + K + M)
+    x, out = torch.randn(M, K, device=gpu, generator=g).bfloat16(), torch.empty(M, N, device=gpu)
+    w = (torch.randn(N, K, device=gpu, generator=g) * K ** -0.5).bfloat16()
+    assert ops.few_rows(x, w, out)
+    ops.linear_f32(x, w, out)
+    want, block = x.double() @ w.double().t(), 256 if N <= 2048 else 128
+    assert float((out.double() - want).norm() / want.norm()) <= 1.2 * 0.4 * 2 ** -24 * (block / 16 + K / block / 2) ** 0.5
+
+
+@pytest.mark.gpu
 def test_linear_accepts_every_form(gpu):
     """Strides, types, sizes and alignments that the kernel does not take stay with the library and give the same product."""
     g = torch.Generator(device=gpu).manual_seed(3)
