@@ -345,16 +345,21 @@ bool run_waves(const Args& a, int waves, hipStream_t s) {
 //   7.1 (RT 1: 7.5, 7.7, 8.1); 8192 x 4096 13.7, 14.1, 15.5 / 13.3, 12.9, 12.7), then 2 or 3 by the rounds, whose cost is
 //   a tile's each and half a tile's for x (10240 x 2048 RT 2 / 3 10.8 / 9.3 [before 11.6]; 17440 16.0 / 14.7 [16.0]; 32768
 //   23.0 / 26 [27.1])
+//   past 40960 outputs rounds run into each other: three only while they are at most 6, full to 7 / 8 (73728 x 2048 walk / three 51.0,
+//   53.4, 55.3 / 49.2, 49.9, 52.1), else the walk of 2048 (50304: 36.9, 37.3, 39.1 / 39.7, 39.9, 41.0), and one, for more rows two
+//   (100352 x 1024 one / two / three 36.2, 38.4, 44.8 / 37.1, 37.9, 40.8 / 39.7, 41.4, 44.0)
 //   one from 8192 deep on (8192 x 8192 23.8, 27.4, 33.0 / 23.4, 23.3, 25.6; RT 2 28.7, 29.1, 29.6)
 //   the walk where many tiles of few blocks, or of many, pass: 12288 x 1536 walk / tiles 8.5 / 8.8, 32768 x 1536 16.9 / 19.2 (8192 x
 //   1536 at 1, 16 rows 6.4, 7.5 / 6.9, 6.9), 28672 x 4096 37.9 / 40.2, against 16384 x 4096 23.6 / 22.6; 12288 x 3072 even
+//   (its widths are those that it is written out for: its waves hold their shares of x and of two tiles in registers, so a K needs a
+//   number of waves and blocks of its own; others, as 2304, take the tiles at every size)
 // Waves of 16-row tiles: a block each up to 8 in one round (12288 x 1024, RT 3: eight 6.2, two 6.9); then four (two of RT 3), eight
 // from 8192 deep on (3000 x 8192 12.4 / 11.4).  Where more rounds cover a wait, one for 8 blocks, at least two (32768 x 2048 two /
 // four 23.0 / 23.7, 16384 x 4096 four / two 22.6 / 25; gated 8192 x 1024 two / eight 7.7 / 9.3), four for 4 blocks.
 // Gated pairs are two tiles of 16 outputs' (1024 x 1024 4.4, 4.8, 5.0 / 4.2, 4.3, 4.3; 8192 x 8192 56, 57, 59 / 45, 46, 47).  Of the
 // walk's widths they are where they come near whole rounds (8192 x 2048 12.7, 13.0, 13.6 / 12.6, 12.6, 12.8; 4096 x 4096 14.0 to
-// 15.9 / 12.2 to 12.5; but 4360 x 2048 9.9 / 10.7, 14336 x 4096 38.7 / 41.1), with few outputs for more than 8 rows (512 x 4096
-// at 1, 16 rows 8.6, 10.7 / 9.4, 9.5).
+// 15.9 / 12.2 to 12.5; but 4360 x 2048 9.9 / 10.7, 6144 x 4096, three rounds of the walk, 19.3 / 20.7, 14336 x 4096 38.7 / 41.1), with
+// few outputs for more than 8 rows (512 x 4096 at 1, 16 rows 8.6, 10.7 / 9.4, 9.5).
 template <int EPI, bool XF>
 bool by_shape(const Args& a, hipStream_t s) {
   if (a.K <= SMALL_K) {
@@ -364,7 +369,7 @@ bool by_shape(const Args& a, hipStream_t s) {
   const int tiles = (a.N + 15) / 16, blocks = a.K / 128;
   bool walks;
   if constexpr (EPI == EPI_GLU) {
-    const bool near = (tiles > 128 && tiles <= 256) || (tiles >= 384 && tiles <= 512) || (tiles <= 128 && a.M > 8);
+    const bool near = (tiles > 128 && tiles <= 256) || (tiles > 384 && tiles <= 512) || (tiles <= 128 && a.M > 8);
     walks = a.K == 3072 || ((a.K == 2048 || a.K == 4096) && !near);
   } else {
     walks = ((a.K == 1536 || a.K == 3072) && a.N > 8192) || (a.K == 1536 && a.N > 4096 && a.M <= 4) || (a.K == 4096 && a.N > 16384);
@@ -388,7 +393,13 @@ bool by_shape(const Args& a, hipStream_t s) {
     }
     const int two = (tiles + 1) / 2, three = (tiles + 2) / 3;
     if (tiles <= 256 || blocks >= 64) return run_waves<1, 16, EPI, XF>(a, waves(1, tiles), s);
-    if (two > 256 && 7 * ((three + 255) / 256) < 5 * ((two + 255) / 256)) return run_waves<3, 16, EPI, XF>(a, waves(3, three), s);
+    const int rounds2 = (two + 255) / 256, rounds3 = (three + 255) / 256;
+    if (two > 1280 && (rounds3 > 6 || 8 * three < 7 * 256 * rounds3)) {
+      if (walk<16, 2, EPI, XF>(a, s)) return true;
+      if (a.K > 512 && (a.M <= 4 || (a.M <= 8 && 10 * two < 9 * 256 * rounds2))) return run_waves<1, 16, EPI, XF>(a, waves(1, tiles), s);
+    } else if (two > 256 && 7 * rounds3 < 5 * rounds2) {
+      return run_waves<3, 16, EPI, XF>(a, waves(3, three), s);
+    }
     return run_waves<2, 16, EPI, XF>(a, waves(2, two), s);
   }
 }
