@@ -7,16 +7,22 @@
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
+constexpr float BF16_MAX = 3.3895313892515355e38f;
+
 struct Parts {
   bf16x8 h, m, l;
 };
 
 // (two at a time: v_cvt_pk_bf16_f32 rounds a pair, and a bf16 is a float's upper half; 5.5 instructions a number, 9.7 one by one)
+// WIDE: numbers past bf16's largest, which would round to an infinity, too (the rest is in the other parts); the chunk walks' states,
+// where it costs 1 % of a walk, of all operands 4
+template <bool WIDE = false>
 SYM_DEV Parts split(f32x4 a, f32x4 b) {
   union {
     unsigned int u[4];
     bf16x8 v;
   } h, m, l;
+  auto fit = [](float x) { return WIDE ? __builtin_amdgcn_fmed3f(x, -BF16_MAX, BF16_MAX) : x; };
   auto round2 = [](float x, float y) {
     const bf16x2 p = __builtin_convertvector((f32x2){x, y}, bf16x2);
     return __builtin_bit_cast(unsigned int, p);
@@ -24,7 +30,7 @@ SYM_DEV Parts split(f32x4 a, f32x4 b) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float x = i < 2 ? a[2 * i] : b[2 * i - 4], y = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
-    h.u[i] = round2(x, y);
+    h.u[i] = round2(fit(x), fit(y));
     const float rx = x - __uint_as_float(h.u[i] << 16), ry = y - __uint_as_float(h.u[i] & 0xffff0000u);
     m.u[i] = round2(rx, ry);
     l.u[i] = round2(rx - __uint_as_float(m.u[i] << 16), ry - __uint_as_float(m.u[i] & 0xffff0000u));

@@ -390,12 +390,12 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
         bj[j] = lds4(fs + 2 * C + 16 * j + 4 * g);
       }
     }
-    Parts s = split(S[0], S[1]);
+    Parts s = split<true>(S[0], S[1]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int t = 0; t < NB; ++t) {
       Parts next = s;
-      if (t + 1 < NB) next = split(S[2 * t + 2], S[2 * t + 3]);
+      if (t + 1 < NB) next = split<true>(S[2 * t + 2], S[2 * t + 3]);
 #pragma unroll
       for (int term = 0; term < (MODE == 0 ? 6 : 3); ++term)
 #pragma unroll

@@ -642,9 +642,11 @@ __global__ __launch_bounds__(128 * MW) void delta_chunk_scan_kernel(DeltaRuleArg
 // decays per channel: k 2^G, q 2^G and k 2^(G_C - G) are staged.  NB: 32-channel blocks (N <= 32 NB, N a multiple of 8).
 // What is left is the chain of a chunk, its products a third (4000 tokens in one run, us a chunk: 2.5; without the products of the
 // state 1.8, without staging 2.4).  256 registers a lane: with more allowed the compiler keeps a part in AGPRs (348 -> 396).
-// Prep and walk, fp32 products / parts, 8 x 128 x 256, us: one decay per head 3 runs of 510 91 / 62, 8 of 1000 222 / 161, one of
-// 4000 529 / 348, of 100 35 / 26; per channel 108 / 87, 290 / 217, 567 / 420, 45 / 38.  Error against 64 bits no larger (rms of the outputs
+// Prep and walk, fp32 products / parts, 8 x 128 x 256, us: one decay per head 3 runs of 510 91 / 62, 8 of 1000 222 / 162, one of
+// 4000 529 / 355, of 100 35 / 26; per channel 108 / 87, 290 / 217, 567 / 420, 45 / 38.  Error against 64 bits no larger (rms of the outputs
 // 2.2e-7 / 2.1e-7 at 510 rows, 3.8e-7 / 3.2e-7 with slow decays).
+// An infinity or NaN of the state or a value ends as NaN in its own column from its chunk on, as with fp32 products, which meet 0 x
+// infinity in T and Aqk.
 template <bool CHANNEL, int NB, int MW>
 __global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(DeltaRuleArgs a) {
   constexpr int ST = 64 * MW;                            // staging threads
@@ -703,8 +705,8 @@ __global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(Del
         glast = last[0];
       }
     };
-    auto put = [&](bf16* m, int tt, f32x4 lo, f32x4 hi) {
-      const Parts x = split(lo, hi);
+    auto put = [&](bf16* m, int tt, f32x4 lo, f32x4 hi, auto wide) {
+      const Parts x = split<decltype(wide)::value>(lo, hi);
       auto half = [&](int part, bf16x8 v) {
         Pack8 w;
         w.v = v;
@@ -730,12 +732,12 @@ __global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(Del
               e[i][r] = __builtin_amdgcn_exp2f(rg[u][i][r]);
               w[i][r] = __builtin_amdgcn_exp2f(fminf(gl[i][r] - rg[u][i][r], 0.f));      // (rows past the run's end: k = 0)
             }
-          put(st, tt, rk[u][0] * e[0], rk[u][1] * e[1]);
-          put(st + oQ, tt, rq[u][0] * e[0], rq[u][1] * e[1]);
-          put(st + oH, tt, rk[u][0] * w[0], rk[u][1] * w[1]);
+          put(st, tt, rk[u][0] * e[0], rk[u][1] * e[1], std::false_type());
+          put(st + oQ, tt, rq[u][0] * e[0], rq[u][1] * e[1], std::true_type());
+          put(st + oH, tt, rk[u][0] * w[0], rk[u][1] * w[1], std::false_type());
         } else {
-          put(st, tt, rk[u][0], rk[u][1]);
-          put(st + oQ, tt, rq[u][0], rq[u][1]);
+          put(st, tt, rk[u][0], rk[u][1], std::false_type());
+          put(st + oQ, tt, rq[u][0], rq[u][1], std::true_type());
         }
       }
       if constexpr (CHANNEL) {
@@ -827,7 +829,7 @@ __global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(Del
       dh = fs[2 * C];
     }
     f32x4 K[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, O[2] = {K[0], K[0]};
-    Parts s = split(S[0], S[1]);
+    Parts s = split<true>(S[0], S[1]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
@@ -835,7 +837,7 @@ __global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(Del
       f32x4 d[2];
       if constexpr (CHANNEL) d[0] = lds4(fs + 32 * b + 4 * g), d[1] = lds4(fs + 32 * b + 16 + 4 * g);
       Parts next = s;
-      if (b + 1 < NB) next = split(S[2 * b + 2], S[2 * b + 3]);
+      if (b + 1 < NB) next = split<true>(S[2 * b + 2], S[2 * b + 3]);
 #pragma unroll
       for (int term = 0; term < 6; ++term) {   // the smallest terms first
         constexpr int mine[6] = {0, 2, 1, 1, 0, 0};
@@ -881,7 +883,7 @@ __global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(Del
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) U1 = mfma4(m[2][r], R1[r], U1);
-    const Parts u = CHANNEL ? split(U0, U1) : split(U0 * w[0], U1 * w[1]);
+    const Parts u = CHANNEL ? split<true>(U0, U1) : split<true>(U0 * w[0], U1 * w[1]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       O[0] = mfma4(m[3][r], U0[r], O[0]);

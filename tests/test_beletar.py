@@ -735,6 +735,45 @@ def test_delta_rule_in_parts(channel, strong, rows, shape):
     assert torch.equal(state[1].cpu(), start) and float(y[na + nb].min()) == 1e4
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("where,value", [("state", 3.4e38), ("state", -3.4e38), ("q", 3.4e38), ("state", float("inf")), ("state", float("nan")),
+                                         ("v", -float("inf"))])
+def test_delta_rule_of_extreme_values(channel, where, value):
+    """The bf16 model's chunk walk where a number is past bf16's largest, 3.39e38: it is a number like others, the bound that of the
+    parts relative to the column it scales, or to the row's terms.  An infinity and NaN stay in their value column, from their token on, as the fp32
+    products leave them; everything else is unharmed."""
+    H, N, P, n = 2, 64, 32, 100
+    q, k, v, dz, dtb, A, bz, lg, _, _ = _delta_case(channel, H, H, N, P, n, 3)
+    v, start = (0.25 * v).bfloat16(), 0.1 * torch.randn(2, H, N, P)
+    at = {"state": start[0, 0, 5], "v": v[40, 0], "q": q[40, 0]}[where]
+    at[3] = value
+    clean = [torch.nan_to_num(t.double(), 0.0, 0.0, 0.0) for t in (q, k, v)]
+    S0 = torch.nan_to_num(start[0].double(), 0.0, 0.0, 0.0)
+    want, S = O.delta_rule(clean[0], clean[1], clean[2], lg, torch.sigmoid(bz.double()), S0)
+    prev, save = torch.tensor([-2] + list(range(n - 1)), dtype=torch.int32), torch.full((n,), -1, dtype=torch.int32)
+    save[-1] = 1
+    y, ws = torch.empty(n, H, P), torch.empty(n, H, ops.delta_ws_cols(channel, N))
+    tiles = torch.tensor([[0, 0], [0, 64]], dtype=torch.int32)
+    q, k, v, dz, bz, y, ws, prev, save, cu, tiles, start, dtb, A = _dev(
+        "cuda", q, k, v, dz, bz, y, ws, prev, save, torch.tensor([0, n], dtype=torch.int32), tiles, start, dtb, A)
+    assert ops.delta_rule(channel, q, k, v, dz, dtb, A, bz, start, cu, prev, save, 1, y, tiles, ws) == 0
+    got, end = y.cpu().double(), start[1].cpu().double()
+    if torch.isfinite(torch.tensor(value)):
+        scale, ends = want.abs().amax(0, keepdim=True), S.abs().amax(1, keepdim=True)
+        if where == "q":                       # (a row's terms may cancel: its bound is relative to them)
+            scale = torch.ones(n, 1, 1, dtype=torch.float64)
+            scale[40] = value
+    else:
+        first = 40 if where == "v" else 0
+        assert not bool(torch.isfinite(got[first:, 0, 3]).any()) and not bool(torch.isfinite(end[0, :, 3]).any())
+        # (an output of v's chunk ahead of its token may meet 0 x infinity)
+        got[32 if where == "v" else 0:, 0, 3], end[0, :, 3] = want[32 if where == "v" else 0:, 0, 3], S[0, :, 3]
+        scale, ends = want.abs().max(), S.abs().max()
+    assert bool(((got - want).abs() <= 6.5e-6 * scale.clamp(min=1.0)).all())
+    assert bool(((end - S).abs() <= 3.2e-5 * ends.clamp(min=1.0)).all())
+
+
 @pytest.mark.parametrize("device,impl", FORMS)
 @pytest.mark.parametrize("channel", [False, True])
 def test_delta_rule_strong_decays_and_one_key_again(device, impl, channel):

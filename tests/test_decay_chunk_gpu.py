@@ -145,6 +145,20 @@ def test_values_that_are_not_finite(gpu, mode, what, value, H, N, P, G, lens):
     assert torch.equal(out[out.isfinite()], clean[out.isfinite()]) and torch.equal(ends[ends.isfinite()], state[ends.isfinite()])
 
 
+@pytest.mark.parametrize("mode", [ops.DECAY_CHANNEL_GATE, ops.DECAY_STEP_SIZE])
+@pytest.mark.parametrize("value", [3.4e38, -3.4e38])
+def test_states_past_the_largest_bf16(gpu, mode, value):
+    """A state between bf16's largest and fp32's is a number like others: the bounds relative to the columns that it scales."""
+    c = _Case(gpu, mode, 4, 64, 64, 2, [100, 31])
+    c.state[0, 1, 5, 3] = value
+    c.k[:, 5] = 0                              # (nothing is added to it, and what is read of it stays below fp32's largest)
+    c.q[:, 5] *= 0.125
+    want, ends = c.exact()
+    out, state = c.run(True)
+    for got, w in ((out.double(), want), (state.double(), ends)):
+        assert bool(((got - w).abs() <= 4e-6 * w.abs().amax(0 if w is want else 2, keepdim=True)).all())
+
+
 @pytest.mark.parametrize("form", ["odd channels", "odd stride", "unaligned", "no scratch", "short runs", "wide"])
 def test_forms_that_walk_token_by_token(gpu, form):
     """What the chunked form does not take gives the same recurrence (channel gate, one run from zero)."""
