@@ -602,68 +602,43 @@ MID_ROWS = 256  # rows up to which a linear layer may be the medium kernel's (cs
 
 
 def mid_pays(M: int, N: int, K: int, glu: bool = False) -> bool:
-    """Is the medium-row kernel the better choice for N outputs (glu: pairs)?  The lines stand where 15071 measured sizes put them
-    (26 N of 2048 .. 20480, 17 K of 2048 .. 28672, 43 M of 17 .. 256, 700 MB of other weights read in between).  But for layers up
-    to 2048 wide past 128 rows, 20 of the 8210 accepted sizes take 1.03 to 1.06 of the library's time; all take 0.81 on average.
+    """Is the medium-row kernel the better choice for N outputs (glu: pairs, the launch that multiplies them counted)?  Against the
+    library on 7287 sizes (21 M of 17 .. 256, 17 N of 768 .. 20480, 11 K of 1024 .. 14336, 1 GB of weights in turn), which the lines
+    follow; what it accepts takes 0.75 of the library's time, 14 sizes of 4614 (those of the host's line apart) more than 1.04.  The
+    library's time jumps where its tiles come out even, so the lines are its as much as the kernel's.  us, library / kernel:
 
-    us, library / kernel.  Up to 48 rows nearly always: 2048 x 2560 at 32 9.2 / 8.4, 17440 x 2048 at 32 22.0 / 19.0, 8192 x 4608 at
-    24 18.8 / 18.1; but 11008 x 5120 at 28 28.4 / 29.8, and a K that is a power of two sets all rows' starts on the same memory
-    channels, which tells where there are many: 8192 x 4096 at 24 17.1 / 20.4, 4096 x 8192 18.7 / 21.1.  Past that by slices of a
-    long K over few outputs (2048 x 8192 at 64 22.1 / 14.3, 96 21.0 / 16.7; 4096 x 14336 at 129 53.2 / 39.3, 190 59.1 / 47.3) and for
-    wide outputs (17440 x 2048 at 161 30.0 / 26.2, 248 33.6 / 31.7; 17440 x 3072 at 96 32.2 / 29.8, 120 34.7 / 33.4, 168 42.6 / 38.0, 208
-    43.0 / 42.1).  The library is slower at row counts in 32s, so no line is drawn at those alone: 6144 x 4096 at 200 25.8 / 31.1.
-    Pairs, with the launch that multiplied them: 8192 x 2048 at 64 22.1 / 19.5, 129 29.5 / 26.9, 161 29.7 / 30.2; 11008 x 2048 at 208
-    39.2 / 35.0; 7168 x 4096 at 49 29.5 / 33.3.
+    up to 64 rows nearly everywhere: 1024 x 2048 at 32 8.4 / 6.2, 2048 x 2048 at 40 8.5 / 7.0, 6160 x 4096 at 24 14.3 / 12.6, 8192 x 4096
+    at 24 15.9 / 13.2, 8192 x 8192 at 64 31.9 / 28.4; not 2560 x 1536 at 64 7.8 / 8.4, and some that are let through lose, 2048 x 2560 at
+    56 7.4 / 8.2
+    to 160 rows for wide outputs or a long K: 4096 x 14336 at 128 75.0 / 35.1, 17440 x 2048 at 144 29.3 / 22.3; short K over few outputs is
+    the library's (2048 x 2048 at 112 8.6 / 9.4), and so is where its tiles fill the CUs (8192 x 2560 at 144 18.6 / 20.6, 14336 x 5120 at
+    160 46.6 / 50.7)
+    past that a long K over few outputs: 4096 x 4096 at 192 32.8 / 18.7, 2048 x 8192 at 256 26.6 / 24.7; and 209 to 256 rows of 5120 to
+    10240 outputs, for which it has no good tile (5120 x 5120 at 224 44.7 / 27.6), but at 240 (8192 x 3072 24.6 / 26.8)
+    pairs nearly everywhere, a launch being saved: 8192 x 3072 at 64 26.0 / 21.9, 5120 x 5120 at 160 47.6 / 36.5; not 2048 x 1536 at 208
+    14.0 / 17.7
 
-    Past 128 rows of layers up to 2048 wide the host counts too: a prompt step that runs eagerly is not ahead of it there, and the
-    library's call costs it 20 us, this kernel's 8.5.  6144 x 2048 at 190 rows is 15.6 / 20.3, pairs 8192 x 2048 at 208 31.2 / 35.5,
-    and four layers of 200 rows with both on the kernel take 751 us, with both on the library 825 (250 rows: 815, 823).
+    Layers 2048 wide past 160 rows by the host's time: a prompt step that runs eagerly is not ahead of it there, and the library's
+    call costs it 20 us, this kernel's 8.5.  6160 x 2048 at 208 rows is 17.0 / 21.4, pairs 3664 x 2048 20.5 / 25.7, and four layers of
+    200 rows with both on the kernel take 751 us, with both on the library 825 (250 rows: 815, 823).
 
     More than 20480 outputs, or 16384 pairs, are more columns than one wave of workgroups has."""
-    if K < 2048 or N < 2048:
+    if K < 1536 or not 1024 <= N <= (16384 if glu else 20480):
         return False
+    if K == 2048 and M > 160 and N >= (2048 if glu else 4096):  # (the host's line)
+        return True
     if glu:
-        if M <= 64:
-            return K < 8192 and N <= 16384 and (K <= 2304 or not 5120 < N < 9216)
-        return K <= 2048 and M > 128 and N <= 16384
-    if N >= 16384:
-        return N <= 20480 and (K <= 2048 or (N > 16384 and (M <= 112 or (128 < M <= 192 and K <= 8192))))
-    power = K > 2048 and K & (K - 1) == 0
-    if M > 160:
-        return N >= 4096 and (K <= 2048 or (K >= 8192 and not power and N <= 6144 and M <= 192))
-    if M > 48:
-        return K >= 8192 and N <= (6144 if power else 10240) and (M <= 96 or N >= 4096)
-    if N <= 6144:
-        return (N < 4096 or K < 8192 or not power) if M <= 32 else (N >= 4096 or K >= 4096)
-    return not power and K <= ((9216 if M <= 32 else 1 << 20) if N <= 10240 else 4608)
-
-
-def mid_pays_wide(M: int, N: int, K: int, glu: bool = False) -> bool:
-    """... and where the kernel came ahead when its weights went past the caches, its workgroups started at spread places of K and its
-    column groups came in 32s and 48s too: 0.73 of the library's time on the sizes that mid_pays names (0.85 of its own before), 0.76
-    on these.  5763 measured sizes (17 to 256 rows, 1024 to 20480 outputs, K of 1536 to 14336), us, library / kernel.
-
-    Up to 64 rows nearly everywhere: 2048 x 2048 at 40 8.6 / 7.0, 1024 x 2048 at 32 8.5 / 6.2, 3664 x 2048 at 48 12.1 / 8.8, 14336 x
-    4096 at 64 27.0 / 24.4, but 2560 x 1536 at 64 7.9 / 8.4.  Past that short K over few outputs is the library's (2048 x 2048 at 100
-    8.6 / 9.3, 3072 x 1536 at 100 8.1 / 10.1), past 104 also outputs where its tiles come out even (8192 x 2560 at 144 18.6 / 20.6,
-    14336 x 3072 at 128 26.5 / 27.8, 17440 x 5120 at 128 49.0 / 52.9; 14336 x 5120 at 176 47.1 / 52.9); past 160 rows K is to be long
-    (4096 x 4096 at 176 22.6 / 18.0, 8192 x 3072 21.1 / 24.6), past 192 longer, but the library has no good tile for 209 to 256 rows
-    of 5120 to 10240 outputs (5120 x 5120 at 224 45.1 / 27.7).  Pairs are ahead nearly everywhere, a launch being saved (8192 x 3072 at
-    64 25.9 / 21.9, 5120 x 5120 at 160 48.0 / 36.5; not 2048 x 1536 at 200 13.9 / 17.6)."""
-    if K < 1536 or N < 1024:
-        return False
-    if glu:
-        return N <= 16384 and (M <= 64 or N >= 5120 or (M <= 192 and (N >= 3072 or (N >= 2048 and K >= 2048)))
-                               or (N >= 3072 and K >= 4096))
-    if M <= 64 or N > 20480:
-        return N <= 20480 and (M <= 48 or K >= 2048 or not 2304 < N < 3584)
+        return M <= 64 or N >= 5120 or (M <= 192 and (N >= 3072 or (N >= 2048 and K >= 2048))) or (N >= 3072 and K >= 4096)
+    if M <= 64:
+        return M <= 48 or K >= 2048 or not 2304 < N < 3584
     if M <= 160:
         even = K > 2304 and ((8192 <= N <= 10240 and 104 < M <= 144 and K <= 3072)
                              or (12288 <= N and M > 112 and K <= 6144 and (N < 16384 or M <= 128)))
         return (N >= 6144 or (N >= 3072 and K >= 2048) or (N >= 2048 and K >= 3072)) and not even
     if M <= 192:
         return (N >= 16384 and K <= 8192) if N >= 12288 else (K < 2048 and N >= 6144) or (K >= 4096 and N >= 3072) or (K >= 8192 and N >= 2048)
-    return (K < 2048 and N >= 8192) or (2048 <= N <= 10240 and (K >= 6144 or (M > 208 and N >= 5120 and K >= 2560)))
+    odd = M > 208 and (K >= 4608 or not 224 < M <= 240)
+    return (K < 2048 and N >= 8192) or (2048 <= N <= 10240 and (K >= 6144 or (odd and N >= 5120 and K >= 2560)))
 
 
 def mid_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None, ws, glu: bool = False) -> bool:
@@ -676,8 +651,7 @@ def _mid(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, glu: bool = False)
     if x.dim() != 2 or not FEW_ROWS < x.shape[0] <= MID_ROWS or out.dim() != 2:
         return False
     M, K = x.shape
-    N = out.shape[1]
-    if not (mid_pays(M, N, K, glu) or mid_pays_wide(M, N, K, glu)) or K % 64 or K > 1 << 20 or out.dtype != torch.bfloat16 or 2 * w.numel() > 0x7FFFFFFF:
+    if not mid_pays(M, out.shape[1], K, glu) or K % 64 or K > 1 << 20 or out.dtype != torch.bfloat16 or 2 * w.numel() > 0x7FFFFFFF:
         return False
     return K <= x.stride(0) <= 1 << 20 and out.stride(0) <= 1 << 28 and _own_linear(x, w, out)
 
