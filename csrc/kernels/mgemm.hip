@@ -58,21 +58,21 @@ SYM_DEV void mg_dma_nt(__amdgpu_buffer_rsrc_t r, int voff, int soff, char* lds) 
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_t*)lds, 16, voff, soff, 0, 2);
 }
 
-// CT weight tiles, WV waves of RW of them (the last wave may have fewer).  A chunk's 2 MT x DMAs and 2 CT weight DMAs, 1 KB each, go
-// round the waves; where they do not divide, the last ones twice
+// CT weight tiles, WV waves of RW of them.  A chunk's 2 MT x DMAs and 2 CT weight DMAs, 1 KB each, go round the waves; x's last ones
+// twice where they do not divide
 template <int MT, int CT, int WV>
 struct MgCfg {
-  static constexpr int RW = (CT + WV - 1) / WV;
+  static constexpr int RW = CT / WV;
   static constexpr int XB = 16 * MT * 128;                   // x bytes of one 64-deep chunk
   static constexpr int WB = CT * 2 * 1024;                   // weight bytes of one chunk (2 blocks per tile)
   static constexpr int SLOT = XB + WB;
   static constexpr int SLOTS = MG_LDS / SLOT > 8 ? 8 : MG_LDS / SLOT;
   static constexpr int D = SLOTS - 1;                        // chunks in flight ahead of the computed one
   static constexpr int NX = (2 * MT + WV - 1) / WV;          // x, weight DMA instructions per wave per chunk
-  static constexpr int NB = (2 * CT + WV - 1) / WV;
+  static constexpr int NB = 2 * RW;
   static constexpr int NDMA = NX + NB;
   static constexpr int VM_KEEP = (D - 1) * NDMA;             // younger DMAs left in flight at the wait
-  static_assert(D >= 1 && VM_KEEP <= 63, "mgemm config");
+  static_assert(CT == RW * WV && D >= 1 && VM_KEEP <= 63, "mgemm config");
 };
 
 // MT: 16-token tiles (M <= 16 MT); CT: 16-row weight tiles.  nt: the weights past the caches.  Weights MFMA-preshuffled
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
   int vw[C::NB];
 #pragma unroll
   for (int i = 0; i < C::NB; ++i) {
-    const int b = min(C::NB * wid + i, 2 * CT - 1);
+    const int b = C::NB * wid + i;
     vw[i] = ((b >> 1) * (K / 32) + k0 / 32 + (b & 1)) * 1024 + lane * 16;
   }
 
@@ -127,10 +127,10 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
     char* const dw = smem + slot * C::SLOT + C::XB;
     if (nt) {
 #pragma unroll
-      for (int i = 0; i < C::NB; ++i) mg_dma_nt(rw, vw[i], wo, dw + min(C::NB * wid + i, 2 * CT - 1) * 1024);
+      for (int i = 0; i < C::NB; ++i) mg_dma_nt(rw, vw[i], wo, dw + (C::NB * wid + i) * 1024);
     } else {
 #pragma unroll
-      for (int i = 0; i < C::NB; ++i) mg_dma(rw, vw[i], wo, dw + min(C::NB * wid + i, 2 * CT - 1) * 1024);
+      for (int i = 0; i < C::NB; ++i) mg_dma(rw, vw[i], wo, dw + (C::NB * wid + i) * 1024);
     }
   };
 
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
       for (int u = 0; u < PER; ++u) {
         const int i = PER * mt + u;
         if (!reads || i >= READS) continue;
-        if (i < RW) next.w[i] = *(const bf16x8*)(sb + wo_l + (2 * min(wid * RW + i, CT - 1) + s) * 1024);
+        if (i < RW) next.w[i] = *(const bf16x8*)(sb + wo_l + (2 * (wid * RW + i) + s) * 1024);
         else next.x[i - RW] = *(const bf16x8*)(sb + (s ? xo1 : xo0) + (i - RW) * 2048);
       }
       if (multiplies) {
@@ -263,7 +263,6 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
   if (EPI < 0 || S > 1) {
 #pragma unroll
     for (int rt = 0; rt < RW; ++rt) {
-      if (CT % RW && wid * RW + rt >= CT) continue;
       const int n = 16 * (tile0 + rt) + 4 * (lane >> 4);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
@@ -309,7 +308,6 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
     }
 #pragma unroll
     for (int rt = 0; rt < RW; ++rt) {
-      if (CT % RW && wid * RW + rt >= CT) continue;
       if (EPI == DECODE_EPI_ARGMAX && 16 * (tile0 + rt) >= N) continue;
       const int n = 16 * (tile0 + rt) + 4 * (lane >> 4);
 #pragma unroll
