@@ -35,7 +35,7 @@ def timed(fn, reps=20, rounds=5):
     return sorted(ts)[len(ts) // 2]
 
 
-NTS = [0]
+NTS = [1]      # (weights past the caches: what serves)
 
 
 def main():
@@ -43,7 +43,7 @@ def main():
     torch.manual_seed(0)
     Ts = [int(t) for t in os.environ.get("MG_TS", "80,128,192,256").split(",")]
     global NTS
-    NTS = [int(v) for v in os.environ.get("MG_NT", "0").split(",")]
+    NTS = [int(v) for v in os.environ.get("MG_NT", "1").split(",")]
     shapes = [("qkv", 6144, 4096), ("o", 4096, 4096), ("gate_up", 28672, 4096), ("down", 4096, 14336)]
     only = os.environ.get("MG_SHAPES")
     if only:
@@ -105,11 +105,11 @@ def main():
                         torch.ops.symmetry_amd.mgemm_nt(nt)
                         t = timed(lambda: ops.mgemm(x, ws, y, rw))
                         tc = timed(lambda: (ops.mgemm(x, ws, y, rw), consume(y)))
-                        print(json.dumps({"T": T, "gemm": name, "arm": f"mgemm rw{rw} S{S}" + (" nt" if nt else ""),
+                        print(json.dumps({"T": T, "gemm": name, "arm": f"mgemm rw{rw} S{S}" + ("" if nt else " cached"),
                                           "wgs": wgs, "gemm_us": round(t, 2), "with_consumer_us": round(tc, 2),
                                           "speedup_vs_lib": round(t_lib_c / tc, 3), "max_err": round(err, 5),
                                           "chosen": pick == (rw, S)}), flush=True)
-                    torch.ops.symmetry_amd.mgemm_nt(0)
+                    torch.ops.symmetry_amd.mgemm_nt(1)
                     del y
             del x
         del w, ws
