@@ -292,9 +292,16 @@ class TransformerLM:
 
     def _lm_head(self, rows: int):
         """(weight, wshuf) of the decode lm_head for a ``rows``-row sampling launch: the MFMA-preshuffled copy, if there is one (1
-        row of 128256 x 4096 189.5 -> 175.1 us, 24 rows 209 -> 188, 64 rows 233 -> 203; narrow models' row-tile variants of 17 rows
-        and more read the row-major weight: 32 rows of 50304 x 1024 33.0 / 33.2)."""
-        return self._dgw(-1, "lm_head") if rows <= 16 or self.cfg.hidden_size >= 1024 else (self.w["lm_head"], False)
+        row of 128256 x 4096 189.5 -> 175.1 us, 24 rows 209 -> 188, 64 rows 233 -> 203), also where outputs are too few for the
+        medium-row kernel and the decode GEMM's row tiles read it (a shard, row-major / copy: 8192 x 4096 at 17 rows 21.8 / 19.8, 64
+        30.5 / 26.7; 8016 x 2048 at 32 19.9 / 17.6; 4096 x 4096 at 64 24.9 / 22.4; only 8192 x 8192 at 17 35.9 / 36.8).  Not past 16
+        rows of models narrower than 1024, and up to 32 of 1024 over many outputs: short chains of K that the medium-row kernel pays
+        a round's start and end for (50304 x 1024 at 17 rows 31.8 / 34.0, 128256 x 1024 at 32 65.1 / 68.6, but 40960 x 1024 at 32
+        31.6 / 27.4, 50304 x 1024 at 64 47.3 / 42.4, 50304 x 1280 at 17 43.1 / 38.7)."""
+        d = self.cfg.hidden_size
+        if rows <= 16 or d > 1024 or (d == 1024 and (rows > 32 or self.vocab_shard <= 40960)):
+            return self._dgw(-1, "lm_head")
+        return self.w["lm_head"], False
 
     def _dgw(self, i: int, name: str):
         """(weight, wshuf) for decode GEMM `name` of layer i (i = -1: the lm_head)."""

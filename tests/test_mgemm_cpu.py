@@ -238,3 +238,18 @@ def test_grouped_pgemm_planner_and_reference():
     ref = torch.zeros(10, N)
     reference.grouped_gemm(xs, W, offsets, 1, ref, ops.GROUPED_F32)
     assert torch.allclose(slabs.sum(0)[2:], ref[2:], atol=1e-4) and (slabs[:, :2] == 5.0).all()
+
+
+@pytest.mark.parametrize("hidden,vocab,copied", [(768, 50304, {16}), (1024, 40960, {16, 17, 33, 64}), (1024, 50304, {16, 33, 64}),
+                                                 (1280, 50304, {16, 17, 33, 64}), (4096, 8192, {16, 17, 33, 64})])
+def test_weight_of_the_sampling_head(hidden, vocab, copied):
+    """The preshuffled copy where it was measured ahead, the row-major weight where that was, or where there is no copy."""
+    from types import SimpleNamespace
+
+    from symmetry_amd.models.transformer import TransformerLM
+
+    for copy in ({(-1, "lm_head"): "copy"}, {}):
+        m = SimpleNamespace(cfg=SimpleNamespace(hidden_size=hidden), vocab_shard=vocab, w={"lm_head": "rows"}, dgw=copy)
+        m._dgw = lambda i, name, m=m: TransformerLM._dgw(m, i, name)
+        for rows in (16, 17, 33, 64):
+            assert TransformerLM._lm_head(m, rows) == (("copy", True) if copy and rows in copied else ("rows", False)), rows
