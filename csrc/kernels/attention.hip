@@ -46,7 +46,8 @@ namespace {
 // ---------------------------------------------------------------------------------------------
 // Whole contexts on more units (sequence, kv head) than CUs: workgroup i gets the i-th longest, and those of the second round (of
 // two at most), from the last CU to the first, the rest, so that a CU's two share out evenly; of more rounds the short ones come
-// last.  All of a round is resident: what a CU has to read is what it takes (64 contexts of 450 .. 1350 tokens, 8 heads: in the
+// last.  Up to 64 sequences, whose lengths the lanes of a wave hold and rank; more keep the batch's order, turned.
+// All of a round is resident: what a CU has to read is what it takes (64 contexts of 450 .. 1350 tokens, 8 heads: in the
 // order of the batch 60.3 us, rows of it turned 59.4, so 56.1; the longest first 59.0; pairs on neighbouring CUs 61.3; 236 MB that are
 // read and not used 40.6).  A group's K loaded under the softmax before it took as long.
 constexpr int DECODE_CUS = 256;

@@ -67,7 +67,6 @@ SYM_DEV void load8(const bf16* p, float* f) {
   for (int i = 0; i < 8; ++i) f[i] = (float)pk.h[i];
 }
 
-// Non-temporal 16-byte load (streamed-once weights: MI355X_MICROARCH.md row nt-weights).
 // Where a workgroup of a weight stream starts its walk over the nch chunks of its K range (it wraps round).  In step, all workgroups
 // ask for the same bytes of their rows; a row's length is near a power of two, so these lie on a few of the memory channels.  Each
 // XCD starts an eighth further on than the one before, and an XCD's workgroups at a spread of places: where x (rows x K) would
@@ -77,6 +76,7 @@ SYM_DEV int first_chunk(unsigned wg, int nch, long long x_bytes) {
   return (int)(((wg & 7) * (unsigned)nch / 8 + (wg >> 3) * spread) % (unsigned)nch);
 }
 
+// Non-temporal 16-byte load (weights that are streamed once).
 SYM_DEV u32x4 ld_nt16(const bf16* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
 
 // A lane's registers from the lane 8 further in its row of 16, in the banks of MASK only (0x3: lanes 0-7, 0xc: 8-15).

@@ -122,10 +122,10 @@ void launch_mgemm(const bf16* x, const bf16* Wshuf, float* y, int M, int N, int 
 // mgemm with a fused consumer epilogue (DECODE_EPI_QKV / RESID / SWIGLU / F32 of decode_epi.h): y is the
 // [S][M][N] fp32 slab scratch (S > 1: in-launch split-K reduction by the last workgroup of each column group),
 // counters [N / (64 rw)] ints, zero before the first launch (re-armed by the kernel)
-// mgemm over all of K with the sampling keys' epilogue (e.y: logits too), 17..64 rows; false: the decode GEMM's call
-bool launch_mgemm_argmax(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEpi& e, hipStream_t s);
 void launch_mgemm_epi(int epi, const bf16* x, const bf16* Wshuf, float* y, int M, int N, int K, int S, int rw,
                       const DecodeEpi& e, int* counters, hipStream_t s);
+// mgemm over all of K with the sampling keys' epilogue (e.y: logits too), 17..64 rows, no scratch; false: the decode GEMM's call
+bool launch_mgemm_argmax(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEpi& e, hipStream_t s);
 void set_mgemm_nt(int on);  // non-temporal weight DMA (A/B knob)
 
 // pgemm.hip -- prefill projection GEMM (hundreds+ rows) on the MFMA-preshuffled weights: tile shape `cfg`

@@ -24,7 +24,7 @@
 //   * a step's fragments are read from LDS while the step before is multiplied: with one wave a SIMD nothing else covers the
 //     reads (a ring of its own for the weights, two chunks deeper, was slower, also with waves of its own that fill it);
 //   * what bounds it is the bytes in flight: 137 rows of 28672 x 4096 take 50 us with no product at all, and as many with them.
-//     So x tiles come in steps of 16 rows (a slot less of padding is a slot more of the ring), the chunk's DMAs are dealt to the
+//     So x tiles come in steps of 16 rows up to 192 and of 32 above (a slot less of padding is a slot more of the ring), the chunk's DMAs are dealt to the
 //     waves one by one, and the weights are loaded past the caches (read once; x stays in the L2).  Against row tiles in steps of
 //     32 and cached weights, us: 28672 x 4096 at 20 rows 41.9 -> 38.7, 64 43.1 -> 40.5, 137 57.8 -> 50.9, 192 65.0 -> 62.9;
 //     4096 x 14336 at 64 24.3 -> 22.8, 137 31.6 -> 28.6, 240 46.1 -> 40.4; 4096 x 4096 at 137 14.5 -> 13.4.
@@ -374,7 +374,7 @@ void launch_mt(const bf16* x, const bf16* W, float* y, int M, int N, int K, int 
   else launch_ct<MT, 8, EPI>(x, W, y, M, N, K, S, e, counters, s);
 }
 
-// Row tiles by EPI: steps of 16 rows where the form is used by default (the others, coarser)
+// Row tiles by EPI: steps of 16 rows up to 192 and of 32 above where the form is used by default (the others, coarser)
 template <int EPI>
 void launch_epi_m(const bf16* x, const bf16* W, float* y, int M, int N, int K, int S, int rw, const DecodeEpi& e,
                   int* counters, hipStream_t s) {
@@ -411,7 +411,7 @@ void launch_argmax(const bf16* x, const bf16* W, int M, int N, int K, const Deco
 // 8192 at 48 119 / 97 / 92; 128256 x 2048 at 64 150 / 123 / 126; 128256 x 4096 at 32 195 / 193 / 188, 64 233 / 235 / 203; 64000 x
 // 1024 at 17 34.1 / 35.6 / 36.0, 64 49 / 44 / 43.  So 128 past 32 rows of a long K, and where 64 make a second round of few (20480 x
 // 2048 at 24 rows 29.5 / 26.5 / 25.1, 24576 x 4096 at 48 54.5 / 50.4 / 42.1), but 64 in one round (16384 x 4096 at 64 51.1 / 34.1 /
-// 40.7).  Fewer outputs leave CUs idle (10240 x 8192 at 17 rows 51.4 / 33.8, but 8192 x 4096 20.5 / 23.1).
+// 40.7).  Fewer outputs leave CUs idle (10240 x 8192 at 17 rows 51.4 / 33.8, but 8192 x 4096 20.5 / 23.1) and stay with the decode GEMM, on this layout too (transformer.py::_lm_head).
 bool launch_mgemm_argmax(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEpi& e, hipStream_t s) {
   if (!e.wshuf || M <= 16 || M > 64 || K % 64 || K < 1024 || K > 1 << 20 || N % 16 || N < 10240) return false;
   if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W)) % 16) return false;
