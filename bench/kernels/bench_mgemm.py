@@ -35,15 +35,10 @@ def timed(fn, reps=20, rounds=5):
     return sorted(ts)[len(ts) // 2]
 
 
-NTS = [1]      # (weights past the caches: what serves)
-
-
 def main():
     dev = torch.device("cuda")
     torch.manual_seed(0)
     Ts = [int(t) for t in os.environ.get("MG_TS", "80,128,192,256").split(",")]
-    global NTS
-    NTS = [int(v) for v in os.environ.get("MG_NT", "1").split(",")]
     shapes = [("qkv", 6144, 4096), ("o", 4096, 4096), ("gate_up", 28672, 4096), ("down", 4096, 14336)]
     only = os.environ.get("MG_SHAPES")
     if only:
@@ -101,15 +96,12 @@ def main():
                     ops.mgemm(x, ws, y, rw)
                     torch.cuda.synchronize()
                     err = (y.sum(0) - ref).abs().max().item()
-                    for nt in NTS:
-                        torch.ops.symmetry_amd.mgemm_nt(nt)
-                        t = timed(lambda: ops.mgemm(x, ws, y, rw))
-                        tc = timed(lambda: (ops.mgemm(x, ws, y, rw), consume(y)))
-                        print(json.dumps({"T": T, "gemm": name, "arm": f"mgemm rw{rw} S{S}" + ("" if nt else " cached"),
-                                          "wgs": wgs, "gemm_us": round(t, 2), "with_consumer_us": round(tc, 2),
-                                          "speedup_vs_lib": round(t_lib_c / tc, 3), "max_err": round(err, 5),
-                                          "chosen": pick == (rw, S)}), flush=True)
-                    torch.ops.symmetry_amd.mgemm_nt(1)
+                    t = timed(lambda: ops.mgemm(x, ws, y, rw))
+                    tc = timed(lambda: (ops.mgemm(x, ws, y, rw), consume(y)))
+                    print(json.dumps({"T": T, "gemm": name, "arm": f"mgemm rw{rw} S{S}",
+                                      "wgs": wgs, "gemm_us": round(t, 2), "with_consumer_us": round(tc, 2),
+                                      "speedup_vs_lib": round(t_lib_c / tc, 3), "max_err": round(err, 5),
+                                      "chosen": pick == (rw, S)}), flush=True)
                     del y
             del x
         del w, ws

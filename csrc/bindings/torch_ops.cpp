@@ -1224,7 +1224,6 @@ TORCH_LIBRARY(symmetry_amd, m) {
       &attn_prefill);
   m.def("skinny_gemm(Tensor x, Tensor w, Tensor(a!) y, int variant=0) -> ()", &skinny_gemm);
   m.def("mgemm(Tensor x, Tensor w, Tensor(a!) y, int rw) -> ()", &mgemm);
-  m.def("mgemm_nt(int on) -> ()", [](int64_t on) { set_mgemm_nt((int)on); });
   m.def("pgemm(Tensor x, Tensor w, Tensor(a!) y, int cfg, int S, Tensor? slab, Tensor? counters) -> ()", &pgemm);
   m.def(
       "pg_qkv(Tensor x, Tensor W, Tensor? ss_in, float eps, Tensor positions, Tensor slots, Tensor cos_sin, "

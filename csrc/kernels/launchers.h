@@ -126,7 +126,6 @@ void launch_mgemm_epi(int epi, const bf16* x, const bf16* Wshuf, float* y, int M
                       const DecodeEpi& e, int* counters, hipStream_t s);
 // mgemm over all of K with the sampling keys' epilogue (e.y: logits too), 17..64 rows, no scratch; false: the decode GEMM's call
 bool launch_mgemm_argmax(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEpi& e, hipStream_t s);
-void set_mgemm_nt(int on);  // non-temporal weight DMA (A/B knob)
 
 // pgemm.hip -- prefill projection GEMM (hundreds+ rows) on the MFMA-preshuffled weights: tile shape `cfg`
 // (pgemm_cfg_shape: BM tokens x BN features per 512-thread block), S k-splits over grid.y (S > 1: slab

@@ -30,7 +30,8 @@
 //     4096 x 14336 at 64 24.3 -> 22.8, 137 31.6 -> 28.6, 240 46.1 -> 40.4; 4096 x 4096 at 137 14.5 -> 13.4.
 //     Workgroups start at different chunks (first_chunk), in step -> so, us: 28672 x 4096 at 24 rows 38.8 -> 37.9, 64 40.7 -> 39.7;
 //     16384 x 2048 at 24 14.7 -> 13.1, 137 21.6 -> 20.9; 4096 x 4096 at 24 10.1 -> 8.0, 64 10.8 -> 9.2; 2048 x 8192 at 24 8.9 -> 7.9;
-//     8192 x 8192 at 24 25.3 -> 21.9; 22016 x 4096 at 137 48.9 -> 47.5.  A K range for every
+//     8192 x 8192 at 24 25.3 -> 21.9, 225 in four slices 42.3 -> 40.7 (51.5 if an XCD's start at one place); 22016 x 4096 at 137 48.9 -> 47.5;
+//     but 2560 x 2560 at 97, slices of 8 chunks, 7.9 -> 8.2: those stay in step.  A K range for every
 //     wave, x in registers, was slower (64 to 70 at 137 rows): its waves wait for the weights each by itself;
 //   * the 16x16 accumulator of (weight tile, token tile) holds 4 consecutive features of one token per
 //     lane: one float4 store per accumulator into the slab.
@@ -75,7 +76,7 @@ struct MgCfg {
   static_assert(CT == RW * WV && D >= 1 && VM_KEEP <= 63, "mgemm config");
 };
 
-// MT: 16-token tiles (M <= 16 MT); CT: 16-row weight tiles.  nt: the weights past the caches.  Weights MFMA-preshuffled
+// MT: 16-token tiles (M <= 16 MT); CT: 16-row weight tiles.  Weights MFMA-preshuffled
 // (models/layout.py::preshuffle): block (t, kb) = 16 rows x 32 k, 1 KB in fragment order.
 // EPI < 0: the k split's fp32 slab is the output (the consumer kernel sums the slabs).  EPI >= 0: a fused
 // consumer (decode_epi.h): with one split the accumulators go straight to epilogue<EPI>; with S splits every
@@ -87,7 +88,7 @@ struct MgCfg {
 template <int MT, int CT, int EPI, int WV>
 __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restrict__ x, const bf16* __restrict__ W,
                                                            float* __restrict__ y, int M, int N, int K, int kslice,
-                                                           DecodeEpi e, int* __restrict__ counters, int nt) {
+                                                           DecodeEpi e, int* __restrict__ counters) {
   using C = MgCfg<MT, CT, WV>;
   constexpr int RW = C::RW;
   __shared__ __attribute__((aligned(1024))) char smem[C::SLOTS * C::SLOT];
@@ -118,20 +119,16 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
     vw[i] = ((b >> 1) * (K / 32) + k0 / 32 + (b & 1)) * 1024 + lane * 16;
   }
 
-  const int turn = first_chunk(blockIdx.x + gridDim.x * split, nch, (long long)M * K * 2);
+  // (of a few chunks, in step.  Spread also where x is past an L2, whose slices of K are not)
+  const int turn = nch < 16 ? 0 : first_chunk(blockIdx.x + gridDim.x * split, nch, 0);
   auto issue = [&](int c, int slot) {
     c = c + turn < nch ? c + turn : c + turn - nch;
     const int xo = c * 128, wo = c * 2048;
 #pragma unroll
     for (int i = 0; i < C::NX; ++i) mg_dma(rx, vx[i], xo, smem + slot * C::SLOT + min(C::NX * wid + i, 2 * MT - 1) * 1024);
     char* const dw = smem + slot * C::SLOT + C::XB;
-    if (nt) {
 #pragma unroll
-      for (int i = 0; i < C::NB; ++i) mg_dma_nt(rw, vw[i], wo, dw + (C::NB * wid + i) * 1024);
-    } else {
-#pragma unroll
-      for (int i = 0; i < C::NB; ++i) mg_dma(rw, vw[i], wo, dw + (C::NB * wid + i) * 1024);
-    }
+    for (int i = 0; i < C::NB; ++i) mg_dma_nt(rw, vw[i], wo, dw + (C::NB * wid + i) * 1024);
   };
 
   // ---- fragment reads: x lane holds token (16 mt + (lane & 15)), k 8 (lane >> 4) .. + 8 of step s
@@ -341,12 +338,10 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
   }
 }
 
-int g_mgemm_nt = 1;
-
 template <int MT, int CT, int EPI, int WV = 4>
 void launch_ct(const bf16* x, const bf16* W, float* y, int M, int N, int K, int S, const DecodeEpi& e, int* counters,
                hipStream_t s) {
-  mgemm_kernel<MT, CT, EPI, WV><<<dim3(N / (16 * CT), S), 64 * WV, 0, s>>>(x, W, y, M, N, K, K / S, e, counters, g_mgemm_nt);
+  mgemm_kernel<MT, CT, EPI, WV><<<dim3(N / (16 * CT), S), 64 * WV, 0, s>>>(x, W, y, M, N, K, K / S, e, counters);
 }
 
 template <int MT, int EPI>
@@ -396,7 +391,7 @@ template <int CT>
 void launch_argmax(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEpi& e, hipStream_t s) {
   const int groups = (N + 16 * CT - 1) / (16 * CT);
 #define MG_ARGMAX(t) \
-  mgemm_kernel<t, CT, DECODE_EPI_ARGMAX, 4><<<groups, 256, 0, s>>>(x, W, nullptr, M, N, K, K, e, nullptr, g_mgemm_nt)
+  mgemm_kernel<t, CT, DECODE_EPI_ARGMAX, 4><<<groups, 256, 0, s>>>(x, W, nullptr, M, N, K, K, e, nullptr)
   if (M <= 32) MG_ARGMAX(2);
   else if (M <= 48) MG_ARGMAX(3);
   else MG_ARGMAX(4);
@@ -420,8 +415,6 @@ bool launch_mgemm_argmax(const bf16* x, const bf16* W, int M, int N, int K, cons
   else launch_argmax<4>(x, W, M, N, K, e, s);
   return true;
 }
-
-void set_mgemm_nt(int on) { g_mgemm_nt = on; }
 
 void launch_mgemm(const bf16* x, const bf16* Wshuf, float* y, int M, int N, int K, int S, int rw, hipStream_t s) {
   launch_epi_m<-1>(x, Wshuf, y, M, N, K, S, rw, DecodeEpi{}, nullptr, s);

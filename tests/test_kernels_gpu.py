@@ -310,10 +310,10 @@ def test_logits_argmax(gpu):
 
 
 @pytest.mark.parametrize("M", [1, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 256])
-@pytest.mark.parametrize("chunks", [1, 2, 3, 4, 5, 8, 9, 13])
+@pytest.mark.parametrize("chunks", [1, 2, 3, 4, 5, 8, 9, 13, 15, 16, 37])
 def test_mgemm_tiles_and_ring(gpu, M, chunks):
-    """Every tile of rows at its ends, over k slices of fewer chunks than the ring has slots, as many, and one to several more,
-    for each number of weight tiles a wave.  fp32 sums of K terms err by about sqrt(K) 2^-24 of the terms' norm."""
+    """Every tile of rows at its ends, over k slices of fewer chunks than the ring has slots, as many, and one to several more
+    (from 16 on walked from other places), for each number of weight tiles a wave.  fp32 sums of K terms err by about sqrt(K) 2^-24 of the terms' norm."""
     from symmetry_amd.models.layout import preshuffle
 
     K = 2 * 64 * chunks
