@@ -46,35 +46,42 @@ namespace {
 // ---------------------------------------------------------------------------------------------
 // Whole contexts on more units (sequence, kv head) than CUs: workgroup i gets the i-th longest, and those of the second round (of
 // two at most), from the last CU to the first, the rest, so that a CU's two share out evenly; of more rounds the short ones come
-// last.  Up to 64 sequences, whose lengths the lanes of a wave hold and rank; more keep the batch's order, turned.
+// last.  Up to 64 sequences, whose lengths the lanes of a wave hold; more keep the batch's order, turned.
 // All of a round is resident: what a CU has to read is what it takes (64 contexts of 450 .. 1350 tokens, 8 heads: in the
 // order of the batch 60.3 us, rows of it turned 59.4, so 56.1; the longest first 59.0; pairs on neighbouring CUs 61.3; 236 MB that are
 // read and not used 40.6).  A group's K loaded under the softmax before it took as long.
 constexpr int DECODE_CUS = 256;
 
-SYM_DEV void by_length(const int* __restrict__ ctx_lens, int num_seqs, int Hkv, int& seq, int& kvh) {
+// The lengths are below 2^bits, and that of the rank is found bit by bit: the largest that more contexts than the rank reach.  (Each
+// lane's rank counted over all sequences instead: 64 of 450 .. 1350 tokens, 8 heads, 47.3 us, so 45.1, in the batch's order 52.6.)
+SYM_DEV void by_length(const int* __restrict__ ctx_lens, int num_seqs, int Hkv, int bits, int& seq, int& kvh) {
   const int units = num_seqs * Hkv, id = kvh * num_seqs + seq, lane = threadIdx.x & 63;
   const int k = id < DECODE_CUS || units > 2 * DECODE_CUS ? id : units - 1 - (id - DECODE_CUS);
   const int mine = (unsigned)k / (unsigned)Hkv;
   kvh = k - mine * Hkv;
-  const int len = lane < num_seqs ? ctx_lens[lane] : -1;
-  int rank = 0;
-  for (int j = 0; j < num_seqs; ++j) {
-    const int other = __builtin_amdgcn_readlane(len, j);
-    rank += other > len || (other == len && j < lane);
+  const int len = lane < num_seqs ? min(max(ctx_lens[lane], 0), (1 << bits) - 1) : -1;
+  int t = 0;
+  for (int b = bits - 1; b >= 0; --b) {
+    const int up = t | 1 << b;
+    if (__popcll(__ballot(len >= up)) > mine) t = up;
   }
-  seq = __builtin_ctzll(__ballot(rank == mine));
+  // (every ballot by all lanes: behind a && it would be one of those that are left)
+  const unsigned long long same = __ballot(len == t);
+  const int among = mine - (int)__popcll(__ballot(len > t));      // of like contexts the first first
+  const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(same >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)same, 0));
+  seq = __builtin_ctzll(same & __ballot(before == among));
 }
 
 // GMAX >= G query heads per kv head: the cross-wave merge stages GMAX columns in LDS (GMAX = 4 for
 // Llama-3 GQA: 17 KB instead of 68 KB, so LDS no longer caps the resident workgroups per CU)
-template <int GMAX, bool UNEVEN>
+// ORDER: the launcher's `order` is not 0 (a kernel of its own: the others' loads stood 0.3 us later with it inside)
+template <int GMAX, bool UNEVEN, bool ORDER>
 __global__ __launch_bounds__(DWAVES * 64, 4) void attn_decode_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
     const int* __restrict__ block_tables, const int* __restrict__ ctx_lens, bf16* __restrict__ out,
     float* __restrict__ tmp_o, float* __restrict__ tmp_ml, int* __restrict__ counters, int num_seqs, int Hq, int Hkv,
     int G, int BS, int max_blocks, int max_parts, int parts, int slots_log2, int further, float scale_log2, unsigned inv,
-    unsigned inv_heads) {
+    unsigned inv_heads, int order) {
   // UNEVEN: grid y = part * Hkv + kvh, and past Hkv * parts the further partitions, `further` items for each head (items in
   // the grid's last rows, so that they start behind the others: between them, a batch of like contexts that fills the chip
   // found its workgroups spread unevenly over the CUs, 64 x 900 tokens 61 instead of 55 us).
@@ -89,14 +96,15 @@ __global__ __launch_bounds__(DWAVES * 64, 4) void attn_decode_kernel(
       if (seq >= further) return;
     }
   }
-  if (parts == 1 && part == 0 && num_seqs <= 64 && num_seqs * Hkv > DECODE_CUS) {
-    by_length(ctx_lens, num_seqs, Hkv, seq, kvh);
-  } else if (num_seqs >= 8 && 2 * num_seqs * Hkv > DECODE_CUS && part < parts) {
-    // Workgroups go round the eight XCDs, and on one round its CUs: of 8 n sequences an XCD would get every eighth with all its
-    // heads, and a CU two heads of one.  Each row of the grid starts a sequence further on (48 of 300 .. 900 tokens, 4 heads, in
-    // halves: 22.4 -> 20.2 us; 24 in fifths 13.4 / 13.4, fewer are left as they are).
-    seq += (blockIdx.y + gridDim.y * blockIdx.z) & 7;
-    if (seq >= num_seqs) seq -= num_seqs;
+  if constexpr (ORDER) {
+    if (order > 0) {
+      if (part == 0) by_length(ctx_lens, num_seqs, Hkv, order, seq, kvh);
+    } else if (part < parts) {
+      // Workgroups go round the eight XCDs: of 8 n sequences an XCD would get every eighth with all its heads, and a CU several
+      // heads of one.  Each row of the grid starts a sequence further on.
+      seq += (blockIdx.y + gridDim.y * blockIdx.z) & 7;
+      if (seq >= num_seqs) seq -= num_seqs;
+    }
   }
   attn_decode_unit<GMAX, UNEVEN>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, num_seqs,
                                  Hq, Hkv, G, BS, max_blocks, max_parts, scale_log2, inv, seq, kvh, part, parts,
@@ -809,19 +817,28 @@ void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache,
                            : dim3(num_seqs, Hkv, parts);
   const unsigned inv = (unsigned)((1ull << 32) / parts) + 1;  // (not used for one partition)
   const unsigned inv_heads = (unsigned)((1ull << 31) / Hkv) + 1;
+  // Contexts by length (> 0: the bits of a length), the batch's order turned (-1), or as it is.  By length, us, as it is / so, 8 heads:
+  // 64 of 225 .. 675 29.0 / 25.2, of 450 .. 1350 52.6 / 45.1, of 120 with one of 1200 39.2 / 24.6; like contexts pay the lengths' round
+  // trip (64 of 900 47.1 / 47.9), and tables of 512 tokens, where all contexts are a step or two, stay (64 of 60, ranks counted 6.4 / 9.5).
+  // Turned: 96 of 120 with one of 1200, 8 heads 42.7 / 30.1, 128 of 60 with one of 600, 4 heads 20.9 / 14.6; an odd number is spread as
+  // it is (65 of 120 with one of 1200: turned 39.5, not 24.4), and contexts in parts are too (48 of 225 .. 675, 4 heads 17.1 / 17.6).
+  const long long room = (long long)max_blocks * BS;      // (no context is longer)
+  int order = 0;
+  if (parts == 1 && units > DECODE_CUS && room > 512 && room < 1 << 30)
+    order = num_seqs <= 64 ? 32 - __builtin_clz((unsigned)room) : num_seqs % 2 == 0 ? -1 : 0;
   auto run = [&](auto kern) {
     kern<<<grid, DWAVES * 64, 0, s>>>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, num_seqs,
                                       Hq, Hkv, G, BS, max_blocks, max_parts, parts, slots_log2, further, scale_log2, inv,
-                                      inv_heads);
+                                      inv_heads, order);
   };
-  auto pick = [&](auto u) {
-    constexpr bool U = decltype(u)::value != 0;
-    if (G <= 4) run(attn_decode_kernel<4, U>);
-    else if (G <= 8) run(attn_decode_kernel<8, U>);
-    else run(attn_decode_kernel<16, U>);
+  auto pick = [&](auto u, auto o) {
+    constexpr bool U = decltype(u)::value != 0, O = decltype(o)::value != 0;
+    if (G <= 4) run(attn_decode_kernel<4, U, O>);
+    else if (G <= 8) run(attn_decode_kernel<8, U, O>);
+    else run(attn_decode_kernel<16, U, O>);
   };
-  if (uneven) pick(IntC<1>{});
-  else pick(IntC<0>{});
+  if (uneven) order ? pick(IntC<1>{}, IntC<1>{}) : pick(IntC<1>{}, IntC<0>{});
+  else order ? pick(IntC<0>{}, IntC<1>{}) : pick(IntC<0>{}, IntC<0>{});
 }
 
 // Workgroups of the 64-row x 4-head kernel up to which the row kernel takes a prompt step: below, most CUs would idle; above,

@@ -162,9 +162,11 @@ def test_attn_decode(gpu, Hq, Hkv, BS):
 # more units than CUs (whole contexts, given out by length): two full rounds, a ragged second, more rounds, one head; a context far above
 # the others; past 64 sequences and below 256 units the batch's order, turned
 @pytest.mark.parametrize("S,Hq,Hkv,long", [(64, 32, 8, 0), (49, 32, 8, 0), (64, 32, 16, 0), (64, 32, 8, 3000), (65, 32, 8, 0), (48, 16, 4, 0),
-                                           (33, 32, 8, 1500), (63, 63, 63, 0)])
-def test_attn_decode_many_sequences(gpu, S, Hq, Hkv, long):
-    """Every (sequence, head) is somebody's: lengths with ties, the shortest and an empty context, whose rows stay as they are."""
+                                           (33, 32, 8, 1500), (63, 63, 63, 0), (96, 32, 8, 0), (97, 16, 4, 1500), (128, 16, 4, 0)])
+@pytest.mark.parametrize("width", [0, 9, 33])
+def test_attn_decode_many_sequences(gpu, S, Hq, Hkv, long, width):
+    """Every (sequence, head) is somebody's: lengths with ties, the shortest and an empty context, whose rows stay as they are; tables as
+    wide as the contexts (512 tokens: in the batch's order) and wider."""
     g = torch.Generator(device=gpu).manual_seed(S + Hkv)
     lens = [(37 * i * i + 11 * i) % 400 + 1 for i in range(S)]
     lens[3] = lens[S - 1] = lens[7]
@@ -172,6 +174,7 @@ def test_attn_decode_many_sequences(gpu, S, Hq, Hkv, long):
     if long:
         lens[S // 2] = long
     kc, vc, bt = _random_paged(gpu, lens, Hkv, 64, g)
+    bt = torch.nn.functional.pad(bt, (0, max(0, width - bt.shape[1]))).contiguous()
     q = torch.randn(S, Hq, 128, device=gpu, generator=g).bfloat16()
     ctx = torch.tensor(lens, device=gpu, dtype=torch.int32)
     max_parts = (bt.shape[1] * 64 + ops.ATTN_DECODE_PART - 1) // ops.ATTN_DECODE_PART
