@@ -539,10 +539,12 @@ __global__ __launch_bounds__(64 * NW) void expert_walk_kernel(ExpertArgs a) {
 SYM_DEV int chunk_swz(int row) { return (row >> 1) & 7; }
 
 // Tiles of up to 128 rows of an expert x 128 weight rows.  At a few dozen rows an expert it is a weight stream: workgroups start at
-// different stages of K (first_chunk; 16 experts, gated, in step -> so, us: 1536 x 2048 192 rows 50.9 -> 45.9, 256 49.5 -> 43.8, 800
-// 51.7 -> 46.8; 8 of 4096 x 4096 200 rows 130 -> 103; 2048 x 1536, whose rows are no power of two apart, 28.9 -> 28.5; 0.97 on average of
-// 145 sizes; the persistent tiles, which share rows in their L2, do not gain).  The place is the weight columns', not the
-// workgroup's: a row's sums are the same in every row tile and whatever other rows an expert or its neighbours have.
+// different stages of K (first_chunk; in step -> so, us: 16 experts, gated 1536 x 2048, 192 rows 50.9 -> 45.9, 800 51.7 -> 46.8; 8 of
+// 4096 x 4096 200 rows 132 -> 106; the persistent tiles, which share rows in their L2, do not gain).  Long rows that are no power
+// of two apart, or so many that rounds of workgroups are out of step by themselves, do not gain either: 2048 x 3072 of 8 experts,
+// gated 54.7 -> 56.7, 768 x 5120 73.2 -> 75.1, 16 of 4096 x 4096 198 -> 206.  The place is the weight columns', not the workgroup's:
+// a row's sums are the same in every row tile and whatever other rows an expert or its neighbours have.  (About a hundred rows of
+// an expert are no stream any more: 32 experts, gated 1024 x 4096, 3600 rows 171 -> 181.)
 template <int BM, int BN, int WR, int WC, int EPI>
 __global__ __launch_bounds__(64 * WR * WC) void expert_tile_kernel(ExpertArgs a) {
   constexpr int NWV = WR * WC, WN = BN / WC, MS = BM / WR / 16, NS = WN / 16;   // 16-row subtiles of a wave
@@ -589,7 +591,8 @@ __global__ __launch_bounds__(64 * WR * WC) void expert_tile_kernel(ExpertArgs a)
     bsrc[i] = reinterpret_cast<const bf16*>(a.W) + ((long long)e * (EPI == EPI_GLU ? 2 : 1) * N + n) * K + 8 * ch;
   }
   const unsigned int lds0 = lds_address(smem) + __builtin_amdgcn_readfirstlane(wave) * 1024;
-  const int nk = K / 64, turn = first_chunk(bx, nk, 0);
+  const int nk = K / 64;
+  const int turn = K <= 2048 || ((K & (K - 1)) == 0 && a.E * nb < 1024) ? first_chunk(bx, nk, 0) : 0;
   auto stage = [&](int kt, int buf) {
     kt = kt + turn < nk ? kt + turn : kt + turn - nk;
     const unsigned int base = lds0 + buf * STAGE;

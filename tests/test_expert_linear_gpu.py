@@ -140,7 +140,7 @@ def test_a_device_that_is_not_the_current_one():
 
 
 @pytest.mark.parametrize("glu", [False, True])
-@pytest.mark.parametrize("N,K", [(300, 2048), (2048, 1536)])
+@pytest.mark.parametrize("N,K", [(300, 2048), (2048, 1536), (300, 4096), (300, 2560)])
 def test_rows_of_tiles_sum_alike(N, K, glu):
     """A row's bits do not depend on the tile that it lies in, nor on how many rows its expert and the others have."""
     torch.manual_seed(N)
