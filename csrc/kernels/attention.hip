@@ -81,7 +81,7 @@ __global__ __launch_bounds__(DWAVES * 64, 4) void attn_decode_kernel(
     const int* __restrict__ block_tables, const int* __restrict__ ctx_lens, bf16* __restrict__ out,
     float* __restrict__ tmp_o, float* __restrict__ tmp_ml, int* __restrict__ counters, int num_seqs, int Hq, int Hkv,
     int G, int BS, int max_blocks, int max_parts, int parts, int slots_log2, int further, float scale_log2, unsigned inv,
-    unsigned inv_heads, int order) {
+    unsigned inv_heads) {
   // UNEVEN: grid y = part * Hkv + kvh, and past Hkv * parts the further partitions, `further` items for each head (items in
   // the grid's last rows, so that they start behind the others: between them, a batch of like contexts that fills the chip
   // found its workgroups spread unevenly over the CUs, 64 x 900 tokens 61 instead of 55 us).
@@ -97,6 +97,8 @@ __global__ __launch_bounds__(DWAVES * 64, 4) void attn_decode_kernel(
     }
   }
   if constexpr (ORDER) {
+    const int order = slots_log2 >> 8;      // (in the argument's upper bytes)
+    slots_log2 &= 255;
     if (order > 0) {
       if (part == 0) by_length(ctx_lens, num_seqs, Hkv, order, seq, kvh);
     } else if (part < parts) {
@@ -828,8 +830,8 @@ void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache,
     order = num_seqs <= 64 ? 32 - __builtin_clz((unsigned)room) : num_seqs % 2 == 0 ? -1 : 0;
   auto run = [&](auto kern) {
     kern<<<grid, DWAVES * 64, 0, s>>>(q, k_cache, v_cache, block_tables, ctx_lens, out, tmp_o, tmp_ml, counters, num_seqs,
-                                      Hq, Hkv, G, BS, max_blocks, max_parts, parts, slots_log2, further, scale_log2, inv,
-                                      inv_heads, order);
+                                      Hq, Hkv, G, BS, max_blocks, max_parts, parts, slots_log2 | order * 256, further, scale_log2, inv,
+                                      inv_heads);
   };
   auto pick = [&](auto u, auto o) {
     constexpr bool U = decltype(u)::value != 0, O = decltype(o)::value != 0;
