@@ -602,25 +602,28 @@ MID_ROWS = 256  # rows up to which a linear layer may be the medium kernel's (cs
 
 
 def mid_pays(M: int, N: int, K: int, glu: bool = False) -> bool:
-    """Is the medium-row kernel the better choice for N outputs (glu: pairs, the launch that multiplies them counted)?  Against the
-    library on 7287 sizes (21 M of 17 .. 256, 17 N of 768 .. 20480, 11 K of 1024 .. 14336, 1 GB of weights in turn), which the lines
-    follow; what it accepts takes 0.75 of the library's time, 14 sizes of 4614 (those of the host's line apart) more than 1.04.  The
-    library's time jumps where its tiles come out even, so the lines are its as much as the kernel's.  us, library / kernel:
+    """Is the medium-row kernel the better choice for N outputs (glu: pairs, the launch that multiplies them counted)?  The lines follow
+    29832 sizes drawn over 17 .. 256 rows, 768 .. 20480 outputs and K of 1024 .. 14336 (1 GB of weights in turn); what is accepted takes
+    0.79 of the library's time.  The library's time jumps where its tiles come out even, and where rows are a multiple of 32, for which
+    it has poor ones (8192 x 3072 at 216 rows 1.07 of its time, at 224 0.88): no line is drawn at those alone.  us, library / kernel:
 
     up to 64 rows nearly everywhere: 1024 x 2048 at 32 8.4 / 6.2, 2048 x 2048 at 40 8.5 / 7.0, 6160 x 4096 at 24 14.3 / 12.6, 8192 x 4096
-    at 24 15.9 / 13.2, 8192 x 8192 at 64 31.9 / 28.4; not 2560 x 1536 at 64 7.8 / 8.4, and some that are let through lose, 2048 x 2560 at
-    56 7.4 / 8.2
+    at 24 15.9 / 13.2, 8192 x 8192 at 64 31.9 / 28.4; not 2560 x 1536 at 64 7.8 / 8.4
     to 160 rows for wide outputs or a long K: 4096 x 14336 at 128 75.0 / 35.1, 17440 x 2048 at 144 29.3 / 22.3; short K over few outputs is
     the library's (2048 x 2048 at 112 8.6 / 9.4), and so is where its tiles fill the CUs (8192 x 2560 at 144 18.6 / 20.6, 14336 x 5120 at
     160 46.6 / 50.7)
-    past that a long K over few outputs: 4096 x 4096 at 192 32.8 / 18.7, 2048 x 8192 at 256 26.6 / 24.7; and 209 to 256 rows of 5120 to
-    10240 outputs, for which it has no good tile (5120 x 5120 at 224 44.7 / 27.6), but at 240 (8192 x 3072 24.6 / 26.8)
-    pairs nearly everywhere, a launch being saved: 8192 x 3072 at 64 26.0 / 21.9, 5120 x 5120 at 160 47.6 / 36.5; not 2048 x 1536 at 208
-    14.0 / 17.7
+    past that a long K over few outputs: 4096 x 4096 at 192 32.8 / 18.7, 2048 x 8192 at 256 26.6 / 24.7, not past 10240 (10464 x 4096 at
+    177 31.9 / 35.1, 10496 x 14336 at 189 106 / 126); and 209 to 256 rows of 5120 to 10240 outputs, for which it has no good tile, with K
+    from 4608 on (5120 x 5120 at 224 44.7 / 27.6; but 5600 x 2688 at 210 19.2 / 25.0, 6112 x 3072 at 254 22.4 / 27.6)
+    pairs nearly everywhere up to 192 rows, a launch being saved: 8192 x 3072 at 64 26.0 / 21.9, 5120 x 5120 at 160 47.6 / 36.5; not
+    2048 x 1536 at 208 14.0 / 17.7.  Past that by the mean of a band's sizes, kernel / library: 12288 and more 0.90, from 8192 with K up
+    to 4096 0.94 (past it 1.04: 12128 x 10560 at 214 149.6 / 166.0), from 3072 with K past 4096 0.85 (up to it 1.00)
 
-    Layers 2048 wide past 160 rows by the host's time: a prompt step that runs eagerly is not ahead of it there, and the library's
-    call costs it 20 us, this kernel's 8.5.  6160 x 2048 at 208 rows is 17.0 / 21.4, pairs 3664 x 2048 20.5 / 25.7, and four layers of
-    200 rows with both on the kernel take 751 us, with both on the library 825 (250 rows: 815, 823).
+    By the host's time: a prompt step that runs eagerly is not ahead of the device in models 2048 wide, and the library's call costs it 20
+    us, this kernel's 8.5.  So outputs of 3072 and more are taken up to 160 rows also where the device takes longer (3744 x 2048 at 103
+    10.0 / 11.9, 4496 x 2048 at 156 11.9 / 17.8, 2144 x 4096 at 141 13.9 / 16.2: four layers with two such, 70 to 158 rows, 645 / 620, two
+    with one, 128 to 145 rows, 518 / 498), and past that at 2048 (6160 at 208 17.0 / 21.4, pairs 3664 20.5 / 25.7; four layers of 200 rows
+    825 / 751, of 250 823 / 815).
 
     More than 20480 outputs, or 16384 pairs, are more columns than one wave of workgroups has."""
     if K < 1536 or not 1024 <= N <= (16384 if glu else 20480):
@@ -628,7 +631,9 @@ def mid_pays(M: int, N: int, K: int, glu: bool = False) -> bool:
     if K == 2048 and M > 160 and N >= (2048 if glu else 4096):  # (the host's line)
         return True
     if glu:
-        return M <= 64 or N >= 5120 or (M <= 192 and (N >= 3072 or (N >= 2048 and K >= 2048))) or (N >= 3072 and K >= 4096)
+        if M <= 192:
+            return M <= 64 or N >= 3072 or (N >= 2048 and K >= 2048)
+        return N >= 12288 or (K <= 4096 if N >= 8192 else N >= 3072 and K > 4096)
     if M <= 64:
         return M <= 48 or K >= 2048 or not 2304 < N < 3584
     if M <= 160:
@@ -636,9 +641,10 @@ def mid_pays(M: int, N: int, K: int, glu: bool = False) -> bool:
                              or (12288 <= N and M > 112 and K <= 6144 and (N < 16384 or M <= 128)))
         return (N >= 6144 or (N >= 3072 and K >= 2048) or (N >= 2048 and K >= 3072)) and not even
     if M <= 192:
-        return (N >= 16384 and K <= 8192) if N >= 12288 else (K < 2048 and N >= 6144) or (K >= 4096 and N >= 3072) or (K >= 8192 and N >= 2048)
-    odd = M > 208 and (K >= 4608 or not 224 < M <= 240)
-    return (K < 2048 and N >= 8192) or (2048 <= N <= 10240 and (K >= 6144 or (odd and N >= 5120 and K >= 2560)))
+        if N >= 12288:
+            return N >= 16384 and K <= 8192
+        return (K < 2048 and N >= 6144) or (N <= 10240 and ((K >= 4096 and N >= 3072) or (K >= 8192 and N >= 2048)))
+    return (K < 2048 and N >= 8192) or (2048 <= N <= 10240 and (K >= 6144 or (M > 208 and N >= 5120 and K >= 4608)))
 
 
 def mid_rows(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None, ws, glu: bool = False) -> bool:

@@ -91,6 +91,7 @@ def _edges(n):
     (_edges(65), (32, 8)),                                  # units past a third of the chip: one partition of several steps
     (_edges(40), (32, 8)), (_edges(30), (32, 8)),           # two and three partitions, steps that do not divide by them
     (_edges(7), (16, 16)), (_edges(3), (64, 8)),
+    (EDGES, (32, 2)), (_edges(70), (60, 5)), (_edges(6), (27, 3)), (_edges(40), (20, 4)), (_edges(9), (6, 2)),   # 16, 12, 9, 5 and 3 queries a head
     ([4700], (32, 4)), ([4673], (32, 4)), ([33], (8, 2)),   # one sequence: a partition for every step
 ])
 @pytest.mark.parametrize("BS", [32, 64])

@@ -108,14 +108,18 @@ MEASURED = {
     (17440, 2048, False): {17: True, 144: True, 161: True, 193: True, 250: True},
     (17440, 3072, False): {17: True, 128: False, 129: True, 192: True, 193: False},
     (14336, 3072, False): {112: True, 113: False, 160: False}, (14336, 5120, False): {112: True, 160: False, 176: False},
-    (8192, 2560, False): {104: True, 105: False, 144: False, 145: True, 176: False, 208: False, 209: True, 224: True, 225: False, 240: False, 241: True},
-    (8192, 3072, False): {240: False, 256: True}, (5120, 5120, False): {208: False, 224: True, 240: True},
+    (8192, 2560, False): {104: True, 105: False, 144: False, 145: True, 176: False, 208: False, 209: False, 224: False, 241: False},
+    (8192, 4544, False): {209: False, 256: False}, (8192, 4608, False): {208: False, 209: True, 256: True},
+    (5120, 5120, False): {208: False, 224: True, 240: True}, (10240, 8192, False): {161: True, 192: True, 256: True},
+    (10256, 8192, False): {160: True, 161: False, 192: False, 256: False}, (10256, 1984, False): {161: True, 192: True},
     (6160, 4096, False): {24: True, 48: True, 160: True, 192: True, 200: False}, (4096, 4096, False): {176: True, 192: True, 193: False},
     (8192, 4096, False): {17: True, 64: True, 192: True, 208: False}, (8192, 8192, False): {17: True, 64: True, 256: True},
     (2048, 8192, False): {17: True, 96: True, 176: True, 256: True}, (4096, 14336, False): {17: True, 128: True, 190: True, 256: True},
     (8192, 2048, True): {17: True, 64: True, 128: True, 160: True, 208: True}, (3664, 2048, True): {160: True, 208: True},
     (2048, 1536, True): {64: True, 65: False, 208: False}, (2048, 2048, True): {192: True, 208: True}, (2044, 2048, True): {65: False, 208: False},
     (8192, 3072, True): {64: True, 200: True}, (3072, 3072, True): {192: True, 193: False}, (5120, 5120, True): {160: True, 256: True},
+    (5120, 4096, True): {192: True, 193: False}, (3072, 4160, True): {193: True}, (3068, 4160, True): {193: False}, (8192, 4096, True): {193: True},
+    (8192, 4160, True): {192: True, 193: False}, (12284, 4160, True): {193: False}, (12288, 4160, True): {193: True},
 }
 
 
