@@ -349,7 +349,8 @@ bool run_waves(const Args& a, int waves, hipStream_t s) {
 //   past 40960 outputs rounds run into each other: three only while they are at most 6, full to 7 / 8 (73728 x 2048 walk / three 51.0,
 //   53.4, 55.3 / 49.2, 49.9, 52.1), else the walk of 2048 (50304: 36.9, 37.3, 39.1 / 39.7, 39.9, 41.0), and one, for more rows two
 //   (100352 x 1024 one / two / three 36.2, 38.4, 44.8 / 37.1, 37.9, 40.8 / 39.7, 41.4, 44.0)
-//   one from 8192 deep on (8192 x 8192 23.8, 27.4, 33.0 / 23.4, 23.3, 25.6; RT 2 28.7, 29.1, 29.6)
+//   one from 8192 deep on (8192 x 8192 23.8, 27.4, 33.0 / 23.4, 23.3, 25.6; RT 2 28.7, 29.1, 29.6), where K has eight or four shares: two
+//   waves of one tile have too few loads out (32768 x 9472 at 1, 16 rows 108.8, 122.4, so 92.0, 94.2, before 91.8, 137.6)
 //   the walk where many tiles of few blocks, or of many, pass: 12288 x 1536 walk / tiles 8.5 / 8.8, 32768 x 1536 16.9 / 19.2 (8192 x
 //   1536 at 1, 16 rows 6.4, 7.5 / 6.9, 6.9), 28672 x 4096 37.9 / 40.2, against 16384 x 4096 23.6 / 22.6; 12288 x 3072 even
 //   (its widths are those that it is written out for: its waves hold their shares of x and of two tiles in registers, so a K needs a
@@ -393,7 +394,7 @@ bool by_shape(const Args& a, hipStream_t s) {
         return true;
     }
     const int two = (tiles + 1) / 2, three = (tiles + 2) / 3;
-    if (tiles <= 256 || blocks >= 64) return run_waves<1, 16, EPI, XF>(a, waves(1, tiles), s);
+    if (tiles <= 256 || (blocks >= 64 && blocks % 4 == 0)) return run_waves<1, 16, EPI, XF>(a, waves(1, tiles), s);
     const int rounds2 = (two + 255) / 256, rounds3 = (three + 255) / 256;
     if (two > 1280 && (rounds3 > 6 || 8 * three < 7 * 256 * rounds3)) {
       if (walk<16, 2, EPI, XF>(a, s)) return true;

@@ -56,7 +56,8 @@ def test_row_linear_tiles_in_turn(gpu, M, N, K):
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,K", [(12, 512), (2044, 768), (2048, 1024), (60, 1280), (28, 1536), (36, 1792), (2048, 2816), (20, 8192), (36, 3072),
                                  (2052, 512), (4096, 768), (4092, 1280), (4100, 1024), (8192, 512), (8188, 2816), (8196, 768), (12292, 512),
-                                 (17444, 1280), (24572, 512), (2052, 8192), (40964, 768), (50304, 768), (49148, 768), (73732, 512)])
+                                 (17444, 1280), (24572, 512), (2052, 8192), (40964, 768), (50304, 768), (49148, 768), (73732, 512),
+                                 (4100, 8448), (8196, 8448)])
 @pytest.mark.parametrize("M", [1, 8, 9, 16])
 def test_row_linear_waves_and_tiles(gpu, M, N, K):
     """Every number of waves, 8-row tiles up to 2048 outputs, then one, two and three 16-row tiles a workgroup, at the lines between
