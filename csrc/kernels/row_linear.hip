@@ -339,8 +339,8 @@ bool run_waves(const Args& a, int waves, hipStream_t s) {
 //   up to 2048: 8-row tiles, so that 2048 outputs are 256 workgroups.  Up to 8 blocks of K a wave each, then four waves (2048 x
 //   2048 3.9, 4.5, 5.2 / 4.0, 4.2, 4.8; x 4096 5.5, 6.6, 8.4 / 5.4, 5.6, 7.2; x 14336 12.7, 15.7, 21.6 / 11.6, 12.4, 16.7); M8
 //   with eight where their shares would lie 4 KB apart (2048 x 8192, 8 rows: four 8.9, eight 8.8, before 10.3; x 16384 19.4,
-//   16.7, 18.1); squared ReLUs of more than 8 rows, of which every workgroup takes all, with eight or six (9 to 16 rows of 2048 x 8192
-//   four 13.3, eight 12.7, before 12.6; 512 x 8192 12.9, 11.5, 11.9; 264 x 3072 four 6.4, six 6.0, before 6.2)
+//   16.7, 18.1); squared ReLUs, of which every workgroup takes all, with eight or six (9 to 16 rows of 2048 x 8192 four 13.3, eight
+//   12.7, before 12.6; 512 x 8192 12.9, 11.5, 11.9; 264 x 3072 four 6.4, six 6.0, before 6.2; 1 to 8 of 512 x 4096 5.4, 5.1, 5.3)
 //   from 2049 on 16-row tiles, RT of them sharing x: 1 or 2 while that is one round of the 256 CUs (2560 x 2048 4.9, 6.2, 7.7 /
 //   4.9, 5.0, 5.2 (8-row tiles 5.0, 5.2, 7.5); 4096 x 2048 6.4, 6.6, 7.5 / 5.2, 5.3, 5.6; 6144 x 2048 8.3, 8.5, 9.0 / 6.9, 6.9,
 //   7.1 (RT 1: 7.5, 7.7, 8.1); 8192 x 4096 13.7, 14.1, 15.5 / 13.3, 12.9, 12.7), then 2 or 3 by the rounds, whose cost is
@@ -389,8 +389,8 @@ bool by_shape(const Args& a, hipStream_t s) {
   } else {
     if (a.N <= 2048 && a.K % 256 == 0) {
       const int deep = a.K / 256;
-      if (a.M <= 8 ? run_waves<1, 8, EPI, XF, true>(a, deep <= 8 ? deep : deep % 32 ? 4 : 8, s)
-                   : run_waves<1, 8, EPI, XF>(a, deep <= 8 ? deep : !XF ? 4 : deep % 8 ? 6 : 8, s))
+      const int most = XF ? (deep % 8 ? 6 : 8) : a.M <= 8 && deep % 32 == 0 ? 8 : 4, shares = deep <= 8 ? deep : most;
+      if (a.M <= 8 ? run_waves<1, 8, EPI, XF, true>(a, shares, s) : run_waves<1, 8, EPI, XF>(a, shares, s))
         return true;
     }
     const int two = (tiles + 1) / 2, three = (tiles + 2) / 3;
