@@ -296,12 +296,15 @@ class TransformerLM:
         medium-row kernel and the decode GEMM's row tiles read it (a shard, row-major / copy: 8192 x 4096 at 17 rows 21.8 / 19.8, 64
         30.5 / 26.7; 8016 x 2048 at 32 19.9 / 17.6; 4096 x 4096 at 64 24.9 / 22.4; only 8192 x 8192 at 17 35.9 / 36.8).  Not past 16
         rows of models narrower than 1024, and up to 32 of 1024 over many outputs: short chains of K that the medium-row kernel pays
-        a round's start and end for (50304 x 1024 at 17 rows 31.8 / 34.0, 128256 x 1024 at 32 65.1 / 68.6, but 40960 x 1024 at 32
-        31.6 / 27.4, 50304 x 1024 at 64 47.3 / 42.4, 50304 x 1280 at 17 43.1 / 38.7)."""
-        d = self.cfg.hidden_size
-        if rows <= 16 or d > 1024 or (d == 1024 and (rows > 32 or self.vocab_shard <= 40960)):
-            return self._dgw(-1, "lm_head")
-        return self.w["lm_head"], False
+        a round's start and end for (50304 x 1024 at 17 rows 32.3 / 34.9, 128256 x 1024 at 32 61.8 / 68.7, but 49152 at 32 32.5 /
+        29.6, 50304 at 40 43.1 / 39.6, 50304 x 1280 at 17 43.1 / 38.7).  The row-major weight's kernels share x among four tiles of
+        16 outputs, past 24 rows eight; vocabularies that these do not divide take one by one (119968 x 1024 at 17 100.4 / 65.8, 70000
+        at 32 73.7 / 44.3)."""
+        if rows > 16 and self.cfg.hidden_size <= 1024:
+            together, few = (64, 40960) if rows <= 24 else (128, 49152)
+            if self.cfg.hidden_size < 1024 or (rows <= 32 and self.vocab_shard > few and self.vocab_shard % together == 0):
+                return self.w["lm_head"], False
+        return self._dgw(-1, "lm_head")
 
     def _dgw(self, i: int, name: str):
         """(weight, wshuf) for decode GEMM `name` of layer i (i = -1: the lm_head)."""

@@ -240,8 +240,9 @@ def test_grouped_pgemm_planner_and_reference():
     assert torch.allclose(slabs.sum(0)[2:], ref[2:], atol=1e-4) and (slabs[:, :2] == 5.0).all()
 
 
-@pytest.mark.parametrize("hidden,vocab,copied", [(768, 50304, {16}), (1024, 40960, {16, 17, 33, 64}), (1024, 50304, {16, 33, 64}),
-                                                 (1280, 50304, {16, 17, 33, 64}), (4096, 8192, {16, 17, 33, 64})])
+@pytest.mark.parametrize("hidden,vocab,copied", [(768, 50304, {16}), (1024, 40960, {16, 17, 25, 33, 64}), (1024, 50304, {16, 33, 64}),
+                                                 (1024, 49152, {16, 25, 33, 64}), (1024, 70000, {16, 17, 25, 33, 64}), (1024, 50240, {16, 25, 33, 64}),
+                                                 (1280, 50304, {16, 17, 25, 33, 64}), (4096, 8192, {16, 17, 25, 33, 64})])
 def test_weight_of_the_sampling_head(hidden, vocab, copied):
     """The preshuffled copy where it was measured ahead, the row-major weight where that was, or where there is no copy."""
     from types import SimpleNamespace
@@ -251,5 +252,5 @@ def test_weight_of_the_sampling_head(hidden, vocab, copied):
     for copy in ({(-1, "lm_head"): "copy"}, {}):
         m = SimpleNamespace(cfg=SimpleNamespace(hidden_size=hidden), vocab_shard=vocab, w={"lm_head": "rows"}, dgw=copy)
         m._dgw = lambda i, name, m=m: TransformerLM._dgw(m, i, name)
-        for rows in (16, 17, 33, 64):
+        for rows in (16, 17, 25, 33, 64):
             assert TransformerLM._lm_head(m, rows) == (("copy", True) if copy and rows in copied else ("rows", False)), rows
