@@ -726,14 +726,15 @@ def mid_f32_pays(M: int, N: int, K: int) -> bool:
     37.5 / 33.1; 32000 x 4096 at 17 58.5 / 44.8, 48 67.0 / 49.3; 65536 x 4096 at 32 125 / 94; 10240 x 8192 at 40 44.0 / 40.6, 64
     44.2 / 48.4; 50304 x 4096 at 64 99 / 106; 128256 x 4096 at 48 220 / 211.  Else they are even or the library's: 32000 x 5120 at
     32 62.8 / 61.7, 65536 x 2560 at 40 69.4 / 72.8, 50304 x 1536 at 17 33.8 / 35.4, and so are outputs that leave CUs idle, in a
-    round or the second (8192 x 4096 at 17 17.1 / 20.2; 20480 x 3072 at 17 29.2 / 30.1).  At 2048 many rows of 32769 to 65535 outputs
-    are the library's (50304 at 64 51.5 / 57.2), at 1024 all wide ones are (32768 at 64 16.7 / 18.9, 50304 at 17 22.3 / 25.9, 64
-    25.0 / 34.8, 128256 at 32 57.7 / 59.4) but where it has no good tile (81920 at 24 55.2 / 35.4)."""
+    round or the second (8192 x 4096 at 17 17.1 / 20.2; 20480 x 3072 at 17 29.2 / 30.1).  The library has good tiles for 49152 to 65535
+    outputs (2400 drawn sizes): there 8192 deep ones are its (52528 at 26 163 / 177), many rows of 2048 (50304 at 64 51.5 / 57.2), and at
+    1024 all past 32768 (50304 at 17 22.3 / 25.9, 64 25.0 / 34.8; but 68816 at 18 89 / 34, 110544 at 29 83 / 52), where it has them for
+    more than 48 rows from 81920 on too (96288 at 59 47.6 / 56.4)."""
     if not FEW_ROWS < M <= (64 if K <= 2048 else 48) or K < 1024 or K & (K - 1):
         return False
     if K == 1024 and N > 28608:
-        return (N <= 32768 and M <= 48) or 81920 <= N <= 100352
-    if K == 2048 and M > 40 and 32768 < N < 65536:
+        return (N <= 32768 or N >= 65536) and (M <= 48 or 65536 <= N < 81920)
+    if 49152 <= N < 65536 and (K == 8192 or (K == 2048 and M > 40)):
         return False
     return 10240 <= N <= 16384 or N > 28608
 

@@ -164,7 +164,8 @@ def test_plans(gpu, M, N, K, glu):
 # row tiles at their ends; a last workgroup of one output quad and one round more; K of two parts and of many; wider rows of x and out
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(17, 10240, 1024), (32, 10244, 2048), (33, 16384, 1024), (48, 28612, 2048), (49, 10240, 2048),
-                                   (64, 30724, 2048), (48, 10300, 4096), (40, 32772, 2048), (64, 65540, 2048)])
+                                   (64, 30724, 2048), (48, 10300, 4096), (40, 32772, 2048), (64, 65540, 2048),
+                                   (64, 49148, 2048), (64, 65536, 1024), (48, 81924, 1024)])
 def test_fp32_outputs(gpu, M, N, K):
     """linear_f32's sums against 64-bit ones: a chain of 8 instructions a part of 256 and the parts' own chain, each of fp32 sums: the
     error's norm stays under 2^-24 (sqrt(8) + sqrt(K / 256)) of the result's."""
@@ -192,7 +193,8 @@ def test_fp32_outputs_that_stay_with_the_library(gpu):
     flat = rnd(10240 * 2048 + 8)
     forms = [(rnd(65, 2048), rnd(10240, 2048)), (rnd(49, 4096), rnd(10240, 4096)), (rnd(17, 2304), rnd(10240, 2304)),
              (rnd(17, 2048), rnd(20480, 2048)), (rnd(17, 1024), rnd(32772, 1024)), (rnd(49, 1024), rnd(30720, 1024)),
-             (rnd(41, 2048), rnd(32772, 2048)), (rnd(17, 2048), rnd(10236, 2048)), (rnd(17, 2048), rnd(10242, 2048)),
+             (rnd(41, 2048), rnd(49152, 2048)), (rnd(49, 1024), rnd(81920, 1024)), (rnd(17, 8192), rnd(49152, 8192)),
+             (rnd(17, 2048), rnd(10236, 2048)), (rnd(17, 2048), rnd(10242, 2048)),
              (rnd(17, 2048), flat[1:1 + 10240 * 2048].view(10240, 2048)), (rnd(2048, 17).t(), rnd(10240, 2048)),
              (rnd(17, 2048), rnd(2048, 10240).t()), (rnd(1, 2048).expand(20, 2048), rnd(10240, 2048))]
     for x, w in forms:
