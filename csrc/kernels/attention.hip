@@ -46,14 +46,15 @@ namespace {
 // ---------------------------------------------------------------------------------------------
 // Whole contexts on more units (sequence, kv head) than CUs: workgroup i gets the i-th longest, and those of the second round (of
 // two at most), from the last CU to the first, the rest, so that a CU's two share out evenly; of more rounds the short ones come
-// last.  Up to 64 sequences, whose lengths the lanes of a wave hold; more keep the batch's order, turned.
+// last.  Up to 64 sequences, whose lengths the lanes of a wave hold; more keep the batch's order, an even
+// number of them turned.
 // All of a round is resident: what a CU has to read is what it takes (64 contexts of 450 .. 1350 tokens, 8 heads: in the
 // order of the batch 60.3 us, rows of it turned 59.4, so 56.1; the longest first 59.0; pairs on neighbouring CUs 61.3; 236 MB that are
 // read and not used 40.6).  A group's K loaded under the softmax before it took as long.
 constexpr int DECODE_CUS = 256;
 
 // The lengths are below 2^bits, and that of the rank is found bit by bit: the largest that more contexts than the rank reach.  (Each
-// lane's rank counted over all sequences instead: 64 of 450 .. 1350 tokens, 8 heads, 47.3 us, so 45.1, in the batch's order 52.6.)
+// lane's rank counted over all sequences instead: 64 of 450 .. 1350 tokens, 8 heads, 41.6 us, so 39.4, in the batch's order 46.3.)
 SYM_DEV void by_length(const int* __restrict__ ctx_lens, int num_seqs, int Hkv, int bits, int& seq, int& kvh) {
   const int units = num_seqs * Hkv, id = kvh * num_seqs + seq, lane = threadIdx.x & 63;
   const int k = id < DECODE_CUS || units > 2 * DECODE_CUS ? id : units - 1 - (id - DECODE_CUS);
@@ -820,10 +821,11 @@ void launch_attn_decode(const bf16* q, const bf16* k_cache, const bf16* v_cache,
   const unsigned inv = (unsigned)((1ull << 32) / parts) + 1;  // (not used for one partition)
   const unsigned inv_heads = (unsigned)((1ull << 31) / Hkv) + 1;
   // Contexts by length (> 0: the bits of a length), the batch's order turned (-1), or as it is.  By length, us, as it is / so, 8 heads:
-  // 64 of 225 .. 675 29.0 / 25.2, of 450 .. 1350 52.6 / 45.1, of 120 with one of 1200 39.2 / 24.6; like contexts pay the lengths' round
-  // trip (64 of 900 47.1 / 47.9), and tables of 512 tokens, where all contexts are a step or two, stay (64 of 60, ranks counted 6.4 / 9.5).
-  // Turned: 96 of 120 with one of 1200, 8 heads 42.7 / 30.1, 128 of 60 with one of 600, 4 heads 20.9 / 14.6; an odd number is spread as
-  // it is (65 of 120 with one of 1200: turned 39.5, not 24.4), and contexts in parts are too (48 of 225 .. 675, 4 heads 17.1 / 17.6).
+  // 64 of 225 .. 675 25.3 / 22.7, of 450 .. 1350 46.3 / 39.4, of 120 with one of 1200 36.8 / 23.2, of 900 39.2 / 39.1 (one batch over
+  // and over, its K/V partly in the last-level cache); not behind tables of 512 tokens, where all contexts are a step or two (64 of 60
+  // 5.7, ranks counted 8.9).  Turned: 96 of 120 with one of 1200, 8 heads 37.2 / 26.5, 128 of 60 with one of 600, 4 heads 19.8 /
+  // 13.1; an odd number is spread as it is (65 of 120 with one of 1200: turned 36.7, not 22.5), and contexts in parts are too (48 of
+  // 225 .. 675, 4 heads 16.1 / 16.5).
   const long long room = (long long)max_blocks * BS;      // (no context is longer)
   int order = 0;
   if (parts == 1 && units > DECODE_CUS && room > 512 && room < 1 << 30)
