@@ -3,7 +3,7 @@
 Weights are rotated over enough copies (>= 1 GiB) that every call streams
 from HBM, as in a real decode step (the 256 MiB Infinity Cache would
 otherwise serve repeated calls).  Variants are timed interleaved in one
-process (cdna_hip_programming.md §5.4 rule 24).
+process.
 """
 import argparse
 import json

@@ -1,6 +1,6 @@
 """Ablation probe of the prefill GEMM's main loop (csrc/kernels/pgemm.hip built standalone with -DPG_PROBE):
 full kernel vs no MFMAs (PG_ABLATE=1: DMA intake + LDS reads alone) vs no DMAs after the prologue (PG_ABLATE=2:
-MFMAs on stale slots), per tile config -- which side bounds a k-step (cdna_hip_programming.md §5.4 rule 17).
+MFMAs on stale slots), per tile config -- which side bounds a k-step.
 
   python bench/kernels/pgemm_probe.py --build     (CPU: compiles bench/kernels/pg_probe_*.so)
   python bench/kernels/pgemm_probe.py --tokens 768 --shape 28672 4096 --cfgs 0 1

@@ -347,7 +347,7 @@ __global__ __launch_bounds__(128 * HPW) void attn_prefill_lds_kernel(
 // Prefill, 32x32x16 MFMA (K4, default for GQA groups of 4k heads): same workgroup shape as the
 // LDS-staged kernel above (4 query heads of one kv head x 64 query rows, 8 waves, every K/V tile read
 // from the paged cache once per workgroup and double-buffered through LDS), with the per-wave math
-// re-tiled for v_mfma_f32_32x32x16_bf16 (cdna_hip_programming.md §3, T12-T14):
+// re-tiled for v_mfma_f32_32x32x16_bf16:
 //   * a wave owns 32 query rows of one head; per 64-key tile it issues 16 S^T MFMAs and 16 P.V MFMAs
 //     (32 cycles each); the online softmax runs per 32-key subtile over 16 scores per lane;
 //   * S^T = K . Q^T with the K rows permuted (row r loads key r with bits 2 and 3 swapped) so that
@@ -393,7 +393,7 @@ constexpr float kRescaleThr = 8.f;  // T13 threshold, log2 units
 //     [rescale decision for j]  ->  S(j+1) = K . Q^T MFMAs  ||  exp2 / bf16 pack / row-sum of S(j)
 //                               ->  P(j) . V MFMAs         ||  row max of S(j+1)
 // (an MFMA holds the wave's issue for 8 of its 32 cycles, so independent VALU placed between MFMAs
-// runs in the remaining slots; cdna_hip_programming.md T15, MI355X_MICROARCH.md cycle constants).
+// runs in the remaining slots).
 // Masks apply only to the <= 2 subtiles of a wave that touch the causal diagonal / context end (a
 // uniform branch).  K/V tiles are TRIPLE-buffered in LDS (107.5 KB, one workgroup per CU at this
 // register budget anyway): tile t+1 is resident while tile t is consumed, so S(j+1) can cross a tile

@@ -32,7 +32,7 @@ SYM_DEV void store4bf(bf16* p, float a, float b, float c, float d) {
 // Epilogue of one finished 16x16 accumulator tile (rows n0.., columns = token rows 16*mt..).
 // Lane (r16, h) holds rows n0 + 4h .. n0 + 4h + 3 of token row m = 16 * mt + r16.
 // 4 bf16 as one 8-byte write-through (sc1) store: visible to a consumer on another XCD once the
-// storing wave's vmcnt has drained (MI355X_MICROARCH.md hand-off table)
+// storing wave's vmcnt has drained
 SYM_DEV void store4bf_sc1(bf16* p, float a, float b, float c, float d) {
   Pack8 pk;
   pk.h[0] = (bf16)a;

@@ -58,7 +58,7 @@ SYM_DEV float ss_row_share(const float* __restrict__ row, int n, int lane) {
 // streaming 262 KB each): workgroup blk computes tile blk / KS over the k range of split blk % KS, stores its
 // reduced 16 x 16 fp32 partial write-through into the split-K workspace, drains, and bumps the tile's counter;
 // the workgroup whose add completes the set sums the KS partials in split order (bitwise reproducible), applies
-// the row scale and runs the epilogue, then re-arms the counter (graph-replay safe).  MI355X_MICROARCH.md
+// the row scale and runs the epilogue, then re-arms the counter (graph-replay safe).  The
 // hand-off: sc1 payload stores + agent-scope add, agent-scope (L2-bypassing) loads by the last arriver.
 template <int MT, int NW, int U, int RT, int EPI, int KS = 1>
 SYM_DEV void gemm_tile(const bf16* __restrict__ x, const bf16* __restrict__ W, int M, int N, int K,
@@ -507,7 +507,7 @@ SYM_DEV void xres_body(const bf16* __restrict__ x, const bf16* __restrict__ W, i
   }
   if constexpr (KS > 1) {
     if (wid != 0 || np == 0) return;
-    // MI355X_MICROARCH.md hand-off: write-through payload, vmcnt drain, relaxed agent add; the last split's
+    // hand-off: write-through payload, vmcnt drain, relaxed agent add; the last split's
     // wave reads the payloads with agent-scope (L2-bypassing) loads
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     int last = 0;

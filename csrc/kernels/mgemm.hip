@@ -17,7 +17,7 @@
 //   * x AND the weight blocks stream through an LDS ring of 64-deep chunks by LDS-DMA (buffer loads: x
 //     rows past M read as zeros), up to 7 chunks ahead (as many as 160 KB of LDS holds), so one counted
 //     vmcnt per chunk covers both operands (an ordinary weight load beside LDS-DMA makes hipcc drain
-//     vmcnt to 0 at its first use: cdna_hip_programming.md §5 item 4(b)); a preshuffled weight block is
+//     vmcnt to 0 at its first use); a preshuffled weight block is
 //     1 KB in fragment order, so its DMA and its ds_read_b128 are both lane-linear; the 16-B chunk index
 //     of each 128-B x row is XOR-swizzled with (row >> 1) & 7 on the DMA source and on the read, which
 //     makes the x fragment reads bank-conflict free;
@@ -81,7 +81,7 @@ struct MgCfg {
 // EPI < 0: the k split's fp32 slab is the output (the consumer kernel sums the slabs).  EPI >= 0: a fused
 // consumer (decode_epi.h): with one split the accumulators go straight to epilogue<EPI>; with S splits every
 // workgroup stores its slab, and the LAST of the S workgroups of a column group (agent-scope release /
-// acquire around a per-group counter, cdna_hip_programming.md §5 "In-launch split-K reduction") sums the S
+// acquire around a per-group counter) sums the S
 // slabs of its columns in the accumulator layout, applies the deferred-RMSNorm row scale (e.ss_in) and runs
 // the epilogue -- the separate rope_cache / add+RMSNorm / SwiGLU launches of the slab path disappear.
 // `counters` [N / (16 CT)] start at zero and are re-armed by the last arriver (graph-replay safe).
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(64 * WV, 1) void mgemm_kernel(const bf16* __restric
     if (S > 1) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's slab stores are out
       __syncthreads();
-      // hand-off without L2 maintenance (MI355X_MICROARCH.md): write-through slab stores drained above,
+      // hand-off without L2 maintenance: write-through slab stores drained above,
       // relaxed agent add, the last split reads the slabs with agent-scope (L2-bypassing) loads.  Agent
       // fences here wrote back / invalidated the XCD's whole L2 once per workgroup: the fused general path
       // ran 6.22 vs 4.43 ms per 64-client step (profiles/r3/mg_fused_ab.jsonl).

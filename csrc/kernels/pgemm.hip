@@ -14,13 +14,13 @@
 //   * orientation Y^T = W . x^T on v_mfma_f32_16x16x32_bf16: a preshuffled weight block (16 rows x 32 k)
 //     is 1 KB in A-fragment order, so its LDS-DMA and its ds_read_b128 are lane-linear (conflict-free);
 //     x rows are the B operand, staged as 64-B rows per slot with the 16-B chunk XOR-swizzled by (row >> 1) & 3
-//     on the DMA source and on the read (conflict-free ds_read_b128, cdna_hip_programming.md T2 / rule 21);
+//     on the DMA source and on the read (conflict-free ds_read_b128);
 //   * both operands by LDS-DMA (buffer_load ... lds) into a ring of 32-deep k slots (4-6 slots, up to 155 KB of
 //     the 160 KB LDS): D = slots - 1 steps are in flight, one counted vmcnt per step (every wave issues the
 //     same number of DMAs per slot -- a surplus instruction fills a dummy region), one barrier per step, the
-//     refill of the slot freed by that barrier issued before the step's MFMAs (cdna_hip_programming.md
-//     "Pipelining across barriers": raw s_barrier, never vmcnt(0) in the loop); x rows past M read as zeros;
-//   * XCD-aware tile order (cdna_hip_programming.md T1, the bijective form): consecutive tiles -- the
+//     refill of the slot freed by that barrier issued before the step's MFMAs (a raw
+//     s_barrier, never vmcnt(0) in the loop: loads stay in flight across it); x rows past M read as zeros;
+//   * XCD-aware tile order (a bijection of the workgroups): consecutive tiles -- the
 //     m-tiles of one weight column block -- run on one XCD, so each weight block is fetched from HBM once
 //     per XCD and the x slices stay L2-resident;
 //   * epilogues from the accumulators (decode_epi.h's 16x16 tile layout: lane (r16, h) holds features
@@ -242,8 +242,8 @@ __global__ __launch_bounds__(PG_THR, 1) void pgemm_kernel(const bf16* __restrict
 
   // Ping-pong over two wave groups (one wave of each per SIMD): group A (waves 0-3) reads step c's fragments in
   // phase 2c and runs its MFMAs in phase 2c + 1; group B (waves 4-7) reads in 2c + 1 and computes in 2c + 2 -- in
-  // every phase one wave of each SIMD feeds the matrix pipe while its partner reads LDS and issues DMAs
-  // (MI355X_MICROARCH.md "Two waves per SIMD").  Step c lives in slot c % SLOTS; a wave's read phase of step c
+  // every phase one wave of each SIMD feeds the matrix pipe while its partner reads LDS and issues DMAs.
+  // Step c lives in slot c % SLOTS; a wave's read phase of step c
   // also issues its share of step c + SLOTS - 1 into the slot of step c - 1 (read by both groups before).  Before
   // the barrier that opens phase 2c every wave has waited for its own DMAs of step c (vmcnt, the SLOTS - 2
   // younger steps stay in flight), so the barrier publishes the whole slot.

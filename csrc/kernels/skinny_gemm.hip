@@ -14,8 +14,8 @@
 // k split; the 4 waves split the workgroup's k range and are summed through
 // LDS.  Across workgroups the k split S writes fp32 partial slabs
 // y[S][M][N] that the consumer kernel (norm / rope / swiglu) sums in its
-// prologue -- no extra reduce launch (cdna_hip_programming.md §5, "combine
-// in the NEXT kernel's prologue").  S is chosen on the host so the grid has
+// prologue -- no extra reduce launch.
+// S is chosen on the host so the grid has
 // ~1024 workgroups (4 per CU) while keeping >= 2 k blocks per wave.
 //
 // Epilogue EPI_ARGMAX (lm_head, S == 1): instead of logits the kernel emits

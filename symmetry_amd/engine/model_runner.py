@@ -5,8 +5,7 @@
   moved with ONE async H2D copy.
 * Decode steps replay a hipGraph captured per (batch-size bucket, context
   bucket) (``torch.cuda.CUDAGraph`` is hipGraph on ROCm): the ~200 kernel
-  launches of a Llama-3-8B step become one graph launch (MI355X_MICROARCH.md
-  rows **boundary** / **graph-replay-floor**).  The context bucket bounds the
+  launches of a Llama-3-8B step become one graph launch.  The context bucket bounds the
   block-table width and therefore the split-KV grid of decode attention, so
   short chats do not launch thousands of empty partition workgroups.  Padded
   rows write no cache (slot -1) and read only the reserved block 0.
