@@ -62,7 +62,7 @@ T* optptr(const OptTensor& t) {
 }
 
 void embed_norm(const Tensor& ids, const OptTensor& src, const OptTensor& prev, const Tensor& table, const Tensor& w,
-                double eps, double offset, Tensor& x) {
+                double eps, double offset, Tensor& x, const OptTensor& w2, const OptTensor& out) {
   const int f32 = act(table, "table");
   dtype(ids, at::kInt, "ids");
   dtype(x, at::kFloat, "x");
@@ -75,8 +75,14 @@ void embed_norm(const Tensor& ids, const OptTensor& src, const OptTensor& prev, 
     dtype(*prev, at::kInt, "prev");
     TORCH_CHECK(src->numel() >= T, "embed_norm: src too short");
   }
+  TORCH_CHECK(w2.has_value() == out.has_value(), "embed_norm: out and its weight together");
+  if (out.has_value()) {
+    dtype(*w2, at::kFloat, "w2");
+    same_act(*out, f32, "out");
+    TORCH_CHECK(w2->numel() == d && out->numel() == T * d, "embed_norm: out shape");
+  }
   launch_embed_norm(ptr<int>(ids), optptr<int>(src), optptr<int>(prev), table.data_ptr(), ptr<float>(w), (float)eps,
-                    (float)offset, ptr<float>(x), (int)T, (int)d, f32, cur_stream(x));
+                    (float)offset, ptr<float>(x), optptr<float>(w2), optptr<void>(out), (int)T, (int)d, f32, cur_stream(x));
 }
 
 void rms_norm_rows(const Tensor& x, const OptTensor& rows, const Tensor& w, double eps, double offset, Tensor& out) {
@@ -97,7 +103,8 @@ void rms_norm_rows(const Tensor& x, const OptTensor& rows, const Tensor& w, doub
 }
 
 void residual_mix_norm(Tensor& x, const Tensor& a, double sa, const OptTensor& bias_a, const OptTensor& b, double sb,
-                       const OptTensor& c, double sc, const OptTensor& w, double eps, double offset, OptTensor out) {
+                       const OptTensor& c, double sc, const OptTensor& w, double eps, double offset, OptTensor out, const OptTensor& ss,
+                       int64_t ssn, double ss_eps) {
   dtype(x, at::kFloat, "x");
   TORCH_CHECK(x.dim() == 2, "residual_mix_norm: x [T, d]");
   const int64_t T = x.size(0), d = x.size(1);
@@ -133,6 +140,11 @@ void residual_mix_norm(Tensor& x, const Tensor& a, double sa, const OptTensor& b
     r.out = out->data_ptr();
     r.w = ptr<float>(*w);
   }
+  if (ss.has_value()) {
+    dtype(*ss, at::kFloat, "ss");
+    TORCH_CHECK(ss->dim() == 2 && ss->size(0) == T && ss->size(1) >= 1 && ss->size(1) <= 4096 && ssn >= 1, "residual_mix_norm: ss [T, n]");
+    r.ss = ptr<float>(*ss), r.nss = (int)ss->size(1), r.ssn = (float)ssn, r.ss_eps = (float)ss_eps;
+  }
   r.eps = (float)eps;
   r.offset = (float)offset;
   r.T = (int)T;
@@ -140,7 +152,7 @@ void residual_mix_norm(Tensor& x, const Tensor& a, double sa, const OptTensor& b
   launch_residual_mix_norm(r, f32, cur_stream(x));
 }
 
-void qkv_rope_cache(const Tensor& z, const OptTensor& bias, int64_t H, int64_t G, int64_t dk, int64_t dv,
+QkvRopeArgs rope_args(const Tensor& z, const OptTensor& bias, int64_t H, int64_t G, int64_t dk, int64_t dv,
                     const Tensor& positions, const Tensor& slots, const OptTensor& rope, Tensor& q_out, Tensor& k_cache,
                     Tensor& v_cache, int64_t half_dims) {
   const int f32 = act(z, "z", false);
@@ -178,12 +190,19 @@ void qkv_rope_cache(const Tensor& z, const OptTensor& bias, int64_t H, int64_t G
   a.q_out = q_out.data_ptr();
   a.k_cache = k_cache.data_ptr();
   a.v_cache = v_cache.data_ptr();
-  launch_qkv_rope_cache(a, (int)T, f32, cur_stream(z));
+  return a;
 }
 
-int64_t window_attn(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
+void qkv_rope_cache(const Tensor& z, const OptTensor& bias, int64_t H, int64_t G, int64_t dk, int64_t dv,
+                    const Tensor& positions, const Tensor& slots, const OptTensor& rope, Tensor& q_out, Tensor& k_cache,
+                    Tensor& v_cache, int64_t half_dims) {
+  const QkvRopeArgs a = rope_args(z, bias, H, G, dk, dv, positions, slots, rope, q_out, k_cache, v_cache, half_dims);
+  launch_qkv_rope_cache(a, (int)z.size(0), z.scalar_type() == at::kFloat, cur_stream(z));
+}
+
+WindowAttnArgs attn_args(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
                     const Tensor& row_seq, const Tensor& positions, int64_t window, double scale, const OptTensor& gate,
-                    Tensor& out, const OptTensor& tiles, const OptTensor& cu_q, int64_t impl, const OptTensor& bias,
+                    Tensor& out, const OptTensor& tiles, const OptTensor& cu_q, const OptTensor& bias,
                     int64_t keep_first, const OptTensor& sink, double softcap, const OptTensor& key_scale,
                     const OptTensor& part_o, const OptTensor& part_ml, const OptTensor& counters, int64_t part_keys) {
   const int f32 = act(q, "q");
@@ -257,15 +276,26 @@ int64_t window_attn(const Tensor& q, const Tensor& k_cache, const Tensor& v_cach
   a.out = out.data_ptr();
   a.window = (int)window;
   a.scale = (float)scale;
-  return launch_window_attn(a, f32, (int)impl, cur_stream(q));
+  return a;
 }
 
-void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dz, const Tensor& dbias,
+int64_t window_attn(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables,
+                    const Tensor& row_seq, const Tensor& positions, int64_t window, double scale, const OptTensor& gate,
+                    Tensor& out, const OptTensor& tiles, const OptTensor& cu_q, int64_t impl, const OptTensor& bias,
+                    int64_t keep_first, const OptTensor& sink, double softcap, const OptTensor& key_scale,
+                    const OptTensor& part_o, const OptTensor& part_ml, const OptTensor& counters, int64_t part_keys) {
+  const WindowAttnArgs a = attn_args(q, k_cache, v_cache, block_tables, row_seq, positions, window, scale, gate, out, tiles, cu_q, bias,
+                                     keep_first, sink, softcap, key_scale, part_o, part_ml, counters, part_keys);
+  return launch_window_attn(a, q.scalar_type() == at::kFloat, (int)impl, cur_stream(q));
+}
+
+DecayScanArgs scan_args(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dz, const Tensor& dbias,
                 const OptTensor& rate, double tau, const OptTensor& skip, double q_scale, int64_t H, int64_t N, int64_t P,
                 int64_t hpg, Tensor& state, const OptTensor& cu_q, const Tensor& prev_row, const Tensor& save_slot,
-                int64_t runs, Tensor& out, const OptTensor& mout, const OptTensor& tiles, const OptTensor& ws) {
+                int64_t runs, const OptTensor& out, const OptTensor& low, const OptTensor& mout, const OptTensor& tiles,
+                        const OptTensor& ws) {
   const int f32 = act(v, "v", false);
-  dtype(out, at::kFloat, "out");
+  if (out.has_value()) dtype(*out, at::kFloat, "out");
   dtype(dbias, at::kFloat, "dbias");
   dtype(prev_row, at::kInt, "prev_row");
   dtype(save_slot, at::kInt, "save_slot");
@@ -281,8 +311,14 @@ void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v,
   a.ldq = view2(q, f32, T, groups * N, "q");
   a.ldk = view2(k, f32, T, groups * N, "k");
   a.ldv = view2(v, f32, T, H * P, "v");
-  a.ldd = view2(dz, mode == 2 ? 1 : f32, T, mode == 0 ? H * N : (mode == 1 ? H : 2 * H), "dz");
-  TORCH_CHECK(dbias.numel() == (mode == 0 ? H * N : (mode == 1 ? H : 2 * H)) && out.numel() == T * H * PS &&
+  if (low.has_value()) {
+    TORCH_CHECK(mode == 0 && !f32 && dz.dim() == 2 && dz.size(0) == H * N, "decay_scan: a low-rank dz is its factor [H N, rank]");
+    dtype(dz, at::kBFloat16, "dz");
+    view2(*low, f32, T, dz.size(1), "low");
+  } else {
+    a.ldd = view2(dz, mode == 2 ? 1 : f32, T, mode == 0 ? H * N : (mode == 1 ? H : 2 * H), "dz");
+  }
+  TORCH_CHECK(dbias.numel() == (mode == 0 ? H * N : (mode == 1 ? H : 2 * H)) && (!out.has_value() || out->numel() == T * H * PS) &&
                   prev_row.numel() >= T && save_slot.numel() >= T, "decay_scan: shapes");
   if (mode == 2) {
     TORCH_CHECK(mout.has_value() && !skip.has_value(), "decay_scan: the log-gate mode writes its maxima and has no skip");
@@ -321,7 +357,7 @@ void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v,
   a.prev_row = ptr<int>(prev_row);
   a.save_slot = ptr<int>(save_slot);
   a.runs = (int)runs, a.T = (int)T;
-  a.out = ptr<float>(out);
+  a.out = optptr<float>(out);
   if (tiles.has_value() && ws.has_value()) {
     dtype(*tiles, at::kInt, "tiles");
     dtype(*ws, at::kFloat, "ws");
@@ -330,7 +366,66 @@ void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v,
     a.tiles = ptr<int>(*tiles), a.ntiles = (int)tiles->size(0);
     a.ws = ptr<float>(*ws);
   }
-  launch_decay_scan(a, f32, cur_stream(v));
+  return a;
+}
+
+void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dz, const Tensor& dbias,
+                const OptTensor& rate, double tau, const OptTensor& skip, double q_scale, int64_t H, int64_t N, int64_t P,
+                int64_t hpg, Tensor& state, const OptTensor& cu_q, const Tensor& prev_row, const Tensor& save_slot,
+                int64_t runs, Tensor& out, const OptTensor& mout, const OptTensor& tiles, const OptTensor& ws) {
+  const DecayScanArgs a = scan_args(mode, q, k, v, dz, dbias, rate, tau, skip, q_scale, H, N, P, hpg, state, cu_q, prev_row, save_slot,
+                                    runs, out, std::nullopt, mout, tiles, ws);
+  launch_decay_scan(a, v.scalar_type() == at::kFloat, cur_stream(v));
+}
+
+// one token a run, bf16: the scan and the head's norm, weight and gate
+DecayTokenArgs token_args(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dz, const OptTensor& low,
+                          const Tensor& dbias, const OptTensor& rate, double tau, const OptTensor& skip, double q_scale, int64_t H,
+                          int64_t N, int64_t P, int64_t hpg, Tensor& state, const Tensor& prev_row, const Tensor& save_slot,
+                          const Tensor& gate, const Tensor& w, double eps, bool sigmoid, Tensor& out, const OptTensor& ss) {
+  TORCH_CHECK(mode == 0 || mode == 1, "decay_token: mode");
+  DecayTokenArgs d{};
+  const int64_t T = v.size(0);
+  same_act(v, 0, "v", false);
+  d.s = scan_args(mode, q, k, v, dz, dbias, rate, tau, skip, q_scale, H, N, P, hpg, state, std::nullopt, prev_row, save_slot, T,
+                  std::nullopt, low, std::nullopt, std::nullopt, std::nullopt);
+  if (low.has_value()) d.low = low->data_ptr(), d.ldl = T > 1 ? low->stride(0) : dz.size(1), d.rank = (int)dz.size(1);
+  d.ldg = view2(gate, 0, T, H * P, "gate");
+  d.gate = gate.data_ptr();
+  dtype(w, at::kFloat, "w");
+  same_act(out, 0, "out");
+  TORCH_CHECK(w.numel() > 0 && w.numel() <= H * P && (H * P) % w.numel() == 0 && out.numel() == T * H * P, "decay_token: shapes");
+  d.w = ptr<float>(w), d.wlen = (int)w.numel(), d.eps = (float)eps, d.sigmoid = sigmoid;
+  d.out = out.data_ptr();
+  if (ss.has_value()) {
+    dtype(*ss, at::kFloat, "ss");
+    TORCH_CHECK(ss->numel() == T * H, "decay_token: ss [T, H]");
+    d.ss = ptr<float>(*ss);
+  }
+  return d;
+}
+
+bool decay_token(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dz, const OptTensor& low,
+                 const Tensor& dbias, const OptTensor& rate, double tau, const OptTensor& skip, double q_scale, int64_t H, int64_t N,
+                 int64_t P, int64_t hpg, Tensor& state, const Tensor& prev_row, const Tensor& save_slot, const Tensor& gate,
+                 const Tensor& w, double eps, bool sigmoid, Tensor& out, const OptTensor& ss) {
+  return launch_decay_token(token_args(mode, q, k, v, dz, low, dbias, rate, tau, skip, q_scale, H, N, P, hpg, state, prev_row, save_slot,
+                                       gate, w, eps, sigmoid, out, ss),
+                            cur_stream(v));
+}
+
+bool window_attn_decay(const Tensor& q, const Tensor& k_cache, const Tensor& v_cache, const Tensor& block_tables, const Tensor& row_seq,
+                       const Tensor& positions, int64_t window, double scale, const OptTensor& gate, Tensor& out, Tensor& part_o,
+                       Tensor& part_ml, Tensor& counters, int64_t part_keys, const Tensor& dq, const Tensor& dk, const Tensor& dv,
+                       const Tensor& dz, const OptTensor& low, const Tensor& dbias, double tau, double q_scale, int64_t H, int64_t N,
+                       int64_t P, Tensor& state, const Tensor& prev_row, const Tensor& save_slot, const Tensor& ngate, const Tensor& w,
+                       double eps, Tensor& gy) {
+  same_act(q, 0, "q");
+  const WindowAttnArgs a = attn_args(q, k_cache, v_cache, block_tables, row_seq, positions, window, scale, gate, out, std::nullopt,
+                                     std::nullopt, std::nullopt, 0, std::nullopt, 0., std::nullopt, part_o, part_ml, counters, part_keys);
+  const DecayTokenArgs d = token_args(0, dq, dk, dv, dz, low, dbias, std::nullopt, tau, std::nullopt, q_scale, H, N, P, 1, state, prev_row,
+                                      save_slot, ngate, w, eps, false, gy, std::nullopt);
+  return launch_split_attn_decay(a, d, cur_stream(q));
 }
 
 void gated_group_norm(const Tensor& y, const Tensor& gate, const Tensor& w, double eps, int64_t group, bool gate_first,
@@ -413,17 +508,20 @@ void conv_state_update(const Tensor& xin, Tensor& state, const OptTensor& cu_q, 
   launch_conv_state_update(a, f32, cur_stream(xin));
 }
 
-// y = f(x) . W^T for 1 to 16 rows; x and out may be column ranges; relu2: squared ReLU of x first; glu: W's rows are
-// [gate | up] and out = silu(gate) * up
-void row_linear(const Tensor& x, const Tensor& w, Tensor& out, bool relu2, bool glu) {
+// the operands of a few-row product, checked; glu: w's rows are [gate | up]
+struct RowOperands {
+  const void *x, *w;
+  void* out;
+  int64_t ldx, ldo;
+  int M, N, K;
+};
+RowOperands row_operands(const Tensor& x, const Tensor& w, Tensor& out, bool f32, bool glu) {
   gpu(x, "x", false);
   gpu(out, "out", false);
   dtype(w, at::kBFloat16, "w");
   TORCH_CHECK(x.scalar_type() == at::kBFloat16 && x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "row_linear: x bf16, 2-d operands");
   const int64_t M = x.size(0), K = x.size(1), N = out.size(1);
-  const bool f32 = out.scalar_type() == at::kFloat;
-  TORCH_CHECK(f32 || out.scalar_type() == at::kBFloat16, "row_linear: out bf16 or fp32");
-  TORCH_CHECK(!(f32 && (relu2 || glu)) && !(relu2 && glu), "row_linear: one of fp32 output, relu2, glu");
+  TORCH_CHECK(out.scalar_type() == (f32 ? at::kFloat : at::kBFloat16), "row_linear: out bf16 or fp32");
   TORCH_CHECK(M >= 1 && M <= 16 && out.size(0) == M, "row_linear: 1 to 16 rows");
   TORCH_CHECK(w.size(1) == K && w.size(0) == (glu ? 2 * N : N), "row_linear: w does not fit x and out");
   TORCH_CHECK(K >= 8 && K % 8 == 0 && K <= (1 << 22) && N >= 4 && N % 4 == 0 && N <= (1 << 30), "row_linear: K in 8s, N in 4s");
@@ -433,10 +531,59 @@ void row_linear(const Tensor& x, const Tensor& w, Tensor& out, bool relu2, bool 
   TORCH_CHECK((uintptr_t)x.data_ptr() % 16 == 0 && (uintptr_t)w.data_ptr() % 16 == 0 &&
                   (uintptr_t)out.data_ptr() % (f32 ? 16 : 8) == 0,
               "row_linear: alignment");
+  return {x.data_ptr(), w.data_ptr(), out.data_ptr(), ldx, ldo, (int)M, (int)N, (int)K};
+}
+
+// y = f(x) . W^T for 1 to 16 rows; x and out may be column ranges; relu2: squared ReLU of x first; glu: W's rows are
+// [gate | up] and out = silu(gate) * up
+void row_linear(const Tensor& x, const Tensor& w, Tensor& out, bool relu2, bool glu) {
+  const bool f32 = out.scalar_type() == at::kFloat;
+  TORCH_CHECK(!(f32 && (relu2 || glu)) && !(relu2 && glu), "row_linear: one of fp32 output, relu2, glu");
+  const RowOperands o = row_operands(x, w, out, f32, glu);
   const at::OptionalDeviceGuard g(x.device());
-  TORCH_CHECK(launch_row_linear(x.data_ptr(), ldx, w.data_ptr(), out.data_ptr(), ldo, (int)M, (int)N, (int)K, f32, relu2, glu,
-                                cur_stream(x)),
-              "row_linear: K = ", K, " is neither at most 256 nor a multiple of 256");
+  TORCH_CHECK(launch_row_linear(o.x, o.ldx, o.w, o.out, o.ldo, o.M, o.N, o.K, f32, relu2, glu, cur_stream(x)), "row_linear: K = ", o.K,
+              " is neither at most 256 nor a multiple of 256");
+}
+
+// two products of the same sizes; false: not one of its sizes
+bool row_linear_two(const Tensor& x0, const Tensor& w0, Tensor& out0, const Tensor& x1, const Tensor& w1, Tensor& out1) {
+  const RowOperands a = row_operands(x0, w0, out0, false, false), b = row_operands(x1, w1, out1, false, false);
+  if (a.M != b.M || a.N != b.N || a.K != b.K) return false;
+  const at::OptionalDeviceGuard g(x0.device());
+  const void *x[2] = {a.x, b.x}, *w[2] = {a.w, b.w};
+  void* out[2] = {a.out, b.out};
+  const long long ldx[2] = {a.ldx, b.ldx}, ldo[2] = {a.ldo, b.ldo};
+  return launch_row_linear_two(x, ldx, w, out, ldo, a.M, a.N, a.K, cur_stream(x0));
+}
+
+bool beside(const Tensor& x, const Tensor& w, Tensor& out, const RowRide& r) {
+  const RowOperands o = row_operands(x, w, out, false, false);
+  const at::OptionalDeviceGuard g(x.device());
+  return launch_row_linear_beside(o.x, o.ldx, o.w, o.out, o.ldo, o.M, o.N, o.K, r, cur_stream(x));
+}
+
+// relu(x)^2 . W^T and qkv_rope_cache in one launch; false: not one of its sizes
+bool row_linear_rope(const Tensor& x, const Tensor& w, Tensor& out, const Tensor& z, const OptTensor& bias, int64_t H, int64_t G,
+                     int64_t dk, int64_t dv, const Tensor& positions, const Tensor& slots, const OptTensor& rope, Tensor& q_out,
+                     Tensor& k_cache, Tensor& v_cache) {
+  same_act(z, 0, "z", false);
+  TORCH_CHECK(z.dim() == 2 && z.size(0) <= 65535, "row_linear_rope: z [T, n]");
+  RowRide r{};
+  r.rope = rope_args(z, bias, H, G, dk, dv, positions, slots, rope, q_out, k_cache, v_cache, 0);
+  r.rows = (int)z.size(0);
+  return beside(x, w, out, r);
+}
+
+// relu(x)^2 . W^T and causal_conv_silu (every row a run of its own) in one launch; false: not one of its sizes
+bool row_linear_conv(const Tensor& x, const Tensor& w, Tensor& out, const Tensor& xin, const Tensor& cw, const Tensor& cb, Tensor& state,
+                     const Tensor& prev_row, const Tensor& save_slot, Tensor& cout) {
+  same_act(cout, 0, "cout");
+  RowRide r{};
+  r.conv = conv_args(xin, cw, cb, state, std::nullopt, std::nullopt, prev_row, save_slot, xin.size(0), 0);
+  TORCH_CHECK(cout.numel() == (int64_t)r.conv.T * r.conv.C && r.conv.T <= 65535, "row_linear_conv: out shape");
+  r.conv.out = cout.data_ptr();
+  r.rows = r.conv.T;
+  return beside(x, w, out, r);
 }
 
 // y = x . W^T of 17 to 256 rows in bf16; x and out may be column ranges; glu as above; false: the sizes have no kernel
@@ -1216,12 +1363,13 @@ int64_t delta_rule(bool channel, const Tensor& q, const Tensor& k, const Tensor&
 }  // namespace
 
 TORCH_LIBRARY(symmetry_amd_hybrid, m) {
-  m.def("embed_norm(Tensor ids, Tensor? src, Tensor? prev, Tensor table, Tensor w, float eps, float offset, Tensor(a!) x) -> ()",
+  m.def("embed_norm(Tensor ids, Tensor? src, Tensor? prev, Tensor table, Tensor w, float eps, float offset, Tensor(a!) x, "
+        "Tensor? w2=None, Tensor(b!)? out=None) -> ()",
         &embed_norm);
   m.def("rms_norm_rows(Tensor x, Tensor? rows, Tensor w, float eps, float offset, Tensor(a!) out) -> ()", &rms_norm_rows);
   m.def(
       "residual_mix_norm(Tensor(a!) x, Tensor a, float sa, Tensor? bias_a, Tensor? b, float sb, Tensor? c, float sc, "
-      "Tensor? w, float eps, float offset, Tensor(b!)? out) -> ()",
+      "Tensor? w, float eps, float offset, Tensor(b!)? out, Tensor? ss=None, int ssn=1, float ss_eps=0.) -> ()",
       &residual_mix_norm);
   m.def(
       "qkv_rope_cache(Tensor z, Tensor? bias, int H, int G, int dk, int dv, Tensor positions, Tensor slots, Tensor? rope, "
@@ -1248,6 +1396,26 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
   m.def("conv_state_update(Tensor xin, Tensor(a!) state, Tensor? cu_q, Tensor prev_row, Tensor save_slot, int runs) -> ()",
         &conv_state_update);
   m.def("row_linear(Tensor x, Tensor w, Tensor(a!) out, bool relu2, bool glu) -> ()", &row_linear);
+  m.def("row_linear_two(Tensor x0, Tensor w0, Tensor(a!) out0, Tensor x1, Tensor w1, Tensor(b!) out1) -> bool", &row_linear_two);
+  m.def(
+      "row_linear_rope(Tensor x, Tensor w, Tensor(a!) out, Tensor z, Tensor? bias, int H, int G, int dk, int dv, Tensor positions, "
+      "Tensor slots, Tensor? rope, Tensor(b!) q_out, Tensor(c!) k_cache, Tensor(d!) v_cache) -> bool",
+      &row_linear_rope);
+  m.def(
+      "row_linear_conv(Tensor x, Tensor w, Tensor(a!) out, Tensor xin, Tensor cw, Tensor cb, Tensor(b!) state, Tensor prev_row, "
+      "Tensor save_slot, Tensor(c!) cout) -> bool",
+      &row_linear_conv);
+  m.def(
+      "decay_token(int mode, Tensor q, Tensor k, Tensor v, Tensor dz, Tensor? low, Tensor dbias, Tensor? rate, float tau, Tensor? skip, "
+      "float q_scale, int H, int N, int P, int hpg, Tensor(a!) state, Tensor prev_row, Tensor save_slot, Tensor gate, Tensor w, "
+      "float eps, bool sigmoid, Tensor(b!) out, Tensor(c!)? ss) -> bool",
+      &decay_token);
+  m.def(
+      "window_attn_decay(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor row_seq, Tensor positions, int window, "
+      "float scale, Tensor? gate, Tensor(a!) out, Tensor(b!) part_o, Tensor(c!) part_ml, Tensor(d!) counters, int part_keys, Tensor dq, "
+      "Tensor dk, Tensor dv, Tensor dz, Tensor? low, Tensor dbias, float tau, float q_scale, int H, int N, int P, Tensor(e!) state, "
+      "Tensor prev_row, Tensor save_slot, Tensor ngate, Tensor w, float eps, Tensor(f!) gy) -> bool",
+      &window_attn_decay);
   m.def("mid_linear_f32(Tensor x, Tensor w, Tensor(a!) out) -> bool", &mid_linear_f32);
   m.def("mid_linear(Tensor x, Tensor w, Tensor(a!) out, bool glu, Tensor(b!) slab, Tensor(c!) counters) -> bool", &mid_linear);
   m.def("relu_sq(Tensor a, Tensor(a!) out) -> ()", &relu_sq);

@@ -23,6 +23,7 @@
 // transcendental part of the decay evaluated once per (token, channel) there; the next batch's global loads are in
 // flight while the current batch is computed (two LDS buffers, one barrier per batch).
 #include "common.h"
+#include "decay_token.h"
 #include "hybrid_launchers.h"
 
 namespace {
@@ -260,7 +261,38 @@ void launch_mode(const DecayScanArgs& a, hipStream_t s) {
   else launch_one<T, MODE, 64, 8, 4>(a, s);   // N <= 256; half the batch keeps LDS under 64 KB
 }
 
+template <int MODE, int PQ, int NPAD>
+__global__ __launch_bounds__(DECAY_NT) void decay_token_kernel(DecayTokenArgs d) {
+  __shared__ __attribute__((aligned(16))) float lds[decay_token_lds(4 * PQ) / 4];
+  decay_token_block<MODE, PQ, NPAD>(d, blockIdx.x, blockIdx.y, lds);
+}
+
+template <int MODE, int NPAD>
+void launch_token(const DecayTokenArgs& d, hipStream_t s) {
+  const dim3 grid(d.s.H, d.s.runs);
+  if (d.s.P == 64) decay_token_kernel<MODE, 16, NPAD><<<grid, DECAY_NT, 0, s>>>(d);
+  else if (d.s.P == 128) decay_token_kernel<MODE, 32, NPAD><<<grid, DECAY_NT, 0, s>>>(d);
+  else decay_token_kernel<MODE, 64, NPAD><<<grid, DECAY_NT, 0, s>>>(d);
+}
+
 }  // namespace
+
+bool decay_token_takes(const DecayTokenArgs& d) {
+  const DecayScanArgs& a = d.s;
+  const auto al = [](const void* p, int to) { return reinterpret_cast<uintptr_t>(p) % to == 0; };
+  if (a.mode > 1 || a.cu_q || a.T != a.runs || a.runs < 1 || a.runs > 65535 || (a.N != 64 && a.N != 128) ||
+      (a.P != 64 && a.P != 128 && a.P != 256) || (d.low && (a.mode || d.rank < 8 || d.rank % 8 || d.rank > 256 || d.ldl % 8)))
+    return false;
+  return al(a.state, 16) && a.state_stride % 4 == 0 && al(a.v, 8) && a.ldv % 4 == 0 &&
+         (!d.low || (al(d.low, 16) && al(a.dz, 16)));
+}
+
+bool launch_decay_token(const DecayTokenArgs& d, hipStream_t s) {
+  if (!decay_token_takes(d)) return false;
+  if (d.s.mode == 0) d.s.N == 64 ? launch_token<0, 64>(d, s) : launch_token<0, 128>(d, s);
+  else d.s.N == 64 ? launch_token<1, 64>(d, s) : launch_token<1, 128>(d, s);
+  return true;
+}
 
 void launch_decay_scan(const DecayScanArgs& a, int f32, hipStream_t s) {
   if (a.runs <= 0 || a.T <= 0) return;

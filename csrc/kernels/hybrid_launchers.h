@@ -14,13 +14,14 @@
 #include <array>
 
 // ---- hybrid_rows.hip -----------------------------------------------------------------------------------
-// x[row] = table[token] / rms * (offset + w), token = src[row] >= 0 ? prev[src[row]] : ids[row]
+// x[row] = table[token] / rms * (offset + w), token = src[row] >= 0 ? prev[src[row]] : ids[row]; out (or null) = x / rms * (offset + w2)
 void launch_embed_norm(const int* ids, const int* src, const int* prev, const void* table, const float* w, float eps,
-                       float offset, float* x, int T, int d, int f32, hipStream_t s);
+                       float offset, float* x, const float* w2, void* out, int T, int d, int f32, hipStream_t s);
 // out[i] = x[rows ? rows[i] : i] / rms * (offset + w)
 void launch_rms_norm_rows(const float* x, const long long* rows, const float* w, float eps, float offset, void* out,
                           int n, int d, int f32, hipStream_t s);
-// x += sa * (a + bias_a) + sb * b + sc * c (bias_a, b, c optional; each of a, b, c bf16 or fp32: *_f32);
+// x += sa * (a + bias_a) + sb * b + sc * c (bias_a, b, c optional; each of a, b, c bf16 or fp32: *_f32); with ss, a is times
+// 1 / sqrt(sum of ss[row][0 .. nss) / ssn + ss_eps): the factor of a norm that a's product was formed without;
 // out (optional, activation dtype) = x_new / rms * (offset + w)
 struct ResidualMixArgs {
   float* x;
@@ -30,6 +31,7 @@ struct ResidualMixArgs {
   const float* w; float eps, offset;
   void* out;
   int T, d;
+  const float* ss; int nss; float ssn, ss_eps;
 };
 void launch_residual_mix_norm(const ResidualMixArgs& a, int f32, hipStream_t s);
 // z[t] = q (H dk) | k (G dk) | v (G dv), + bias (optional); q and k turn on their first 2 * pairs entries by
@@ -78,6 +80,19 @@ bool launch_mid_linear_f32(const void* x, long long ldx, const void* W, float* o
 // out = x . W^T (relu2: of relu(x)^2; glu: silu(gate) * up of W's [gate | up] rows); false: this K has no kernel
 bool launch_row_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int f32_out,
                        int relu2, int glu, hipStream_t s);
+// two products of the same sizes in one launch
+bool launch_row_linear_two(const void* const x[2], const long long ldx[2], const void* const W[2], void* const out[2], const long long ldo[2],
+                           int M, int N, int K, hipStream_t s);
+// out = relu(x)^2 . W^T, and beside it row work of other tensors: a convolution whose rows are runs of their own where conv.out is
+// set, else rope
+struct RowRide {
+  QkvRopeArgs rope;
+  ConvArgs conv;
+  int rows;
+  int per_row;   // workgroups a row (set by the launcher)
+};
+bool launch_row_linear_beside(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, const RowRide& r,
+                              hipStream_t s);
 // out = relu(a)^2
 void launch_relu_sq(const void* a, long long lda, void* out, int R, int F, int f32, hipStream_t s);
 // out = silu(gate) * up
@@ -254,6 +269,9 @@ int launch_window_attn(const WindowAttnArgs& a, int f32, int impl, hipStream_t s
 bool launch_prompt_attn(const WindowAttnArgs& a, hipStream_t s);
 // split_attention.hip: single rows with part_o set, causal, bf16, dk = dv in 32, 48, .. 128, H / G <= 16; false: not for these
 bool launch_split_attn(const WindowAttnArgs& a, hipStream_t s);
+struct DecayTokenArgs;
+// both at once, workgroups side by side; false: not one of its sizes, nothing is launched
+bool launch_split_attn_decay(const WindowAttnArgs& a, const DecayTokenArgs& d, hipStream_t s);
 
 // ---- decay_scan.hip ------------------------------------------------------------------------------------
 struct DecayScanArgs {
@@ -290,6 +308,22 @@ struct DecayScanArgs {
 bool decay_chunk_takes(const DecayScanArgs& a);
 void launch_decay_chunks(const DecayScanArgs& a, hipStream_t s);
 void launch_decay_scan(const DecayScanArgs& a, int f32, hipStream_t s);
+// One token a run in bf16 (cu_q null, T = runs; s.out is not written), with what follows the scan: out [T][H P] =
+// y / rms(head) * w * s(gate), s = silu or sigmoid; with ss: out = y s(gate) w as it is, and ss [T][H] the sums of (y s(gate))^2, for
+// a norm over all heads whose factor the next product applies
+struct DecayTokenArgs {
+  DecayScanArgs s;
+  const void* low; long long ldl; int rank;   // mode 0: not null: s.dz is [H N][rank] and the pre-activations are bf16(low . dz^T)
+  const void* gate; long long ldg;              // [T][H P]
+  const float* w; int wlen; float eps;          // w [wlen] repeats over the columns
+  int sigmoid;
+  void* out;
+  float* ss;
+};
+// false: not one of its sizes (N 64 or 128, P 64, 128 or 256, modes 0 and 1, rows in eights)
+bool launch_decay_token(const DecayTokenArgs& a, hipStream_t s);
+// the rules of launch_decay_token, without a launch
+bool decay_token_takes(const DecayTokenArgs& a);
 
 // ---- delta_rule.hip ------------------------------------------------------------------------------------
 // S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  out = S^T q  per head over every run, beta = sigmoid(bz[h]),

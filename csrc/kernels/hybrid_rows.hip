@@ -22,6 +22,7 @@
 // rotations, gates and sums are fp32; only the stored activations take the activation dtype T (bf16 or float).
 #include "common.h"
 #include "hybrid_launchers.h"
+#include "row_units.h"
 #include "wave_dot.h"
 
 namespace {
@@ -44,7 +45,8 @@ template <typename T, int BT>
 __global__ __launch_bounds__(BT) void embed_norm_kernel(const int* __restrict__ ids, const int* __restrict__ src,
                                                         const int* __restrict__ prev, const T* __restrict__ table,
                                                         const float* __restrict__ w, float eps, float offset,
-                                                        float* __restrict__ x, int d) {
+                                                        float* __restrict__ x, int d, const float* __restrict__ w2,
+                                                        T* __restrict__ out) {
   __shared__ float scratch[BT / 64];
   const int row = blockIdx.x;
   const int sr = src ? src[row] : -1;
@@ -56,7 +58,16 @@ __global__ __launch_bounds__(BT) void embed_norm_kernel(const int* __restrict__ 
     sq += v * v;
   }
   const float r = 1.f / sqrtf(block_sum<BT>(sq, scratch) / (float)d + eps);
-  for (int c = threadIdx.x; c < d; c += BT) x[(long long)row * d + c] = (float)t[c] * r * (offset + w[c]);
+  float s2 = 0.f;
+  for (int c = threadIdx.x; c < d; c += BT) {
+    const float v = (float)t[c] * r * (offset + w[c]);
+    x[(long long)row * d + c] = v;
+    s2 += v * v;
+  }
+  if (!out) return;
+  const float r2 = 1.f / sqrtf(block_sum<BT>(s2, scratch) / (float)d + eps);
+  for (int c = threadIdx.x; c < d; c += BT)
+    out[(long long)row * d + c] = (T)((float)t[c] * r * (offset + w[c]) * r2 * (offset + w2[c]));
 }
 
 // The same for prompt rows in bf16, d <= 8 BT in eights: a row is read once, in 16-byte pieces (column by column and twice: 40 ->
@@ -65,7 +76,8 @@ template <int BT>
 __global__ __launch_bounds__(BT) void embed_norm_vec_kernel(const int* __restrict__ ids, const int* __restrict__ src,
                                                             const int* __restrict__ prev, const bf16* __restrict__ table,
                                                             const float* __restrict__ w, float eps, float offset,
-                                                            float* __restrict__ x, int d) {
+                                                            float* __restrict__ x, int d, const float* __restrict__ w2,
+                                                            bf16* __restrict__ out) {
   __shared__ float scratch[BT / 64];
   const int row = blockIdx.x, c = 8 * threadIdx.x;
   const int sr = src ? src[row] : -1;
@@ -79,10 +91,22 @@ __global__ __launch_bounds__(BT) void embed_norm_vec_kernel(const int* __restric
     for (int i = 0; i < 8; ++i) sq += v[i] * v[i];
   }
   const float r = 1.f / sqrtf(block_sum<BT>(sq, scratch) / (float)d + eps);
-  if (!on) return;
+  sq = 0.f;
+  if (on) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = v[i] * r * (offset + wv[i]);
-  store8f(x + (long long)row * d + c, v);
+    for (int i = 0; i < 8; ++i) {
+      v[i] = v[i] * r * (offset + wv[i]);
+      sq += v[i] * v[i];
+    }
+    store8f(x + (long long)row * d + c, v);
+  }
+  if (!out) return;
+  const float r2 = 1.f / sqrtf(block_sum<BT>(sq, scratch) / (float)d + eps);
+  if (!on) return;
+  load8f(w2 + c, wv);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = v[i] * r2 * (offset + wv[i]);
+  store8(out + (long long)row * d + c, v);
 }
 
 template <typename T, int BT>
@@ -98,15 +122,25 @@ __global__ __launch_bounds__(BT) void rms_norm_rows_kernel(const float* __restri
   for (int c = threadIdx.x; c < d; c += BT) out[(long long)i * d + c] = (T)(xr[c] * r * (offset + w[c]));
 }
 
+// the factor of a row whose norm is applied here
+SYM_DEV float sum_factor(const ResidualMixArgs& a, int row) {
+  if (!a.ss) return 1.f;
+  float t = 0.f;
+  for (int i = threadIdx.x & 63; i < a.nss; i += 64) t += a.ss[(long long)row * a.nss + i];
+  return 1.f / sqrtf(wave_sum(t) / a.ssn + a.ss_eps);
+}
+
 template <typename T, int BT>
 __global__ __launch_bounds__(BT) void residual_mix_norm_kernel(ResidualMixArgs a) {
   __shared__ float scratch[BT / 64];
   const int row = blockIdx.x, d = a.d;
   float* xr = a.x + (long long)row * d;
   const long long o = (long long)row * d;
-  float sq = 0.f;
-  for (int c = threadIdx.x; c < d; c += BT) {
-    float s = ldf(a.a, a.a_f32, o + c);
+  constexpr int KEEP = 4;      // columns a thread holds from the sum to the norm (further ones it reads back)
+  float keep[KEEP], sq = 0.f;
+  const float f = sum_factor(a, row);
+  auto mix = [&](int c) {
+    float s = ldf(a.a, a.a_f32, o + c) * f;
     if (a.bias_a) s += a.bias_a[c];
     s *= a.sa;
     if (a.b) s += a.sb * ldf(a.b, a.b_f32, o + c);
@@ -114,12 +148,19 @@ __global__ __launch_bounds__(BT) void residual_mix_norm_kernel(ResidualMixArgs a
     const float xn = xr[c] + s;
     xr[c] = xn;
     sq += xn * xn;
-  }
+    return xn;
+  };
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i)
+    if ((int)threadIdx.x + BT * i < d) keep[i] = mix(threadIdx.x + BT * i);
+  for (int c = threadIdx.x + BT * KEEP; c < d; c += BT) mix(c);
   if (!a.out) return;
   const float r = 1.f / sqrtf(block_sum<BT>(sq, scratch) / (float)d + a.eps);
   T* out = reinterpret_cast<T*>(a.out) + o;
-  // (each thread re-reads the columns it wrote itself)
-  for (int c = threadIdx.x; c < d; c += BT) out[c] = (T)(xr[c] * r * (a.offset + a.w[c]));
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i)
+    if ((int)threadIdx.x + BT * i < d) out[threadIdx.x + BT * i] = (T)(keep[i] * r * (a.offset + a.w[threadIdx.x + BT * i]));
+  for (int c = threadIdx.x + BT * KEEP; c < d; c += BT) out[c] = (T)(xr[c] * r * (a.offset + a.w[c]));
 }
 
 // The same for widths of 8 to 8 NT in eights, bf16 out: a thread's eight columns stay in registers from the stream's load to the
@@ -134,10 +175,13 @@ __global__ __launch_bounds__(NT) void residual_mix_vec_kernel(ResidualMixArgs a)
   const long long o = (long long)blockIdx.x * a.d + c;
   const bool on = c < a.d;
   float x[8], sq = 0.f;
+  const float f = sum_factor(a, blockIdx.x);
   if (on) {
     float s[8], t[8];
     load8f(a.x + o, x);
     ld8f(a.a, a.a_f32, o, s);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s[i] *= f;
     if (a.bias_a) {
       load8f(a.bias_a + c, t);
 #pragma unroll
@@ -175,38 +219,7 @@ __global__ __launch_bounds__(NT) void residual_mix_vec_kernel(ResidualMixArgs a)
 
 template <typename T, int BT>
 __global__ __launch_bounds__(BT) void qkv_rope_cache_kernel(QkvRopeArgs a) {
-  const int row = blockIdx.x;
-  const T* z = reinterpret_cast<const T*>(a.z) + (long long)row * a.ldz;
-  const int nq = a.H * a.dk, nk = a.G * a.dk, nv = a.G * a.dv;
-  const int rot = 2 * a.pairs;
-  const float* cs = a.rope ? a.rope + (long long)a.positions[row] * rot : nullptr;   // [pairs][2]
-  const int slot = a.slots[row];
-  T* qo = reinterpret_cast<T*>(a.q_out) + (long long)row * nq;
-  T* kc = slot >= 0 ? reinterpret_cast<T*>(a.k_cache) + (long long)slot * nk : nullptr;
-  T* vc = slot >= 0 ? reinterpret_cast<T*>(a.v_cache) + (long long)slot * nv : nullptr;
-  for (int i = threadIdx.x; i < nq + nk; i += BT) {
-    const int e = i < nq ? i % a.dk : (i - nq) % a.dk;   // entry within its head
-    float v = (float)z[i] + (a.bias ? a.bias[i] : 0.f);
-    if (e < rot) {
-      if (a.half) {                                      // entry e with entry e +- pairs, table pair e mod pairs
-        const bool lo = e < a.pairs;
-        const int j = lo ? i + a.pairs : i - a.pairs, pi = lo ? e : e - a.pairs;
-        const float u = (float)z[j] + (a.bias ? a.bias[j] : 0.f);
-        const float c = cs[2 * pi], s = cs[2 * pi + 1];
-        v = lo ? v * c - u * s : v * c + u * s;
-      } else {
-        const int j = i - e + (e ^ 1);                   // the pair's other entry
-        const float u = (float)z[j] + (a.bias ? a.bias[j] : 0.f);
-        const float c = cs[e & ~1], s = cs[(e & ~1) + 1];
-        v = (e & 1) ? v * c + u * s : v * c - u * s;
-      }
-    }
-    if (i < nq) qo[i] = (T)v;
-    else if (kc) kc[i - nq] = (T)v;
-  }
-  if (vc)
-    for (int i = threadIdx.x; i < nv; i += BT)
-      vc[i] = (T)((float)z[nq + nk + i] + (a.bias ? a.bias[nq + nk + i] : 0.f));
+  qkv_rope_row<T>(a, blockIdx.x, threadIdx.x, BT);
 }
 
 // The same for prompt rows in bf16 whose pairs are neighbours: eight entries a thread, heads and rotary part in eights, so a piece is
@@ -325,14 +338,13 @@ __global__ __launch_bounds__(NT) void gated_group_norm_lanes_kernel(const float*
   store8(out + at, v);
 }
 
-constexpr int MAX_TAPS = 16;
-
 // grid (T, ceil(C / NT)): one thread per (row, channel).  SAVE: every row is a run of its own, whose newest inputs the same
 // thread moves on (one launch less of a decode step; each of the two takes 4.6 us at 8 rows of 4352)
 template <typename T, bool SAVE>
 __global__ __launch_bounds__(NT) void causal_conv_silu_kernel(ConvArgs a) {
   const int row = blockIdx.x, c = blockIdx.y * NT + threadIdx.x;
   if (c >= a.C) return;
+  if constexpr (SAVE) return conv_silu_save<T>(a, row, c);
   const int s0 = a.cu_q ? a.cu_q[a.row_seq[row]] : row;
   const int j = row - s0, taps = a.taps;
   const int pr = a.prev_row[s0];
@@ -340,25 +352,6 @@ __global__ __launch_bounds__(NT) void causal_conv_silu_kernel(ConvArgs a) {
   const T* x = reinterpret_cast<const T*>(a.xin);
   const T* w = reinterpret_cast<const T*>(a.w) + (long long)c * taps;
   float acc = a.b[c];
-  if constexpr (SAVE) {
-    const int sv = a.save_slot[row];
-    T old[MAX_TAPS];                     // old[m]: m + 1 positions back
-#pragma unroll
-    for (int m = 0; m < MAX_TAPS - 1; ++m)
-      if (m < taps - 1) old[m] = st ? st[(long long)(taps - 2 - m) * a.C + c] : (T)0.f;
-    const T now = x[(long long)row * a.ldx + c];
-    acc += (float)w[taps - 1] * (float)now;
-#pragma unroll
-    for (int m = 0; m < MAX_TAPS - 1; ++m)
-      if (m < taps - 1) acc += (float)w[taps - 2 - m] * (float)old[m];
-    reinterpret_cast<T*>(a.out)[(long long)row * a.C + c] = (T)(acc * sigmoidf(acc));
-    if (sv < 0) return;
-    T* dst = reinterpret_cast<T*>(a.state) + (long long)sv * a.state_stride + c;
-#pragma unroll
-    for (int m = 0; m < MAX_TAPS - 1; ++m)
-      if (m < taps - 1) dst[(long long)(taps - 2 - m) * a.C] = m == 0 ? now : old[m - 1];
-    return;
-  }
   for (int i = 0; i < taps; ++i) {       // i positions back
     float v = 0.f;
     if (i <= j) v = (float)x[(long long)(row - i) * a.ldx + c];
@@ -938,18 +931,19 @@ static inline bool wide_rows(int rows, int width) { return rows <= 512 && width 
   }
 
 void launch_embed_norm(const int* ids, const int* src, const int* prev, const void* table, const float* w, float eps,
-                       float offset, float* x, int T_, int d, int f32, hipStream_t s) {
+                       float offset, float* x, const float* w2, void* out, int T_, int d, int f32, hipStream_t s) {
   if (T_ <= 0) return;
-  const uintptr_t at = reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x);
+  const uintptr_t at = reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x) |
+                       reinterpret_cast<uintptr_t>(w2) | reinterpret_cast<uintptr_t>(out);
   if (!f32 && T_ > 512 && d % 8 == 0 && d <= 4096 && at % 16 == 0) {      // (fewer rows: the wider workgroups' latency counts)
-    if (d <= 2048) embed_norm_vec_kernel<256><<<T_, 256, 0, s>>>(ids, src, prev, (const bf16*)table, w, eps, offset, x, d);
-    else embed_norm_vec_kernel<512><<<T_, 512, 0, s>>>(ids, src, prev, (const bf16*)table, w, eps, offset, x, d);
+    if (d <= 2048) embed_norm_vec_kernel<256><<<T_, 256, 0, s>>>(ids, src, prev, (const bf16*)table, w, eps, offset, x, d, w2, (bf16*)out);
+    else embed_norm_vec_kernel<512><<<T_, 512, 0, s>>>(ids, src, prev, (const bf16*)table, w, eps, offset, x, d, w2, (bf16*)out);
     return;
   }
   if (wide_rows(T_, d)) {
-    DISPATCH_T(f32, (embed_norm_kernel<T, 1024><<<T_, 1024, 0, s>>>(ids, src, prev, (const T*)table, w, eps, offset, x, d));)
+    DISPATCH_T(f32, (embed_norm_kernel<T, 1024><<<T_, 1024, 0, s>>>(ids, src, prev, (const T*)table, w, eps, offset, x, d, w2, (T*)out));)
   } else {
-    DISPATCH_T(f32, (embed_norm_kernel<T, NT><<<T_, NT, 0, s>>>(ids, src, prev, (const T*)table, w, eps, offset, x, d));)
+    DISPATCH_T(f32, (embed_norm_kernel<T, NT><<<T_, NT, 0, s>>>(ids, src, prev, (const T*)table, w, eps, offset, x, d, w2, (T*)out));)
   }
 }
 

@@ -11,6 +11,7 @@
 // whose rows are [gate | up] (EPI_GLU: a workgroup computes both rows of its outputs).
 #include "common.h"
 #include "hybrid_launchers.h"
+#include "row_units.h"
 
 #include <type_traits>
 
@@ -25,6 +26,10 @@ struct Args {
   void* out;
   long long ldo;
   int M, N, K;  // EPI_GLU: N outputs, W has 2 N rows
+};
+// a launch's problems (blockIdx.y), of the same sizes
+struct Problems {
+  Args p[2];
 };
 
 SYM_DEV void relu_squared(Pack8& x) {
@@ -70,8 +75,28 @@ SYM_DEV void store_rows(const Args& a, int n0, int lane, f32x4 v, f32x4 u) {
 // M8: RH = 8 and at most 8 rows of x, which then are read like the weights.  One product of the two registers as they are
 // holds the first half's result in its upper left quarter and the second's in its lower right one (the others mix the halves
 // and are dropped): half the x traffic, which is twice the weights' otherwise, half the matrix products and no exchange.
-template <int RT, int RH, int NW, int EPI, bool XF, bool M8 = false>
-__global__ __launch_bounds__(NW * 64) void row_linear_kernel(Args a) {
+//
+// More: what a launch does beside its product.  RowRide: row work that the product does not read, by the workgroups behind its tiles (a
+// decode step's rotation or convolution beside the feed-forward's second product; launches of 4.7 us each, most of it latency).
+struct Nothing {};
+SYM_DEV void ride(const RowRide& r, int wg, int threads) {
+  const int row = wg / r.per_row, part = wg - row * r.per_row;
+  const int first = part * threads + (int)threadIdx.x;
+  if (r.conv.out) {
+    if (first < r.conv.C) conv_silu_save<bf16>(r.conv, row, first);
+  } else {
+    qkv_rope_row<bf16>(r.rope, row, first, threads * r.per_row);
+  }
+}
+
+template <int RT, int RH, int NW, int EPI, bool XF, bool M8 = false, typename More = Nothing>
+__global__ __launch_bounds__(NW * 64) void row_linear_kernel(Problems ps, More more) {
+  const Args& a = ps.p[blockIdx.y];
+  if constexpr (std::is_same<More, RowRide>::value) {
+    constexpr int out = EPI == EPI_GLU ? RH : RH * RT;
+    const int tiles = (a.N + out - 1) / out;
+    if ((int)blockIdx.x >= tiles) return ride(more, blockIdx.x - tiles, NW * 64);
+  }
   static_assert(!M8 || (RH == 8 && RT == 1 && EPI != EPI_GLU), "M8: one tile of 8 rows");
   constexpr int UK = RH == 16 ? 128 : 256;
   constexpr int XL = RH == 16 || M8 ? 1 : 2;      // x: 128-deep (M8: 256-deep) parts of a block
@@ -301,9 +326,17 @@ __global__ __launch_bounds__(64) void row_linear_small_kernel(Args a) {
   store_rows<16, EPI>(a, n0, lane, acc[0], acc[RT - 1]);
 }
 
+// what a launch does: its problem, and a second one of the same sizes or work beside it, or null
+struct Job {
+  const Args &a, *second;
+  const RowRide* beside;
+  bool plain() const { return !second && !beside; }
+};
+
 template <int NW, int KB, int EPI, bool XF>
-bool walk(const Args& a, hipStream_t s) {
-  if (a.K != 64 * NW * KB) return false;
+bool walk(const Job& j, hipStream_t s) {
+  const Args& a = j.a;
+  if (a.K != 64 * NW * KB || !j.plain()) return false;
   constexpr int OUT = EPI == EPI_GLU ? 8 : 16;
   const int tiles = (a.N + OUT - 1) / OUT;
   row_linear_walk_kernel<NW, KB, EPI, XF><<<tiles < 256 ? tiles : 256, NW * 64, 0, s>>>(a);
@@ -311,28 +344,42 @@ bool walk(const Args& a, hipStream_t s) {
 }
 
 template <int RT, int RH, int NW, int EPI, bool XF, bool M8>
-bool run(const Args& a, hipStream_t s) {
+bool run(const Job& j, hipStream_t s) {
+  const Args& a = j.a;
   if (a.K % ((RH == 16 ? 128 : 256) * NW)) return false;
   constexpr int rows = EPI == EPI_GLU ? RH : RH * RT;
-  row_linear_kernel<RT, RH, NW, EPI, XF, M8><<<(a.N + rows - 1) / rows, NW * 64, 0, s>>>(a);
-  return true;
+  const int tiles = (a.N + rows - 1) / rows;
+  const Problems ps{{a, j.second ? *j.second : a}};
+  if (!j.beside) {
+    row_linear_kernel<RT, RH, NW, EPI, XF, M8><<<dim3(tiles, j.second ? 2 : 1), NW * 64, 0, s>>>(ps, Nothing{});
+    return true;
+  }
+  if constexpr (EPI == EPI_BF16 && XF) {
+    if (j.beside) {
+      RowRide r = *j.beside;
+      r.per_row = r.conv.out ? (r.conv.C + NW * 64 - 1) / (NW * 64) : 2;
+      row_linear_kernel<RT, RH, NW, EPI, XF, M8, RowRide><<<tiles + r.per_row * r.rows, NW * 64, 0, s>>>(ps, r);
+      return true;
+    }
+  }
+  return false;
 }
 
 // With `waves` waves if these divide K's blocks, else with another number of them
 template <int RT, int RH, int EPI, bool XF, bool M8 = false>
-bool run_waves(const Args& a, int waves, hipStream_t s) {
+bool run_waves(const Job& j, int waves, hipStream_t s) {
   switch (waves) {
-    case 8: if (run<RT, RH, 8, EPI, XF, M8>(a, s)) return true; break;
-    case 6: if (run<RT, RH, 6, EPI, XF, M8>(a, s)) return true; break;
-    case 2: if (run<RT, RH, 2, EPI, XF, M8>(a, s)) return true; break;
+    case 8: if (run<RT, RH, 8, EPI, XF, M8>(j, s)) return true; break;
+    case 6: if (run<RT, RH, 6, EPI, XF, M8>(j, s)) return true; break;
+    case 2: if (run<RT, RH, 2, EPI, XF, M8>(j, s)) return true; break;
     default: break;
   }
-  if (run<RT, RH, 4, EPI, XF, M8>(a, s)) return true;
+  if (run<RT, RH, 4, EPI, XF, M8>(j, s)) return true;
   if constexpr (RH == 8)
-    if (run<RT, RH, 7, EPI, XF, M8>(a, s) || run<RT, RH, 6, EPI, XF, M8>(a, s) || run<RT, RH, 5, EPI, XF, M8>(a, s) ||
-        run<RT, RH, 3, EPI, XF, M8>(a, s))
+    if (run<RT, RH, 7, EPI, XF, M8>(j, s) || run<RT, RH, 6, EPI, XF, M8>(j, s) || run<RT, RH, 5, EPI, XF, M8>(j, s) ||
+        run<RT, RH, 3, EPI, XF, M8>(j, s))
       return true;
-  return run<RT, RH, 2, EPI, XF, M8>(a, s);      // (RH 16: takes every K, an even number of blocks)
+  return run<RT, RH, 2, EPI, XF, M8>(j, s);      // (RH 16: takes every K, an even number of blocks)
 }
 
 // Tile by the number of outputs (us; before / now: rows of neighbouring lanes / of lane quads, at 1, 8, 16 rows):
@@ -363,8 +410,10 @@ bool run_waves(const Args& a, int waves, hipStream_t s) {
 // 15.9 / 12.2 to 12.5; but 4360 x 2048 9.9 / 10.7, 6144 x 4096, three rounds of the walk, 19.3 / 20.7, 14336 x 4096 38.7 / 41.1), with
 // few outputs for more than 8 rows (512 x 4096 at 1, 16 rows 8.6, 10.7 / 9.4, 9.5).
 template <int EPI, bool XF>
-bool by_shape(const Args& a, hipStream_t s) {
+bool by_shape(const Job& j, hipStream_t s) {
+  const Args& a = j.a;
   if (a.K <= SMALL_K) {
+    if (!j.plain()) return false;
     row_linear_small_kernel<EPI, XF><<<(a.N + 15) / 16, 64, 0, s>>>(a);
     return true;
   }
@@ -376,7 +425,8 @@ bool by_shape(const Args& a, hipStream_t s) {
   } else {
     walks = ((a.K == 1536 || a.K == 3072) && a.N > 8192) || (a.K == 1536 && a.N > 4096 && a.M <= 4) || (a.K == 4096 && a.N > 16384);
   }
-  if (walks && (walk<8, 3, EPI, XF>(a, s) || walk<8, 6, EPI, XF>(a, s) || walk<8, 8, EPI, XF>(a, s))) return true;
+  if (walks && !j.plain()) return false;
+  if (walks && (walk<8, 3, EPI, XF>(j, s) || walk<8, 6, EPI, XF>(j, s) || walk<8, 8, EPI, XF>(j, s))) return true;
   auto waves = [&](int rt, int wgs) {
     const bool one = wgs <= 256;
     if (blocks <= (one ? 8 : 4)) return blocks;
@@ -384,25 +434,26 @@ bool by_shape(const Args& a, hipStream_t s) {
     return one && rt < 3 ? 4 : blocks <= 20 ? 2 : 4;
   };
   if constexpr (EPI == EPI_GLU) {
-    if (walks && walk<16, 2, EPI, XF>(a, s)) return true;
-    return run_waves<2, 16, EPI, XF>(a, waves(2, tiles), s);
+    if (walks && walk<16, 2, EPI, XF>(j, s)) return true;
+    return run_waves<2, 16, EPI, XF>(j, waves(2, tiles), s);
   } else {
     if (a.N <= 2048 && a.K % 256 == 0) {
       const int deep = a.K / 256;
       const int most = XF ? (deep % 8 ? 6 : 8) : a.M <= 8 && deep % 32 == 0 ? 8 : 4, shares = deep <= 8 ? deep : most;
-      if (a.M <= 8 ? run_waves<1, 8, EPI, XF, true>(a, shares, s) : run_waves<1, 8, EPI, XF>(a, shares, s))
+      if (a.M <= 8 ? run_waves<1, 8, EPI, XF, true>(j, shares, s) : run_waves<1, 8, EPI, XF>(j, shares, s))
         return true;
     }
     const int two = (tiles + 1) / 2, three = (tiles + 2) / 3;
-    if (tiles <= 256 || (blocks >= 64 && blocks % 4 == 0)) return run_waves<1, 16, EPI, XF>(a, waves(1, tiles), s);
+    if (tiles <= 256 || (blocks >= 64 && blocks % 4 == 0)) return run_waves<1, 16, EPI, XF>(j, waves(1, tiles), s);
     const int rounds2 = (two + 255) / 256, rounds3 = (three + 255) / 256;
     if (two > 1280 && (rounds3 > 6 || 8 * three < 7 * 256 * rounds3)) {
-      if (walk<16, 2, EPI, XF>(a, s)) return true;
-      if (a.K > 512 && (a.M <= 4 || (a.M <= 8 && 10 * two < 9 * 256 * rounds2))) return run_waves<1, 16, EPI, XF>(a, waves(1, tiles), s);
+      if (a.K == 2048 && !j.plain()) return false;
+      if (walk<16, 2, EPI, XF>(j, s)) return true;
+      if (a.K > 512 && (a.M <= 4 || (a.M <= 8 && 10 * two < 9 * 256 * rounds2))) return run_waves<1, 16, EPI, XF>(j, waves(1, tiles), s);
     } else if (two > 256 && 7 * rounds3 < 5 * rounds2) {
-      return run_waves<3, 16, EPI, XF>(a, waves(3, three), s);
+      return run_waves<3, 16, EPI, XF>(j, waves(3, three), s);
     }
-    return run_waves<2, 16, EPI, XF>(a, waves(2, two), s);
+    return run_waves<2, 16, EPI, XF>(j, waves(2, two), s);
   }
 }
 
@@ -411,6 +462,20 @@ bool by_shape(const Args& a, hipStream_t s) {
 bool launch_row_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int f32_out,
                        int relu2, int glu, hipStream_t s) {
   const Args a{(const bf16*)x, ldx, (const bf16*)W, out, ldo, M, N, K};
-  return glu ? by_shape<EPI_GLU, false>(a, s) : f32_out ? by_shape<EPI_F32, false>(a, s)
-         : relu2 ? by_shape<EPI_BF16, true>(a, s) : by_shape<EPI_BF16, false>(a, s);
+  const Job j{a, nullptr, nullptr};
+  return glu ? by_shape<EPI_GLU, false>(j, s) : f32_out ? by_shape<EPI_F32, false>(j, s)
+         : relu2 ? by_shape<EPI_BF16, true>(j, s) : by_shape<EPI_BF16, false>(j, s);
+}
+
+bool launch_row_linear_two(const void* const x[2], const long long ldx[2], const void* const W[2], void* const out[2], const long long ldo[2],
+                           int M, int N, int K, hipStream_t s) {
+  const Args a{(const bf16*)x[0], ldx[0], (const bf16*)W[0], out[0], ldo[0], M, N, K};
+  const Args b{(const bf16*)x[1], ldx[1], (const bf16*)W[1], out[1], ldo[1], M, N, K};
+  return by_shape<EPI_BF16, false>(Job{a, &b, nullptr}, s);
+}
+
+bool launch_row_linear_beside(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, const RowRide& r,
+                              hipStream_t s) {
+  const Args a{(const bf16*)x, ldx, (const bf16*)W, out, ldo, M, N, K};
+  return by_shape<EPI_BF16, true>(Job{a, nullptr, &r}, s);
 }

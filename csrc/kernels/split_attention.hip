@@ -14,6 +14,7 @@
 // an arrival counter per (row, group): the workgroup that arrives last sums them in order, writes the output and sets the
 // counter back to zero (nobody waits).  Softmax statistics and partial sums are fp32.
 #include "attn_tiles.h"
+#include "decay_token.h"
 #include "hybrid_launchers.h"
 
 namespace {
@@ -33,12 +34,10 @@ SYM_DEV float2 collect(const float* p) {
 }
 
 template <int D, bool KEYV, bool ONE, bool WIN>
-__global__ __launch_bounds__(64 * NW) void split_attn_kernel(WindowAttnArgs a) {
+SYM_DEV void split_attn_block(const WindowAttnArgs& a, int part, int g, int row, char* smem) {
   constexpr int CH = row_chunks(D), KD = (D + 31) / 32, VT = D / 16, ROWS = STEP * CH * 16;   // bytes of a step's rows
   constexpr int NL = STEP * CH / 64;                   // direct loads of a step's keys (and as many of its values)
   constexpr int STAGE = (KEYV ? 1 : 2) * ROWS + 256, LDO = D + 4;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int part = blockIdx.x, g = blockIdx.y, row = blockIdx.z;
   const int ctx = a.positions[row] + 1, first = WIN ? max(0, ctx - a.window) : 0, base = first & ~(STEP - 1);
   const int lo = base + part * a.part_keys;
   if (lo >= ctx) return;
@@ -259,12 +258,63 @@ __global__ __launch_bounds__(64 * NW) void split_attn_kernel(WindowAttnArgs a) {
 }
 
 template <int D, bool KEYV, bool ONE, bool WIN>
-void launch(const WindowAttnArgs& a, hipStream_t s) {
+__global__ __launch_bounds__(64 * NW) void split_attn_kernel(WindowAttnArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  split_attn_block<D, KEYV, ONE, WIN>(a, blockIdx.x, blockIdx.y, blockIdx.z, smem);
+}
+
+// With the recurrence of the same rows beside it (its workgroups first: all of a length, while short contexts' workgroups end at
+// once): neither reads what the other writes, and a decode step's rows leave room for both.
+template <int D, bool WIN, int PQ>
+__global__ __launch_bounds__(64 * NW) void split_attn_decay_kernel(WindowAttnArgs a, DecayTokenArgs d) {
+  static_assert(DECAY_NT == 64 * NW, "one workgroup size");
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int scans = d.s.H * d.s.runs;
+  int i = blockIdx.x;
+  if (i < scans) {
+    decay_token_block<0, PQ, 128>(d, i % d.s.H, i / d.s.H, reinterpret_cast<float*>(smem));
+    return;
+  }
+  i -= scans;
+  const int part = i % a.max_parts, rest = i / a.max_parts;
+  split_attn_block<D, false, true, WIN>(a, part, rest % a.G, rest / a.G, smem);
+}
+
+template <int D, bool KEYV>
+int lds_bytes(const WindowAttnArgs& a) {
   constexpr int stage = (KEYV ? 1 : 2) * STEP * row_chunks(D) * 16 + 256;
   const int rep = a.H / a.G;
   int lds = NW * stage;
   lds = max(lds, (int)(NW * rep * (D + 6) * sizeof(float)));
-  lds = max(lds, (int)(a.max_parts * rep * 2 * sizeof(float)));
+  return max(lds, (int)(a.max_parts * rep * 2 * sizeof(float)));
+}
+
+template <int D, bool WIN, int PQ>
+void launch_with(const WindowAttnArgs& a, const DecayTokenArgs& d, hipStream_t s) {
+  const int lds = max(lds_bytes<D, false>(a), decay_token_lds(4 * PQ));
+  static bool once = false;
+  if (!once) {
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&split_attn_decay_kernel<D, WIN, PQ>),
+                        hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
+    once = true;
+  }
+  const int wgs = d.s.H * d.s.runs + a.max_parts * a.G * a.T;
+  split_attn_decay_kernel<D, WIN, PQ><<<wgs, 64 * NW, lds, s>>>(a, d);
+}
+
+template <int D, bool WIN>
+bool launch_with_p(const WindowAttnArgs& a, const DecayTokenArgs& d, hipStream_t s) {
+  switch (d.s.P) {
+    case 64: launch_with<D, WIN, 16>(a, d, s); return true;
+    case 128: launch_with<D, WIN, 32>(a, d, s); return true;
+    case 256: launch_with<D, WIN, 64>(a, d, s); return true;
+    default: return false;
+  }
+}
+
+template <int D, bool KEYV, bool ONE, bool WIN>
+void launch(const WindowAttnArgs& a, hipStream_t s) {
+  const int lds = lds_bytes<D, KEYV>(a);
   static bool once = false;
   if (!once) {
     hipFuncSetAttribute(reinterpret_cast<const void*>(&split_attn_kernel<D, KEYV, ONE, WIN>),
@@ -296,12 +346,15 @@ void launch_d(const WindowAttnArgs& a, hipStream_t s) {
 
 }  // namespace
 
-bool launch_split_attn(const WindowAttnArgs& a, hipStream_t s) {
+static bool takes(const WindowAttnArgs& a) {
   const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (!a.part_o || !a.part_ml || !a.counters || a.part_keys < STEP || a.part_keys % STEP || a.max_parts < 1 ||
+  return !(!a.part_o || !a.part_ml || !a.counters || a.part_keys < STEP || a.part_keys % STEP || a.max_parts < 1 ||
       a.max_parts > MAX_PARTS || a.dk != a.dv || a.bias || (a.window < NO_WINDOW && (a.keep_first > 0 || a.k_cache == a.v_cache)) || a.H / a.G > MAX_REP || a.T > 65535 ||
-      a.G > 65535 || !al(a.q) || !al(a.k_cache) || !al(a.v_cache) || !al(a.out) || !al(a.part_o))
-    return false;
+      a.G > 65535 || !al(a.q) || !al(a.k_cache) || !al(a.v_cache) || !al(a.out) || !al(a.part_o));
+}
+
+bool launch_split_attn(const WindowAttnArgs& a, hipStream_t s) {
+  if (!takes(a)) return false;
   switch (a.dk) {
     case 32: launch_d<32>(a, s); return true;
     case 48: launch_d<48>(a, s); return true;
@@ -312,4 +365,19 @@ bool launch_split_attn(const WindowAttnArgs& a, hipStream_t s) {
     case 128: launch_d<128>(a, s); return true;
     default: return false;
   }
+}
+
+bool launch_split_attn_decay(const WindowAttnArgs& args, const DecayTokenArgs& d, hipStream_t s) {
+  WindowAttnArgs a = args;
+  a.bs_shift = -1;
+  for (int b = 5; b < 31; ++b)
+    if (a.BS == 1 << b) a.bs_shift = b;
+  const long long wgs = (long long)d.s.H * d.s.runs + (long long)a.max_parts * a.G * a.T;
+  if (a.bs_shift < 0 || a.k_cache == a.v_cache || a.tiles || a.T < 1 || d.s.mode != 0 || d.s.N != 128 || wgs > (1 << 30) || !takes(a) ||
+      !decay_token_takes(d))
+    return false;
+  const bool win = a.window < NO_WINDOW;
+  if (a.dk == 64) return win ? launch_with_p<64, true>(a, d, s) : launch_with_p<64, false>(a, d, s);
+  if (a.dk == 128) return win ? launch_with_p<128, true>(a, d, s) : launch_with_p<128, false>(a, d, s);
+  return false;
 }

@@ -247,31 +247,46 @@ class LemunexLM:
         ops.moe_mix(y2, dst, ids, wts, k, E, h, shared, sgate, out)
         return out
 
-    def _ff(self, P: dict, h: torch.Tensor, z: torch.Tensor):
+    def _ff(self, i: int, P: dict, h: torch.Tensor, z: torch.Tensor, b: ForwardBatch, cache: HybridCache):
+        """-> (the feed-forward's output or None, whether the mixer's row work in front of attention or scan went along).  The
+        feed-forward does not read the mixer, so in few rows of a decode step the second product's launch takes that work with it."""
         mlp = P["mlp"]
         if mlp is None:
-            return None
+            return None, False
         if isinstance(mlp, RoutedSpec):
-            return self._routed(P, h, z)
+            return self._routed(P, h, z), False
         up, out = self._cols(z, P, "up"), self._buf("ff.down", (h.shape[0], P["down"].shape[0]))
         if self.dtype == torch.bfloat16 and ops.few_rows(up, P["down"], out):  # the squared ReLU on the way in
-            ops.row_linear(up, P["down"], out, relu2=True)
-            return out
+            if b.kind != "decode":
+                along = False
+            elif P["kind"] == "parallel":
+                along = ops.row_linear_rope(up, P["down"], out, *self._rope_args(i, P, b, cache, z))
+            else:
+                along = ops.row_linear_conv(up, P["down"], out, self._cols(z, P, "xbc"), P["conv"], P["conv.b"], cache.conv[i],
+                                            b.prev_row, b.save_slot, self._buf("ssm.xc", (z.shape[0], P["mixer"].conv_channels)))
+            if not along:
+                ops.row_linear(up, P["down"], out, relu2=True)
+            return out, along
         act = self._buf("ff.act", (h.shape[0], mlp.ff))
         ops.relu_sq(up, act)
-        return self._linear("ff.down", act, P["down"])
+        return self._linear("ff.down", act, P["down"]), False
 
-    def _pair(self, i: int, P: dict, b: ForwardBatch, cache: HybridCache, z: torch.Tensor, runs: int):
+    def _rope_args(self, i: int, P: dict, b: ForwardBatch, cache: HybridCache, z: torch.Tensor) -> tuple:
+        a = P["mixer"].left
+        return (self._cols(z, P, "left"), P["left.b"], a.heads, a.kv_heads, a.dim, a.vdim, b.positions, b.slot_mapping, P["rope"],
+                self._buf("att.q", (z.shape[0], a.heads, a.dim)), cache.k[i], cache.v[i])
+
+    def _pair(self, i: int, P: dict, b: ForwardBatch, cache: HybridCache, z: torch.Tensor, runs: int, roped: bool):
         """Both halves of a parallel mixer -> (attention output, linear-attention output), each [T, d] before its scale."""
         m = P["mixer"]
         a, g = m.left, m.right
         T = z.shape[0]
         prefill = b.kind != "decode"
         # windowed attention
-        c0, n = P["cols"]["left"]
-        q = self._buf("att.q", (T, a.heads, a.dim))
-        ops.qkv_rope_cache(z[:, c0:c0 + n], P["left.b"], a.heads, a.kv_heads, a.dim, a.vdim, b.positions, b.slot_mapping,
-                           P["rope"], q, cache.k[i], cache.v[i])
+        rope = self._rope_args(i, P, b, cache, z)
+        if not roped:
+            ops.qkv_rope_cache(*rope)
+        q = rope[9]
         att = self._buf("att.o", (T, a.heads, a.vdim))
         split = None
         if not prefill and self.device.type != "cpu" and self.dtype == torch.bfloat16 and ops.window_ranges(T, a.heads, a.kv_heads):
@@ -279,9 +294,24 @@ class LemunexLM:
             split = (self._buf("att.part_o", (T, a.heads, parts, a.vdim), torch.float32),
                      self._buf("att.part_ml", (T, a.heads, parts, 2), torch.float32),
                      self.ws.get("att.counters", (T * a.kv_heads,), torch.int32, self.device, zeros=True), keys)
-        ops.window_attn(q, cache.k[i], cache.v[i], b.block_tables, b.row_seq, b.positions, a.window, a.scale,
-                        self._cols(z, P, "left.g"), att, b.tiles if prefill else None, b.cu_q if prefill else None, split=split)
-        left = self._linear("att.out", att.view(T, a.heads * a.vdim), P["left.o"])
+        att2, gy = att.view(T, a.heads * a.vdim), self._buf("rec.gy", (T, g.heads * g.vdim))
+        left, right = self._buf("att.out", (T, P["left.o"].shape[0])), self._buf("gla.out", (T, P["right.o"].shape[0]))
+        attn = (q, cache.k[i], cache.v[i], b.block_tables, b.row_seq, b.positions, a.window, a.scale, self._cols(z, P, "left.g"), att)
+        if not prefill and self.dtype == torch.bfloat16:
+            # a token's recurrence, its norm and gate in one launch, beside the attention where that goes in ranges
+            token = (self._cols(z, P, "right.q"), self._cols(z, P, "right.k"), self._cols(z, P, "right.v"), P["right.a2"],
+                     self._cols(z, P, "right.a1"), P["right.a2.b"], g.tau)
+            sizes = (g.dim ** -0.5, g.heads, g.dim, g.vdim)
+            tail = (cache.rec[i], b.prev_row, b.save_slot, self._cols(z, P, "right.g"), P["right.norm"], self.cfg.norm_eps, gy)
+            done = split is not None and ops.window_attn_decay(*attn, split, *token, *sizes, *tail)
+            if not done and ops.decay_token(ops.DECAY_CHANNEL_GATE, *token, None, *sizes, 1, *tail):
+                ops.window_attn(*attn, split=split)
+                done = True
+            if done:
+                ops.linear_two(att2, P["left.o"], left, gy, P["right.o"], right, self.ws)
+                return left, right
+        ops.window_attn(*attn, b.tiles if prefill else None, b.cu_q if prefill else None, split=split)
+        ops.linear(att2, P["left.o"], left, self.ws)
         # gated linear attention
         dz = self._linear("gla.dz", self._cols(z, P, "right.a1"), P["right.a2"])
         y = self._buf("rec.y", (T, g.heads * g.vdim), torch.float32)
@@ -291,29 +321,37 @@ class LemunexLM:
         ops.decay_scan(ops.DECAY_CHANNEL_GATE, self._cols(z, P, "right.q"), self._cols(z, P, "right.k"),
                        self._cols(z, P, "right.v"), dz, P["right.a2.b"], g.tau, None, g.dim ** -0.5, g.heads, g.dim,
                        g.vdim, 1, cache.rec[i], b.cu_q if prefill else None, b.prev_row, b.save_slot, runs, y, tiles=tiles, ws=ws)
-        gy = self._buf("rec.gy", (T, g.heads * g.vdim))
         ops.gated_group_norm(y, self._cols(z, P, "right.g"), P["right.norm"], self.cfg.norm_eps, g.vdim, False, gy)
-        right = self._linear("gla.out", gy, P["right.o"])
-        return left, right
+        return left, ops.linear(gy, P["right.o"], right, self.ws)
 
-    def _ssm(self, i: int, P: dict, b: ForwardBatch, cache: HybridCache, z: torch.Tensor, runs: int) -> torch.Tensor:
+    def _ssm(self, i: int, P: dict, b: ForwardBatch, cache: HybridCache, z: torch.Tensor, runs: int, convolved: bool):
+        """-> (the mixer's output [T, d], None or the sums of squares [T, heads] whose norm's factor it still lacks)."""
         m = P["mixer"]
         T = z.shape[0]
         cu = b.cu_q if b.kind != "decode" else None
         xin = self._cols(z, P, "xbc")
         xc = self._buf("ssm.xc", (T, m.conv_channels))
-        ops.causal_conv_silu(xin, P["conv"], P["conv.b"], cache.conv[i], cu, b.row_seq, b.prev_row, runs, xc,
-                             b.save_slot if cu is None else None)
+        if not convolved:
+            ops.causal_conv_silu(xin, P["conv"], P["conv.b"], cache.conv[i], cu, b.row_seq, b.prev_row, runs, xc,
+                                 b.save_slot if cu is None else None)
         if cu is not None:
             ops.conv_state_update(xin, cache.conv[i], cu, b.prev_row, b.save_slot, runs)
         inner, gn = m.inner, m.groups * m.state
+        if cu is None and self.dtype == torch.bfloat16 and m.norm_groups == 1:
+            # one token: scan, gate and the norm's weight in one launch; the norm's factor is one number a row, which the product keeps
+            # and the sum into the stream applies
+            gy, ss = self._buf("rec.gy", (T, inner)), self._buf("rec.ss", (T, m.heads), torch.float32)
+            if ops.decay_token(ops.DECAY_STEP_SIZE, xc[:, inner + gn:], xc[:, inner:inner + gn], xc[:, :inner], self._cols(z, P, "dt"),
+                               None, P["dt_bias"], P["A_log"], P["D"], 1.0, m.heads, m.state, m.vdim, m.heads // m.groups,
+                               cache.rec[i], b.prev_row, b.save_slot, self._cols(z, P, "z"), P["norm"], self.cfg.norm_eps, gy, ss):
+                return self._linear("ssm.out", gy, P["o"]), ss
         y = self._buf("rec.y", (T, inner), torch.float32)
         ops.decay_scan(ops.DECAY_STEP_SIZE, xc[:, inner + gn:], xc[:, inner:inner + gn], xc[:, :inner],
                        self._cols(z, P, "dt"), P["dt_bias"], P["A_log"], P["D"], 1.0, m.heads, m.state, m.vdim,
                        m.heads // m.groups, cache.rec[i], cu, b.prev_row, b.save_slot, runs, y)
         gy = self._buf("rec.gy", (T, inner))
         ops.gated_group_norm(y, self._cols(z, P, "z"), P["norm"], self.cfg.norm_eps, inner // m.norm_groups, True, gy)
-        return self._linear("ssm.out", gy, P["o"])
+        return self._linear("ssm.out", gy, P["o"]), None
 
     @torch.no_grad()
     def forward(self, b: ForwardBatch, cache: HybridCache) -> torch.Tensor:
@@ -326,27 +364,27 @@ class LemunexLM:
         h = self._buf("h", (T, d))
         src = b.src if b.src is not None and b.kind == "decode" else None
         ops.embed_norm(b.input_ids, self.embed, self.embed_norm, eps, NORM_OFFSET, x, src,
-                       self.last_ids if src is not None else None)
-        ops.rms_norm_rows(x, None, self.L[0]["norm1"], eps, NORM_OFFSET, h)
+                       self.last_ids if src is not None else None, self.L[0]["norm1"], h)
+        # (a decode step's rows are the head's, so the last sum's norm is the head's as well)
+        head = self._buf("logits.xn", (T, d)) if b.kind == "decode" and T == b.num_seqs and (b.sample or b.need_logits) else None
         for i, P in enumerate(self.L):
             z = self._linear("z", h, P["w_h"])
-            ff = self._ff(P, h, z)
-            nxt = self.L[i + 1]["norm1"] if i + 1 < len(self.L) else None
-            out = h if nxt is not None else None
+            ff, along = self._ff(i, P, h, z, b, cache)
+            nxt, out = (self.L[i + 1]["norm1"], h) if i + 1 < len(self.L) else (self.final_norm if head is not None else None, head)
             if P["kind"] == "parallel":
-                left, right = self._pair(i, P, b, cache, z, runs)
+                left, right = self._pair(i, P, b, cache, z, runs, along)
                 m = P["mixer"]
                 ops.residual_mix_norm(x, left, m.left_scale, P["left.o.b"], right, m.right_scale, ff, 1.0, nxt, eps,
                                       NORM_OFFSET, out)
             else:
-                mix = self._ssm(i, P, b, cache, z, runs)
-                ops.residual_mix_norm(x, mix, 1.0, None, ff, 1.0, None, 0.0, nxt, eps, NORM_OFFSET, out)
+                mix, ss = self._ssm(i, P, b, cache, z, runs, along)
+                ops.residual_mix_norm(x, mix, 1.0, None, ff, 1.0, None, 0.0, nxt, eps, NORM_OFFSET, out, ss, P["mixer"].inner, eps)
         n = b.num_seqs
         ids = self.last_ids[:n]
         self.last_logits = None
         if b.sample or b.need_logits:
             rows = None if b.kind == "decode" else b.last_idx
-            logits = self._logits("logits", x, rows, n)
+            logits = self._logits("logits", x, rows, n, head)
             if b.need_logits:
                 self.last_logits = logits
             if b.sample:
@@ -358,11 +396,12 @@ class LemunexLM:
             self.last_logits = self._logits("want_logits", x, b.logit_rows, int(b.logit_rows.numel()))
         return ids
 
-    def _logits(self, name: str, x: torch.Tensor, rows, n: int) -> torch.Tensor:
-        """fp32 logits [n, V] = n(x[rows], g_f) . W_head^T (fp32 output from the library GEMM)."""
+    def _logits(self, name: str, x: torch.Tensor, rows, n: int, xn=None) -> torch.Tensor:
+        """fp32 logits [n, V] = n(x[rows], g_f) . W_head^T (fp32 output from the library GEMM); ``xn``: the norm, where it is at hand."""
         cfg = self.cfg
-        xn = self._buf(name + ".xn", (n, cfg.hidden_size))
-        ops.rms_norm_rows(x, rows, self.final_norm, cfg.norm_eps, NORM_OFFSET, xn)
+        if xn is None:
+            xn = self._buf(name + ".xn", (n, cfg.hidden_size))
+            ops.rms_norm_rows(x, rows, self.final_norm, cfg.norm_eps, NORM_OFFSET, xn)
         logits = self._buf(name, (n, cfg.vocab_size), torch.float32)
         ops.linear_f32(xn, self.head, logits)
         return logits

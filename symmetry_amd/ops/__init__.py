@@ -692,6 +692,28 @@ def row_linear(x, w, out, relu2: bool = False, glu: bool = False) -> None:
     return reference.row_linear(x, w, out, relu2, glu)
 
 
+def row_linear_rope(x, w, out, z, bias, H, G, dk, dv, positions, slots, rope, q_out, k_cache, v_cache) -> bool:
+    """row_linear(x, w, out, relu2=True) and qkv_rope_cache of other tensors in one launch (few_rows operands); False where there is no
+    such launch: nothing has been done."""
+    return _gpu(x) and _hyb().row_linear_rope(x, w, out, z, bias, int(H), int(G), int(dk), int(dv), positions, slots, rope, q_out,
+                                              k_cache, v_cache)
+
+
+def row_linear_conv(x, w, out, xin, cw, cb, state, prev_row, save_slot, cout) -> bool:
+    """row_linear(x, w, out, relu2=True) and causal_conv_silu of other tensors, every row a run of its own, in one launch (few_rows
+    operands); False where there is no such launch: nothing has been done."""
+    return _gpu(x) and _hyb().row_linear_conv(x, w, out, xin, cw, cb, state, prev_row, save_slot, cout)
+
+
+def linear_two(x0, w0, out0, x1, w1, out1, ws=None) -> None:
+    """``linear`` twice, in one launch where few-row operands have the same sizes (two of 2048 x 2048 at 8 rows: 9.4 us apart)."""
+    if few_rows(x0, w0, out0) and few_rows(x1, w1, out1) and out0.dtype == out1.dtype == torch.bfloat16:
+        if out0.shape[1] == w0.shape[0] and out1.shape[1] == w1.shape[0] and _hyb().row_linear_two(x0, w0, out0, x1, w1, out1):
+            return
+    linear(x0, w0, out0, ws)
+    linear(x1, w1, out1, ws)
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, ws=None) -> torch.Tensor:
     """``x @ w.T``: the few-row kernel up to 16 rows (2048 x 2048 at 8 rows 4.8 us, the library 8.5; 17688 x 2048 21.9 / 49.6),
     with a workspace ``ws`` (a model's: ``get(name, shape, dtype, device, zeros)``) the medium-row kernel up to 256, else the library GEMM (hipBLASLt through torch, the library heuristic; a
@@ -943,11 +965,14 @@ def _hyb():
     return _native.hybrid_ops()
 
 
-def embed_norm(ids, table, w, eps, offset, x, src=None, prev=None):
-    """x (fp32) = table[token] / rms * (offset + w); rows with src >= 0 take the token prev[src]."""
+def embed_norm(ids, table, w, eps, offset, x, src=None, prev=None, w2=None, out=None):
+    """x (fp32) = table[token] / rms * (offset + w); rows with src >= 0 take the token prev[src].  With ``out``: rms_norm_rows of x
+    with w2 in the same pass."""
     if _gpu(x):
-        return _hyb().embed_norm(ids, src, prev, table, w, float(eps), float(offset), x)
-    return reference.embed_norm(reference.resolve_ids(ids, src, prev), table, w, eps, offset, x)
+        return _hyb().embed_norm(ids, src, prev, table, w, float(eps), float(offset), x, w2, out)
+    reference.embed_norm(reference.resolve_ids(ids, src, prev), table, w, eps, offset, x)
+    if out is not None:
+        reference.rms_norm_rows(x, None, w2, eps, offset, out)
 
 
 def rms_norm_rows(x, rows, w, eps, offset, out):
@@ -957,12 +982,15 @@ def rms_norm_rows(x, rows, w, eps, offset, out):
     return reference.rms_norm_rows(x, rows, w, eps, offset, out)
 
 
-def residual_mix_norm(x, a, sa, bias_a, b, sb, c, sc, w=None, eps=0.0, offset=0.0, out=None):
+def residual_mix_norm(x, a, sa, bias_a, b, sb, c, sc, w=None, eps=0.0, offset=0.0, out=None, ss=None, ssn=1, ss_eps=0.0):
     """x += sa * (a + bias_a) + sb * b + sc * c in fp32 (bias_a, b, c optional); with ``out``: out = x / rms * (offset
-    + w), the next layer's normalised input, from the same pass."""
+    + w), the next layer's normalised input, from the same pass.  ``ss`` fp32 [T, n]: a's rows are first multiplied by
+    1 / sqrt(sum(ss) / ssn + ss_eps), the factor of a norm that a was formed without (``decay_token``)."""
     if _gpu(x):
         return _hyb().residual_mix_norm(x, a, float(sa), bias_a, b, float(sb), c, float(sc), w, float(eps),
-                                        float(offset), out)
+                                        float(offset), out, ss, int(ssn), float(ss_eps))
+    if ss is not None:
+        a = a.float().view_as(x) / torch.sqrt(ss.sum(1, keepdim=True) / ssn + ss_eps)
     return reference.residual_mix_norm(x, a, sa, bias_a, b, sb, c, sc, w, eps, offset, out)
 
 
@@ -1052,6 +1080,29 @@ def decay_scan(mode, q, k, v, dz, dbias, dparam, skip, q_scale, H, N, P, hpg, st
                                  int(runs), out, mout, tiles, ws)
     return reference.decay_scan(mode, q, k, v, dz, dbias, dparam, skip, q_scale, H, N, P, hpg, state, cu_q, prev_row,
                                 save_slot, runs, out, mout)
+
+
+def decay_token(mode, q, k, v, dz, low, dbias, dparam, skip, q_scale, H, N, P, hpg, state, prev_row, save_slot, gate, w, eps, out,
+                ss=None, sigmoid=False) -> bool:
+    """decay_scan of rows that are runs of their own (decode steps, bf16) and what follows it, in one launch: out bf16 [T, H P] =
+    gated_group_norm(., gate, w, eps, P, False).  ``ss`` fp32 [T, H]: out = y silu(gate) w as it is and ss its heads' sums of
+    (y silu(gate))^2, for a norm over all heads whose factor a later sum applies (``residual_mix_norm``).  ``low`` [T, rank] (channel
+    gate): dz [H N, rank] is the second factor of the pre-activations, which are rounded to bf16.  False: not one of its sizes,
+    nothing has been done."""
+    if not _gpu(out):
+        return False
+    dp = dparam if torch.is_tensor(dparam) else None
+    return _hyb().decay_token(int(mode), q, k, v, dz, low, dbias, dp, 0.0 if dp is not None else float(dparam), skip, float(q_scale),
+                              int(H), int(N), int(P), int(hpg), state, prev_row, save_slot, gate, w, float(eps), bool(sigmoid), out, ss)
+
+
+def window_attn_decay(q, k_cache, v_cache, block_tables, row_seq, positions, window, scale, gate, out, split, dq, dk, dv, dz, low, dbias,
+                      tau, q_scale, H, N, P, state, prev_row, save_slot, ngate, w, eps, gy) -> bool:
+    """window_attn (``split`` given) and decay_token (channel gate) of the same rows side by side in one launch; False: not one of its
+    sizes, nothing has been done."""
+    return _gpu(q) and _hyb().window_attn_decay(q, k_cache, v_cache, block_tables, row_seq, positions, int(window), float(scale), gate, out,
+                                                *split, dq, dk, dv, dz, low, dbias, float(tau), float(q_scale), int(H), int(N), int(P),
+                                                state, prev_row, save_slot, ngate, w, float(eps), gy)
 
 
 def decay_ws_cols(N: int) -> int:
