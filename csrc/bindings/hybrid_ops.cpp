@@ -1246,6 +1246,33 @@ void residual_layer_norm(Tensor& x, const OptTensor& base, const OptTensor& a, c
   launch_residual_layer_norm(r, f32, cur_stream(x));
 }
 
+// x = table[token] * scale and its layer norm
+void embed_layer_norm(const Tensor& ids, const OptTensor& src, const OptTensor& prev, const Tensor& table, double scale, Tensor& x,
+                      const Tensor& w, const Tensor& bias, double eps, Tensor& out) {
+  const int f32 = act(table, "table");
+  dtype(ids, at::kInt, "ids");
+  dtype(x, at::kFloat, "x");
+  dtype(w, at::kFloat, "w");
+  dtype(bias, at::kFloat, "bias");
+  same_act(out, f32, "out");
+  const int64_t T = ids.numel(), d = table.size(1);
+  TORCH_CHECK(table.dim() == 2 && x.numel() == T * d && out.numel() == T * d && w.numel() == d && bias.numel() == d,
+              "embed_layer_norm: shapes");
+  ResidualLnArgs r{};
+  if (src.has_value()) {
+    TORCH_CHECK(prev.has_value(), "embed_layer_norm: src without prev");
+    dtype(*src, at::kInt, "src");
+    dtype(*prev, at::kInt, "prev");
+    TORCH_CHECK(src->numel() >= T, "embed_layer_norm: src too short");
+    r.src = ptr<int>(*src), r.prev = ptr<int>(*prev);
+  }
+  r.ids = ptr<int>(ids), r.table = table.data_ptr(), r.scale = (float)scale;
+  r.x = ptr<float>(x), r.w = ptr<float>(w), r.bias = ptr<float>(bias), r.eps = (float)eps;
+  r.out = out.data_ptr();
+  r.n = (int)T, r.d = (int)d;
+  launch_residual_layer_norm(r, f32, cur_stream(x));
+}
+
 void conv_silu_qkv(const Tensor& z, const Tensor& w, Tensor& state, const OptTensor& cu_q, const OptTensor& row_seq,
                    const Tensor& prev_row, const OptTensor& save_slot, int64_t runs, int64_t G, int64_t N, int64_t H,
                    int64_t P, double q_scale, double unit_eps, Tensor& q_out, Tensor& k_out, Tensor& v_out, const OptTensor& gx,
@@ -1358,6 +1385,53 @@ int64_t delta_rule(bool channel, const Tensor& q, const Tensor& k, const Tensor&
   a.out = ptr<float>(out);
   a.T = (int)T, a.H = (int)H, a.G = (int)G, a.N = (int)N, a.P = (int)P, a.hpg = (int)(H / G), a.runs = (int)runs;
   return launch_delta_rule(a, channel ? 1 : 0, f32, (int)impl, cur_stream(out));
+}
+
+// one token of every row, bf16: convolution, recurrence, norm and gate; false: not one of its sizes
+bool delta_token(const Tensor& z, const Tensor& cw, Tensor& conv, const Tensor& prev_row, const Tensor& save_slot, int64_t H, int64_t N,
+                 int64_t P, double q_scale, double unit_eps, const Tensor& gx, const Tensor& gw, const OptTensor& a1, const OptTensor& a2,
+                 const Tensor& dt_bias, const Tensor& A_log, Tensor& state, const Tensor& gate, const OptTensor& g2, const Tensor& w,
+                 double eps, Tensor& out) {
+  const bool channel = a1.has_value();
+  TORCH_CHECK(z.dim() == 2 && cw.dim() == 2 && conv.dim() == 3 && state.dim() == 4 && gw.dim() == 2, "delta_token: ranks");
+  TORCH_CHECK(H > 0 && N > 0 && P > 0 && H <= 65535, "delta_token: sizes");
+  DeltaTokenArgs a{};
+  const int64_t T = z.size(0), C = 2 * H * N + H * P;
+  a.ldz = view2(z, 0, T, C, "z");
+  same_act(cw, 0, "cw");
+  same_act(conv, 0, "conv");
+  same_act(gw, 0, "gw");
+  same_act(out, 0, "out");
+  for (const Tensor* t : std::initializer_list<const Tensor*>{&dt_bias, &A_log, &state, &w}) dtype(*t, at::kFloat, "delta_token: fp32");
+  dtype(prev_row, at::kInt, "prev_row");
+  dtype(save_slot, at::kInt, "save_slot");
+  a.taps = (int)cw.size(1);
+  a.ldgx = view2(gx, 0, T, gw.size(1), "gx");
+  TORCH_CHECK(cw.size(0) == C && conv.size(1) == a.taps - 1 && conv.size(2) == C && gw.size(0) >= (channel ? H : 2 * H) &&
+                  dt_bias.numel() == (channel ? H * N : H) && A_log.numel() == H && state.size(1) == H && state.size(2) == N &&
+                  state.size(3) == P && prev_row.numel() >= T && save_slot.numel() >= T && w.numel() == P && out.numel() == T * H * P,
+              "delta_token: shapes");
+  if (channel) {
+    TORCH_CHECK(a2.has_value() && g2.has_value() && a2->dim() == 2 && g2->dim() == 2, "delta_token: a1 without a2 and g2");
+    same_act(*a2, 0, "a2");
+    same_act(*g2, 0, "g2");
+    a.rank = (int)a2->size(1), a.grank = (int)g2->size(1);
+    TORCH_CHECK(a2->size(0) == H * N && g2->size(0) == H * P, "delta_token: factor shapes");
+    a.lda1 = view2(*a1, 0, T, a.rank, "a1");
+    a.a1 = a1->data_ptr(), a.a2 = a2->data_ptr(), a.g2 = g2->data_ptr();
+  }
+  a.ldg = view2(gate, 0, T, channel ? a.grank : H * P, "gate");
+  a.z = z.data_ptr(), a.cw = cw.data_ptr(), a.conv = conv.data_ptr(), a.conv_stride = conv.stride(0);
+  a.q_scale = (float)q_scale, a.unit_eps = (float)unit_eps;
+  a.gx = gx.data_ptr(), a.gw = gw.data_ptr(), a.gd = (int)gw.size(1);
+  a.gate = gate.data_ptr();
+  a.dt_bias = ptr<float>(dt_bias), a.A_log = ptr<float>(A_log);
+  a.state = ptr<float>(state), a.state_stride = state.stride(0);
+  a.prev_row = ptr<int>(prev_row), a.save_slot = ptr<int>(save_slot);
+  a.w = ptr<float>(w), a.eps = (float)eps;
+  a.out = out.data_ptr();
+  a.T = (int)T, a.H = (int)H, a.N = (int)N, a.P = (int)P;
+  return launch_delta_token(a, cur_stream(z));
 }
 
 }  // namespace
@@ -1488,6 +1562,15 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
       &conv_qkv_cache);
   m.def("memory_norm_gate(Tensor y, Tensor m, Tensor gate, Tensor w, float eps, Tensor(a!) out) -> ()", &memory_norm_gate);
   m.def("clamped_glu(Tensor gu, float limit, float alpha, Tensor(a!) out) -> ()", &hyb_clamped_glu);
+  m.def(
+      "embed_layer_norm(Tensor ids, Tensor? src, Tensor? prev, Tensor table, float scale, Tensor(a!) x, Tensor w, Tensor bias, float eps, "
+      "Tensor(b!) out) -> ()",
+      &embed_layer_norm);
+  m.def(
+      "delta_token(Tensor z, Tensor cw, Tensor(a!) conv, Tensor prev_row, Tensor save_slot, int H, int N, int P, float q_scale, "
+      "float unit_eps, Tensor gx, Tensor gw, Tensor? a1, Tensor? a2, Tensor dt_bias, Tensor A_log, Tensor(b!) state, Tensor gate, "
+      "Tensor? g2, Tensor w, float eps, Tensor(c!) out) -> bool",
+      &delta_token);
   m.def(
       "residual_layer_norm(Tensor(a!) x, Tensor? base, Tensor? a, Tensor? b, Tensor? w, Tensor? bias, float eps, Tensor? rows, "
       "Tensor(b!)? out) -> ()",

@@ -350,6 +350,36 @@ struct DeltaRuleArgs {
 // impl 0: the chunked form where tiles and ws are given; 1: token by token.  Returns the form used.
 int launch_delta_rule(const DeltaRuleArgs& a, int channel, int f32, int impl, hipStream_t s);
 
+// ---- delta_token.hip -----------------------------------------------------------------------------------
+// One token of every row (each a run of its own) in bf16: z = q (H N) | k (H N) | v (H P) through the carried convolution, silu, unit
+// q and k as for ConvSiluArgs; the recurrence as for DeltaRuleArgs with bz = gx . gw[0 .. H)^T and dz = gx . gw[H .. 2 H)^T, or
+// (a1 given) a1 . a2^T per channel; out [T][H P] = y / rms(head) * w * silu(gate), or with a1 * sigmoid(bf16(gate . g2^T))
+struct DeltaTokenArgs {
+  const void* z; long long ldz;
+  const void* cw;                         // [2 H N + H P][taps]
+  void* conv; long long conv_stride;      // [slots][taps - 1][2 H N + H P]
+  float q_scale, unit_eps;
+  const void* gx; long long ldgx;         // [T][gd]
+  const void* gw;                         // [H or 2 H][gd]
+  int gd;
+  const void* a1; long long lda1;         // [T][rank] or null
+  const void* a2;                         // [H N][rank]
+  const void* gate; long long ldg;        // [T][H P], or with a1 [T][grank]
+  const void* g2;                         // [H P][grank]
+  int rank, grank;
+  const float* dt_bias;                   // [H], or with a1 [H N]
+  const float* A_log;
+  float* state; long long state_stride;   // [slots][H][N][P]
+  const int* prev_row;
+  const int* save_slot;
+  const float* w;                         // [P]
+  float eps;
+  void* out;
+  int T, H, N, P, taps;
+};
+// false: not one of its sizes (N 128, P 64, 128 or 256, four taps, ranks in 32s)
+bool launch_delta_token(const DeltaTokenArgs& a, hipStream_t s);
+
 // ---- stream_rows.hip -----------------------------------------------------------------------------------
 // x[row][s] (s < S) = table[token] + pair_table[(p mul_prev + token mul_cur) mod buckets]; p = the token of row
 // prev_row[row] (>= 0), tok_state[-(prev_row[row] + 2)] (<= -2) or none (-1: row `buckets` of pair_table); pair_table null:
@@ -420,6 +450,9 @@ struct ResidualLnArgs {
   const long long* rows;
   void* out;            // [n][d] activation dtype or null
   int n, d;             // rows of the launch
+  // or null: base is table[token] * scale (activation dtype), token as for launch_embed_norm
+  const void* table; float scale;
+  const int* ids; const int* src; const int* prev;
 };
 void launch_residual_layer_norm(const ResidualLnArgs& a, int f32, hipStream_t s);
 // z[t] = q (G N) | k (G N) | v (H P) through the causal per-channel convolution w [C][taps] (as for ConvQkvArgs), then

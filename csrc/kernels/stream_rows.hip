@@ -265,7 +265,8 @@ __global__ __launch_bounds__(BT) void residual_layer_norm_kernel(ResidualLnArgs 
   const long long o = (long long)row * d;
   float* x = a.x + xrow * d;
   const float* base = a.base ? a.base + xrow * d : x;
-  const bool upd = a.base || a.a || a.b;
+  const T* token = a.table ? reinterpret_cast<const T*>(a.table) + token_of(a.ids, a.src, a.prev, row) * d : nullptr;
+  const bool upd = a.base || a.a || a.b || a.table;
   float sum = 0.f, sq = 0.f;
   if constexpr (VPT > 0) {
     float4 v[VPT];
@@ -274,7 +275,12 @@ __global__ __launch_bounds__(BT) void residual_layer_norm_kernel(ResidualLnArgs 
       const int c = 4 * (threadIdx.x + BT * i);
       v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (c < d) {
-        v[i] = *reinterpret_cast<const float4*>(base + c);
+        if (a.table) {
+          v[i] = ld4(token, sizeof(T) == 4, c);
+          v[i].x *= a.scale, v[i].y *= a.scale, v[i].z *= a.scale, v[i].w *= a.scale;
+        } else {
+          v[i] = *reinterpret_cast<const float4*>(base + c);
+        }
         if (a.a) {
           const float4 t = ld4(a.a, a.a_f32, o + c);
           v[i].x += t.x, v[i].y += t.y, v[i].z += t.z, v[i].w += t.w;
@@ -316,7 +322,7 @@ __global__ __launch_bounds__(BT) void residual_layer_norm_kernel(ResidualLnArgs 
     }
   } else {
     for (int c = threadIdx.x; c < d; c += BT) {
-      float v = base[c];
+      float v = a.table ? (float)token[c] * a.scale : base[c];
       if (a.a) v += ldf(a.a, a.a_f32, o + c);
       if (a.b) v += ldf(a.b, a.b_f32, o + c);
       if (upd) x[c] = v;
@@ -582,7 +588,8 @@ void launch_logit_softcap(float* x, long long n, float cap, hipStream_t s) {
 void launch_residual_layer_norm(const ResidualLnArgs& a, int f32, hipStream_t s) {
   if (a.n <= 0) return;
   const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  const bool vec = a.d % 4 == 0 && al(a.x) && al(a.base) && al(a.a) && al(a.b) && al(a.w) && al(a.bias) && al(a.out);
+  const bool vec = a.d % 4 == 0 && al(a.x) && al(a.base) && al(a.a) && al(a.b) && al(a.w) && al(a.bias) && al(a.out) &&
+                   al(a.table);
 #define LN(BT, VPT) DISPATCH_T(f32, (residual_layer_norm_kernel<T, BT, VPT><<<a.n, BT, 0, s>>>(a));)
   const int q = a.d / 4;
   if (!vec || q > 8 * 256) {

@@ -28,7 +28,8 @@ that reads a sublayer's input is one row block of one fused weight (a single lib
 sizes and decays, whose GEMMs leave their fp32 accumulator unrounded; the kernels take column ranges as views.  Step
 launches per layer run: GEMM (the mixer's projections), then
     delta:   GEMM W_b | W_a (fp32; channel decays: W_b, W_a2), conv_silu_qkv (+ conv_state_update in prompt steps; in
-             decode steps W_b | W_a ride along in this launch), delta_rule, (GEMM W_g2,) gated_group_norm, GEMM W_o
+             decode steps W_b | W_a ride along in this launch), delta_rule, (GEMM W_g2,) gated_group_norm, GEMM W_o; in decode
+             steps of the sizes it is written for, delta_token does everything up to W_o
     latent:  latent_prep, bmm (absorb W_uk), rope_pairs, latent_attn (sink, gate), bmm (W_uv), GEMM W_o
     residual_layer_norm; GEMM gate|up, silu_mul, GEMM down; residual_layer_norm (+ e in front of a loop's next pass)
 All intermediates live in the preallocated Workspace, so decode steps are hipGraph-capturable.
@@ -194,6 +195,13 @@ class BeletarLM:
         prefill = b.kind != "decode"
         cu = b.cu_q if prefill else None
         z = self._linear("z", h, P["w_h"])
+        gy = self._buf("del.gy", (T, H * V))
+        if not prefill and self.dtype == torch.bfloat16 and G == H:
+            low = (self._cols(z, P, "a1"), P["a2"], P["g2"]) if m.channel else None
+            if ops.delta_token(self._cols(z, P, "qkv"), P["conv"], cache.conv[n], b.prev_row, b.save_slot, H, N, V, N ** -0.5, UNIT_EPS,
+                               (h, P["gates"]), low, P["dt_bias"], P["A_log"], cache.rec[n], self._cols(z, P, "g1" if low else "g"),
+                               P["norm"], self.cfg.norm_eps, gy):
+                return self._linear("mix.out", gy, P["o"])
         # (a decode step's few rows take these few outputs along in the convolution's launch)
         along = None
         if not prefill and T <= GATES_ALONG_ROWS:
@@ -217,7 +225,6 @@ class BeletarLM:
         ops.delta_rule(m.channel, q, k, v, dz, P["dt_bias"], P["A_log"], gates[:, :H], cache.rec[n], cu, b.prev_row,
                        b.save_slot, runs, y, tiles, ws)
         gate = self._linear("del.g", self._cols(z, P, "g1"), P["g2"]) if m.channel else self._cols(z, P, "g")
-        gy = self._buf("del.gy", (T, H * V))
         ops.gated_group_norm(y, gate, P["norm"], self.cfg.norm_eps, V, False, gy, sigmoid=m.channel)
         return self._linear("mix.out", gy, P["o"])
 
@@ -268,9 +275,10 @@ class BeletarLM:
         e = self._buf("e", (T, d), torch.float32) if self.loops else x
         h = self._buf("h", (T, d))
         src = b.src if b.src is not None and not prefill else None
-        ops.embed_scale(b.input_ids, self.embed, cfg.embed_scale, e, src, self.last_ids if src is not None else None)
         w, bias = self.subs[0][1]["norm1"]
-        ops.residual_layer_norm(e, w=w, bias=bias, eps=eps, out=h)
+        ops.embed_layer_norm(b.input_ids, self.embed, cfg.embed_scale, e, w, bias, eps, h, src, self.last_ids if src is not None else None)
+        # (a decode step's rows are the head's, so the last sum's norm is the head's as well)
+        head = self._buf("logits.xn", (T, d)) if not prefill and T == b.num_seqs and (b.sample or b.need_logits) else None
         base = e if self.loops else None
         for s, (n, P, which, _) in enumerate(self.subs):
             if which == 2:
@@ -285,6 +293,8 @@ class BeletarLM:
             if nxt is not None:
                 w, bias = nxt[1][f"norm{nxt[2]}"]
                 kw = {"w": w, "bias": bias, "eps": eps, "out": h}
+            elif head is not None and self.layer_outputs is None:
+                kw = {"w": self.final_norm[0], "bias": self.final_norm[1], "eps": eps, "out": head}
             if self.layer_outputs is not None and (nxt is None or nxt[0] != n):
                 ops.residual_layer_norm(x, y, base=base)
                 self.layer_outputs.append(x.clone())
@@ -298,7 +308,7 @@ class BeletarLM:
         self.last_logits = None
         if b.sample or b.need_logits:
             rows = None if not prefill else b.last_idx
-            logits = self._logits("logits", x, rows, n)
+            logits = self._logits("logits", x, rows, n, head if self.layer_outputs is None else None)
             if b.need_logits:
                 self.last_logits = logits
             if b.sample:
@@ -310,9 +320,10 @@ class BeletarLM:
             self.last_logits = self._logits("want_logits", x, b.logit_rows, int(b.logit_rows.numel()))
         return ids
 
-    def _logits(self, name: str, x: torch.Tensor, rows, n: int) -> torch.Tensor:
-        """fp32 logits [n, V] = n_f(x[rows]) . E^T (fp32 output from the library GEMM)."""
-        xn = self._buf(name + ".xn", (n, self.cfg.hidden_size))
-        w, bias = self.final_norm
-        ops.residual_layer_norm(x, w=w, bias=bias, eps=self.cfg.norm_eps, rows=rows, out=xn)
+    def _logits(self, name: str, x: torch.Tensor, rows, n: int, xn=None) -> torch.Tensor:
+        """fp32 logits [n, V] = n_f(x[rows]) . E^T (fp32 output from the library GEMM); ``xn``: the norm, where it is at hand."""
+        if xn is None:
+            xn = self._buf(name + ".xn", (n, self.cfg.hidden_size))
+            w, bias = self.final_norm
+            ops.residual_layer_norm(x, w=w, bias=bias, eps=self.cfg.norm_eps, rows=rows, out=xn)
         return self._linear_f32(name, xn, self.embed)

@@ -1337,6 +1337,14 @@ def residual_layer_norm(x, a=None, b=None, w=None, bias=None, eps=0.0, rows=None
     return reference.residual_layer_norm(x, a, b, w, bias, eps, rows, out, base)
 
 
+def embed_layer_norm(ids, table, scale, x, w, bias, eps, out, src=None, prev=None):
+    """embed_scale and the layer norm of its rows in one pass."""
+    if _gpu(x):
+        return _hyb().embed_layer_norm(ids, src, prev, table, float(scale), x, w, bias, float(eps), out)
+    reference.embed_scale(reference.resolve_ids(ids, src, prev), table, scale, x)
+    reference.residual_layer_norm(x, None, None, w, bias, eps, None, out, None)
+
+
 def conv_silu_qkv(z, w, state, cu_q, row_seq, prev_row, runs, G, N, H, P, q_scale, unit_eps, q_out, k_out, v_out,
                   save_slot=None, gates=None):
     """z [T, G N | G N | H P] (a view) = q | k | v through the causal per-channel convolution w [C, taps] over every run
@@ -1383,6 +1391,19 @@ def delta_rule(channel, q, k, v, dz, dt_bias, A_log, bz, state, cu_q, prev_row, 
                                  out, tiles, ws, DELTA_IMPL if impl is None else int(impl))
     reference.delta_rule(channel, q, k, v, dz, dt_bias, A_log, bz, state, cu_q, prev_row, save_slot, runs, out)
     return 1
+
+
+def delta_token(z, cw, conv, prev_row, save_slot, H, N, P, q_scale, unit_eps, gates, low, dt_bias, A_log, state, gate, w, eps, out) -> bool:
+    """A decode step's rows (each a run of its own, bf16, as many query / key heads as value heads) from the projection z to the gated
+    heads, one launch: conv_silu_qkv with save_slot, delta_rule, gated_group_norm(., gate, w, eps, P, False) -> out bf16 [T, H P].
+    ``gates`` = (x [T, d], W [H or 2 H, d]): bz = x W[:H]^T, dz = x W[H:]^T in fp32.  ``low`` = (a1 [T, r], a2 [H N, r], g2 [H P, r']):
+    decays per channel dz = a1 a2^T in fp32, and the gate is sigmoid of bf16(gate g2^T), gate [T, r'].  False: not one of its sizes,
+    nothing has been done."""
+    if not _gpu(z):
+        return False
+    a1, a2, g2 = low if low is not None else (None, None, None)
+    return _hyb().delta_token(z, cw, conv, prev_row, save_slot, int(H), int(N), int(P), float(q_scale), float(unit_eps), *gates, a1, a2,
+                              dt_bias, A_log, state, gate, g2, w, float(eps), out)
 
 
 # ---- attention whose values are its keys, routed squared-ReLU experts (csrc/kernels/hybrid_rows.hip, routed_ff.hip) ----

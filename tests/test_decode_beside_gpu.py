@@ -213,3 +213,57 @@ def test_embedding_with_the_first_norm(T, d):
     ops.rms_norm_rows(y, None, w2, 1e-5, 1.0, want)
     assert torch.equal(x, y)
     assert torch.allclose(h.float(), want.float(), rtol=2 ** -7, atol=1e-6)      # (the sums of squares in another order)
+
+
+@pytest.mark.parametrize("T,H,P,rank,grank", [(1, 8, 256, 0, 0), (6, 3, 128, 0, 0), (16, 8, 64, 0, 0), (65, 2, 256, 0, 0),
+                                              (1, 8, 256, 128, 128), (5, 3, 128, 32, 64), (9, 4, 64, 96, 160)])
+def test_delta_token(T, H, P, rank, grank):
+    N, d, taps, channel = 128, 2048 if H == 8 else 264, 4, rank > 0
+    C = 2 * H * N + H * P
+    wide = rnd(T, C + (rank + grank if channel else H * P) + 8, seed=1)
+    z = wide[:, :C]
+    x, gw = rnd(T, d, seed=2), rnd(H if channel else 2 * H, d, scale=d ** -0.5, seed=3)
+    cw, conv = rnd(C, taps, scale=0.5, seed=4), rnd(2 * T + 1, taps - 1, C, seed=5)
+    bias, alog = rnd(H * N if channel else H, dtype=F32, seed=6) - 2, rnd(H, dtype=F32, seed=7)
+    state, w = rnd(2 * T + 1, H, N, P, dtype=F32, scale=0.3, seed=8), 1 + 0.1 * rnd(P, dtype=F32, seed=9)
+    prev, save = slots_of(T, state.shape[0])
+    gates = x.float() @ gw.float().t()
+    if channel:
+        a1, g1 = wide[:, C:C + rank], wide[:, C + rank:C + rank + grank]
+        a2, g2 = rnd(H * N, rank, scale=rank ** -0.5, seed=10), rnd(H * P, grank, scale=grank ** -0.5, seed=11)
+        dz, gate, low, gin = a1.float() @ a2.float().t(), (g1.float() @ g2.float().t()).to(B16), (a1, a2, g2), g1
+    else:
+        dz, gate, low = gates[:, H:], wide[:, C:C + H * P], None
+        gin = gate
+    st, cs = state.clone(), conv.clone()
+    q, k, v, y = torch.empty(T, H, N), torch.empty(T, H, N), torch.empty(T, H, P, dtype=B16), torch.empty(T, H * P)
+    reference.conv_silu_qkv(z, cw, cs, None, prev, T, H, N, H, P, N ** -0.5, 1e-6, q, k, v)
+    reference.conv_state_update(z, cs, None, prev, save, T)
+    reference.delta_rule(channel, q, k, v, dz, bias, alog, gates[:, :H], st, None, prev, save, T, y)
+    want = torch.empty(T, H * P)
+    reference.gated_group_norm(y, gate, w, 1e-5, P, False, want, channel)
+    gz, gcs, gst, out = gpu(z), conv.cuda(), state.cuda(), torch.empty(T, H * P, dtype=B16, device="cuda")
+    done = ops.delta_token(gz, cw.cuda(), gcs, prev.cuda(), save.cuda(), H, N, P, N ** -0.5, 1e-6, (x.cuda(), gw.cuda()),
+                           tuple(map(gpu, low)) if low else None, bias.cuda(), alog.cuda(), gst, gpu(gin), w.cuda(), 1e-5, out)
+    assert done
+    assert torch.equal(gcs.cpu(), cs)
+    # fp32 but for the roundings to bf16 of the values (an ulp where a sum's order turns one), the gate's factor and the result
+    assert torch.allclose(gst.cpu(), st, rtol=1e-4, atol=2e-3)
+    assert (gst.cpu() - st).norm() < 1e-4 * st.norm()
+    err = (out.float().cpu() - want).norm() / want.norm()
+    assert err < 2.5e-3, err            # (one rounding to bf16: 2^-9 / sqrt(3) of a value uniform in its binade, 1.7e-3 with the gate's)
+    assert torch.allclose(out.float().cpu(), want, rtol=2 ** -6, atol=2e-2)
+
+
+@pytest.mark.parametrize("T,d", [(1, 2048), (7, 1000), (300, 4096), (600, 1001)])
+def test_embedding_with_the_first_layer_norm(T, d):
+    ids = torch.randint(0, 50, (T,), dtype=I32, generator=torch.Generator().manual_seed(1)).cuda()
+    src = torch.tensor([r % 3 - 1 for r in range(T)], dtype=I32).cuda()
+    prev = torch.tensor([7, 9], dtype=I32).cuda()
+    table, w, b = rnd(50, d, seed=2).cuda(), rnd(d, dtype=F32, seed=3).cuda(), rnd(d, dtype=F32, seed=4).cuda()
+    x, y = torch.empty(T, d, device="cuda"), torch.empty(T, d, device="cuda")
+    h, want = torch.empty(T, d, dtype=B16, device="cuda"), torch.empty(T, d, dtype=B16, device="cuda")
+    ops.embed_layer_norm(ids, table, 8.0, x, w, b, 1e-6, h, src, prev)
+    ops.embed_scale(ids, table, 8.0, y, src, prev)
+    ops.residual_layer_norm(y, w=w, bias=b, eps=1e-6, out=want)
+    assert torch.equal(x, y) and torch.equal(h, want)
