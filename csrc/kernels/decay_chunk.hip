@@ -13,7 +13,7 @@
 // Precision: q, k and v are bf16, so they are exact operands of v_mfma_f32_16x16x32_bf16, which accumulates in fp32.  An
 // fp32 operand (the state, a scaled vector, the scores) is used as the sum of three bf16 parts (bf16_parts.h).
 //
-// Work split: grid (P / 64, heads, runs), 4 waves of 16 value columns and ALL of N: the state stays in accumulator registers
+// Work split: grid (P / 64, heads, runs), waves of 16 value columns with all of N or half of it: the state stays in accumulator registers
 // for the whole run.  An accumulator's rows are 4 (lane / 16) + r, a B operand's contraction index is 8 (lane / 16) + j; with
 // the contraction taken in the order j < 4: 4 g + j, else 16 + 4 g + j - 4, two accumulator tiles ARE a B operand, and the A
 // operand is read in the same order (two 8-byte LDS reads).  The same holds for the values and, computed transposed, for the
@@ -215,24 +215,39 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
   }
 }
 
+// bytes of LDS of a walk: two stages, mode 1's sums, the parts that waves hand over
+constexpr int scan_lds(int mode, int NB, int HV) {
+  const int NP = 32 * NB, rows = (mode == 0 ? 6 : 2) * C * (NP + 8) * 2;
+  return 2 * (rows + (mode == 0 ? (C * LT + NP) * 4 : 0)) + (mode == 1 ? 8 * HV * 3 * C * 4 : 0) + (HV - 1) * 16 * 4 * HV * 128;
+}
+
 // ---- the walk ------------------------------------------------------------------------------------------------------------
-// NB: 32-channel blocks of the state (N <= 32 NB).  256 registers a lane, although LDS leaves mode 0 one workgroup a CU: with more
-// allowed the compiler keeps a part in AGPRs, and 8 heads x 128 x 256 take, us, 64 runs of 50 tokens 100 -> 165, 128 of 50 214 ->
-// 415, 8 of 1012 131 -> 140.
-template <int MODE, int NB>
-__global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a) {
+// NB: 32-channel blocks of the state (N <= 32 NB).  HV: 2 where two waves share 16 columns, each with half of N: the parts of the
+// state, which are formed anew for every chunk, and the staging are most of the vector work, and with a wave a SIMD (mode 0's LDS
+// leaves one workgroup a CU) nothing covers the waits.  Each of the two finishes one of the chunk's row tiles and hands its part of the
+// other over in LDS; it is read behind the chunk's barrier and stored a chunk later (8 heads x 128 x 256, us: 8 runs of 1012 tokens 210
+// -> 197, 2 of 750 101 -> 92; 64 x 128 x 64, 2 of 750, 84.5 -> 80.5).  256 registers a lane: with more allowed the
+// compiler keeps a part in AGPRs, which was slower.
+template <int MODE, int NB, int HV>
+__global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanArgs a) {
+  constexpr int TH = NT * HV, NWV = 4 * HV, NBW = NB / HV, TI = 2 / HV;
   constexpr int NP = 32 * NB, LQ = NP + 8;              // LQ: bf16 pitch of a [C][NP] matrix
   constexpr int PL = MODE == 0 ? 3 : 1;                 // bf16 parts of the staged vectors
   constexpr int oK = PL * C * LQ, oF = oK + PL * C * LQ;      // in bf16: q | k, a part behind the other
-  constexpr int FS = MODE == 0 ? C * LT + NP : 3 * C;   // floats: A | 2^(G_C), or G | its low part | b
+  constexpr int FS = MODE == 0 ? C * LT + NP : 0;       // floats: A | 2^(G_C)
   constexpr int STAGE = oF * 2 + FS * 4;                // bytes
+  constexpr int SUMS = MODE == 1 ? 2 * NWV * 3 * C : 0; // floats, mode 1: G | its low part | b of 2 NWV chunks
   static_assert(STAGE % 16 == 0, "stages start at multiples of 16 bytes");
+  static_assert(2 * STAGE + SUMS * 4 + (HV - 1) * 16 * NWV * 128 == scan_lds(MODE, NB, HV), "the launch's LDS");
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  float* const sums = reinterpret_cast<float*>(smem + 2 * STAGE);
+  f32x4* const given = reinterpret_cast<f32x4*>(smem + 2 * STAGE + SUMS * 4);      // [2][NWV][64]
   const int N = a.N, P = a.P, h = blockIdx.y, run = blockIdx.z;
   const int s0 = a.cu_q[run], s1 = a.cu_q[run + 1];
   if (s1 <= s0) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
-  const int p = blockIdx.x * 64 + wave * 16 + col;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, g = lane >> 4;
+  const int hf = HV == 2 ? wave >> 2 : 0, ch0 = 32 * NBW * hf;      // the wave's channels
+  const int p = blockIdx.x * 64 + (wave & 3) * 16 + col;
   const bool pin = p < P;
   const int chunks = (s1 - s0 + C - 1) / C;
   const int pr = a.prev_row[s0], sv = a.save_slot[s1 - 1];
@@ -246,15 +261,14 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
   float* out = a.out + ((long long)s0 * a.H + h) * P;
   const long long orow = (long long)a.H * P;
   const int ldv = (int)a.ldv * 2, ldo = (int)orow * 4;                            // (decay_chunk_takes bounds them)
-  const int vo = pin ? 4 * g * ldv + 2 * p : NO_PLACE, oo = pin ? 4 * g * ldo + 4 * p : NO_PLACE;
+  const int vo = pin ? 4 * g * ldv + 2 * p : NO_PLACE, oo = pin ? (4 * g + 16 * hf) * ldo + 4 * p : NO_PLACE;
 
   // staging: thread (token tt, 8 channels from c8), PASS tokens apart
-  constexpr int GR = NP / 8, TSTEP = NT / GR, PASS = (C + TSTEP - 1) / TSTEP;
+  constexpr int GR = NP / 8, TSTEP = TH / GR, PASS = (C + TSTEP - 1) / TSTEP;
   const int c8 = 8 * (tid % GR), tt0 = tid / GR;
   const bool nin = c8 < N && tt0 < C;                   // (N is a multiple of 8)
   Pack8 rq[PASS], rk[MODE == 1 ? PASS : 1];
   f32x4 rp[MODE == 0 ? PASS : 1][2], ry[MODE == 0 ? PASS : 1][2], pl, ra;   // mode 0: 2^(G_i), k_i 2^(G_C - G_i), 2^(G_C)
-  float rdt = 0.f;
   bf16 vn[8];
   int qo[PASS], ko[PASS], wo[PASS];
 #pragma unroll
@@ -279,12 +293,11 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
           ry[u][i] = row16f(bw, wo[u] + (nin ? 4 * N + 16 * i : 0));
         }
       pl = 4 * tid < N ? lds4(ws + (t0 + nt - 1) * wrow + C + 4 * tid) : f32x4{0.f, 0.f, 0.f, 0.f};
-      ra = row16f(bw, (tid / 8) * (int)wrow * 4 + 16 * (tid % 8));
+      ra = row16f(bw, tid < 8 * C ? (tid / 8) * (int)wrow * 4 + 16 * (tid % 8) : NO_PLACE);
     } else {
       const __amdgpu_buffer_rsrc_t bk = chunk_rows(k + t0 * a.ldk, a.ldk * 2, nt, N * 2);
 #pragma unroll
       for (int u = 0; u < PASS; ++u) rk[u].u = row16(bk, ko[u]);
-      if (tid < C) rdt = (float)row2(chunk_rows(dt + t0 * a.ldd, a.ldd * 2, nt, 2), tid * (int)a.ldd * 2) + a.dbias[h];
     }
   };
   auto fetch_v = [&](int c) {
@@ -292,11 +305,27 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
 #pragma unroll
     for (int i = 0; i < 8; ++i) vn[i] = row2(bv, vo + (pin ? (16 * (i >> 2) + (i & 3)) * ldv : 0));
   };
-  const float rate2 = MODE == 1 ? expf(a.rate[h]) * LOG2E : 0.f;
+  // Mode 1: a chunk's step sizes and the running sum of its log decays, by one wave; the waves do those of the NWV chunks ahead
+  // together (one wave a chunk, the others waited for it: 64 x 128 x 64, 8 runs of 1012 tokens, 190 -> 186 us).  The sum is a pair of floats: with step sizes that forget in a few tokens
+  // it grows to hundreds, and the differences of neighbours, which are what counts, would keep few of its digits.
+  const float rate2 = MODE == 1 ? expf(a.rate[h]) * LOG2E : 0.f, dbias = MODE == 1 ? a.dbias[h] : 0.f;
+  float rdt = 0.f;
+  auto fetch_step = [&](int c) { rdt = lane < s1 - s0 - c * C && lane < C ? (float)dt[(long long)(c * C + lane) * a.ldd] + dbias : 0.f; };
+  auto sum_steps = [&](int c) {
+    if (c >= chunks) return;
+    const int nt = min(C, s1 - s0 - c * C);
+    const float b = lane < nt ? softplus_exact(rdt) : 0.f;
+    double s = lane < nt ? log_decay(-(double)rate2 * b) : 0.0;
+    s = prefix32(s, lane);
+    float* fs = sums + (c & (2 * NWV - 1)) * 3 * C;
+    if (lane < C) {
+      fs[lane] = (float)s;
+      fs[C + lane] = (float)(s - (double)(float)s);
+      fs[2 * C + lane] = b;
+    }
+  };
   auto stash = [&](int c) {
     bf16* st = reinterpret_cast<bf16*>(smem + (c & 1) * STAGE);
-    float* fs = reinterpret_cast<float*>(st + oF);
-    const int nt = min(C, s1 - s0 - c * C);
 #pragma unroll
     for (int u = 0; u < PASS; ++u) {
       const int tt = tt0 + TSTEP * u;
@@ -318,39 +347,39 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
       }
     }
     if constexpr (MODE == 0) {
-      *reinterpret_cast<f32x4*>(fs + (tid / 8) * LT + 4 * (tid % 8)) = ra;
+      float* fs = reinterpret_cast<float*>(st + oF);
+      if (tid < 8 * C) *reinterpret_cast<f32x4*>(fs + (tid / 8) * LT + 4 * (tid % 8)) = ra;
       if (4 * tid < NP) *reinterpret_cast<f32x4*>(fs + C * LT + 4 * tid) = pl;
-    } else if (wave == 0) {
-      // running sum over the chunk's tokens as a pair of floats: with step sizes that forget in a few tokens the sum grows
-      // to hundreds, and the differences of neighbours, which are what counts, would keep few of its digits
-      const float b = tid < nt ? softplus_exact(rdt) : 0.f;
-      double s = tid < nt ? log_decay(-(double)rate2 * b) : 0.0;
-      s = prefix32(s, tid);
-      if (tid < C) {
-        fs[tid] = (float)s;
-        fs[C + tid] = (float)(s - (double)(float)s);
-        fs[2 * C + tid] = b;
-      }
     }
   };
 
-  f32x4 S[2 * NB];
+  f32x4 S[2 * NBW];
   const bool old = pr <= -2 && pin;
   const float* st0 = a.state + (old ? (long long)(-(pr + 2)) * a.state_stride + (long long)h * N * P + p : 0);
 #pragma unroll
-  for (int t = 0; t < 2 * NB; ++t)
+  for (int t = 0; t < 2 * NBW; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int n = 16 * t + 4 * g + r;
+      const int n = ch0 + 16 * t + 4 * g + r;
       S[t][r] = old && n < N ? st0[(long long)n * P] : 0.f;
     }
   const float skip = a.skip ? a.skip[h] : 0.f;
   fetch(0);
   fetch_v(0);
+  if constexpr (MODE == 1) {
+    fetch_step(wave);
+    sum_steps(wave);
+  }
   stash(0);
   __syncthreads();
+  f32x4 mine = {0.f, 0.f, 0.f, 0.f};                    // HV 2: the wave's row tile of the chunk before, without the other's part
+  auto store_tile = [&](int c, int i, f32x4 y) {        // row tile i past the wave's first
+    const __amdgpu_buffer_rsrc_t bo = chunk_rows(out + (long long)c * C * orow, orow * 4, min(C, s1 - s0 - c * C), P * 4);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y[r]), bo, oo + (pin ? (16 * i + r) * ldo : 0), 0, 0);
+  };
   for (int c = 0; c < chunks; ++c) {
-    const int nt = min(C, s1 - s0 - c * C);
     Pack8 V;
 #pragma unroll
     for (int i = 0; i < 8; ++i) V.h[i] = vn[i];
@@ -359,12 +388,16 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
       fetch(c + 1);
       fetch_v(c + 1);
     }
+    if constexpr (MODE == 1)
+      if (c % NWV == 0 && c + NWV < chunks) fetch_step(c + NWV + wave);
     __builtin_amdgcn_sched_barrier(0);                  // the next chunk's loads in flight ahead of this one's products
+    if constexpr (HV == 2)
+      if (c) store_tile(c - 1, 0, mine + a.q_scale * given[(((c - 1) & 1) * NWV + wave) * 64 + lane]);
     const bf16* st = reinterpret_cast<const bf16*>(smem + (c & 1) * STAGE);
-    const float* fs = reinterpret_cast<const float*>(st + oF);
-    const bf16* Qr = st + col * LQ + 4 * g;
+    const float* fs = MODE == 0 ? reinterpret_cast<const float*>(st + oF) : sums + (c & (2 * NWV - 1)) * 3 * C;
+    const bf16* Qr = st + col * LQ + 4 * g + ch0;
     f32x4 O[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    f32x4 A[2][2];                                      // scores of row tile i, columns 4 g + r and 16 + 4 g + r
+    f32x4 A[TI][2];                                     // scores of row tile i, columns 4 g + r and 16 + 4 g + r
     f32x4 gj[2], lj[2], bj[2];
     // A wave or two a SIMD: LDS reads stand a step ahead of the products that take them, and the parts of the next state tiles
     // are formed between products (left to the compiler, every read was waited for: half of the walk).
@@ -376,12 +409,12 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
         for (int i = 0; i < 2; ++i) qf[t & 1][part][i] = pair4(Qr + (part * C + 16 * i) * LQ + 32 * t);
     };
     load_q(0);
-    if (NB > 1) load_q(1);
+    if (NBW > 1) load_q(1);
     if constexpr (MODE == 0) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) A[i][j] = lds4(fs + (16 * i + col) * LT + 16 * j + 4 * g);
+        for (int j = 0; j < 2; ++j) A[i][j] = lds4(fs + (16 * (i + hf) + col) * LT + 16 * j + 4 * g);
     } else {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
@@ -393,9 +426,9 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
     Parts s = split<true>(S[0], S[1]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < NB; ++t) {
+    for (int t = 0; t < NBW; ++t) {
       Parts next = s;
-      if (t + 1 < NB) next = split<true>(S[2 * t + 2], S[2 * t + 3]);
+      if (t + 1 < NBW) next = split<true>(S[2 * t + 2], S[2 * t + 3]);
 #pragma unroll
       for (int term = 0; term < (MODE == 0 ? 6 : 3); ++term)
 #pragma unroll
@@ -409,7 +442,7 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
             O[i] = mfma16(f[0][i], term == 0 ? s.l : term == 1 ? s.m : s.h, O[i]);
           }
         }
-      if (t + 2 < NB) load_q(t + 2);
+      if (t + 2 < NBW) load_q(t + 2);
       s = next;
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -430,63 +463,71 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
       bad = min(bad, __shfl_xor(bad, 32, 64));
     }
     if constexpr (MODE == 1) {
-      bf16x8 kf[2][NB], qn[2][NB];
-      float gi[2], li[2];
+      bf16x8 kf[2][NB], qn[TI][NB];
+      float gi[TI], li[TI];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        gi[i] = fs[16 * i + col], li[i] = fs[C + 16 * i + col];
+      for (int i = 0; i < TI; ++i) {
+        gi[i] = fs[16 * (i + hf) + col], li[i] = fs[C + 16 * (i + hf) + col];
 #pragma unroll
-        for (int t = 0; t < NB; ++t) {
-          kf[i][t] = *reinterpret_cast<const bf16x8*>(st + oK + (16 * i + col) * LQ + 8 * g + 32 * t);
-          qn[i][t] = *reinterpret_cast<const bf16x8*>(st + (16 * i + col) * LQ + 8 * g + 32 * t);
-        }
+        for (int t = 0; t < NB; ++t)
+          qn[i][t] = *reinterpret_cast<const bf16x8*>(st + (16 * (i + hf) + col) * LQ + 8 * g + 32 * t);
       }
+      const bool second = HV == 1 || hf;                // (the first row tile sees the first columns only)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int t = 0; t < NB; ++t)
+          if (i == 0 || second) kf[i][t] = *reinterpret_cast<const bf16x8*>(st + oK + (16 * i + col) * LQ + 8 * g + 32 * t);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) O[j][r] *= pow2(gj[j][r]);      // (rows 4 g + r of O too)
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) A[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int t = 0; t < NB; ++t) {
-        A[0][0] = mfma16(kf[0][t], qn[0][t], A[0][0]);
-        A[1][0] = mfma16(kf[0][t], qn[1][t], A[1][0]);
-        A[1][1] = mfma16(kf[1][t], qn[1][t], A[1][1]);
+#pragma unroll
+        for (int i = 0; i < TI; ++i) A[i][0] = mfma16(kf[0][t], qn[i][t], A[i][0]);
+        if (second) A[TI - 1][1] = mfma16(kf[1][t], qn[TI - 1][t], A[TI - 1][1]);
       }
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int j = 0; j <= i; ++j)
+        for (int j = 0; j < (HV == 1 ? i + 1 : 2); ++j)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const float w = pow2((gi[i] - gj[j][r]) + (li[i] - lj[j][r])) * bj[j][r];
             float y = A[i][j][r] * w;
             asm volatile("" : "+v"(y));                 // (a select, no branch around the exponential)
-            A[i][j][r] = j < i || 4 * g + r <= col ? y : 0.f;
+            A[i][j][r] = j < i + hf || (j == i + hf && 4 * g + r <= col) ? y : 0.f;
           }
     }
     // k^T as an A operand in the accumulators' order: 16 channels of 4 tokens at 4 g, 4 at 16 + 4 g (LDS transpose reads)
-    const char* Kt = reinterpret_cast<const char*>(st + oK + (4 * g + (col >> 2)) * LQ) + 8 * (col & 3);
+    const char* Kt = reinterpret_cast<const char*>(st + oK + (4 * g + (col >> 2)) * LQ + ch0) + 8 * (col & 3);
     auto turned = [&](int part, int t) {
       Pack8 f;
       const uint2 x = read_tr(Kt + (part * C * LQ + 16 * t) * 2), y = read_tr(Kt + ((part * C + 16) * LQ + 16 * t) * 2);
       f.u = make_uint4(x.x, x.y, y.x, y.y);
       return f.v;
     };
-    bf16x8 kt[2 * NB];                                  // of the part at hand
+    bf16x8 kt[2 * NBW];                                 // of the part at hand
 #pragma unroll
-    for (int t = 0; t < 2 * NB; ++t) kt[t] = turned(PL - 1, t);
-    f32x4 dec[MODE == 0 ? 2 * NB : 1];
+    for (int t = 0; t < 2 * NBW; ++t) kt[t] = turned(PL - 1, t);
+    f32x4 dec[MODE == 0 ? 2 * NBW : 1];
     if constexpr (MODE == 0) {
 #pragma unroll
-      for (int t = 0; t < 2 * NB; ++t) dec[t] = lds4(fs + C * LT + 16 * t + 4 * g);
+      for (int t = 0; t < 2 * NBW; ++t) dec[t] = lds4(fs + C * LT + ch0 + 16 * t + 4 * g);
+    }
+    if constexpr (HV == 2) {
+      given[((c & 1) * NWV + (wave ^ 4)) * 64 + lane] = hf ? O[0] : O[1];
+      if (hf) O[0] = O[1];
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < TI; ++i) {
       const Parts u = split(A[i][0], A[i][1]);
       O[i] = mfma16(u.l, W.v, O[i]);
       O[i] = mfma16(u.m, W.v, O[i]);
@@ -494,35 +535,33 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
     }
     if (bad < C) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (16 * i + 4 * g + r >= bad) O[i][r] = __builtin_nanf("");
+          if (16 * (i + hf) + 4 * g + r >= bad) O[i][r] = __builtin_nanf("");
     }
-    {
-      const __amdgpu_buffer_rsrc_t bo = chunk_rows(out + (long long)c * C * orow, orow * 4, nt, P * 4);
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TI; ++i) {
+      f32x4 y;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float y = a.q_scale * O[i][r] + skip * (float)V.h[4 * i + r];
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), bo, oo + (pin ? (16 * i + r) * ldo : 0), 0, 0);
-        }
+      for (int r = 0; r < 4; ++r) y[r] = a.q_scale * O[i][r] + skip * (float)(HV == 2 && hf ? V.h[4 + r] : V.h[4 * i + r]);
+      if constexpr (HV == 2) mine = y;
+      else store_tile(c, i, y);
     }
     if constexpr (MODE == 0) {
 #pragma unroll
-      for (int t = 0; t < 2 * NB; ++t) S[t] *= dec[t];
+      for (int t = 0; t < 2 * NBW; ++t) S[t] *= dec[t];
 #pragma unroll
       for (int part = 2; part >= 0; --part) {
-        bf16x8 nk[2 * NB];
+        bf16x8 nk[2 * NBW];
 #pragma unroll
-        for (int t = 0; t < 2 * NB; ++t)
+        for (int t = 0; t < 2 * NBW; ++t)
           if (part) nk[t] = turned(part - 1, t);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < 2 * NB; ++t) S[t] = mfma16(kt[t], V.v, S[t]);
+        for (int t = 0; t < 2 * NBW; ++t) S[t] = mfma16(kt[t], V.v, S[t]);
 #pragma unroll
-        for (int t = 0; t < 2 * NB; ++t)
+        for (int t = 0; t < 2 * NBW; ++t)
           if (part) kt[t] = nk[t];
       }
     } else {
@@ -534,44 +573,60 @@ __global__ __launch_bounds__(NT, 2) void decay_chunk_scan_kernel(DecayScanArgs a
         for (int r = 0; r < 4; ++r) w[j][r] = pow2((gc - gj[j][r]) + (lc - lj[j][r])) * bj[j][r] * (float)V.h[4 * j + r];
       const Parts u = split(w[0], w[1]);
 #pragma unroll
-      for (int t = 0; t < 2 * NB; ++t) S[t] = mfma16(kt[t], u.l, S[t] * d);
+      for (int t = 0; t < 2 * NBW; ++t) S[t] = mfma16(kt[t], u.l, S[t] * d);
 #pragma unroll
-      for (int t = 0; t < 2 * NB; ++t) S[t] = mfma16(kt[t], u.m, S[t]);
+      for (int t = 0; t < 2 * NBW; ++t) S[t] = mfma16(kt[t], u.m, S[t]);
 #pragma unroll
-      for (int t = 0; t < 2 * NB; ++t) S[t] = mfma16(kt[t], u.h, S[t]);
+      for (int t = 0; t < 2 * NBW; ++t) S[t] = mfma16(kt[t], u.h, S[t]);
+      if (c % NWV == NWV / 2 && c + NWV / 2 < chunks) sum_steps(c + NWV / 2 + wave);
     }
     if (more) stash(c + 1);
     __syncthreads();                                    // chunk c + 1 is staged, chunk c has been read
   }
+  if constexpr (HV == 2) store_tile(chunks - 1, 0, mine + a.q_scale * given[(((chunks - 1) & 1) * NWV + wave) * 64 + lane]);
   if (sv >= 0 && pin) {
     float* so = a.state + (long long)sv * a.state_stride + (long long)h * N * P + p;
 #pragma unroll
-    for (int t = 0; t < 2 * NB; ++t)
+    for (int t = 0; t < 2 * NBW; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int n = 16 * t + 4 * g + r;
+        const int n = ch0 + 16 * t + 4 * g + r;
         if (n < N) so[(long long)n * P] = S[t][r];
       }
   }
 }
 
-template <int MODE, int NB>
-void launch_chunks(const DecayScanArgs& a, hipStream_t s) {
-  constexpr int NP = 32 * NB, LQ = NP + 8, PL = MODE == 0 ? 3 : 1;
-  constexpr int elems = 2 * PL * C * LQ;
-  constexpr int lds = 2 * (elems * 2 + (MODE == 0 ? C * LT + NP : 3 * C) * 4);
-  constexpr int prep = 4 * C * (NP + 4) * 4;
+template <int MODE, int NB, int HV>
+void launch_scan(const DecayScanArgs& a, hipStream_t s) {
+  constexpr int lds = scan_lds(MODE, NB, HV);
   static const bool raised = [] {
-    const auto raise = [](const void* f, int bytes) {
-      if (bytes > 64 * 1024) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    };
-    raise(reinterpret_cast<const void*>(&decay_chunk_scan_kernel<MODE, NB>), lds);
-    if (MODE == 0) raise(reinterpret_cast<const void*>(&decay_chunk_prep_kernel<2 * NB>), prep);
+    if (lds > 64 * 1024)
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&decay_chunk_scan_kernel<MODE, NB, HV>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     return true;
   }();
   (void)raised;
-  if constexpr (MODE == 0) decay_chunk_prep_kernel<2 * NB><<<dim3(2 * a.ntiles, a.H), NT, prep, s>>>(a);
-  decay_chunk_scan_kernel<MODE, NB><<<dim3((a.P + 63) / 64, a.H, a.runs), NT, lds, s>>>(a);
+  decay_chunk_scan_kernel<MODE, NB, HV><<<dim3((a.P + 63) / 64, a.H, a.runs), NT * HV, lds, s>>>(a);
+}
+
+template <int MODE, int NB>
+void launch_chunks(const DecayScanArgs& a, hipStream_t s) {
+  if constexpr (MODE == 0) {
+    constexpr int prep = 4 * C * (32 * NB + 4) * 4;
+    static const bool raised = [] {
+      if (prep > 64 * 1024)
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&decay_chunk_prep_kernel<2 * NB>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, prep);
+      return true;
+    }();
+    (void)raised;
+    decay_chunk_prep_kernel<2 * NB><<<dim3(2 * a.ntiles, a.H), NT, prep, s>>>(a);
+  }
+  if constexpr (NB > 1) {
+    // eight waves a workgroup where LDS (mode 0) or their number (at most one a CU) leaves one of them on a CU
+    if (MODE == 0 || (long long)((a.P + 63) / 64) * a.H * a.runs <= 256) return launch_scan<MODE, NB, 2>(a, s);
+  }
+  launch_scan<MODE, NB, 1>(a, s);
 }
 
 template <int MODE>
