@@ -169,7 +169,9 @@ class BeletarLM:
             P["norm2"] = (f("norm2"), f("norm2.b"))
             P["w_gu"] = torch.cat([t("mlp.gate"), t("mlp.up")], 0).contiguous()
             P["w_down"] = t("mlp.down")
-        P["w_h"], P["cols"] = fz.weight(), fz.cols
+        w_h = fz.weight()
+        P["w_wide"], P["cols"] = ops.pad_wide(w_h), fz.cols
+        P["w_h"] = P["w_wide"][:w_h.shape[0]]
         return P
 
     # ------------------------------------------------------------------------------------------
@@ -184,6 +186,10 @@ class BeletarLM:
         """x [R, K] @ w[N, K]^T -> fp32 [R, N] (the library GEMM's accumulator, unrounded)."""
         return ops.linear_f32(x, w, self._buf(name, (x.shape[0], w.shape[0]), torch.float32))
 
+    def _fused(self, h: torch.Tensor, P: dict) -> torch.Tensor:
+        """Everything that reads a sublayer's input h, in one product."""
+        return ops.linear_wide(h, P["w_wide"], P["w_h"], lambda n: self._buf("z", (h.shape[0], n)), self.ws)
+
     @staticmethod
     def _cols(z: torch.Tensor, P: dict, name: str) -> torch.Tensor:
         c0, n = P["cols"][name]
@@ -194,7 +200,7 @@ class BeletarLM:
         T, H, G, N, V = h.shape[0], m.heads, m.kv_heads, m.dim, m.vdim
         prefill = b.kind != "decode"
         cu = b.cu_q if prefill else None
-        z = self._linear("z", h, P["w_h"])
+        z = self._fused(h, P)
         gy = self._buf("del.gy", (T, H * V))
         if not prefill and self.dtype == torch.bfloat16 and G == H:
             low = (self._cols(z, P, "a1"), P["a2"], P["g2"]) if m.channel else None
@@ -232,7 +238,7 @@ class BeletarLM:
         m = P["mixer"]
         T, H, r, rot, dn = h.shape[0], m.heads, m.kv_rank, m.rot_dim, m.dim
         plane = cache.lat[n]
-        z = self._linear("z", h, P["w_h"])
+        z = self._fused(h, P)
         ops.latent_prep(self._cols(z, P, "dkv"), 0, r, rot, None, P["gkv"], self.cfg.norm_eps, b.positions, b.slot_mapping,
                         P["rope"], None, plane)
         q = self._cols(z, P, "q").unflatten(1, (H, dn + rot))

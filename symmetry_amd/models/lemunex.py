@@ -188,7 +188,9 @@ class LemunexLM:
                 fz.add("shared.up", t("mlp.shared.up"))
                 fz.add("shared.sg", t("mlp.shared.sg"))
                 P["shared.down"] = t("mlp.shared.down")
-        P["w_h"], P["cols"] = fz.weight(), fz.cols
+        w_h = fz.weight()
+        P["w_wide"], P["cols"] = ops.pad_wide(w_h), fz.cols
+        P["w_h"] = P["w_wide"][:w_h.shape[0]]
         return P
 
     # ------------------------------------------------------------------------------------------
@@ -198,6 +200,10 @@ class LemunexLM:
     def _linear(self, name: str, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """x [R, K] @ w[N, K]^T -> [R, N] in the activation dtype (fp32 accumulation)."""
         return ops.linear(x, w, self._buf(name, (x.shape[0], w.shape[0])), self.ws)
+
+    def _fused(self, h: torch.Tensor, P: dict) -> torch.Tensor:
+        """Everything that reads a sublayer's input h, in one product."""
+        return ops.linear_wide(h, P["w_wide"], P["w_h"], lambda n: self._buf("z", (h.shape[0], n)), self.ws)
 
     @staticmethod
     def _cols(z: torch.Tensor, P: dict, name: str) -> torch.Tensor:
@@ -368,7 +374,7 @@ class LemunexLM:
         # (a decode step's rows are the head's, so the last sum's norm is the head's as well)
         head = self._buf("logits.xn", (T, d)) if b.kind == "decode" and T == b.num_seqs and (b.sample or b.need_logits) else None
         for i, P in enumerate(self.L):
-            z = self._linear("z", h, P["w_h"])
+            z = self._fused(h, P)
             ff, along = self._ff(i, P, h, z, b, cache)
             nxt, out = (self.L[i + 1]["norm1"], h) if i + 1 < len(self.L) else (self.final_norm if head is not None else None, head)
             if P["kind"] == "parallel":

@@ -718,14 +718,43 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, ws
     """``x @ w.T``: the few-row kernel up to 16 rows (2048 x 2048 at 8 rows 4.8 us, the library 8.5; 17688 x 2048 21.9 / 49.6),
     with a workspace ``ws`` (a model's: ``get(name, shape, dtype, device, zeros)``) the medium-row kernel up to 256, else the library GEMM (hipBLASLt through torch, the library heuristic; a
     tuned-solution table measured neutral end to end and was removed: profiles/r4/blaslt_tuned_ab.jsonl)."""
+    if own_linear(x, w, out, ws):
+        return out
+    return torch.matmul(x, w.t(), out=out)
+
+
+def own_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None, ws=None) -> bool:
+    """``linear`` where a kernel of ours takes the operands; False: nothing has been done."""
     if not _traced(x, w, out) and x.dim() == 2 and x.shape[0] <= MID_ROWS:
         if x.shape[0] <= FEW_ROWS:
             if _few(x, w, out) and out.dtype == torch.bfloat16 and out.shape[1] == w.shape[0]:
                 row_linear(x, w, out)
-                return out
+                return True
         elif ws is not None and _mid(x, w, out) and out.shape[1] == w.shape[0] and mid_linear(x, w, out, ws):
+            return True
+    return False
+
+
+WIDE_ROWS = 256  # rows of the library's widest weight tiles
+
+
+def pad_wide(w: torch.Tensor) -> torch.Tensor:
+    """w [n, K] with zero rows up to a multiple of WIDE_ROWS, for ``linear_wide``."""
+    pad = -w.shape[0] % WIDE_ROWS
+    return torch.cat([w, torch.zeros(pad, w.shape[1], dtype=w.dtype, device=w.device)], 0).contiguous() if pad else w
+
+
+def linear_wide(x: torch.Tensor, w: torch.Tensor, head: torch.Tensor, get, ws=None) -> torch.Tensor:
+    """x @ head.T, ``head`` the first rows of a weight ``w`` whose rows go on with zeros up to whole tiles of the library GEMM (``pad_wide``): it computes these
+    outputs too, since it is faster on whole tiles and rows of whole lines (2048 deep, us: 3664 / 3840 outputs at 1530 rows 31.7 /
+    28.0, at 8100 118 / 91; 17440 / 17664 at 300 33.1 / 29.0, at 1530 102 / 87, at 8100 471 / 464).  ``get(columns)``: the output
+    buffer.  Returns head's columns."""
+    n = head.shape[0]
+    if n < w.shape[0] and x.shape[0] <= MID_ROWS:
+        out = get(n)
+        if own_linear(x, head, out, ws):
             return out
-    return torch.matmul(x, w.t(), out=out)
+    return linear(x, w, get(w.shape[0]), ws)[:, :n]
 
 
 def linear_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:

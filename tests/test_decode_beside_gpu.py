@@ -267,3 +267,15 @@ def test_embedding_with_the_first_layer_norm(T, d):
     ops.embed_scale(ids, table, 8.0, y, src, prev)
     ops.residual_layer_norm(y, w=w, bias=b, eps=1e-6, out=want)
     assert torch.equal(x, y) and torch.equal(h, want)
+
+
+@pytest.mark.parametrize("M", [1, 16, 40, 256, 257, 700])
+def test_padded_weights_leave_the_same_columns(M):
+    n, K = 3664, 2048
+    x, w = rnd(M, K, seed=1).cuda(), rnd(n, K, scale=K ** -0.5, seed=2).cuda()
+    wide = ops.pad_wide(w)
+    assert wide.shape[0] == 3840 and torch.equal(wide[:n], w) and not wide[n:].any()
+    got = ops.linear_wide(x, wide, wide[:n], lambda c: torch.empty(M, c, dtype=B16, device="cuda"))
+    want = x.float() @ w.float().t()
+    assert got.shape == (M, n)
+    assert torch.allclose(got.float(), want, rtol=2 ** -7, atol=1e-3)
