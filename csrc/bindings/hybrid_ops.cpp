@@ -548,12 +548,30 @@ void row_linear(const Tensor& x, const Tensor& w, Tensor& out, bool relu2, bool 
 // two products of the same sizes; false: not one of its sizes
 bool row_linear_two(const Tensor& x0, const Tensor& w0, Tensor& out0, const Tensor& x1, const Tensor& w1, Tensor& out1) {
   const RowOperands a = row_operands(x0, w0, out0, false, false), b = row_operands(x1, w1, out1, false, false);
-  if (a.M != b.M || a.N != b.N || a.K != b.K) return false;
+  if (a.M != b.M || a.N != b.N || a.K != b.K || a.ldx != b.ldx || a.ldo != b.ldo) return false;
   const at::OptionalDeviceGuard g(x0.device());
-  const void *x[2] = {a.x, b.x}, *w[2] = {a.w, b.w};
-  void* out[2] = {a.out, b.out};
-  const long long ldx[2] = {a.ldx, b.ldx}, ldo[2] = {a.ldo, b.ldo};
-  return launch_row_linear_two(x, ldx, w, out, ldo, a.M, a.N, a.K, cur_stream(x0));
+  const auto apart = [](const void* p, const void* q) { return (long long)((intptr_t)q - (intptr_t)p); };
+  return launch_row_linear_many(a.x, a.ldx, apart(a.x, b.x), a.w, apart(a.w, b.w), a.out, a.ldo, apart(a.out, b.out), 2, a.M, a.N, a.K,
+                                cur_stream(x0));
+}
+
+// out[:, h] = x[:, h] . w[h]^T: x [M, H, K], w [H, N, K], out [M, H, N]; false: not one of its sizes or layouts
+bool row_linear_heads(const Tensor& x, const Tensor& w, Tensor& out) {
+  gpu(x, "x", false);
+  gpu(out, "out", false);
+  dtype(w, at::kBFloat16, "w");
+  TORCH_CHECK(x.dim() == 3 && w.dim() == 3 && out.dim() == 3 && x.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16,
+              "row_linear_heads: x [M, H, K], w [H, N, K], out [M, H, N] in bf16");
+  const int64_t M = x.size(0), H = x.size(1), K = x.size(2), N = out.size(2);
+  TORCH_CHECK(out.size(0) == M && out.size(1) == H && w.size(0) == H && w.size(1) == N && w.size(2) == K, "row_linear_heads: shapes");
+  const auto al = [](const Tensor& t, int to) { return (uintptr_t)t.data_ptr() % to == 0; };
+  if (M < 1 || M > 256 || H > 65535 || K < 8 || K % 8 || K > 1 << 16 || N < 4 || N % 4 || N > 1 << 20 || x.stride(2) != 1 ||
+      out.stride(2) != 1 || x.stride(1) % 8 || x.stride(0) % 8 || x.stride(0) < 0 || x.stride(0) > 1 << 24 || out.stride(0) % 4 ||
+      out.stride(1) % 4 || !al(x, 16) || !al(w, 16) || !al(out, 8))
+    return false;
+  const at::OptionalDeviceGuard g(x.device());
+  return launch_row_linear_many(x.data_ptr(), x.stride(0), 2 * x.stride(1), w.data_ptr(), 2 * N * K, out.data_ptr(), out.stride(0),
+                                2 * out.stride(1), (int)H, (int)M, (int)N, (int)K, cur_stream(x));
 }
 
 bool beside(const Tensor& x, const Tensor& w, Tensor& out, const RowRide& r) {
@@ -1470,6 +1488,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
   m.def("conv_state_update(Tensor xin, Tensor(a!) state, Tensor? cu_q, Tensor prev_row, Tensor save_slot, int runs) -> ()",
         &conv_state_update);
   m.def("row_linear(Tensor x, Tensor w, Tensor(a!) out, bool relu2, bool glu) -> ()", &row_linear);
+  m.def("row_linear_heads(Tensor x, Tensor w, Tensor(a!) out) -> bool", &row_linear_heads);
   m.def("row_linear_two(Tensor x0, Tensor w0, Tensor(a!) out0, Tensor x1, Tensor w1, Tensor(b!) out1) -> bool", &row_linear_two);
   m.def(
       "row_linear_rope(Tensor x, Tensor w, Tensor(a!) out, Tensor z, Tensor? bias, int H, int G, int dk, int dv, Tensor positions, "

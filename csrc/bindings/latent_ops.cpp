@@ -135,7 +135,7 @@ void layer_norm(const Tensor& x, const OptTensor& rows, const Tensor& w, double 
 
 void latent_prep(const Tensor& z, int64_t q_rank, int64_t kv_rank, int64_t rot, const OptTensor& wq, const OptTensor& wkv,
                  double eps, const Tensor& positions, const Tensor& slots, const Tensor& rope, const OptTensor& cq,
-                 const OptTensor& cache, int64_t half_dims) {
+                 const OptTensor& cache, int64_t half_dims, const OptTensor& q_src, const OptTensor& q_dst) {
   const int f32 = act(z, "z", false);
   TORCH_CHECK(q_rank >= 0 && (q_rank == 0 || (wq.has_value() && cq.has_value())), "latent_prep: the query latent needs wq and cq");
   if (q_rank > 0) {
@@ -175,6 +175,17 @@ void latent_prep(const Tensor& z, int64_t q_rank, int64_t kv_rank, int64_t rot, 
   a.slots = ptr<int>(slots);
   a.rope = ptr<float>(rope);
   a.cq = q_rank > 0 ? cq->data_ptr() : nullptr;
+  TORCH_CHECK(q_src.has_value() == q_dst.has_value(), "latent_prep: q_src and q_dst together");
+  if (q_src.has_value()) {
+    same_act(*q_src, f32, "q_src", false);
+    same_act(*q_dst, f32, "q_dst", false);
+    TORCH_CHECK(q_src->dim() == 3 && q_src->sizes() == q_dst->sizes() && q_src->size(0) == T && q_src->size(2) == rot &&
+                    q_src->stride(2) == 1 && q_dst->stride(2) == 1 && rope.dim() == 3 && rope.size(1) == rot / 2 && rope.size(2) == 2,
+                "latent_prep: q_src, q_dst [T, H, rot] views with unit inner stride");
+    a.q_src = q_src->data_ptr(), a.qs_t = q_src->stride(0), a.qs_h = q_src->stride(1);
+    a.q_dst = q_dst->data_ptr(), a.qd_t = q_dst->stride(0), a.qd_h = q_dst->stride(1);
+    a.H = (int)q_src->size(1);
+  }
   launch_latent_prep(a, (int)T, f32, cur_stream(z));
 }
 
@@ -354,7 +365,7 @@ TORCH_LIBRARY(symmetry_amd_latent, m) {
   m.def("layer_norm(Tensor x, Tensor? rows, Tensor w, float eps, Tensor(a!) out) -> ()", &layer_norm);
   m.def(
       "latent_prep(Tensor z, int q_rank, int kv_rank, int rot, Tensor? wq, Tensor? wkv, float eps, Tensor positions, "
-      "Tensor slots, Tensor rope, Tensor(a!)? cq, Tensor(b!)? cache, int half_dims) -> ()",
+      "Tensor slots, Tensor rope, Tensor(a!)? cq, Tensor(b!)? cache, int half_dims, Tensor? q_src=None, Tensor(c!)? q_dst=None) -> ()",
       &latent_prep);
   m.def("rope_pairs(Tensor src, Tensor(a!) dst, Tensor positions, Tensor rope, int half_dims) -> ()", &rope_pairs);
   m.def(

@@ -80,9 +80,9 @@ bool launch_mid_linear_f32(const void* x, long long ldx, const void* W, float* o
 // out = x . W^T (relu2: of relu(x)^2; glu: silu(gate) * up of W's [gate | up] rows); false: this K has no kernel
 bool launch_row_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int f32_out,
                        int relu2, int glu, hipStream_t s);
-// two products of the same sizes in one launch
-bool launch_row_linear_two(const void* const x[2], const long long ldx[2], const void* const W[2], void* const out[2], const long long ldo[2],
-                           int M, int N, int K, hipStream_t s);
+// `count` products of the same sizes and row strides in one launch, their operands dx, dw, dout bytes apart; any M
+bool launch_row_linear_many(const void* x, long long ldx, long long dx, const void* W, long long dw, void* out, long long ldo, long long dout,
+                            int count, int M, int N, int K, hipStream_t s);
 // out = relu(x)^2 . W^T, and beside it row work of other tensors: a convolution whose rows are runs of their own where conv.out is
 // set, else rope
 struct RowRide {

@@ -30,6 +30,7 @@
 // bf16 weights of a lane ARE its B operand of the second product (the 32 keys of a tile are consumed in the order
 // the accumulator layout hands them out, and the V^T fragment reads follow the same order), and the softmax
 // statistics of a query vector live in the 4 lanes that share its accumulator column.
+#include "attn_tiles.h"
 #include "common.h"
 #include "latent_launchers.h"
 
@@ -67,9 +68,30 @@ SYM_DEV float out_factor(const LatentAttnArgs& a, long long row, int h, float m,
 }
 
 template <typename T>
+SYM_DEV void rope_row(const T* __restrict__ src, long long s_t, long long s_h, T* __restrict__ dst, long long d_t, long long d_h,
+                      const int* __restrict__ positions, const float* __restrict__ rope, int H, int rot, int half_dims) {
+  const int row = blockIdx.x;
+  const float* cs = rope + (long long)positions[row] * rot;
+  const int half = rot / 2;
+  for (int i = threadIdx.x; i < H * half; i += NT) {
+    const int h = i / half, p = i - h * half;
+    int e0, e1;
+    pair_entries(p, half_dims, e0, e1);
+    const T* s = src + row * s_t + h * s_h;
+    T* o = dst + row * d_t + h * d_h;
+    const float u = (float)s[e0], v = (float)s[e1];
+    const float co = cs[2 * p], si = cs[2 * p + 1];
+    o[e0] = (T)(u * co - v * si);
+    o[e1] = (T)(v * co + u * si);
+  }
+}
+
+template <typename T>
 __global__ __launch_bounds__(NT) void latent_prep_kernel(LatentPrepArgs a) {
   __shared__ float scratch[NT / 64];
   const int row = blockIdx.x;
+  if (blockIdx.y)
+    return rope_row<T>((const T*)a.q_src, a.qs_t, a.qs_h, (T*)a.q_dst, a.qd_t, a.qd_h, a.positions, a.rope, a.H, a.rot, a.half_dims);
   const T* z = (const T*)a.z + (long long)row * a.nz;
   float ss = 0.f;
   if (a.q_rank > 0) {   // (launch-uniform)
@@ -112,20 +134,7 @@ __global__ __launch_bounds__(NT) void rope_pairs_kernel(const T* __restrict__ sr
                                                         const int* __restrict__ positions,
                                                         const float* __restrict__ rope, int H, int rot,
                                                         int half_dims) {
-  const int row = blockIdx.x;
-  const float* cs = rope + (long long)positions[row] * rot;
-  const int half = rot / 2;
-  for (int i = threadIdx.x; i < H * half; i += NT) {
-    const int h = i / half, p = i - h * half;
-    int e0, e1;
-    pair_entries(p, half_dims, e0, e1);
-    const T* s = src + row * s_t + h * s_h;
-    T* o = dst + row * d_t + h * d_h;
-    const float u = (float)s[e0], v = (float)s[e1];
-    const float co = cs[2 * p], si = cs[2 * p + 1];
-    o[e0] = (T)(u * co - v * si);
-    o[e1] = (T)(v * co + u * si);
-  }
+  rope_row<T>(src, s_t, s_h, dst, d_t, d_h, positions, rope, H, rot, half_dims);
 }
 
 // fp32 dot of a query held in LDS with one cache row (16-byte loads when the row length allows)
@@ -231,48 +240,86 @@ __global__ __launch_bounds__(64) void latent_attn_wave_kernel(LatentAttnArgs a) 
   }
 }
 
-// Combine the split-KV partials of one (row, head): four waves.  The per-partition weights exp(m_p - m) are computed
-// once (threads over partitions, kept in LDS); then wave w sums partitions w, w + 4, .. with every lane owning up to
-// 8 latent dims in registers (a partition's loads all in flight), and the four partial sums meet in LDS.
+// Combine the split-KV partials of one (row, head): four waves, wave w partitions w, w + 4, ..
+// Up to 64 partitions of a multiple of 4 dims, the rule: a wave's loads of 32 are all in flight before the first is used (the
+// statistics first: 16 rows of 16 heads and 10 partitions 11.2 us, so 5.0).  More: the weights exp(m_p - m) go through LDS.
 template <typename T>
 __global__ __launch_bounds__(256) void latent_attn_merge_kernel(LatentAttnArgs a) {
+  __shared__ __attribute__((aligned(16))) float red[4][512];
   __shared__ float wp[1024];
-  __shared__ float red[4][512];
   __shared__ float stat[8];
-  const int row = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int row = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const long long p0 = ((long long)row * a.H + h) * a.parts;
   // partitions that hold keys: the row's range starts at its window's first key (at 0 without a window)
   const int seen = a.window > 0 ? min(a.positions[row] + 1, a.window) : a.positions[row] + 1;
   const int np = min(a.parts, (seen + a.part_tokens - 1) / a.part_tokens);
-  float m = -INFINITY;
-  for (int p = tid; p < np; p += 256) m = fmaxf(m, a.part_ml[2 * (p0 + p)]);
-  m = wave_max(m);
-  if (lane == 0) stat[wave] = m;
-  __syncthreads();
-  m = fmaxf(fmaxf(stat[0], stat[1]), fmaxf(stat[2], stat[3]));
-  float l = 0.f;
-  for (int p = tid; p < np; p += 256) {
-    const float w = __expf(a.part_ml[2 * (p0 + p)] - m);
-    wp[p] = w;
-    l += a.part_ml[2 * (p0 + p) + 1] * w;
-  }
-  l = wave_sum(l);
-  if (lane == 0) stat[4 + wave] = l;
-  __syncthreads();
-  const float inv = out_factor<T>(a, row, h, m, stat[4] + stat[5] + stat[6] + stat[7]);
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int p = wave; p < np; p += 4) {
-    const float* po = a.part_o + (p0 + p) * a.kv_rank;
-    const float w = wp[p];
+  float m = -INFINITY, l = 0.f, inv;
+  if (np <= 64 && a.kv_rank % 4 == 0) {
+    const int c = 4 * lane, c2 = c + 256;
+    f32x4 x[8][2];
+    auto load = [&](int from) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int c = lane + 64 * i;
-      if (c < a.kv_rank) acc[i] += po[c] * w;
+      for (int i = 0; i < 8; ++i) {
+        x[i][0] = x[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (from + 4 * i < np) {
+          const float* po = a.part_o + (p0 + from + 4 * i) * a.kv_rank;
+          if (c < a.kv_rank) x[i][0] = *reinterpret_cast<const f32x4*>(po + c);
+          if (c2 < a.kv_rank) x[i][1] = *reinterpret_cast<const f32x4*>(po + c2);
+        }
+      }
+    };
+    load(wave);
+    float mp = -INFINITY, lp = 0.f;      // lane p: partition p's
+    if (lane < np) mp = a.part_ml[2 * (p0 + lane)], lp = a.part_ml[2 * (p0 + lane) + 1];
+    m = wave_max(mp);
+    const float w = lane < np ? __expf(mp - m) : 0.f;
+    l = wave_sum(lp * w);
+    inv = out_factor<T>(a, row, h, m, l);
+    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+    auto sum = [&](int from) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float wi = __shfl(w, from + 4 * i, 64);      // (past np: 0 times 0)
+        s0 += x[i][0] * wi;
+        s1 += x[i][1] * wi;
+      }
+    };
+    sum(wave);
+    if (np > 32) {
+      load(32 + wave);
+      sum(32 + wave);
     }
-  }
+    *reinterpret_cast<f32x4*>(red[wave] + c) = s0;
+    *reinterpret_cast<f32x4*>(red[wave] + c2) = s1;
+  } else {
+    for (int p = tid; p < np; p += 256) m = fmaxf(m, a.part_ml[2 * (p0 + p)]);
+    m = wave_max(m);
+    if (lane == 0) stat[wave] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(stat[0], stat[1]), fmaxf(stat[2], stat[3]));
+    for (int p = tid; p < np; p += 256) {
+      const float w = __expf(a.part_ml[2 * (p0 + p)] - m);
+      wp[p] = w;
+      l += a.part_ml[2 * (p0 + p) + 1] * w;
+    }
+    l = wave_sum(l);
+    if (lane == 0) stat[4 + wave] = l;
+    __syncthreads();
+    inv = out_factor<T>(a, row, h, m, stat[4] + stat[5] + stat[6] + stat[7]);
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int p = wave; p < np; p += 4) {
+      const float* po = a.part_o + (p0 + p) * a.kv_rank;
+      const float w = wp[p];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) red[wave][lane + 64 * i] = acc[i];
+      for (int i = 0; i < 8; ++i) {
+        const int c = lane + 64 * i;
+        if (c < a.kv_rank) acc[i] += po[c] * w;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) red[wave][lane + 64 * i] = acc[i];
+  }
   __syncthreads();
   T* out = (T*)a.out + ((long long)row * a.H + h) * a.kv_rank;
   for (int c = tid; c < a.kv_rank; c += 256) out[c] = (T)((red[0][c] + red[1][c] + red[2][c] + red[3][c]) * inv);
@@ -533,6 +580,267 @@ __global__ __launch_bounds__(64 * NW) void latent_attn_mfma_kernel(LatentAttnArg
   }
 }
 
+// ---- latent 512 + rotary 64 over cache blocks of 32 tokens or a larger power of two, without a window ------------------------------
+// A wave owns 16 query vectors and all 512 dims of their sum (128 accumulator registers beside 72 of queries), so nothing is exchanged
+// between the products.  A tile of 32 cache rows lies in LDS once, as it comes (direct loads, 16-byte chunks at c ^ spread(row), so that
+// neither the reads along rows, for the scores, nor the LDS transpose reads down them, for the sum, collide): staged through registers,
+// and a second time transposed in 2-byte stores, a tile cost more than its products.
+// Prompts: four waves, 64 rows of a head, two stages; the two workgroups of a CU cover each other's barriers (us: one prompt of 4000
+// tokens, 16 heads, 1282 -> 383, three of 510 100 -> 46, two of 200 33.7 -> 21.2; eight waves of two heads with three stages 385, 55, 28.8).
+// What bounds it is LDS: 68 KB read a wave and tile, twice the products' time.
+// Decode steps: four waves with a tile of their own each, 16 heads of one row; the waves meet in LDS (16 rows of 600 keys 14.8 -> 8.9,
+// 40 32 -> 17.9).
+constexpr int LAT_DK = 576, LAT_R = 512, LAT_ROW = 2 * LAT_DK, LAT_CH = LAT_ROW / 16, LAT_STAGE = KT * LAT_ROW;
+constexpr int LAT_PITCH = LAT_R + 4;      // floats of a head's sum where decode waves meet
+
+// the XOR on a row's chunks: the three bits above its lowest, turned round (two rows are 32 banks apart)
+SYM_DEV int lat_spread(int r) { return ((r >> 1 & 1) << 2) | (r >> 1 & 2) | (r >> 3 & 1); }
+
+struct LatTile {      // a lane's places in a tile
+  int k[2], v[4];     // bytes: key row n, chunk 4 s + g (of s's parity); value rows 4 g + n / 4, dims 16 dt .. (of dt mod 4)
+  SYM_DEV explicit LatTile(int lane) {
+    const int n = lane & 15, g = lane >> 4, sn = lat_spread(n), vr = 4 * g + (n >> 2), sv = lat_spread(vr);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) k[i] = n * LAT_ROW + 16 * ((4 * i + g) ^ sn);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = vr * LAT_ROW + 16 * ((2 * i + ((n & 3) >> 1)) ^ sv) + 8 * (n & 1);
+  }
+};
+
+typedef __attribute__((address_space(3))) const char* LdsPtr;      // (generic pointers: every read's address was computed apart)
+
+// one tile: S holds keys k0 ..; of them the lane's query vector sees those up to limit, and up to k_hi - 1.  edge: some vector of
+// the wave sees only a part
+SYM_DEV void lat_multiply(LdsPtr S, const LatTile& at, const bf16x8 (&qf)[18], f32x4 (&o)[32], float& m, float& l, float scale,
+                          int k0, int limit, int k_hi, bool edge, int g) {
+  const LdsPtr kp[2] = {S + at.k[0], S + at.k[1]}, vp[4] = {S + at.v[0], S + at.v[1], S + at.v[2], S + at.v[3]};
+  // Four operands are read ahead of the product at hand, the sum's first ones under the softmax (left to the compiler, with the
+  // registers nearly full, every read was waited for: 3.0 us a tile).
+  constexpr int AHEAD = 4;
+  bf16x8 f[AHEAD];
+  auto key = [&](int i) {      // scores: the operand's k step i / 2, keys 16 (i % 2) ..
+    return *(__attribute__((address_space(3))) const bf16x8*)(kp[i / 2 & 1] + 128 * (i / 4) + 16 * LAT_ROW * (i & 1));
+  };
+  auto turned = [](LdsPtr p) {
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p));
+  };
+  auto value = [&](int dt) {
+    const LdsPtr p = vp[dt & 3] + 128 * (dt >> 2);
+    const uint2 lo = turned(p), hi = turned(p + 16 * LAT_ROW);
+    Pack8 va;
+    va.u = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    return va.v;
+  };
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) f[i] = key(i);
+  f32x4 st[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int i = 0; i < 36; ++i) {
+    __builtin_amdgcn_sched_barrier(0);
+    st[i & 1] = mfma16(f[i % AHEAD], qf[i / 2], st[i & 1]);
+    f[i % AHEAD] = i + AHEAD < 36 ? key(i + AHEAD) : value(i + AHEAD - 36);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  float mx = -INFINITY;
+#pragma unroll
+  for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float v = st[sub][i] * scale;
+      if (edge) {
+        const int key = k0 + sub * 16 + g * 4 + i;
+        if (key > limit || key >= k_hi) v = -INFINITY;
+      }
+      st[sub][i] = v;
+      mx = fmaxf(mx, v);
+    }
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  // (deferred rescale, as below)
+  if (__any(mx > m + 8.f)) {
+    const float m_new = fmaxf(m, mx);
+    const float alpha = m_new == -INFINITY ? 1.f : __expf(m - m_new);
+    l *= alpha;
+#pragma unroll
+    for (int dt = 0; dt < 32; ++dt) o[dt] = o[dt] * alpha;
+    m = m_new;
+  }
+  float ps = 0.f;
+  Pack8 pb;
+#pragma unroll
+  for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float p = m == -INFINITY ? 0.f : __expf(st[sub][i] - m);
+      ps += p;
+      pb.h[sub * 4 + i] = (bf16)p;
+    }
+  ps += __shfl_xor(ps, 16, 64);
+  ps += __shfl_xor(ps, 32, 64);
+  l += ps;
+#pragma unroll
+  for (int dt = 0; dt < 32; ++dt) {
+    __builtin_amdgcn_sched_barrier(0);
+    o[dt] = mfma16(f[dt % AHEAD], pb.v, o[dt]);
+    if (dt + AHEAD < 32) f[dt % AHEAD] = value(dt + AHEAD);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Wave loads [first], [first + step], .. of a tile's 36, as many as COUNT (past the end: the last once more); keys past k_hi - 1 read
+// that one's row
+template <int COUNT>
+SYM_DEV void lat_stage(const LatentAttnArgs& a, const int* bt, int k0, int k_hi, unsigned int lds, int first, int step, int lane) {
+  // (a scalar load: a vector load's wait would be for the tiles in flight as well)
+  const int block = ((__attribute__((address_space(4))) const int*)(uintptr_t)bt)[k0 >> a.bs_shift];
+  const char* base = reinterpret_cast<const char*>(a.cache) + (((long long)block << a.bs_shift) + (k0 & (a.BS - 1))) * LAT_ROW;
+  const int last = k_hi - 1 - k0;
+  asm volatile("" : "+v"(lane));      // (the lane's places are formed anew: held over a tile they are registers that its products need)
+#pragma unroll COUNT < 10 ? COUNT : 4
+  for (int i = 0; i < COUNT; ++i) {
+    const int j = min(first + i * step, LAT_STAGE / 1024 - 1), at = 64 * j + lane, r = at / LAT_CH, c = (at - r * LAT_CH) ^ lat_spread(r);
+    direct_load16(base + min(r, last) * LAT_ROW + 16 * c, lds + 1024 * j);
+  }
+}
+
+__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(LatentAttnArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
+  const int seq = a.tiles[2 * blockIdx.y], off = a.tiles[2 * blockIdx.y + 1];
+  const int q0 = a.cu_q[seq], qlen = a.cu_q[seq + 1] - q0;
+  if (off >= qlen) return;      // padding tile
+  const int head = blockIdx.x, r16 = off + 16 * wave, rin = r16 + n;
+  const bool valid = rin < qlen;
+  const int qrow = q0 + min(rin, qlen - 1), limit = a.positions[qrow];
+  const int k_hi = a.positions[q0 + min(off + 63, qlen - 1)] + 1;      // a run's rows are consecutive positions
+  const int wave_hi = r16 < qlen ? a.positions[q0 + min(r16 + 15, qlen - 1)] + 1 : 0;
+  const int wave_lo = a.positions[q0 + min(r16, qlen - 1)] + 1;       // keys every query vector of the wave sees
+  const bf16* qp = reinterpret_cast<const bf16*>(a.q) + ((long long)qrow * a.H + head) * LAT_DK + 8 * g;
+  const int* bt = a.block_tables + (long long)seq * a.max_blocks;
+  const unsigned int lds0 = lds_address(smem);
+  const LatTile at(lane);
+  bf16x8 qf[18];
+#pragma unroll
+  for (int s = 0; s < 18; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qp + 32 * s);
+  f32x4 o[32];
+#pragma unroll
+  for (int i = 0; i < 32; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  constexpr int LOADS = LAT_STAGE / 1024 / 4;
+  static_assert(LAT_STAGE % 4096 == 0, "whole loads a wave");
+  auto stage = [&](int t) { lat_stage<LOADS>(a, bt, KT * t, k_hi, lds0 + (t & 1) * LAT_STAGE, wave, 4, lane); };
+  const int tiles = (k_hi + KT - 1) / KT;
+  stage(0);
+  for (int t = 0; t < tiles; ++t) {
+    // this wave's share of tile t has landed; behind the barrier everyone's has, and the stage of tile t - 1 has been read
+    __builtin_amdgcn_s_waitcnt(0x0070);      // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (t + 1 < tiles) stage(t + 1);
+    const int k0 = KT * t;
+    if (k0 < wave_hi)
+      lat_multiply((LdsPtr)smem + (t & 1) * LAT_STAGE, at, qf, o, m, l, a.scale, k0, limit, k_hi, k0 + KT > wave_lo, g);
+    asm volatile("" ::: "memory");
+  }
+  if (!valid) return;
+  bf16* out = reinterpret_cast<bf16*>(a.out) + ((long long)qrow * a.H + head) * LAT_R + 4 * g;
+  const float inv = out_factor<bf16>(a, qrow, head, m, l);
+#pragma unroll
+  for (int dt = 0; dt < 32; ++dt) {
+    bf16x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = (bf16)(o[dt][i] * inv);
+    *reinterpret_cast<bf16x4*>(out + 16 * dt) = v;
+  }
+}
+
+__global__ __launch_bounds__(256, 2) void latent_row_kernel(LatentAttnArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 15, g = lane >> 4;
+  const int row = blockIdx.x, part = blockIdx.z, h0 = 16 * blockIdx.y, limit = a.positions[row];
+  const int k_lo = a.parts > 1 ? part * a.part_tokens : 0, k_hi = a.parts > 1 ? min(limit + 1, k_lo + a.part_tokens) : limit + 1;
+  if (k_lo >= k_hi) return;      // a partition past this row's keys: the merge never reads it
+  const bf16* qp = reinterpret_cast<const bf16*>(a.q) + ((long long)row * a.H + min(h0 + n, a.H - 1)) * LAT_DK + 8 * g;
+  const int* bt = a.block_tables + (long long)a.row_seq[row] * a.max_blocks;
+  const unsigned int lds = lds_address(smem) + wave * LAT_STAGE;
+  const LatTile at(lane);
+  int k0 = k_lo + KT * wave;
+  if (k0 < k_hi) lat_stage<LAT_STAGE / 1024>(a, bt, k0, k_hi, lds, 0, 1, lane);
+  bf16x8 qf[18];
+#pragma unroll
+  for (int s = 0; s < 18; ++s) qf[s] = *reinterpret_cast<const bf16x8*>(qp + 32 * s);
+  f32x4 o[32];
+#pragma unroll
+  for (int i = 0; i < 32; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  for (; k0 < k_hi; k0 += 4 * KT) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    lat_multiply((LdsPtr)smem + wave * LAT_STAGE, at, qf, o, m, l, a.scale, k0, limit, k_hi, k0 + KT > k_hi, g);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the tile has been read)
+    if (k0 + 4 * KT < k_hi) lat_stage<LAT_STAGE / 1024>(a, bt, k0 + 4 * KT, k_hi, lds, 0, 1, lane);
+  }
+  // the waves meet: [4][16][LAT_PITCH] sums, [4][16] maxima and sums of weights
+  __syncthreads();
+  float* so = reinterpret_cast<float*>(smem);
+  float *sm = so + 4 * 16 * LAT_PITCH, *sl = sm + 64;
+#pragma unroll
+  for (int dt = 0; dt < 32; ++dt) *reinterpret_cast<f32x4*>(so + (16 * wave + n) * LAT_PITCH + 16 * dt + 4 * g) = o[dt];
+  if (g == 0) sm[16 * wave + n] = m, sl[16 * wave + n] = l;
+  __syncthreads();
+  // a thread: one head, 4 of every 64 dims
+  const int q = threadIdx.x >> 4, c = 4 * (threadIdx.x & 15), head = h0 + q;
+  if (head >= a.H) return;
+  const float M = fmaxf(fmaxf(sm[q], sm[16 + q]), fmaxf(sm[32 + q], sm[48 + q]));      // (a wave has keys: finite)
+  float f[4], L = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    f[w] = __expf(sm[16 * w + q] - M);      // a wave without keys: 0
+    L += f[w] * sl[16 * w + q];
+  }
+  const long long pi = ((long long)row * a.H + head) * a.parts + part;
+  const float inv = a.parts == 1 ? out_factor<bf16>(a, row, head, M, L) : 1.f;
+#pragma unroll
+  for (int i = 0; i < LAT_R / 64; ++i) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) v += f[w] * *reinterpret_cast<const f32x4*>(so + (16 * w + q) * LAT_PITCH + 64 * i + c);
+    if (a.parts > 1) {
+      *reinterpret_cast<f32x4*>(a.part_o + pi * LAT_R + 64 * i + c) = v;
+    } else {
+      bf16x4 b;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[j] = (bf16)(v[j] * inv);
+      *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16*>(a.out) + ((long long)row * a.H + head) * LAT_R + 64 * i + c) = b;
+    }
+  }
+  if (a.parts > 1 && c == 0) {
+    a.part_ml[2 * pi] = M;
+    a.part_ml[2 * pi + 1] = L;
+  }
+}
+
+constexpr int LAT_ROW_LDS = 4 * LAT_STAGE > 4 * (4 * 16 * LAT_PITCH + 128) ? 4 * LAT_STAGE : 4 * (4 * 16 * LAT_PITCH + 128);
+
+bool lat_dispatch(const LatentAttnArgs& a, hipStream_t s) {
+  const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  if (a.Dk != LAT_DK || a.kv_rank != LAT_R || a.window > 0 || a.bs_shift < 5 || !al(a.cache) || !al(a.q) || !al(a.out) || !al(a.part_o))
+    return false;
+  static const bool raised = [] {
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_prompt_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_row_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    return true;
+  }();
+  (void)raised;
+  if (a.tiles) {
+    if (a.ntiles > 65535) return false;
+    latent_prompt_kernel<<<dim3(a.H, a.ntiles), 256, 2 * LAT_STAGE, s>>>(a);
+  } else {
+    if (a.part_tokens % KT || a.parts > 65535) return false;
+    latent_row_kernel<<<dim3(a.T, (a.H + 15) / 16, a.parts), 256, LAT_ROW_LDS, s>>>(a);
+  }
+  return true;
+}
+
 template <int NKM, int RTM, bool DECODE, int NW, int DSPLIT, bool EXACT>
 void mfma_launch_one(const LatentAttnArgs& a, dim3 grid, hipStream_t s) {
   const size_t lds = 2 * ((size_t)KT * (a.Dk + 8) + (size_t)a.kv_rank * LDV) * sizeof(bf16) +  // two stages
@@ -567,6 +875,7 @@ void mfma_launch(const LatentAttnArgs& a, hipStream_t s) {
 bool mfma_dispatch(const LatentAttnArgs& a, hipStream_t s) {
   const int nk = a.Dk / 32, rt = a.kv_rank / 16;
   if (a.Dk % 32 || a.kv_rank % 16 || nk > 18 || rt > 32 || a.part_tokens % KT) return false;
+  if (lat_dispatch(a, s)) return true;
   if (nk == 18 && rt == 32) mfma_launch<18, 32, true>(a, s);       // latent 512 + rotary 64
   else mfma_launch<18, 32, false>(a, s);                           // every other tiled shape
   return true;
@@ -588,8 +897,9 @@ void attn_dispatch(const LatentAttnArgs& a, hipStream_t s) {
 
 void launch_latent_prep(const LatentPrepArgs& a, int T, int f32, hipStream_t s) {
   if (T <= 0) return;
-  if (f32) latent_prep_kernel<float><<<T, NT, 0, s>>>(a);
-  else latent_prep_kernel<bf16><<<T, NT, 0, s>>>(a);
+  const dim3 grid(T, a.q_dst ? 2 : 1);
+  if (f32) latent_prep_kernel<float><<<grid, NT, 0, s>>>(a);
+  else latent_prep_kernel<bf16><<<grid, NT, 0, s>>>(a);
 }
 
 void launch_rope_pairs(const void* src, long long s_t, long long s_h, void* dst, long long d_t, long long d_h,

@@ -39,6 +39,10 @@ struct LatentPrepArgs {
   const float* rope;    // [max_pos][rot / 2][2] cos, sin
   void* cq;             // [T][q_rank]
   void* cache;          // [rows][kv_rank + rot]
+  // or null: the rotary of q_src[t][h][0..rot) -> q_dst as well (element strides; by workgroups of their own)
+  const void* q_src; long long qs_t, qs_h;
+  void* q_dst; long long qd_t, qd_h;
+  int H;
 };
 void launch_latent_prep(const LatentPrepArgs& a, int T, int f32, hipStream_t s);
 // rotary of src[t][h][0..rot) -> dst[t][h][0..rot) (element strides given); half_dims as in LatentPrepArgs

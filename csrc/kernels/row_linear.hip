@@ -27,10 +27,21 @@ struct Args {
   long long ldo;
   int M, N, K;  // EPI_GLU: N outputs, W has 2 N rows
 };
-// a launch's problems (blockIdx.y), of the same sizes
+// a launch's problems (blockIdx.y), of the same sizes and strides, these many bytes apart; rows past 16 by blockIdx.z
 struct Problems {
-  Args p[2];
+  Args a;
+  long long dx, dw, dout;
 };
+template <int EPI>
+SYM_DEV Args problem(const Problems& ps) {
+  Args a = ps.a;
+  const int y = blockIdx.y, z = blockIdx.z;
+  a.x = reinterpret_cast<const bf16*>(reinterpret_cast<const char*>(a.x) + y * ps.dx) + 16 * z * a.ldx;
+  a.W = reinterpret_cast<const bf16*>(reinterpret_cast<const char*>(a.W) + y * ps.dw);
+  a.out = reinterpret_cast<char*>(a.out) + y * ps.dout + 16 * z * a.ldo * (EPI == EPI_F32 ? 4 : 2);
+  a.M = min(16, a.M - 16 * z);
+  return a;
+}
 
 SYM_DEV void relu_squared(Pack8& x) {
 #pragma unroll
@@ -91,7 +102,7 @@ SYM_DEV void ride(const RowRide& r, int wg, int threads) {
 
 template <int RT, int RH, int NW, int EPI, bool XF, bool M8 = false, typename More = Nothing>
 __global__ __launch_bounds__(NW * 64) void row_linear_kernel(Problems ps, More more) {
-  const Args& a = ps.p[blockIdx.y];
+  const Args a = problem<EPI>(ps);
   if constexpr (std::is_same<More, RowRide>::value) {
     constexpr int out = EPI == EPI_GLU ? RH : RH * RT;
     const int tiles = (a.N + out - 1) / out;
@@ -303,7 +314,8 @@ __global__ __launch_bounds__(NW * 64) void row_linear_walk_kernel(Args a) {
 constexpr int SMALL_K = 256;
 
 template <int EPI, bool XF>
-__global__ __launch_bounds__(64) void row_linear_small_kernel(Args a) {
+__global__ __launch_bounds__(64) void row_linear_small_kernel(Problems ps) {
+  const Args a = problem<EPI>(ps);
   constexpr int RT = EPI == EPI_GLU ? 2 : 1;
   const int lane = threadIdx.x, r16 = lane & 15, h = lane >> 4, n0 = blockIdx.x * 16;
   const bf16* wr = a.W + (long long)min(n0 + r16, a.N - 1) * a.K + 8 * h;
@@ -326,16 +338,18 @@ __global__ __launch_bounds__(64) void row_linear_small_kernel(Args a) {
   store_rows<16, EPI>(a, n0, lane, acc[0], acc[RT - 1]);
 }
 
-// what a launch does: its problem, and a second one of the same sizes or work beside it, or null
+// what a launch does: its problems, how many, and work beside them or null
 struct Job {
-  const Args &a, *second;
+  const Problems& ps;
+  int count;
   const RowRide* beside;
-  bool plain() const { return !second && !beside; }
+  bool plain() const { return count == 1 && !beside && ps.a.M <= 16; }
+  dim3 grid(int tiles) const { return dim3(tiles, count, (ps.a.M + 15) / 16); }
 };
 
 template <int NW, int KB, int EPI, bool XF>
 bool walk(const Job& j, hipStream_t s) {
-  const Args& a = j.a;
+  const Args& a = j.ps.a;
   if (a.K != 64 * NW * KB || !j.plain()) return false;
   constexpr int OUT = EPI == EPI_GLU ? 8 : 16;
   const int tiles = (a.N + OUT - 1) / OUT;
@@ -345,20 +359,19 @@ bool walk(const Job& j, hipStream_t s) {
 
 template <int RT, int RH, int NW, int EPI, bool XF, bool M8>
 bool run(const Job& j, hipStream_t s) {
-  const Args& a = j.a;
+  const Args& a = j.ps.a;
   if (a.K % ((RH == 16 ? 128 : 256) * NW)) return false;
   constexpr int rows = EPI == EPI_GLU ? RH : RH * RT;
   const int tiles = (a.N + rows - 1) / rows;
-  const Problems ps{{a, j.second ? *j.second : a}};
   if (!j.beside) {
-    row_linear_kernel<RT, RH, NW, EPI, XF, M8><<<dim3(tiles, j.second ? 2 : 1), NW * 64, 0, s>>>(ps, Nothing{});
+    row_linear_kernel<RT, RH, NW, EPI, XF, M8><<<j.grid(tiles), NW * 64, 0, s>>>(j.ps, Nothing{});
     return true;
   }
   if constexpr (EPI == EPI_BF16 && XF) {
     if (j.beside) {
       RowRide r = *j.beside;
       r.per_row = r.conv.out ? (r.conv.C + NW * 64 - 1) / (NW * 64) : 2;
-      row_linear_kernel<RT, RH, NW, EPI, XF, M8, RowRide><<<tiles + r.per_row * r.rows, NW * 64, 0, s>>>(ps, r);
+      row_linear_kernel<RT, RH, NW, EPI, XF, M8, RowRide><<<tiles + r.per_row * r.rows, NW * 64, 0, s>>>(j.ps, r);
       return true;
     }
   }
@@ -411,10 +424,10 @@ bool run_waves(const Job& j, int waves, hipStream_t s) {
 // few outputs for more than 8 rows (512 x 4096 at 1, 16 rows 8.6, 10.7 / 9.4, 9.5).
 template <int EPI, bool XF>
 bool by_shape(const Job& j, hipStream_t s) {
-  const Args& a = j.a;
+  const Args& a = j.ps.a;
   if (a.K <= SMALL_K) {
-    if (!j.plain()) return false;
-    row_linear_small_kernel<EPI, XF><<<(a.N + 15) / 16, 64, 0, s>>>(a);
+    if (j.beside) return false;
+    row_linear_small_kernel<EPI, XF><<<j.grid((a.N + 15) / 16), 64, 0, s>>>(j.ps);
     return true;
   }
   const int tiles = (a.N + 15) / 16, blocks = a.K / 128;
@@ -461,21 +474,20 @@ bool by_shape(const Job& j, hipStream_t s) {
 
 bool launch_row_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int f32_out,
                        int relu2, int glu, hipStream_t s) {
-  const Args a{(const bf16*)x, ldx, (const bf16*)W, out, ldo, M, N, K};
-  const Job j{a, nullptr, nullptr};
+  const Problems ps{{(const bf16*)x, ldx, (const bf16*)W, out, ldo, M, N, K}, 0, 0, 0};
+  const Job j{ps, 1, nullptr};
   return glu ? by_shape<EPI_GLU, false>(j, s) : f32_out ? by_shape<EPI_F32, false>(j, s)
          : relu2 ? by_shape<EPI_BF16, true>(j, s) : by_shape<EPI_BF16, false>(j, s);
 }
 
-bool launch_row_linear_two(const void* const x[2], const long long ldx[2], const void* const W[2], void* const out[2], const long long ldo[2],
-                           int M, int N, int K, hipStream_t s) {
-  const Args a{(const bf16*)x[0], ldx[0], (const bf16*)W[0], out[0], ldo[0], M, N, K};
-  const Args b{(const bf16*)x[1], ldx[1], (const bf16*)W[1], out[1], ldo[1], M, N, K};
-  return by_shape<EPI_BF16, false>(Job{a, &b, nullptr}, s);
+bool launch_row_linear_many(const void* x, long long ldx, long long dx, const void* W, long long dw, void* out, long long ldo, long long dout,
+                            int count, int M, int N, int K, hipStream_t s) {
+  const Problems ps{{(const bf16*)x, ldx, (const bf16*)W, out, ldo, M, N, K}, dx, dw, dout};
+  return by_shape<EPI_BF16, false>(Job{ps, count, nullptr}, s);
 }
 
 bool launch_row_linear_beside(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, const RowRide& r,
                               hipStream_t s) {
-  const Args a{(const bf16*)x, ldx, (const bf16*)W, out, ldo, M, N, K};
-  return by_shape<EPI_BF16, true>(Job{a, nullptr, &r}, s);
+  const Problems ps{{(const bf16*)x, ldx, (const bf16*)W, out, ldo, M, N, K}, 0, 0, 0};
+  return by_shape<EPI_BF16, true>(Job{ps, 1, &r}, s);
 }

@@ -155,7 +155,7 @@ def build_latent(verbose: bool = False, force: bool = False) -> str:
     (``torch.ops.symmetry_amd_latent``)."""
     os.makedirs(OBJ, exist_ok=True)
     kdir = os.path.join(CSRC, "kernels")
-    headers = [os.path.join(kdir, "common.h"), os.path.join(kdir, "latent_launchers.h")]
+    headers = [os.path.join(kdir, h) for h in ("common.h", "attn_tiles.h", "direct_lds.h", "latent_launchers.h")]
     tinc, tlib, abi = _torch_paths()
     jobs, objs = [], []
     for name in LATENT_KERNELS:

@@ -30,7 +30,8 @@ launches per layer run: GEMM (the mixer's projections), then
     delta:   GEMM W_b | W_a (fp32; channel decays: W_b, W_a2), conv_silu_qkv (+ conv_state_update in prompt steps; in
              decode steps W_b | W_a ride along in this launch), delta_rule, (GEMM W_g2,) gated_group_norm, GEMM W_o; in decode
              steps of the sizes it is written for, delta_token does everything up to W_o
-    latent:  latent_prep, bmm (absorb W_uk), rope_pairs, latent_attn (sink, gate), bmm (W_uv), GEMM W_o
+    latent:  latent_prep (with the queries' rotary), a product a head (absorb W_uk), latent_attn (sink, gate), a product a head (W_uv),
+             GEMM W_o
     residual_layer_norm; GEMM gate|up, silu_mul, GEMM down; residual_layer_norm (+ e in front of a loop's next pass)
 All intermediates live in the preallocated Workspace, so decode steps are hipGraph-capturable.
 
@@ -152,7 +153,8 @@ class BeletarLM:
                 fz.add(nm, t("mix." + nm))
             P["gkv"], P["sink"] = t("mix.dkv.norm"), f("mix.sink")
             P["uk"] = t("mix.uk").view(m.heads, m.dim, m.kv_rank)                                   # [H, dn, r]
-            P["uv"] = t("mix.uv").view(m.heads, m.vdim, m.kv_rank).transpose(1, 2).contiguous()     # [H, r, dv]
+            P["uv_t"] = t("mix.uv").view(m.heads, m.vdim, m.kv_rank).contiguous()                   # [H, dv, r]
+            P["uk_t"], P["uv"] = P["uk"].transpose(1, 2).contiguous(), P["uv_t"].transpose(1, 2).contiguous()
             P["rope"] = self._rope_table(m, max_pos)
         else:
             fz.add("qkv", torch.cat([t("mix.q"), t("mix.k"), t("mix.v")], 0))
@@ -239,16 +241,16 @@ class BeletarLM:
         T, H, r, rot, dn = h.shape[0], m.heads, m.kv_rank, m.rot_dim, m.dim
         plane = cache.lat[n]
         z = self._fused(h, P)
-        ops.latent_prep(self._cols(z, P, "dkv"), 0, r, rot, None, P["gkv"], self.cfg.norm_eps, b.positions, b.slot_mapping,
-                        P["rope"], None, plane)
         q = self._cols(z, P, "q").unflatten(1, (H, dn + rot))
         qa = self._buf("lat.qa", (T, H, r + rot))
-        torch.bmm(q[:, :, :dn].transpose(0, 1), P["uk"], out=qa[:, :, :r].transpose(0, 1))
-        ops.rope_pairs(q[:, :, dn:], qa[:, :, r:], b.positions, P["rope"])
+        ops.latent_prep(self._cols(z, P, "dkv"), 0, r, rot, None, P["gkv"], self.cfg.norm_eps, b.positions, b.slot_mapping,
+                        P["rope"], None, plane, q_rot=(q[:, :, dn:], qa[:, :, r:]))
+        ops.linear_heads(q[:, :, :dn], P["uk"], P["uk_t"], qa[:, :, :r])
         olat = self._buf("lat.o", (T, H, r))
         part_o = part_ml = None
         if b.kind == "decode" and self.device.type != "cpu":
-            parts = ops.latent_attn_parts(T, b.block_tables.shape[1] * cache.block_size)
+            # (many rows: partitions of a whole step of the kernel's waves; 64 of 300 keys 18.8 / 13.9 us, 3 of 617 8.9 / 10.2)
+            parts = ops.latent_attn_parts(T, b.block_tables.shape[1] * cache.block_size, min_tokens=128 if T >= 16 else 64)
             if parts > 1:
                 part_o = self._buf("lat.part_o", (T, H, parts, r), torch.float32)
                 part_ml = self._buf("lat.part_ml", (T, H, parts, 2), torch.float32)
@@ -256,7 +258,7 @@ class BeletarLM:
         ops.latent_attn(qa, plane, b.block_tables, b.row_seq, b.positions, m.scale, r, olat, part_o, part_ml,
                         b.tiles if tiled else None, b.cu_q if tiled else None, sink=P["sink"], gate=self._cols(z, P, "g"))
         ov = self._buf("lat.ov", (T, H * m.vdim))
-        torch.bmm(olat.transpose(0, 1), P["uv"], out=ov.view(T, H, m.vdim).transpose(0, 1))
+        ops.linear_heads(olat, P["uv"], P["uv_t"], ov.view(T, H, m.vdim))
         return self._linear("mix.out", ov, P["o"])
 
     def _ff(self, P: dict, h: torch.Tensor) -> torch.Tensor:

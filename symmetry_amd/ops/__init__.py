@@ -705,6 +705,19 @@ def row_linear_conv(x, w, out, xin, cw, cb, state, prev_row, save_slot, cout) ->
     return _gpu(x) and _hyb().row_linear_conv(x, w, out, xin, cw, cb, state, prev_row, save_slot, cout)
 
 
+HEAD_ROWS = 64      # rows up to which a product a head is row_linear_heads
+
+
+def linear_heads(x, w, wt, out) -> None:
+    """out[:, h] = x[:, h] @ w[h] for x [M, H, K], w [H, K, N], out [M, H, N] (views of wider rows); ``wt`` [H, N, K]: the same weight
+    transposed, or None.  With it bf16 of up to HEAD_ROWS rows are the few-row kernel's, a head a row of workgroups (16 heads of
+    512 -> 128 at 16 rows: the library's batched product 9.7 us, 16 workgroups), else that batched product."""
+    if (wt is not None and _gpu(x) and x.dtype == torch.bfloat16 and x.shape[0] <= HEAD_ROWS and not _traced(x, wt, out)
+            and not torch.is_grad_enabled() and torch.autograd.forward_ad._current_level < 0 and _hyb().row_linear_heads(x, wt, out)):
+        return
+    torch.bmm(x.transpose(0, 1), w, out=out.transpose(0, 1))
+
+
 def linear_two(x0, w0, out0, x1, w1, out1, ws=None) -> None:
     """``linear`` twice, in one launch where few-row operands have the same sizes (two of 2048 x 2048 at 8 rows: 9.4 us apart)."""
     if few_rows(x0, w0, out0) and few_rows(x1, w1, out1) and out0.dtype == out1.dtype == torch.bfloat16:
@@ -893,15 +906,18 @@ def rope_table(max_pos: int, dims: int, base: float, scaling: dict | None = None
     return reference.rope_table(max_pos, dims, base, scaling)
 
 
-def latent_prep(z, q_rank, kv_rank, rot, wq, wkv, eps, positions, slots, rope, cq, cache, half_dims=0):
+def latent_prep(z, q_rank, kv_rank, rot, wq, wkv, eps, positions, slots, rope, cq, cache, half_dims=0, q_rot=None):
     """z [T, q_rank (+ kv_rank + rot)] (a view: further columns may follow in its rows) -> cq = rms_norm(z[:, :q_rank]) *
     wq; with a kv part (kv_rank > 0) the token's cache row (slot >= 0) becomes [rms_norm(z kv part) * wkv | rotary(z rot
     part)].  ``half_dims`` = 0: rotary pairs (2i, 2i + 1); > 0: the half layout, entry i < half_dims / 2 paired with
-    i + half_dims / 2 and the entries past half_dims passing.  ``q_rank`` = 0: no query latent (wq and cq None)."""
+    i + half_dims / 2 and the entries past half_dims passing.  ``q_rank`` = 0: no query latent (wq and cq None).
+    ``q_rot`` = (src, dst): rope_pairs of the queries in the same launch."""
     if _gpu(z):
         return _lat().latent_prep(z, int(q_rank), int(kv_rank), int(rot), wq, wkv, float(eps), positions, slots, rope,
-                                  cq, cache, int(half_dims))
-    return reference.latent_prep(z, q_rank, kv_rank, rot, wq, wkv, eps, positions, slots, rope, cq, cache, half_dims)
+                                  cq, cache, int(half_dims), *(q_rot or ()))
+    reference.latent_prep(z, q_rank, kv_rank, rot, wq, wkv, eps, positions, slots, rope, cq, cache, half_dims)
+    if q_rot is not None:
+        reference.rope_pairs(*q_rot, positions, rope, half_dims)
 
 
 def rope_pairs(src, dst, positions, rope, half_dims=0):

@@ -279,3 +279,34 @@ def test_padded_weights_leave_the_same_columns(M):
     want = x.float() @ w.float().t()
     assert got.shape == (M, n)
     assert torch.allclose(got.float(), want, rtol=2 ** -7, atol=1e-3)
+
+
+@pytest.mark.parametrize("M,H,N,K", [(1, 16, 512, 128), (16, 16, 128, 512), (9, 3, 100, 1024), (17, 16, 128, 512), (64, 5, 512, 128),
+                                     (40, 2, 4096, 2048), (65, 4, 128, 512), (3, 2, 64, 24)])
+def test_products_a_head(M, H, N, K):
+    wide = rnd(M, H, K + 64, seed=1).cuda()
+    x, w = wide[:, :, :K], rnd(H, N, K, scale=K ** -0.5, seed=2).cuda()
+    out = torch.zeros(M, H, N + 64, dtype=B16, device="cuda")
+    with torch.no_grad():
+        ops.linear_heads(x, w.transpose(1, 2).contiguous(), w, out[:, :, :N])
+    want = torch.einsum("mhk,hnk->mhn", x.float().cpu(), w.float().cpu())
+    assert torch.allclose(out[:, :, :N].float().cpu(), want, rtol=2 ** -7, atol=1e-3)
+    assert not out[:, :, N:].any()
+
+
+@pytest.mark.parametrize("T", [1, 40])
+def test_latent_prep_turns_the_queries(T):
+    H, r, rot = 5, 512, 64
+    z, q = rnd(T, r + rot + 8, seed=1).cuda()[:, :r + rot], rnd(T, H, 200, seed=2).cuda()
+    pos, slot = torch.arange(T, dtype=I32).cuda() + 3, torch.arange(T, dtype=I32).cuda()
+    rope, w = rnd(64, rot // 2, 2, dtype=F32, seed=3).cuda(), rnd(r, seed=4).cuda()
+    got = []
+    for side in range(2):
+        plane, dst = torch.zeros(2, 64, r + rot, dtype=B16, device="cuda"), torch.zeros(T, H, r + rot, dtype=B16, device="cuda")
+        if side:
+            ops.latent_prep(z, 0, r, rot, None, w, 1e-6, pos, slot, rope, None, plane, q_rot=(q[:, :, 136:], dst[:, :, r:]))
+        else:
+            ops.latent_prep(z, 0, r, rot, None, w, 1e-6, pos, slot, rope, None, plane)
+            ops.rope_pairs(q[:, :, 136:], dst[:, :, r:], pos, rope)
+        got.append((plane, dst))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
