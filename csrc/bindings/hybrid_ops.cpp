@@ -369,12 +369,25 @@ DecayScanArgs scan_args(int64_t mode, const Tensor& q, const Tensor& k, const Te
   return a;
 }
 
+int64_t decay_scratch(int64_t mode, int64_t T, int64_t runs, int64_t H, int64_t N, int64_t P) {
+  TORCH_CHECK(mode >= 0 && mode <= 2 && T >= 0 && runs >= 0 && H > 0 && N >= 1 && N <= 256 && P >= 1, "decay_scratch: sizes");
+  return std::max<int64_t>(mode == 0 ? T * H * (32 + 2 * N) : 0, decay_chunk_scratch((int)mode, T, runs, H, (int)N));
+}
+
 void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dz, const Tensor& dbias,
                 const OptTensor& rate, double tau, const OptTensor& skip, double q_scale, int64_t H, int64_t N, int64_t P,
                 int64_t hpg, Tensor& state, const OptTensor& cu_q, const Tensor& prev_row, const Tensor& save_slot,
                 int64_t runs, Tensor& out, const OptTensor& mout, const OptTensor& tiles, const OptTensor& ws) {
-  const DecayScanArgs a = scan_args(mode, q, k, v, dz, dbias, rate, tau, skip, q_scale, H, N, P, hpg, state, cu_q, prev_row, save_slot,
-                                    runs, out, std::nullopt, mout, tiles, ws);
+  DecayScanArgs a = scan_args(mode, q, k, v, dz, dbias, rate, tau, skip, q_scale, H, N, P, hpg, state, cu_q, prev_row, save_slot,
+                              runs, out, std::nullopt, mout, tiles, ws);
+  Tensor own;      // (a scratch of 32 + 2 N floats a row and head is taken, and is not enough)
+  if (a.ws && v.scalar_type() != at::kFloat && decay_chunk_takes(a)) {
+    const int64_t need = decay_chunk_scratch(a.mode, a.T, a.runs, a.H, a.N);
+    if (ws->numel() < need) {
+      own = at::empty({need}, ws->options());
+      a.ws = ptr<float>(own);
+    }
+  }
   launch_decay_scan(a, v.scalar_type() == at::kFloat, cur_stream(v));
 }
 
@@ -1473,6 +1486,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
       "int keep_first, Tensor? sink, float softcap=0., Tensor? key_scale=None, Tensor(b!)? part_o=None, "
       "Tensor(c!)? part_ml=None, Tensor(d!)? counters=None, int part_keys=0) -> int",
       &window_attn);
+  m.def("decay_scratch(int mode, int T, int runs, int H, int N, int P) -> int", &decay_scratch);
   m.def(
       "decay_scan(int mode, Tensor q, Tensor k, Tensor v, Tensor dz, Tensor dbias, Tensor? rate, float tau, Tensor? skip, "
       "float q_scale, int H, int N, int P, int hpg, Tensor(a!) state, Tensor? cu_q, Tensor prev_row, Tensor save_slot, "

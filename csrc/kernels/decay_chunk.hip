@@ -24,6 +24,7 @@
 #include "attn_tiles.h"
 #include "bf16_parts.h"
 #include "hybrid_launchers.h"
+#include "walk_places.h"
 
 #include <algorithm>
 
@@ -66,8 +67,19 @@ SYM_DEV double prefix32(double v, int lane) {
   return lane < 16 ? v : v + __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// mode 0's scratch per (row, head): row of A | 2^(G_i) | k_i 2^(G_C - G_i)
-__host__ __device__ inline int ws_cols(int N) { return C + 2 * N; }
+// mode 0's scratch, a block per chunk and head: the bf16 parts of q_i 2^(G_i) | those of k_i 2^(G_C - G_i), each 3 [C][NP] | A fp32
+// [C][C] | 2^(G_C) fp32 [NP], as the walk keeps it in LDS: 16-byte pieces of a row are exchanged by its number (row_turn, score_turn), so that
+// reads along the rows and LDS transpose reads meet no bank twice; rows and channels past the end are 0.  Bytes, in whole KB.  The parts
+// are formed here once, not by every slab's workgroup in the walk, which only copies (8 heads x 128 x 256, walk, us: 8 runs of 612 to
+// 1546 tokens 195 -> 178, one of 7900 870 -> 782; the launch that forms them stays at 81).
+constexpr int chunk_block(int NP) { return (6 * C * NP * 2 + C * C * 4 + NP * 4 + 1023) / 1024 * 1024; }
+inline int padded(int N) { return N <= 32 ? 32 : N <= 64 ? 64 : 128; }
+template <int NP>
+SYM_DEV int row_turn(int row) { return (((row & 7) << 1) | ((row >> 3) & 1)) & (NP / 8 - 1); }
+SYM_DEV int score_turn(int row) { return (row >> 1) & 7; }
+// a run's first block: runs need no more than a block past their rows' share
+SYM_DEV long long first_block(int s0, int run) { return (s0 >> 5) + run; }
+__host__ __device__ inline int ws_cols(int N) { return C + 2 * N; }      // (floats a row and head that a caller's scratch has at least)
 
 // ---- mode 0: decays and scores A of every chunk, grid (64-row tiles x 2 chunks, heads) ----------------------------------
 // G is held as a pair of floats: what counts are its differences, and once a few tokens of a chunk forget hard, G is in the
@@ -122,9 +134,7 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
     qS[tt * LD + n] = in ? (float)qv[e] : 0.f;
   }
   __syncthreads();
-  const int wc = ws_cols(N);
-  float* ws = a.ws + (r0 * a.H + h) * wc;
-  const long long wrow = (long long)a.H * wc;
+  char* const ws = reinterpret_cast<char*>(a.ws) + ((first_block(q0, seq) + off / C + sub) * a.H + h) * chunk_block(NP);
   if (tid < NP) {
     double g = 0.;
 #pragma unroll 8
@@ -136,14 +146,33 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
     }
   }
   __syncthreads();
-#pragma unroll 4
-  for (int i = tid; i < C * NP; i += NT) {     // (G stands still past the run's end, so the last row's is G_C)
-    const int tt = i / NP, n = i % NP;
-    if (tt >= nt || n >= N) continue;
-    const float gi = GS[tt * LD + n], li = LS[tt * LD + n];
-    ws[tt * wrow + C + n] = pow2(gi);
-    ws[tt * wrow + C + N + n] = kS[tt * LD + n] * pow2((GS[(C - 1) * LD + n] - gi) + (LS[(C - 1) * LD + n] - li));
+#pragma unroll
+  for (int u = 0; u < (C * NP / 8 + NT - 1) / NT; ++u) {      // (G stands still past the run's end, so the last row's is G_C)
+    const int i = tid + NT * u;
+    if (C * NP / 8 % NT && i >= C * NP / 8) break;
+    const int tt = i / (NP / 8), ch = i % (NP / 8), at = tt * LD + 8 * ch, end = (C - 1) * LD + 8 * ch;
+    f32x4 x[2], y[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const f32x4 gi = lds4(GS + at + 4 * e), li = lds4(LS + at + 4 * e), gc = lds4(GS + end + 4 * e), lc = lds4(LS + end + 4 * e);
+      const f32x4 qi = lds4(qS + at + 4 * e), ki = lds4(kS + at + 4 * e);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x[e][r] = qi[r] * pow2(gi[r]);
+        y[e][r] = ki[r] * pow2((gc[r] - gi[r]) + (lc[r] - li[r]));
+      }
+    }
+    const Parts sx = split(x[0], x[1]), sy = split(y[0], y[1]);
+    bf16* to = reinterpret_cast<bf16*>(ws) + tt * NP + 8 * (ch ^ row_turn<NP>(tt));
+    *reinterpret_cast<bf16x8*>(to) = sx.h;
+    *reinterpret_cast<bf16x8*>(to + C * NP) = sx.m;
+    *reinterpret_cast<bf16x8*>(to + 2 * C * NP) = sx.l;
+    *reinterpret_cast<bf16x8*>(to + 3 * C * NP) = sy.h;
+    *reinterpret_cast<bf16x8*>(to + 4 * C * NP) = sy.m;
+    *reinterpret_cast<bf16x8*>(to + 5 * C * NP) = sy.l;
   }
+  float* const scores = reinterpret_cast<float*>(ws + 6 * C * NP * 2);
+  if (tid < NP) scores[C * C + tid] = tid < N ? pow2(GS[(C - 1) * LD + tid]) : 0.f;
   const int col = lane & 15, g = lane >> 4;
   // rows 16 .., columns .. 15: the waves take the channel tiles in turn
   f32x4 d = {0.f, 0.f, 0.f, 0.f};
@@ -211,14 +240,14 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
     const int i = (tid + NT * u) / C, j = (tid + NT * u) % C;
     const float* x = XS + i * LT + j;
     const float v = j <= i ? (x[0] + x[C * LT]) + (x[2 * C * LT] + x[3 * C * LT]) : 0.f;
-    if (i < nt) ws[i * wrow + j] = v;
+    scores[i * C + 4 * ((j >> 2) ^ score_turn(i)) + (j & 3)] = i < nt ? v : 0.f;
   }
 }
 
 // bytes of LDS of a walk: two stages, mode 1's sums, the parts that waves hand over
 constexpr int scan_lds(int mode, int NB, int HV) {
-  const int NP = 32 * NB, rows = (mode == 0 ? 6 : 2) * C * (NP + 8) * 2;
-  return 2 * (rows + (mode == 0 ? (C * LT + NP) * 4 : 0)) + (mode == 1 ? 8 * HV * 3 * C * 4 : 0) + (HV - 1) * 16 * 4 * HV * 128;
+  const int NP = 32 * NB;
+  return 2 * (mode == 0 ? chunk_block(NP) : 2 * C * (NP + 8) * 2) + (mode == 1 ? 8 * HV * 3 * C * 4 : 0) + (HV - 1) * 16 * 4 * HV * 128;
 }
 
 // ---- the walk ------------------------------------------------------------------------------------------------------------
@@ -229,25 +258,26 @@ constexpr int scan_lds(int mode, int NB, int HV) {
 // -> 197, 2 of 750 101 -> 92; 64 x 128 x 64, 2 of 750, 84.5 -> 80.5).  256 registers a lane: with more allowed the
 // compiler keeps a part in AGPRs, which was slower.
 template <int MODE, int NB, int HV>
-__global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanArgs a) {
+__global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanArgs a, int unit) {
   constexpr int TH = NT * HV, NWV = 4 * HV, NBW = NB / HV, TI = 2 / HV;
-  constexpr int NP = 32 * NB, LQ = NP + 8;              // LQ: bf16 pitch of a [C][NP] matrix
+  constexpr int NP = 32 * NB, LQ = MODE == 0 ? NP : NP + 8;   // LQ: bf16 pitch of a [C][NP] matrix
   constexpr int PL = MODE == 0 ? 3 : 1;                 // bf16 parts of the staged vectors
   constexpr int oK = PL * C * LQ, oF = oK + PL * C * LQ;      // in bf16: q | k, a part behind the other
-  constexpr int FS = MODE == 0 ? C * LT + NP : 0;       // floats: A | 2^(G_C)
-  constexpr int STAGE = oF * 2 + FS * 4;                // bytes
+  constexpr int STAGE = MODE == 0 ? chunk_block(NP) : oF * 2; // bytes; behind oF in mode 0: A | 2^(G_C)
   constexpr int SUMS = MODE == 1 ? 2 * NWV * 3 * C : 0; // floats, mode 1: G | its low part | b of 2 NWV chunks
   static_assert(STAGE % 16 == 0, "stages start at multiples of 16 bytes");
   static_assert(2 * STAGE + SUMS * 4 + (HV - 1) * 16 * NWV * 128 == scan_lds(MODE, NB, HV), "the launch's LDS");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* const sums = reinterpret_cast<float*>(smem + 2 * STAGE);
   f32x4* const given = reinterpret_cast<f32x4*>(smem + 2 * STAGE + SUMS * 4);      // [2][NWV][64]
-  const int N = a.N, P = a.P, h = blockIdx.y, run = blockIdx.z;
+  const int N = a.N, P = a.P;
+  const WalkPlace at = walk_place(unit);
+  const int slab = at.slab, h = at.head, run = at.run;
   const int s0 = a.cu_q[run], s1 = a.cu_q[run + 1];
   if (s1 <= s0) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, g = lane >> 4;
   const int hf = HV == 2 ? wave >> 2 : 0, ch0 = 32 * NBW * hf;      // the wave's channels
-  const int p = blockIdx.x * 64 + (wave & 3) * 16 + col;
+  const int p = slab * 64 + (wave & 3) * 16 + col;
   const bool pin = p < P;
   const int chunks = (s1 - s0 + C - 1) / C;
   const int pr = a.prev_row[s0], sv = a.save_slot[s1 - 1];
@@ -255,47 +285,38 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
   const bf16* k = reinterpret_cast<const bf16*>(a.k) + s0 * a.ldk + (h / a.hpg) * N;
   const bf16* v = reinterpret_cast<const bf16*>(a.v) + s0 * a.ldv + (long long)h * P;
   const bf16* dt = reinterpret_cast<const bf16*>(a.dz) + s0 * a.ldd + h;          // mode 1
-  const int wc = ws_cols(N);
-  const long long wrow = (long long)a.H * wc;
-  const float* ws = MODE == 0 ? a.ws + ((long long)s0 * a.H + h) * wc : nullptr;
+  const char* block = MODE == 0 ? reinterpret_cast<const char*>(a.ws) + (first_block(s0, run) * a.H + h) * STAGE : nullptr;
   float* out = a.out + ((long long)s0 * a.H + h) * P;
   const long long orow = (long long)a.H * P;
   const int ldv = (int)a.ldv * 2, ldo = (int)orow * 4;                            // (decay_chunk_takes bounds them)
   const int vo = pin ? 4 * g * ldv + 2 * p : NO_PLACE, oo = pin ? (4 * g + 16 * hf) * ldo + 4 * p : NO_PLACE;
 
-  // staging: thread (token tt, 8 channels from c8), PASS tokens apart
+  // staging, mode 0: the chunk's block as it lies, by direct loads; mode 1: thread (token tt, 8 channels from c8), PASS tokens apart
   constexpr int GR = NP / 8, TSTEP = TH / GR, PASS = (C + TSTEP - 1) / TSTEP;
   const int c8 = 8 * (tid % GR), tt0 = tid / GR;
   const bool nin = c8 < N && tt0 < C;                   // (N is a multiple of 8)
-  Pack8 rq[PASS], rk[MODE == 1 ? PASS : 1];
-  f32x4 rp[MODE == 0 ? PASS : 1][2], ry[MODE == 0 ? PASS : 1][2], pl, ra;   // mode 0: 2^(G_i), k_i 2^(G_C - G_i), 2^(G_C)
+  Pack8 rq[PASS], rk[PASS];
   bf16 vn[8];
-  int qo[PASS], ko[PASS], wo[PASS];
+  int qo[PASS], ko[PASS];
 #pragma unroll
   for (int u = 0; u < PASS; ++u) {
     const int tt = tt0 + TSTEP * u;
     qo[u] = nin ? tt * (int)a.ldq * 2 + 2 * c8 : NO_PLACE;
     ko[u] = nin ? tt * (int)a.ldk * 2 + 2 * c8 : NO_PLACE;
-    wo[u] = nin ? tt * (int)wrow * 4 + 4 * (C + c8) : NO_PLACE;
   }
+  const unsigned int lds0 = lds_address(smem) + wave * 1024;
   auto fetch = [&](int c) {
-    const int t0 = c * C, nt = min(C, s1 - s0 - t0);
-    const __amdgpu_buffer_rsrc_t bq = chunk_rows(q + t0 * a.ldq, a.ldq * 2, nt, N * 2);
-#pragma unroll
-    for (int u = 0; u < PASS; ++u) rq[u].u = row16(bq, qo[u]);
     if constexpr (MODE == 0) {
-      const __amdgpu_buffer_rsrc_t bw = chunk_rows(ws + t0 * wrow, wrow * 4, nt, wc * 4);
+      const u32x4 from = buffer_words(block + (long long)c * a.H * STAGE, STAGE);
 #pragma unroll
-      for (int u = 0; u < PASS; ++u)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          rp[u][i] = row16f(bw, wo[u] + (nin ? 16 * i : 0));
-          ry[u][i] = row16f(bw, wo[u] + (nin ? 4 * N + 16 * i : 0));
-        }
-      pl = 4 * tid < N ? lds4(ws + (t0 + nt - 1) * wrow + C + 4 * tid) : f32x4{0.f, 0.f, 0.f, 0.f};
-      ra = row16f(bw, tid < 8 * C ? (tid / 8) * (int)wrow * 4 + 16 * (tid % 8) : NO_PLACE);
+      for (int i = 0; i < (STAGE / 1024 + NWV - 1) / NWV; ++i)
+        if (NWV * i + wave < STAGE / 1024) direct_buffer_load16(from, 16 * lane, 1024 * (NWV * i + wave), lds0 + (c & 1) * STAGE + 1024 * NWV * i);
     } else {
+      const int t0 = c * C, nt = min(C, s1 - s0 - t0);
+      const __amdgpu_buffer_rsrc_t bq = chunk_rows(q + t0 * a.ldq, a.ldq * 2, nt, N * 2);
       const __amdgpu_buffer_rsrc_t bk = chunk_rows(k + t0 * a.ldk, a.ldk * 2, nt, N * 2);
+#pragma unroll
+      for (int u = 0; u < PASS; ++u) rq[u].u = row16(bq, qo[u]);
 #pragma unroll
       for (int u = 0; u < PASS; ++u) rk[u].u = row16(bk, ko[u]);
     }
@@ -325,33 +346,32 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
     }
   };
   auto stash = [&](int c) {
-    bf16* st = reinterpret_cast<bf16*>(smem + (c & 1) * STAGE);
+    if constexpr (MODE == 0) {
+      wait_direct_loads();
+    } else {
+      bf16* st = reinterpret_cast<bf16*>(smem + (c & 1) * STAGE);
 #pragma unroll
-    for (int u = 0; u < PASS; ++u) {
-      const int tt = tt0 + TSTEP * u;
-      if (tt >= C) break;
-      if constexpr (MODE == 1) {
+      for (int u = 0; u < PASS; ++u) {
+        const int tt = tt0 + TSTEP * u;
+        if (tt >= C) break;
         *reinterpret_cast<uint4*>(st + tt * LQ + c8) = rq[u].u;
         *reinterpret_cast<uint4*>(st + oK + tt * LQ + c8) = rk[u].u;
-      } else {
-        f32x4 x[2];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i >> 2][i & 3] = (float)rq[u].h[i] * rp[u][i >> 2][i & 3];
-        const Parts sx = split(x[0], x[1]), sy = split(ry[u][0], ry[u][1]);
-        *reinterpret_cast<bf16x8*>(st + tt * LQ + c8) = sx.h;
-        *reinterpret_cast<bf16x8*>(st + (C + tt) * LQ + c8) = sx.m;
-        *reinterpret_cast<bf16x8*>(st + (2 * C + tt) * LQ + c8) = sx.l;
-        *reinterpret_cast<bf16x8*>(st + oK + tt * LQ + c8) = sy.h;
-        *reinterpret_cast<bf16x8*>(st + oK + (C + tt) * LQ + c8) = sy.m;
-        *reinterpret_cast<bf16x8*>(st + oK + (2 * C + tt) * LQ + c8) = sy.l;
       }
     }
-    if constexpr (MODE == 0) {
-      float* fs = reinterpret_cast<float*>(st + oF);
-      if (tid < 8 * C) *reinterpret_cast<f32x4*>(fs + (tid / 8) * LT + 4 * (tid % 8)) = ra;
-      if (4 * tid < NP) *reinterpret_cast<f32x4*>(fs + C * LT + 4 * tid) = pl;
-    }
   };
+  // mode 0's places in the block, bytes: of q's 8-byte pieces, of k's for the transpose reads, of A's quads
+  int qx[NBW][2], kx[2 * NBW], ax[2];
+  if constexpr (MODE == 0) {
+    const int kr = 4 * g + (col >> 2);
+#pragma unroll
+    for (int t = 0; t < NBW; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) qx[t][i] = col * NP * 2 + 16 * ((ch0 / 8 + 4 * t + 2 * i + (g >> 1)) ^ row_turn<NP>(col)) + 8 * (g & 1);
+#pragma unroll
+    for (int t = 0; t < 2 * NBW; ++t) kx[t] = kr * NP * 2 + 16 * ((ch0 / 8 + 2 * t + ((col & 3) >> 1)) ^ row_turn<NP>(kr)) + 8 * (col & 1);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) ax[j] = col * C * 4 + 16 * ((4 * j + g) ^ score_turn(col));
+  }
 
   f32x4 S[2 * NBW];
   const bool old = pr <= -2 && pin;
@@ -406,7 +426,17 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
 #pragma unroll
       for (int part = 0; part < PL; ++part)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) qf[t & 1][part][i] = pair4(Qr + (part * C + 16 * i) * LQ + 32 * t);
+        for (int i = 0; i < 2; ++i) {
+          if constexpr (MODE == 0) {
+            const char* from = reinterpret_cast<const char*>(st) + (part * C + 16 * i) * NP * 2;
+            Pack8 f;
+            const uint2 x = *reinterpret_cast<const uint2*>(from + qx[t][0]), y = *reinterpret_cast<const uint2*>(from + qx[t][1]);
+            f.u = make_uint4(x.x, x.y, y.x, y.y);
+            qf[t & 1][part][i] = f.v;
+          } else {
+            qf[t & 1][part][i] = pair4(Qr + (part * C + 16 * i) * LQ + 32 * t);
+          }
+        }
     };
     load_q(0);
     if (NBW > 1) load_q(1);
@@ -414,7 +444,7 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
 #pragma unroll
       for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) A[i][j] = lds4(fs + (16 * (i + hf) + col) * LT + 16 * j + 4 * g);
+        for (int j = 0; j < 2; ++j) A[i][j] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(fs + 16 * (i + hf) * C) + ax[j]);
     } else {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
@@ -509,7 +539,8 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
     const char* Kt = reinterpret_cast<const char*>(st + oK + (4 * g + (col >> 2)) * LQ + ch0) + 8 * (col & 3);
     auto turned = [&](int part, int t) {
       Pack8 f;
-      const uint2 x = read_tr(Kt + (part * C * LQ + 16 * t) * 2), y = read_tr(Kt + ((part * C + 16) * LQ + 16 * t) * 2);
+      const char* from = MODE == 0 ? reinterpret_cast<const char*>(st + oK) + kx[t] : Kt + 32 * t;
+      const uint2 x = read_tr(from + part * C * LQ * 2), y = read_tr(from + (part * C + 16) * LQ * 2);
       f.u = make_uint4(x.x, x.y, y.x, y.y);
       return f.v;
     };
@@ -519,7 +550,7 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
     f32x4 dec[MODE == 0 ? 2 * NBW : 1];
     if constexpr (MODE == 0) {
 #pragma unroll
-      for (int t = 0; t < 2 * NBW; ++t) dec[t] = lds4(fs + C * LT + ch0 + 16 * t + 4 * g);
+      for (int t = 0; t < 2 * NBW; ++t) dec[t] = lds4(fs + C * C + ch0 + 16 * t + 4 * g);
     }
     if constexpr (HV == 2) {
       given[((c & 1) * NWV + (wave ^ 4)) * 64 + lane] = hf ? O[0] : O[1];
@@ -606,7 +637,9 @@ void launch_scan(const DecayScanArgs& a, hipStream_t s) {
     return true;
   }();
   (void)raised;
-  decay_chunk_scan_kernel<MODE, NB, HV><<<dim3((a.P + 63) / 64, a.H, a.runs), NT * HV, lds, s>>>(a);
+  const int slabs = (a.P + 63) / 64;
+  const long long total = (long long)slabs * a.H * a.runs;
+  decay_chunk_scan_kernel<MODE, NB, HV><<<dim3(slabs, a.H, a.runs), NT * HV, lds, s>>>(a, walk_unit(total, slabs));
 }
 
 template <int MODE, int NB>
@@ -651,6 +684,12 @@ bool decay_chunk_takes(const DecayScanArgs& a) {
   constexpr long long top = 1 << 24;      // (a chunk of 32 rows is addressed by 32-bit offsets)
   if (std::max({a.ldq, a.ldk, a.ldv, a.ldd, (long long)a.H * a.P, (long long)a.H * ws_cols(a.N)}) > top) return false;
   return a.mode == 1 || (a.tiles && a.ntiles > 0 && a.ws && (uintptr_t)a.ws % 16 == 0);
+}
+
+// floats of the chunked form's scratch: a block per chunk and head (0: none)
+long long decay_chunk_scratch(int mode, long long T, long long runs, long long H, int N) {
+  if (mode != 0 || N > 128) return 0;
+  return (T / C + runs + 1) * H * (chunk_block(padded(N)) / 4);
 }
 
 void launch_decay_chunks(const DecayScanArgs& a, hipStream_t s) {

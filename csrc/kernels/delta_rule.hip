@@ -37,6 +37,7 @@
 #include "bf16_parts.h"
 #include "common.h"
 #include "hybrid_launchers.h"
+#include "walk_places.h"
 
 namespace {
 
@@ -648,7 +649,7 @@ __global__ __launch_bounds__(128 * MW) void delta_chunk_scan_kernel(DeltaRuleArg
 // An infinity or NaN of the state or a value ends as NaN in its own column from its chunk on, as with fp32 products, which meet 0 x
 // infinity in T and Aqk.
 template <bool CHANNEL, int NB, int MW>
-__global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(DeltaRuleArgs a) {
+__global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(DeltaRuleArgs a, int unit) {
   constexpr int ST = 64 * MW;                            // staging threads
   constexpr int NP = 32 * NB, LQ = NP + 8;               // LQ: bf16 pitch of a [C][NP] matrix
   constexpr int PART = C * LQ, oQ = 3 * PART, oH = CHANNEL ? 6 * PART : 0, MATS = CHANNEL ? 3 : 2;
@@ -657,7 +658,8 @@ __global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(Del
   static_assert(STAGE % 16 == 0 && 2 * STAGE <= 160 * 1024, "two stages");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int N = a.N, P = a.P;
-  const int h = blockIdx.y, run = blockIdx.z;
+  const WalkPlace at = walk_place(unit);
+  const int slab = at.slab, h = at.head, run = at.run;
   const int s0 = a.cu_q[run], s1 = a.cu_q[run + 1];
   if (s1 <= s0) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -767,7 +769,7 @@ __global__ __launch_bounds__(128 * MW, 4 / MW) void delta_chunk_parts_kernel(Del
   }
   // ---- multiplying waves -----------------------------------------------------------------------------------------
   const int col = lane & 15, g = lane >> 4;
-  const int p = blockIdx.x * 16 * MW + wave * 16 + col;
+  const int p = slab * 16 * MW + wave * 16 + col;
   const bool pin = p < P;
   const int pr = a.prev_row[s0];
   const int sv = a.save_slot[s1 - 1];
@@ -972,7 +974,9 @@ void launch_parts(const DeltaRuleArgs& a, hipStream_t s) {
   constexpr int lds = 2 * ((CHANNEL ? 9 : 6) * C * (32 * NB + 8) * 2 + (CHANNEL ? 32 * NB : 2 * C + 4) * 4);
   static const bool raised = (raise_lds(reinterpret_cast<const void*>(&delta_chunk_parts_kernel<CHANNEL, NB, MW>)), true);
   (void)raised;
-  delta_chunk_parts_kernel<CHANNEL, NB, MW><<<dim3((a.P + 16 * MW - 1) / (16 * MW), a.H, a.runs), 128 * MW, lds, s>>>(a);
+  const int slabs = (a.P + 16 * MW - 1) / (16 * MW);
+  const long long total = (long long)slabs * a.H * a.runs;
+  delta_chunk_parts_kernel<CHANNEL, NB, MW><<<dim3(slabs, a.H, a.runs), 128 * MW, lds, s>>>(a, walk_unit(total, slabs));
 }
 
 template <typename T, bool CHANNEL, int NN>

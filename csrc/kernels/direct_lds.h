@@ -12,6 +12,10 @@ SYM_DEV void direct_load16(const void* src, unsigned int lds) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }
 // the same through a buffer's four words: its base, + `off` bytes of the lane, + `soff` bytes
+SYM_DEV u32x4 buffer_words(const void* base, long long bytes) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(base);
+  return u32x4{(unsigned int)p, (unsigned int)(p >> 32) & 0xffffu, (unsigned int)bytes, 0x00020000u};
+}
 SYM_DEV void direct_buffer_load16(u32x4 buf, int off, int soff, unsigned int lds) {
   asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(off), "s"(buf), "s"(soff)
                : "memory", "m0");

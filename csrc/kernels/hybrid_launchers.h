@@ -300,12 +300,13 @@ struct DecayScanArgs {
   const int* save_slot;
   int runs, T;
   float* out;           // [T][H][P]
-  // chunked form (decay_chunk.hip), mode 0: 64-row tiles (run, first row), and fp32 scratch [T][H][32 + 2 N]
+  // chunked form (decay_chunk.hip), mode 0: 64-row tiles (run, first row), and decay_chunk_scratch() floats
   const int* tiles;
   int ntiles;
   float* ws;
 };
 bool decay_chunk_takes(const DecayScanArgs& a);
+long long decay_chunk_scratch(int mode, long long T, long long runs, long long H, int N);
 void launch_decay_chunks(const DecayScanArgs& a, hipStream_t s);
 void launch_decay_scan(const DecayScanArgs& a, int f32, hipStream_t s);
 // One token a run in bf16 (cu_q null, T = runs; s.out is not written), with what follows the scan: out [T][H P] =

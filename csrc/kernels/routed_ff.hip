@@ -683,11 +683,6 @@ struct ExpertTile {
   int e, r0, rows, n0, half;      // half: 128 rows at most
 };
 
-SYM_DEV u32x4 buffer_words(const void* base, long long bytes) {
-  const uintptr_t p = reinterpret_cast<uintptr_t>(base);
-  return u32x4{(unsigned int)p, (unsigned int)(p >> 32) & 0xffffu, (unsigned int)bytes, 0x00020000u};
-}
-
 SYM_DEV int lanes_upto(int v, int lane) {      // inclusive sum over the lanes
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {

@@ -323,7 +323,7 @@ class LemunexLM:
         y = self._buf("rec.y", (T, g.heads * g.vdim), torch.float32)
         tiles = ws = None
         if prefill and self.dtype == torch.bfloat16 and self.device.type != "cpu":   # (the 32-bit model walks token by token)
-            tiles, ws = b.tiles, self._buf("gla.ws", (T, g.heads, ops.decay_ws_cols(g.dim)), torch.float32)
+            tiles, ws = b.tiles, self._buf("gla.ws", (ops.decay_scratch(ops.DECAY_CHANNEL_GATE, T, runs, g.heads, g.dim, g.vdim),), torch.float32)
         ops.decay_scan(ops.DECAY_CHANNEL_GATE, self._cols(z, P, "right.q"), self._cols(z, P, "right.k"),
                        self._cols(z, P, "right.v"), dz, P["right.a2.b"], g.tau, None, g.dim ** -0.5, g.heads, g.dim,
                        g.vdim, 1, cache.rec[i], b.cu_q if prefill else None, b.prev_row, b.save_slot, runs, y, tiles=tiles, ws=ws)

@@ -1151,9 +1151,13 @@ def window_attn_decay(q, k_cache, v_cache, block_tables, row_seq, positions, win
 
 
 def decay_ws_cols(N: int) -> int:
-    """Columns of decay_scan's chunk scratch per row and head: a score row, the channels' decays since the chunk's start and the
-    keys decayed to its end."""
+    """Columns per row and head that decay_scan's scratch has at least; decay_scratch's size spares it one of its own."""
     return 32 + 2 * N
+
+
+def decay_scratch(mode, T, runs, H, N, P) -> int:
+    """Floats of scratch that decay_scan's chunked form of a step of T rows in ``runs`` runs works in."""
+    return _hyb().decay_scratch(int(mode), int(T), int(runs), int(H), int(N), int(P))
 
 
 def memory_norm_gate(y, m, gate, w, eps, out):

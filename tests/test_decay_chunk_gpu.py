@@ -212,3 +212,16 @@ def test_value_rows_that_overlap(gpu, mode, step):
     for a, b in ((want, out), (end, state)):
         ok = b.isfinite()
         assert float((a[ok] - b[ok]).norm() / b[ok].norm()) <= 4e-6       # (both within 2e-6 of the exact ones)
+
+
+@pytest.mark.parametrize("H,N,P,G,lens", SHAPES)
+def test_scratch_of_its_own_or_the_callers(gpu, H, N, P, G, lens):
+    """A scratch too small for the chunks' blocks is taken and stands for one of the walk's own: the same numbers."""
+    c = _Case(gpu, ops.DECAY_CHANNEL_GATE, H, N, P, G, lens)
+    start = c.state.clone()
+    out, state = (t.clone() for t in c.run(True))
+    c.state.copy_(start)
+    c.ws = torch.full((ops.decay_scratch(c.mode, c.T, c.R, H, N, P),), float("nan"), device=gpu)
+    assert c.ws.numel() >= c.T * H * ops.decay_ws_cols(N)
+    for got, want in zip(c.run(True), (out, state)):
+        assert torch.equal(got, want)
