@@ -371,7 +371,7 @@ DecayScanArgs scan_args(int64_t mode, const Tensor& q, const Tensor& k, const Te
 
 int64_t decay_scratch(int64_t mode, int64_t T, int64_t runs, int64_t H, int64_t N, int64_t P) {
   TORCH_CHECK(mode >= 0 && mode <= 2 && T >= 0 && runs >= 0 && H > 0 && N >= 1 && N <= 256 && P >= 1, "decay_scratch: sizes");
-  return std::max<int64_t>(mode == 0 ? T * H * (32 + 2 * N) : 0, decay_chunk_scratch((int)mode, T, runs, H, (int)N));
+  return std::max<int64_t>(mode == 0 ? T * H * (32 + 2 * N) : 0, decay_chunk_scratch((int)mode, T, runs, H, (int)N, P));
 }
 
 void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dz, const Tensor& dbias,
@@ -380,13 +380,16 @@ void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v,
                 int64_t runs, Tensor& out, const OptTensor& mout, const OptTensor& tiles, const OptTensor& ws) {
   DecayScanArgs a = scan_args(mode, q, k, v, dz, dbias, rate, tau, skip, q_scale, H, N, P, hpg, state, cu_q, prev_row, save_slot,
                               runs, out, std::nullopt, mout, tiles, ws);
-  Tensor own;      // (a scratch of 32 + 2 N floats a row and head is taken, and is not enough)
-  if (a.ws && v.scalar_type() != at::kFloat && decay_chunk_takes(a)) {
-    const int64_t need = decay_chunk_scratch(a.mode, a.T, a.runs, a.H, a.N);
-    if (ws->numel() < need) {
+  Tensor own;
+  if (ws.has_value() && mode <= 1 && v.scalar_type() != at::kFloat && decay_chunk_takes(a)) {
+    dtype(*ws, at::kFloat, "ws");
+    const int64_t need = decay_chunk_scratch(a.mode, a.T, a.runs, a.H, a.N, a.P);
+    a.ws = ptr<float>(*ws);
+    if (ws->numel() < need) {      // (32 + 2 N floats a row and head are taken, and are not enough)
       own = at::empty({need}, ws->options());
       a.ws = ptr<float>(own);
     }
+    decay_chunk_segments(a);
   }
   launch_decay_scan(a, v.scalar_type() == at::kFloat, cur_stream(v));
 }

@@ -8,12 +8,13 @@
 // chunk and S_0 the state in front of it,
 //     o_i = (q_i 2^(G_i))^T S_0 + sum_{j <= i} A_ij v_j,     A_ij = b_j sum_n q_in k_jn 2^(G_in - G_jn)
 //     S_C = 2^(G_C) S_0 + sum_j (k_j 2^(G_C - G_j) b_j) v_j^T                 (every exponent <= 0: nothing overflows)
-// is matrix products; a run's chunks are walked in order.
+// is matrix products; a run's chunks are walked in order, few long runs in segments at once (a segment's state from 0 and its decays
+// first, then each segment from the states in front of it).
 //
 // Precision: q, k and v are bf16, so they are exact operands of v_mfma_f32_16x16x32_bf16, which accumulates in fp32.  An
 // fp32 operand (the state, a scaled vector, the scores) is used as the sum of three bf16 parts (bf16_parts.h).
 //
-// Work split: grid (P / 64, heads, runs), waves of 16 value columns with all of N or half of it: the state stays in accumulator registers
+// Work split: grid (P / 64, heads, runs or segments), waves of 16 value columns with all of N or half of it: the state stays in accumulator registers
 // for the whole run.  An accumulator's rows are 4 (lane / 16) + r, a B operand's contraction index is 8 (lane / 16) + j; with
 // the contraction taken in the order j < 4: 4 g + j, else 16 + 4 g + j - 4, two accumulator tiles ARE a B operand, and the A
 // operand is read in the same order (two 8-byte LDS reads).  The same holds for the values and, computed transposed, for the
@@ -244,6 +245,63 @@ __global__ __launch_bounds__(NT) void decay_chunk_prep_kernel(DecayScanArgs a) {
   }
 }
 
+// ---- segments of runs ------------------------------------------------------------------------------------------------------
+// Runs too few to give every CU a workgroup (mode 1: two) are cut: as many segments as there are workgroups for, none longer than it
+// must be, the same number of chunks in each of a run's but for one.  All workgroups find the same from the same lengths.
+constexpr int SEGMENTS_MAX = 16;      // (and fewer runs than that: a row of 16 lanes holds them)
+
+// Segments that a step's walks have workgroups for; 0: whole runs.  The walk of the states is 2 / 5 of a walk, and a launch and the
+// states in front of a segment cost about 4 chunks (mode 1, with two workgroups a CU: 8).  Walks, us, whole / in segments: 8 heads x 128 x
+// 256, one run of 130 tokens 19 / 19.5, of 300 33 / 20.5, of 7900 782 / 183, 2 of 300 36 / 27, 4 of 175 30 / 32, 4 of 500 74 / 66,
+// 6 of 1000 140 / 165; 64 x 128 x 64, one of 130 21 / 25, of 300 36 / 30, of 7900 776 / 218, 2 of 300 37 / 36, 2 of 1000 105 / 68,
+// 3 of 267 37 / 39, 4 of 500 75 / 77.
+int walk_segments(int mode, long long T, long long runs, long long H, long long P) {
+  const long long per = H * ((P + 63) / 64);
+  const long long n = std::min<long long>(SEGMENTS_MAX, (mode == 0 ? 256 : 512) / per);
+  if (mode > 1 || runs < 1 || n < 2 * runs) return 0;
+  return T >= (mode == 0 ? 96 * runs + 384 * runs * runs / n : 128 * runs + 768 * runs * runs / n) ? (int)n : 0;
+}
+
+struct Segment {
+  int run, from, to;            // chunks of the run
+  int place, of, item0;         // its number among the run's, how many these are, the run's first item
+};
+
+SYM_DEV int row_total(int v) {      // over a row of 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
+SYM_DEV bool find_segment(const int* cu_q, int runs, int items, int item, Segment& s) {
+  const int lane = threadIdx.x & 15;
+  const int n = lane < runs ? (max(0, cu_q[lane + 1] - cu_q[lane]) + C - 1) / C : 0;
+  auto pieces = [&](int len) { return (int)((unsigned)(n + len - 1) / (unsigned)len); };
+  int lo = max(2, (row_total(n) + items - 1) / items), hi = lo;      // the shortest that are no more than `items`
+  while (row_total(pieces(hi)) > items) hi *= 2;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (row_total(pieces(mid)) > items) lo = mid + 1;
+    else hi = mid;
+  }
+  const int k = pieces(hi);
+  int upto = k;
+  upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xf, 0xf, false);
+  upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xf, 0xf, false);
+  upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xf, 0xf, false);
+  upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xf, 0xf, false);
+  const int run = __builtin_popcountll(__ballot(upto <= item) & 0xffff);
+  if (run >= runs) return false;
+  const int chunks = __builtin_amdgcn_readlane(n, run);
+  s.run = run, s.of = __builtin_amdgcn_readlane(k, run);
+  s.item0 = __builtin_amdgcn_readlane(upto, run) - s.of;
+  s.place = item - s.item0;
+  s.from = chunks * s.place / s.of, s.to = chunks * (s.place + 1) / s.of;
+  return true;
+}
+
 // bytes of LDS of a walk: two stages, mode 1's sums, the parts that waves hand over
 constexpr int scan_lds(int mode, int NB, int HV) {
   const int NP = 32 * NB;
@@ -257,7 +315,12 @@ constexpr int scan_lds(int mode, int NB, int HV) {
 // other over in LDS; it is read behind the chunk's barrier and stored a chunk later (8 heads x 128 x 256, us: 8 runs of 1012 tokens 210
 // -> 197, 2 of 750 101 -> 92; 64 x 128 x 64, 2 of 750, 84.5 -> 80.5).  256 registers a lane: with more allowed the
 // compiler keeps a part in AGPRs, which was slower.
-template <int MODE, int NB, int HV>
+// WALK: WHOLE runs, grid z their number; or, where the runs are few (walk_segments), segments of them: the STATES that all segments but
+// a run's last add up from 0 (the first: from the run's state), with their channels' decays, then the SEGMENTS themselves, each from the
+// states in front of it.
+enum { WHOLE, STATES, SEGMENTS };
+
+template <int MODE, int NB, int HV, int WALK>
 __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanArgs a, int unit) {
   constexpr int TH = NT * HV, NWV = 4 * HV, NBW = NB / HV, TI = 2 / HV;
   constexpr int NP = 32 * NB, LQ = MODE == 0 ? NP : NP + 8;   // LQ: bf16 pitch of a [C][NP] matrix
@@ -272,20 +335,24 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
   f32x4* const given = reinterpret_cast<f32x4*>(smem + 2 * STAGE + SUMS * 4);      // [2][NWV][64]
   const int N = a.N, P = a.P;
   const WalkPlace at = walk_place(unit);
-  const int slab = at.slab, h = at.head, run = at.run;
-  const int s0 = a.cu_q[run], s1 = a.cu_q[run + 1];
-  if (s1 <= s0) return;
+  const int slab = at.slab, h = at.head;
+  Segment seg{at.run, 0, 0, 0, 1, 0};
+  if constexpr (WALK != WHOLE)
+    if (!find_segment(a.cu_q, a.runs, a.segments, at.run, seg)) return;
+  const int run = seg.run, q0 = a.cu_q[run];
+  const int s0 = WALK == WHOLE ? q0 : q0 + C * seg.from, s1 = WALK == WHOLE ? a.cu_q[run + 1] : min(a.cu_q[run + 1], q0 + C * seg.to);
+  if (s1 <= s0 || (WALK == STATES && seg.place + 1 == seg.of)) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, g = lane >> 4;
   const int hf = HV == 2 ? wave >> 2 : 0, ch0 = 32 * NBW * hf;      // the wave's channels
   const int p = slab * 64 + (wave & 3) * 16 + col;
   const bool pin = p < P;
   const int chunks = (s1 - s0 + C - 1) / C;
-  const int pr = a.prev_row[s0], sv = a.save_slot[s1 - 1];
+  const int pr = a.prev_row[q0], sv = a.save_slot[s1 - 1];      // (a save_slot in the middle of a run is no one's)
   const bf16* q = reinterpret_cast<const bf16*>(a.q) + s0 * a.ldq + (h / a.hpg) * N;
   const bf16* k = reinterpret_cast<const bf16*>(a.k) + s0 * a.ldk + (h / a.hpg) * N;
   const bf16* v = reinterpret_cast<const bf16*>(a.v) + s0 * a.ldv + (long long)h * P;
   const bf16* dt = reinterpret_cast<const bf16*>(a.dz) + s0 * a.ldd + h;          // mode 1
-  const char* block = MODE == 0 ? reinterpret_cast<const char*>(a.ws) + (first_block(s0, run) * a.H + h) * STAGE : nullptr;
+  const char* block = MODE == 0 ? reinterpret_cast<const char*>(a.ws) + ((first_block(q0, run) + seg.from) * a.H + h) * STAGE : nullptr;
   float* out = a.out + ((long long)s0 * a.H + h) * P;
   const long long orow = (long long)a.H * P;
   const int ldv = (int)a.ldv * 2, ldo = (int)orow * 4;                            // (decay_chunk_takes bounds them)
@@ -310,13 +377,15 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
       const u32x4 from = buffer_words(block + (long long)c * a.H * STAGE, STAGE);
 #pragma unroll
       for (int i = 0; i < (STAGE / 1024 + NWV - 1) / NWV; ++i)
-        if (NWV * i + wave < STAGE / 1024) direct_buffer_load16(from, 16 * lane, 1024 * (NWV * i + wave), lds0 + (c & 1) * STAGE + 1024 * NWV * i);
+        if (NWV * i + wave >= (WALK == STATES ? oK * 2 / 1024 : 0) && NWV * i + wave < STAGE / 1024)
+          direct_buffer_load16(from, 16 * lane, 1024 * (NWV * i + wave), lds0 + (c & 1) * STAGE + 1024 * NWV * i);
     } else {
       const int t0 = c * C, nt = min(C, s1 - s0 - t0);
       const __amdgpu_buffer_rsrc_t bq = chunk_rows(q + t0 * a.ldq, a.ldq * 2, nt, N * 2);
       const __amdgpu_buffer_rsrc_t bk = chunk_rows(k + t0 * a.ldk, a.ldk * 2, nt, N * 2);
 #pragma unroll
-      for (int u = 0; u < PASS; ++u) rq[u].u = row16(bq, qo[u]);
+      for (int u = 0; u < PASS; ++u)
+        if (WALK != STATES) rq[u].u = row16(bq, qo[u]);
 #pragma unroll
       for (int u = 0; u < PASS; ++u) rk[u].u = row16(bk, ko[u]);
     }
@@ -354,7 +423,7 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
       for (int u = 0; u < PASS; ++u) {
         const int tt = tt0 + TSTEP * u;
         if (tt >= C) break;
-        *reinterpret_cast<uint4*>(st + tt * LQ + c8) = rq[u].u;
+        if (WALK != STATES) *reinterpret_cast<uint4*>(st + tt * LQ + c8) = rq[u].u;
         *reinterpret_cast<uint4*>(st + oK + tt * LQ + c8) = rk[u].u;
       }
     }
@@ -373,8 +442,18 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
     for (int j = 0; j < 2; ++j) ax[j] = col * C * 4 + 16 * ((4 * j + g) ^ score_turn(col));
   }
 
+  fetch(0);
+  fetch_v(0);
   f32x4 S[2 * NBW];
-  const bool old = pr <= -2 && pin;
+  // a segment's states (and a split run's own, in the place of its last segment, which hands on none: a run's state may be saved
+  // where it came from) in the order of the accumulators, and behind them all their decays
+  const int slabs = (P + 63) / 64;
+  auto state_of = [&](int item) {
+    return reinterpret_cast<f32x4*>(a.seg) + ((((long long)item * a.H + h) * slabs + slab) * 8 * NB + wave * 2 * NBW) * 64 + lane;
+  };
+  float* const decays = a.seg + (long long)a.segments * a.H * slabs * 64 * NP + (long long)h * NP;      // + item H NP
+  const bool own = WALK == WHOLE || (WALK == STATES ? seg.place == 0 : seg.of == 1);
+  const bool old = own && pr <= -2 && pin;
   const float* st0 = a.state + (old ? (long long)(-(pr + 2)) * a.state_stride + (long long)h * N * P + p : 0);
 #pragma unroll
   for (int t = 0; t < 2 * NBW; ++t)
@@ -383,9 +462,42 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
       const int n = ch0 + 16 * t + 4 * g + r;
       S[t][r] = old && n < N ? st0[(long long)n * P] : 0.f;
     }
+  if constexpr (WALK == STATES) {
+    if (own)
+#pragma unroll
+      for (int t = 0; t < 2 * NBW; ++t) state_of(seg.item0 + seg.of - 1)[64 * t] = S[t];
+  }
+  if constexpr (WALK == SEGMENTS) {
+    if (!own) {
+      // four segments' at once: one wait for each four
+      constexpr int AT = 4;
+      const int parts = max(seg.place, 1), first = seg.place ? seg.item0 : seg.item0 + seg.of - 1;
+      for (int i0 = 0; i0 < parts; i0 += AT) {
+        f32x4 u[AT][2 * NBW], d[AT][MODE == 0 ? 2 * NBW : 1];
+#pragma unroll
+        for (int i = 0; i < AT; ++i) {
+          const int item = first + min(i0 + i, parts - 1);
+#pragma unroll
+          for (int t = 0; t < 2 * NBW; ++t) {
+            u[i][t] = state_of(item)[64 * t];
+            if (MODE == 0) d[i][MODE == 0 ? t : 0] = lds4(decays + (long long)item * a.H * NP + ch0 + 16 * t + 4 * g);
+          }
+          if (MODE == 1) d[i][0][0] = decays[(long long)item * a.H * NP];
+        }
+#pragma unroll
+        for (int i = 0; i < AT; ++i)
+          if (i0 + i < parts) {
+#pragma unroll
+            for (int t = 0; t < 2 * NBW; ++t)
+              S[t] = i0 + i == 0 ? u[i][t] : (MODE == 0 ? S[t] * d[i][MODE == 0 ? t : 0] : S[t] * d[i][0][0]) + u[i][t];
+          }
+      }
+    }
+  }
+  f32x4 gone[MODE == 0 ? 2 * NBW : 1];      // STATES: the segment's decays
+#pragma unroll
+  for (int t = 0; t < (MODE == 0 ? 2 * NBW : 1); ++t) gone[t] = f32x4{1.f, 1.f, 1.f, 1.f};
   const float skip = a.skip ? a.skip[h] : 0.f;
-  fetch(0);
-  fetch_v(0);
   if constexpr (MODE == 1) {
     fetch_step(wave);
     sum_steps(wave);
@@ -411,7 +523,7 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
     if constexpr (MODE == 1)
       if (c % NWV == 0 && c + NWV < chunks) fetch_step(c + NWV + wave);
     __builtin_amdgcn_sched_barrier(0);                  // the next chunk's loads in flight ahead of this one's products
-    if constexpr (HV == 2)
+    if constexpr (HV == 2 && WALK != STATES)
       if (c) store_tile(c - 1, 0, mine + a.q_scale * given[(((c - 1) & 1) * NWV + wave) * 64 + lane]);
     const bf16* st = reinterpret_cast<const bf16*>(smem + (c & 1) * STAGE);
     const float* fs = MODE == 0 ? reinterpret_cast<const float*>(st + oF) : sums + (c & (2 * NWV - 1)) * 3 * C;
@@ -438,14 +550,17 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
           }
         }
     };
-    load_q(0);
-    if (NBW > 1) load_q(1);
-    if constexpr (MODE == 0) {
+    if constexpr (WALK != STATES) {
+      load_q(0);
+      if (NBW > 1) load_q(1);
+    }
+    if constexpr (MODE == 0 && WALK != STATES) {
 #pragma unroll
       for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) A[i][j] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(fs + 16 * (i + hf) * C) + ax[j]);
-    } else {
+    }
+    if constexpr (MODE == 1) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         gj[j] = lds4(fs + 16 * j + 4 * g);
@@ -453,28 +568,30 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
         bj[j] = lds4(fs + 2 * C + 16 * j + 4 * g);
       }
     }
-    Parts s = split<true>(S[0], S[1]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int t = 0; t < NBW; ++t) {
-      Parts next = s;
-      if (t + 1 < NBW) next = split<true>(S[2 * t + 2], S[2 * t + 3]);
-#pragma unroll
-      for (int term = 0; term < (MODE == 0 ? 6 : 3); ++term)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {                   // the smallest terms first
-          const auto& f = qf[t & 1];
-          if constexpr (MODE == 0) {
-            constexpr int qp[6] = {0, 2, 1, 1, 0, 0};
-            const bf16x8 sp = term == 0 ? s.l : term == 2 || term == 4 ? s.m : s.h;
-            O[i] = mfma16(f[qp[term]][i], sp, O[i]);
-          } else {
-            O[i] = mfma16(f[0][i], term == 0 ? s.l : term == 1 ? s.m : s.h, O[i]);
-          }
-        }
-      if (t + 2 < NBW) load_q(t + 2);
-      s = next;
+    if constexpr (WALK != STATES) {
+      Parts s = split<true>(S[0], S[1]);
       __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < NBW; ++t) {
+        Parts next = s;
+        if (t + 1 < NBW) next = split<true>(S[2 * t + 2], S[2 * t + 3]);
+#pragma unroll
+        for (int term = 0; term < (MODE == 0 ? 6 : 3); ++term)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {                   // the smallest terms first
+            const auto& f = qf[t & 1];
+            if constexpr (MODE == 0) {
+              constexpr int qp[6] = {0, 2, 1, 1, 0, 0};
+              const bf16x8 sp = term == 0 ? s.l : term == 2 || term == 4 ? s.m : s.h;
+              O[i] = mfma16(f[qp[term]][i], sp, O[i]);
+            } else {
+              O[i] = mfma16(f[0][i], term == 0 ? s.l : term == 1 ? s.m : s.h, O[i]);
+            }
+          }
+        if (t + 2 < NBW) load_q(t + 2);
+        s = next;
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     // The product of scores and values runs over the scores' masked half as well, where 0 x inf would reach the rows in front
     // of a value that is not finite: it is left out of the product, and its column is NaN from its token on.
@@ -482,7 +599,7 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
     int bad = C;
     const uint4 e = V.u;
     const auto ones = [](unsigned x) { return (x & 0x7f807f80u) + 0x00800080u; };     // bits 15, 31: an exponent of all ones
-    if (__any(((ones(e.x) | ones(e.y) | ones(e.z) | ones(e.w)) & 0x80008000u) != 0)) {
+    if (WALK != STATES && __any(((ones(e.x) | ones(e.y) | ones(e.z) | ones(e.w)) & 0x80008000u) != 0)) {
 #pragma unroll
       for (int i = 7; i >= 0; --i)
         if (!__builtin_isfinite((float)V.h[i])) {
@@ -492,7 +609,7 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
       bad = min(bad, __shfl_xor(bad, 16, 64));
       bad = min(bad, __shfl_xor(bad, 32, 64));
     }
-    if constexpr (MODE == 1) {
+    if constexpr (MODE == 1 && WALK != STATES) {
       bf16x8 kf[2][NB], qn[TI][NB];
       float gi[TI], li[TI];
 #pragma unroll
@@ -552,36 +669,41 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
 #pragma unroll
       for (int t = 0; t < 2 * NBW; ++t) dec[t] = lds4(fs + C * C + ch0 + 16 * t + 4 * g);
     }
-    if constexpr (HV == 2) {
+    if constexpr (HV == 2 && WALK != STATES) {
       given[((c & 1) * NWV + (wave ^ 4)) * 64 + lane] = hf ? O[0] : O[1];
       if (hf) O[0] = O[1];
     }
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (WALK != STATES) {
 #pragma unroll
-    for (int i = 0; i < TI; ++i) {
-      const Parts u = split(A[i][0], A[i][1]);
-      O[i] = mfma16(u.l, W.v, O[i]);
-      O[i] = mfma16(u.m, W.v, O[i]);
-      O[i] = mfma16(u.h, W.v, O[i]);
-    }
-    if (bad < C) {
+      for (int i = 0; i < TI; ++i) {
+        const Parts u = split(A[i][0], A[i][1]);
+        O[i] = mfma16(u.l, W.v, O[i]);
+        O[i] = mfma16(u.m, W.v, O[i]);
+        O[i] = mfma16(u.h, W.v, O[i]);
+      }
+      if (bad < C) {
 #pragma unroll
-      for (int i = 0; i < TI; ++i)
+        for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (16 * (i + hf) + 4 * g + r >= bad) O[i][r] = __builtin_nanf("");
-    }
+          for (int r = 0; r < 4; ++r)
+            if (16 * (i + hf) + 4 * g + r >= bad) O[i][r] = __builtin_nanf("");
+      }
 #pragma unroll
-    for (int i = 0; i < TI; ++i) {
-      f32x4 y;
+      for (int i = 0; i < TI; ++i) {
+        f32x4 y;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) y[r] = a.q_scale * O[i][r] + skip * (float)(HV == 2 && hf ? V.h[4 + r] : V.h[4 * i + r]);
-      if constexpr (HV == 2) mine = y;
-      else store_tile(c, i, y);
+        for (int r = 0; r < 4; ++r) y[r] = a.q_scale * O[i][r] + skip * (float)(HV == 2 && hf ? V.h[4 + r] : V.h[4 * i + r]);
+        if constexpr (HV == 2) mine = y;
+        else store_tile(c, i, y);
+      }
     }
     if constexpr (MODE == 0) {
 #pragma unroll
-      for (int t = 0; t < 2 * NBW; ++t) S[t] *= dec[t];
+      for (int t = 0; t < 2 * NBW; ++t) {
+        S[t] *= dec[t];
+        if (WALK == STATES) gone[t] *= dec[t];
+      }
 #pragma unroll
       for (int part = 2; part >= 0; --part) {
         bf16x8 nk[2 * NBW];
@@ -597,6 +719,7 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
       }
     } else {
       const float gc = fs[C - 1], lc = fs[2 * C - 1], d = pow2(gc);     // (G stands still past the run's end)
+      if (WALK == STATES) gone[0] *= d;
       f32x4 w[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j)
@@ -614,8 +737,21 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
     if (more) stash(c + 1);
     __syncthreads();                                    // chunk c + 1 is staged, chunk c has been read
   }
+  if constexpr (WALK == STATES) {
+    const int item = seg.item0 + seg.place;
+#pragma unroll
+    for (int t = 0; t < 2 * NBW; ++t) state_of(item)[64 * t] = S[t];
+    if (slab == 0 && (wave & 3) == 0 && col == 0) {
+      float* to = decays + (long long)item * a.H * NP;
+#pragma unroll
+      for (int t = 0; t < (MODE == 0 ? 2 * NBW : 1); ++t)
+        if (MODE == 0) *reinterpret_cast<f32x4*>(to + ch0 + 16 * t + 4 * g) = gone[t];
+        else if (lane == 0 && hf == 0) to[0] = gone[0][0];
+    }
+    return;
+  }
   if constexpr (HV == 2) store_tile(chunks - 1, 0, mine + a.q_scale * given[(((chunks - 1) & 1) * NWV + wave) * 64 + lane]);
-  if (sv >= 0 && pin) {
+  if (sv >= 0 && pin && (WALK == WHOLE || seg.place + 1 == seg.of)) {
     float* so = a.state + (long long)sv * a.state_stride + (long long)h * N * P + p;
 #pragma unroll
     for (int t = 0; t < 2 * NBW; ++t)
@@ -627,19 +763,28 @@ __global__ __launch_bounds__(NT * HV, 2) void decay_chunk_scan_kernel(DecayScanA
   }
 }
 
-template <int MODE, int NB, int HV>
-void launch_scan(const DecayScanArgs& a, hipStream_t s) {
+template <int MODE, int NB, int HV, int WALK>
+void launch_walk(const DecayScanArgs& a, hipStream_t s) {
   constexpr int lds = scan_lds(MODE, NB, HV);
   static const bool raised = [] {
     if (lds > 64 * 1024)
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&decay_chunk_scan_kernel<MODE, NB, HV>),
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&decay_chunk_scan_kernel<MODE, NB, HV, WALK>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     return true;
   }();
   (void)raised;
-  const int slabs = (a.P + 63) / 64;
-  const long long total = (long long)slabs * a.H * a.runs;
-  decay_chunk_scan_kernel<MODE, NB, HV><<<dim3(slabs, a.H, a.runs), NT * HV, lds, s>>>(a, walk_unit(total, slabs));
+  const int slabs = (a.P + 63) / 64, z = WALK == WHOLE ? a.runs : a.segments;
+  decay_chunk_scan_kernel<MODE, NB, HV, WALK><<<dim3(slabs, a.H, z), NT * HV, lds, s>>>(a, walk_unit((long long)slabs * a.H * z, slabs));
+}
+
+template <int MODE, int NB, int HV>
+void launch_scan(const DecayScanArgs& a, hipStream_t s) {
+  if (a.segments > a.runs) {
+    launch_walk<MODE, NB, HV, STATES>(a, s);
+    launch_walk<MODE, NB, HV, SEGMENTS>(a, s);
+  } else {
+    launch_walk<MODE, NB, HV, WHOLE>(a, s);
+  }
 }
 
 template <int MODE, int NB>
@@ -657,7 +802,7 @@ void launch_chunks(const DecayScanArgs& a, hipStream_t s) {
   }
   if constexpr (NB > 1) {
     // eight waves a workgroup where LDS (mode 0) or their number (at most one a CU) leaves one of them on a CU
-    if (MODE == 0 || (long long)((a.P + 63) / 64) * a.H * a.runs <= 256) return launch_scan<MODE, NB, 2>(a, s);
+    if (MODE == 0 || (long long)((a.P + 63) / 64) * a.H * std::max(a.runs, a.segments) <= 256) return launch_scan<MODE, NB, 2>(a, s);
   }
   launch_scan<MODE, NB, 1>(a, s);
 }
@@ -686,10 +831,17 @@ bool decay_chunk_takes(const DecayScanArgs& a) {
   return a.mode == 1 || (a.tiles && a.ntiles > 0 && a.ws && (uintptr_t)a.ws % 16 == 0);
 }
 
-// floats of the chunked form's scratch: a block per chunk and head (0: none)
-long long decay_chunk_scratch(int mode, long long T, long long runs, long long H, int N) {
-  if (mode != 0 || N > 128) return 0;
-  return (T / C + runs + 1) * H * (chunk_block(padded(N)) / 4);
+// floats of the chunked form's scratch: mode 0's blocks, then the segments' states and decays
+static long long block_floats(int mode, long long T, long long runs, long long H, int N) {
+  return mode == 0 ? (T / C + runs + 1) * H * (chunk_block(padded(N)) / 4) : 0;
+}
+long long decay_chunk_scratch(int mode, long long T, long long runs, long long H, int N, long long P) {
+  if (mode > 1 || N > 128) return 0;
+  return block_floats(mode, T, runs, H, N) + walk_segments(mode, T, runs, H, P) * H * ((P + 63) / 64 * 64 + 1) * padded(N);
+}
+void decay_chunk_segments(DecayScanArgs& a) {
+  a.segments = (uintptr_t)a.ws % 16 == 0 ? walk_segments(a.mode, a.T, a.runs, a.H, a.P) : 0;
+  a.seg = a.ws + block_floats(a.mode, a.T, a.runs, a.H, a.N);
 }
 
 void launch_decay_chunks(const DecayScanArgs& a, hipStream_t s) {

@@ -304,9 +304,12 @@ struct DecayScanArgs {
   const int* tiles;
   int ntiles;
   float* ws;
+  int segments;         // decay_chunk_segments: of the runs, all in all at most; 0: whole runs
+  float* seg;           // their states and decays
 };
 bool decay_chunk_takes(const DecayScanArgs& a);
-long long decay_chunk_scratch(int mode, long long T, long long runs, long long H, int N);
+long long decay_chunk_scratch(int mode, long long T, long long runs, long long H, int N, long long P);
+void decay_chunk_segments(DecayScanArgs& a);      // ws holds decay_chunk_scratch() floats: few runs are walked in segments
 void launch_decay_chunks(const DecayScanArgs& a, hipStream_t s);
 void launch_decay_scan(const DecayScanArgs& a, int f32, hipStream_t s);
 // One token a run in bf16 (cu_q null, T = runs; s.out is not written), with what follows the scan: out [T][H P] =

@@ -351,10 +351,12 @@ class LemunexLM:
                                None, P["dt_bias"], P["A_log"], P["D"], 1.0, m.heads, m.state, m.vdim, m.heads // m.groups,
                                cache.rec[i], b.prev_row, b.save_slot, self._cols(z, P, "z"), P["norm"], self.cfg.norm_eps, gy, ss):
                 return self._linear("ssm.out", gy, P["o"]), ss
-        y = self._buf("rec.y", (T, inner), torch.float32)
+        y, ws = self._buf("rec.y", (T, inner), torch.float32), None
+        if cu is not None and self.dtype == torch.bfloat16 and self.device.type != "cpu":
+            ws = self._buf("ssm.ws", (ops.decay_scratch(ops.DECAY_STEP_SIZE, T, runs, m.heads, m.state, m.vdim),), torch.float32)
         ops.decay_scan(ops.DECAY_STEP_SIZE, xc[:, inner + gn:], xc[:, inner:inner + gn], xc[:, :inner],
                        self._cols(z, P, "dt"), P["dt_bias"], P["A_log"], P["D"], 1.0, m.heads, m.state, m.vdim,
-                       m.heads // m.groups, cache.rec[i], cu, b.prev_row, b.save_slot, runs, y)
+                       m.heads // m.groups, cache.rec[i], cu, b.prev_row, b.save_slot, runs, y, ws=ws)
         gy = self._buf("rec.gy", (T, inner))
         ops.gated_group_norm(y, self._cols(z, P, "z"), P["norm"], self.cfg.norm_eps, inner // m.norm_groups, True, gy)
         return self._linear("ssm.out", gy, P["o"]), None

@@ -1117,7 +1117,8 @@ def decay_scan(mode, q, k, v, dz, dbias, dparam, skip, q_scale, H, N, P, hpg, st
     q / k [T, (H / hpg) N]: head h reads group h // hpg.  A run starts from state[slot] if prev_row[first] <= -2
     (slot = -(v + 2)), else from zero; it ends in state[save_slot[last]] (>= 0).  out fp32 [T, H, P].
     Prompt steps in bf16 walk their runs in chunks (csrc/kernels/decay_chunk.hip); the channel gate needs ``tiles`` (the
-    step's 64-row tiles) and ``ws`` (fp32, decay_ws_cols per row and head) for that, else it goes token by token."""
+    step's 64-row tiles) and ``ws`` (fp32, decay_ws_cols per row and head) for that, else it goes token by token.  With ``ws``
+    (decay_scratch floats; the step size without ``tiles``) few long runs are walked in segments at once."""
     if _gpu(out):
         dp = dparam if torch.is_tensor(dparam) else None
         return _hyb().decay_scan(int(mode), q, k, v, dz, dbias, dp, 0.0 if dp is not None else float(dparam), skip,
@@ -1155,6 +1156,7 @@ def decay_ws_cols(N: int) -> int:
     return 32 + 2 * N
 
 
+@functools.lru_cache(maxsize=1024)
 def decay_scratch(mode, T, runs, H, N, P) -> int:
     """Floats of scratch that decay_scan's chunked form of a step of T rows in ``runs`` runs works in."""
     return _hyb().decay_scratch(int(mode), int(T), int(runs), int(H), int(N), int(P))

@@ -225,3 +225,27 @@ def test_scratch_of_its_own_or_the_callers(gpu, H, N, P, G, lens):
     assert c.ws.numel() >= c.T * H * ops.decay_ws_cols(N)
     for got, want in zip(c.run(True), (out, state)):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("mode", [ops.DECAY_CHANNEL_GATE, ops.DECAY_STEP_SIZE])
+@pytest.mark.parametrize("shift", [0.0, -40.0])
+@pytest.mark.parametrize("H,N,P,G,lens", [(3, 128, 80, 3, [700]), (4, 64, 64, 2, [33, 1, 1000]), (2, 24, 16, 1, [257]), (8, 128, 256, 8, [1000, 64]),
+                                          (20, 128, 64, 4, [800, 31, 500])])
+def test_few_long_runs(gpu, mode, shift, H, N, P, G, lens):
+    """Runs cut into segments: ends of segments inside and at the end of runs, runs shorter than one, a state saved where it came from.
+    The bounds of whole runs: a segment's state passes the same roundings, one more for every segment."""
+    c = _Case(gpu, mode, H, N, P, G, lens)
+    c.dz = (c.dz.float() + shift).bfloat16()
+    c.ws = torch.full((ops.decay_scratch(mode, c.T, c.R, H, N, P),), float("nan"), device=gpu)
+    c.tiles = c.tiles if mode == ops.DECAY_CHANNEL_GATE else None
+    assert ops.decay_scratch(ops.DECAY_STEP_SIZE, c.T, c.R, H, N, P) > 0      # (segments' states: they are cut)
+    c.check()
+    for i in range(c.R):      # run i's state: from slot i + .. into the same slot
+        if i not in c.fresh:
+            c.save[c.save == c.R + i] = i
+    want, ends = c.exact()
+    out, _ = c.run(True)
+    assert float((out.double() - want).norm() / want.norm()) <= 2e-6
+    for i in range(c.R):
+        if i not in c.fresh:
+            assert float((c.state[i].double() - ends[i]).norm() / ends[i].norm()) <= 2e-6
