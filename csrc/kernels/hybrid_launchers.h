@@ -227,6 +227,9 @@ struct ExpertArgs {
 bool expert_linear_mfma(const ExpertArgs& a, int f32);
 const std::array<int, 4>& expert_walk_widths();      // widths K that the walk is built for
 int expert_linear_form(const ExpertArgs& a, bool mfma, int cus);      // (sizes only)
+// one expert of all rows, gated (E 1, no offsets); false: another path is ahead at these sizes
+bool dense_glu_pays(long long M, long long N, long long K, int cus);
+bool launch_dense_glu(const ExpertArgs& a, hipStream_t s);
 // impl -1: by shape; 0 all shapes, 1 weight stream, 2 / 3 tiles, 4 weight walk.  Returns the form used.
 int launch_expert_linear(const ExpertArgs& a, int f32, int impl, hipStream_t s);
 

@@ -701,7 +701,7 @@ __global__ __launch_bounds__(512, 1) void expert_persist_kernel(ExpertArgs a) {
 
   // ---- this workgroup's tiles.  Whole and half row tiles of an expert; lane l: those of all experts up to its share of them
   auto segment = [&](int e, int& r0, int& r1, int& w, int& h) {
-    r0 = a.offsets[e], r1 = max(r0, min(a.offsets[e + 1], a.R));
+    r0 = a.offsets ? a.offsets[e] : 0, r1 = a.offsets ? max(r0, min(a.offsets[e + 1], a.R)) : a.R;      // (no offsets: all rows one's)
     const int left = (r1 - r0) & 255;
     w = (r1 - r0) / 256 + (left > 128), h = left > 0 && left <= 128;
   };
@@ -1032,6 +1032,30 @@ static bool persists(const ExpertArgs& a, int per, int cus) {
   const long long tiles = (a.glu ? (a.N + 127) / 128 : cols) * a.E * std::max(1, (per + 255) / 256);
   if (a.K < 1024) return per >= 1024 && a.N >= 1024 && tiles >= (a.glu ? 1 : 2) * cus;
   return per >= 128 && 10 * tiles >= 3 * cus && (!a.glu || 10 * full <= 7 * cus || full >= cus);
+}
+
+// A dense gated projection of many rows is one expert's: rounds of tiles that the XCDs' workgroups take (a half one 5 / 9 of a whole
+// one), as the kernel deals them out.  Its tiles run at 1.2 to 1.3 PFLOP/s and save the launch that multiplies; against the library's
+// product and that launch it is ahead where its rounds are full to 0.6, from 4096 wide on, where the library's are better, to 0.8.
+// us, library / tiles (rounds' fill): 8192 x 2048 at 400 rows 38.9 / 33.8 (0.70), 513 43.1 / 47.4 (0.50), 600 45.5 / 46.8 (0.59), 700 49.9 /
+// 47.8 (0.68), 1000 64.9 / 56.2, 1530 99 / 84.5, 2600 189 / 153, 8100 462 / 444; 5632 x 2048 at 800 42.3 / 46.5 (0.54), 1000 58 / 47
+// (0.67), 8100 404 / 305; 1536 x 6144 at 1800 69.1 / 69.7 (0.59), 3000 102 / 117 (0.55); 14336 x 4096 at 400 103 / 107 (0.68), 700 158 / 160
+// (0.77), 1000 204 / 204 (0.85), 2600 586 / 506, 8100 1399 / 1412; 11008 x 4096 at 1530 314 / 236, 8100 1229 / 1104.
+bool dense_glu_pays(long long M, long long N, long long K, int cus) {
+  if (M <= 256 || N < 256 || K < 1024) return false;
+  const long long cols = (N + 127) / 128, left = M % 256, wgs = std::max(1, cus / 8);
+  const long long w = (cols * (M / 256 + (left > 128)) + 7) / 8, h = left > 0 && left <= 128 ? (cols + 7) / 8 : 0;      // an XCD's, whole and half
+  const long long over = w % wgs, halves = (over + h + wgs - 1) / wgs, uncut = over ? 9 + 5 * (halves - 1) : 5 * halves;
+  const long long ninths = 9 * (w / wgs) + (over ? std::min(uncut, 5 * ((2 * over + h + wgs - 1) / wgs)) : uncut);
+  // fill: M cols / 256 whole tiles' work over 8 wgs workgroups, against the rounds
+  return 9 * 10 * M * cols >= (K >= 4096 ? 8 : 6) * 256 * 8 * wgs * ninths;
+}
+
+bool launch_dense_glu(const ExpertArgs& a, hipStream_t s) {
+  const int cus = cu_count();
+  if (!expert_linear_mfma(a, 0) || !persist_fits(a) || !dense_glu_pays(a.R, a.N, a.K, cus)) return false;
+  launch_persist<EPI_GLU>(a, cus, s);
+  return true;
 }
 
 // The form that a call takes by its sizes: 0 all shapes, 1 weight stream, 2 / 3 tiles of 128 / 256, 4 the walk.

@@ -681,7 +681,10 @@ def linear_glu(x, w, out, ws) -> bool:
     if _few(x, w, out):
         row_linear(x, w, out, glu=True)
         return True
-    return ws is not None and _mid(x, w, out, True) and w.shape[0] == 2 * out.shape[1] and mid_linear(x, w, out, ws, True)
+    if ws is not None and _mid(x, w, out, True) and w.shape[0] == 2 * out.shape[1] and mid_linear(x, w, out, ws, True):
+        return True
+    return (x.dim() == 2 and x.shape[0] > MID_ROWS and _own_linear(x, w, out) and x.is_contiguous() and out.is_contiguous()
+            and out.dtype == torch.bfloat16 and w.shape[0] == 2 * out.shape[1] and _hyb().linear_glu_wide(x, w, out))
 
 
 def row_linear(x, w, out, relu2: bool = False, glu: bool = False) -> None:

@@ -74,3 +74,13 @@ def test_sizes_that_are_none_are_refused():
     for bad in ((0, 16, 64, 64), (4, 0, 64, 64), (4, 16, 0, 64), (4, 16, 64, 0), (4, 16, 1 << 31, 64)):
         with pytest.raises(RuntimeError, match="sizes"):
             form(*bad, rows=4)
+
+
+def test_dense_gated_projections_need_full_rounds():
+    """256 CUs; whole tiles of 256 rows x 128 pairs, half ones 5 / 9 of their time: 0.6 of a round's work to be done, from 4096 wide 0.8."""
+    pays = ops._hyb().dense_glu_pays
+    assert [pays(M, 8192, 2048) for M in (256, 320, 400, 513, 600, 700, 1530, 8100)] == [False, False, True, False, False, True, True, True]
+    assert [pays(M, 5632, 2048) for M in (700, 800, 1000)] == [False, False, True]
+    assert [pays(M, 14336, 4096) for M in (400, 700, 1000, 1100)] == [False, False, True, True]
+    assert [pays(4000, 8192, K) for K in (960, 1024)] == [False, True] and not pays(4000, 255, 2048)
+    assert pays(1600, 2048, 2048, 64) and pays(400, 2048, 2048, 64) == pays(400, 8192, 2048, 256)

@@ -293,3 +293,25 @@ def test_choices_among_infinite_logits(R):
     w = torch.empty(R * k, device="cuda")
     ops.route_topk(x, Wr, bias.cuda(), k, ids, w, off, dst, src)
     assert ids.view(R, k).tolist() == [[7, 1, 2, 3]] * R and w.view(R, k).tolist() == [[1.0, 0.0, 0.0, 0.0]] * R
+
+
+@pytest.mark.parametrize("M,N,K", [(2817, 1024, 1024), (1280, 2180, 1088), (400, 8192, 2048), (1025, 8192, 2048)])
+def test_dense_gated_projection(M, N, K):
+    """linear_glu of many rows: one expert's persistent tiles.  The gated product's bound from above."""
+    torch.manual_seed(M)
+    x, W = torch.randn(M, K, device="cuda").to(BF16), (torch.randn(2 * N, K, device="cuda") * K ** -0.5).to(BF16)
+    out = torch.full((M + 1, N), 7.0, dtype=BF16, device="cuda")
+    with torch.no_grad():
+        assert ops.linear_glu(x, W, out[:M], None)
+        p = x.double() @ W.double().t()
+        g, u = p[:, :N], p[:, N:]
+        want = g / (1 + torch.exp(-g)) * u
+        eps = 4 * K ** 0.5 * 2.0 ** -24 * x.double().norm(dim=1).max() * W.double().norm(dim=1).max()
+        bound = 2.0 ** -8 * want.abs() + 1.1 * eps * (g.abs() + u.abs()) + 2.0 ** -20 * want.abs() + 1e-30
+        assert ((out[:M].double() - want).abs() <= bound).all() and (out[M] == 7.0).all()
+        wide = torch.empty(M, K + 64, device="cuda", dtype=BF16)
+        assert not ops.linear_glu(wide[:, :K], W, out[:M], None)                    # rows of x apart
+        assert not ops.linear_glu(x, W, torch.empty(M, N + 8, device="cuda", dtype=BF16)[:, :N], None)
+        assert not ops.linear_glu(x[:300], W[:512], torch.empty(300, 256, device="cuda", dtype=BF16), None)      # the library's sizes
+    x.requires_grad_(True)
+    assert not ops.linear_glu(x, W, out[:M], None)
