@@ -975,17 +975,17 @@ int64_t expert_linear(const Tensor& x, const OptTensor& src, const Tensor& W, co
   return launch_expert_linear(a, f32, (int)impl, cur_stream(x));
 }
 
-// out = silu(gate) * up of x . w^T, w [2 N][K]'s rows [gate | up], many rows in bf16; false: another path is ahead at these sizes
-bool linear_glu_wide(const Tensor& x, const Tensor& w, Tensor& out) {
+// out = silu(gate) * up of x . w^T, w [2 N][K]'s rows [gate | up] or by eights in turn, many rows in bf16; false: another path is ahead
+bool linear_glu_wide(const Tensor& x, const Tensor& w, Tensor& out, bool eights) {
   same_act(x, 0, "x");
   same_act(w, 0, "w");
   same_act(out, 0, "out");
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2 && w.size(1) == x.size(1) && w.size(0) == 2 * out.size(1) &&
-                  out.size(0) == x.size(0) && std::max({x.size(0), w.size(0), w.size(1)}) < (1LL << 30),
+                  out.size(0) == x.size(0) && (!eights || out.size(1) % 8 == 0) && std::max({x.size(0), w.size(0), w.size(1)}) < (1LL << 30),
               "linear_glu_wide: shapes");
   ExpertArgs a{};
   a.x = x.data_ptr(), a.W = w.data_ptr(), a.y = out.data_ptr();
-  a.R = a.xrows = (int)x.size(0), a.E = 1, a.N = (int)out.size(1), a.K = (int)w.size(1), a.glu = 1;
+  a.R = a.xrows = (int)x.size(0), a.E = 1, a.N = (int)out.size(1), a.K = (int)w.size(1), a.glu = 1, a.eights = eights;
   const at::OptionalDeviceGuard g(x.device());
   return launch_dense_glu(a, cur_stream(x));
 }
@@ -1589,7 +1589,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
       "expert_linear(Tensor x, Tensor? src, Tensor W, Tensor offsets, Tensor(a!) y, bool relu2, int impl=-1, bool glu=False) -> int",
       &expert_linear);
   m.def("expert_walk_widths() -> int[]", &walk_widths);
-  m.def("linear_glu_wide(Tensor x, Tensor w, Tensor(a!) out) -> bool", &linear_glu_wide);
+  m.def("linear_glu_wide(Tensor x, Tensor w, Tensor(a!) out, bool eights=False) -> bool", &linear_glu_wide);
   m.def("dense_glu_pays(int M, int N, int K, int cus=256) -> bool",
         [](int64_t M, int64_t N, int64_t K, int64_t cus) { return dense_glu_pays(M, N, K, (int)cus); });
   m.def("expert_linear_choice(int R, int E, int N, int K, int xrows, bool glu, bool f32_out, int cus=256) -> int", &expert_linear_choice);

@@ -222,6 +222,7 @@ struct ExpertArgs {
   int xrows;      // rows of x
   int glu;        // W [E][2 N][K] holds [gate | up] rows, y = silu(gate) * up
   int f32_out;    // y fp32 (neither relu2 nor glu)
+  int eights;     // launch_dense_glu: W's rows are 8 gate rows, the 8 up rows of the same outputs, the next 8 ..
 };
 // the MFMA forms take it (the only ones with glu and f32_out)
 bool expert_linear_mfma(const ExpertArgs& a, int f32);

@@ -761,13 +761,15 @@ __global__ __launch_bounds__(512, 1) void expert_persist_kernel(ExpertArgs a) {
       aoff[i] = (a.src ? a.src[p] : p) * K * 2 + 16 * lch;
     }
     const int up = EPI == EPI_GLU ? (lrow >> 5) * N : 0;
-    boff = (t.n0 + (EPI == EPI_GLU ? lrow & 31 : lrow) + up) * K * 2 + 16 * lch;
-    blast = (N - 1 + up) * K * 2 + 16 * lch;
+    int row = t.n0 + (EPI == EPI_GLU ? lrow & 31 : lrow) + up, last = N - 1 + up;
+    if (EPI == EPI_GLU && a.eights) row = 2 * t.n0 + 2 * (lrow & 24) + (lrow & 7) + 8 * (lrow >> 5), last = 2 * N - 1;
+    boff = row * K * 2 + 16 * lch;
+    blast = last * K * 2 + 16 * lch;
     const long long wrows = (EPI == EPI_GLU ? 2LL : 1LL) * N;
     wbuf = buffer_words(reinterpret_cast<const bf16*>(a.W) + t.e * wrows * K, wrows * K * 2);
   };
   const unsigned int lds0 = lds_address(smem) + wave * 1024;
-  const int wstep = OUT / 4 * K * 2;
+  const int wstep = OUT / 4 * (EPI == EPI_GLU && a.eights ? 2 : 1) * K * 2;
   unsigned int afill = 0, bfill = 0;      // the buffers to fill
   auto load_a = [&](int i) {
     if (i < 2 || !ahalf) direct_buffer_load16(xbuf, aoff[i], kx, lds0 + afill + 8192 * i);
@@ -1051,6 +1053,8 @@ bool dense_glu_pays(long long M, long long N, long long K, int cus) {
   return 9 * 10 * M * cols >= (K >= 4096 ? 8 : 6) * 256 * 8 * wgs * ninths;
 }
 
+// (weights whose rows come by eights, in prompt steps of four layers, us: 8192 x 2048, 420 rows 554 -> 510, 1500 1146 -> 1085, 8000 3694 ->
+// 3542; 14336 x 4096, 1100 rows 2172 -> 2113, 2600 4512 -> 4186, 8100 10944 -> 10881)
 bool launch_dense_glu(const ExpertArgs& a, hipStream_t s) {
   const int cus = cu_count();
   if (!expert_linear_mfma(a, 0) || !persist_fits(a) || !dense_glu_pays(a.R, a.N, a.K, cus)) return false;

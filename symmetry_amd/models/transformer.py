@@ -627,12 +627,12 @@ class TransformerLM:
                 continue
             else:
                 ops.add_rms_norm(o, resid, w.layer(i, "ln2"), eps, x)
+                w_gu = self.dgw[(i, "w_gu")] if pg_gu is not None else self._row_major(i, "w_gu")
+                act = None if w_gu is None else self._buf("act", (T, w_gu.shape[0] // 2), torch.bfloat16)
                 if pg_gu is not None:
                     # gate_up + SwiGLU in one prefill-GEMM launch on the preshuffled copy (no [T, 2F] intermediate)
-                    w_gu = self.dgw[(i, "w_gu")]
-                    act = self._buf("act", (T, w_gu.shape[0] // 2), torch.bfloat16)
                     ops.pg_swiglu(x, w_gu, None, eps, act, pg_gu)
-                else:
+                elif not ops.linear_swiglu(x, w_gu, act):  # (... or on the row-major weight, many rows)
                     gu = self._linear("gu", x, self._row_major(i, "w_gu"), wshuf=self._shuf(i, "w_gu"))
                     F = gu.shape[-1] // 2
                     act = self._buf("act", (T, F), torch.bfloat16)

@@ -683,8 +683,18 @@ def linear_glu(x, w, out, ws) -> bool:
         return True
     if ws is not None and _mid(x, w, out, True) and w.shape[0] == 2 * out.shape[1] and mid_linear(x, w, out, ws, True):
         return True
+    return _wide_glu(x, w, out, False)
+
+
+def _wide_glu(x, w, out, eights: bool) -> bool:
     return (x.dim() == 2 and x.shape[0] > MID_ROWS and _own_linear(x, w, out) and x.is_contiguous() and out.is_contiguous()
-            and out.dtype == torch.bfloat16 and w.shape[0] == 2 * out.shape[1] and _hyb().linear_glu_wide(x, w, out))
+            and out.dtype == torch.bfloat16 and w.shape[0] == 2 * out.shape[1] and (not eights or out.shape[1] % 8 == 0)
+            and _hyb().linear_glu_wide(x, w, out, eights))
+
+
+def linear_swiglu(x, w, out) -> bool:
+    """linear_glu of many rows for w in the decode layout (8 gate rows, the 8 up rows of the same outputs, the next 8 ..)."""
+    return w is not None and not _traced(x, w, out) and _wide_glu(x, w, out, True)
 
 
 def row_linear(x, w, out, relu2: bool = False, glu: bool = False) -> None:

@@ -309,6 +309,10 @@ def test_dense_gated_projection(M, N, K):
         eps = 4 * K ** 0.5 * 2.0 ** -24 * x.double().norm(dim=1).max() * W.double().norm(dim=1).max()
         bound = 2.0 ** -8 * want.abs() + 1.1 * eps * (g.abs() + u.abs()) + 2.0 ** -20 * want.abs() + 1e-30
         assert ((out[:M].double() - want).abs() <= bound).all() and (out[M] == 7.0).all()
+        turned = torch.full_like(out, 7.0)                                          # eight gate rows, the eight up rows, the next ..
+        eights = W.view(2, -1, 8, K).transpose(0, 1).reshape(2 * N, K) if N % 8 == 0 else W
+        assert ops.linear_swiglu(x, eights, turned[:M]) == (N % 8 == 0)
+        assert N % 8 or torch.equal(turned, out)
         wide = torch.empty(M, K + 64, device="cuda", dtype=BF16)
         assert not ops.linear_glu(wide[:, :K], W, out[:M], None)                    # rows of x apart
         assert not ops.linear_glu(x, W, torch.empty(M, N + 8, device="cuda", dtype=BF16)[:, :N], None)
