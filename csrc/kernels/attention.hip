@@ -372,6 +372,8 @@ SYM_DEV f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
+
 SYM_DEV float xhalf_max(float v) {  // max with the lane 32 apart (same query column, other key half)
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
@@ -390,28 +392,17 @@ constexpr float kRescaleThr = 8.f;  // T13 threshold, log2 units
 // Same workgroup / wave decomposition and operand tricks as described above, restructured so
 // that a wave's VALU work hides under its own MFMAs: the online-softmax update is per 32-key subtile
 // and the loop body for subtile j is
-//     [rescale decision for j]  ->  S(j+1) = K . Q^T MFMAs  ||  exp2 / bf16 pack / row-sum of S(j)
-//                               ->  P(j) . V MFMAs         ||  row max of S(j+1)
-// (an MFMA holds the wave's issue for 8 of its 32 cycles, so independent VALU placed between MFMAs
-// runs in the remaining slots).
+//     [rescale decision for j]  ->  S(j+1) = K . Q^T MFMAs  ||  second half of P(j): exp2, bf16, sum
+//                               ->  P(j) . V MFMAs          ||  row max of S(j+1), first half of P(j+1)
 // Masks apply only to the <= 2 subtiles of a wave that touch the causal diagonal / context end (a
-// uniform branch).  K/V tiles are TRIPLE-buffered in LDS (107.5 KB, one workgroup per CU at this
-// register budget anyway): tile t+1 is resident while tile t is consumed, so S(j+1) can cross a tile
-// boundary, and tile t+2's global loads are in flight for a whole iteration.
+// uniform branch).  Three K/V tiles in LDS (96 KB, one workgroup per CU at this register budget anyway),
+// filled by direct loads: tile t+1 is resident while tile t is consumed, so S(j+1) can cross a tile
+// boundary, and tile t+2 loads for a whole iteration.  16-byte chunk i of a K row r is stored at i ^ (r & 15),
+// of a V^T row at i ^ ((r >> 1) & 7): operand reads meet no bank twice.
+// What bounds it is power: matrix cores busy 0.51 of the cycles, at 1.8 GHz (a large product: 0.82 at 1.7).  So what counts is
+// work beside the products; with the tiles through registers (addresses, waits, LDS stores: a fifth of the time) -> so, us: 32 heads,
+// one prompt of 7900 tokens 577 -> 542, 8 of 1012 131 -> 128, 16 heads, 3 of 1000 behind 1000 82 -> 76.
 // ---------------------------------------------------------------------------------------------
-SYM_DEV void s_subtile(const bf16* __restrict__ sk, const bf16x8 (&qf)[8], f32x16& acc) {
-  const int lane = threadIdx.x & 63;
-  const int r = lane & 31, hh = lane >> 5;
-  const int pr = (r & 3) | ((r & 4) << 1) | ((r & 8) >> 1) | (r & 16);  // bits 2 <-> 3
-  const bf16* kr = sk + pr * KST + 64 * hh;
-  bf16x8 kf[8];
-#pragma unroll
-  for (int kk = 0; kk < 8; ++kk) kf[kk] = *reinterpret_cast<const bf16x8*>(kr + 8 * kk);
-  acc = f32x16{};
-#pragma unroll
-  for (int kk = 0; kk < 8; ++kk) acc = mfma32(kf[kk], qf[kk], acc);
-}
-
 SYM_DEV void mask_subtile(f32x16& s, int kbase, int mypos) {
   const int hh = (threadIdx.x & 63) >> 5;
   const int lim = mypos - kbase - 8 * hh;  // register i holds key kbase + 16 (i >> 3) + 8 hh + (i & 7)
@@ -434,9 +425,8 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_m32p_kernel(
     const int* __restrict__ tiles, bf16* __restrict__ out, int Hq, int Hkv, int bs_shift, int max_blocks,
     float scale_log2) {
   const int BS = 1 << bs_shift, bs_mask = BS - 1;  // power-of-two blocks: no integer division per tile
-  constexpr int HPW = 4, KROWS = 32, VROWS = 64;
-  constexpr int TILE_ELEMS = 64 * KST + D * VST;  // one K tile + one V^T tile
-  __shared__ bf16 smem[3 * TILE_ELEMS];
+  constexpr int HPW = 4, KB = 64 * 256, TB = KB + 128 * 128;  // bytes of a K tile, of a K and a V^T tile
+  __shared__ __attribute__((aligned(1024))) char smem[3 * TB];
   const int tile = blockIdx.y, kvh = blockIdx.x;  // tiles arrive heaviest first (engine order)
   const int G = Hq / Hkv;
   const int lane = threadIdx.x & 63;
@@ -459,7 +449,43 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_m32p_kernel(
   const int myrow = row0 + c;
   const bool row_ok = myrow < qlen;
   const int mypos = row_ok ? pos0 + myrow : ctx - 1;  // rows past the prompt attend like the last one
+  const int last = ctx - 1;
+  const int ntiles = (kend_wg + 63) / 64;
 
+  // A wave's four direct loads of a tile: K rows 8 wid .. + 7 (two of 4 rows), V^T rows 16 wid .. + 15 (two of 8); the chunk that a lane
+  // takes from its row stands at its own place.  A group of 8 keys is in one block.  Its block's id, a K and a V one a lane, is
+  // fetched a tile ahead.  K rows past the context are whatever the block holds (their scores are masked), V's chunks there are the
+  // context's last (finite: the cache is zero-initialised and only ever written with finite K/V).
+  const int krow = 8 * wid + (lane >> 4), vrow = 16 * wid + (lane >> 3);
+  const char* const kbase = reinterpret_cast<const char*>(k_cache + (long long)kvh * BS * D);
+  const char* const vbase = reinterpret_cast<const char*>(v_cache + (long long)kvh * BS * D + (long long)vrow * BS);
+  const unsigned bbytes = (unsigned)(Hkv * BS * D) * 2;
+  const int kch0 = 16 * ((lane & 15) ^ (krow & 15)), kch1 = 16 * ((lane & 15) ^ ((krow + 4) & 15));
+  const int vch0 = (lane & 7) ^ ((vrow >> 1) & 7), vch1 = (lane & 7) ^ (((vrow + 8) >> 1) & 7);
+  const unsigned lds0 = lds_address(smem) + wid * 2048;
+  struct Ids { int k, v0, v1; };
+  auto fetch_ids = [&](int t) {
+    const int t0 = 64 * t;
+    return Ids{bt[min(t0 + 8 * wid, last) >> bs_shift], bt[min(t0 + 8 * vch0, last) >> bs_shift], bt[min(t0 + 8 * vch1, last) >> bs_shift]};
+  };
+  auto issue = [&](int t, int buf, const Ids& id) {
+    const int t0 = 64 * t, at = lds0 + buf * TB;
+    const char* kb = kbase + (size_t)(unsigned)id.k * bbytes + (((t0 + krow) & bs_mask) << 8);
+    direct_load16(kb + kch0, at);
+    direct_load16(kb + 1024 + kch1, at + 1024);
+    const int v0 = min(t0 + 8 * vch0, last & ~7), v1 = min(t0 + 8 * vch1, last & ~7);
+    direct_load16(vbase + (size_t)(unsigned)id.v0 * bbytes + 2 * (v0 & bs_mask), at + KB);
+    direct_load16(vbase + (size_t)(unsigned)id.v1 * bbytes + 2 * (v1 & bs_mask) + 16 * BS, at + KB + 1024);
+  };
+
+  // prologue: tiles 0 and 1 (one memory round trip), the queries behind them
+  Ids ids{};
+  if (ntiles > 0) {
+    const Ids i0 = fetch_ids(0), i1 = fetch_ids(ntiles > 1 ? 1 : 0);
+    if (ntiles > 2) ids = fetch_ids(2);
+    issue(0, 0, i0);
+    if (ntiles > 1) issue(1, 1, i1);
+  }
   bf16x8 qf[8];
   if (row_ok) {
     const bf16* qp = q + ((long long)(qstart + myrow) * Hq + head) * D + 64 * hh;
@@ -473,122 +499,121 @@ __global__ __launch_bounds__(512, 2) void attn_prefill_m32p_kernel(
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = f32x16{};
   float m = -INFINITY, lsum = 0.f;
-
-  // Cooperative tile staging: 2 x 16 B of K and of V per thread.  The paged-cache block ids of a tile are
-  // fetched one tile AHEAD of its K/V loads, so issuing those loads never waits on a block-table read.
-  // Keys past the context read the block of the last key (finite: the cache is zero-initialised and only
-  // ever written with finite K/V; masked anyway).
-  const int ck = threadIdx.x >> 4, pk = (threadIdx.x & 15) * 8;
-  const int dv = threadIdx.x >> 3, tv8 = 8 * (threadIdx.x & 7);
-  const long long kvoff = (long long)kvh * BS * D;
-  const size_t bstride = (size_t)Hkv * BS * D;
-  const int last = ctx - 1;
-  const int ntiles = (kend_wg + 63) / 64;
-  struct Ids { int k0, k1, v; };
-  struct Stage { uint4 k0, k1, v0, v1; };
-  auto fetch_ids = [&](int t0) {
-    return Ids{bt[min(t0 + ck, last) >> bs_shift], bt[min(t0 + ck + KROWS, last) >> bs_shift],
-               bt[min(t0 + tv8, last) >> bs_shift]};
-  };
-  // per-thread constant parts of the K / V addresses (elements)
-  const bf16* kbase = k_cache + kvoff + pk;
-  const bf16* vbase = v_cache + kvoff + (long long)dv * BS;
-  auto issue = [&](int t0, const Ids& id) {
-    const int k0 = min(t0 + ck, last), k1 = min(t0 + ck + KROWS, last), v0 = min(t0 + tv8, last & ~7);
-    Stage st;
-    st.k0 = *reinterpret_cast<const uint4*>(kbase + (size_t)(unsigned)id.k0 * bstride + ((k0 & bs_mask) << 7));
-    st.k1 = *reinterpret_cast<const uint4*>(kbase + (size_t)(unsigned)id.k1 * bstride + ((k1 & bs_mask) << 7));
-    const bf16* vb = vbase + (size_t)(unsigned)id.v * bstride + (v0 & bs_mask);
-    st.v0 = *reinterpret_cast<const uint4*>(vb);
-    st.v1 = *reinterpret_cast<const uint4*>(vb + VROWS * BS);
-    return st;
-  };
-  auto store = [&](int t, const Stage& st) {
-    bf16* sk = smem + (t % 3) * TILE_ELEMS;
-    bf16* sv = sk + 64 * KST;
-    *reinterpret_cast<uint4*>(sk + ck * KST + pk) = st.k0;
-    *reinterpret_cast<uint4*>(sk + (ck + KROWS) * KST + pk) = st.k1;
-    *reinterpret_cast<uint4*>(sv + dv * VST + tv8) = st.v0;
-    *reinterpret_cast<uint4*>(sv + (dv + VROWS) * VST + tv8) = st.v1;
-  };
-
-  // prologue: tiles 0 and 1 loaded together (one memory round trip), tile 2's loads in flight
-  Stage stg;
-  Ids ids;
-  if (ntiles > 0) {
-    const Ids i0 = fetch_ids(0), i1 = fetch_ids(ntiles > 1 ? 64 : 0);
-    stg = issue(0, i0);
-    Stage s1;
-    if (ntiles > 1) s1 = issue(64, i1);
-    if (ntiles > 2) ids = fetch_ids(128);
-    store(0, stg);
-    if (ntiles > 1) store(1, s1);
-  }
+  // (the queries have arrived as well: unsaid, every S product of the loop waits for them anew, which by then is for the tiles in flight)
+  wait_direct_loads();
   __syncthreads();
-  if (ntiles > 2) {
-    stg = issue(128, ids);
-    if (ntiles > 3) ids = fetch_ids(192);
-  }
 
+  // LDS operand addresses: K row pr + 32 i (i: subtile of the tile), chunk 8 hh + kk; V^T row c + 32 dt, chunk hh + 2 x
+  const int pr = (c & 3) | ((c & 4) << 1) | ((c & 8) >> 1) | (c & 16);  // bits 2 <-> 3
+  int kx[8], vx[4];
+  const unsigned base = lds_address(smem);
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) kx[kk] = base + pr * 256 + 16 * ((8 * hh + kk) ^ (pr & 15));
+#pragma unroll
+  for (int x = 0; x < 4; ++x) vx[x] = base + KB + c * 128 + 16 * ((hh + 2 * x) ^ ((c >> 1) & 7));
+  auto operand = [&](int at) { return *reinterpret_cast<const lds_bf16x8*>((unsigned)at); };
+
+  // The 16 products of a step, 8 of S(j + 1) and 8 of P(j) . V, take their LDS operands from a ring that is read RING products ahead,
+  // over the ends of steps (the next K subtile is resident).  The vector work stands between them, about as much at each: the second
+  // half of P(j), the row max of S(j + 1), and with the running maximum as it is the first half of P(j + 1), which is formed anew
+  // where the next step masks or rescales.
+  constexpr int RING = 4;
+  bf16x8 f[RING];
   f32x16 sa, sb;  // scores of the current / next subtile (named: static register allocation)
-  float tmax = -INFINITY;
+  Pack8 first;      // P(j)'s first half
+  first.u = make_uint4(0, 0, 0, 0);
+  float tmax = -INFINITY, fsum = 0.f;
+  sa = f32x16{};
   if (nsub > 0) {
-    s_subtile(smem, qf, sa);
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) sa = mfma32(operand(kx[kk]), qf[kk], sa);
     tmax = subtile_max(sa, scale_log2);
+#pragma unroll
+    for (int n = 0; n < RING; ++n) f[n] = operand(kx[n] + 8192);
   }
-
-  // one subtile step: j = 2 it + ST, current scores in SC, next into SN
-#define SUBTILE_STEP(ST, SC, SN)                                                                          \
-  do {                                                                                                    \
-    const int j = 2 * it + (ST);                                                                          \
-    if (j < nsub) {                                                                                       \
-      if (32 * j + 31 > minpos_w) { /* diagonal / context-end subtile: mask, then its true max */         \
-        mask_subtile(SC, 32 * j, mypos);                                                                  \
-        tmax = subtile_max(SC, scale_log2);                                                               \
-      }                                                                                                   \
-      if (!__all(tmax <= m + kRescaleThr)) {                                                              \
-        const float mn = fmaxf(m, tmax);                                                                  \
-        const float alpha = __builtin_amdgcn_exp2f(m - mn); /* first subtile: m = -inf, alpha = 0 */      \
-        m = mn;                                                                                           \
-        lsum *= alpha;                                                                                    \
-        _Pragma("unroll") for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;                                  \
-      }                                                                                                   \
-      /* branch-free from here: S(j+1) unconditionally (past the wave's last subtile it is an unused */   \
-      /* stale-LDS product) so the exps of S(j) interleave with its MFMAs, and S(j+1)'s row max with */   \
-      /* the P.V MFMAs (an upper bound until a masked subtile recomputes it above) */                    \
-      s_subtile((ST) == 0 ? cur_k + 32 * KST : nxt_k, qf, SN);                                            \
-      Pack8 pf[2];                                                                                        \
-      float psum = 0.f;                                                                                   \
-      _Pragma("unroll") for (int i = 0; i < 16; ++i) {                                                    \
-        const float p = __builtin_amdgcn_exp2f(fmaf(SC[i], scale_log2, -m));                              \
-        psum += p;                                                                                        \
-        pf[i >> 3].h[i & 7] = (bf16)p;                                                                    \
-      }                                                                                                   \
-      lsum += psum;                                                                                       \
-      _Pragma("unroll") for (int ks = 0; ks < 2; ++ks)                                                    \
-        _Pragma("unroll") for (int dt = 0; dt < 4; ++dt) {                                                \
-          const bf16x8 vf = *reinterpret_cast<const bf16x8*>(cur_v + (32 * dt + c) * VST + 32 * (ST) +    \
-                                                             16 * ks + 8 * hh);                           \
-          o[dt] = mfma32(vf, pf[ks].v, o[dt]);                                                            \
-        }                                                                                                 \
-      tmax = subtile_max(SN, scale_log2);                                                                 \
-    }                                                                                                     \
-  } while (0)
-
-  for (int it = 0; it < ntiles; ++it) {
-    const bf16* cur_k = smem + (it % 3) * TILE_ELEMS;
-    const bf16* cur_v = cur_k + 64 * KST;
-    const bf16* nxt_k = smem + ((it + 1) % 3) * TILE_ELEMS;
-    SUBTILE_STEP(0, sa, sb);
-    SUBTILE_STEP(1, sb, sa);
-    if (it + 2 < ntiles) store(it + 2, stg);
-    __syncthreads();
-    if (it + 3 < ntiles) {
-      stg = issue(64 * (it + 3), ids);
-      if (it + 4 < ntiles) ids = fetch_ids(64 * (it + 4));
+  auto prob = [&](float s) { return __builtin_amdgcn_exp2f(fmaf(s, scale_log2, -m)); };
+  // step j = 2 it + ST: scores of subtile j in sc, of the next one into sn; to_next: from this tile's buffer to the next one's
+  auto step = [&](auto st, int j, f32x16& sc, f32x16& sn, int to_next) __attribute__((always_inline)) {
+    constexpr int ST = decltype(st)::value;
+    if (j >= nsub) return;
+    const bool mask = 32 * j + 31 > minpos_w;  // diagonal / context-end subtile: mask, then its true max
+    if (mask) {
+      mask_subtile(sc, 32 * j, mypos);
+      tmax = subtile_max(sc, scale_log2);
     }
+    const bool rescale = !__all(tmax <= m + kRescaleThr);
+    if (rescale) {
+      const float mn = fmaxf(m, tmax);
+      const float alpha = __builtin_amdgcn_exp2f(m - mn);  // first subtile: m = -inf, alpha = 0
+      m = mn;
+      lsum *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
+    }
+    if (mask || rescale) {
+      fsum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float p = prob(sc[i]);
+        fsum += p;
+        first.h[i] = (bf16)p;
+      }
+    }
+    // branch-free from here: S(j + 1) unconditionally (past the wave's last subtile it is an unused stale-LDS product); its row max
+    // is an upper bound until a masked subtile recomputes it above
+    Pack8 pf[2];
+    pf[0] = first;
+    float psum = fsum, top = -INFINITY;
+    fsum = 0.f;
+    sn = f32x16{};
+#pragma unroll
+    for (int n = 0; n < 16; ++n) {
+      if (n < 8) sn = mfma32(f[n % RING], qf[n & 7], sn);
+      else o[n & 3] = mfma32(f[n % RING], pf[(n - 8) >> 2].v, o[n & 3]);
+      // k of S(j + 1): the tile's second half (ST 0), the next tile's first; then V; then k of S(j + 2), a half on
+      const int to = n + RING;
+      if (ST == 0 && to == 8)
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) kx[kk] += to_next;
+      if (to < 8) f[n % RING] = operand(kx[to] + (ST ? 0 : 8192));
+      else if (to < 16) f[n % RING] = operand(vx[2 * ST + ((to - 8) >> 2)] + 4096 * (to & 3));
+      else f[n % RING] = operand(kx[to - 16] + (ST ? 8192 : 0));
+      if (n < 8) {
+        const float p = prob(sc[8 + n]);
+        psum += p;
+        pf[1].h[n] = (bf16)p;
+      } else if (n >= 9 && n < 12) {
+#pragma unroll
+        for (int i = 6 * (n - 9); i < (n == 11 ? 16 : 6 * (n - 8)); i += 2) top = fmaxf(fmaxf(top, sn[i]), sn[i + 1]);
+      } else if (n >= 12) {
+#pragma unroll
+        for (int i = 2 * (n - 12); i < 2 * (n - 11); ++i) {
+          const float p = prob(sn[i]);
+          fsum += p;
+          first.h[i] = (bf16)p;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    lsum += psum;
+    tmax = xhalf_max(top) * scale_log2;
+  };
+
+  int buf = 0;
+  for (int it = 0; it < ntiles; ++it) {
+    const int next = buf == 2 ? 0 : buf + 1, to_next = (next - buf) * TB;
+    if (it + 2 < ntiles) {
+      issue(it + 2, next == 2 ? 0 : next + 1, ids);  // (into the buffer of the tile before this one)
+      if (it + 3 < ntiles) ids = fetch_ids(it + 3);
+    }
+    step(IntC<0>{}, 2 * it, sa, sb, to_next);
+    step(IntC<1>{}, 2 * it + 1, sb, sa, to_next);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) vx[x] += to_next;
+    buf = next;
+    wait_direct_loads();
+    __syncthreads();
   }
-#undef SUBTILE_STEP
   const float l = xhalf_sum(lsum);
   if (!row_ok) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;
