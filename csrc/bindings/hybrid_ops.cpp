@@ -620,6 +620,33 @@ bool row_linear_conv(const Tensor& x, const Tensor& w, Tensor& out, const Tensor
   return beside(x, w, out, r);
 }
 
+// out = x . w^T of many rows in bf16; x and out may be column ranges; rows: of a tile, splits: of K (more than one: with a workspace);
+// false: no such form
+bool tile_linear(const Tensor& x, const Tensor& w, Tensor& out, int64_t rows, int64_t splits, const OptTensor& slab,
+                 const OptTensor& counters) {
+  gpu(x, "x", false);
+  gpu(out, "out", false);
+  dtype(w, at::kBFloat16, "w");
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16 && x.dim() == 2 && w.dim() == 2 && out.dim() == 2,
+              "tile_linear: bf16, 2-d operands");
+  const int64_t M = x.size(0), K = x.size(1), N = out.size(1), top = 0x7fffffff;
+  TORCH_CHECK(M >= 1 && out.size(0) == M && w.size(1) == K && w.size(0) == N && N >= 1 && w.is_contiguous(), "tile_linear: shapes");
+  TORCH_CHECK(K >= 512 && K % 64 == 0 && 2 * N * K <= top, "tile_linear: K in 64s from 512 on, weights below 2 GiB");
+  TORCH_CHECK(x.stride(1) == 1 && out.stride(1) == 1, "tile_linear: inner strides must be 1");
+  const int64_t ldx = M > 1 ? x.stride(0) : K, ldo = M > 1 ? out.stride(0) : N;
+  TORCH_CHECK(ldx >= K && ldx % 8 == 0 && ldo >= N && M <= (1 << 24) && ldx <= (1 << 24) && 2 * M * ldx <= top, "tile_linear: row strides");
+  TORCH_CHECK((uintptr_t)x.data_ptr() % 16 == 0 && (uintptr_t)w.data_ptr() % 16 == 0, "tile_linear: alignment");
+  TORCH_CHECK(rows >= 1 && rows <= 1024 && splits >= 1 && splits <= 256 && slab.has_value() == counters.has_value(), "tile_linear: form");
+  if (slab) {
+    dtype(*slab, at::kFloat, "slab");
+    dtype(*counters, at::kInt, "counters");
+    TORCH_CHECK(slab->numel() >= MID_SLAB && counters->numel() >= 256 && (uintptr_t)slab->data_ptr() % 16 == 0, "tile_linear: workspace");
+  }
+  const at::OptionalDeviceGuard g(x.device());
+  return launch_tile_linear(x.data_ptr(), ldx, w.data_ptr(), out.data_ptr(), ldo, (int)M, (int)N, (int)K, (int)rows, (int)splits,
+                            slab ? slab->data_ptr<float>() : nullptr, slab ? counters->data_ptr<int>() : nullptr, cur_stream(x));
+}
+
 // y = x . W^T of 17 to 256 rows in bf16; x and out may be column ranges; glu as above; false: the sizes have no kernel
 bool mid_linear(const Tensor& x, const Tensor& w, Tensor& out, bool glu, Tensor& slab, Tensor& counters) {
   gpu(x, "x", false);
@@ -1542,6 +1569,8 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
       "Tensor prev_row, Tensor save_slot, Tensor ngate, Tensor w, float eps, Tensor(f!) gy) -> bool",
       &window_attn_decay);
   m.def("mid_linear_f32(Tensor x, Tensor w, Tensor(a!) out) -> bool", &mid_linear_f32);
+  m.def("tile_linear(Tensor x, Tensor w, Tensor(a!) out, int rows, int splits=1, Tensor(b!)? slab=None, Tensor(c!)? counters=None) -> bool",
+        &tile_linear);
   m.def("mid_linear(Tensor x, Tensor w, Tensor(a!) out, bool glu, Tensor(b!) slab, Tensor(c!) counters) -> bool", &mid_linear);
   m.def("relu_sq(Tensor a, Tensor(a!) out) -> ()", &relu_sq);
   m.def("silu_mul(Tensor gate, Tensor up, Tensor(a!) out) -> ()", &silu_mul);

@@ -52,7 +52,7 @@ LATENT_BINDINGS = ("latent_ops.cpp",)
 HYBRID_SO = os.path.join(PKG, "_C_hybrid.so")
 HYBRID_KERNELS = ("hybrid_rows.hip", "stream_rows.hip", "norm_rows.hip", "routed_ff.hip", "window_attention.hip", "prompt_attention.hip",
                   "split_attention.hip", "decay_scan.hip", "decay_chunk.hip", "delta_rule.hip", "delta_token.hip", "row_linear.hip",
-                  "mid_linear.hip")
+                  "mid_linear.hip", "tile_linear.hip")
 HYBRID_SHARED = ("glu_moe.hip",)
 HYBRID_BINDINGS = ("hybrid_ops.cpp",)
 NET_SO = os.path.join(PKG, "net", "_native.so")
@@ -186,7 +186,7 @@ def build_latent(verbose: bool = False, force: bool = False) -> str:
 
 
 def build_hybrid(verbose: bool = False, force: bool = False) -> str:
-    """csrc/kernels/{hybrid_rows,stream_rows,norm_rows,routed_ff,window_attention,prompt_attention,split_attention,decay_scan,decay_chunk,delta_rule,delta_token,row_linear,mid_linear,glu_moe}.hip + csrc/bindings/hybrid_ops.cpp ->
+    """csrc/kernels/{hybrid_rows,stream_rows,norm_rows,routed_ff,window_attention,prompt_attention,split_attention,decay_scan,decay_chunk,delta_rule,delta_token,row_linear,mid_linear,tile_linear,glu_moe}.hip + csrc/bindings/hybrid_ops.cpp ->
     symmetry_amd/_C_hybrid.so (``torch.ops.symmetry_amd_hybrid``)."""
     os.makedirs(OBJ, exist_ok=True)
     kdir = os.path.join(CSRC, "kernels")

@@ -674,6 +674,48 @@ def mid_workspace(ws, device):
             ws.get("linear.counters", (256,), torch.int32, device, zeros=True))
 
 
+@functools.lru_cache(4096)
+def tile_plan(M: int, N: int, K: int, ws: bool) -> tuple[int, int] | None:
+    """(rows of a tile, slices of K) of the tile kernel (csrc/kernels/tile_linear.hip) for x of more than MID_ROWS rows, None where the
+    library is ahead; ``ws``: the call has a workspace.  One round of 256 tiles is what the kernel is made for.  420 sizes drawn over
+    257 .. 1700 rows, 768 .. 9000 outputs, weights past the caches, kernel / library (mean, worst):
+
+    K up to 2048: tiles of 64 rows that fill half a round, 1024 0.85 (0.88), 1536 0.85 (0.90), 2048 0.93 (1.07); of 128 past that, 0.87
+    (0.96), 0.87 (0.98), 0.90 (0.99); two rounds are the library's (3072 x 2048 at 1530 rows 24.0 / 34.6 us), and K of 2560 1.00 (1.13).
+    In slices: 4096, tiles of 64 a third to half a round in two 0.93 (0.94), fewer 1.07; longer K, tiles of 128 a quarter to half a round in
+    two, 8192 0.87 (0.96), 14336 0.83 (0.94), and a quarter in four, 0.89 (1.02) and 0.74 (0.88); 5120 1.0 (1.09).
+
+    Fewer tiles with K up to 2048 take 1.1 to 1.2 of the library's 12 to 13 us (in two slices where that fits, 1.08 to 1.13), but the
+    library's call costs the host 20 us and this one 9, and prompt steps of recurrent stacks of so few rows are not ahead of the device:
+    four layers, 300 rows, 814 -> 753 and 648 -> 616 us.  Those are the ones that have a workspace."""
+    if M <= MID_ROWS or K < 1024 or K % 64 or N < 512:
+        return None
+    small, large = -(-M // 64) * -(-N // 128), -(-M // 128) * -(-N // 128)
+    if K <= 2048:
+        if small <= 128:
+            return None if not ws else (64, 2) if K >= 1792 and small <= 85 else (64, 1)
+        return (64, 1) if small <= 256 else (128, 1) if large <= 256 else None
+    if not ws:
+        return None
+    if K <= 4096:
+        return (64, 2) if K > 3584 and 85 < small <= 128 else None
+    if K >= 6144:
+        return (128, 2) if small > 128 >= large else (128, 4) if small <= (128 if K >= 12288 else 85) and large <= 64 else None
+    return None
+
+
+def tile_linear(x, w, out, ws=None) -> bool:
+    """out [M, N] bf16 = x @ w.T on the tile kernel; False where it does not take the operands or the library is ahead."""
+    if _traced(x, w, out) or x.dim() != 2 or w.dim() != 2 or out.dim() != 2:
+        return False
+    (M, K), N = x.shape, w.shape[0]
+    plan = tile_plan(M, N, K, ws is not None)
+    if (plan is None or N != out.shape[1] or out.dtype != torch.bfloat16 or not K <= x.stride(0) <= 1 << 20 or out.stride(0) > 1 << 28
+            or 2 * max(M * x.stride(0), N * K) > 0x7FFFFFFF or not _own_linear(x, w, out)):
+        return False
+    return _hyb().tile_linear(x, w, out, *plan, *(mid_workspace(ws, x.device) if plan[1] > 1 else ()))
+
+
 def linear_glu(x, w, out, ws) -> bool:
     """out = silu(gate) * up with w's [gate | up] rows in one launch, where a kernel takes the operands."""
     if _traced(x, w, out):
@@ -742,7 +784,8 @@ def linear_two(x0, w0, out0, x1, w1, out1, ws=None) -> None:
 
 def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, ws=None) -> torch.Tensor:
     """``x @ w.T``: the few-row kernel up to 16 rows (2048 x 2048 at 8 rows 4.8 us, the library 8.5; 17688 x 2048 21.9 / 49.6),
-    with a workspace ``ws`` (a model's: ``get(name, shape, dtype, device, zeros)``) the medium-row kernel up to 256, else the library GEMM (hipBLASLt through torch, the library heuristic; a
+    with a workspace ``ws`` (a model's: ``get(name, shape, dtype, device, zeros)``) the medium-row kernel up to 256, past that the tile
+    kernel where its tiles are one round of the CUs (tile_plan), else the library GEMM (hipBLASLt through torch, the library heuristic; a
     tuned-solution table measured neutral end to end and was removed: profiles/r4/blaslt_tuned_ab.jsonl)."""
     if own_linear(x, w, out, ws):
         return out
@@ -751,7 +794,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, ws
 
 def own_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None, ws=None) -> bool:
     """``linear`` where a kernel of ours takes the operands; False: nothing has been done."""
-    if not _traced(x, w, out) and x.dim() == 2 and x.shape[0] <= MID_ROWS:
+    if not _traced(x, w, out) and x.dim() == 2:
+        if x.shape[0] > MID_ROWS:
+            return tile_linear(x, w, out, ws)
         if x.shape[0] <= FEW_ROWS:
             if _few(x, w, out) and out.dtype == torch.bfloat16 and out.shape[1] == w.shape[0]:
                 row_linear(x, w, out)
