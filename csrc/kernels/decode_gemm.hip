@@ -130,6 +130,50 @@ SYM_DEV void gemm_tile(const bf16* __restrict__ x, const bf16* __restrict__ W, i
 
   int b = 0;
   bool rn_done = false;
+  if constexpr (RT == 1 && MT == 1) {
+    // Weights that pass by the caches: a ring of U k-blocks.  A block's registers take the block U further on as soon as it is
+    // multiplied, so U blocks are always in flight; in rounds of U each waited for a round trip.  us at 1 / 5 / 10 / 16 rows: 4096 x 14336
+    // 22.9 / 23.6 / 23.6 / 25.5 -> 19.2 / 19.7 / 20.4 / 23.2 (6.1 to 5.1 TB/s), 2048 x 8192 in two slices 10.5 / 10.8 / 11.6 / 12.6 ->
+    // 9.0 / 9.1 / 9.5 / 10.1; twice the depth or the waves take as long.  (Rows past M re-read the last one, into columns that nobody looks at: the wait for a
+    // load in a branch of its own counts nothing that was asked for behind it.)
+    if (e.wnt && nblk >= U) {
+      Pack8 wa[U][2], xa[U][2];
+      auto load = [&](int u, int blk64) {
+        const int ko = blk64 * 64;
+        wa[u][0].w = ld_nt16(wrow[0] + ko * wmul);
+        wa[u][1].w = ld_nt16(wrow[0] + ko * wmul + wsec);
+        xa[u][0].u = *reinterpret_cast<const uint4*>(xrow[0] + ko);
+        xa[u][1].u = *reinterpret_cast<const uint4*>(xrow[0] + ko + 32);
+      };
+      auto multiply = [&](int u) {
+        acc[0][0] = mfma16(wa[u][0].v, xa[u][0].v, acc[0][0]);
+        acc[0][0] = mfma16(wa[u][1].v, xa[u][1].v, acc[0][0]);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+#pragma unroll
+      for (int u = 0; u < U; ++u) load(u, u);
+      __builtin_amdgcn_sched_barrier(0);
+      row_scales();
+      rn_done = true;
+      for (; b + 2 * U <= nblk; b += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          multiply(u);
+          load(u, b + U + u);
+        }
+      }
+      const int rem = nblk - b - U;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        multiply(u);
+        if (u < rem) load(u, b + U + u);
+      }
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u)
+        if (u < rem) multiply(u);
+      b = nblk;
+    }
+  }
   for (; b + U <= nblk; b += U) {
     Pack8 wa[U][RT][2], xa[U][MT][2];
 #pragma unroll
@@ -432,7 +476,25 @@ SYM_DEV void xres_body(const bf16* __restrict__ x, const bf16* __restrict__ W, i
       wa[j][1].u = on ? *reinterpret_cast<const uint4*>(wp + j * 64 * wmul + wsec) : make_uint4(0, 0, 0, 0);
     }
   };
-  load_w(0);
+  // Whole tiles of shallow weights: D of them in flight, each in registers of its own (one of 2048 deep rows is 64 KB a CU, less than the
+  // stream's latency wants: 16384 x 2048 at 1 / 10 rows 14.1 / 14.3 -> 13.1 / 13.5 us)
+  constexpr int D = U == 1 ? 4 : U == 2 ? 2 : 1;
+  Pack8 ahead[D][U][2];
+  const bool deep = D > 1 && KS == 1 && P == 0 && nf >= D && e.wnt;
+  auto load_ahead = [&](int d, int i) {
+    const bf16* wp = wptr(b + i * G);
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      ahead[d][j][0].w = ld_nt16(wp + j * 64 * wmul);
+      ahead[d][j][1].w = ld_nt16(wp + j * 64 * wmul + wsec);
+    }
+  };
+  if (deep) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load_ahead(d, d);
+  } else {
+    load_w(0);
+  }
   const bool xok = r16 < M;
   const bf16* xrow = x + (long long)min(r16, M - 1) * K + kbeg + 8 * h;
   Pack8 xa[U][2];
@@ -467,6 +529,51 @@ SYM_DEV void xres_body(const bf16* __restrict__ x, const bf16* __restrict__ W, i
     epilogue<EPI>(e, v, t, m, mok && (hf < 0 || (h & 1) == hf), h, N, xep);
   };
   int buf = 0;
+  auto reduce = [&](f32x4 acc) {      // wave 0: the waves' sum
+    red[buf][wid][lane] = acc;
+    __syncthreads();
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (wid == 0) {
+      v = red[buf][0][lane];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) {
+        v += red[buf][w][lane];
+        // partials in registers at a time: as many as the 128 of a lane of sixteen waves have room for beside the weights (four at a
+        // time were four LDS latencies at the end of every tile: a step of 17 such launches 418.0 -> 416.1 us, 2048 wide 265.6 -> 263.3)
+        if ((w & (U > 2 ? 7 : 15)) == (U > 2 ? 7 : 15)) asm volatile("" : "+v"(v)::"memory");
+      }
+    }
+    buf ^= 1;
+    return v;
+  };
+  if constexpr (D > 1 && KS == 1) {
+    if (deep) {
+      auto tile = [&](int d, int i, bool more) __attribute__((always_inline)) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+          acc = mfma16(ahead[d][j][0].v, xa[j][0].v, acc);
+          acc = mfma16(ahead[d][j][1].v, xa[j][1].v, acc);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) load_ahead(d, i + D);
+        const f32x4 v = reduce(acc);
+        if (wid == 0) finish(v, b + i * G);
+      };
+      int i = 0;
+      for (; i + 2 * D <= nf; i += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) tile(d, i + d, true);
+      }
+      const int rem = nf - i - D;
+#pragma unroll
+      for (int d = 0; d < D; ++d) tile(d, i + d, d < rem);
+#pragma unroll
+      for (int d = 0; d < D - 1; ++d)
+        if (d < rem) tile(d, i + D + d, false);
+      return;
+    }
+  }
   for (int i = 0; i < nu; ++i) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     if (unit_active(i)) {
@@ -479,17 +586,8 @@ SYM_DEV void xres_body(const bf16* __restrict__ x, const bf16* __restrict__ W, i
     // keep the next loads behind this tile's MFMAs: they reuse wa's registers (no renamed second copy)
     __builtin_amdgcn_sched_barrier(0);
     if (i + 1 < nu) load_w(i + 1);  // next unit's weight stream in flight during this unit's reduction/epilogue
-    red[buf][wid][lane] = acc;
-    __syncthreads();
+    const f32x4 v = reduce(acc);
     if (wid == 0) {
-      f32x4 v = red[buf][0][lane];
-#pragma unroll
-      for (int w = 1; w < NW; ++w) {
-        v += red[buf][w][lane];
-        // partials in registers at a time: as many as the 128 of a lane of sixteen waves have room for beside the weights (four at a
-        // time were four LDS latencies at the end of every tile: a step of 17 such launches 418.0 -> 416.1 us, 2048 wide 265.6 -> 263.3)
-        if ((w & (U > 2 ? 7 : 15)) == (U > 2 ? 7 : 15)) asm volatile("" : "+v"(v)::"memory");
-      }
       if (i < nf) {
         finish(v, unit_tile(i));
       } else if constexpr (KS == 1) {  // row half of a remainder tile
@@ -503,7 +601,6 @@ SYM_DEV void xres_body(const bf16* __restrict__ x, const bf16* __restrict__ W, i
         __hip_atomic_store(slot + 1, w64[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
-    buf ^= 1;
   }
   if constexpr (KS > 1) {
     if (wid != 0 || np == 0) return;
@@ -546,6 +643,15 @@ __global__ __launch_bounds__(1024) void decode_gemm_xres_kernel(const bf16* __re
 }
 
 int g_num_cus = 0;
+int cus() {
+  if (g_num_cus == 0) {
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&g_num_cus, hipDeviceAttributeMultiprocessorCount, dev);
+    g_num_cus = std::max(1, g_num_cus);
+  }
+  return g_num_cus;
+}
 
 // Remainder split: OFF by default.  Measured (profiles/r3/ksplit_ab.jsonl, alternating runs): 8B 10 clients
 // 3.308 vs 3.230 ms per step, TP = 8 shard 1.576 vs 1.538, TP = 4 1.965 vs 1.817 -- at these sizes the launch
@@ -583,13 +689,7 @@ void go_xres_ks(const bf16* x, const bf16* W, int M, int N, int K, const DecodeE
 template <int EPI>
 bool go_xres(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEpi& e, hipStream_t s) {
   if (M > 16 || K % 1024 || K > 4096) return false;
-  if (!g_num_cus) {
-    int dev = 0;
-    hipGetDevice(&dev);
-    hipDeviceGetAttribute(&g_num_cus, hipDeviceAttributeMultiprocessorCount, dev);
-    g_num_cus = std::max(1, g_num_cus);
-  }
-  const int C = g_num_cus;
+  const int C = cus();
   const int ntiles = N / 16;
   const int per = (ntiles + C - 1) / C;  // whole tiles: equal tile count per workgroup
   // XAR keeps one epoch slot per walked tile in LDS: the real tiles-per-workgroup count (a partitioned GPU has
@@ -686,14 +786,8 @@ void launch_mt(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEp
     // K = 8192): whole-tile workgroups would leave 176 of 256 CUs idle, so split K in two across 8-wave
     // workgroups (profiles/r4/dg_tile_ksplit.jsonl: 12.93 -> 9.31 us at M = 1, 13.45 -> 9.88 at 4, 14.11 -> 11.39
     // at 10; 4 splits or 4 waves lose to it)
-    if (g_num_cus == 0) {
-      int dev = 0;
-      hipGetDevice(&dev);
-      hipDeviceGetAttribute(&g_num_cus, hipDeviceAttributeMultiprocessorCount, dev);
-      g_num_cus = std::max(1, g_num_cus);
-    }
     const int tiles = N / 16;
-    if (2 * tiles <= g_num_cus) v = ks_fits<MT, EPI>(N, K, 2, 8, e) ? 23 : (ks_fits<MT, EPI>(N, K, 2, 4, e) ? 21 : v);
+    if (2 * tiles <= cus()) v = ks_fits<MT, EPI>(N, K, 2, 8, e) ? 23 : (ks_fits<MT, EPI>(N, K, 2, 4, e) ? 21 : v);
   }
   if ((v == 21 || v == 23) && !ks_fits<MT, EPI>(N, K, 2, v == 21 ? 4 : 8, e)) v = -2;
   if ((v == 22 || v == 24) && !ks_fits<MT, EPI>(N, K, 4, v == 22 ? 4 : 8, e)) v = -2;
@@ -719,7 +813,11 @@ void launch_mt(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEp
       // qkv 15.6 -> 13.4, lm_head 205.9 -> 190.5; = variant 2 on the one-tile-per-CU O projection), except
       // the vocabulary projection at <= 2 rows where the 8-wave split stays ahead (lm_head 171 vs 177-183 us;
       // at 4 rows the walk wins, 179 vs 186: profiles/r4/dg_lm_head_small_m.jsonl)
-      if (M <= 16 && K % 1024 == 0 && K <= 4096 && !(N >= 65536 && M <= 2)) v = 11;
+      // (a walk of one tile is no walk: up to a tile a CU 8 waves with their ring of blocks, 4096 x 4096 at 1 / 10 / 16 rows 9.0 / 10.1 /
+      // 11.2 -> 7.7 / 8.2 / 8.9 us, 2048 x 2048 5.5 / 6.2 / 6.7 -> 4.6 / 5.1 / 5.6, 3072 x 2048 5.8 / 6.8 / 7.5 -> 5.0 / 6.1 / 6.8; of 1024
+      // deep rows both take 4.2; at a tile and a half a CU, 6144 x 4096, the walk is ahead from 10 rows on, 12.4 / 13.7)
+      if (M <= 16 && K % 1024 == 0 && K >= 2048 && K <= 4096 && EPI != DECODE_EPI_XAR && N / 16 <= cus()) v = 0;
+      else if (M <= 16 && K % 1024 == 0 && K <= 4096 && !(N >= 65536 && M <= 2)) v = 11;
       // wide N at 2..16 rows otherwise (Llama-3-70B at TP <= 4: gate_up, lm_head; K = 8192): 4 waves per tile.
       // (The round-1 pick, 7 resident 4-wave workgroups per CU -- variant 8, launch bounds (256, 7) -- now spills
       // 32 VGPRs to scratch with the grown epilogues: 70B gate_up 293-317 vs 165-204 us at 8-16 rows,
@@ -741,13 +839,7 @@ void launch_mt(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEp
       // per 8-wave workgroup when that grid is a whole number of rounds over the CUs, else 4 waves per tile
       // (profiles/r4/dg_70b_row.jsonl, 4 rows: gate_up 179.4 -> 163.4 us, down 92.6 -> 85.7, o 31.1 -> 29.8,
       // qkv 41.2 -> 40.1)
-      if (g_num_cus == 0) {
-        int dev = 0;
-        hipGetDevice(&dev);
-        hipDeviceGetAttribute(&g_num_cus, hipDeviceAttributeMultiprocessorCount, dev);
-        g_num_cus = std::max(1, g_num_cus);
-      }
-      v = (N % 32 == 0 && (N / 32) % g_num_cus == 0) ? 3 : (K >= 4096 && K % 256 == 0 ? 4 : 0);
+      v = (N % 32 == 0 && (N / 32) % cus() == 0) ? 3 : (K >= 4096 && K % 256 == 0 ? 4 : 0);
     } else if (N >= 12288) {
       // row-major wide N above 16 rows (the lm_head, whose weights are never preshuffled): 4 row tiles per
       // workgroup, lm_head 268 -> 224 us at M = 24, 421 -> 335 at M = 64 (profiles/decode_gemm_bigm_row_r1.jsonl)

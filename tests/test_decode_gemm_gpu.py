@@ -44,6 +44,24 @@ def test_dg_f32(gpu, M, N, K):
     _close(y, y_ref, atol=2e-3, rtol=1e-2)
 
 
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("N,K", [(160, 512), (160, 1536), (160, 2560), (64, 3584), (4096, 2048), (64, 5120), (2048, 8192), (4112, 6656),
+                                 (8192, 2048), (8208, 2048), (20480, 2048), (4128, 1024), (16400, 1024), (36864, 1024)])
+def test_streams_in_flight(gpu, M, N, K):
+    """Preshuffled weights past the caches: fewer k-blocks a wave than its ring has, as many, a part more, twice as many and more; K in
+    two slices; walks of 1 to 9 tiles a workgroup, two or four of them in flight.  fp32 sums of K products of bf16 values against 64
+    bits: off by about sqrt(K) 2^-24 of the vectors' norms at most, four times that is allowed."""
+    from symmetry_amd.models.layout import preshuffle
+
+    print("dg_f32", M, N, K, flush=True)
+    x, W, _ = _inputs(gpu, M, N, K, seed=4, ss=False)
+    y = torch.empty(M, N, device=gpu)
+    ops.dg_f32(x, preshuffle(W), None, 0.0, y, wshuf=True)
+    want = x.double() @ W.double().t()
+    bound = 4 * K ** 0.5 * 2.0 ** -24 * float(x.double().norm(dim=1).max() * W.double().norm(dim=1).max())
+    assert float((y.double() - want).abs().max()) <= bound
+
+
 @pytest.mark.parametrize("M", MS)
 @pytest.mark.parametrize("N,K", [(4096, 4096), (1024, 1792)])
 def test_dg_resid(gpu, M, N, K):
