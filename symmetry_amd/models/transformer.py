@@ -215,6 +215,7 @@ class TransformerLM:
         if self.device.type != "cpu":
             ops.decode_ks_ws(self.device)  # allocated before any graph capture (stable address)
         self.single_copy = False  # decode_weights="replace": the layer weights exist only MFMA-preshuffled
+        self.decode_only_copies = False  # prompts keep the bf16 products of the row-major weights, whatever copies there are
         self.dgw = self._decode_copies(decode_weights)
         self.tp_reduced_bytes: dict[str, int] = {}  # bytes per rank of the last general-path all-reduce
 
@@ -230,7 +231,7 @@ class TransformerLM:
           grouped prefill GEMM kernels); the fp32 oracle and exports unshuffle (layout.natural_tensors);
         * "shared": row-major only (the decode GEMMs' row-major variants);
         * "auto": MoE models "replace" (profiles/r6/e2e_mixtral_c5_single_copy.jsonl: equal end to end, 90 GB
-          less); dense models "preshuffled" when the copy fits next to the KV cache's need (transformer.copy_budget;
+          less), or where the experts' shapes do not tile for it copies of wqkv and wo for decode steps; dense models "preshuffled" when the copy fits next to the KV cache's need (transformer.copy_budget;
           their prefill is faster on the library GEMMs), "replace" otherwise (70B on one GPU: 141 GB of layer
           weights), row-major only where neither applies."""
         if not self.fused or mode == "shared" or (self.device.type == "cpu" and mode != "replace"):
@@ -245,10 +246,14 @@ class TransformerLM:
             # launch) only from what the same budget has left, so it never costs a model its layer copies.  The
             # budget: what is left after the KV cache's need and a 6 GB workspace reserve
             budget = copy_budget(self.device, self.kv_reserve)
-            if self.moe is not None:
-                mode = "replace" if self.moe.single_copy_ok() else "shared"
-                if mode == "shared":
+            if self.moe is not None and not self.moe.single_copy_ok():
+                # (the experts keep their rows; the attention's projections of decode steps, a few per cent of the weights, have a copy
+                # beside theirs: 8 rows of 3072 x 2048 7.6 -> 5.9 us, of 2048 x 2048 6.1 -> 4.9)
+                if extra > budget:
                     return {}
+                head, self.decode_only_copies = None, True
+            elif self.moe is not None:
+                mode = "replace"
             elif extra > budget:
                 mode = "replace"
             if head is not None and (mode == "replace" or extra + head.numel() * 2 > budget):
@@ -315,7 +320,7 @@ class TransformerLM:
 
     def _shuf(self, i: int, name: str):
         """The MFMA-preshuffled copy of weight `name` of layer i, or None (medium-M prefill GEMMs)."""
-        return self.dgw.get((i, name))
+        return None if self.decode_only_copies else self.dgw.get((i, name))
 
     def _fused_supported(self) -> bool:
         """Shape contract of the fused decode GEMMs: D == 128, every K % 256 == 0, every N % 16 == 0."""
