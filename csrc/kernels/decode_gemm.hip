@@ -478,7 +478,7 @@ SYM_DEV void xres_body(const bf16* __restrict__ x, const bf16* __restrict__ W, i
   };
   // Whole tiles of shallow weights: D of them in flight, each in registers of its own (one of 2048 deep rows is 64 KB a CU, less than the
   // stream's latency wants: 16384 x 2048 at 1 / 10 rows 14.1 / 14.3 -> 13.1 / 13.5 us)
-  constexpr int D = U == 1 ? 4 : U == 2 ? 2 : 1;
+  constexpr int D = EPI == DECODE_EPI_ARGMAX ? 1 : U == 1 ? 4 : U == 2 ? 2 : 1;
   Pack8 ahead[D][U][2];
   const bool deep = D > 1 && KS == 1 && P == 0 && nf >= D && e.wnt;
   auto load_ahead = [&](int d, int i) {
@@ -817,6 +817,12 @@ void launch_mt(const bf16* x, const bf16* W, int M, int N, int K, const DecodeEp
       // 11.2 -> 7.7 / 8.2 / 8.9 us, 2048 x 2048 5.5 / 6.2 / 6.7 -> 4.6 / 5.1 / 5.6, 3072 x 2048 5.8 / 6.8 / 7.5 -> 5.0 / 6.1 / 6.8; of 1024
       // deep rows both take 4.2; at a tile and a half a CU, 6144 x 4096, the walk is ahead from 10 rows on, 12.4 / 13.7)
       if (M <= 16 && K % 1024 == 0 && K >= 2048 && K <= 4096 && EPI != DECODE_EPI_XAR && N / 16 <= cus()) v = 0;
+      // (vocabulary projections, whose tiles end with a sampling epilogue that a walk waits for: rings of blocks, four waves a tile, of few
+      // rows, 32768 x 2048 at 1 / 6 rows with logits 31.1 / 31.7 -> 26.2 / 28.2, 8 32.1 / 29.3 but 128256 x 2048 at 8 without 89 / 92;
+      // 128256 x 2048 at 1 / 6 96 / 102 -> 82 / 91; 32768 x 4096 at 1 / 4 45.7 / 45.6 -> 43.2 / 46.0; 1024 deep, two tiles a workgroup,
+      // 50304 outputs at 1 / 16 32.4 / 35.2 -> 24.1 / 29.8.  Two tiles of a walk in flight took 1.08 of one)
+      else if (EPI == DECODE_EPI_ARGMAX && M <= 16 && K == 1024) v = 6;
+      else if (EPI == DECODE_EPI_ARGMAX && ((K == 2048 && M <= 6) || (K == 4096 && M <= 2))) v = 4;
       else if (M <= 16 && K % 1024 == 0 && K <= 4096 && !(N >= 65536 && M <= 2)) v = 11;
       // wide N at 2..16 rows otherwise (Llama-3-70B at TP <= 4: gate_up, lm_head; K = 8192): 4 waves per tile.
       // (The round-1 pick, 7 resident 4-wave workgroups per CU -- variant 8, launch bounds (256, 7) -- now spills

@@ -619,3 +619,23 @@ def test_xres_row_halves_bitwise(gpu, M, what, Hq, Hkv, N):
         act_r = torch.empty(M, N // 2, dtype=torch.bfloat16)
         ref.dg_swiglu(x.cpu(), W.cpu(), s.cpu(), 1e-5, act_r)
         _close(halves[0], act_r, atol=3e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("M", [1, 6, 7, 16])
+@pytest.mark.parametrize("N,K", [(1024, 1024), (16416, 1024), (8208, 2048), (16032, 2048), (528, 4096)])
+def test_vocabulary_rows(gpu, M, N, K):
+    """The sampling head's forms on preshuffled weights: logits within four times the bound of K fp32 sums of their 64-bit values, and
+    the ids that these logits give."""
+    from symmetry_amd.models.layout import preshuffle
+
+    print("dg_argmax", M, N, K, flush=True)
+    x, W, _ = _inputs(gpu, M, N, K, seed=21, ss=False)
+    temps, seeds = torch.zeros(M, device=gpu), torch.zeros(M, device=gpu, dtype=torch.int64)
+    step = torch.tensor([3], device=gpu, dtype=torch.int64)
+    tk, keys = torch.empty(M * (N // 16), device=gpu, dtype=torch.int64), torch.empty(M, device=gpu, dtype=torch.int64)
+    ids, logits = torch.empty(M, device=gpu, dtype=torch.int32), torch.empty(M, N, device=gpu)
+    ops.dg_argmax(x, preshuffle(W), None, 0.0, temps, seeds, step, tk, keys, ids, 0, logits, wshuf=True)
+    want = x.double() @ W.double().t()
+    bound = 4 * K ** 0.5 * 2.0 ** -24 * float(x.double().norm(dim=1).max() * W.double().norm(dim=1).max())
+    assert float((logits.double() - want).abs().max()) <= bound
+    assert torch.equal(ids.long(), logits.argmax(1))
