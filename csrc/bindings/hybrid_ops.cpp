@@ -620,6 +620,24 @@ bool row_linear_conv(const Tensor& x, const Tensor& w, Tensor& out, const Tensor
   return beside(x, w, out, r);
 }
 
+// out (fp32) = x . w^T of up to 16 outputs, bf16 operands; x and out may be column ranges
+void narrow_linear(const Tensor& x, const Tensor& w, Tensor& out) {
+  gpu(x, "x", false);
+  gpu(out, "out", false);
+  dtype(w, at::kBFloat16, "w");
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kFloat && x.dim() == 2 && w.dim() == 2 && out.dim() == 2,
+              "narrow_linear: bf16 operands, fp32 out, 2-d");
+  const int64_t M = x.size(0), K = x.size(1), N = out.size(1);
+  TORCH_CHECK(M >= 1 && M <= (1 << 24) && out.size(0) == M && w.size(1) == K && w.size(0) == N && w.is_contiguous(), "narrow_linear: shapes");
+  TORCH_CHECK(K >= 128 && K % 128 == 0 && K <= (1 << 22) && N >= 4 && N % 4 == 0 && N <= 16, "narrow_linear: K in 128s, N in 4s up to 16");
+  TORCH_CHECK(x.stride(1) == 1 && out.stride(1) == 1, "narrow_linear: inner strides must be 1");
+  const int64_t ldx = M > 1 ? x.stride(0) : K, ldo = M > 1 ? out.stride(0) : N;
+  TORCH_CHECK(ldx >= K && ldx % 8 == 0 && ldo >= N && ldo % 4 == 0, "narrow_linear: row strides");
+  TORCH_CHECK(((uintptr_t)x.data_ptr() | (uintptr_t)w.data_ptr() | (uintptr_t)out.data_ptr()) % 16 == 0, "narrow_linear: alignment");
+  const at::OptionalDeviceGuard g(x.device());
+  launch_narrow_linear(x.data_ptr(), ldx, w.data_ptr(), out.data_ptr<float>(), ldo, (int)M, (int)N, (int)K, cur_stream(x));
+}
+
 // out = x . w^T of many rows in bf16; x and out may be column ranges; rows: of a tile, splits: of K (more than one: with a workspace);
 // false: no such form
 bool tile_linear(const Tensor& x, const Tensor& w, Tensor& out, int64_t rows, int64_t splits, const OptTensor& slab,
@@ -1569,6 +1587,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
       "Tensor prev_row, Tensor save_slot, Tensor ngate, Tensor w, float eps, Tensor(f!) gy) -> bool",
       &window_attn_decay);
   m.def("mid_linear_f32(Tensor x, Tensor w, Tensor(a!) out) -> bool", &mid_linear_f32);
+  m.def("narrow_linear(Tensor x, Tensor w, Tensor(a!) out) -> ()", &narrow_linear);
   m.def("tile_linear(Tensor x, Tensor w, Tensor(a!) out, int rows, int splits=1, Tensor(b!)? slab=None, Tensor(c!)? counters=None) -> bool",
         &tile_linear);
   m.def("mid_linear(Tensor x, Tensor w, Tensor(a!) out, bool glu, Tensor(b!) slab, Tensor(c!) counters) -> bool", &mid_linear);

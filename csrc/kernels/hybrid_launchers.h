@@ -77,6 +77,8 @@ constexpr long long MID_SLAB = 256LL * 128 * 256;
 bool launch_mid_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int glu, float* slab,
                        int* counters, hipStream_t s);
 bool launch_mid_linear_f32(const void* x, long long ldx, const void* W, float* out, long long ldo, int M, int N, int K, hipStream_t s);
+// out (fp32) = x . W^T of up to 16 outputs
+void launch_narrow_linear(const void* x, long long ldx, const void* W, float* out, long long ldo, int M, int N, int K, hipStream_t s);
 // y = x . w^T of many rows, tiles of `rows` (64, 128) x 128, K in `splits` slices (of more than one: slab and counters as above, 256 tiles
 // and slices at most); false: no such form
 bool launch_tile_linear(const void* x, long long ldx, const void* w, void* y, long long ldy, int M, int N, int K, int rows, int splits,

@@ -338,6 +338,57 @@ __global__ __launch_bounds__(64) void row_linear_small_kernel(Problems ps) {
   store_rows<16, EPI>(a, n0, lane, acc[0], acc[RT - 1]);
 }
 
+// Up to 16 outputs of many rows into fp32 (step sizes and gates of a prompt step): 16 rows a workgroup, whose waves take the 128-deep
+// blocks of K in turn, read as row_linear_kernel reads them, two in flight, and meet in LDS.  What a CU takes in bounds it: 16 x 2048 at
+// 300 / 1530 / 8100 rows 4.4 / 4.5 / 7.1 us (neighbouring lanes on different rows 5.5 / 5.6 / 9.4; the library 5.5 / 5.3 / 21.1, behind a
+// prompt step's other launches 10.5 at 1530), 16 x 1024 3.5 / 3.6 / 5.0 (4.3 / 4.3 / 9.7); 4096 deep it is behind, 6.7 / 6.8 (6.2 / 6.3).
+constexpr int NARROW_WAVES = 8;
+
+__global__ __launch_bounds__(64 * NARROW_WAVES) void narrow_linear_kernel(Args a) {
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, h = lane >> 4;
+  const int m0 = 16 * blockIdx.x, blocks = a.K / 128, in = 8 * ((lane & 3) + 4 * h);
+  const bf16 *xr[4], *wr[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    xr[i] = a.x + min(m0 + (lane & 12) + i, a.M - 1) * a.ldx + in;
+    wr[i] = a.W + (long long)min((lane & 12) + i, a.N - 1) * a.K + in;
+  }
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int b = wid; b < blocks; b += 2 * NARROW_WAVES) {
+    u32x4 x[2][4], w[2][4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int k = 128 * min(b + u * NARROW_WAVES, blocks - 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[u][i] = *reinterpret_cast<const u32x4*>(xr[i] + k);
+        w[u][i] = *reinterpret_cast<const u32x4*>(wr[i] + k);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (b + u * NARROW_WAVES >= blocks) break;
+      quad_transpose(x[u][0], x[u][1], x[u][2], x[u][3]);
+      quad_transpose(w[u][0], w[u][1], w[u][2], w[u][3]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        Pack8 p, q;
+        p.w = w[u][i], q.w = x[u][i];
+        acc = mfma16(p.v, q.v, acc);
+      }
+    }
+  }
+  __shared__ f32x4 red[NARROW_WAVES][64];
+  red[wid][lane] = acc;
+  __syncthreads();
+  if (wid) return;
+#pragma unroll
+  for (int i = 1; i < NARROW_WAVES; ++i) acc += red[i][lane];
+  const int m = m0 + r16, n = 4 * h;      // N is a multiple of 4
+  if (m < a.M && n < a.N) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + m * a.ldo + n) = acc;
+}
+
 // what a launch does: its problems, how many, and work beside them or null
 struct Job {
   const Problems& ps;
@@ -471,6 +522,11 @@ bool by_shape(const Job& j, hipStream_t s) {
 }
 
 }  // namespace
+
+void launch_narrow_linear(const void* x, long long ldx, const void* W, float* out, long long ldo, int M, int N, int K, hipStream_t s) {
+  const Args a{(const bf16*)x, ldx, (const bf16*)W, out, ldo, M, N, K};
+  narrow_linear_kernel<<<(M + 15) / 16, 64 * NARROW_WAVES, 0, s>>>(a);
+}
 
 bool launch_row_linear(const void* x, long long ldx, const void* W, void* out, long long ldo, int M, int N, int K, int f32_out,
                        int relu2, int glu, hipStream_t s) {

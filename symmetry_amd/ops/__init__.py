@@ -837,9 +837,24 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Ten
     if few_rows(x, w, out) and out.dtype == torch.float32 and out.shape[1] == w.shape[0]:
         row_linear(x, w, out)
         return out
+    if narrow_f32(x, w, out):
+        _hyb().narrow_linear(x, w, out)
+        return out
     if mid_f32(x, w, out) and _hyb().mid_linear_f32(x, w, out):
         return out
     return torch.mm(x, w.t(), out_dtype=torch.float32, out=out)
+
+
+NARROW, NARROW_K = 16, 2048  # outputs and K up to which fp32 results of more than FEW_ROWS rows are narrow_linear's (its times stand in row_linear.hip)
+
+
+def narrow_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+    """Is x @ w.T into fp32 ``out`` the kernel's for few outputs of many rows?"""
+    if _traced(x, w, out) or x.dim() != 2 or w.dim() != 2 or out.dim() != 2:
+        return False
+    (M, K), N = x.shape, w.shape[0]
+    return (FEW_ROWS < M <= 1 << 24 and 0 < N <= NARROW and N == out.shape[1] and 128 <= K <= NARROW_K and K % 128 == 0
+            and out.dtype == torch.float32 and x.stride(0) >= K and _own_linear(x, w, out))
 
 
 def mid_f32_pays(M: int, N: int, K: int) -> bool:

@@ -199,3 +199,22 @@ def test_row_linear_reference_cpu():
     assert torch.equal(out, (y[:, :8] * torch.sigmoid(y[:, :8]) * y[:, 8:]).bfloat16())
     ops.row_linear(x, w[:8], out, relu2=True)
     assert torch.equal(out, ((torch.relu(x.float()) ** 2).bfloat16().float() @ w[:8].float().t()).bfloat16())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [17, 32, 33, 500])
+@pytest.mark.parametrize("N,K", [(4, 128), (16, 896), (12, 1152), (8, 1920), (16, 2048)])
+def test_few_outputs_of_many_rows(gpu, M, N, K):
+    """ops.linear_f32 of up to 16 outputs: blocks of K that fill no turn of the waves, one and more; column ranges of wider matrices.
+    fp32 sums of K products against 64 bits, at most four times sqrt(K) 2^-24 of the vectors' norms."""
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    x = torch.randn(M, K + 24, device=gpu, generator=g).bfloat16()[:, 8:8 + K]
+    w = (torch.randn(N, K, device=gpu, generator=g) * K ** -0.5).bfloat16()
+    room = torch.full((M + 1, N + 8), 7.0, device=gpu)
+    out = room[:M, :N]
+    assert ops.narrow_f32(x, w, out) and not ops.narrow_f32(x[:16], w, out[:16]) and not ops.narrow_f32(x[:, 1:], w[:, 1:], out)
+    ops.linear_f32(x, w, out)
+    want = x.double() @ w.double().t()
+    bound = 4 * K ** 0.5 * 2.0 ** -24 * float(x.double().norm(dim=1).max() * w.double().norm(dim=1).max())
+    assert float((out.double() - want).abs().max()) <= bound
+    assert bool((room[:, N:] == 7).all()) and bool((room[M] == 7).all())
