@@ -77,6 +77,11 @@ SYM_DEV int first_chunk(unsigned wg, int nch, long long x_bytes) {
   return (int)(((wg & 7) * (unsigned)nch / 8 + (wg >> 3) * spread) % (unsigned)nch);
 }
 
+// A matrix product's result is in its registers some 11 cycles of waiting later.  The compiler puts these in along a block, but not where a
+// branch that is taken stands between the product and what reads it (a tile in 100 was wrong in a fourth of its columns): such results
+// pass through here.
+SYM_DEV void settle(f32x4& v) { asm volatile("s_nop 15" : "+v"(v)); }
+
 // Non-temporal 16-byte load (weights that are streamed once).
 SYM_DEV u32x4 ld_nt16(const bf16* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
 

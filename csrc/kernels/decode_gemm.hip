@@ -166,11 +166,15 @@ SYM_DEV void gemm_tile(const bf16* __restrict__ x, const bf16* __restrict__ W, i
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         multiply(u);
+        settle(acc[0][0]);
         if (u < rem) load(u, b + U + u);
       }
 #pragma unroll
       for (int u = 0; u < U - 1; ++u)
-        if (u < rem) multiply(u);
+        if (u < rem) {
+          multiply(u);
+          settle(acc[0][0]);
+        }
       b = nblk;
     }
   }
@@ -255,7 +259,10 @@ SYM_DEV void gemm_tile(const bf16* __restrict__ x, const bf16* __restrict__ W, i
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) red[wid][rt * MT + mt][lane] = acc[rt][mt];
+    for (int mt = 0; mt < MT; ++mt) {
+      settle(acc[rt][mt]);
+      red[wid][rt * MT + mt][lane] = acc[rt][mt];
+    }
   __syncthreads();
   if constexpr (EPI == DECODE_EPI_XAR) {
     if (threadIdx.x == 0) {
@@ -530,6 +537,7 @@ SYM_DEV void xres_body(const bf16* __restrict__ x, const bf16* __restrict__ W, i
   };
   int buf = 0;
   auto reduce = [&](f32x4 acc) {      // wave 0: the waves' sum
+    settle(acc);
     red[buf][wid][lane] = acc;
     __syncthreads();
     f32x4 v = {0.f, 0.f, 0.f, 0.f};

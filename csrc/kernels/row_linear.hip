@@ -377,8 +377,10 @@ __global__ __launch_bounds__(64 * NARROW_WAVES) void narrow_linear_kernel(Args a
         p.w = w[u][i], q.w = x[u][i];
         acc = mfma16(p.v, q.v, acc);
       }
+      settle(acc);
     }
   }
+  settle(acc);
   __shared__ f32x4 red[NARROW_WAVES][64];
   red[wid][lane] = acc;
   __syncthreads();

@@ -150,6 +150,7 @@ __global__ __launch_bounds__(256, 2) void tile_linear_kernel(TileArgs a) {
   }
   first_half();
   second_half(Zero{}, 0);
+  settle(acc[3][FM - 1]);      // (the last of them)
 
   if (S > 1) {
     // parts as they lie in the registers, written through; the last arriver reads them past its L2
