@@ -163,18 +163,23 @@ SYM_DEV void gemm_tile(const bf16* __restrict__ x, const bf16* __restrict__ W, i
         }
       }
       const int rem = nblk - b - U;
+      if (rem == 0) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        multiply(u);
-        settle(acc[0][0]);
-        if (u < rem) load(u, b + U + u);
-      }
+        for (int u = 0; u < U; ++u) multiply(u);
+      } else {
 #pragma unroll
-      for (int u = 0; u < U - 1; ++u)
-        if (u < rem) {
+        for (int u = 0; u < U; ++u) {
           multiply(u);
           settle(acc[0][0]);
+          if (u < rem) load(u, b + U + u);
         }
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u)
+          if (u < rem) {
+            multiply(u);
+            settle(acc[0][0]);
+          }
+      }
       b = nblk;
     }
   }
