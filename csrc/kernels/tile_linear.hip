@@ -9,6 +9,10 @@
 // conflict; a wave's weight rows are read in an order in which a lane's 16 outputs of a row lie side by side: it stores 32 bytes.
 // K is split where tiles would leave half of the CUs idle: of a tile's workgroups the last to arrive adds the parts in their order (nobody
 // waits; the counter is set back to zero).
+// A stage takes 0.25 us at 64 rows and 0.34 at 128, most of it LDS traffic, start and end 3 to 4.5.  Library -> so, us: 1000 rows of 2048 x
+// 2048 15.9 -> 14.0, 700 of 2048 x 8192 in two slices 44.4 -> 38.9, 331 of 4864 x 14336 in two 88 -> 71.3; the rule's lines stand in
+// ops.tile_plan.  (The bound of two workgroups a CU keeps the sums in the registers that products write: with all 512 the compiler moved
+// them in the loop, 1000 rows of 2048 x 2048 18.1.)
 #include <algorithm>
 #include <type_traits>
 
