@@ -26,6 +26,7 @@ from __future__ import annotations
 import concurrent.futures as cf
 import glob
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -76,6 +77,23 @@ def _newer(target: str, deps) -> bool:
     return any(os.path.getmtime(d) > t for d in deps if os.path.exists(d))
 
 
+def _includes(src: str, *dirs: str) -> list[str]:
+    """The headers that ``src`` includes by name in quotes, itself or through one of them, from its own folder or ``dirs``."""
+    seen: dict[str, None] = {}
+    todo = [src]
+    while todo:
+        path = todo.pop()
+        with open(path, encoding="utf-8") as f:
+            names = re.findall(r'^\s*#\s*include\s+"([^"]+)"', f.read(), re.M)
+        for name in names:
+            for d in (os.path.dirname(path), *dirs):
+                h = os.path.join(d, name)
+                if os.path.exists(h) and h not in seen:
+                    seen[h] = None
+                    todo.append(h)
+    return list(seen)
+
+
 def _run(cmd, verbose: bool):
     if verbose:
         print(" ".join(cmd), flush=True)
@@ -112,10 +130,6 @@ NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 def build_kernels(verbose: bool = False, force: bool = False) -> str:
     os.makedirs(OBJ, exist_ok=True)
     kdir = os.path.join(CSRC, "kernels")
-    # (the family libraries' launcher headers are not included by these translation units)
-    headers = [h for h in glob.glob(os.path.join(kdir, "*.h")) + glob.glob(os.path.join(kdir, "*.cuh"))
-               if os.path.basename(h) not in ("latent_launchers.h", "hybrid_launchers.h", "wave_dot.h", "direct_lds.h",
-                                           "attn_tiles.h", "bf16_parts.h", "walk_places.h", "decay_token.h", "row_units.h")]
     sources = sorted(s for s in glob.glob(os.path.join(kdir, "*.hip"))
                      if os.path.basename(s) not in LATENT_KERNELS + HYBRID_KERNELS)
     tinc, tlib, abi = _torch_paths()
@@ -124,13 +138,13 @@ def build_kernels(verbose: bool = False, force: bool = False) -> str:
     for src in sources:
         obj = os.path.join(OBJ, os.path.basename(src) + ".o")
         objs.append(obj)
-        if force or _newer(obj, [src] + headers):
+        if force or _newer(obj, [src] + _includes(src)):
             jobs.append([HIPCC, "-c", src, "-o", obj, "-I", kdir] + HIP_FLAGS + NO_PACKED_FP32)
     for bsrc in sorted(b for b in glob.glob(os.path.join(CSRC, "bindings", "*.cpp"))
                        if os.path.basename(b) not in LATENT_BINDINGS + HYBRID_BINDINGS):
         bobj = os.path.join(OBJ, "bind_" + os.path.basename(bsrc) + ".o")
         objs.append(bobj)
-        if force or _newer(bobj, [bsrc] + headers):
+        if force or _newer(bobj, [bsrc] + _includes(bsrc, kdir)):
             cmd = [HIPCC, "-c", bsrc, "-o", bobj, "-I", kdir, "-O2", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
                    "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
                    "-DTORCH_EXTENSION_NAME=_C", "-Wno-unused-result", "-Wno-deprecated-declarations"]
@@ -155,18 +169,17 @@ def build_latent(verbose: bool = False, force: bool = False) -> str:
     (``torch.ops.symmetry_amd_latent``)."""
     os.makedirs(OBJ, exist_ok=True)
     kdir = os.path.join(CSRC, "kernels")
-    headers = [os.path.join(kdir, h) for h in ("common.h", "attn_tiles.h", "direct_lds.h", "latent_launchers.h")]
     tinc, tlib, abi = _torch_paths()
     jobs, objs = [], []
     for name in LATENT_KERNELS:
         src, obj = os.path.join(kdir, name), os.path.join(OBJ, name + ".o")
         objs.append(obj)
-        if force or _newer(obj, [src] + headers):
+        if force or _newer(obj, [src] + _includes(src)):
             jobs.append([HIPCC, "-c", src, "-o", obj, "-I", kdir] + HIP_FLAGS + NO_PACKED_FP32)
     for name in LATENT_BINDINGS:
         src, obj = os.path.join(CSRC, "bindings", name), os.path.join(OBJ, "bind_" + name + ".o")
         objs.append(obj)
-        if force or _newer(obj, [src] + headers):
+        if force or _newer(obj, [src] + _includes(src, kdir)):
             cmd = [HIPCC, "-c", src, "-o", obj, "-I", kdir, "-O2", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
                    "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
                    "-DTORCH_EXTENSION_NAME=_C_latent", "-Wno-unused-result", "-Wno-deprecated-declarations"]
@@ -190,19 +203,17 @@ def build_hybrid(verbose: bool = False, force: bool = False) -> str:
     symmetry_amd/_C_hybrid.so (``torch.ops.symmetry_amd_hybrid``)."""
     os.makedirs(OBJ, exist_ok=True)
     kdir = os.path.join(CSRC, "kernels")
-    headers = [os.path.join(kdir, h) for h in ("common.h", "wave_dot.h", "direct_lds.h", "attn_tiles.h", "bf16_parts.h", "walk_places.h", "decay_token.h", "row_units.h", "hybrid_launchers.h",
-                                                  "latent_launchers.h")]
     tinc, tlib, abi = _torch_paths()
     jobs, objs = [], []
     for name in HYBRID_KERNELS + HYBRID_SHARED:
         src, obj = os.path.join(kdir, name), os.path.join(OBJ, name + ".o")
         objs.append(obj)
-        if force or _newer(obj, [src] + headers):
+        if force or _newer(obj, [src] + _includes(src)):
             jobs.append([HIPCC, "-c", src, "-o", obj, "-I", kdir] + HIP_FLAGS + NO_PACKED_FP32)
     for name in HYBRID_BINDINGS:
         src, obj = os.path.join(CSRC, "bindings", name), os.path.join(OBJ, "bind_" + name + ".o")
         objs.append(obj)
-        if force or _newer(obj, [src] + headers):
+        if force or _newer(obj, [src] + _includes(src, kdir)):
             cmd = [HIPCC, "-c", src, "-o", obj, "-I", kdir, "-O2", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
                    "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
                    "-DTORCH_EXTENSION_NAME=_C_hybrid", "-Wno-unused-result", "-Wno-deprecated-declarations"]
