@@ -804,7 +804,7 @@ void launch_chunks(const DecayScanArgs& a, hipStream_t s) {
     // eight waves a workgroup where LDS (mode 0) or their number (at most one a CU) leaves one of them on a CU
     if (MODE == 0 || (long long)((a.P + 63) / 64) * a.H * std::max(a.runs, a.segments) <= 256) return launch_scan<MODE, NB, 2>(a, s);
   }
-  launch_scan<MODE, NB, 1>(a, s);
+  if constexpr (MODE == 1 || NB == 1) launch_scan<MODE, NB, 1>(a, s);
 }
 
 template <int MODE>

@@ -9,6 +9,9 @@ the compiler itself leaves along a block).
 M0: one wait state between the scalar instruction that writes it and a load to LDS, which takes its LDS address from there.  The compiler
 does not look into assembly, so these loads bring theirs along.
 
+Scalar registers: five wait states between a vector instruction that writes one and a memory instruction that reads it.  The compiler's
+own spills are such writes, and where assembly reads them behind, it does not put the wait states in.
+
 Wide stores: one wait state before a vector instruction overwrites data of more than 64 bits a lane.
 """
 import concurrent.futures
@@ -92,12 +95,27 @@ def after(code, i, need, hit):
     return sorted(found)
 
 
+MEMORY = ("global_", "buffer_", "flat_", "scratch_")
+
+
+@functools.lru_cache(1 << 14)
+def scalars(text):
+    out = {"vcc"} if re.search(r"\bvcc\b", text) else set()
+    for first, last, one in re.findall(r"(?<!\w)s(?:\[(\d+):(\d+)\]|(\d+))(?![\w:\[])", text):
+        out.update(range(int(first), int(last) + 1) if first else [int(one)])
+    return frozenset(out)
+
+
 def close(code):
-    """[(place, place, wait states between)] of M0 and the loads to LDS that read it, of wide stores and what overwrites their data."""
+    """[(place, place, wait states between)] of M0 and the loads to LDS that read it, of scalar registers that a vector instruction writes
+    and memory instructions that read them, of wide stores and what overwrites their data."""
     found = []
     for i, (op, text, _) in enumerate(code):
         if op.startswith("s_") and re.match(r"m0\b", text):
-            rest = after(code, i, 1, lambda o, t: re.search(r"_lds_|\blds\b", o + " " + t) and o.startswith(("global_", "buffer_")))
+            rest = after(code, i, 1, lambda o, t: re.search(r"_lds_|\blds\b", o + " " + t) and o.startswith(MEMORY))
+        elif op.startswith("v_") and re.match(r"s\[?\d|vcc", text):
+            to = scalars(re.match(r"s\[\d+:\d+\]|\w+", text)[0])
+            rest = after(code, i, 5, lambda o, t: o.startswith(MEMORY) and scalars(t) & to)
         elif re.match(r"(global|flat|buffer|scratch)_store_dwordx[34]$", op):
             data = operands(text)[0 if op.startswith("buffer") else 1]
             rest = after(code, i, 1, lambda o, t: o.startswith("v_") and not o.startswith("v_mfma") and operands(t)[0] & data)
@@ -168,11 +186,14 @@ def test_matrix_results():
     assert early([product, ("v_mfma_f32_32x32x16_bf16", "a[0:15], v[4:7], v[8:11], a[0:15]", None), nop(6), store, end]) == [(0, 3, 7)]
 
 
-def test_m0_and_stores():
+def test_m0_scalars_and_stores():
     m0, load, end = ("s_mov_b32", "m0, s5", None), ("buffer_load_dwordx4", "v58, s[8:11], s39 offen lds", None), ("s_endpgm", "", None)
     nop = ("s_nop", "0", None)
     assert close([m0, load, end]) == [(0, 1, 0)] and close([m0, nop, load, end]) == []
     assert close([m0, ("s_branch", "", 3), end, ("global_load_lds_dwordx4", "v[6:7], off", None), end]) == []
+    spill = ("v_readlane_b32", "s39, v234, 5", None)
+    assert close([spill, nop, load, end]) == [(0, 2, 1)] and close([spill, ("s_nop", "4", None), load, end]) == []
+    assert close([("v_readlane_b32", "s40, v234, 5", None), load, end]) == [] and close([("v_cmp_gt_i32_e32", "vcc, 5, v1", None), load]) == []
     store = ("global_store_dwordx4", "v[0:1], v[4:7], off sc0 sc1", None)
     assert close([store, ("v_mov_b32_e32", "v5, 0", None), end]) == [(0, 1, 0)] and close([store, nop, ("v_mov_b32_e32", "v5, 0", None), end]) == []
     assert close([store, ("v_mov_b32_e32", "v0, 0", None), end]) == []
