@@ -398,7 +398,7 @@ void decay_scan(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v,
 DecayTokenArgs token_args(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dz, const OptTensor& low,
                           const Tensor& dbias, const OptTensor& rate, double tau, const OptTensor& skip, double q_scale, int64_t H,
                           int64_t N, int64_t P, int64_t hpg, Tensor& state, const Tensor& prev_row, const Tensor& save_slot,
-                          const Tensor& gate, const Tensor& w, double eps, bool sigmoid, Tensor& out, const OptTensor& ss) {
+                          const Tensor& gate, const Tensor& w, double eps, Tensor& out, const OptTensor& ss) {
   TORCH_CHECK(mode == 0 || mode == 1, "decay_token: mode");
   DecayTokenArgs d{};
   const int64_t T = v.size(0);
@@ -411,7 +411,7 @@ DecayTokenArgs token_args(int64_t mode, const Tensor& q, const Tensor& k, const 
   dtype(w, at::kFloat, "w");
   same_act(out, 0, "out");
   TORCH_CHECK(w.numel() > 0 && w.numel() <= H * P && (H * P) % w.numel() == 0 && out.numel() == T * H * P, "decay_token: shapes");
-  d.w = ptr<float>(w), d.wlen = (int)w.numel(), d.eps = (float)eps, d.sigmoid = sigmoid;
+  d.w = ptr<float>(w), d.wlen = (int)w.numel(), d.eps = (float)eps;
   d.out = out.data_ptr();
   if (ss.has_value()) {
     dtype(*ss, at::kFloat, "ss");
@@ -424,9 +424,9 @@ DecayTokenArgs token_args(int64_t mode, const Tensor& q, const Tensor& k, const 
 bool decay_token(int64_t mode, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& dz, const OptTensor& low,
                  const Tensor& dbias, const OptTensor& rate, double tau, const OptTensor& skip, double q_scale, int64_t H, int64_t N,
                  int64_t P, int64_t hpg, Tensor& state, const Tensor& prev_row, const Tensor& save_slot, const Tensor& gate,
-                 const Tensor& w, double eps, bool sigmoid, Tensor& out, const OptTensor& ss) {
+                 const Tensor& w, double eps, Tensor& out, const OptTensor& ss) {
   return launch_decay_token(token_args(mode, q, k, v, dz, low, dbias, rate, tau, skip, q_scale, H, N, P, hpg, state, prev_row, save_slot,
-                                       gate, w, eps, sigmoid, out, ss),
+                                       gate, w, eps, out, ss),
                             cur_stream(v));
 }
 
@@ -440,7 +440,7 @@ bool window_attn_decay(const Tensor& q, const Tensor& k_cache, const Tensor& v_c
   const WindowAttnArgs a = attn_args(q, k_cache, v_cache, block_tables, row_seq, positions, window, scale, gate, out, std::nullopt,
                                      std::nullopt, std::nullopt, 0, std::nullopt, 0., std::nullopt, part_o, part_ml, counters, part_keys);
   const DecayTokenArgs d = token_args(0, dq, dk, dv, dz, low, dbias, std::nullopt, tau, std::nullopt, q_scale, H, N, P, 1, state, prev_row,
-                                      save_slot, ngate, w, eps, false, gy, std::nullopt);
+                                      save_slot, ngate, w, eps, gy, std::nullopt);
   return launch_split_attn_decay(a, d, cur_stream(q));
 }
 
@@ -1578,7 +1578,7 @@ TORCH_LIBRARY(symmetry_amd_hybrid, m) {
   m.def(
       "decay_token(int mode, Tensor q, Tensor k, Tensor v, Tensor dz, Tensor? low, Tensor dbias, Tensor? rate, float tau, Tensor? skip, "
       "float q_scale, int H, int N, int P, int hpg, Tensor(a!) state, Tensor prev_row, Tensor save_slot, Tensor gate, Tensor w, "
-      "float eps, bool sigmoid, Tensor(b!) out, Tensor(c!)? ss) -> bool",
+      "float eps, Tensor(b!) out, Tensor(c!)? ss) -> bool",
       &decay_token);
   m.def(
       "window_attn_decay(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor row_seq, Tensor positions, int window, "

@@ -96,8 +96,7 @@ SYM_DEV void decay_token_block(const DecayTokenArgs& d, int h, int run, float* l
   float y = 0.f;
   if (tid < P) {
     y = (red[tid] + red[P + tid]) + (red[2 * P + tid] + red[3 * P + tid]) + (a.skip ? a.skip[h] * own : 0.f);
-    const float s = 1.f / (1.f + expf(-gate));
-    gate = d.sigmoid ? s : gate * s;
+    gate *= 1.f / (1.f + expf(-gate));
     if (d.ss) y *= gate;
   }
   const float sq = block_sum<DECAY_NT>(y * y, scratch);

@@ -50,14 +50,17 @@ __global__ __launch_bounds__(NT) void delta_token_kernel(DeltaTokenArgs a) {
     w = *reinterpret_cast<const uint4*>(reinterpret_cast<const bf16*>(a.cw) + (long long)c * TAPS);
   } else if (wave >= 4) {
     const bf16 *g = reinterpret_cast<const bf16*>(a.gx) + row * a.ldgx, *w0 = reinterpret_cast<const bf16*>(a.gw) + (long long)h * a.gd,
-               *w1 = w0 + (CHANNEL ? 0 : (long long)a.H * a.gd);
+               *w1 = w0 + (long long)a.H * a.gd;
     for (int i = 8 * (tid - 256); i < a.gd; i += 8 * 256) {
       float gv[8], wv[8], uv[8];
       load8(g + i, gv);
       load8(w0 + i, wv);
-      load8(w1 + i, uv);
+      if constexpr (!CHANNEL) load8(w1 + i, uv);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) d0 += gv[j] * wv[j], d1 += gv[j] * uv[j];
+      for (int j = 0; j < 8; ++j) {
+        d0 += gv[j] * wv[j];
+        if constexpr (!CHANNEL) d1 += gv[j] * uv[j];
+      }
     }
   }
   const float rate = expf(a.A_log[h]);
@@ -165,7 +168,7 @@ __global__ __launch_bounds__(NT) void delta_token_kernel(DeltaTokenArgs a) {
     }
   } else if (wave >= 4) {
     d0 = wave_sum(d0);
-    d1 = wave_sum(d1);
+    if constexpr (!CHANNEL) d1 = wave_sum(d1);
     if (lane == 0) dots[wave - 4] = d0, dots[wave] = d1;
   }
   __syncthreads();

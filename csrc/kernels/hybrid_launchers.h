@@ -323,14 +323,13 @@ void decay_chunk_segments(DecayScanArgs& a);      // ws holds decay_chunk_scratc
 void launch_decay_chunks(const DecayScanArgs& a, hipStream_t s);
 void launch_decay_scan(const DecayScanArgs& a, int f32, hipStream_t s);
 // One token a run in bf16 (cu_q null, T = runs; s.out is not written), with what follows the scan: out [T][H P] =
-// y / rms(head) * w * s(gate), s = silu or sigmoid; with ss: out = y s(gate) w as it is, and ss [T][H] the sums of (y s(gate))^2, for
-// a norm over all heads whose factor the next product applies
+// y / rms(head) * w * silu(gate); with ss: out = y silu(gate) w as it is, and ss [T][H] the sums of (y silu(gate))^2, for a norm over
+// all heads whose factor the next sum applies
 struct DecayTokenArgs {
   DecayScanArgs s;
   const void* low; long long ldl; int rank;   // mode 0: not null: s.dz is [H N][rank] and the pre-activations are bf16(low . dz^T)
   const void* gate; long long ldg;              // [T][H P]
   const float* w; int wlen; float eps;          // w [wlen] repeats over the columns
-  int sigmoid;
   void* out;
   float* ss;
 };

@@ -1202,7 +1202,7 @@ def decay_scan(mode, q, k, v, dz, dbias, dparam, skip, q_scale, H, N, P, hpg, st
 
 
 def decay_token(mode, q, k, v, dz, low, dbias, dparam, skip, q_scale, H, N, P, hpg, state, prev_row, save_slot, gate, w, eps, out,
-                ss=None, sigmoid=False) -> bool:
+                ss=None) -> bool:
     """decay_scan of rows that are runs of their own (decode steps, bf16) and what follows it, in one launch: out bf16 [T, H P] =
     gated_group_norm(., gate, w, eps, P, False).  ``ss`` fp32 [T, H]: out = y silu(gate) w as it is and ss its heads' sums of
     (y silu(gate))^2, for a norm over all heads whose factor a later sum applies (``residual_mix_norm``).  ``low`` [T, rank] (channel
@@ -1212,7 +1212,7 @@ def decay_token(mode, q, k, v, dz, low, dbias, dparam, skip, q_scale, H, N, P, h
         return False
     dp = dparam if torch.is_tensor(dparam) else None
     return _hyb().decay_token(int(mode), q, k, v, dz, low, dbias, dp, 0.0 if dp is not None else float(dparam), skip, float(q_scale),
-                              int(H), int(N), int(P), int(hpg), state, prev_row, save_slot, gate, w, float(eps), bool(sigmoid), out, ss)
+                              int(H), int(N), int(P), int(hpg), state, prev_row, save_slot, gate, w, float(eps), out, ss)
 
 
 def window_attn_decay(q, k_cache, v_cache, block_tables, row_seq, positions, window, scale, gate, out, split, dq, dk, dv, dz, low, dbias,
