@@ -249,8 +249,9 @@ class BeletarLM:
         olat = self._buf("lat.o", (T, H, r))
         part_o = part_ml = None
         if b.kind == "decode" and self.device.type != "cpu":
-            # (many rows: partitions of a whole step of the kernel's waves; 64 of 300 keys 18.8 / 13.9 us, 3 of 617 8.9 / 10.2)
-            parts = ops.latent_attn_parts(T, b.block_tables.shape[1] * cache.block_size, min_tokens=128 if T >= 16 else 64)
+            span = b.block_tables.shape[1] * cache.block_size
+            least = ops.latent_row_tokens(T, H, span, r, rot, cache.block_size) if self.dtype == torch.bfloat16 else 64
+            parts = ops.latent_attn_parts(T, span, min_tokens=least)
             if parts > 1:
                 part_o = self._buf("lat.part_o", (T, H, parts, r), torch.float32)
                 part_ml = self._buf("lat.part_ml", (T, H, parts, 2), torch.float32)

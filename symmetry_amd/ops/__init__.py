@@ -1007,6 +1007,21 @@ def latent_attn_parts(rows: int, span: int, target_wgs: int = 512, min_tokens: i
     return max(1, min(-(-span // min_tokens), -(-target_wgs // max(1, rows)), 1024))
 
 
+def latent_row_tokens(rows: int, heads: int, span: int, kv_rank: int, rot: int, block: int) -> int:
+    """``min_tokens`` of latent_attn_parts for a decode step in bf16: 64, and 128 for the kernel of 512 + 64 entries over blocks of 32
+    tokens and more where partitions of 64 keys, all of them full, would be more than its one workgroup a CU, or more than 64 a row,
+    which the merge takes through LDS.  16 heads, us with 64 / 128 at contexts of a mean:
+
+    512 tokens of table   16 rows of 250 11.4 / 12.4   32 of 340 12.5 / 13.0 | 36 of 100 12.2 / 13.0, of 340 18.7 / 13.7   64 of 250 20.2 / 14.6
+    2048                  8 rows of 500 11.7 / 12.5, of 1360 13.1 / 13.1 | 10 of 500 12.4 / 13.1, of 1360 19.3 / 14.2   16 of 500 12.0 / 12.8, of
+                          700 17.4 / 13.0, of 1360 22.0 / 16.4   24 of 500 12.9 / 13.3, of 900 23.4 / 16.5, of 1360 25.1 / 26.4   40 of 700 25.5 / 25.2
+    8192                  1 row of 5000 62.2 / 14.5   4 76.7 / 16.8   16 37.3 / 37.1 (32 partitions either way)"""
+    if (kv_rank, rot) != (512, 64) or block < 32 or block & (block - 1):
+        return 64
+    parts = -(-span // 64)
+    return 128 if parts > 64 or rows * -(-heads // 16) * parts > 256 else 64
+
+
 LATENT_ATTN_IMPL = 1 if os.environ.get("SYMMETRY_LATENT_ATTN", "mfma") == "wave" else 0  # A/B: the all-shapes kernel
 
 
