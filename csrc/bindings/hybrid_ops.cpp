@@ -1,12 +1,11 @@
-// TORCH_LIBRARY registration of the kernels in hybrid_rows.hip, stream_rows.hip, norm_rows.hip, routed_ff.hip,
-// window_attention.hip, decay_scan.hip and delta_rule.hip, plus the expert-segment kernels of glu_moe.hip that the routed
-// feed-forward shares (symmetry_amd/_C_hybrid.so, namespace symmetry_amd_hybrid).
+// TORCH_LIBRARY registration of the kernels that hybrid_launchers.h names, plus the expert-segment kernels of glu_moe.hip that the
+// routed feed-forward shares (symmetry_amd/_C_hybrid.so, namespace symmetry_amd_hybrid).
 //
-// Out-parameter style like the other kernel libraries: the caller pre-allocates, nothing is allocated here, every
-// launch goes to torch's current HIP stream (hipGraph-capturable), and every shape / dtype / range the kernels and
-// their grids assume is checked on the host before the launch.  Activation tensors are all bf16 or all fp32; which
-// one is read off the first activation argument.  "view" arguments may be column ranges of a wider matrix (unit inner
-// stride, any row stride).
+// Out-parameter style like the other kernel libraries: the caller pre-allocates, and nothing is allocated here but decay_scan's scratch
+// where the caller's is smaller than decay_scratch says.  Every launch goes to torch's current HIP stream (hipGraph-capturable), and
+// every shape / dtype / range the kernels and their grids assume is checked on the host before the launch.  Activation tensors are
+// all bf16 or all fp32; which one is read off the first activation argument.  "view" arguments may be column ranges of a wider matrix
+// (unit inner stride, any row stride).
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>

@@ -77,9 +77,10 @@ SYM_DEV int first_chunk(unsigned wg, int nch, long long x_bytes) {
   return (int)(((wg & 7) * (unsigned)nch / 8 + (wg >> 3) * spread) % (unsigned)nch);
 }
 
-// A matrix product's result is in its registers some 11 cycles of waiting later.  The compiler puts these in along a block, but not where a
-// branch that is taken stands between the product and what reads it (a tile in 100 was wrong in a fourth of its columns): such results
-// pass through here.
+// A matrix product's result is in its registers 8 wait states later (32 x 32: 12).  The compiler puts these in, but on some paths through
+// taken branches it leaves up to seven of them out: 36864 x 1024 at 16 rows had a fourth of a tile's columns wrong in three of 200 runs,
+// some 6 tiles in 10^6, which a test's one run does not show.  Results of kernels whose code had such a path pass through here;
+// tests/test_wait_states_cpu.py walks the code of all of them.
 SYM_DEV void settle(f32x4& v) { asm volatile("s_nop 15" : "+v"(v)); }
 
 // Non-temporal 16-byte load (weights that are streamed once).

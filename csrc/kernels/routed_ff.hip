@@ -677,8 +677,9 @@ void launch_tiles(const ExpertArgs& a, hipStream_t s) {
 // stages run on over the tile boundaries: a tile's first two load while the last products and the epilogue of the one before run.
 // Every XCD walks its run of the tiles whole ones first; the whole ones that would be left for a last partial round are cut in two.
 // The gated epilogue's division is a product with v_rcp_f32's reciprocal: the matrix cores wait for it, and its error (1 ulp of fp32) is none
-// of the result's (2048 x 2048 at 2048 rows, against 64 bits 0.001659324 of the norm either way; 8192 x 2048 dense, 8100 rows 432 -> 417 us,
-// 4096 x 1024, 4000 rows 64.8 -> 61.3).  Loads, reads and products stand in turns: all of an operand's loads at once 420 -> 447.
+// of the result's (2048 x 2048 at 2048 rows, against 64 bits 0.001659324 of the norm either way, and at 4 to 64 experts of 768 to 14336
+// outputs, gates of 0.1 to 8, the same to nine places too; 8192 x 2048 dense, 8100 rows 432 -> 417 us, 4096 x 1024, 4000 rows 64.8 ->
+// 61.3).  Loads, reads and products stand in turns: all of an operand's loads at once 420 -> 447.
 // LDS rows as in expert_tile_kernel.  K % 64 == 0, K >= PERSIST_K, x and an expert's weights below 2 GiB.
 constexpr int PERSIST_K = 512, PERSIST_OP = 32 * 1024, PERSIST_LDS = 5 * PERSIST_OP;
 

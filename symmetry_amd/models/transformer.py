@@ -231,9 +231,10 @@ class TransformerLM:
           grouped prefill GEMM kernels); the fp32 oracle and exports unshuffle (layout.natural_tensors);
         * "shared": row-major only (the decode GEMMs' row-major variants);
         * "auto": MoE models "replace" (profiles/r6/e2e_mixtral_c5_single_copy.jsonl: equal end to end, 90 GB
-          less), or where the experts' shapes do not tile for it copies of wqkv and wo for decode steps; dense models "preshuffled" when the copy fits next to the KV cache's need (transformer.copy_budget;
-          their prefill is faster on the library GEMMs), "replace" otherwise (70B on one GPU: 141 GB of layer
-          weights), row-major only where neither applies."""
+          less), or where the experts' shapes do not tile for it copies of wqkv and wo for decode steps; dense models
+          "preshuffled" when the copy fits next to the KV cache's need (transformer.copy_budget; their prefill is faster
+          on the library GEMMs), "replace" otherwise (70B on one GPU: 141 GB of layer weights), row-major only where
+          neither applies."""
         if not self.fused or mode == "shared" or (self.device.type == "cpu" and mode != "replace"):
             return {}
         names = ["wqkv", "wo"] + ([] if self.cfg.is_moe else ["w_gu", "w_down"])
@@ -248,7 +249,8 @@ class TransformerLM:
             budget = copy_budget(self.device, self.kv_reserve)
             if self.moe is not None and not self.moe.single_copy_ok():
                 # (the experts keep their rows; the attention's projections of decode steps, a few per cent of the weights, have a copy
-                # beside theirs: 8 rows of 3072 x 2048 7.6 -> 5.9 us, of 2048 x 2048 6.1 -> 4.9)
+                # beside theirs: 8 rows of 3072 x 2048 7.6 -> 5.9 us, of 2048 x 2048 6.1 -> 4.9; steps of four layers of 16 experts at 1 / 8 /
+                # 17 / 32 / 64 rows 233 / 367 / 434 / 476 / 570 -> 225 / 356 / 423 / 473 / 560, at 96 and 128 as without)
                 if extra > budget:
                     return {}
                 head, self.decode_only_copies = None, True

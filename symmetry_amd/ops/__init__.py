@@ -687,7 +687,8 @@ def tile_plan(M: int, N: int, K: int, ws: bool) -> tuple[int, int] | None:
 
     Fewer tiles with K up to 2048 take 1.1 to 1.2 of the library's 12 to 13 us (in two slices where that fits, 1.08 to 1.13), but the
     library's call costs the host 20 us and this one 9, and prompt steps of recurrent stacks of so few rows are not ahead of the device:
-    four layers, 300 rows, 814 -> 753 and 648 -> 616 us.  Those are the ones that have a workspace."""
+    four layers, 300 rows, 814 -> 753 and 648 -> 616 us.  Those are the ones that have a workspace; steps that a graph replays, where the
+    host's time does not count, end at 256 rows."""
     if M <= MID_ROWS or K < 1024 or K % 64 or N < 512:
         return None
     small, large = -(-M // 64) * -(-N // 128), -(-M // 128) * -(-N // 128)

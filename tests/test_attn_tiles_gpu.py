@@ -1,5 +1,5 @@
 """Prompt attention over key tiles of 64 in LDS (csrc/kernels/attention.hip, attn_prefill_m32p_kernel) against attention in 64 bits, at the
-ends of its tiles and subtiles, for every block size that it takes.
+ends of its tiles and subtiles, for blocks of half a tile (the entry takes no smaller ones) to two.
 
 Bound: a weight is rounded to bf16 (8 bits: at most 2^-8 of it) in front of the product with the values, the result once more (2^-8 of
 it); scores and sums are fp32 (2^-20 of the weights covers both)."""

@@ -50,7 +50,8 @@ def test_dg_f32(gpu, M, N, K):
 def test_streams_in_flight(gpu, M, N, K):
     """Preshuffled weights past the caches: fewer k-blocks a wave than its ring has, as many, a part more, twice as many and more; K in
     two slices; walks of 1 to 9 tiles a workgroup, two or four of them in flight.  fp32 sums of K products of bf16 values against 64
-    bits: off by about sqrt(K) 2^-24 of the vectors' norms at most, four times that is allowed."""
+    bits: off by about sqrt(K) 2^-24 of the vectors' norms at most, four times that is allowed.  (A sum that is stored too early, a few in
+    10^6 tiles, is not seen here: test_wait_states_cpu.py looks for that in the code.)"""
     from symmetry_amd.models.layout import preshuffle
 
     print("dg_f32", M, N, K, flush=True)
